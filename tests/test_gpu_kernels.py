@@ -134,6 +134,26 @@ def test_gemm_plain_rows_do_not_depend_on_the_batch(ops, dtype, k):
         assert torch.equal(full[rows], part), rows
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,k,most", [(70, 65, 70), (3584, 260, 200), (4700, 516, 130), (9000, 1000, 70), (8192, 68, 1000), (257, 1, 129)])
+def test_gemm_plain_layouts(ops, dtype, n, k, most):
+    """Every layout that row counts choose against these widths (one or two tiles of 16 rows either way a wavefront,
+    tiles of 64 and of 128): the same bits for a row in all of them, and the bound of a sum of four chains of K / 4
+    rounded steps, (K / 4 + 4) 2^-24 of the sum of the magnitudes."""
+    g = torch.Generator().manual_seed(n + k)
+    x = torch.randn(most, k, generator=g).to(dtype).to(DEV)
+    w = torch.randn(n, k, generator=g).to(dtype).to(DEV)
+    whole = ops.gemm_plain(x, w, out_float32=True)
+    room = (k / 4 + 64 + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)  # (a range is rounded up to 64)
+    assert bool(((whole.double() - x.double() @ w.double().T).abs() <= room).all())
+    wide = torch.full((most, k + 3), float("nan"), dtype=dtype, device=DEV)  # rows that 16-byte loads do not fit
+    wide[:, :k] = x
+    for m in (1, 15, 16, 17, 32, 33, 64, 65, 128, 129):
+        if m <= most:
+            assert torch.equal(ops.gemm_plain(x[:m], w, out_float32=True), whole[:m]), m
+            assert torch.equal(ops.gemm_plain(wide[:m, :k], w, out_float32=True), whole[:m]), m
+
+
 @pytest.mark.parametrize("m", [1, 5, 16, 17, 33, 64, 65, 100, 128])
 @pytest.mark.parametrize("n,k", [(7, 8), (130, 104), (320, 96), (3584, 1000), (301, 2056), (4608, 3584), (33000, 136)])
 def test_gemm_skinny(ops, m, n, k):

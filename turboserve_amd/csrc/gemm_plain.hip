@@ -1,186 +1,483 @@
-// Y[M, N] = X[M, K] * W[N, K]^T (+ bias[N]) with plain 32-bit fused multiply-adds: no matrix
-// cores, no reduced-precision mode.  This is the product of the true 32-bit path (the
-// reference's F.linear, src/turboserve/engine/model/layers.py:142, at dtype float32) and the
-// checked stand-in for any faster product.  Every output element is one k-ordered chain of
-// fmaf, so a row's result does not depend on which other rows are in the batch.
+// Y[M, N] = X[M, K] * W[N, K]^T (+ bias[N]) in true 32-bit, no reduced-precision mode: the product
+// of the true 32-bit path (the reference's F.linear, src/turboserve/engine/model/layers.py:142, at
+// dtype float32) and of bfloat16 operands whose K the 16-byte loads of the other products do not divide.
 //
-// Tiles of 64 x 64 outputs per 256-thread block, 16-deep slices of K staged through LDS; every
-// load and store is bounds-checked, so M, N and K are arbitrary.
+// Every output is the sum, in order, of up to four chains, one per range of K (`range_of`: a quarter of K
+// rounded up to 64); a chain is fused multiply-adds in the order of k, each rounded once to 32-bit.
+// The chains run on the matrix cores: v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32 add their
+// two (four) products to the accumulator one after the other, in the order of k, each step a fused
+// multiply-add rounded to nearest with denormals kept (a loop of fmaf gives the same bits; compared
+// over random, widely spread, denormal and cancelling operands at K of 4 to 3,584).  So a row's
+// result depends neither on which other rows are in the batch nor on which of the two layouts
+// below runs it, both run at the matrix cores' 157 TFLOP/s, twice what unpacked vector
+// multiply-adds allow, and a few rows against a long K get four times the wavefronts one chain would.
+//
+// Microseconds at the 7B shape, one chain of vector multiply-adds (64 x 64 tiles; up to 32 rows one output a thread)
+// -> these: gate|up at 8 / 64 / 500 rows 194 -> 122, 765 -> 208, 3,048 -> 1,142 (119 TFLOP/s); down 220 -> 60, 3,402 -> 159,
+// 3,365 -> 724; o 35 -> 15, 581 -> 38, 581 -> 139; q|k|v 41 -> 23, 579 -> 72, 638 -> 195; the head at 8 rows 637 -> 433.
 #include "common.hpp"
 
-#define GP_BM 64
-#define GP_BN 64
-#define GP_BK 16
+namespace {
 
-template <typename TIn, typename TOut>
-__global__ void __launch_bounds__(256)
-gemm_plain_kernel(TOut* __restrict__ y, const TIn* __restrict__ x, const TIn* __restrict__ w,
-                  const TIn* __restrict__ bias, int m, int n, int k, long x_stride, long y_stride) {
-  __shared__ float xs[GP_BK][GP_BM + 1];
-  __shared__ float ws[GP_BK][GP_BN + 1];
-  const int tid = threadIdx.x;
-  const int tx = tid % 16;
-  const int ty = tid / 16;
-  const int m0 = blockIdx.y * GP_BM;
-  const int n0 = blockIdx.x * GP_BN;
+typedef float gp_f32x4 __attribute__((ext_vector_type(4)));
+typedef float gp_f32x16 __attribute__((ext_vector_type(16)));
+typedef unsigned int gp_u32x2 __attribute__((ext_vector_type(2)));
 
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+constexpr int GP_DIES = 8;
+constexpr int GP_UNITS = 256;  // compute units of an MI355X
 
-  for (int k0 = 0; k0 < k; k0 += GP_BK) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int idx = tid + i * 256;
-      const int r = idx / GP_BK;
-      const int c = idx % GP_BK;
-      const int gm = m0 + r;
-      const int gn = n0 + r;
-      const int gk = k0 + c;
-      xs[c][r] = (gm < m && gk < k) ? to_float(x[(size_t)gm * x_stride + gk]) : 0.f;
-      ws[c][r] = (gn < n && gk < k) ? to_float(w[(size_t)gn * k + gk]) : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < GP_BK; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = xs[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = ws[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
+// Four consecutive elements of one row as they lie in memory, and as 32-bit values.
+template <typename TIn>
+struct Quad;
+template <>
+struct Quad<float> {
+  gp_f32x4 v;
+  __device__ __forceinline__ void load(const float* p) { v = *reinterpret_cast<const gp_f32x4*>(p); }
+  __device__ __forceinline__ void set(int i, float f) { v[i] = f; }
+  __device__ __forceinline__ gp_f32x4 values() const { return v; }
+};
+template <>
+struct Quad<bf16_t> {
+  gp_u32x2 v;
+  __device__ __forceinline__ void load(const bf16_t* p) { v = *reinterpret_cast<const gp_u32x2*>(p); }
+  __device__ __forceinline__ void set(int i, bf16_t f) {
+    const unsigned int other = v[i / 2];
+    const unsigned int both = i & 1 ? (other & 0xffffu) | ((unsigned int)f.bits << 16) : (other & 0xffff0000u) | f.bits;
+    v[i / 2] = both;
   }
-
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gm = m0 + ty * 4 + i;
-    if (gm >= m) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gn = n0 + tx * 4 + j;
-      if (gn >= n) continue;
-      float v = acc[i][j];
-      if (bias) v += to_float(bias[gn]);
-      y[(size_t)gm * y_stride + gn] = from_float<TOut>(v);
-    }
+  __device__ __forceinline__ gp_f32x4 values() const {
+    const unsigned int lo = v[0], hi = v[1];
+    return gp_f32x4{__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(hi << 16),
+                    __uint_as_float(hi & 0xffff0000u)};
   }
-}
+};
 
-// The same product, the same chain of fmaf per output (so the same bits), laid out for a few
-// rows: a decode step's products in the 32-bit path are bound by reading W, and 64 x 64 tiles
-// give eight rows against [3584, 18944] 56 workgroups that each walk 4.8 MB.  Here a workgroup
-// owns 16 x 16 outputs, one per thread, and walks K in slices of 64 that travel global ->
-// registers -> LDS (two buffers, one barrier a slice); a thread fetches four consecutive k of one
-// row (one 16-byte load where K allows), so a row's slice is 256 contiguous bytes, and its loads
-// are GF_AHEAD slices ahead of the arithmetic (a ring of registers).  Every load is unconditional
-// (addresses clamped into the tensor, what lies outside replaced by zero afterwards), so that
-// the compiler can count the loads in flight.
-#define GF_BM 16
-#define GF_BN 16
-#define GF_BK 64
-#define GF_ROW (GF_BK + 4)  // floats; keeps rows 16-byte aligned and apart in the banks
-#ifndef GF_AHEAD
-#define GF_AHEAD 2  // slices of loads in flight (even)
-#endif
+// The length of a range of K, the same for every layout: a function of K alone.
+__host__ __device__ constexpr int range_of(int k) { return (((k + 3) / 4 + 63) / 64) * 64; }
 
-typedef float gf_f32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int gf_u32x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ void few_rows_load4(float (&dst)[4], const float* p) {
-  const gf_f32x4 v = *reinterpret_cast<const gf_f32x4*>(p);
-  dst[0] = v[0], dst[1] = v[1], dst[2] = v[2], dst[3] = v[3];
-}
-__device__ __forceinline__ void few_rows_load4(float (&dst)[4], const bf16_t* p) {
-  const gf_u32x2 v = *reinterpret_cast<const gf_u32x2*>(p);
-  dst[0] = __uint_as_float(v[0] << 16), dst[1] = __uint_as_float(v[0] & 0xffff0000u);
-  dst[2] = __uint_as_float(v[1] << 16), dst[3] = __uint_as_float(v[1] & 0xffff0000u);
-}
-
-// Four consecutive k of one row, from k0 on; zeros for a row or a k outside the tensor.  VEC: K, the
-// row stride and the base address are multiples of four elements, so the four lie in the tensor
-// together or not at all and travel as one load.
+// Elements k0 + lane_k .. + 3 of a row: one load where VEC (K, the row strides and the base
+// addresses are multiples of four elements), else one by one.  Always inside the row: what lies past
+// its end is read from its last elements instead and cleared by the caller.
+template <bool VEC>
+struct RowOffset {  // of a tile's row from its first one, in elements: 32 bits where VEC (K and the row strides below 2^25)
+  typedef uint32_t type;
+};
+template <>
+struct RowOffset<false> {
+  typedef size_t type;
+};
 template <bool VEC, typename TIn>
-__device__ __forceinline__ void few_rows_fetch(float (&dst)[4], const TIn* base, long stride, int row, int rows, int k0,
-                                               int k) {
-  const TIn* from = base + (size_t)min(row, rows - 1) * stride;
+__device__ __forceinline__ void fetch_quad(Quad<TIn>& q, const TIn* base, typename RowOffset<VEC>::type row, int k0, int lane_k, int k) {
   if (VEC) {
-    few_rows_load4(dst, from + min(k0, k - 4));
-    const bool inside = row < rows && k0 < k;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dst[i] = inside ? dst[i] : 0.f;
+    q.load(base + k0 + (row + min(lane_k, k - 4 - k0)));
   } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float v = to_float(from[min(k0 + i, k - 1)]);
-      dst[i] = (row < rows && k0 + i < k) ? v : 0.f;
-    }
+    for (int i = 0; i < 4; ++i) q.set(i, base[k0 + (row + min(lane_k + i, k - 1 - k0))]);
   }
 }
 
-template <bool VEC, typename TIn, typename TOut>
-__global__ void __launch_bounds__(256)
-gemm_plain_few_rows_kernel(TOut* __restrict__ y, const TIn* __restrict__ x, const TIn* __restrict__ w,
-                           const TIn* __restrict__ bias, int m, int n, int k, long x_stride, long y_stride) {
-  __shared__ __attribute__((aligned(16))) float xs[2][GF_BM][GF_ROW];
-  __shared__ __attribute__((aligned(16))) float ws[2][GF_BN][GF_ROW];
-  const int tid = threadIdx.x;
-  const int m0 = blockIdx.y * GF_BM;
-  const int n0 = blockIdx.x * GF_BN;
-  const int fetch_row = tid / 16;       // the row of both tiles this thread fetches ...
-  const int fetch_k = (tid % 16) * 4;   // ... and its four consecutive k within a slice
-  const int out_m = tid % 16;           // the output this thread owns
-  const int out_n = tid / 16;
-  float xr[GF_AHEAD][4], wr[GF_AHEAD][4];  // slot j: a slice whose number is j modulo GF_AHEAD
-  auto fetch = [&](int slot, int slice) __attribute__((always_inline)) {
-    few_rows_fetch<VEC>(xr[slot], x, x_stride, m0 + fetch_row, m, slice * GF_BK + fetch_k, k);
-    few_rows_fetch<VEC>(wr[slot], w, (long)k, n0 + fetch_row, n, slice * GF_BK + fetch_k, k);
-  };
-  auto stage = [&](int slot, int buf) __attribute__((always_inline)) {
+// Clear the elements of a quad that lie past the row's end; `left`: how many lie inside.
+__device__ __forceinline__ void clear_past(gp_f32x4& v, int left) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      xs[buf][fetch_row][fetch_k + i] = xr[slot][i];
-      ws[buf][fetch_row][fetch_k + i] = wr[slot][i];
+  for (int i = 0; i < 4; ++i) v[i] = i < left ? v[i] : 0.f;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Many rows: a workgroup of 2 x 2 wavefronts owns 64 TM activation rows by 64 TN weight rows, a
+// wavefront TM x TN tiles of 32 x 32.  Bound by the matrix cores (an iteration of BK is BK TM TN / 2
+// instructions of 64 cycles a wavefront); loads go out two iterations ahead into one of two sets of registers.
+// In LDS every 8 k of a row lie as 0 2 4 6 1 3 5 7: the half of the wavefront that supplies the even
+// (odd) k of four consecutive instructions reads them as 16 bytes; rows are 4 floats longer than
+// their k, so that sixteen rows' pieces touch every bank once.
+template <int TM, int TN, int BK, bool VEC, typename TIn, typename TOut>
+__global__ void __launch_bounds__(256)
+gemm_plain_kernel(TOut* __restrict__ y, const TIn* __restrict__ x, const TIn* __restrict__ w,
+                  const TIn* __restrict__ bias, int m, int n, int k, long x_stride, long y_stride, int m_tiles, int n_tiles) {
+  constexpr int BM = 64 * TM, BN = 64 * TN, ROW = BK + 4, QUADS = BK / 4, PASS = 256 / QUADS;
+  constexpr int PX = BM / PASS, PW = BN / PASS;
+  __shared__ __attribute__((aligned(16))) float lds[2][(BM + BN) * ROW];
+  // Workgroup id -> tile: ids go to the eight dies in turn; the tiles of activation rows over one weight
+  // tile follow one another on one die and share the weights in its L2.
+  const int die = blockIdx.x % GP_DIES, turn = blockIdx.x / GP_DIES;
+  const int n_tile = (turn / m_tiles) * GP_DIES + die;
+  if (n_tile >= n_tiles) return;  // the whole workgroup leaves together
+  const int m0 = (turn % m_tiles) * BM, n0 = n_tile * BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 31, half = lane >> 5;
+  const int wave_m = wave >> 1, wave_n = wave & 1;
+
+  // A quad's address: the tile's first row (the same for the workgroup) and a 32-bit offset of the row.
+  const int quad_k = 4 * (tid % QUADS), quad_row = tid / QUADS;
+  const TIn* xbase = x + (size_t)m0 * x_stride;
+  const TIn* wbase = w + (size_t)n0 * k;
+  typedef typename RowOffset<VEC>::type Row;
+  Row xrow[PX], wrow[PW];
+#pragma unroll
+  for (int i = 0; i < PX; ++i) xrow[i] = (Row)min(quad_row + PASS * i, m - 1 - m0) * (Row)x_stride;
+#pragma unroll
+  for (int i = 0; i < PW; ++i) wrow[i] = (Row)min(quad_row + PASS * i, n - 1 - n0) * (Row)k;
+
+  struct Set {
+    Quad<TIn> x[PX], w[PW];
+  };
+  const int iters = (k + BK - 1) / BK;
+  auto fetch = [&](Set& s, int it) __attribute__((always_inline)) {
+    const int k0 = min(it, iters - 1) * BK;
+#pragma unroll
+    for (int i = 0; i < PX; ++i) fetch_quad<VEC>(s.x[i], xbase, xrow[i], k0, quad_k, k);
+#pragma unroll
+    for (int i = 0; i < PW; ++i) fetch_quad<VEC>(s.w[i], wbase, wrow[i], k0, quad_k, k);
+  };
+  const int at = quad_row * ROW + (quad_k & ~7) + (quad_k & 4) / 2;  // of the quad's even k; the odd ones 4 behind
+  auto stage = [&](const Set& s, int it, int buf) __attribute__((always_inline)) {
+    float* to = lds[buf] + at;
+    const int left = k - (it * BK + quad_k);
+    auto put = [&](gp_f32x4 v, int row) __attribute__((always_inline)) {
+      clear_past(v, left);
+      *reinterpret_cast<float2*>(to + row * ROW) = make_float2(v[0], v[2]);
+      *reinterpret_cast<float2*>(to + row * ROW + 4) = make_float2(v[1], v[3]);
+    };
+#pragma unroll
+    for (int i = 0; i < PX; ++i) put(s.x[i].values(), PASS * i);
+#pragma unroll
+    for (int i = 0; i < PW; ++i) put(s.w[i].values(), BM + PASS * i);
+  };
+
+  gp_f32x16 acc[TM][TN], sum[TM][TN];  // the range's chain, the ranges before it
+#pragma unroll
+  for (int a = 0; a < TM; ++a) {
+#pragma unroll
+    for (int b = 0; b < TN; ++b) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f, sum[a][b][i] = 0.f;
+    }
+  }
+  constexpr int GROUPS = BK / 8;  // eight k at a time
+  struct Frags {
+    gp_f32x4 x[TM], w[TN];
+  };
+  auto read = [&](Frags& f, int buf, int g) __attribute__((always_inline)) {
+    const float* xs = lds[buf] + (wave_m * 32 * TM + r) * ROW + 4 * half + 8 * g;
+    const float* ws = lds[buf] + (BM + wave_n * 32 * TN + r) * ROW + 4 * half + 8 * g;
+#pragma unroll
+    for (int a = 0; a < TM; ++a) f.x[a] = *reinterpret_cast<const gp_f32x4*>(xs + a * 32 * ROW);
+#pragma unroll
+    for (int b = 0; b < TN; ++b) f.w[b] = *reinterpret_cast<const gp_f32x4*>(ws + b * 32 * ROW);
+  };
+  auto multiply = [&](const Frags& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+      for (int a = 0; a < TM; ++a) {
+#pragma unroll
+        for (int b = 0; b < TN; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(f.x[a][s], f.w[b][s], acc[a][b], 0, 0, 0);
+      }
     }
   };
-#pragma unroll
-  for (int j = 0; j < GF_AHEAD; ++j) fetch(j, j);  // slices past the end read the last k again and count as zeros
-  stage(0, 0);
+
+  const int range_iters = range_of(k) / BK;
+  int range_end = min(range_iters, iters);
+  Set s0, s1;
+  fetch(s0, 0);
+  fetch(s1, 1);
+  stage(s0, 0, 0);
   __syncthreads();
-  float acc = 0.f;
-  const int slices = (k + GF_BK - 1) / GF_BK;
-  for (int s0 = 0; s0 < slices; s0 += GF_AHEAD) {
+  // Buffer it & 1 holds iteration it, f[0] its first group; `next` holds it + 1 and goes to the other buffer; `free`
+  // takes the loads of it + 2 (past the end: the last iteration's again, never read).  A group's fragments are
+  // read while the one before it is multiplied, the next iteration's first across the barrier: a wavefront that
+  // reaches it has what it reads of this buffer in registers and its part of the other one in LDS.
+  Frags f[2];
+  read(f[0], 0, 0);
+  auto round = [&](int it, Set& next, Set& free) __attribute__((always_inline)) {
+    const int buf = it & 1;
+    fetch(free, it + 2);
+    if (TM * TN > 1) {
+      // Sixteen matrix instructions a group: the staging and the loads are asked for between them, a little behind
+      // each (500 rows of gate|up 1,194 -> 1,154 us); behind four (tiles of 64 x 64) they are faster in one piece
+      // (down at 128 rows 390 us, interleaved 419).
+      stage(next, it + 1, buf ^ 1);
 #pragma unroll
-    for (int j = 0; j < GF_AHEAD; ++j) {
-      const int s = s0 + j;
-      if (s < slices) {  // the same for every thread of the grid
-        const int buf = j & 1;  // GF_AHEAD is even: slice s lies in buffer s & 1 = j & 1
-        fetch(j, s + GF_AHEAD);  // slot j held slice s, which is in LDS already
-        const float* a = xs[buf][out_m];
-        const float* b = ws[buf][out_n];
+      for (int g = 0; g + 1 < GROUPS; ++g) {
+        read(f[(g + 1) & 1], buf, g + 1);
+        multiply(f[g & 1]);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x100, TM + TN, 0);  // DS read
 #pragma unroll
-        for (int kk = 0; kk < GF_BK; ++kk) acc = fmaf(a[kk], b[kk], acc);  // in the order of k
-        // The other buffer was last read in the slice before this one, which every thread has left.
-        stage((j + 1) % GF_AHEAD, buf ^ 1);
-        __syncthreads();
+      for (int i = 0; i < 4 * TM * TN * (GROUPS - 1); ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // VALU
+        __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);  // DS write
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // VMEM read
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
+      }
+    } else {
+#pragma unroll
+      for (int g = 0; g + 1 < GROUPS; ++g) {
+        if (g == GROUPS / 2) stage(next, it + 1, buf ^ 1);
+        read(f[(g + 1) & 1], buf, g + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(f[g & 1]);
+      }
+    }
+    __syncthreads();
+    read(f[GROUPS & 1], buf ^ 1, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(f[(GROUPS - 1) & 1]);
+    if (it + 1 == range_end) {  // the same for every thread
+#pragma unroll
+      for (int a = 0; a < TM; ++a) {
+#pragma unroll
+        for (int b = 0; b < TN; ++b) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sum[a][b][i] += acc[a][b][i], acc[a][b][i] = 0.f;
+        }
+      }
+      range_end = min(range_end + range_iters, iters);
+    }
+  };
+  for (int it = 0; it < iters; it += 2) {
+    round(it, s1, s0);
+    if (it + 1 >= iters) break;
+    round(it + 1, s0, s1);
+  }
+
+  // sum[a][b][i]: activation row 32 (wave_m TM + a) + 8 (i / 4) + 4 half + i % 4, weight row 32 (wave_n TN + b) + r.
+#pragma unroll
+  for (int b = 0; b < TN; ++b) {
+    const int col = n0 + (wave_n * TN + b) * 32 + r;
+    if (col >= n) continue;
+    const float bv = bias ? to_float(bias[col]) : 0.f;
+#pragma unroll
+    for (int a = 0; a < TM; ++a) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int row = m0 + (wave_m * TM + a) * 32 + 8 * (i / 4) + 4 * half + i % 4;
+        if (row < m) y[(size_t)row * y_stride + col] = from_float<TOut>(bias ? sum[a][b][i] + bv : sum[a][b][i]);
       }
     }
   }
-  const int gm = m0 + out_m, gn = n0 + out_n;
-  if (gm < m && gn < n) {
-    if (bias) acc += to_float(bias[gn]);
-    y[(size_t)gm * y_stride + gn] = from_float<TOut>(acc);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Few rows: a workgroup owns 16 MT activation rows by 16 NT weight rows, each of its four wavefronts one range of
+// K; both operands go straight from memory into registers, AHEAD slices of 64 k in flight, without LDS
+// or a barrier before the ranges' sums meet at the end: bound by reading W.
+// Lane (r, g) = (lane % 16, lane / 16) loads 16 bytes of row r: elements 4 g .. 4 g + 3 of every 16, 64 bytes of each of
+// sixteen rows an instruction; four lane swaps (permlane32/16) turn the 4 x 4 of groups and
+// elements round, so that step s of the 16 holds element 4 s + g: the order of k.
+// The loads are plain ones: an instruction takes half a line, and marked non-temporal the other half
+// came from memory again (gate|up at 8 rows 152 us, plain 131; 120 with two weight tiles a wavefront).
+__device__ __forceinline__ void turn_quads(gp_f32x4& v) {
+  float e0 = v[0], e1 = v[1], e2 = v[2], e3 = v[3];
+  auto swap32 = [](float& a, float& b) __attribute__((always_inline)) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(s[0]);
+    b = __uint_as_float(s[1]);
+  };
+  auto swap16 = [](float& a, float& b) __attribute__((always_inline)) {
+    const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(s[0]);
+    b = __uint_as_float(s[1]);
+  };
+  swap32(e0, e2);
+  swap32(e1, e3);
+  swap16(e0, e1);
+  swap16(e2, e3);
+  v = gp_f32x4{e0, e1, e2, e3};
+}
+
+template <int MT, int NT, int AHEAD, bool VEC, typename TIn, typename TOut>
+__global__ void __launch_bounds__(256)
+gemm_plain_few_rows_kernel(TOut* __restrict__ y, const TIn* __restrict__ x, const TIn* __restrict__ w,
+                           const TIn* __restrict__ bias, int m, int n, int k, long x_stride, long y_stride) {
+  constexpr int SLICE = 64, QUADS = SLICE / 16;
+  __shared__ gp_f32x4 parts[3][MT * NT][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the same for the wavefront, and known to be
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  const int range = range_of(k), start = wave * range, end = min(start + range, k);  // this wavefront's k (none: start >= end)
+  const TIn* xbase = x + (size_t)m0 * x_stride;
+  const TIn* wbase = w + (size_t)n0 * k;
+  typedef typename RowOffset<VEC>::type Row;
+  Row xrow[MT], wrow[NT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) xrow[t] = (Row)min(16 * t + r, m - 1 - m0) * (Row)x_stride;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) wrow[t] = (Row)min(16 * t + r, n - 1 - n0) * (Row)k;
+
+  struct Set {
+    Quad<TIn> x[MT][QUADS], w[NT][QUADS];
+  };
+  gp_f32x4 acc[MT][NT];
+#pragma unroll
+  for (int a = 0; a < MT; ++a) {
+#pragma unroll
+    for (int b = 0; b < NT; ++b) acc[a][b] = gp_f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  auto fetch = [&](Set& s, int k0, bool whole) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < QUADS; ++c) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) fetch_quad<VEC>(s.w[t][c], wbase, wrow[t], k0, 16 * c + 4 * g, whole ? 0x7fffffff : k);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) fetch_quad<VEC>(s.x[t][c], xbase, xrow[t], k0, 16 * c + 4 * g, whole ? 0x7fffffff : k);
+    }
+  };
+  auto consume = [&](const Set& s, int left) __attribute__((always_inline)) {  // left: elements of the slice inside the row
+#pragma unroll
+    for (int c = 0; c < QUADS; ++c) {
+      gp_f32x4 xv[MT], wv[NT];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        xv[t] = s.x[t][c].values();
+        if (left < SLICE) clear_past(xv[t], left - 16 * c - 4 * g);
+        turn_quads(xv[t]);
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        wv[t] = s.w[t][c].values();
+        if (left < SLICE) clear_past(wv[t], left - 16 * c - 4 * g);
+        turn_quads(wv[t]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+#pragma unroll
+        for (int a = 0; a < MT; ++a) {
+#pragma unroll
+          for (int b = 0; b < NT; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[a][e], wv[b][e], acc[a][b], 0, 0, 0);
+        }
+      }
+    }
+  };
+
+  const int slices = start < end ? (end - start) / SLICE : 0;  // whole ones
+  if (slices > 0) {
+    Set ring[AHEAD];  // slot j: a slice whose number is j modulo AHEAD
+    const int last = start + (slices - 1) * SLICE;
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) fetch(ring[j], min(start + j * SLICE, last), true);  // past the end: the last slice again
+    int s0 = 0;
+    for (; s0 + AHEAD <= slices; s0 += AHEAD) {
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) {
+        consume(ring[j], SLICE);
+        fetch(ring[j], min(start + (s0 + j + AHEAD) * SLICE, last), true);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+      if (s0 + j < slices) consume(ring[j], SLICE);
+  }
+  if (start + slices * SLICE < end) {  // the rest of a K that is no multiple of 64
+    Set rest;
+    fetch(rest, start + slices * SLICE, false);
+    consume(rest, end - start - slices * SLICE);
+  }
+
+  if (wave > 0) {
+#pragma unroll
+    for (int a = 0; a < MT; ++a) {
+#pragma unroll
+      for (int b = 0; b < NT; ++b) parts[wave - 1][a * NT + b][lane] = acc[a][b];
+    }
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  // acc[a][b][i]: activation row m0 + 16 a + 4 g + i, weight row n0 + 16 b + r.
+#pragma unroll
+  for (int b = 0; b < NT; ++b) {
+    const int col = n0 + 16 * b + r;
+    if (col >= n) continue;
+    const float bv = bias ? to_float(bias[col]) : 0.f;
+#pragma unroll
+    for (int a = 0; a < MT; ++a) {
+      gp_f32x4 sum = gp_f32x4{0.f, 0.f, 0.f, 0.f} + acc[a][b];
+#pragma unroll
+      for (int p = 1; p < 4; ++p)
+        if (p * range < k) sum += parts[p - 1][a * NT + b][lane];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = m0 + 16 * a + 4 * g + i;
+        if (row < m) y[(size_t)row * y_stride + col] = from_float<TOut>(bias ? sum[i] + bv : sum[i]);
+      }
+    }
   }
 }
 
-// Rows up to which the layout for a few rows runs.
-#define GF_MAX_ROWS 32
+inline long ceil_of(long a, long b) { return (a + b - 1) / b; }
+
+// Which layout runs a product: the one whose workgroups are through soonest, one a compute unit at a time.  Microseconds
+// at K = 3,584, measured over q|k|v, o, gate|up and the head of the 7B shape at 1 to 2,048 rows (all grow with K alike):
+// a round of workgroups of 16 x 16 outputs takes 13, of 16 x 32 24, 32 x 16 22, 32 x 32 37 (more weight rows a
+// wavefront read the activations less often, fewer give more workgroups), of 64 x 64 65, of 128 x 128 235, and the
+// first round of some a little more.
+enum PlainKind { FEW_1_1, FEW_1_2, FEW_2_1, FEW_2_2, TILES_64, TILES_128 };
+
+inline PlainKind plain_kind(int m, int n) {
+  static const struct {
+    PlainKind kind;
+    int rows, cols, start, round;
+  } layouts[] = {{FEW_1_1, 16, 16, 3, 13}, {FEW_1_2, 16, 32, 0, 24}, {FEW_2_1, 32, 16, 3, 22},
+                 {FEW_2_2, 32, 32, 0, 37}, {TILES_64, 64, 64, 12, 65}, {TILES_128, 128, 128, 0, 235}};
+  PlainKind best = TILES_128;
+  long least = -1;
+  for (const auto& l : layouts) {
+    const long cost = l.start + l.round * ceil_of(ceil_of(m, l.rows) * ceil_of(n, l.cols), GP_UNITS);
+    if (least < 0 || cost < least) best = l.kind, least = cost;
+  }
+  return best;
+}
+
+template <typename TIn, typename TOut>
+int launch_plain(void* y, const void* x, const void* w, const void* bias, int m, int n, int k, long x_stride,
+                 long y_stride, hipStream_t stream) {
+  const size_t quad = 4 * sizeof(TIn);
+  const bool vec = k % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)x % quad == 0 && (uintptr_t)w % quad == 0 &&
+                   x_stride < (1L << 25) && k < (1 << 25);
+#define TS_PLAIN_ARGS (TOut*)y, (const TIn*)x, (const TIn*)w, (const TIn*)bias, m, n, k, x_stride, y_stride
+#define TS_PLAIN_TILED(T, BK, V)                                                                                      \
+  do {                                                                                                               \
+    const int m_tiles = (int)ceil_of(m, 64 * T), n_tiles = (int)ceil_of(n, 64 * T);                                  \
+    const long ids = ceil_of(n_tiles, GP_DIES) * GP_DIES * m_tiles;                                                  \
+    if (ids > 0x7fffffffL) return TS_ERR_SHAPE;                                                                      \
+    hipLaunchKernelGGL((gemm_plain_kernel<T, T, BK, V, TIn, TOut>), dim3((unsigned)ids), dim3(256), 0, stream,       \
+                       TS_PLAIN_ARGS, m_tiles, n_tiles);                                                             \
+  } while (0)
+#define TS_PLAIN_FEW(MT, NT, AHEAD, V)                                                                                \
+  do {                                                                                                               \
+    dim3 grid((unsigned)ceil_of(n, 16 * NT), (unsigned)ceil_of(m, 16 * MT));                                         \
+    if (grid.y > 65535) return TS_ERR_SHAPE;                                                                         \
+    hipLaunchKernelGGL((gemm_plain_few_rows_kernel<MT, NT, AHEAD, V, TIn, TOut>), grid, dim3(256), 0, stream,        \
+                       TS_PLAIN_ARGS);                                                                               \
+  } while (0)
+  switch (plain_kind(m, n)) {
+    case FEW_1_1:
+      if (vec) TS_PLAIN_FEW(1, 1, 3, true); else TS_PLAIN_FEW(1, 1, 2, false);
+      break;
+    case FEW_1_2:
+      if (vec) TS_PLAIN_FEW(1, 2, 3, true); else TS_PLAIN_FEW(1, 2, 2, false);
+      break;
+    case FEW_2_1:
+      if (vec) TS_PLAIN_FEW(2, 1, 3, true); else TS_PLAIN_FEW(2, 1, 2, false);
+      break;
+    case FEW_2_2:
+      if (vec) TS_PLAIN_FEW(2, 2, 2, true); else TS_PLAIN_FEW(2, 2, 2, false);
+      break;
+    case TILES_64:
+      if (vec) TS_PLAIN_TILED(1, 32, true); else TS_PLAIN_TILED(1, 32, false);
+      break;
+    case TILES_128:
+      if (vec) TS_PLAIN_TILED(2, 16, true); else TS_PLAIN_TILED(2, 16, false);
+      break;
+  }
+#undef TS_PLAIN_FEW
+#undef TS_PLAIN_TILED
+#undef TS_PLAIN_ARGS
+  return ts_launch_status();
+}
+
+}  // namespace
 
 // dtype: type of x, w and bias.  out_f32 != 0: y is float whatever dtype is.
 extern "C" int ts_gemm_plain(void* y, const void* x, const void* w, const void* bias, int m, int n,
@@ -188,34 +485,8 @@ extern "C" int ts_gemm_plain(void* y, const void* x, const void* w, const void* 
                              hipStream_t stream) {
   if (m == 0 || n == 0) return TS_OK;
   if (!y || !x || !w || k < 1 || x_stride < k || y_stride < n) return TS_ERR_ARG;
-  dim3 grid((n + GP_BN - 1) / GP_BN, (m + GP_BM - 1) / GP_BM), block(256);
-  if (grid.y > 65535) return TS_ERR_SHAPE;
-  if (m <= GF_MAX_ROWS) {
-    dim3 few((n + GF_BN - 1) / GF_BN, (m + GF_BM - 1) / GF_BM);
-    const size_t elem = dtype == TS_F32 ? 4 : 2;
-    const bool vec = k % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)x % (4 * elem) == 0 && (uintptr_t)w % (4 * elem) == 0;
-#define TS_FEW_ROWS(V, TI, TO) \
-  hipLaunchKernelGGL((gemm_plain_few_rows_kernel<V, TI, TO>), few, block, 0, stream, (TO*)y, (const TI*)x, (const TI*)w, \
-                     (const TI*)bias, m, n, k, x_stride, y_stride)
-    if (dtype == TS_F32) {
-      if (vec) TS_FEW_ROWS(true, float, float); else TS_FEW_ROWS(false, float, float);
-    } else if (dtype == TS_BF16 && out_f32) {
-      if (vec) TS_FEW_ROWS(true, bf16_t, float); else TS_FEW_ROWS(false, bf16_t, float);
-    } else if (dtype == TS_BF16) {
-      if (vec) TS_FEW_ROWS(true, bf16_t, bf16_t); else TS_FEW_ROWS(false, bf16_t, bf16_t);
-    } else {
-      return TS_ERR_DTYPE;
-    }
-#undef TS_FEW_ROWS
-    return ts_launch_status();
-  }
-  if (dtype == TS_F32)
-    hipLaunchKernelGGL((gemm_plain_kernel<float, float>), grid, block, 0, stream, (float*)y, (const float*)x, (const float*)w, (const float*)bias, m, n, k, x_stride, y_stride);
-  else if (dtype == TS_BF16 && out_f32)
-    hipLaunchKernelGGL((gemm_plain_kernel<bf16_t, float>), grid, block, 0, stream, (float*)y, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, m, n, k, x_stride, y_stride);
-  else if (dtype == TS_BF16)
-    hipLaunchKernelGGL((gemm_plain_kernel<bf16_t, bf16_t>), grid, block, 0, stream, (bf16_t*)y, (const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, m, n, k, x_stride, y_stride);
-  else
-    return TS_ERR_DTYPE;
-  return ts_launch_status();
+  if (dtype == TS_F32) return launch_plain<float, float>(y, x, w, bias, m, n, k, x_stride, y_stride, stream);
+  if (dtype != TS_BF16) return TS_ERR_DTYPE;
+  if (out_f32) return launch_plain<bf16_t, float>(y, x, w, bias, m, n, k, x_stride, y_stride, stream);
+  return launch_plain<bf16_t, bf16_t>(y, x, w, bias, m, n, k, x_stride, y_stride, stream);
 }
