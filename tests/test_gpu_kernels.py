@@ -642,6 +642,78 @@ def test_attention_generic(ops, dtype, heads, kv_heads, dim, page, window):
     torch.testing.assert_close(got, case.expected, **tol(dtype))
 
 
+FLOAT32_RULES = {
+    "causal": {},
+    "window": {"window": 20},
+    "window 70, first keys": {"window": 70, "keep_first": 5},
+    "chunks, sinks": {"chunk": 48, "sinks": 2.0, "sink_scores": True},
+    "slopes, cap": {"slopes": True, "softcap": 3.0},
+    "bias, window": {"distance_bias": 30, "window": 64, "out_scale": 0.5},
+}
+
+
+@pytest.mark.parametrize("rule", FLOAT32_RULES)
+@pytest.mark.parametrize("heads,kv_heads,dim,page", [g for g in ATTENTION_GEOMETRIES if g[3] >= 16])
+def test_attention_float32(ops, monkeypatch, heads, kv_heads, dim, page, rule):
+    """The 32-bit attention on the matrix cores against the generic kernel, for contexts at the edges of its tiles of
+    64 keys and blocks of 16, blocks of 16 rows that hold several requests' tokens, and every rule; a token's bits are the
+    same in a block of its request's tokens, among others', alone with its tiles side by side and alone with its
+    tiles folded by one wavefront."""
+    rule = dict(FLOAT32_RULES[rule])
+    window = rule.pop("window", None)
+    seqs = [(70, 37), (33, 33), (90, 7), (1, 1), (129, 2), (64, 3), (65, 1), (200, 1), (128, 1), (17, 1)]
+    case = PagedCase(torch.float32, heads, kv_heads, dim, page, seqs, None, seed=dim)
+    g = torch.Generator().manual_seed(heads)
+    more = {name: (torch.rand(heads, generator=g) * 0.3).to(DEV) for name in ("slopes", "sink_scores") if rule.pop(name, None)}
+    if "distance_bias" in rule:
+        more["distance_bias"] = torch.randn(heads, rule.pop("distance_bias"), generator=g).to(DEV)
+    more.update(rule)
+    pages = (case.dev(case.kp), case.dev(case.vp), case.dev(case.table))
+    q = case.dev(case.q)
+
+    def run(tokens, single):
+        at = torch.tensor(tokens, device=DEV)
+        args = (q[at].contiguous(), heads * dim, *pages, case.ints(case.token_seq)[at].contiguous(), case.ints(case.positions)[at].contiguous(),
+                heads, dim ** -0.5, window)
+        if single is None:
+            return ops.paged_attention_generic(*args, **more)
+        assert ops.float32_attention_supported(args[0], args[1], args[2], args[3])
+        return ops.attention_float32(*args, num_single=single, max_single_context=200, **more)
+
+    every = list(range(case.qsl[-1]))
+    whole = run(every, 0)
+    torch.testing.assert_close(whole, run(every, None), **tol(torch.float32))
+    assert torch.equal(run(every, 5)[-5:], whole[-5:])  # requests of one token, tile by tile
+    picked = [3, 36, 37, 69, 76, 77, 79, 82]  # tokens of several requests in one block of rows
+    assert torch.equal(run(picked, 0), whole[picked])
+    alone = [0, 20, 36, 60, 75, 78, 80, 84]
+    assert torch.equal(run(alone, len(alone)), whole[alone])
+    monkeypatch.setattr(ops, "float32_attention_scratch", 0)
+    assert torch.equal(run(alone, len(alone)), whole[alone])
+
+
+def test_attention_float32_keeps_values_apart(ops):
+    """A value that is no finite number reaches the rows that see its key and no other: a token's own, in the middle of a
+    block of rows; and what lies in a page behind a request's last token reaches nobody."""
+    heads, kv_heads, dim, page, seqs = 6, 2, 64, 16, [(70, 40), (21, 21), (150, 1)]
+    case = PagedCase(torch.float32, heads, kv_heads, dim, page, seqs, None, seed=5)
+    run = lambda: ops.attention_float32(
+        case.dev(case.q), heads * dim, case.dev(case.kp), case.dev(case.vp), case.dev(case.table), case.ints(case.token_seq),
+        case.ints(case.positions), heads, dim ** -0.5, None, num_single=1, max_single_context=150)
+    clean = run()
+    for s, (ctx, _) in enumerate(seqs):  # behind every request's last token
+        if ctx % page:
+            case.kp[case.table[s, ctx // page], :, ctx % page:] = float("nan")
+            case.vp[case.table[s, ctx // page], :, :, ctx % page:] = float("inf")
+    assert torch.equal(run(), clean)
+    case.vp[case.table[0, 55 // page], :, :, 55 % page] = float("inf")  # the value of request 0's token 55, row 25 of the step
+    case.vp[case.table[1, 7 // page], :, :, 7 % page] = float("nan")
+    got = run()
+    hit = torch.tensor([(s == 0 and p >= 55) or (s == 1 and p >= 7) for s, p in zip(case.token_seq, case.positions)], device=DEV)
+    assert torch.equal(got[~hit], clean[~hit])
+    assert not bool(torch.isfinite(got[hit]).any())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("window", [None, 20])
 def test_attention_generic_with_a_bias_by_distance(ops, dtype, window):

@@ -44,6 +44,7 @@ MODULES: dict[str, tuple[str, ...]] = {
         "bigram.hip",
         "moe.hip",
         "attention_generic.hip",
+        "attention_f32.hip",
         "attention_tiles.hip",
         "gemm_plain.hip",
         "gemm_skinny.hip",

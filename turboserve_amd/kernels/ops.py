@@ -72,6 +72,9 @@ _SIGNATURES: dict[str, dict[str, list]] = {
                                        c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                                        c_float, c_float, c_int, c_void_p, c_int, c_float, c_void_p, c_void_p, c_int, c_int, c_int,
                                        c_long, c_float, c_void_p],
+        "ts_attention_f32": [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
+                             *[c_int] * 6, c_float, c_float, c_int, c_void_p, c_int, c_float, c_void_p, c_void_p, c_int, c_int,
+                             c_long, c_float, c_int, c_void_p, c_void_p, c_int, c_void_p],
         "ts_attention_tiles": [c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
                                c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_int,
                                c_int, c_float, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_long, c_float, c_void_p],
@@ -1596,6 +1599,77 @@ class Ops:
             int(chunk or 0), float(sinks), _ptr(sink_scores), _ptr(distance_bias),
             0 if distance_bias is None else distance_bias.shape[1], int(keep_first), dtype_code(q.dtype), out_stride, float(out_scale),
             self.stream()), "ts_paged_attention_generic")
+        return result
+
+    #: Head sizes of the 32-bit attention on the matrix cores (``csrc/attention_f32.hip``).
+    float32_attention_dims = (16, 32, 48, 64, 80, 96, 128, 256)
+    #: Bytes that single tokens' tiles may take side by side; above it a wavefront folds all tiles of its token
+    #: itself, with the same bits (a tile of 64 keys leaves 130 floats a head at a head size of 128, 6% of its keys and values).
+    float32_attention_scratch = 256 << 20
+
+    def float32_attention_supported(self, q: torch.Tensor, q_stride: int, k_pages: torch.Tensor, v_pages: torch.Tensor | None,
+                                    out: tuple[torch.Tensor, int] | None = None) -> bool:
+        """Whether :meth:`attention_float32` takes this layer: 32-bit, a head size it is built for, values as
+        wide in pages of their own, pages of 16 keys or more, rows that 16-byte accesses fit.  All of it is
+        the layer's and the cache's geometry, never the step's, so a request's steps agree."""
+        if q.dtype != torch.float32 or v_pages is None or k_pages.dtype != torch.float32 or v_pages.dtype != torch.float32:
+            return False
+        block_size, head_dim = k_pages.shape[2], k_pages.shape[3]
+        placed = out is None or (out[0].stride(0) % 4 == 0 and (out[0].data_ptr() + 4 * out[1]) % 16 == 0)
+        return (head_dim in self.float32_attention_dims and v_pages.shape[2] == head_dim and block_size >= 16
+                and q_stride % 4 == 0 and q.data_ptr() % 16 == 0 and placed)
+
+    def attention_float32(
+        self, q: torch.Tensor, q_stride: int, k_pages: torch.Tensor, v_pages: torch.Tensor, block_table: torch.Tensor,
+        token_seq: torch.Tensor, positions: torch.Tensor, heads: int, scale: float, window: int | None,
+        slopes: torch.Tensor | None = None, softcap: float = 0.0, *, num_single: int, max_single_context: int,
+        chunk: int | None = None, sinks: float = 0.0, sink_scores: torch.Tensor | None = None,
+        distance_bias: torch.Tensor | None = None, keep_first: int = 0, out_scale: float = 1.0,
+        out: tuple[torch.Tensor, int] | None = None,
+    ) -> torch.Tensor:
+        """What :meth:`paged_attention_generic` computes, in 32-bit throughout, on the matrix cores' 32-bit
+        instructions (:meth:`float32_attention_supported` says for which layers).  The last ``num_single`` tokens of the
+        step are one request's each, holding ``max_single_context`` tokens at most; those before them
+        may be any.  A token's result does not depend on which of the two it is among: its keys are taken in tiles of 64,
+        folded in order, by one wavefront for 16 tokens of a head, or, for single tokens, tile by tile side by side."""
+        _gpu(q, k_pages, v_pages, block_table, token_seq, positions)
+        self._score_tables(heads, sinks, sink_scores, distance_bias)
+        if slopes is not None:
+            _gpu(slopes)
+            _need(slopes.dtype == torch.float32 and slopes.is_contiguous() and slopes.numel() == heads,
+                  "slopes must be contiguous float32 [heads]")
+        for name, ints in (("block_table", block_table), ("token_seq", token_seq), ("positions", positions)):
+            _i32(ints, name)
+        _check_pages(k_pages, v_pages, q.dtype)
+        _need(self.float32_attention_supported(q, q_stride, k_pages, v_pages, out), "a geometry the 32-bit attention does not take")
+        _, kv_heads, block_size, head_dim = k_pages.shape
+        tokens = positions.numel()
+        _need((chunk is None or chunk >= 1) and sinks >= 0.0, "a chunk is at least one position, sinks are not negative")
+        _need(q.is_contiguous() and q.numel() >= tokens * q_stride and q_stride >= heads * head_dim, "q does not hold [T, q_stride] rows")
+        _need(block_table.dim() == 2 and token_seq.numel() == tokens, "block_table [S, MB], token_seq [T]")
+        _need(1 <= kv_heads and heads % kv_heads == 0 and heads <= 65535, f"{heads} query heads on {kv_heads} KV heads")
+        _need(0 <= num_single <= tokens and (num_single == 0 or max_single_context >= 1), "single tokens are the step's last")
+        result, pointer, out_stride = self._columns_of(out, tokens, heads * head_dim, q.dtype, q.device)
+
+        def launch(first: int, count: int, mode: int, partial=None, ml=None, max_tiles: int = 0) -> None:
+            _check(self.core.ts_attention_f32(
+                pointer, _ptr(q), q_stride, _ptr(k_pages), _ptr(v_pages), _ptr(block_table), block_table.shape[1], _ptr(token_seq),
+                _ptr(positions), first, count, heads, kv_heads, head_dim, block_size, float(scale), float(softcap), int(window or 0),
+                _ptr(slopes), int(chunk or 0), float(sinks), _ptr(sink_scores), _ptr(distance_bias),
+                0 if distance_bias is None else distance_bias.shape[1], int(keep_first), out_stride, float(out_scale), mode,
+                _ptr(partial), _ptr(ml), max_tiles, self.stream()), "ts_attention_f32")
+
+        launch(0, tokens - num_single, 0)
+        if num_single > 0:
+            seen = min(max_single_context, window or max_single_context, chunk or max_single_context)
+            max_tiles = min(-(-max_single_context // 64), -(-seen // 64) + 1 + -(-keep_first // 64))
+            slots = num_single * heads * max_tiles
+            if 4 * slots * (head_dim + 2) <= self.float32_attention_scratch:
+                partial = torch.empty(slots * head_dim, dtype=torch.float32, device=q.device)
+                ml = torch.empty(slots * 2, dtype=torch.float32, device=q.device)
+                launch(tokens - num_single, num_single, 2, partial, ml, max_tiles)
+            else:
+                launch(tokens - num_single, num_single, 1)
         return result
 
     @staticmethod

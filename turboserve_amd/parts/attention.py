@@ -346,8 +346,8 @@ class GroupedQueryAttention(Mixer):
         bfloat16 runs use the matrix-core kernels where the geometry allows: one launch for the
         multi-token requests at the front of the batch, one for the single-token requests
         behind them; a position encoding that biases the scores, a chunk mask, sinks or values of
-        another width than the keys go through the tiled matrix-core kernel that takes them; every
-        32-bit run and any other geometry goes through the generic kernel."""
+        another width than the keys go through the tiled matrix-core kernel that takes them.  32-bit
+        runs use the 32-bit kernel where the geometry allows; any other goes through the generic kernel."""
         ops = self.runtime.ops
         table = ctx.block_tables[cache.group]
         slopes = self.position.score_slopes(self.num_heads)
@@ -380,8 +380,13 @@ class GroupedQueryAttention(Mixer):
             return tiled_attention(ops, qkv, q_stride, cache.k, cache.v, table, ctx, heads=self.num_heads, scale=self.scale,
                                    window=self.window, chunk=self.chunk, sinks=self.sinks, slopes=slopes, softcap=self.softcap,
                                    sink_scores=self.sink_scores, distance_bias=bias, keep_first=self.keep_first, out_scale=scale, out=out)
+        rule = dict(chunk=self.chunk, sinks=self.sinks, sink_scores=self.sink_scores, distance_bias=bias, keep_first=self.keep_first,
+                    out_scale=scale, out=out)
+        if ops.float32_attention_supported(qkv, q_stride, cache.k, cache.v, out):
+            return ops.attention_float32(
+                qkv, q_stride, cache.k, cache.v, table, ctx.token_seq, ctx.positions, self.num_heads, self.scale, self.window, slopes,
+                self.softcap, num_single=ctx.num_decode_seqs,
+                max_single_context=min(ctx.max_decode_context_len, table.shape[1] * cache.block_size), **rule)
         return ops.paged_attention_generic(
             qkv, q_stride, cache.k, cache.v, table, ctx.token_seq, ctx.positions,
-            self.num_heads, self.scale, self.window, slopes, self.softcap, chunk=self.chunk, sinks=self.sinks,
-            sink_scores=self.sink_scores, distance_bias=bias, keep_first=self.keep_first, out_scale=scale, out=out,
-        )
+            self.num_heads, self.scale, self.window, slopes, self.softcap, **rule)
