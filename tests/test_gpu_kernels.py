@@ -345,6 +345,71 @@ def test_gemm_wide_rows_do_not_depend_on_the_batch_and_plans_fill_the_device(ops
     torch.testing.assert_close(ops.dense(sums, torch.bfloat16).float(), x[:200].float() @ w.float().t(), rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("tn,tm", [(8, 8), (8, 6), (8, 5), (5, 10), (5, 8), (4, 8), (4, 5), (4, 4)])
+@pytest.mark.parametrize("m,n,k,splits", [(1, 16, 64, 1), (129, 272, 64, 1), (257, 48, 128, 2), (321, 528, 192, 3), (700, 1040, 448, 2)])
+def test_gemm_block_every_tile(ops, tn, tm, m, n, k, splits):
+    """Blocks of the largest product, one tile short and one over in both directions, ranges of K
+    of one to seven iterations, rows of x apart, a bias, the three results and rules of the gated unit; against
+    the exact product and the kernel that takes any K and N.  Bounds: k + 1 roundings of 2^-24 of
+    the terms' sizes for the sums, half a unit of bfloat16 (2^-8) more for a rounded result, and for the
+    gated one what the unit makes of its operands' bounds (its slope in the gate stays below 1.2 for these rules)."""
+    from turboserve_amd.kernels.ops import GELU_TANH_RULE
+
+    g = torch.Generator().manual_seed(100 * tn + tm + m)
+    x = torch.randn(m, k + 8, generator=g).bfloat16()[:, :k]
+    w = (torch.randn(n, k, generator=g) * 0.3).bfloat16()
+    b = torch.randn(n, generator=g).bfloat16()
+    want = x.double() @ w.double().T + b.double()
+    bound = (k + 1) * 2.0**-24 * (x.double().abs() @ w.double().abs().T + b.double().abs())
+    xd, wd, bd = torch.empty(m, k + 8, dtype=torch.bfloat16, device=DEV)[:, :k].copy_(x), w.to(DEV), b.to(DEV)
+    iters = k // 64
+    per_split = -(-iters // splits)
+    partial = ops.gemm_block(xd, wd, bd, plan=(per_split, splits, tn, tm), sums=True)
+    assert partial.shape == (splits, m, n) and partial.dtype == torch.float32
+    assert bool(((partial.double().sum(0).cpu() - want).abs() <= bound).all())
+    one = ops.gemm_block(xd, wd, bd, plan=(iters, 1, tn, tm))
+    general = ops.gemm_wide(xd, wd, bd, plan=(iters, 1, 4, 128, 8))
+    assert one.shape == general.shape and one.dtype == general.dtype
+    assert bool(((one.double().cpu() - want).abs() <= 2.0**-8 * want.abs() + bound).all())
+    assert bool(((one.double() - general.double()).cpu().abs() <= 2.0**-7 * want.abs() + 2 * bound).all())
+    gate, up = want[:, 0::2], want[:, 1::2]
+    for rule in ((1.0, 0.0, 0.0), (1.702, 7.0, 1.0), GELU_TANH_RULE):
+        steepness, limit, shift = rule[:3]
+        cubic = rule[3] if len(rule) > 3 else 0.0
+        a, u = (gate.clamp(max=limit), up.clamp(-limit, limit)) if limit > 0 else (gate, up)
+        unit = a * torch.sigmoid(steepness * (a + cubic * a**3))
+        exact = unit * (u + shift)
+        slack = 2.0**-8 * exact.abs() + 1.2 * (bound[:, 0::2] + 2.0**-20 * a.abs()) * (u + shift).abs() + unit.abs() * bound[:, 1::2] + 1e-30
+        fused = ops.gemm_block(xd, wd, bd, plan=(iters, 1, tn, tm), gated=True, rule=rule)
+        assert fused.shape == (m, n // 2) and bool(((fused.double().cpu() - exact).abs() <= slack).all()), rule
+    # a row does not depend on the rows beside it, nor a result on what stood in its memory
+    assert torch.equal(ops.gemm_block(xd[m // 2:], wd, bd, plan=(iters, 1, tn, tm)), one[m // 2:])
+
+
+@pytest.mark.parametrize("m,n,k,offset", [(129, 16, 64, 0), (300, 2064, 1088, 0), (200, 500, 264, 0), (200, 512, 264, 0), (200, 520, 256, 0),
+                                          (200, 512, 256, 4), (150, 256, 192, 0)])
+def test_products_of_many_rows_agree_whichever_kernel_takes_them(ops, m, n, k, offset):
+    """The block product runs what it takes (K % 64, N % 16, 16-byte rows) and the wide one the rest;
+    a plan's grid covers K; all three results are the product's."""
+    g = torch.Generator().manual_seed(m + n)
+    flat = torch.randn(m * k + 8, generator=g).bfloat16().to(DEV)
+    x = flat[offset:offset + m * k].view(m, k)
+    w = (torch.randn(n, k, generator=g) / k**0.5).bfloat16().to(DEV)
+    takes = k % 64 == 0 and n % 16 == 0 and offset % 8 == 0
+    assert ops.block_supported(x, w) == takes
+    if takes:
+        for kind in ("sums", "one", "gated"):
+            per_split, splits, tn, tm = ops._block_plan(m, n, k, kind)
+            assert splits == -(-(k // 64) // per_split) and (kind == "sums" or splits == 1)
+    want = x.double() @ w.double().T
+    bound = 2.0**-7 * want.abs() + (k + 1) * 2.0**-24 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((ops.linear(x, w).double() - want).abs() <= bound).all())
+    sums = ops.linear(x, w, for_residual=True)
+    assert bool(((ops.dense(sums, torch.bfloat16).double() - want).abs() <= bound).all())
+    gated = torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2]
+    assert float((ops.linear_swiglu(x, w).double() - gated).abs().max()) <= 2.0**-6 * float(gated.abs().max())
+
+
 def test_library_product_at_a_larger_size_ignores_the_rows_behind(ops, monkeypatch):
     """With sizes set for the library's products, a step's activations are allocated up to the
     next size and the product runs that long; the rows behind the step's own (not-a-numbers

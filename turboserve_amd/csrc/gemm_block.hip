@@ -1,0 +1,394 @@
+// The product of a prompt's step (more rows than a decode step has), in blocks as large as a wavefront's
+// registers take:
+//   Y[m][n] = sum over k of X[m][k] * W[n][k]  (+ bias[n])
+// bfloat16 activations X [M, K] and weights W [N, K] as the checkpoint stores them (F.linear's
+// layout, src/turboserve/engine/model/layers.py:142), 32-bit accumulation on the matrix cores.
+//
+// A workgroup of four wavefronts (2 x 2), one per SIMD, owns NT = 32 TN weight rows by XR = 32 TM activation rows
+// and one range of K, a wavefront TN x TM tiles of v_mfma_f32_16x16x32_bf16: up to 256 registers of sums.  What
+// bounds such a product beside the matrix cores is LDS.  Measured on a compute unit: reads of 16 bytes a lane 210 bytes a
+// cycle (a wavefront alone 30), writes from registers 30 whatever their width, global memory straight to LDS
+// 58.  A block of 256 x 256 reads 128 KB and writes 64 KB per 64 of K, in which its matrix instructions take 2,048
+// cycles: written from registers the 64 KB alone are 2,186, so operands go from global memory straight to LDS
+// (buffer loads with an LDS destination), into rings of three iterations' weight rows and two or three iterations'
+// activation rows, and 64 of K deep because a row of less than a 128-byte line is fetched twice (32 deep: 1.74 against
+// 0.85 ms at 8,192 x 8,192 x 8,192).
+// With one wavefront on a SIMD nothing hides its waits, so nothing waits: a step's activation fragments are
+// read from LDS during the step before it, its weight fragments a tile's instructions after the last use of
+// their registers, and the first ones of the next iteration behind the barrier that ends this one's reads,
+// while most of its second step is still to be multiplied; loads are issued two iterations ahead, one beside each tile's
+// instructions (issued in one go they held the matrix instructions up).
+// Measured, microseconds, against the better of gemm_wide and the library's default kernel (with the kernel that reads or
+// makes the result: SwiGLU, or the norm that takes the partial sums), at 299 / 509 / 2,048 rows: gate|up [37888, 3584] 81 / 124 /
+// 429 against 126 / 158 / 560 (1.3 PFLOP/s), down [3584, 18944] 58 / 79 / 246 against 111 / 90 / 291, o [3584, 3584] 26 / 30 / 73
+// against 35 / 34 / 77, q|k|v [4608, 3584] 27 / 28 / 59 against 23 / 31 / 62.  An iteration of 256 x 256 takes 1.15 us where
+// half the compute units have a workgroup and 1.4 where all do (the matrix instructions 0.85 at the full clock); a
+// workgroup's start takes 2 us and its stores 4.
+#include "common.hpp"
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int BLOCK_DIES = 8;
+constexpr int BLOCK_DEPTH = 64;  // k per iteration: rows of 128 bytes, eight 16-byte pieces
+
+// Raw buffer of `bytes` bytes (below 2 GB): loads beyond its end bring zeros, stores there are dropped.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t block_buffer(const void* at, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(at), 0, (int)bytes, 0x00027000);
+}
+
+__device__ __forceinline__ bf16x8 block_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
+
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+// Two values rounded to nearest even as bfloat16, one instruction.
+__device__ __forceinline__ uint32_t block_pack(float lo, float hi) {
+  uint32_t both;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(both) : "v"(lo), "v"(hi));
+  return both;
+}
+
+// gated_unit (common.hpp) with the hardware's 2^x and reciprocal (both within an ulp), short enough to stand in the stores of
+// every tile.  PLAIN: a rule without limit and cubic.
+template <bool PLAIN>
+__device__ __forceinline__ float block_unit(float g, float u, GluRule rule) {
+  if (!PLAIN && rule.limit > 0.f) {
+    g = fminf(g, rule.limit);
+    u = fminf(fmaxf(u, -rule.limit), rule.limit);
+  }
+  const float inner = !PLAIN && rule.cubic != 0.f ? fmaf(rule.cubic * g * g, g, g) : g;
+  const float e = __builtin_amdgcn_exp2f(inner * (rule.steepness * -1.44269504088896340736f));
+  return g * __builtin_amdgcn_rcpf(1.f + e) * (u + rule.up_shift);
+}
+
+// The two outputs that a lane holds of a tile, whose rows alternate gate, up.
+template <bool PLAIN>
+__device__ __forceinline__ uint32_t block_units(f32x4 v, GluRule rule) {
+  return block_pack(block_unit<PLAIN>(v[0], v[1], rule), block_unit<PLAIN>(v[2], v[3], rule));
+}
+
+// Odd rows of sixteen lanes of a against even rows of b; the upper 32 lanes of a against the lower 32 of b.
+__device__ __forceinline__ u32x2 block_swap16(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(a, b, false, false));
+}
+__device__ __forceinline__ u32x2 block_swap32(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(a, b, false, false));
+}
+
+// At most `LEFT` of this wavefront's loads still on their way, all of its LDS reads done, then the workgroup's barrier.  (A
+// bare barrier: the fence of __syncthreads would wait for every load.)
+template <int LEFT>
+__device__ __forceinline__ void block_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LEFT) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// LDS holds three iterations' weight rows and two or, where they fit, three iterations' activation rows (1,280 rows of 128
+// bytes in all).  LEFT: loads that may be on their way when the next iteration must have landed.
+template <int TN, int TM>
+struct BlockRing {
+  static constexpr int ROWS = 160 * 1024 / (BLOCK_DEPTH * 2);
+  static constexpr int W = 3, X = 32 * 3 * (TN + TM) <= ROWS ? 3 : 2;
+  static constexpr int LEFT = TN + (X - 2) * TM;
+  static constexpr size_t BYTES = (size_t)32 * (W * TN + X * TM) * BLOCK_DEPTH * 2;
+  static_assert(BYTES <= 160 * 1024, "the rings must fit the LDS of a compute unit");
+};
+
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+
+// The body, with two names for the workgroup's LDS: `to` for the loads that write it, `from` for the reads.  __restrict__
+// tells the compiler that they are not the same memory; otherwise it would wait for every load in flight before
+// every read.  What orders them is block_wait, which no access crosses.
+// out: bfloat16 [m, n] (mode 0), partial: float [splits, m, n] (mode 1), out: bfloat16 [m, n / 2] (mode 2; 3: any rule
+// of the gated unit.  Two kernels: with both epilogues behind one loop the compiler moved the sums between registers in it).
+template <int TN, int TM, int MODE>
+__device__ __forceinline__ void
+gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __restrict__ partial, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, long x_stride,
+                  const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int m, int n, int k,
+                  int iters_per_split, int splits, int n_tiles, int m_tiles, GluRule rule) {
+  constexpr int NT = 32 * TN, XR = 32 * TM, ROW = BLOCK_DEPTH;
+  typedef BlockRing<TN, TM> Ring;
+  constexpr int RW = Ring::W, RX = Ring::X;
+  // Workgroup id -> weight tile x range of K (`unit`) and tile of activation rows: ids go to the eight dies in turn; a die
+  // takes an eighth of the workgroups, the activation tiles over one unit one after the other, and shares the unit's
+  // weights in its L2.
+  const int mine = (n_tiles * splits * m_tiles + BLOCK_DIES - 1) / BLOCK_DIES;
+  const int turn = blockIdx.x / BLOCK_DIES, place = blockIdx.x % BLOCK_DIES * mine + turn;
+  const int unit = place / m_tiles;
+  if (unit >= n_tiles * splits) return;  // the whole workgroup leaves together
+  const int m_base = place % m_tiles * XR, n_base = unit % n_tiles * NT, split = unit / n_tiles;
+  const int total = k / BLOCK_DEPTH;
+  const int first = split * iters_per_split, last = min(first + iters_per_split, total);  // exclusive
+  if (first >= last) return;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane16 = lane & 15, group = lane >> 4;
+  const int wave_n = wave >> 1, wave_m = wave & 1;
+
+  // A load moves 1 KB, eight rows of 128 bytes: lane l the 16 bytes that lie at position l % 8 of row l / 8 in LDS, which is
+  // piece (l % 8) ^ key of that row, key = (row / 2) % 8: reads of one piece of sixteen consecutive rows touch every bank
+  // once.  Wavefront v takes the eights v, v + 4, ... of the weight rows and of the activation rows (so a lane's key is
+  // the same for all of them).  Loads beyond a buffer's end (rows beyond N or M, whose results are not stored) bring zeros.
+  const int row0 = 8 * wave + (lane >> 3), piece = (lane & 7) ^ ((row0 >> 1) & 7);
+  const __amdgpu_buffer_rsrc_t wbuf = block_buffer(w + (size_t)n_base * k, ((size_t)(min(n - n_base, NT) - 1) * k + k) * 2);
+  const __amdgpu_buffer_rsrc_t xbuf = block_buffer(x + (size_t)m_base * x_stride, ((size_t)(min(m - m_base, XR) - 1) * x_stride + k) * 2);
+  // A row's place is in the lane's offset, the place in K in the wavefront's: what is compared with the buffer's size is
+  // the first against the size less the second, which is never below 0.
+  int woff = (row0 * k + 8 * piece) * 2, xoff = (row0 * (int)x_stride + 8 * piece) * 2;
+  auto load_w = [&](int j, int it, int slot) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, to + (slot * NT + 32 * j + 8 * wave) * ROW, 16, woff + j * 64 * k, it * (BLOCK_DEPTH * 2), 0, 0);
+  };
+  auto load_x = [&](int j, int it, int slot) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, to + (RW * NT + slot * XR + 32 * j + 8 * wave) * ROW, 16, xoff + j * 64 * (int)x_stride, it * (BLOCK_DEPTH * 2),
+                                             0, 0);
+  };
+
+  // This lane's piece of step s (32 of K) in every row it reads.
+  const int key = (lane16 >> 1) & 7;
+  const lds_u16* const from_w = from + (wave_n * TN * 16 + lane16) * ROW;
+  const lds_u16* const from_x = from + (RW * NT + wave_m * TM * 16 + lane16) * ROW;
+  const int piece_at[2] = {8 * (group ^ key), 8 * ((4 + group) ^ key)};
+  auto read_w = [&](int slot, int s, int a) __attribute__((always_inline)) {
+    return *(const lds_u32x4*)(from_w + (slot * NT + a * 16) * ROW + piece_at[s]);
+  };
+  auto read_x = [&](int slot, int s, int b) __attribute__((always_inline)) {
+    return *(const lds_u32x4*)(from_x + (slot * XR + b * 16) * ROW + piece_at[s]);
+  };
+
+  // acc[a][b][i] = sum for weight row col0 + 16 a + i and activation row m_base + 16 (wave_m TM + b) + lane16; it starts from
+  // the bias (N is a multiple of 16; the last workgroup's tiles beyond N are never stored).
+  const int col0 = n_base + wave_n * TN * 16 + 4 * group;
+  f32x4 acc[TN][TM];
+#pragma unroll
+  for (int a = 0; a < TN; ++a) {
+    f32x4 start = {0.f, 0.f, 0.f, 0.f};
+    if (bias && split == 0) {
+      const u32x2 four = *(const u32x2*)(bias + min(col0 + 16 * a, n - 4));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) start[i] = __builtin_bit_cast(float, i & 1 ? four[i / 2] & 0xffff0000u : four[i / 2] << 16);
+    }
+#pragma unroll
+    for (int b = 0; b < TM; ++b) acc[a][b] = start;
+  }
+  u32x4 xf[2][TM], wf[TN];
+  auto tile = [&](int s, int a, int from, int end) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = from; b < end; ++b)
+      acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(block_bf16x8(wf[a]), block_bf16x8(xf[s][b]), acc[a][b], 0, 0, 0);
+  };
+
+  // Iteration i of the range: its weight rows lie in slot i % RW of their ring, its activation rows in slot i % RX of theirs.
+  const int count = last - first;
+  auto step = [&](int i) __attribute__((always_inline)) { return first + min(i, count - 1); };  // past the end: the last one again, never read
+#pragma unroll
+  for (int s = 0; s < RX; ++s) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      if (s < 2) load_w(j, step(s), s);
+#pragma unroll
+    for (int j = 0; j < TM; ++j) load_x(j, step(s), s);
+  }
+  block_wait<TN + (RX - 1) * TM>();
+#pragma unroll
+  for (int b = 0; b < TM; ++b) xf[0][b] = read_x(0, 0, b);
+#pragma unroll
+  for (int a = 0; a < TN; ++a) wf[a] = read_w(0, 0, a);
+
+  // Top of a round: slots ws and xs hold iteration `it` complete, xf[0] and wf its step 0; the loads of the iterations
+  // behind it are on their way.  The order below is the one that is issued: a few accesses, then matrix
+  // instructions, which run while the next accesses issue.
+#define TS_PIN __builtin_amdgcn_sched_barrier(0)
+  constexpr int EARLY = TN / 2;                     // tiles of step 0 beside which step 1's activations are read
+  constexpr int FREE = TN > 4 ? 2 : 1;              // the barrier stands before this tile of step 1
+  constexpr int BEHIND = TM + FREE;                 // fragments of the next iteration read behind it, with those of each tile done
+  int ws = 0, xs = 0;
+  for (int it = 0; it < count; ++it) {
+    // The offsets of the other rows are added up in each iteration: kept, they would take registers that the sums need.
+    asm volatile("" : "+v"(woff), "+v"(xoff));
+    const int next_w = step(it + 2), next_x = step(it + RX);
+    const int free_w = ws == 0 ? 2 : ws - 1, free_x = xs;
+#pragma unroll
+    for (int a = 0; a < TN; ++a) {
+      TS_PIN;
+      load_w(a, next_w, free_w);
+      TS_PIN;
+      tile(0, a, 0, TM / 2);
+      TS_PIN;
+#pragma unroll
+      for (int b = a * TM / EARLY; b < (a + 1) * TM / EARLY && b < TM; ++b) xf[1][b] = read_x(xs, 1, b);
+      TS_PIN;
+      tile(0, a, TM / 2, TM);
+      TS_PIN;
+      wf[a] = read_w(ws, 1, a);
+    }
+#pragma unroll
+    for (int a = 0; a < TN; ++a) {
+      TS_PIN;
+      if (a == FREE) {
+        // This wavefront has read all of iteration `it` (its fragments are in registers) and its loads of it + 1 have landed;
+        // behind the barrier both hold for the workgroup.
+        block_wait<Ring::LEFT>();
+        ws = ws + 1 == RW ? 0 : ws + 1;
+        xs = xs + 1 == RX ? 0 : xs + 1;
+      }
+      if (a >= FREE) {
+#pragma unroll
+        for (int j = (a - FREE) * BEHIND / (TN - FREE); j < (a - FREE + 1) * BEHIND / (TN - FREE); ++j) {
+          if (j < FREE) wf[j] = read_w(ws, 0, j);
+          else xf[0][j - FREE] = read_x(xs, 0, j - FREE);
+        }
+#pragma unroll
+        for (int j = (a - FREE) * TM / (TN - FREE); j < (a - FREE + 1) * TM / (TN - FREE); ++j) load_x(j, next_x, free_x);
+      }
+      TS_PIN;
+      tile(1, a, 0, TM);
+      TS_PIN;
+      if (a >= FREE) wf[a] = read_w(ws, 0, a);
+    }
+  }
+#undef TS_PIN
+  block_wait<0>();  // loads past the end
+  // The sums leave the loop where they were: without this the compiler rotated them through other registers in some of the
+  // loops (a third of all instructions).
+#pragma unroll
+  for (int a = 0; a < TN; ++a) {
+#pragma unroll
+    for (int b = 0; b < TM; ++b) asm volatile("" : "+a"(acc[a][b]));
+  }
+
+  // What bounds the stores is their number: one takes about 75 cycles, whether its lanes write 4 bytes each or 16, in
+  // pieces of 16 or of 64 bytes a row (256 x 256 outputs: 10.5 us with a store of 8 (gated: 4) bytes a lane for every tile,
+  // 4 with these; gate|up at 2,048 rows 460 -> 429 us).  So every lane writes 16 bytes: the four lanes of a row hold four consecutive
+  // columns of every tile, and exchange them until one holds eight of one of two tiles (gated: all of one of four).
+  // Rows beyond M lie past the buffer's end, tiles beyond N are sent there.
+  constexpr int BYTES = MODE == 1 ? 4 : 2, PER = MODE >= 2 ? 2 : 1;  // of an output element; weight rows of one
+  const int row_bytes = n / PER * BYTES;
+  char* base = MODE == 1 ? (char*)(partial + ((size_t)split * m + m_base) * n) : (char*)out + (size_t)m_base * row_bytes;
+  const __amdgpu_buffer_rsrc_t ybuf = block_buffer(base, (size_t)min(m - m_base, XR) * row_bytes);
+  const int tiles = (n - n_base) / 16 - wave_n * TN;  // of this wavefront's, those that exist
+  const int OUTSIDE = (int)0x80000000;
+  const int tile_bytes = 16 / PER * BYTES;
+  int row_at = (wave_m * TM * 16 + lane16) * row_bytes + (n_base / 16 + wave_n * TN) * tile_bytes;
+#pragma unroll
+  for (int b = 0; b < TM; ++b, row_at += 16 * row_bytes) {
+    constexpr int SHARE = MODE == 0 ? 2 : MODE >= 2 ? 4 : 1;  // tiles exchanged; what TN leaves over is stored tile by tile
+#pragma unroll
+    for (int c = 0; c < TN / SHARE; ++c) {
+      const int a = c * SHARE;
+      int mine = a;
+      u32x4 v;
+      if (MODE == 1) {
+        v = __builtin_bit_cast(u32x4, acc[a][b]);
+      } else if (MODE == 0) {
+        mine += group & 1;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const u32x2 both = block_swap16(block_pack(acc[a][b][2 * h], acc[a][b][2 * h + 1]),
+                                          block_pack(acc[a + SHARE - 1][b][2 * h], acc[a + SHARE - 1][b][2 * h + 1]));
+          v[h] = both[0];
+          v[2 + h] = both[1];
+        }
+      } else {
+        mine += group;
+        uint32_t u[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) u[t] = block_units<MODE == 2>(acc[a + t % SHARE][b], rule);
+        const u32x2 even = block_swap32(u[0], u[2]), odd = block_swap32(u[1], u[3]);
+        const u32x2 low = block_swap16(even[0], odd[0]), high = block_swap16(even[1], odd[1]);
+        v = u32x4{low[0], low[1], high[0], high[1]};
+      }
+      const int at = row_at + mine * tile_bytes + (MODE == 1 ? 16 * group : MODE == 0 ? 8 * (group & 2) : 0);
+      __builtin_amdgcn_raw_buffer_store_b128(v, ybuf, mine < tiles ? at : OUTSIDE, 0, 0);
+    }
+#pragma unroll
+    for (int a = TN / SHARE * SHARE; a < TN; ++a) {
+      const int at = a < tiles ? row_at + a * tile_bytes + tile_bytes / 4 * group : OUTSIDE;
+      if (MODE == 0)
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{block_pack(acc[a][b][0], acc[a][b][1]), block_pack(acc[a][b][2], acc[a][b][3])}, ybuf, at, 0, 0);
+      else
+        __builtin_amdgcn_raw_buffer_store_b32(block_units<MODE == 2>(acc[a][b], rule), ybuf, at, 0, 0);
+    }
+  }
+}
+
+template <int TN, int TM, int MODE>
+__global__ void __launch_bounds__(256, 1)
+gemm_block_kernel(float* __restrict__ partial, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, long x_stride,
+                  const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int m, int n, int k,
+                  int iters_per_split, int splits, int n_tiles, int m_tiles, GluRule rule) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];  // the rings: weight rows, activation rows
+  gemm_block<TN, TM, MODE>((lds_u16*)lds, (const lds_u16*)lds, partial, out, x, x_stride, w, bias, m, n, k, iters_per_split,
+                                 splits, n_tiles, m_tiles, rule);
+}
+
+template <int TN, int TM, int MODE>
+int launch_block_kernel(float* partial, uint16_t* out, const uint16_t* x, long x_stride, const uint16_t* w, const uint16_t* bias,
+                        int m, int n, int k, int iters_per_split, int splits, GluRule rule, hipStream_t stream) {
+  constexpr int NT = 32 * TN, XR = 32 * TM;
+  constexpr size_t lds_bytes = BlockRing<TN, TM>::BYTES;
+  static bool raised = false;  // per process; the attribute belongs to the kernel
+  if (!raised) {
+    if (hipFuncSetAttribute((const void*)gemm_block_kernel<TN, TM, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)lds_bytes) != hipSuccess)
+      return TS_ERR_LAUNCH;
+    raised = true;
+  }
+  const int n_tiles = (n + NT - 1) / NT, m_tiles = (m + XR - 1) / XR;
+  const long units = (long)n_tiles * splits;
+  const long ids = (units * m_tiles + BLOCK_DIES - 1) / BLOCK_DIES * BLOCK_DIES;
+  if (ids > 0x7fffffffL) return TS_ERR_SHAPE;
+  hipLaunchKernelGGL((gemm_block_kernel<TN, TM, MODE>), dim3((unsigned)ids), dim3(256), lds_bytes, stream, partial, out, x,
+                     x_stride, w, bias, m, n, k, iters_per_split, splits, n_tiles, m_tiles, rule);
+  return ts_launch_status();
+}
+
+}  // namespace
+
+// x [m, k] bfloat16 with row stride x_stride; w [n, k] bfloat16 contiguous; bias [n] bfloat16 or null; k a multiple of 64, n of 16.  mode
+// 0: out = bfloat16 [m, n] (splits must be 1); mode 1: partial = float [splits, m, n]; mode 2: out = bfloat16 [m, n / 2] =
+// the gated unit (common.hpp) of a w whose rows alternate gate, up (splits 1).  iters_per_split iterations of 64 of k go to
+// each of `splits` = ceil(k / 64 / iters_per_split) ranges.  tn, tm: 32 tn weight rows by 32 tm activation rows a
+// workgroup.
+extern "C" int ts_gemm_block(float* partial, void* out, const void* x, long x_stride, const void* w, const void* bias,
+                             int m, int n, int k, int iters_per_split, int splits, int tn, int tm, int mode,
+                             float steepness, float limit, float up_shift, float cubic, hipStream_t stream) {
+  if (m == 0 || n == 0) return TS_OK;
+  if (!x || !w || m < 0 || n < 0 || k < 1 || mode < 0 || mode > 2) return TS_ERR_ARG;
+  if ((mode == 1) != (partial != nullptr) || (mode != 1) != (out != nullptr)) return TS_ERR_ARG;
+  if (k % BLOCK_DEPTH != 0 || n % 16 != 0 || x_stride < k || x_stride % 8 != 0 || (uintptr_t)x % 16 != 0 || (uintptr_t)w % 16 != 0)
+    return TS_ERR_SHAPE;
+  // A block's rows are addressed by 31-bit byte offsets from its first one.
+  if (x_stride >= (1L << 21) || k >= (1 << 21) || n >= (1 << 20)) return TS_ERR_SHAPE;
+  const int total = k / BLOCK_DEPTH;
+  if (iters_per_split < 1 || splits != (total + iters_per_split - 1) / iters_per_split) return TS_ERR_SHAPE;
+  if (mode != 1 && splits != 1) return TS_ERR_ARG;
+  const GluRule rule = {steepness, limit, up_shift, cubic};
+  const bool plain = limit <= 0.f && cubic == 0.f;
+#define TS_BLOCK_MODE(TN, TM, MODE)                                                                                          \
+  return launch_block_kernel<TN, TM, MODE>(partial, (uint16_t*)out, (const uint16_t*)x, x_stride, (const uint16_t*)w,        \
+                                           (const uint16_t*)bias, m, n, k, iters_per_split, splits, rule, stream)
+#define TS_BLOCK(TN, TM)                       \
+  if (tn == TN && tm == TM) {                  \
+    if (mode == 0) TS_BLOCK_MODE(TN, TM, 0);   \
+    if (mode == 1) TS_BLOCK_MODE(TN, TM, 1);   \
+    if (plain) TS_BLOCK_MODE(TN, TM, 2);       \
+    TS_BLOCK_MODE(TN, TM, 3);                  \
+  }
+  TS_BLOCK(8, 8)
+  TS_BLOCK(8, 6)
+  TS_BLOCK(8, 5)
+  TS_BLOCK(5, 10)
+  TS_BLOCK(5, 8)
+  TS_BLOCK(4, 8)
+  TS_BLOCK(4, 5)
+  TS_BLOCK(4, 4)
+#undef TS_BLOCK
+#undef TS_BLOCK_MODE
+  return TS_ERR_SHAPE;
+}

@@ -1,4 +1,5 @@
-// The product of steps with more rows than a decode step has (129 rows and up), tiled through LDS:
+// The product of decode steps of many rows, and of longer steps where gemm_block.hip does not take the operands (K no
+// multiple of 64, N none of 16), tiled through LDS:
 //   Y[m][n] = sum over k of X[m][k] * W[n][k]  (+ bias[n])
 // bfloat16 activations X [M, K] and weights W [N, K] as the checkpoint stores them (F.linear's
 // layout, src/turboserve/engine/model/layers.py:142), 32-bit accumulation on the matrix cores.

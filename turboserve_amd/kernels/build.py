@@ -50,6 +50,7 @@ MODULES: dict[str, tuple[str, ...]] = {
         "gemm_skinny.hip",
         "gemm_tiled.hip",
         "gemm_wide.hip",
+        "gemm_block.hip",
         "sampling.hip",
         "probe.hip",
     ),

@@ -146,6 +146,8 @@ _SIGNATURES: dict[str, dict[str, list]] = {
                           c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_wide": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                          c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
+        "ts_gemm_block": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
+                          c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_skinny_resident": [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                     c_int, c_int, c_int, c_void_p],
         "ts_argmax": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
@@ -378,6 +380,7 @@ class Ops:
         self._raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         self._tiled_plans: dict[tuple, tuple[int, int, int]] = {}  # (m, n, k, max_splits) -> grid of the tiled product
         self._wide_plans: dict[tuple, tuple[int, int, int, int, int]] = {}  # (m, n, k, one range) -> grid of the wide product
+        self._block_plans: dict[tuple, tuple[int, int, int, int]] = {}  # (m, n, k, kind) -> grid of the block product
         #: (rows a step's products run at, N, K, kind) -> whether this engine's own product was the
         #: faster one when both were timed (``time_wide_choices``).
         self.wide_choices: dict[tuple, bool] = {}
@@ -2121,12 +2124,98 @@ class Ops:
                    "ts_gemm_tiled")
         return partial
 
-    #: Up to this many rows a product that was not timed against the BLAS library runs this
-    #: engine's own kernel (more than ``skinny_max_rows``: ``gemm_wide``).  At the 7B shape the own
-    #: kernel is the faster one up to about a thousand rows (down projection at 256 / 512 rows: 47 /
-    #: 75 us against the library's best 75 / 116; gate|up with its SwiGLU 78 / 149 against 89 / 151),
-    #: the library above (2,048 rows: gate|up 516 against 402 + 44 us, down 270 against 241).
+    #: Up to this many rows a product that was not timed against the BLAS library and that the block
+    #: product does not take (``block_supported``) runs ``gemm_wide``.  At the 7B shape that kernel
+    #: is the faster one up to about a thousand rows (down projection at 256 / 512 rows: 47 / 75 us
+    #: against the library's best 75 / 116; gate|up with its SwiGLU 78 / 149 against 89 / 151), the
+    #: library above.  0: every product of more than ``skinny_max_rows`` rows is the library's.
     wide_default_rows = 640
+
+    #: The block product's tiles (in 32 weight rows, 32 activation rows) and what an iteration of
+    #: 64 of K takes a compute unit with each, in microseconds: the slope over K of products at 144
+    #: to 2,048 rows that give every compute unit a workgroup.
+    _BLOCK_TILES = {(8, 8): 1.24, (8, 6): 0.99, (8, 5): 0.86, (5, 10): 1.07, (5, 8): 0.88, (4, 8): 0.76, (4, 5): 0.54, (4, 4): 0.50}
+
+    @staticmethod
+    def block_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
+        """Whether ``csrc/gemm_block.hip`` takes a product: bfloat16, K a multiple of 64 (whole
+        lines of 128 bytes), N of 16 (whole tiles), rows of 16-byte pieces, a block's rows within
+        the 31 bits of a buffer's offsets."""
+        n, k = weight.shape
+        return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and k % 64 == 0 and k > 0 and n % 16 == 0
+                and x.stride(1) == 1 and k <= x.stride(0) < 1 << 21 and x.stride(0) % 8 == 0 and n < 1 << 20
+                and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+    def _block_plan(self, m: int, n: int, k: int, kind: str) -> tuple[int, int, int, int]:
+        """(iterations of 64 per range of K, ranges, tile of weight rows, of activation rows) of the
+        block product: the cheapest grid, where a round of workgroups (one per compute unit) takes
+        its iterations and six more (first loads, stores) at the tile's pace, a gated
+        result the unit's time, and partial sums of several ranges their way to the norm, 3.6
+        bytes per nanosecond.  Against every tile with 1 to 16 ranges, timed for the matrices of six shapes (K 2,048 to 18,944) at 144 to
+        2,048 rows, the plan's grid takes 1% more than the fastest on average.
+        ``kind``: "sums" (partial sums may stay), "one" (one bfloat16 result), "gated"."""
+        key = (m, n, k, kind)
+        known = self._block_plans.get(key)
+        if known is not None:
+            return known
+        iters = k // 64
+        best = None
+        for (tn, tm), pace in self._BLOCK_TILES.items():
+            tiles = -(-n // (32 * tn)) * -(-m // (32 * tm))
+            for want in range(1, (min(iters, 16) if kind == "sums" else 1) + 1):
+                per_split = -(-iters // want)
+                splits = -(-iters // per_split)
+                if splits != want:
+                    continue
+                cost = -(-tiles * splits // self.compute_units) * ((per_split + 6) * pace + (0.1 * tn * tm if kind == "gated" else 0.0))
+                if splits > 1:
+                    cost += splits * m * n * 4 / 3.6e6
+                if best is None or cost < best[0]:
+                    best = (cost, per_split, splits, tn, tm)
+        self._block_plans[key] = best[1:]
+        return best[1:]
+
+    def gemm_block(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *,
+                   plan: tuple[int, int, int, int], gated: bool = False, sums: bool = False,
+                   rule: tuple[float, float, float] = (1.0, 0.0, 0.0)) -> torch.Tensor:
+        """``x [M, K] @ weight [N, K]^T (+ bias)`` in blocks of up to 256 x 256 outputs
+        (``csrc/gemm_block.hip``), what ``block_supported`` says.  ``plan`` as :meth:`_block_plan`
+        gives it; results as :meth:`gemm_wide`'s."""
+        _gpu(x, weight, bias)
+        _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1], "x must be [M, K], weight [N, K]")
+        _need(self.block_supported(x, weight), "the block product takes bfloat16 rows of 16-byte pieces, K % 64 == 0 and N % 16 == 0")
+        m, k = x.shape
+        n = weight.shape[0]
+        if bias is not None:
+            _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 8 == 0,
+                  "bias must be bfloat16 [N]")
+        per_split, splits, tn, tm = plan
+        _need(not gated or splits == 1, "the gated result needs one range of K")
+        partial = out = None
+        if gated or (splits == 1 and not sums):
+            out = self.rows_buffer(m, n // 2 if gated else n, torch.bfloat16, x.device)
+        else:
+            partial = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+        _check(self.core.ts_gemm_block(_ptr(partial), _ptr(out), _ptr(x), x.stride(0), _ptr(weight), _ptr(bias), m, n, k, per_split,
+                                       splits, tn, tm, 2 if gated else 1 if out is None else 0, *glu_rule(rule), self.stream()),
+               "ts_gemm_block")
+        return partial if out is None else out
+
+    def _own_product(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, kind: str,
+                     rule: tuple[float, float, float] = (1.0, 0.0, 0.0)):
+        """This engine's product for a step of more rows than the decode products take, as a call
+        without arguments, and whether it runs where no timing was made (``_wide_runs``): the block
+        product always, where it takes the operands (over the matrices above at 144 to 2,048 rows, with the kernel that
+        reads the result, the library's takes 1.32 times as long for gate|up, 1.5 for partial
+        sums, 1.15 for one result; the few it is faster at, up to 1.2 times, follow no size), else ``gemm_wide``."""
+        m, (n, k) = x.shape[0], weight.shape
+        if self.block_supported(x, weight) and (bias is None or bias.data_ptr() % 8 == 0):
+            block = self._block_plan(m, n, k, kind)
+            return lambda: self.gemm_block(x, weight, bias, plan=block, gated=kind == "gated", rule=rule), self.wide_default_rows > 0
+        wide = self._wide_plan(m, n, k, kind != "sums")
+        workgroups = -(-n // (32 * wide[2])) * -(-m // wide[3]) * wide[1]
+        return (lambda: self.gemm_wide(x, weight, bias, plan=wide, gated=kind == "gated", rule=rule),
+                m <= self.wide_default_rows and (2 * workgroups >= self.compute_units or m * n * k < self.library_tuning_min_work))
 
     def _wide_plan(self, m: int, n: int, k: int, one_range: bool) -> tuple[int, int, int, int, int]:
         """(iterations of 64 per range of K, ranges, tile, activation rows, wavefronts) of the wide
@@ -2164,11 +2253,10 @@ class Ops:
         self._wide_plans[key] = best[1:]
         return best[1:]
 
-    def _wide_runs(self, rows: int, n: int, k: int, kind: str, plan, own, library) -> bool:
-        """Whether this engine's own product (with the grid ``plan``), not the BLAS library's, runs
-        a product of ``rows`` rows (more than the decode products take): what a timing found, or,
-        untimed, up to ``wide_default_rows`` rows if the grid gives at least half of the compute
-        units a workgroup.  With ``time_wide_choices`` an unknown product that is worth timing
+    def _wide_runs(self, rows: int, n: int, k: int, kind: str, untimed: bool, own, library) -> bool:
+        """Whether this engine's own product, not the BLAS library's, runs a product of ``rows``
+        rows (more than the decode products take): what a timing found, or ``untimed``
+        (``_own_product``).  With ``time_wide_choices`` an unknown product that is worth timing
         runs both ways here (``own()`` and ``library()``), four launches each behind a warm-up, each
         waited for, the best by device events that see the device's time alone."""
         key = (self.library_rows(rows), n, k, kind)
@@ -2176,8 +2264,7 @@ class Ops:
         if known is not None:
             return known
         if not self.time_wide_choices or rows * n * k < self.library_tuning_min_work:
-            workgroups = -(-n // (32 * plan[2])) * -(-rows // plan[3]) * plan[1]
-            return rows <= self.wide_default_rows and (2 * workgroups >= self.compute_units or rows * n * k < self.library_tuning_min_work)
+            return untimed
         # One launch at a time, each waited for: launches that follow one another without a
         # dependency overlap where a grid leaves compute units idle, and would look faster than
         # they are inside a step.  Each timed launch follows a kernel that keeps the device busy
@@ -2454,10 +2541,10 @@ class Ops:
               and weight.is_contiguous() and x.stride(1) == 1):
             _gpu(x, weight, bias)
             m, (n, k) = x.shape[0], weight.shape
-            plan = self._wide_plan(m, n, k, True)
-            if self._wide_runs(m, n, k, "gated", plan, lambda: self.gemm_wide(x, weight, bias, plan=plan, gated=True, rule=rule),
+            own, untimed = self._own_product(x, weight, bias, "gated", rule)
+            if self._wide_runs(m, n, k, "gated", untimed, own,
                                lambda: self.swiglu(self._library_product(x, weight, bias, None), x.dtype, paired=True, rule=rule)):
-                return self.gemm_wide(x, weight, bias, plan=plan, gated=True, rule=rule)
+                return own()
             return self.swiglu(self._library_product(x, weight, bias, None), x.dtype, paired=True, rule=rule)
         return self.swiglu(self.linear(x, weight, bias), x.dtype, paired=True, rule=rule)
 
@@ -2468,10 +2555,10 @@ class Ops:
         :meth:`gemm_skinny` and return ``[S, M, N]`` 32-bit partial sums for the consumer to add
         up, or, where K is no multiple of 8 (the matrix-core kernels load 16 bytes at a time),
         :meth:`gemm_plain` on bfloat16 operands: slower, but a kernel of this engine, so a
-        recorded step never holds a library call.  Larger batches use :meth:`gemm_wide` or the
+        recorded step never holds a library call.  Larger batches use :meth:`gemm_block`, :meth:`gemm_wide` or the
         BLAS library behind torch (as the reference does for every linear layer,
         src/turboserve/engine/model/layers.py:142), whichever was the faster one when both were
-        timed (``_wide_runs``).  ``for_residual``: the result is what a
+        timed (``_wide_runs``; untimed: ``_own_product``).  ``for_residual``: the result is what a
         norm adds to the 32-bit residual stream, so the library leaves it in 32-bit too (as
         ``[1, M, N]``, one partial sum): the stream then gets the same unrounded addend from a
         prompt's step as from a decode step's partial sums."""
@@ -2486,11 +2573,10 @@ class Ops:
             m, (n, k) = x.shape[0], weight.shape
             # What goes into the residual stream may stay partial sums (the norm adds them up);
             # any other consumer of a step this long wants one bfloat16 result.
-            plan = self._wide_plan(m, n, k, not for_residual)
-            if self._wide_runs(m, n, k, "sums" if for_residual else "one", plan,
-                               lambda: self.gemm_wide(x, weight, bias, plan=plan),
-                               lambda: self._library_product(x, weight, bias, None)):
-                return self.gemm_wide(x, weight, bias, plan=plan)
+            kind = "sums" if for_residual else "one"
+            own, untimed = self._own_product(x, weight, bias, kind)
+            if self._wide_runs(m, n, k, kind, untimed, own, lambda: self._library_product(x, weight, bias, None)):
+                return own()
         if for_residual and self.library_residual_float32:
             out = self._library_product(x, weight, None, torch.float32)
             if bias is not None:
