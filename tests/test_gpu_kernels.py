@@ -56,6 +56,26 @@ def test_rmsnorm_and_fused_residual(ops, dtype, tokens, hidden):
     torch.testing.assert_close(got, plain.rms_norm(total, w.float(), eps)[[tokens - 1, 0]], **tol(dtype))
 
 
+@pytest.mark.parametrize("rows,hidden,splits", [(256, 2052, 3), (257, 2052, 3), (512, 4100, 1), (513, 2048, 1), (513, 2052, 2), (700, 5120, 1),
+                                                (514, 8196, 9), (300, 16384, 1), (600, 16, 17), (513, 16388, 2)])
+def test_add_rmsnorm_at_the_edges_of_its_blocks(ops, rows, hidden, splits):
+    """Rows and widths on both sides of where the threads per row change, bfloat16 addends and 32-bit
+    partial sums: the residual to one rounding per addend, the normalised row to bfloat16 rounding."""
+    g = torch.Generator().manual_seed(rows + hidden)
+    residual = torch.randn(rows, hidden, generator=g)
+    parts = torch.randn(splits, rows, hidden, generator=g)
+    w = (1 + 0.1 * torch.randn(hidden, generator=g)).bfloat16()
+    for pending in (parts, parts[0].bfloat16()) if splits == 1 else (parts,):
+        added = pending.double() if pending.dim() == 2 else pending.double().sum(0)
+        want = residual.double() + added
+        res_dev = residual.to(DEV)
+        got = ops.add_rmsnorm(res_dev, pending.to(DEV), w.to(DEV), 1e-6).double().cpu()
+        sizes = residual.double().abs() + parts.double().abs().sum(0)
+        assert bool(((res_dev.double().cpu() - want).abs() <= (splits + 1) * 2.0**-24 * sizes).all())
+        normed = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + 1e-6) * w.double()
+        assert bool(((got - normed).abs() <= 2.0**-7 * normed.abs() + 1e-5).all())
+
+
 def test_rmsnorm_rounds_before_the_gain(ops):
     """bfloat16: the normalised value is rounded to bfloat16 before the gain multiplies it
     (src/turboserve/engine/model/layers.py:208); a single rounding of the product differs."""
