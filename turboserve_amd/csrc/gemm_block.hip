@@ -233,9 +233,14 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
       if (a == FREE) {
         // This wavefront has read all of iteration `it` (its fragments are in registers) and its loads of it + 1 have landed;
         // behind the barrier both hold for the workgroup.
+#pragma unroll
+        for (int b = 0; b < TM; ++b) asm volatile("" : "+v"(xf[1][b]));
+#pragma unroll
+        for (int j = FREE; j < TN; ++j) asm volatile("" : "+v"(wf[j]));
         block_wait<Ring::LEFT>();
         ws = ws + 1 == RW ? 0 : ws + 1;
         xs = xs + 1 == RX ? 0 : xs + 1;
+        asm volatile("" : "+s"(ws), "+s"(xs));  // the compiler, for which no load writes what it reads, sees new addresses
       }
       if (a >= FREE) {
 #pragma unroll
