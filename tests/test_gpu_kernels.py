@@ -172,6 +172,14 @@ def test_gemm_plain_layouts(ops, dtype, n, k, most):
         if m <= most:
             assert torch.equal(ops.gemm_plain(x[:m], w, out_float32=True), whole[:m]), m
             assert torch.equal(ops.gemm_plain(wide[:m, :k], w, out_float32=True), whole[:m]), m
+    padded = torch.full((most, k + 8), float("nan"), dtype=dtype, device=DEV)  # rows that they fit, what lies behind each not read
+    padded[:, :k] = x
+    w[n // 2] = float("nan")  # nor what lies behind a row of the weights
+    for m in (1, 16, 17, 40):
+        got = ops.gemm_plain(padded[:m, :k], w, out_float32=True)
+        assert bool(got[:, n // 2].isnan().all())
+        got[:, n // 2] = whole[:m, n // 2]
+        assert torch.equal(got, whole[:m]), m
 
 
 @pytest.mark.parametrize("m", [1, 5, 16, 17, 33, 64, 65, 100, 128])

@@ -8,13 +8,13 @@
 // two (four) products to the accumulator one after the other, in the order of k, each step a fused
 // multiply-add rounded to nearest with denormals kept (a loop of fmaf gives the same bits; compared
 // over random, widely spread, denormal and cancelling operands at K of 4 to 3,584).  So a row's
-// result depends neither on which other rows are in the batch nor on which of the two layouts
-// below runs it, both run at the matrix cores' 157 TFLOP/s, twice what unpacked vector
+// result depends neither on which other rows are in the batch nor on which of the layouts
+// below runs it, they run at the matrix cores' 157 TFLOP/s, twice what unpacked vector
 // multiply-adds allow, and a few rows against a long K get four times the wavefronts one chain would.
 //
 // Microseconds at the 7B shape, one chain of vector multiply-adds (64 x 64 tiles; up to 32 rows one output a thread)
-// -> these: gate|up at 8 / 64 / 500 rows 194 -> 122, 765 -> 208, 3,048 -> 1,142 (119 TFLOP/s); down 220 -> 60, 3,402 -> 159,
-// 3,365 -> 724; o 35 -> 15, 581 -> 38, 581 -> 139; q|k|v 41 -> 23, 579 -> 72, 638 -> 195; the head at 8 rows 637 -> 433.
+// -> these: gate|up at 8 / 64 / 500 rows 194 -> 88, 765 -> 208, 3,048 -> 1,142 (119 TFLOP/s); down 220 -> 47, 3,402 -> 155,
+// 3,365 -> 724; o 35 -> 13, 581 -> 29, 581 -> 139; q|k|v 41 -> 18, 579 -> 43, 638 -> 195; the head at 8 rows 637 -> 330.
 #include "common.hpp"
 
 namespace {
@@ -259,14 +259,14 @@ gemm_plain_kernel(TOut* __restrict__ y, const TIn* __restrict__ x, const TIn* __
 }
 
 // ---------------------------------------------------------------------------------------------
-// Few rows: a workgroup owns 16 MT activation rows by 16 NT weight rows, each of its four wavefronts one range of
+// Few rows of bfloat16, or of rows that 16-byte loads do not divide: a workgroup owns 16 MT activation rows by 16 NT weight rows, each of its four wavefronts one range of
 // K; both operands go straight from memory into registers, AHEAD slices of 64 k in flight, without LDS
 // or a barrier before the ranges' sums meet at the end: bound by reading W.
 // Lane (r, g) = (lane % 16, lane / 16) loads 16 bytes of row r: elements 4 g .. 4 g + 3 of every 16, 64 bytes of each of
 // sixteen rows an instruction; four lane swaps (permlane32/16) turn the 4 x 4 of groups and
 // elements round, so that step s of the 16 holds element 4 s + g: the order of k.
 // The loads are plain ones: an instruction takes half a line, and marked non-temporal the other half
-// came from memory again (gate|up at 8 rows 152 us, plain 131; 120 with two weight tiles a wavefront).
+// came from memory again (32-bit gate|up at 8 rows 152 us, plain 131).
 __device__ __forceinline__ void turn_quads(gp_f32x4& v) {
   float e0 = v[0], e1 = v[1], e2 = v[2], e3 = v[3];
   auto swap32 = [](float& a, float& b) __attribute__((always_inline)) {
@@ -405,25 +405,221 @@ gemm_plain_few_rows_kernel(TOut* __restrict__ y, const TIn* __restrict__ x, cons
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same few rows of 32-bit operands, bound by reading W: whole lines, straight from memory to LDS.  Above, an instruction
+// takes 64 bytes of each of sixteen rows and W cannot be marked as read once (4.3 TB/s); here one takes 128 bytes of
+// each of eight, non-temporal where one tile of activation rows reads them.  A wavefront stages its own range
+// in a ring of its own, SLOTS slices of 32 k (a slot is filled again as soon as its fragments are in registers), so nothing
+// meets at a barrier before the ranges' sums.  gate|up at 8 rows 127 -> 88 us (6.1 TB/s), at 32 191 -> 122; the head at 8 441 -> 330
+// (6.6 TB/s); down 61 -> 47, o 16.4 -> 12.6, q|k|v 25 -> 18.  Piece p (16 bytes) of row r lies at position p ^ (r / 2 % 8) of the row's eight:
+// a piece of sixteen rows touches every bank once.  The same chains, bit for bit.
+typedef __attribute__((address_space(3))) float lds_f32;
+typedef __attribute__((address_space(3))) gp_f32x4 lds_f32x4;
+
+template <int MT, int NT>
+struct Stream {
+  static constexpr int SLICE = 32, TILE = 16 * SLICE, LOADS = 2 * (MT + NT);          // of a tile of sixteen rows; of a slice
+  static constexpr int SLOTS = 80 * 1024 / (4 * (MT + NT) * TILE * 4);                // two workgroups a compute unit
+  static constexpr int WAVE = SLOTS * (MT + NT) * TILE;                               // floats of a wavefront's ring
+  static constexpr size_t BYTES = (size_t)4 * WAVE * 4;
+  static_assert(SLOTS >= 2 && (SLOTS - 1) * LOADS < 64 && 2 * BYTES <= 160 * 1024, "a ring of at least two slices, counted by vmcnt");
+  static_assert(WAVE >= MT * NT * 256, "a wavefront's sums fit its ring");
+};
+
+// `to` and `from` are the same memory: __restrict__ keeps the compiler from waiting for every load in flight before every
+// read, so it must not see that two reads have one address either: the slot that stream_wait lets be read is a new value to
+// it (a slot it could follow, it read once for all rounds).
+template <int LEFT>
+__device__ __forceinline__ void stream_wait(int& slot) {
+  asm volatile("s_waitcnt vmcnt(%1)" : "+s"(slot) : "n"(LEFT) : "memory");
+}
+
+template <int MT, int NT, bool ONCE>
+__device__ __forceinline__ void stream_ranges(lds_f32* __restrict__ to, const lds_f32* __restrict__ from, const float* __restrict__ x,
+                                              const float* __restrict__ w, int m, int n, int k, long x_stride,
+                                              gp_f32x4 (&acc)[MT][NT]) {
+  typedef Stream<MT, NT> S;
+  constexpr int SLICE = S::SLICE, TILE = S::TILE, SLOTS = S::SLOTS;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+  const int range = range_of(k), start = wave * range, end = min(start + range, k);  // this wavefront's k
+  if (start >= end) return;
+  const int count = (end - start + SLICE - 1) / SLICE;
+  // A lane loads piece (lane % 8) ^ key of row lane / 8 of eight; the second eight of a tile, whose keys are four further on, piece ^ 4.  Offsets count
+  // from a tile's first row: what lies past the last row's end (rows beyond N or M, k beyond the last row's) brings zeros,
+  // k beyond another row's end that row's neighbours, cleared below.
+  const int row8 = lane >> 3, piece = (lane & 7) ^ (row8 >> 1);
+  const size_t wbytes = (size_t)min(n - n0, 16 * NT) * k * 4, xbytes = ((size_t)(min(m - m0, 16 * MT) - 1) * x_stride + k) * 4;
+  const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w + (size_t)n0 * k), 0, (int)wbytes, 0x00027000);
+  const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + (size_t)m0 * x_stride), 0, (int)xbytes, 0x00027000);
+  uint32_t woff[2 * NT], xoff[2 * MT];
+#pragma unroll
+  for (int j = 0; j < 2 * NT; ++j) woff[j] = ((uint32_t)(8 * j + row8) * (uint32_t)k + start + 4 * (piece ^ (j & 1 ? 4 : 0))) * 4;
+#pragma unroll
+  for (int j = 0; j < 2 * MT; ++j) xoff[j] = ((uint32_t)(8 * j + row8) * (uint32_t)x_stride + start + 4 * (piece ^ (j & 1 ? 4 : 0))) * 4;
+  auto fetch = [&](int i, int slot) __attribute__((always_inline)) {
+    const uint32_t at = (uint32_t)min(i, count - 1) * (SLICE * 4);  // past the end: the last slice again, never read
+    lds_f32* base = to + slot * (MT + NT) * TILE;
+#pragma unroll
+    for (int j = 0; j < 2 * NT; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, base + j * (TILE / 2), 16, woff[j] + at, 0, 0, ONCE ? 2 : 0);
+#pragma unroll
+    for (int j = 0; j < 2 * MT; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, base + NT * TILE + j * (TILE / 2), 16, xoff[j] + at, 0, 0, 0);
+  };
+  struct Frags {
+    gp_f32x4 x[MT][2], w[NT][2];
+  };
+  const int key = (r >> 1) & 7;
+  auto read = [&](Frags& f, int slot) __attribute__((always_inline)) {
+    const lds_f32* base = from + slot * (MT + NT) * TILE + r * SLICE;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int at = 4 * ((4 * c + g) ^ key);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) f.w[t][c] = *(const lds_f32x4*)(base + t * TILE + at);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) f.x[t][c] = *(const lds_f32x4*)(base + (NT + t) * TILE + at);
+    }
+  };
+  auto consume = [&](Frags& f, int left) __attribute__((always_inline)) {  // left: elements of the slice inside the row
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        if (left < SLICE) clear_past(f.x[t][c], left - 16 * c - 4 * g);
+        turn_quads(f.x[t][c]);
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        if (left < SLICE) clear_past(f.w[t][c], left - 16 * c - 4 * g);
+        turn_quads(f.w[t][c]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+#pragma unroll
+        for (int a = 0; a < MT; ++a) {
+#pragma unroll
+          for (int b = 0; b < NT; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.x[a][c][e], f.w[b][c][e], acc[a][b], 0, 0, 0);
+        }
+      }
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < SLOTS; ++j) fetch(j, j);
+  int slot = 0;
+  stream_wait<(SLOTS - 1) * S::LOADS>(slot);
+  Frags f[2];
+  read(f[0], slot);
+  auto round = [&](int i, Frags& now, Frags& next) __attribute__((always_inline)) {
+    // `now` is in registers: its slot is free.
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(now.w[t][c])::"memory");
+#pragma unroll
+      for (int t = 0; t < MT; ++t) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(now.x[t][c])::"memory");
+    }
+    fetch(i + SLOTS, slot);
+    slot = slot + 1 == SLOTS ? 0 : slot + 1;
+    stream_wait<(SLOTS - 1) * S::LOADS>(slot);
+    read(next, slot);
+    consume(now, SLICE);
+  };
+  int i = 0;  // the last slice alone may be cut short
+  for (; i + 2 < count; i += 2) {
+    round(i, f[0], f[1]);
+    round(i + 1, f[1], f[0]);
+  }
+  const int left = end - start - (count - 1) * SLICE;
+  if (i + 1 < count) {
+    round(i, f[0], f[1]);
+    consume(f[1], left);
+  } else {
+    consume(f[0], left);
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // loads past the end
+}
+
+template <int MT, int NT, bool ONCE>
+__global__ void __launch_bounds__(256)
+gemm_plain_stream_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
+                         const float* __restrict__ bias, int m, int n, int k, long x_stride, long y_stride) {
+  typedef Stream<MT, NT> S;
+  extern __shared__ __attribute__((aligned(16))) float ring[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  gp_f32x4 acc[MT][NT];
+#pragma unroll
+  for (int a = 0; a < MT; ++a) {
+#pragma unroll
+    for (int b = 0; b < NT; ++b) acc[a][b] = gp_f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  lds_f32* mine = (lds_f32*)ring + wave * S::WAVE;
+  stream_ranges<MT, NT, ONCE>(mine, mine, x, w, m, n, k, x_stride, acc);
+  // The ranges' sums meet in the rings.
+#pragma unroll
+  for (int a = 0; a < MT; ++a) {
+#pragma unroll
+    for (int b = 0; b < NT; ++b) *(lds_f32x4*)(mine + ((a * NT + b) * 64 + lane) * 4) = acc[a][b];
+  }
+  __syncthreads();
+  // Wavefront v adds up and stores tiles v, v + 4, ...
+  const int r = lane & 15, g = lane >> 4, range = range_of(k);
+#pragma unroll
+  for (int t = 0; t < MT * NT; ++t) {
+    if (t % 4 != wave) continue;
+    const int col = blockIdx.x * 16 * NT + 16 * (t % NT) + r;
+    if (col >= n) continue;
+    gp_f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      if (p == 0 || p * range < k) sum += *(const lds_f32x4*)((lds_f32*)ring + p * S::WAVE + (t * 64 + lane) * 4);
+    const float bv = bias ? bias[col] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = blockIdx.y * 16 * MT + 16 * (t / NT) + 4 * g + i;
+      if (row < m) y[(size_t)row * y_stride + col] = bias ? sum[i] + bv : sum[i];
+    }
+  }
+}
+
+template <int MT, int NT, bool ONCE>
+int launch_stream(void* y, const void* x, const void* w, const void* bias, int m, int n, int k, long x_stride, long y_stride,
+                  dim3 grid, hipStream_t stream) {
+  static bool raised = false;  // per process; the attribute belongs to the kernel
+  if (!raised) {
+    if (hipFuncSetAttribute((const void*)gemm_plain_stream_kernel<MT, NT, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)Stream<MT, NT>::BYTES) != hipSuccess)
+      return TS_ERR_LAUNCH;
+    raised = true;
+  }
+  hipLaunchKernelGGL((gemm_plain_stream_kernel<MT, NT, ONCE>), grid, dim3(256), (Stream<MT, NT>::BYTES), stream, (float*)y,
+                     (const float*)x, (const float*)w, (const float*)bias, m, n, k, x_stride, y_stride);
+  return ts_launch_status();
+}
+
 inline long ceil_of(long a, long b) { return (a + b - 1) / b; }
 
-// Which layout runs a product: the one whose workgroups are through soonest, one a compute unit at a time.  Microseconds
-// at K = 3,584, measured over q|k|v, o, gate|up and the head of the 7B shape at 1 to 2,048 rows (all grow with K alike):
-// a round of workgroups of 16 x 16 outputs takes 13, of 16 x 32 24, 32 x 16 22, 32 x 32 37 (more weight rows a
-// wavefront read the activations less often, fewer give more workgroups), of 64 x 64 65, of 128 x 128 235, and the
-// first round of some a little more.
+// Which layout runs a product: the one whose workgroups are through soonest, a round of one on every compute unit at a time.
+// Half microseconds at K = 3,584, measured over q|k|v, o, gate|up and the head of the 7B shape at 1 to 2,048 rows (all
+// grow with K alike): a round of workgroups of 16 x 16 outputs whose operands go through LDS takes 9.5 us (read straight from
+// memory 13), of 16 x 32 17.5 (24), 32 x 16 15 (22), 32 x 32 24.5 (37) (more weight rows a wavefront read the
+// activations less often, fewer give more workgroups), of 64 x 64 70, of 128 x 128 240, and the first round a little more.
 enum PlainKind { FEW_1_1, FEW_1_2, FEW_2_1, FEW_2_2, TILES_64, TILES_128 };
 
-inline PlainKind plain_kind(int m, int n) {
+inline PlainKind plain_kind(int m, int n, bool stream_reads) {
   static const struct {
     PlainKind kind;
-    int rows, cols, start, round;
-  } layouts[] = {{FEW_1_1, 16, 16, 3, 13}, {FEW_1_2, 16, 32, 0, 24}, {FEW_2_1, 32, 16, 3, 22},
-                 {FEW_2_2, 32, 32, 0, 37}, {TILES_64, 64, 64, 12, 65}, {TILES_128, 128, 128, 0, 235}};
+    int rows, cols, start[2], round[2];  // straight from memory, through LDS
+  } layouts[] = {{FEW_1_1, 16, 16, {6, 6}, {26, 19}}, {FEW_1_2, 16, 32, {0, 2}, {48, 35}}, {FEW_2_1, 32, 16, {6, 8}, {44, 30}},
+                 {FEW_2_2, 32, 32, {0, 4}, {74, 49}}, {TILES_64, 64, 64, {24, 10}, {130, 140}}, {TILES_128, 128, 128, {0, 0}, {470, 480}}};
   PlainKind best = TILES_128;
   long least = -1;
   for (const auto& l : layouts) {
-    const long cost = l.start + l.round * ceil_of(ceil_of(m, l.rows) * ceil_of(n, l.cols), GP_UNITS);
+    const long cost = l.start[stream_reads] + l.round[stream_reads] * ceil_of(ceil_of(m, l.rows) * ceil_of(n, l.cols), GP_UNITS);
     if (least < 0 || cost < least) best = l.kind, least = cost;
   }
   return best;
@@ -435,6 +631,8 @@ int launch_plain(void* y, const void* x, const void* w, const void* bias, int m,
   const size_t quad = 4 * sizeof(TIn);
   const bool vec = k % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)x % quad == 0 && (uintptr_t)w % quad == 0 &&
                    x_stride < (1L << 25) && k < (1 << 25);
+  // 32-bit operands whose rows lie within the 31 bits of a buffer's offsets go through LDS.
+  const bool stream_reads = sizeof(TIn) == 4 && vec && x_stride < (1L << 24) && k < (1 << 24);
 #define TS_PLAIN_ARGS (TOut*)y, (const TIn*)x, (const TIn*)w, (const TIn*)bias, m, n, k, x_stride, y_stride
 #define TS_PLAIN_TILED(T, BK, V)                                                                                      \
   do {                                                                                                               \
@@ -444,25 +642,32 @@ int launch_plain(void* y, const void* x, const void* w, const void* bias, int m,
     hipLaunchKernelGGL((gemm_plain_kernel<T, T, BK, V, TIn, TOut>), dim3((unsigned)ids), dim3(256), 0, stream,       \
                        TS_PLAIN_ARGS, m_tiles, n_tiles);                                                             \
   } while (0)
-#define TS_PLAIN_FEW(MT, NT, AHEAD, V)                                                                                \
+#define TS_PLAIN_FEW(MT, NT, AHEAD)                                                                                   \
   do {                                                                                                               \
     dim3 grid((unsigned)ceil_of(n, 16 * NT), (unsigned)ceil_of(m, 16 * MT));                                         \
     if (grid.y > 65535) return TS_ERR_SHAPE;                                                                         \
-    hipLaunchKernelGGL((gemm_plain_few_rows_kernel<MT, NT, AHEAD, V, TIn, TOut>), grid, dim3(256), 0, stream,        \
-                       TS_PLAIN_ARGS);                                                                               \
+    if (stream_reads)                                                                                                \
+      return grid.y == 1 ? launch_stream<MT, NT, true>(y, x, w, bias, m, n, k, x_stride, y_stride, grid, stream)     \
+                         : launch_stream<MT, NT, false>(y, x, w, bias, m, n, k, x_stride, y_stride, grid, stream);   \
+    if (vec && sizeof(TIn) == 2)                                                                                     \
+      hipLaunchKernelGGL((gemm_plain_few_rows_kernel<MT, NT, AHEAD, sizeof(TIn) == 2, TIn, TOut>), grid, dim3(256),  \
+                         0, stream, TS_PLAIN_ARGS);                                                                  \
+    else                                                                                                             \
+      hipLaunchKernelGGL((gemm_plain_few_rows_kernel<MT, NT, 2, false, TIn, TOut>), grid, dim3(256), 0, stream,      \
+                         TS_PLAIN_ARGS);                                                                             \
   } while (0)
-  switch (plain_kind(m, n)) {
+  switch (plain_kind(m, n, stream_reads)) {
     case FEW_1_1:
-      if (vec) TS_PLAIN_FEW(1, 1, 3, true); else TS_PLAIN_FEW(1, 1, 2, false);
+      TS_PLAIN_FEW(1, 1, 3);
       break;
     case FEW_1_2:
-      if (vec) TS_PLAIN_FEW(1, 2, 3, true); else TS_PLAIN_FEW(1, 2, 2, false);
+      TS_PLAIN_FEW(1, 2, 3);
       break;
     case FEW_2_1:
-      if (vec) TS_PLAIN_FEW(2, 1, 3, true); else TS_PLAIN_FEW(2, 1, 2, false);
+      TS_PLAIN_FEW(2, 1, 3);
       break;
     case FEW_2_2:
-      if (vec) TS_PLAIN_FEW(2, 2, 2, true); else TS_PLAIN_FEW(2, 2, 2, false);
+      TS_PLAIN_FEW(2, 2, 2);
       break;
     case TILES_64:
       if (vec) TS_PLAIN_TILED(1, 32, true); else TS_PLAIN_TILED(1, 32, false);
