@@ -373,6 +373,43 @@ def test_gemm_wide_rows_do_not_depend_on_the_batch_and_plans_fill_the_device(ops
     torch.testing.assert_close(ops.dense(sums, torch.bfloat16).float(), x[:200].float() @ w.float().t(), rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("tile", [1, 2])
+@pytest.mark.parametrize("m,n,k", [(1, 16, 8), (5, 33, 72), (16, 300, 128), (16, 1000, 520), (7, 2048, 2048), (3, 130, 4104), (9, 62, 1600)])
+def test_gemm_stream_every_tile_and_grid(ops, tile, m, n, k):
+    """One slice to more than the ring holds, wavefronts and ranges without any, a K and an N that end inside a slice and
+    a tile, rows of x apart with not-a-numbers between them, a row of weights that is none: the exact
+    product within k + 1 roundings of the terms' sizes, the gated result within bfloat16 rounding of
+    its operands', and a row's bits whatever stands beside it."""
+    g = torch.Generator().manual_seed(tile + n + k)
+    x = torch.full((m, k + 8), float("nan"), dtype=torch.bfloat16)
+    x[:, :k] = torch.randn(m, k, generator=g)
+    w = (torch.randn(n, k, generator=g) * 0.3).bfloat16()
+    b = torch.randn(n, generator=g).bfloat16()
+    want = x[:, :k].double() @ w.double().T + b.double()
+    bound = (k + 1) * 2.0**-24 * (x[:, :k].double().abs() @ w.double().abs().T + b.double().abs())
+    xd, wd, bd = x.to(DEV)[:, :k], w.to(DEV), b.to(DEV)
+    slices = -(-k // 64)
+    for per_wave in sorted({1, 2, 3, -(-slices // 4), -(-slices // 8), slices}):
+        plan = (per_wave, -(-slices // (4 * per_wave)), tile)
+        partial = ops.gemm_stream(xd, wd, bd, plan=plan)
+        assert partial.shape == (plan[1], m, n) and bool(((partial.double().sum(0).cpu() - want).abs() <= bound).all()), plan
+        assert torch.equal(ops.gemm_stream(xd[m // 2:], wd, bd, plan=plan), partial[:, m // 2:])
+    spoiled = wd.clone()
+    spoiled[n // 2] = float("nan")
+    got = ops.gemm_stream(xd, spoiled, bd, plan=plan)
+    assert bool(got[:, :, n // 2].isnan().all())
+    got[:, :, n // 2] = partial[:, :, n // 2]
+    assert torch.equal(got, partial)
+    if n % 2 == 0:
+        gate, up = want[:, 0::2], want[:, 1::2]
+        exact = gate * torch.sigmoid(gate) * up
+        slack = 2.0**-8 * exact.abs() + 1.2 * (bound[:, 0::2] + 2.0**-20 * gate.abs()) * up.abs() + (gate * torch.sigmoid(gate)).abs() * bound[:, 1::2] + 1e-30
+        fused = ops.gemm_stream(xd, wd, bd, plan=(-(-slices // 4), 1, tile), gated=True)
+        assert bool(((fused.double().cpu() - exact).abs() <= slack).all())
+    picked = ops.gemm_skinny(xd, wd, bd)  # a plan's grid covers K
+    assert bool(((picked.double().sum(0).cpu() - want).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("tn,tm", [(8, 8), (8, 6), (8, 5), (5, 10), (5, 8), (4, 8), (4, 5), (4, 4)])
 @pytest.mark.parametrize("m,n,k,splits", [(1, 16, 64, 1), (129, 272, 64, 1), (257, 48, 128, 2), (321, 528, 192, 3), (700, 1040, 448, 2)])
 def test_gemm_block_every_tile(ops, tn, tm, m, n, k, splits):

@@ -460,7 +460,7 @@ __device__ __forceinline__ void stream_ranges(lds_f32* __restrict__ to, const ld
 #pragma unroll
   for (int j = 0; j < 2 * MT; ++j) xoff[j] = ((uint32_t)(8 * j + row8) * (uint32_t)x_stride + start + 4 * (piece ^ (j & 1 ? 4 : 0))) * 4;
   auto fetch = [&](int i, int slot) __attribute__((always_inline)) {
-    const uint32_t at = (uint32_t)min(i, count - 1) * (SLICE * 4);  // past the end: the last slice again, never read
+    const uint32_t at = i < count ? (uint32_t)i * (SLICE * 4) : 0x80000000u;  // past the end: outside the buffers, nothing is fetched
     lds_f32* base = to + slot * (MT + NT) * TILE;
 #pragma unroll
     for (int j = 0; j < 2 * NT; ++j)

@@ -1,0 +1,228 @@
+// The product of a decode step of up to 16 rows, bound by reading the weights once:
+//   Y[m][n] = sum over k of X[m][k] * W[n][k]  (+ bias[n])
+// bfloat16 activations X [M, K] and weights W [N, K] as the checkpoint stores them (F.linear's
+// layout, src/turboserve/engine/model/layers.py:142), 32-bit accumulation on the matrix cores.
+//
+// A workgroup owns 16 NT weight rows and one of S ranges of K, each of its four wavefronts a quarter of the range.  A
+// wavefront stages its part in a ring of its own in LDS, SLOTS slices of 64 k, straight from memory: an instruction takes
+// whole lines, 128 bytes of each of eight rows, non-temporal for the weights, and a slot is filled again as
+// soon as its fragments are in registers.  Nothing meets at a barrier before the quarters' sums, and a small matrix is in
+// flight as a whole: what is left of such a product is one trip to memory.
+// Microseconds at one row, in a graph, against the tiled or the resident kernel (which read half lines, or hand the weights
+// through registers and meet at a barrier every 128 of K; with the SwiGLU where that is in the result): 2,048 x 2,048 4.4 -> 4.0, 2,048 x
+// 8,192 12.2 -> 7.7, 8,192 x 2,048 12.3 -> 7.3, q|k|v [4608, 3584] 8.6 -> 7.9, o [3584, 3584] 8.4 -> 6.2, down [3584, 18944]
+// 24.5 -> 22.0, gate|up [16384, 2048] 17.7 -> 13.4, [37888, 3584] 46.9 -> 41.0, the head [152064, 3584] 178 -> 153 (7.1 TB/s).
+#include "common.hpp"
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+
+constexpr int STREAM_WAVES = 4;
+
+template <int NT>
+struct Ring {
+  static constexpr int SLICE = 64, TILE = 16 * SLICE, LOADS = 2 * (NT + 1);  // of a tile of sixteen rows; of a slice
+  static constexpr int SLOTS = 80 * 1024 / (STREAM_WAVES * (NT + 1) * TILE * 2);  // two workgroups a compute unit
+  static constexpr int WAVE = SLOTS * (NT + 1) * TILE;                          // elements of a wavefront's ring
+  static constexpr size_t BYTES = (size_t)STREAM_WAVES * WAVE * 2;
+  static_assert(SLOTS >= 2 && (SLOTS - 1) * LOADS < 64 && 2 * BYTES <= 160 * 1024, "a ring of at least two slices, counted by vmcnt");
+  static_assert(WAVE * 2 >= NT * 1024, "a wavefront's sums fit its ring");
+};
+
+// `to` and `from` are the same memory: __restrict__ keeps the compiler from waiting for every load in flight before every
+// read, so it must not see that two reads have one address either: the slot that this wait lets be read is a new value to it.
+template <int LEFT>
+__device__ __forceinline__ void stream_wait(int& slot) {
+  asm volatile("s_waitcnt vmcnt(%1)" : "+s"(slot) : "n"(LEFT) : "memory");
+}
+
+// acc[t][i]: weight row n0 + 16 t + 4 (lane / 16) + i, activation row lane % 16, over slices first .. last - 1 of 64 k.
+template <int NT, int SLOTS>
+__device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, const uint16_t* __restrict__ x,
+                                             const uint16_t* __restrict__ w, int m, int n, int k, long x_stride, int n0, int first,
+                                             int last, f32x4* acc) {
+  typedef Ring<NT> R;
+  constexpr int SLICE = R::SLICE, TILE = R::TILE;
+  const int count = last - first;
+  if (count <= 0) return;
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  // A lane loads 16 bytes, piece (lane % 8) ^ key of row lane / 8 of eight, key = row / 2 % 8: a piece of sixteen rows
+  // touches every bank once.  (The second eight rows of a tile have keys four further on: piece ^ 4.)  What lies past the last
+  // row's end (rows beyond N or M) brings zeros, what lies past another row's end (a K that is no multiple of 64) is cleared.
+  const int row8 = lane >> 3, piece = (lane & 7) ^ (row8 >> 1);
+  const size_t wbytes = (size_t)min(n - n0, 16 * NT) * k * 2, xbytes = ((size_t)(m - 1) * x_stride + k) * 2;
+  const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w + (size_t)n0 * k), 0, (int)wbytes, 0x00027000);
+  const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, (int)xbytes, 0x00027000);
+  uint32_t woff[2 * NT], xoff[2];
+#pragma unroll
+  for (int j = 0; j < 2 * NT; ++j) woff[j] = ((uint32_t)(8 * j + row8) * (uint32_t)k + first * SLICE + 8 * (piece ^ (j & 1 ? 4 : 0))) * 2;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) xoff[j] = ((uint32_t)(8 * j + row8) * (uint32_t)x_stride + first * SLICE + 8 * (piece ^ (j & 1 ? 4 : 0))) * 2;
+  auto fetch = [&](int i, int slot) __attribute__((always_inline)) {
+    const uint32_t at = i < count ? (uint32_t)i * (SLICE * 2) : 0x80000000u;  // past the end: outside the buffers, nothing is fetched
+    lds_u16* base = to + slot * (NT + 1) * TILE;
+#pragma unroll
+    for (int j = 0; j < 2 * NT; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, base + j * (TILE / 2), 16, (int)(woff[j] + at), 0, 0, 2);  // non-temporal
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, base + NT * TILE + j * (TILE / 2), 16, (int)(xoff[j] + at), 0, 0, 0);
+  };
+  struct Frags {
+    u32x4 x[2], w[NT][2];
+  };
+  const int key = (r >> 1) & 7;
+  auto read = [&](Frags& f, int slot) __attribute__((always_inline)) {
+    const lds_u16* base = from + slot * (NT + 1) * TILE + r * SLICE;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int at = 8 * ((4 * c + g) ^ key);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) f.w[t][c] = *(const lds_u32x4*)(base + t * TILE + at);
+      f.x[c] = *(const lds_u32x4*)(base + NT * TILE + at);
+    }
+  };
+  auto consume = [&](Frags& f, int left) __attribute__((always_inline)) {  // left: elements of the slice inside the row
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const bool inside = left >= SLICE || 32 * c + 8 * g < left;  // a piece lies inside as a whole
+      const u32x4 none = {0u, 0u, 0u, 0u};
+      if (left < SLICE) f.x[c] = inside ? f.x[c] : none;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        if (left < SLICE) f.w[t][c] = inside ? f.w[t][c] : none;
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, f.w[t][c]), __builtin_bit_cast(bf16x8, f.x[c]), acc[t], 0, 0, 0);
+      }
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < SLOTS; ++j) fetch(j, j);
+  int slot = 0;
+  stream_wait<(SLOTS - 1) * R::LOADS>(slot);
+  Frags f[2];
+  read(f[0], slot);
+  auto round = [&](int i, Frags& now, Frags& next) __attribute__((always_inline)) {
+    // `now` is in registers: its slot is free.
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(now.w[t][c])::"memory");
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(now.x[c])::"memory");
+    }
+    fetch(i + SLOTS, slot);
+    slot = slot + 1 == SLOTS ? 0 : slot + 1;
+    stream_wait<(SLOTS - 1) * R::LOADS>(slot);
+    read(next, slot);
+    consume(now, SLICE);
+  };
+  int i = 0;  // the last slice alone may be cut short
+  for (; i + 2 < count; i += 2) {
+    round(i, f[0], f[1]);
+    round(i + 1, f[1], f[0]);
+  }
+  const int left = k - (last - 1) * SLICE;
+  if (i + 1 < count) {
+    round(i, f[0], f[1]);
+    consume(f[1], left);
+  } else {
+    consume(f[0], left);
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // loads past the end
+}
+
+// partial: float [splits, m, n], or, GATED, out: bfloat16 [m, n / 2], the gated unit (common.hpp) of rows that alternate gate, up.
+template <int NT, bool GATED>
+__global__ void __launch_bounds__(64 * STREAM_WAVES)
+gemm_stream_kernel(float* __restrict__ partial, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, long x_stride,
+                   const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int m, int n, int k, int per_wave, GluRule rule) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t ring[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * 16 * NT, split = blockIdx.y;
+  const int total = (k + Ring<NT>::SLICE - 1) / Ring<NT>::SLICE;
+  const int first = (split * STREAM_WAVES + wave) * per_wave, last = min(first + per_wave, total);
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  lds_u16* mine = (lds_u16*)ring + wave * Ring<NT>::WAVE;
+  stream_range<NT, Ring<NT>::SLOTS>(mine, mine, x, w, m, n, k, x_stride, n0, first, last, acc);
+  // The quarters' sums meet in the rings; wavefront v adds up and stores tile v.
+#pragma unroll
+  for (int t = 0; t < NT; ++t) ((lds_f32x4*)mine)[t * 64 + lane] = acc[t];
+  __syncthreads();
+  if (wave >= NT) return;
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int v = 0; v < STREAM_WAVES; ++v) sum += ((lds_f32x4*)((lds_u16*)ring + v * Ring<NT>::WAVE))[wave * 64 + lane];
+  const int row = lane & 15, col = n0 + 16 * wave + 4 * (lane >> 4);
+  if (row >= m || col >= n) return;
+  if (bias && split == 0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] += to_float(bf16_t{bias[min(col + i, n - 1)]});
+  }
+  if (GATED) {  // n is even: the first pair lies inside
+    uint16_t* at = out + (size_t)row * (n / 2) + col / 2;
+    at[0] = from_float<bf16_t>(gated_unit(sum[0], sum[1], rule)).bits;
+    if (col + 2 < n) at[1] = from_float<bf16_t>(gated_unit(sum[2], sum[3], rule)).bits;
+  } else {
+    float* at = partial + ((size_t)split * m + row) * n + col;
+    if (n % 4 == 0) {
+      *reinterpret_cast<f32x4*>(at) = sum;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (col + i < n) at[i] = sum[i];
+    }
+  }
+}
+
+template <int NT, bool GATED>
+int launch_stream(float* partial, void* out, const void* x, long x_stride, const void* w, const void* bias, int m, int n, int k,
+                  int per_wave, int splits, GluRule rule, hipStream_t stream) {
+  static bool raised = false;  // per process; the attribute belongs to the kernel
+  if (!raised) {
+    if (hipFuncSetAttribute((const void*)gemm_stream_kernel<NT, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)Ring<NT>::BYTES) != hipSuccess)
+      return TS_ERR_LAUNCH;
+    raised = true;
+  }
+  hipLaunchKernelGGL((gemm_stream_kernel<NT, GATED>), dim3((n + 16 * NT - 1) / (16 * NT), splits), dim3(64 * STREAM_WAVES),
+                     Ring<NT>::BYTES, stream, partial, (uint16_t*)out, (const uint16_t*)x, x_stride, (const uint16_t*)w,
+                     (const uint16_t*)bias, m, n, k, per_wave, rule);
+  return ts_launch_status();
+}
+
+}  // namespace
+
+// x [m, k] bfloat16 (m up to 16, k a multiple of 8) with row stride x_stride; w [n, k] bfloat16 contiguous; bias [n] bfloat16 or
+// null.  partial = float [splits, m, n], or out = bfloat16 [m, n / 2] (splits 1, n even): the gated unit of a w whose rows
+// alternate gate, up.  Slices of 64 of k: per_wave to each of the four wavefronts of each of `splits` =
+// ceil(ceil(k / 64) / (4 per_wave)) ranges.  tile: 1 or 2 (16 or 32 weight rows a workgroup).
+extern "C" int ts_gemm_stream(float* partial, void* out, const void* x, long x_stride, const void* w, const void* bias, int m,
+                              int n, int k, int per_wave, int splits, int tile, float steepness, float limit, float up_shift,
+                              float cubic, hipStream_t stream) {
+  if (m == 0 || n == 0) return TS_OK;
+  if (!x || !w || m < 0 || n < 0 || k < 8 || (partial == nullptr) == (out == nullptr)) return TS_ERR_ARG;
+  if (m > 16 || k % 8 != 0 || x_stride < k || x_stride % 8 != 0 || (uintptr_t)x % 16 != 0 || (uintptr_t)w % 16 != 0) return TS_ERR_SHAPE;
+  if (x_stride >= (1L << 24) || k >= (1 << 24)) return TS_ERR_SHAPE;  // a tile's rows lie within 31 bits of its first one
+  if (per_wave < 1 || splits < 1 || splits > 65535) return TS_ERR_SHAPE;
+  if (splits != ((k + 63) / 64 + 4L * per_wave - 1) / (4L * per_wave)) return TS_ERR_SHAPE;
+  if (out && (splits != 1 || n % 2 != 0)) return TS_ERR_ARG;
+  const GluRule rule = {steepness, limit, up_shift, cubic};
+#define TS_STREAM(NT, GATED) return launch_stream<NT, GATED>(partial, out, x, x_stride, w, bias, m, n, k, per_wave, splits, rule, stream)
+  if (tile == 1) {
+    if (out) TS_STREAM(1, true);
+    TS_STREAM(1, false);
+  }
+  if (tile == 2) {
+    if (out) TS_STREAM(2, true);
+    TS_STREAM(2, false);
+  }
+#undef TS_STREAM
+  return TS_ERR_SHAPE;
+}

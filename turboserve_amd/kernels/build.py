@@ -48,6 +48,7 @@ MODULES: dict[str, tuple[str, ...]] = {
         "attention_tiles.hip",
         "gemm_plain.hip",
         "gemm_skinny.hip",
+        "gemm_stream.hip",
         "gemm_tiled.hip",
         "gemm_wide.hip",
         "gemm_block.hip",

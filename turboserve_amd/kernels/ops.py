@@ -148,6 +148,8 @@ _SIGNATURES: dict[str, dict[str, list]] = {
                          c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_block": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                           c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
+        "ts_gemm_stream": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
+                           c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_skinny_resident": [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                     c_int, c_int, c_int, c_void_p],
         "ts_argmax": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p],
@@ -380,6 +382,7 @@ class Ops:
         self._raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         self._tiled_plans: dict[tuple, tuple[int, int, int]] = {}  # (m, n, k, max_splits) -> grid of the tiled product
         self._wide_plans: dict[tuple, tuple[int, int, int, int, int]] = {}  # (m, n, k, one range) -> grid of the wide product
+        self._stream_plans: dict[tuple, tuple[int, int, int] | None] = {}  # (n, k, max_splits) -> grid of the streaming product
         self._block_plans: dict[tuple, tuple[int, int, int, int]] = {}  # (m, n, k, kind) -> grid of the block product
         #: (rows a step's products run at, N, K, kind) -> whether this engine's own product was the
         #: faster one when both were timed (``time_wide_choices``).
@@ -2335,6 +2338,71 @@ class Ops:
                                       splits, tile, x_rows, waves, depth, 1, 1.0, 0.0, 0.0, 0.0, self.stream()), "ts_gemm_wide")
         return partial
 
+    def _stream_plan(self, n: int, k: int, max_splits: int | None) -> tuple[int, int, int] | None:
+        """(slices of 64 per wavefront, ranges of K, tile) of the streaming product: the fewest
+        ranges that keep the memory busy.  What a compute unit reads takes 36 bytes a nanosecond
+        where few units read and all of them together get 6.6 TB/s; a range more costs 0.12 us (its
+        sums, here and in the kernel that adds them up).  (us at one row: 3,584 x 3,584 as 1 / 2 / 4 ranges 8.1 / 6.2 / 7.2, 2,048 x
+        8,192 as 1 / 2 / 4 14 / 10 / 7.7, 8,192 x 2,048 as 1 / 2 7.3 / 7.6.)  None where one range
+        leaves the last round of workgroups so empty that the tiled product is as fast
+        (27,648 x 5,120 at eight rows 48 against 46 us; 37,888 x 3,584, a last round two thirds full, 41.7 against 43.9)."""
+        key = (n, k, max_splits)
+        if key in self._stream_plans:
+            return self._stream_plans[key]
+        slices, tiles, units = -(-k // 64), -(-n // 32), self.compute_units
+        best = None
+        for want in range(1, min(max_splits or 8, 8) + 1):
+            per_wave = -(-slices // (4 * want))
+            splits = -(-slices // (4 * per_wave))
+            if splits != want:
+                continue
+            rounds = -(-tiles * splits // units)
+            cost = max(2.0 * n * k / 6.6e6, rounds * 64.0 * k / splits / 36e3) + 0.12 * splits
+            if best is None or cost < best[0]:
+                best = (cost, per_wave, splits, 2)
+        plan = best[1:]
+        if max_splits == 1 and tiles > 2 * units and 10 * units * -(-tiles // units) > 11 * tiles:
+            plan = None
+        self._stream_plans[key] = plan
+        return plan
+
+    def _stream_runs(self, x: torch.Tensor, weight: torch.Tensor, max_splits: int | None) -> tuple[int, int, int] | None:
+        """The streaming product's grid where it runs a decode-sized product (up to 16 rows)."""
+        n, k = weight.shape
+        if (x.shape[0] > self.stream_max_rows or not 0 < k < 1 << 24 or n == 0 or x.stride(0) >= 1 << 24 or x.data_ptr() % 16 or weight.data_ptr() % 16
+                or x.stride(1) != 1 or not weight.is_contiguous()):
+            return None
+        return self._stream_plan(n, k, max_splits)
+
+    #: Decode-sized products of up to this many rows run the streaming kernel, one tile of activation rows.
+    stream_max_rows = 16
+
+    def gemm_stream(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, plan: tuple[int, int, int],
+                    gated: bool = False, rule: tuple[float, float, float] = (1.0, 0.0, 0.0)) -> torch.Tensor:
+        """``[S, M, N]`` 32-bit partial sums of ``x [M, K] @ weight [N, K]^T`` over ``S`` ranges of
+        K (bias in the first) by the kernel that streams whole lines of the weights through LDS
+        (``csrc/gemm_stream.hip``): M up to 16, K a multiple of 8.  ``plan`` as
+        :meth:`_stream_plan` gives it; ``gated`` as :meth:`gemm_tiled`'s."""
+        _gpu(x, weight, bias)
+        _need(x.dim() == 2 and x.stride(1) == 1 and weight.dim() == 2 and weight.is_contiguous()
+              and x.shape[1] == weight.shape[1], "x must be [M, K] with unit inner stride, weight contiguous [N, K]")
+        _need(self.skinny_supported(x, weight) and x.shape[0] <= self.stream_max_rows, "the streaming product takes bfloat16, M <= 16 and K % 8 == 0")
+        m, k = x.shape
+        n = weight.shape[0]
+        if bias is not None:
+            _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous(), "bias must be bfloat16 [N]")
+        per_wave, splits, tile = plan
+        x_stride = x.stride(0) if m > 1 else max(k, x.stride(0))
+        partial = out = None
+        if gated:
+            _need(splits == 1 and n % 2 == 0, "the gated result needs one range of K and an even number of weight rows")
+            out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
+        else:
+            partial = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+        _check(self.core.ts_gemm_stream(_ptr(partial), _ptr(out), _ptr(x), x_stride, _ptr(weight), _ptr(bias), m, n, k, per_wave,
+                                        splits, tile, *glu_rule(rule), self.stream()), "ts_gemm_stream")
+        return out if gated else partial
+
     def gemm_resident(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
                       *, max_splits: int | None = None) -> torch.Tensor:
         """The same partial sums by the kernel that keeps a split's activations resident in LDS and
@@ -2360,10 +2428,13 @@ class Ops:
     def gemm_skinny(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
                     *, max_splits: int | None = None) -> torch.Tensor:
         """``[S, M, N]`` 32-bit partial sums of ``x [M, K] @ weight [N, K]^T`` over ``S`` ranges of
-        K (bias in the first); their sum over ``S`` is the product.  For decode-sized ``M``: the
-        tiled kernel, except for up to 16 rows against a small matrix (the resident kernel's
-        many small workgroups start faster)."""
+        K (bias in the first); their sum over ``S`` is the product.  For decode-sized ``M``: up to 16
+        rows the streaming kernel (``_stream_plan`` says where not), else the tiled or the wide
+        one; operands that are not 16-byte aligned go to the tiled or the resident one."""
         m, (n, k) = x.shape[0], weight.shape
+        stream = self._stream_runs(x, weight, max_splits)
+        if stream is not None:
+            return self.gemm_stream(x, weight, bias, plan=stream)
         if self._resident_runs(m, n, k):
             return self.gemm_resident(x, weight, bias, max_splits=max_splits)
         if self._few_rows_wide(m, n, k, max_splits):
@@ -2534,6 +2605,9 @@ class Ops:
                     and weight.is_contiguous() and x.stride(1) == 1):
                 wide = self._wide_plan_few_rows(x.shape[0], weight.shape[0], weight.shape[1], 1)
                 return self.gemm_wide(x, weight, bias, plan=wide, gated=True, rule=rule)
+            stream = self._stream_runs(x, weight, 1) if weight.shape[0] % 2 == 0 else None
+            if stream is not None:
+                return self.gemm_stream(x, weight, bias, plan=stream, gated=True, rule=rule)
             plan = self._tiled_plan(x.shape[0], weight.shape[0], weight.shape[1], None)
             if plan[1] == 1 and weight.shape[0] % 2 == 0 and weight.is_contiguous() and x.stride(1) == 1:
                 return self.gemm_tiled(x, weight, bias, plan=plan, gated=True, rule=rule)
