@@ -410,8 +410,9 @@ def test_gemm_stream_every_tile_and_grid(ops, tile, m, n, k):
     assert bool(((picked.double().sum(0).cpu() - want).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("tn,tm", [(8, 8), (8, 6), (8, 5), (5, 10), (5, 8), (4, 8), (4, 5), (4, 4)])
-@pytest.mark.parametrize("m,n,k,splits", [(1, 16, 64, 1), (129, 272, 64, 1), (257, 48, 128, 2), (321, 528, 192, 3), (700, 1040, 448, 2)])
+@pytest.mark.parametrize("tn,tm", [(8, 8), (8, 6), (8, 5), (5, 10), (5, 8), (4, 8), (4, 5), (4, 4)] + [(a, b) for b in (1, 2) for a in (8, 5, 4, 2)]
+                         + [(8, 4), (5, 4), (2, 4)])
+@pytest.mark.parametrize("m,n,k,splits", [(1, 16, 64, 1), (17, 304, 448, 3), (33, 272, 128, 2), (65, 1040, 192, 1), (128, 528, 320, 5), (129, 272, 64, 1), (257, 48, 128, 2), (321, 528, 192, 3), (700, 1040, 448, 2)])
 def test_gemm_block_every_tile(ops, tn, tm, m, n, k, splits):
     """Blocks of the largest product, one tile short and one over in both directions, ranges of K
     of one to seven iterations, rows of x apart, a bias, the three results and rules of the gated unit; against
@@ -420,6 +421,8 @@ def test_gemm_block_every_tile(ops, tn, tm, m, n, k, splits):
     gated one what the unit makes of its operands' bounds (its slope in the gate stays below 1.2 for these rules)."""
     from turboserve_amd.kernels.ops import GELU_TANH_RULE
 
+    if m > 32 * tm and (tm < 4 or (tn, tm) in ((8, 4), (5, 4), (2, 4))):
+        pytest.skip("one tile of activation rows here")
     g = torch.Generator().manual_seed(100 * tn + tm + m)
     x = torch.randn(m, k + 8, generator=g).bfloat16()[:, :k]
     w = (torch.randn(n, k, generator=g) * 0.3).bfloat16()
@@ -451,7 +454,8 @@ def test_gemm_block_every_tile(ops, tn, tm, m, n, k, splits):
     assert torch.equal(ops.gemm_block(xd[m // 2:], wd, bd, plan=(iters, 1, tn, tm)), one[m // 2:])
 
 
-@pytest.mark.parametrize("m,n,k,offset", [(129, 16, 64, 0), (300, 2064, 1088, 0), (200, 500, 264, 0), (200, 512, 264, 0), (200, 520, 256, 0),
+@pytest.mark.parametrize("m,n,k,offset", [(17, 4608, 3584, 0), (32, 2048, 2048, 0), (33, 2064, 576, 0), (64, 512, 64, 0), (65, 528, 640, 0), (128, 272, 1088, 4),
+                                          (100, 1000, 264, 0), (129, 16, 64, 0), (300, 2064, 1088, 0), (200, 500, 264, 0), (200, 512, 264, 0), (200, 520, 256, 0),
                                           (200, 512, 256, 4), (150, 256, 192, 0)])
 def test_products_of_many_rows_agree_whichever_kernel_takes_them(ops, m, n, k, offset):
     """The block product runs what it takes (K % 64, N % 16, 16-byte rows) and the wide one the rest;
@@ -462,13 +466,18 @@ def test_products_of_many_rows_agree_whichever_kernel_takes_them(ops, m, n, k, o
     w = (torch.randn(n, k, generator=g) / k**0.5).bfloat16().to(DEV)
     takes = k % 64 == 0 and n % 16 == 0 and offset % 8 == 0
     assert ops.block_supported(x, w) == takes
-    if takes:
+    if takes and m <= 128:
+        for most in (None, 1, 3):
+            plan = ops._block_few_plan(m, n, k, most)
+            assert plan is None or plan[1] == -(-(k // 64) // plan[0]) <= (most or 12)
+    elif takes:
         for kind in ("sums", "one", "gated"):
             per_split, splits, tn, tm = ops._block_plan(m, n, k, kind)
             assert splits == -(-(k // 64) // per_split) and (kind == "sums" or splits == 1)
     want = x.double() @ w.double().T
     bound = 2.0**-7 * want.abs() + (k + 1) * 2.0**-24 * (x.double().abs() @ w.double().abs().T)
-    assert bool(((ops.linear(x, w).double() - want).abs() <= bound).all())
+    assert bool(((ops.dense(ops.linear(x, w), torch.bfloat16).double() - want).abs() <= bound).all())
+    assert bool(((ops.linear_float32_out(x, w).double() - want).abs() <= bound).all())
     sums = ops.linear(x, w, for_residual=True)
     assert bool(((ops.dense(sums, torch.bfloat16).double() - want).abs() <= bound).all())
     gated = torch.nn.functional.silu(want[:, 0::2]) * want[:, 1::2]

@@ -1,5 +1,5 @@
-// The product of a prompt's step (more rows than a decode step has), in blocks as large as a wavefront's
-// registers take:
+// The product of a prompt's step, in blocks as large as a wavefront's registers take, and of a decode step of 17 to 128 rows,
+// one tile of activation rows:
 //   Y[m][n] = sum over k of X[m][k] * W[n][k]  (+ bias[n])
 // bfloat16 activations X [M, K] and weights W [N, K] as the checkpoint stores them (F.linear's
 // layout, src/turboserve/engine/model/layers.py:142), 32-bit accumulation on the matrix cores.
@@ -24,6 +24,9 @@
 // against 35 / 34 / 77, q|k|v [4608, 3584] 27 / 28 / 59 against 23 / 31 / 62.  An iteration of 256 x 256 takes 1.15 us where
 // half the compute units have a workgroup and 1.4 where all do (the matrix instructions 0.85 at the full clock); a
 // workgroup's start takes 2 us and its stores 4.
+// A decode step's product is bound by reading the weights; 160 weight rows by 64 activation rows a workgroup, the weights
+// non-temporal, take gate|up at 64 rows in 44.1 us (gemm_wide 47.5), 128 rows down in 26.6 (28.6), q|k|v in 11.5 (12.0), o in 10.4
+// (11.1); at 128 rows 50 (60), 33 (37), 14.5 (15.3), 13.7 (14.1).
 #include "common.hpp"
 
 namespace {
@@ -106,7 +109,7 @@ typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 // every read.  What orders them is block_wait, which no access crosses.
 // out: bfloat16 [m, n] (mode 0), partial: float [splits, m, n] (mode 1), out: bfloat16 [m, n / 2] (mode 2; 3: any rule
 // of the gated unit.  Two kernels: with both epilogues behind one loop the compiler moved the sums between registers in it).
-template <int TN, int TM, int MODE>
+template <int TN, int TM, int MODE, bool ONCE>
 __device__ __forceinline__ void
 gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __restrict__ partial, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, long x_stride,
                   const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int m, int n, int k,
@@ -142,7 +145,8 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   // the first against the size less the second, which is never below 0.
   int woff = (row0 * k + 8 * piece) * 2, xoff = (row0 * (int)x_stride + 8 * piece) * 2;
   auto load_w = [&](int j, int it, int slot) __attribute__((always_inline)) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, to + (slot * NT + 32 * j + 8 * wave) * ROW, 16, woff + j * 64 * k, it * (BLOCK_DEPTH * 2), 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, to + (slot * NT + 32 * j + 8 * wave) * ROW, 16, woff + j * 64 * k, it * (BLOCK_DEPTH * 2), 0,
+                                             ONCE ? 2 : 0);  // non-temporal where one tile of activation rows reads them
   };
   auto load_x = [&](int j, int it, int slot) __attribute__((always_inline)) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, to + (RW * NT + slot * XR + 32 * j + 8 * wave) * ROW, 16, xoff + j * 64 * (int)x_stride, it * (BLOCK_DEPTH * 2),
@@ -322,24 +326,24 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   }
 }
 
-template <int TN, int TM, int MODE>
+template <int TN, int TM, int MODE, bool ONCE>
 __global__ void __launch_bounds__(256, 1)
 gemm_block_kernel(float* __restrict__ partial, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, long x_stride,
                   const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int m, int n, int k,
                   int iters_per_split, int splits, int n_tiles, int m_tiles, GluRule rule) {
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];  // the rings: weight rows, activation rows
-  gemm_block<TN, TM, MODE>((lds_u16*)lds, (const lds_u16*)lds, partial, out, x, x_stride, w, bias, m, n, k, iters_per_split,
+  gemm_block<TN, TM, MODE, ONCE>((lds_u16*)lds, (const lds_u16*)lds, partial, out, x, x_stride, w, bias, m, n, k, iters_per_split,
                                  splits, n_tiles, m_tiles, rule);
 }
 
-template <int TN, int TM, int MODE>
+template <int TN, int TM, int MODE, bool ONCE>
 int launch_block_kernel(float* partial, uint16_t* out, const uint16_t* x, long x_stride, const uint16_t* w, const uint16_t* bias,
                         int m, int n, int k, int iters_per_split, int splits, GluRule rule, hipStream_t stream) {
   constexpr int NT = 32 * TN, XR = 32 * TM;
   constexpr size_t lds_bytes = BlockRing<TN, TM>::BYTES;
   static bool raised = false;  // per process; the attribute belongs to the kernel
   if (!raised) {
-    if (hipFuncSetAttribute((const void*)gemm_block_kernel<TN, TM, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute((const void*)gemm_block_kernel<TN, TM, MODE, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds_bytes) != hipSuccess)
       return TS_ERR_LAUNCH;
     raised = true;
@@ -348,7 +352,7 @@ int launch_block_kernel(float* partial, uint16_t* out, const uint16_t* x, long x
   const long units = (long)n_tiles * splits;
   const long ids = (units * m_tiles + BLOCK_DIES - 1) / BLOCK_DIES * BLOCK_DIES;
   if (ids > 0x7fffffffL) return TS_ERR_SHAPE;
-  hipLaunchKernelGGL((gemm_block_kernel<TN, TM, MODE>), dim3((unsigned)ids), dim3(256), lds_bytes, stream, partial, out, x,
+  hipLaunchKernelGGL((gemm_block_kernel<TN, TM, MODE, ONCE>), dim3((unsigned)ids), dim3(256), lds_bytes, stream, partial, out, x,
                      x_stride, w, bias, m, n, k, iters_per_split, splits, n_tiles, m_tiles, rule);
   return ts_launch_status();
 }
@@ -375,24 +379,38 @@ extern "C" int ts_gemm_block(float* partial, void* out, const void* x, long x_st
   if (mode != 1 && splits != 1) return TS_ERR_ARG;
   const GluRule rule = {steepness, limit, up_shift, cubic};
   const bool plain = limit <= 0.f && cubic == 0.f;
-#define TS_BLOCK_MODE(TN, TM, MODE)                                                                                          \
-  return launch_block_kernel<TN, TM, MODE>(partial, (uint16_t*)out, (const uint16_t*)x, x_stride, (const uint16_t*)w,        \
-                                           (const uint16_t*)bias, m, n, k, iters_per_split, splits, rule, stream)
-#define TS_BLOCK(TN, TM)                       \
-  if (tn == TN && tm == TM) {                  \
-    if (mode == 0) TS_BLOCK_MODE(TN, TM, 0);   \
-    if (mode == 1) TS_BLOCK_MODE(TN, TM, 1);   \
-    if (plain) TS_BLOCK_MODE(TN, TM, 2);       \
-    TS_BLOCK_MODE(TN, TM, 3);                  \
+#define TS_BLOCK_MODE(TN, TM, MODE, ONCE)                                                                                    \
+  return launch_block_kernel<TN, TM, MODE, ONCE>(partial, (uint16_t*)out, (const uint16_t*)x, x_stride, (const uint16_t*)w,  \
+                                                 (const uint16_t*)bias, m, n, k, iters_per_split, splits, rule, stream)
+#define TS_BLOCK(TN, TM, ONCE)                       \
+  if (tn == TN && tm == TM && once == ONCE) {        \
+    if (mode == 0) TS_BLOCK_MODE(TN, TM, 0, ONCE);   \
+    if (mode == 1) TS_BLOCK_MODE(TN, TM, 1, ONCE);   \
+    if (plain) TS_BLOCK_MODE(TN, TM, 2, ONCE);       \
+    TS_BLOCK_MODE(TN, TM, 3, ONCE);                  \
   }
-  TS_BLOCK(8, 8)
-  TS_BLOCK(8, 6)
-  TS_BLOCK(8, 5)
-  TS_BLOCK(5, 10)
-  TS_BLOCK(5, 8)
-  TS_BLOCK(4, 8)
-  TS_BLOCK(4, 5)
-  TS_BLOCK(4, 4)
+  const bool once = m <= 32 * tm && tm <= 4;
+  TS_BLOCK(8, 8, false)
+  TS_BLOCK(8, 6, false)
+  TS_BLOCK(8, 5, false)
+  TS_BLOCK(5, 10, false)
+  TS_BLOCK(5, 8, false)
+  TS_BLOCK(4, 8, false)
+  TS_BLOCK(4, 5, false)
+  TS_BLOCK(4, 4, false)
+  // A decode step's rows: one tile of them.
+  TS_BLOCK(8, 1, true)
+  TS_BLOCK(5, 1, true)
+  TS_BLOCK(4, 1, true)
+  TS_BLOCK(2, 1, true)
+  TS_BLOCK(8, 2, true)
+  TS_BLOCK(5, 2, true)
+  TS_BLOCK(4, 2, true)
+  TS_BLOCK(2, 2, true)
+  TS_BLOCK(8, 4, true)
+  TS_BLOCK(5, 4, true)
+  TS_BLOCK(4, 4, true)
+  TS_BLOCK(2, 4, true)
 #undef TS_BLOCK
 #undef TS_BLOCK_MODE
   return TS_ERR_SHAPE;

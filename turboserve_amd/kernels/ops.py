@@ -383,7 +383,7 @@ class Ops:
         self._tiled_plans: dict[tuple, tuple[int, int, int]] = {}  # (m, n, k, max_splits) -> grid of the tiled product
         self._wide_plans: dict[tuple, tuple[int, int, int, int, int]] = {}  # (m, n, k, one range) -> grid of the wide product
         self._stream_plans: dict[tuple, tuple[int, int, int] | None] = {}  # (n, k, max_splits) -> grid of the streaming product
-        self._block_plans: dict[tuple, tuple[int, int, int, int]] = {}  # (m, n, k, kind) -> grid of the block product
+        self._block_plans: dict[tuple, tuple[int, int, int, int] | None] = {}  # (m, n, k, kind) -> grid of the block product
         #: (rows a step's products run at, N, K, kind) -> whether this engine's own product was the
         #: faster one when both were timed (``time_wide_choices``).
         self.wide_choices: dict[tuple, bool] = {}
@@ -2178,6 +2178,36 @@ class Ops:
         self._block_plans[key] = best[1:]
         return best[1:]
 
+    #: What an iteration of 64 of K takes with one tile of activation rows, one workgroup a compute unit, by tile of weight
+    #: rows, in microseconds (at 64 rows; 16,384 to 152,064 weight rows).
+    _BLOCK_ONE_RANGE = {2: 0.50, 4: 0.66, 5: 0.72, 8: 0.93}
+
+    def _block_few_plan(self, m: int, n: int, k: int, max_splits: int | None) -> tuple[int, int, int, int] | None:
+        """The block product's grid for a decode step of 17 to 128 rows, or None where ``gemm_wide``
+        stays: one tile of activation rows.  As one range of K the tile of weight rows whose rounds
+        of workgroups are over first, if its last round is nine tenths full or the rows are more
+        than 64 (at 64 rows 27,648 x 5,120, 216 workgroups, 56 against 55 us; 37,888 x 3,584, 237, 44
+        against 47.5; at 128 rows 70 against 77 and 50 against 60); else tiles of 128 weight rows
+        and as many ranges as give every compute unit a workgroup, of six iterations at least,
+        or tiles of 64 where that would be fewer (2,048 x 2,048 at 64 rows 6.1 against 7.5)."""
+        key = (m, n, k, max_splits)
+        if key in self._block_plans:
+            return self._block_plans[key]
+        units, iters, tm = self.compute_units, k // 64, 1 if m <= 32 else 2 if m <= 64 else 4
+        if max_splits == 1:
+            tn = min(self._BLOCK_ONE_RANGE, key=lambda t: -(-(-(-n // (32 * t))) // units) * self._BLOCK_ONE_RANGE[t])
+            workgroups = -(-n // (32 * tn))
+            filled = m > 64 or 10 * workgroups >= 9 * units * -(-workgroups // units)
+            plan = (iters, 1, tn, tm) if filled else None
+        else:
+            tn, want = 4, max(1, min(12, max_splits or 12, units // -(-n // 128)))
+            if iters // want < 6:
+                tn, want = 2, max(1, min(12, max_splits or 12, units // -(-n // 64)))
+            per_split = -(-iters // min(want, iters))
+            plan = (per_split, -(-iters // per_split), tn, tm)
+        self._block_plans[key] = plan
+        return plan
+
     def gemm_block(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *,
                    plan: tuple[int, int, int, int], gated: bool = False, sums: bool = False,
                    rule: tuple[float, float, float] = (1.0, 0.0, 0.0)) -> torch.Tensor:
@@ -2429,17 +2459,29 @@ class Ops:
                     *, max_splits: int | None = None) -> torch.Tensor:
         """``[S, M, N]`` 32-bit partial sums of ``x [M, K] @ weight [N, K]^T`` over ``S`` ranges of
         K (bias in the first); their sum over ``S`` is the product.  For decode-sized ``M``: up to 16
-        rows the streaming kernel (``_stream_plan`` says where not), else the tiled or the wide
-        one; operands that are not 16-byte aligned go to the tiled or the resident one."""
+        rows the streaming kernel (``_stream_plan`` says where not), above the block product
+        (``_block_few_plan``), else the tiled or the wide one; operands that are not 16-byte aligned go to the tiled or the resident one."""
         m, (n, k) = x.shape[0], weight.shape
         stream = self._stream_runs(x, weight, max_splits)
         if stream is not None:
             return self.gemm_stream(x, weight, bias, plan=stream)
         if self._resident_runs(m, n, k):
             return self.gemm_resident(x, weight, bias, max_splits=max_splits)
+        block = self._block_few_runs(x, weight, bias, max_splits)
+        if block is not None:
+            return self.gemm_block(x, weight, bias, plan=block, sums=True)
         if self._few_rows_wide(m, n, k, max_splits):
             return self.gemm_wide(x, weight, bias, plan=self._wide_plan_few_rows(m, n, k, max_splits), sums=True)
         return self.gemm_tiled(x, weight, bias, max_splits=max_splits)
+
+    def _block_few_runs(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
+                        max_splits: int | None) -> tuple[int, int, int, int] | None:
+        """The block product's grid where it runs a decode-sized product (17 to 128 rows)."""
+        if not self.stream_max_rows < x.shape[0] <= self.skinny_max_rows or not self.block_supported(x, weight):
+            return None
+        if bias is not None and bias.data_ptr() % 8:
+            return None
+        return self._block_few_plan(x.shape[0], weight.shape[0], weight.shape[1], max_splits)
 
     def _few_rows_wide(self, m: int, n: int, k: int, max_splits: int | None) -> bool:
         """Whether a decode-sized product runs the kernel of the steps of many rows
@@ -2601,6 +2643,9 @@ class Ops:
         rule = (1.0, 0.0, 0.0) if rule is None else tuple(float(v) for v in rule)
         if x.dtype == torch.bfloat16 and self.skinny_supported(x, weight) and x.shape[0] <= self.skinny_max_rows:
             _gpu(x, weight, bias)
+            block = self._block_few_runs(x, weight, bias, 1)
+            if block is not None:
+                return self.gemm_block(x, weight, bias, plan=block, gated=True, rule=rule)
             if (self._few_rows_wide(x.shape[0], weight.shape[0], weight.shape[1], 1) and weight.shape[0] % 2 == 0
                     and weight.is_contiguous() and x.stride(1) == 1):
                 wide = self._wide_plan_few_rows(x.shape[0], weight.shape[0], weight.shape[1], 1)
