@@ -10,13 +10,12 @@
 // cycle (a wavefront alone 30), writes from registers 30 whatever their width, global memory straight to LDS
 // 58.  A block of 256 x 256 reads 128 KB and writes 64 KB per 64 of K, in which its matrix instructions take 2,048
 // cycles: written from registers the 64 KB alone are 2,186, so operands go from global memory straight to LDS
-// (buffer loads with an LDS destination), into rings of three iterations' weight rows and two or three iterations'
-// activation rows, and 64 of K deep because a row of less than a 128-byte line is fetched twice (32 deep: 1.74 against
+// (buffer loads with an LDS destination), into rings of three to six iterations, and 64 of K deep because a row of less than a 128-byte line is fetched twice (32 deep: 1.74 against
 // 0.85 ms at 8,192 x 8,192 x 8,192).
 // With one wavefront on a SIMD nothing hides its waits, so nothing waits: a step's activation fragments are
 // read from LDS during the step before it, its weight fragments a tile's instructions after the last use of
 // their registers, and the first ones of the next iteration behind the barrier that ends this one's reads,
-// while most of its second step is still to be multiplied; loads are issued two iterations ahead, one beside each tile's
+// while most of its second step is still to be multiplied; loads are issued two to five iterations ahead, one beside each tile's
 // instructions (issued in one go they held the matrix instructions up).
 // Measured, microseconds, against the better of gemm_wide and the library's default kernel (with the kernel that reads or
 // makes the result: SwiGLU, or the norm that takes the partial sums), at 299 / 509 / 2,048 rows: gate|up [37888, 3584] 81 / 124 /
@@ -90,15 +89,17 @@ __device__ __forceinline__ void block_wait() {
   asm volatile("" ::: "memory");
 }
 
-// LDS holds three iterations' weight rows and two or, where they fit, three iterations' activation rows (1,280 rows of 128
-// bytes in all).  LEFT: loads that may be on their way when the next iteration must have landed.
+// LDS (1,280 rows of 128 bytes) holds W iterations' weight rows and X = W or W - 1 iterations' activation rows: three for the
+// largest blocks, up to six for small ones, whose iterations are shorter than a trip to memory.  LEFT: loads that may be on
+// their way when the next iteration must have landed.
 template <int TN, int TM>
 struct BlockRing {
   static constexpr int ROWS = 160 * 1024 / (BLOCK_DEPTH * 2);
-  static constexpr int W = 3, X = 32 * 3 * (TN + TM) <= ROWS ? 3 : 2;
-  static constexpr int LEFT = TN + (X - 2) * TM;
+  static constexpr bool fits(int w, int x) { return 32 * (w * TN + x * TM) <= ROWS; }
+  static constexpr int W = fits(6, 5) ? 6 : fits(5, 4) ? 5 : fits(4, 3) ? 4 : 3, X = fits(W, W) ? W : W - 1;
+  static constexpr int LEFT = (W - 2) * TN + (X - 2) * TM;
   static constexpr size_t BYTES = (size_t)32 * (W * TN + X * TM) * BLOCK_DEPTH * 2;
-  static_assert(BYTES <= 160 * 1024, "the rings must fit the LDS of a compute unit");
+  static_assert(fits(W, X) && LEFT + TM < 64, "the rings must fit the LDS of a compute unit, their loads vmcnt");
 };
 
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
@@ -144,12 +145,12 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   // A row's place is in the lane's offset, the place in K in the wavefront's: what is compared with the buffer's size is
   // the first against the size less the second, which is never below 0.
   int woff = (row0 * k + 8 * piece) * 2, xoff = (row0 * (int)x_stride + 8 * piece) * 2;
-  auto load_w = [&](int j, int it, int slot) __attribute__((always_inline)) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, to + (slot * NT + 32 * j + 8 * wave) * ROW, 16, woff + j * 64 * k, it * (BLOCK_DEPTH * 2), 0,
+  auto load_w = [&](int j, int off, int it, int slot) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, to + (slot * NT + 32 * j + 8 * wave) * ROW, 16, off + j * 64 * k, it * (BLOCK_DEPTH * 2), 0,
                                              ONCE ? 2 : 0);  // non-temporal where one tile of activation rows reads them
   };
-  auto load_x = [&](int j, int it, int slot) __attribute__((always_inline)) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, to + (RW * NT + slot * XR + 32 * j + 8 * wave) * ROW, 16, xoff + j * 64 * (int)x_stride, it * (BLOCK_DEPTH * 2),
+  auto load_x = [&](int j, int off, int it, int slot) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, to + (RW * NT + slot * XR + 32 * j + 8 * wave) * ROW, 16, off + j * 64 * (int)x_stride, it * (BLOCK_DEPTH * 2),
                                              0, 0);
   };
 
@@ -189,16 +190,17 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
 
   // Iteration i of the range: its weight rows lie in slot i % RW of their ring, its activation rows in slot i % RX of theirs.
   const int count = last - first;
-  auto step = [&](int i) __attribute__((always_inline)) { return first + min(i, count - 1); };  // past the end: the last one again, never read
+  auto step = [&](int i) __attribute__((always_inline)) { return first + min(i, count - 1); };
+  const int outside = (int)0x80000000;  // past every buffer's end: nothing is fetched for an iteration past the range's
 #pragma unroll
   for (int s = 0; s < RX; ++s) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-      if (s < 2) load_w(j, step(s), s);
+      if (s < RW - 1) load_w(j, s < count ? woff : outside, step(s), s);
 #pragma unroll
-    for (int j = 0; j < TM; ++j) load_x(j, step(s), s);
+    for (int j = 0; j < TM; ++j) load_x(j, s < count ? xoff : outside, step(s), s);
   }
-  block_wait<TN + (RX - 1) * TM>();
+  block_wait<Ring::LEFT + TM>();
 #pragma unroll
   for (int b = 0; b < TM; ++b) xf[0][b] = read_x(0, 0, b);
 #pragma unroll
@@ -215,12 +217,13 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   for (int it = 0; it < count; ++it) {
     // The offsets of the other rows are added up in each iteration: kept, they would take registers that the sums need.
     asm volatile("" : "+v"(woff), "+v"(xoff));
-    const int next_w = step(it + 2), next_x = step(it + RX);
-    const int free_w = ws == 0 ? 2 : ws - 1, free_x = xs;
+    const int next_w = step(it + RW - 1), next_x = step(it + RX);
+    const int from_w_at = it + RW - 1 < count ? woff : outside, from_x_at = it + RX < count ? xoff : outside;
+    const int free_w = ws == 0 ? RW - 1 : ws - 1, free_x = xs;
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
       TS_PIN;
-      load_w(a, next_w, free_w);
+      load_w(a, from_w_at, next_w, free_w);
       TS_PIN;
       tile(0, a, 0, TM / 2);
       TS_PIN;
@@ -253,7 +256,7 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
           else xf[0][j - FREE] = read_x(xs, 0, j - FREE);
         }
 #pragma unroll
-        for (int j = (a - FREE) * TM / (TN - FREE); j < (a - FREE + 1) * TM / (TN - FREE); ++j) load_x(j, next_x, free_x);
+        for (int j = (a - FREE) * TM / (TN - FREE); j < (a - FREE + 1) * TM / (TN - FREE); ++j) load_x(j, from_x_at, next_x, free_x);
       }
       TS_PIN;
       tile(1, a, 0, TM);
