@@ -454,6 +454,35 @@ def test_gemm_block_every_tile(ops, tn, tm, m, n, k, splits):
     assert torch.equal(ops.gemm_block(xd[m // 2:], wd, bd, plan=(iters, 1, tn, tm)), one[m // 2:])
 
 
+@pytest.mark.parametrize("m,tn,tm", [(1, 8, 8), (20, 5, 1), (257, 4, 5)])
+def test_gemm_block_gates_of_every_size(ops, m, tn, tm):
+    """silu of every bfloat16 gate from -88.5 (below it expf of its negative is infinite) to 88.5, through a product whose
+    terms beside the gate are zeros: half a unit of bfloat16 (2^-8 of the value) and the 32-bit unit's own few
+    roundings, down to gates whose result is as small as 1e-37, and the bits of the kernel that makes the units of a
+    stored product; beyond, the limits, and NaN stays NaN."""
+    bits = torch.arange(0, 0x42b2, dtype=torch.int32)  # 0 .. 88.5 and, with the sign's bit, 0 .. -88.5
+    gates = torch.cat([bits, bits | 0x8000]).to(torch.int16).view(torch.bfloat16)
+    edges = torch.tensor([-1e4, 1e4, -float("inf"), float("inf"), float("nan")], dtype=torch.bfloat16)
+    pad = torch.zeros(-(gates.numel() + edges.numel()) % 16, dtype=torch.bfloat16)
+    column = torch.cat([gates, edges, pad])
+    w = torch.zeros(2 * column.numel(), 64, dtype=torch.bfloat16)
+    w[0::2, 0], w[1::2, 1] = column, 1.0
+    x = torch.zeros(m, 64, dtype=torch.bfloat16)
+    x[:, 0:2] = 1.0
+    got = ops.gemm_block(x.to(DEV), w.to(DEV), plan=(1, 1, tn, tm), gated=True)
+    stored = ops.swiglu(ops.gemm_block(x.to(DEV), w.to(DEV), plan=(1, 1, tn, tm), sums=True), torch.bfloat16, paired=True)
+    assert torch.equal(got.view(torch.int16)[:, : gates.numel()], stored.view(torch.int16)[:, : gates.numel()])
+    got = got.double().cpu()
+    want = gates.double() * torch.sigmoid(gates.double())
+    normal = want.abs() >= 2.0**-126  # smaller results lose bits in any 32-bit unit
+    count = gates.numel()
+    assert bool(((got[:, :count] - want).abs() <= (2.0**-8 + 2.0**-20) * want.abs())[:, normal].all())
+    assert bool((got[:, :count] - want).abs()[:, ~normal].max() <= 2.0**-126)
+    low, high, lowest, highest, none = got[:, count: count + 5].unbind(1)
+    assert bool((low == 0).all() and (high == edges[1].double()).all() and (highest == float("inf")).all())
+    assert bool(lowest.isnan().all() and none.isnan().all())  # as -inf / (1 + expf(inf)) is
+
+
 @pytest.mark.parametrize("m,n,k,offset", [(17, 4608, 3584, 0), (32, 2048, 2048, 0), (33, 2064, 576, 0), (64, 512, 64, 0), (65, 528, 640, 0), (128, 272, 1088, 4),
                                           (100, 1000, 264, 0), (129, 16, 64, 0), (300, 2064, 1088, 0), (200, 500, 264, 0), (200, 512, 264, 0), (200, 520, 256, 0),
                                           (200, 512, 256, 4), (150, 256, 192, 0)])

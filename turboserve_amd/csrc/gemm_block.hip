@@ -18,11 +18,11 @@
 // while most of its second step is still to be multiplied; loads are issued two to five iterations ahead, one beside each tile's
 // instructions (issued in one go they held the matrix instructions up).
 // Measured, microseconds, against the better of gemm_wide and the library's default kernel (with the kernel that reads or
-// makes the result: SwiGLU, or the norm that takes the partial sums), at 299 / 509 / 2,048 rows: gate|up [37888, 3584] 81 / 124 /
-// 429 against 126 / 158 / 560 (1.3 PFLOP/s), down [3584, 18944] 58 / 79 / 246 against 111 / 90 / 291, o [3584, 3584] 26 / 30 / 73
+// makes the result: SwiGLU, or the norm that takes the partial sums), at 299 / 509 / 2,048 rows: gate|up [37888, 3584] 85 / 139 /
+// 441 against 126 / 158 / 560 (1.26 PFLOP/s), down [3584, 18944] 58 / 79 / 246 against 111 / 90 / 291, o [3584, 3584] 26 / 30 / 73
 // against 35 / 34 / 77, q|k|v [4608, 3584] 27 / 28 / 59 against 23 / 31 / 62.  An iteration of 256 x 256 takes 1.15 us where
 // half the compute units have a workgroup and 1.4 where all do (the matrix instructions 0.85 at the full clock); a
-// workgroup's start takes 2 us and its stores 4.
+// workgroup's start takes 2 us and its stores 4 (gated 9).
 // A decode step's product is bound by reading the weights; 160 weight rows by 64 activation rows a workgroup, the weights
 // non-temporal, take gate|up at 64 rows in 44.1 us (gemm_wide 47.5), 128 rows down in 26.6 (28.6), q|k|v in 11.5 (12.0), o in 10.4
 // (11.1); at 128 rows 50 (60), 33 (37), 14.5 (15.3), 13.7 (14.1).
@@ -53,23 +53,14 @@ __device__ __forceinline__ uint32_t block_pack(float lo, float hi) {
   return both;
 }
 
-// gated_unit (common.hpp) with the hardware's 2^x and reciprocal (both within an ulp), short enough to stand in the stores of
-// every tile.  PLAIN: a rule without limit and cubic.
-template <bool PLAIN>
-__device__ __forceinline__ float block_unit(float g, float u, GluRule rule) {
-  if (!PLAIN && rule.limit > 0.f) {
-    g = fminf(g, rule.limit);
-    u = fminf(fmaxf(u, -rule.limit), rule.limit);
-  }
-  const float inner = !PLAIN && rule.cubic != 0.f ? fmaf(rule.cubic * g * g, g, g) : g;
-  const float e = __builtin_amdgcn_exp2f(inner * (rule.steepness * -1.44269504088896340736f));
-  return g * __builtin_amdgcn_rcpf(1.f + e) * (u + rule.up_shift);
-}
-
-// The two outputs that a lane holds of a tile, whose rows alternate gate, up.
+// The two outputs that a lane holds of a tile, whose rows alternate gate, up: gated_unit as every kernel computes it.  (The
+// hardware's 2^x and reciprocal alone take 5 us less over a block of 256 x 256, gate|up at 2,048 rows 425 us instead of 438, but
+// their error is a tenth larger and gates below -87.3, whose reciprocal is a denormal, come out as 0.)  PLAIN: a rule
+// without limit and cubic.
 template <bool PLAIN>
 __device__ __forceinline__ uint32_t block_units(f32x4 v, GluRule rule) {
-  return block_pack(block_unit<PLAIN>(v[0], v[1], rule), block_unit<PLAIN>(v[2], v[3], rule));
+  if (PLAIN) rule.limit = 0.f, rule.cubic = 0.f;
+  return block_pack(gated_unit(v[0], v[1], rule), gated_unit(v[2], v[3], rule));
 }
 
 // Odd rows of sixteen lanes of a against even rows of b; the upper 32 lanes of a against the lower 32 of b.
@@ -275,8 +266,8 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   }
 
   // What bounds the stores is their number: one takes about 75 cycles, whether its lanes write 4 bytes each or 16, in
-  // pieces of 16 or of 64 bytes a row (256 x 256 outputs: 10.5 us with a store of 8 (gated: 4) bytes a lane for every tile,
-  // 4 with these; gate|up at 2,048 rows 460 -> 429 us).  So every lane writes 16 bytes: the four lanes of a row hold four consecutive
+  // pieces of 16 or of 64 bytes a row (256 x 256 outputs: 10.5 us with a store of 8 bytes a lane for every tile,
+  // 4 with these).  So every lane writes 16 bytes: the four lanes of a row hold four consecutive
   // columns of every tile, and exchange them until one holds eight of one of two tiles (gated: all of one of four).
   // Rows beyond M lie past the buffer's end, tiles beyond N are sent there.
   constexpr int BYTES = MODE == 1 ? 4 : 2, PER = MODE >= 2 ? 2 : 1;  // of an output element; weight rows of one

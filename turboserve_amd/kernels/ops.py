@@ -2170,7 +2170,7 @@ class Ops:
                 splits = -(-iters // per_split)
                 if splits != want:
                     continue
-                cost = -(-tiles * splits // self.compute_units) * ((per_split + 6) * pace + (0.1 * tn * tm if kind == "gated" else 0.0))
+                cost = -(-tiles * splits // self.compute_units) * ((per_split + 6) * pace + (0.18 * tn * tm if kind == "gated" else 0.0))
                 if splits > 1:
                     cost += splits * m * n * 4 / 3.6e6
                 if best is None or cost < best[0]:
