@@ -2242,12 +2242,17 @@ class Ops:
         reads the result, the library's takes 1.32 times as long for gate|up, 1.5 for partial
         sums, 1.15 for one result; the few it is faster at, up to 1.2 times, follow no size), else ``gemm_wide``."""
         m, (n, k) = x.shape[0], weight.shape
+        float32 = kind == "sums" and self.library_residual_float32
         if self.block_supported(x, weight) and (bias is None or bias.data_ptr() % 8 == 0):
             block = self._block_plan(m, n, k, kind)
-            return lambda: self.gemm_block(x, weight, bias, plan=block, gated=kind == "gated", rule=rule), self.wide_default_rows > 0
+            # One range too stays 32-bit up to the rows at which gemm_wide's ranges leave partial sums (a plan of one range
+            # there is wide: 16,384 x 16,384), above as the library's result is.
+            sums = float32 or (kind == "sums" and m <= self.wide_default_rows)
+            return (lambda: self.gemm_block(x, weight, bias, plan=block, gated=kind == "gated", sums=sums, rule=rule),
+                    self.wide_default_rows > 0)
         wide = self._wide_plan(m, n, k, kind != "sums")
         workgroups = -(-n // (32 * wide[2])) * -(-m // wide[3]) * wide[1]
-        return (lambda: self.gemm_wide(x, weight, bias, plan=wide, gated=kind == "gated", rule=rule),
+        return (lambda: self.gemm_wide(x, weight, bias, plan=wide, gated=kind == "gated", sums=float32, rule=rule),
                 m <= self.wide_default_rows and (2 * workgroups >= self.compute_units or m * n * k < self.library_tuning_min_work))
 
     def _wide_plan(self, m: int, n: int, k: int, one_range: bool) -> tuple[int, int, int, int, int]:
@@ -2626,8 +2631,9 @@ class Ops:
             if paused:
                 tunable.enable(True)
 
-    #: Whether a library product whose result goes into the residual stream leaves it in 32-bit.
-    #: Off: the library's kernels with a 32-bit result are slower (a 2,048-token prompt of the 7B
+    #: Whether a product of many rows whose result goes into the residual stream always leaves it in
+    #: 32-bit.  Off: products of one range of K above ``wide_default_rows`` rows round it to bfloat16,
+    #: as do the library's: the library's kernels with a 32-bit result are slower (a 2,048-token prompt of the 7B
     #: shape takes 29.1 ms against 26.2), and the exactness gained is small (140 short prompts in
     #: one step are off by 2.3% of a row's largest logit at most instead of 2.4%, the mean by
     #: 0.62% instead of 0.66%).
@@ -2678,9 +2684,9 @@ class Ops:
         BLAS library behind torch (as the reference does for every linear layer,
         src/turboserve/engine/model/layers.py:142), whichever was the faster one when both were
         timed (``_wide_runs``; untimed: ``_own_product``).  ``for_residual``: the result is what a
-        norm adds to the 32-bit residual stream, so the library leaves it in 32-bit too (as
-        ``[1, M, N]``, one partial sum): the stream then gets the same unrounded addend from a
-        prompt's step as from a decode step's partial sums."""
+        norm adds to the 32-bit residual stream, so it may stay 32-bit partial sums ``[S, M, N]``, and
+        with ``library_residual_float32`` it always does (as ``[1, M, N]`` where it is one range):
+        the stream then gets the same unrounded addend from a prompt's step as from a decode step's."""
         if x.dtype == torch.float32:
             return self.gemm_plain(x, weight, bias)
         _gpu(x, weight, bias)
