@@ -2238,22 +2238,40 @@ class Ops:
                      rule: tuple[float, float, float] = (1.0, 0.0, 0.0)):
         """This engine's product for a step of more rows than the decode products take, as a call
         without arguments, and whether it runs where no timing was made (``_wide_runs``): the block
-        product always, where it takes the operands (over the matrices above at 144 to 2,048 rows, with the kernel that
-        reads the result, the library's takes 1.32 times as long for gate|up, 1.5 for partial
-        sums, 1.15 for one result; the few it is faster at, up to 1.2 times, follow no size), else ``gemm_wide``."""
+        product where it takes the operands, else ``gemm_wide``.  Untimed, ``gemm_wide`` runs up to
+        ``wide_default_rows`` rows if its grid gives half of the compute units a workgroup (or the product is too
+        small to time), the block product there too, for partial sums always, and for one result from a grid on that
+        fills enough of the device (``_block_fill``)."""
         m, (n, k) = x.shape[0], weight.shape
         float32 = kind == "sums" and self.library_residual_float32
+        wide = self._wide_plan(m, n, k, kind != "sums")
+        workgroups = -(-n // (32 * wide[2])) * -(-m // wide[3]) * wide[1]
+        runs = m <= self.wide_default_rows and (2 * workgroups >= self.compute_units or m * n * k < self.library_tuning_min_work)
         if self.block_supported(x, weight) and (bias is None or bias.data_ptr() % 8 == 0):
             block = self._block_plan(m, n, k, kind)
             # One range too stays 32-bit up to the rows at which gemm_wide's ranges leave partial sums (a plan of one range
             # there is wide: 16,384 x 16,384), above as the library's result is.
             sums = float32 or (kind == "sums" and m <= self.wide_default_rows)
-            return (lambda: self.gemm_block(x, weight, bias, plan=block, gated=kind == "gated", sums=sums, rule=rule),
-                    self.wide_default_rows > 0)
-        wide = self._wide_plan(m, n, k, kind != "sums")
-        workgroups = -(-n // (32 * wide[2])) * -(-m // wide[3]) * wide[1]
-        return (lambda: self.gemm_wide(x, weight, bias, plan=wide, gated=kind == "gated", sums=float32, rule=rule),
-                m <= self.wide_default_rows and (2 * workgroups >= self.compute_units or m * n * k < self.library_tuning_min_work))
+            workgroups = -(-n // (32 * block[2])) * -(-m // (32 * block[3])) * block[1]
+            runs = runs or (self.wide_default_rows > 0 and workgroups >= self._block_fill(k, kind) * self.compute_units)
+            return lambda: self.gemm_block(x, weight, bias, plan=block, gated=kind == "gated", sums=sums, rule=rule), runs
+        return lambda: self.gemm_wide(x, weight, bias, plan=wide, gated=kind == "gated", sums=float32, rule=rule), runs
+
+    @staticmethod
+    def _block_fill(k: int, kind: str) -> float:
+        """Workgroups per compute unit from which on the block product is the faster one where nothing
+        was timed.  A narrow product as one range of K leaves units idle, and the library divides its K among them
+        (us with the kernel that reads the result, library / block: 1,024 x 4,096 at 160 rows, 16
+        workgroups, 13 / 32; 2,048 x 8,192 at 512, 64, 37 / 70; 3,584 x 3,584 at 256, 56, 24 / 40; 4,608 x 3,584 at 300, 108, 28 /
+        34, at 400, 144, 45 / 34; 2,048 x 8,192 at 1,500, 192, 60 / 72).  A gated result saves a pass of its
+        own: the shorter K, the fewer workgroups do (1,024 x 1,024 at 160 rows, 16, 13.4 / 12.5; 5,632 x 2,048 at 256, 88,
+        26 / 21; 2,816 x 2,048 at 300, 66, 15.5 / 18.5; 3,584 x 3,584 at 512, 112, 31 / 37).  Over 22 shapes at 129 to 2,048 rows what this picks
+        is at most 1.11 times as slow as the library, and 1% slower than the faster one on average."""
+        if kind == "sums":
+            return 0.0
+        if kind == "gated":
+            return max(0.0, min(7 / 8, (k - 768) / 4608))
+        return 9 / 16 if k <= 4096 else 7 / 8
 
     def _wide_plan(self, m: int, n: int, k: int, one_range: bool) -> tuple[int, int, int, int, int]:
         """(iterations of 64 per range of K, ranges, tile, activation rows, wavefronts) of the wide
