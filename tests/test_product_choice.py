@@ -62,3 +62,19 @@ def test_one_result_of_a_narrow_product_is_left_to_the_library():
         assert runs(m, n, k, "gated"), (m, n, k)
     ops.wide_default_rows = 0
     assert not any(runs(m, 37888, 3584, kind) for m in (200, 2048) for kind in ("one", "gated", "sums"))
+
+
+def test_short_ranges_of_partial_sums_run_the_wide_product():
+    """Up to ``wide_default_rows`` rows and eleven iterations of 64 a range; 32-bit sums either way."""
+    ops = Planner()
+
+    def picked(m, n, k):
+        own, runs = ops._own_product(*operands(m, n, k), None, "sums")
+        kernel, plan, float32 = own()
+        assert runs and (float32 or m > 640), (m, n, k)
+        return kernel
+
+    for m, n, k in ((512, 2048, 2048), (640, 2048, 2048), (400, 1024, 4096), (256, 1536, 2048), (640, 512, 512), (256, 768, 3072)):
+        assert picked(m, n, k) == "wide", (m, n, k)
+    for m, n, k in ((129, 3584, 3584), (299, 3584, 18944), (640, 5120, 13824), (700, 2048, 2048), (300, 2048, 8192), (640, 2560, 2560)):
+        assert picked(m, n, k) == "block", (m, n, k)

@@ -2241,13 +2241,18 @@ class Ops:
         product where it takes the operands, else ``gemm_wide``.  Untimed, ``gemm_wide`` runs up to
         ``wide_default_rows`` rows if its grid gives half of the compute units a workgroup (or the product is too
         small to time), the block product there too, for partial sums always, and for one result from a grid on that
-        fills enough of the device (``_block_fill``)."""
+        fills enough of the device (``_block_fill``).  Partial sums whose ranges would be short come from ``gemm_wide``
+        up to ``wide_default_rows`` rows: its eight wavefronts have started sooner than the block's rings are full (us with the norm
+        that adds them up, wide / block: 2,048 x 2,048 at 512 rows 20.8 / 23.9, 1,024 x 4,096 at 400 18.0 / 20.1, 1,536 x 2,048 at
+        640 21.4 / 23.5; over 13 such shapes at 129 to 640 rows 4% on average)."""
         m, (n, k) = x.shape[0], weight.shape
         float32 = kind == "sums" and self.library_residual_float32
         wide = self._wide_plan(m, n, k, kind != "sums")
         workgroups = -(-n // (32 * wide[2])) * -(-m // wide[3]) * wide[1]
         runs = m <= self.wide_default_rows and (2 * workgroups >= self.compute_units or m * n * k < self.library_tuning_min_work)
-        if self.block_supported(x, weight) and (bias is None or bias.data_ptr() % 8 == 0):
+        block_takes = self.block_supported(x, weight) and (bias is None or bias.data_ptr() % 8 == 0)
+        short = block_takes and kind == "sums" and m <= self.wide_default_rows and wide[0] <= 11
+        if block_takes and not short:
             block = self._block_plan(m, n, k, kind)
             # One range too stays 32-bit up to the rows at which gemm_wide's ranges leave partial sums (a plan of one range
             # there is wide: 16,384 x 16,384), above as the library's result is.
@@ -2255,7 +2260,7 @@ class Ops:
             workgroups = -(-n // (32 * block[2])) * -(-m // (32 * block[3])) * block[1]
             runs = runs or (self.wide_default_rows > 0 and workgroups >= self._block_fill(k, kind) * self.compute_units)
             return lambda: self.gemm_block(x, weight, bias, plan=block, gated=kind == "gated", sums=sums, rule=rule), runs
-        return lambda: self.gemm_wide(x, weight, bias, plan=wide, gated=kind == "gated", sums=float32, rule=rule), runs
+        return lambda: self.gemm_wide(x, weight, bias, plan=wide, gated=kind == "gated", sums=float32 or short, rule=rule), runs or short
 
     @staticmethod
     def _block_fill(k: int, kind: str) -> float:
