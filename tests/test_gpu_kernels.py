@@ -76,6 +76,26 @@ def test_add_rmsnorm_at_the_edges_of_its_blocks(ops, rows, hidden, splits):
         assert bool(((got - normed).abs() <= 2.0**-7 * normed.abs() + 1e-5).all())
 
 
+@pytest.mark.parametrize("hidden", [16, 1100, 2048, 3584, 5120, 8196, 12288, 16384, 1101])
+@pytest.mark.parametrize("post", [False, True])
+def test_add_rmsnorm_of_a_32_bit_row_does_not_depend_on_the_rows_beside_it(ops, hidden, post):
+    """32-bit rows at steps of 1 to 1,100 rows, on both sides of where the threads per row change: the same bits, with and
+    without a norm of the addend's own, for the row as written and for a row picked out."""
+    g = torch.Generator().manual_seed(hidden)
+    residual, pending = torch.randn(1100, hidden, generator=g).to(DEV), torch.randn(2, 1100, hidden, generator=g).to(DEV)
+    w, gain = (1 + 0.1 * torch.randn(2, hidden, generator=g)).to(DEV)
+    extra = dict(pending_norm=(gain, 1e-6, 0.5)) if post else {}
+    want, stream = None, None
+    for rows in (1100, 1025, 1024, 513, 512, 257, 256, 1):
+        into = residual[:rows].clone()
+        got = ops.add_rmsnorm(into, pending[:, :rows].contiguous(), w, 1e-6, **extra)
+        if want is None:
+            want, stream = got.clone(), into.clone()
+        assert torch.equal(got, want[:rows]) and torch.equal(into, stream[:rows]), rows
+    picked = torch.tensor([3, 1, 1099], dtype=torch.int32, device=DEV)
+    assert torch.equal(ops.add_rmsnorm(residual.clone(), pending, w, 1e-6, picked, **extra), want[picked.long()])
+
+
 def test_rmsnorm_rounds_before_the_gain(ops):
     """bfloat16: the normalised value is rounded to bfloat16 before the gain multiplies it
     (src/turboserve/engine/model/layers.py:208); a single rounding of the product differs."""

@@ -239,7 +239,34 @@ __device__ __forceinline__ void add_splits4(const P* p, int splits, size_t strid
 
 #define NORM_ITEMS 4
 
-template <typename T, typename P, bool POST>
+// 32-bit rows say which of the two roundings falls away (left to itself the compiler contracted a thread's first two
+// squares one way for some items and the other way for others).
+template <typename T>
+__device__ __forceinline__ void add_square(float& sum, float v) {
+  if (sizeof(T) == 4) sum = fmaf(v, v, sum);
+  else sum += v * v;
+}
+
+// A row's sum.  SUMS = 1,024 / blockDim.x (at most NORM_ITEMS): in the order of 1,024 threads, whatever threads take the row:
+// `part[i]` is what thread (t + i blockDim.x) of 1,024 has added up, and what follows is what those would do, the sums of
+// 64 lanes, then those of the wavefronts in their order.  (0.1 to 0.4 us more than SUMS = 1, a sum per thread.)
+template <int SUMS>
+__device__ __forceinline__ float row_sum(const float (&part)[SUMS], float* scratch) {
+  const int lane = threadIdx.x & (TS_WAVE - 1), wave = threadIdx.x / TS_WAVE, waves = blockDim.x / TS_WAVE;
+  float v[SUMS];
+#pragma unroll
+  for (int i = 0; i < SUMS; ++i) v[i] = wave_sum(part[i]);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < SUMS; ++i)
+    if (lane == 0) scratch[i * waves + wave] = v[i];
+  __syncthreads();
+  float total = 0.f;
+  for (int w = 0; w < SUMS * waves; ++w) total += scratch[w];
+  return total;
+}
+
+template <typename T, typename P, bool POST, int SUMS>
 __global__ void add_rmsnorm_vec4_kernel(T* __restrict__ y, float* __restrict__ residual,
                                         const P* __restrict__ pending, int splits, size_t split_stride,
                                         const T* __restrict__ w, const int* __restrict__ rows, float eps,
@@ -252,11 +279,11 @@ __global__ void add_rmsnorm_vec4_kernel(T* __restrict__ y, float* __restrict__ r
   const size_t out_base = (size_t)blockIdx.x * hidden;
   const int quads = hidden / 4;
   float s[NORM_ITEMS][4], g[NORM_ITEMS][4];
-  float ss = 0.f;
+  float part[SUMS] = {};
   if (POST) {
     // The pending output with its own norm: its sum of squares first, then the residual sum.
     float p[NORM_ITEMS][4], pg[NORM_ITEMS][4];
-    float pss = 0.f;
+    float post_part[SUMS] = {};
 #pragma unroll
     for (int it = 0; it < NORM_ITEMS; ++it) {
       const int qd = threadIdx.x + it * blockDim.x;
@@ -268,10 +295,10 @@ __global__ void add_rmsnorm_vec4_kernel(T* __restrict__ y, float* __restrict__ r
         for (int e = 0; e < 4; ++e) p[it][e] = 0.f;
         add_splits4(pending + in_base + 4 * qd, splits, split_stride, p[it]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) pss += p[it][e] * p[it][e];
+        for (int e = 0; e < 4; ++e) add_square<T>(post_part[it % SUMS], p[it][e]);
       }
     }
-    pss = block_sum(pss, scratch);
+    const float pss = row_sum(post_part, scratch);
     const float by = rsqrtf(pss / (float)hidden + post.eps) * post.scale;
 #pragma unroll
     for (int it = 0; it < NORM_ITEMS; ++it) {
@@ -280,7 +307,7 @@ __global__ void add_rmsnorm_vec4_kernel(T* __restrict__ y, float* __restrict__ r
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           s[it][e] += p[it][e] * by * pg[it][e];
-          ss += s[it][e] * s[it][e];
+          add_square<T>(part[it % SUMS], s[it][e]);
         }
         if (!rows) Vec4Of<float>::store(residual + in_base + 4 * qd, s[it]);
       }
@@ -296,10 +323,10 @@ __global__ void add_rmsnorm_vec4_kernel(T* __restrict__ y, float* __restrict__ r
       if (also) add_splits4(also + in_base + 4 * qd, also_splits, also_stride, s[it]);
       if ((pending || also) && !rows) Vec4Of<float>::store(residual + in_base + 4 * qd, s[it]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) ss += s[it][e] * s[it][e];
+      for (int e = 0; e < 4; ++e) add_square<T>(part[it % SUMS], s[it][e]);
     }
   }
-  ss = block_sum(ss, scratch);
+  const float ss = row_sum(part, scratch);
   const float rstd = rsqrtf(ss / (float)hidden + eps);
 #pragma unroll
   for (int it = 0; it < NORM_ITEMS; ++it) {
@@ -322,27 +349,38 @@ static void launch_add_rmsnorm(void* y, float* residual, const void* pending, in
   // Few rows (decode): one large block per row.  Many rows: as few threads as take a row in NORM_ITEMS items, but a power of
   // two, which fills the compute units' four SIMDs evenly (2,080 rows of 5,120 with a bfloat16 addend: 320 threads 44 us,
   // 512 35, 640 52; 2,048 rows of 2,048: 128 13, 256 15, 320 23), twice as many while all rows run at
-  // once and the units have room (299 rows of 3,584, nine partial sums: 256 16 us, 512 14.5, 1,024 17).
+  // once and the units have room (299 rows of 3,584, nine partial sums: 256 16 us, 512 14.5, 1,024 17; 300 rows of 5,120:
+  // 512 8.4, 1,024 11.5; 32-bit rows of 3,584 at 300: 256 6.8, 512 7.2), and at rows that two or three such rounds
+  // take, no fewer than 256 for a wide row (700 rows of 2,048: 128 8.5, 256 7.7; at 1,024 rows 9.2 and 8.8).
+  constexpr bool FLOAT32 = sizeof(T) == 4;
   const int need = (hidden / 4 + NORM_ITEMS - 1) / NORM_ITEMS;
   int threads = 128;
   while (threads < need) threads *= 2;
-  if (out_rows <= 512 && threads <= 512) threads *= 2;
+  if (out_rows <= 512 && threads <= (FLOAT32 ? 128 : 256)) threads *= 2;
+  else if (out_rows <= 1024 && hidden > 1024 && threads < 256) threads = 256;
   if (out_rows <= 256 && threads < 1024) threads = 1024;
   const PostNorm<T> post = {(const T*)post_gain, post_eps, post_scale};
+#define TS_NORM(POST, SUMS)                                                                                                   \
+  hipLaunchKernelGGL((add_rmsnorm_vec4_kernel<T, P, POST, SUMS>), dim3(out_rows), dim3(threads), 0, stream, (T*)y, residual,   \
+                     (const P*)pending, splits, (size_t)split_stride, (const T*)w, rows, eps, hidden, gain_offset,             \
+                     one_rounding, also, also_splits, (size_t)also_stride, post)
+// 32-bit rows: a row's bits do not depend on how many rows the step has.
+#define TS_NORM_SUMS(POST)                                   \
+  if (!FLOAT32 || threads == 1024) TS_NORM(POST, 1);         \
+  else if (threads == 512) TS_NORM(POST, FLOAT32 ? 2 : 1);   \
+  else TS_NORM(POST, FLOAT32 ? 4 : 1)
   if (hidden % 4 == 0 && threads <= 1024 && post_gain) {
-    hipLaunchKernelGGL((add_rmsnorm_vec4_kernel<T, P, true>), dim3(out_rows), dim3(threads), 0, stream, (T*)y, residual,
-                       (const P*)pending, splits, (size_t)split_stride, (const T*)w, rows, eps, hidden, gain_offset,
-                       one_rounding, also, also_splits, (size_t)also_stride, post);
+    TS_NORM_SUMS(true);
   } else if (hidden % 4 == 0 && threads <= 1024) {
-    hipLaunchKernelGGL((add_rmsnorm_vec4_kernel<T, P, false>), dim3(out_rows), dim3(threads), 0, stream, (T*)y, residual,
-                       (const P*)pending, splits, (size_t)split_stride, (const T*)w, rows, eps, hidden, gain_offset,
-                       one_rounding, also, also_splits, (size_t)also_stride, post);
+    TS_NORM_SUMS(false);
   } else {
     hipLaunchKernelGGL((add_rmsnorm_kernel<T, P>), dim3(out_rows), dim3(hidden <= 1024 ? 256 : 1024), 0, stream,
                        (T*)y, residual, (const P*)pending, splits, (size_t)split_stride, (const T*)w, rows, eps,
                        hidden, gain_offset, one_rounding, also, also_splits, (size_t)also_stride, post);
   }
 }
+#undef TS_NORM
+#undef TS_NORM_SUMS
 
 // `out_rows` = rows of y written: the number of entries of `rows` if given, else the tokens.
 // pending_f32 != 0: `pending` holds `splits` 32-bit partial sums, `split_stride` elements apart.
