@@ -1,5 +1,5 @@
-"""Which kernel and grid a product runs, by its sizes alone: the choices of ``kernels/ops.py``, played on the CPU with tensors
-that have sizes and no memory.  The grids named were timed on a device of 256 compute units."""
+"""Which kernel and grid a product or an attention runs, by its sizes alone: the choices of ``kernels/ops.py``, played on the CPU,
+mostly with tensors that have sizes and no memory.  The grids named were timed on a device of 256 compute units."""
 
 from __future__ import annotations
 
@@ -78,3 +78,19 @@ def test_short_ranges_of_partial_sums_run_the_wide_product():
         assert picked(m, n, k) == "wide", (m, n, k)
     for m, n, k in ((129, 3584, 3584), (299, 3584, 18944), (640, 5120, 13824), (700, 2048, 2048), (300, 2048, 8192), (640, 2560, 2560)):
         assert picked(m, n, k) == "block", (m, n, k)
+
+
+def test_32_bit_attention_is_asked_only_for_what_it_takes():
+    """Pages of 24 keys and pages or rows that 16-byte accesses do not fit stay with the kernel that takes any geometry."""
+    ops = Planner()
+
+    def asked(page=16, dim=64, value_dim=64, shift=0, stride=256, dtype=torch.float32):
+        room = torch.zeros(4 * page * max(dim, value_dim) + 4, dtype=dtype)
+        k = room[shift: shift + 2 * page * dim].view(1, 2, page, dim)
+        v = room[: 2 * page * value_dim].view(1, 2, value_dim, page)
+        return ops.float32_attention_supported(torch.zeros(3, stride, dtype=dtype), stride, k, v)
+
+    assert asked() and asked(page=64) and asked(dim=128, value_dim=128)
+    assert not asked(page=24) and not asked(page=8) and not asked(page=48)
+    assert not asked(shift=1) and asked(shift=4)
+    assert not asked(stride=257) and not asked(dim=72, value_dim=72) and not asked(value_dim=32) and not asked(dtype=torch.bfloat16)

@@ -1616,13 +1616,14 @@ class Ops:
     def float32_attention_supported(self, q: torch.Tensor, q_stride: int, k_pages: torch.Tensor, v_pages: torch.Tensor | None,
                                     out: tuple[torch.Tensor, int] | None = None) -> bool:
         """Whether :meth:`attention_float32` takes this layer: 32-bit, a head size it is built for, values as
-        wide in pages of their own, pages of 16 keys or more, rows that 16-byte accesses fit.  All of it is
-        the layer's and the cache's geometry, never the step's, so a request's steps agree."""
+        wide in pages of their own, pages of 16 keys or a larger power of two, rows and pages that 16-byte accesses
+        fit.  All of it is the layer's and the cache's geometry, never the step's, so a request's steps agree."""
         if q.dtype != torch.float32 or v_pages is None or k_pages.dtype != torch.float32 or v_pages.dtype != torch.float32:
             return False
         block_size, head_dim = k_pages.shape[2], k_pages.shape[3]
         placed = out is None or (out[0].stride(0) % 4 == 0 and (out[0].data_ptr() + 4 * out[1]) % 16 == 0)
         return (head_dim in self.float32_attention_dims and v_pages.shape[2] == head_dim and block_size >= 16
+                and block_size & (block_size - 1) == 0 and k_pages.data_ptr() % 16 == 0 and v_pages.data_ptr() % 16 == 0
                 and q_stride % 4 == 0 and q.data_ptr() % 16 == 0 and placed)
 
     def attention_float32(
