@@ -880,6 +880,84 @@ def test_attention_float32(ops, monkeypatch, heads, kv_heads, dim, page, rule):
     assert torch.equal(run(alone, len(alone)), whole[alone])
 
 
+class LongSingles:
+    """Requests of one token each behind contexts of up to some thousand keys, in scrambled pages; 32-bit."""
+
+    def __init__(self, contexts, heads, kv_heads, dim, page, seed):
+        g = torch.Generator().manual_seed(seed)
+        pages = sum(-(-c // page) for c in contexts)
+        order = torch.randperm(pages, generator=g).to(torch.int32)
+        self.heads, self.dim, self.contexts = heads, dim, contexts
+        self.kp = torch.randn(pages, kv_heads, page, dim, generator=g).to(DEV)
+        self.vp = torch.randn(pages, kv_heads, dim, page, generator=g).to(DEV)
+        self.table = torch.zeros(len(contexts), max(-(-c // page) for c in contexts), dtype=torch.int32)
+        used = 0
+        for s, c in enumerate(contexts):
+            self.table[s, : -(-c // page)] = order[used: used + -(-c // page)]
+            used += -(-c // page)
+        self.table = self.table.to(DEV)
+        self.q = torch.randn(len(contexts), heads * dim, generator=g).to(DEV)
+
+    def run(self, ops, picked, generic=False, **rule):
+        ints = lambda values: torch.tensor(values, dtype=torch.int32, device=DEV)
+        window = rule.pop("window", None)
+        args = (self.q[picked].contiguous(), self.heads * self.dim, self.kp, self.vp, self.table, ints(picked),
+                ints([self.contexts[s] - 1 for s in picked]), self.heads, self.dim ** -0.5, window)
+        if generic:
+            return ops.paged_attention_generic(*args, **rule)
+        return ops.attention_float32(*args, num_single=len(picked), max_single_context=max(self.contexts), **rule)
+
+
+class Modes:
+    """The library, noting the mode and the tokens of every launch of the 32-bit attention."""
+
+    def __init__(self, core):
+        self.core, self.seen = core, []
+
+    def __getattr__(self, name):
+        if name != "ts_attention_f32":
+            return getattr(self.core, name)
+
+        def launch(*args):
+            self.seen.append((args[-5], args[10]))  # mode, tokens
+            return self.core.ts_attention_f32(*args)
+
+        return launch
+
+
+@pytest.mark.parametrize("rule", [{}, {"window": 1500, "keep_first": 70}, {"chunk": 700, "sinks": 1.0}])
+@pytest.mark.parametrize("heads,kv_heads,dim,page", [(8, 8, 16, 16), (34, 2, 64, 32), (6, 3, 256, 16)])
+def test_attention_float32_of_many_long_requests(ops, monkeypatch, heads, kv_heads, dim, page, rule):
+    """More tiles than a launch has workgroups side by side (8,192), so that a workgroup takes several of a token's tiles,
+    with contexts that end before, inside and behind its stride; and more tokens than the scratch holds, which
+    go in groups: the bits of the same requests run a few at a time, and of one wavefront folding all tiles."""
+    singles = {8: 60, 34: 70, 6: 90}[heads]  # up to two wavefronts a compute unit
+    ragged = [1, 63, 64, 65, 1000, 1023, 1024, 1025, 2100, 2599, 2600]
+    contexts = [ragged[s % len(ragged)] + 64 * (s // len(ragged) % 3) for s in range(singles)]
+    case = LongSingles(contexts, heads, kv_heads, dim, page, seed=heads)
+    per = -(-(heads // kv_heads) // 16)
+    assert 8192 // (singles * kv_heads * per) < -(-max(contexts) // 64)
+    every = list(range(singles))
+    noting = Modes(ops.core)
+    monkeypatch.setattr(ops, "core", noting)
+    whole = case.run(ops, every, **rule)
+    assert [m for m in noting.seen if m[1]] == [(2, singles)]
+    torch.testing.assert_close(whole, case.run(ops, every, generic=True, **rule), **tol(torch.float32))
+    few = torch.cat([case.run(ops, every[i: i + 2], **rule) for i in range(0, singles, 2)])
+    assert torch.equal(whole, few)
+    tiles = -(-max(contexts) // 64)
+    seen = min([max(contexts), *[rule[name] for name in ("window", "chunk") if name in rule]])
+    tiles = min(tiles, -(-seen // 64) + 1 + -(-rule.get("keep_first", 0) // 64))
+    token = 4 * heads * tiles * (dim + 2)
+    for scratch, modes in ((9 * token, 2), (token, 2), (token - 1, 1)):
+        noting.seen.clear()
+        monkeypatch.setattr(ops, "float32_attention_scratch", scratch)
+        assert torch.equal(case.run(ops, every, **rule), whole)
+        launched = [m for m in noting.seen if m[1]]
+        assert {m[0] for m in launched} == {modes} and sum(m[1] for m in launched) == singles
+        assert modes == 1 or all(m[1] * token <= scratch for m in launched)
+
+
 def test_attention_float32_keeps_values_apart(ops):
     """A value that is no finite number reaches the rows that see its key and no other: a token's own, in the middle of a
     block of rows; and what lies in a page behind a request's last token reaches nobody."""

@@ -1609,8 +1609,11 @@ class Ops:
 
     #: Head sizes of the 32-bit attention on the matrix cores (``csrc/attention_f32.hip``).
     float32_attention_dims = (16, 32, 48, 64, 80, 96, 128, 256)
-    #: Bytes that single tokens' tiles may take side by side; above it a wavefront folds all tiles of its token
-    #: itself, with the same bits (a tile of 64 keys leaves 130 floats a head at a head size of 128, 6% of its keys and values).
+    #: Bytes that single tokens' tiles may take side by side (a tile of 64 keys leaves 130 floats a head at a head size of
+    #: 128, 6% of its keys and values).  More tokens than it holds go one group after the other through the same memory,
+    #: or, where the tokens' wavefronts fill the device by themselves (or it does not hold one token's tiles), a
+    #: wavefront folds all tiles of its token itself.  The bits are the same.  (us, 28 heads of 128 on 4 KV heads, groups / folded:
+    #: 64 requests of 16,000 keys 959 / 1,776, 96 1,489 / 1,837, 128 1,933 / 1,869, 256 of 12,000 2,890 / 2,113.)
     float32_attention_scratch = 256 << 20
 
     def float32_attention_supported(self, q: torch.Tensor, q_stride: int, k_pages: torch.Tensor, v_pages: torch.Tensor | None,
@@ -1670,13 +1673,17 @@ class Ops:
         if num_single > 0:
             seen = min(max_single_context, window or max_single_context, chunk or max_single_context)
             max_tiles = min(-(-max_single_context // 64), -(-seen // 64) + 1 + -(-keep_first // 64))
-            slots = num_single * heads * max_tiles
-            if 4 * slots * (head_dim + 2) <= self.float32_attention_scratch:
-                partial = torch.empty(slots * head_dim, dtype=torch.float32, device=q.device)
-                ml = torch.empty(slots * 2, dtype=torch.float32, device=q.device)
-                launch(tokens - num_single, num_single, 2, partial, ml, max_tiles)
-            else:
-                launch(tokens - num_single, num_single, 1)
+            fit = self.float32_attention_scratch // (4 * heads * max_tiles * (head_dim + 2))
+            if fit < num_single and num_single * kv_heads * -(-(heads // kv_heads) // 16) > 2 * self.compute_units:
+                fit = 0
+            most = min(num_single, fit or num_single, 65535)  # tokens of a launch: what the scratch holds and a grid takes
+            group = -(-num_single // -(-num_single // most))
+            partial = ml = None
+            if fit:
+                partial = torch.empty(group * heads * max_tiles * head_dim, dtype=torch.float32, device=q.device)
+                ml = torch.empty(group * heads * max_tiles * 2, dtype=torch.float32, device=q.device)
+            for first in range(tokens - num_single, tokens, group):
+                launch(first, min(group, tokens - first), 2 if fit else 1, partial, ml, max_tiles if fit else 0)
         return result
 
     @staticmethod
