@@ -958,6 +958,30 @@ def test_attention_float32_of_many_long_requests(ops, monkeypatch, heads, kv_hea
         assert modes == 1 or all(m[1] * token <= scratch for m in launched)
 
 
+def test_attention_float32_stays_inside_its_scratch(ops, monkeypatch):
+    """A caller that understates the longest context gets that many tiles' keys and no access outside the scratch, whose
+    neighbours stay as they are."""
+    case = LongSingles([200, 64, 130, 300], 4, 2, 64, 16, seed=1)
+    made = []
+
+    def framed(size, **kw):
+        room = torch.full((size + 2 * 4096,), 7.0, **kw)
+        made.append((room, size))
+        return room[4096: 4096 + size]
+
+    def run():
+        ints = lambda values: torch.tensor(values, dtype=torch.int32, device=DEV)
+        return ops.attention_float32(case.q, 256, case.kp, case.vp, case.table, ints([0, 1, 2, 3]), ints([199, 63, 129, 299]), 4, 0.125, None,
+                                     num_single=4, max_single_context=128)
+
+    real = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda size, *a, **kw: framed(size, **kw) if isinstance(size, int) else real(size, *a, **kw))
+    got = run()
+    monkeypatch.undo()
+    assert len(made) == 2 and all(bool((room[:4096] == 7).all() and (room[4096 + size:] == 7).all()) for room, size in made)
+    assert torch.equal(got[1], case.run(ops, [1])[0]) and bool(got.isfinite().all())
+
+
 def test_attention_float32_keeps_values_apart(ops):
     """A value that is no finite number reaches the rows that see its key and no other: a token's own, in the middle of a
     block of rows; and what lies in a page behind a request's last token reaches nobody."""

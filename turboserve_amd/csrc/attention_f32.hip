@@ -159,7 +159,7 @@ attention_f32_kernel(float* __restrict__ out, long out_stride, float out_scale, 
     const int* table = block_table + (size_t)seq * table_width;
     first = last_row + 1;
 
-    const int tiles = walk.count();
+    const int tiles = TILES ? min(walk.count(), max_tiles) : walk.count();  // never past a token's share of the scratch
     const int step = TILES ? gridDim.x : 1;
     int ordinal = TILES ? blockIdx.x : 0;
     if (ordinal >= tiles) continue;
@@ -331,7 +331,7 @@ attention_f32_combine_kernel(float* __restrict__ out, long out_stride, float out
   const int t = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
   const int p = positions[first_token + t];
   const int lo = lowest_key(p, rule);
-  const int tiles = walk_of(lo, lo, p, rule.keep_first).count();
+  const int tiles = min(walk_of(lo, lo, p, rule.keep_first).count(), max_tiles);
   if (d >= dim) return;
   float m = rule.sinks > 0.f ? (rule.sink_scores ? rule.sink_scores[h] : 0.f) : -INFINITY;
   float l = rule.sinks > 0.f ? rule.sinks : 0.f;
@@ -353,7 +353,8 @@ attention_f32_combine_kernel(float* __restrict__ out, long out_stride, float out
 // The arguments of ts_paged_attention_generic for `tokens` tokens from first_token on (q, out, token_seq and positions are
 // the whole step's).  mode 0: rows are 16 consecutive tokens of a head; 1: the heads of one token, folded in place; 2: the
 // heads of one token, the tiles side by side: partial [tokens, heads, max_tiles, dim] and ml [tokens, heads, max_tiles, 2]
-// (32-bit), max_tiles no smaller than any token's tiles: ceil((keys it can see, kept first ones apart) / 64) + 1 + ceil(keep_first / 64).
+// (32-bit), max_tiles no smaller than any token's tiles: ceil((keys it can see, kept first ones apart) / 64) + 1 + ceil(keep_first / 64)
+// (a token that has more is cut there: nothing is read or written outside the scratch).
 extern "C" int ts_attention_f32(void* out, const void* q, long q_stride, const void* k_pages, const void* v_pages,
                                 const int* block_table, int table_width, const int* token_seq, const int* positions,
                                 int first_token, int tokens, int heads, int kv_heads, int dim, int block_size,
