@@ -94,3 +94,37 @@ def test_32_bit_attention_is_asked_only_for_what_it_takes():
     assert not asked(page=24) and not asked(page=8) and not asked(page=48)
     assert not asked(shift=1) and asked(shift=4)
     assert not asked(stride=257) and not asked(dim=72, value_dim=72) and not asked(value_dim=32) and not asked(dtype=torch.bfloat16)
+
+
+def test_wide_matrices_at_17_to_128_rows():
+    """(ranges of K, tile of weight rows) of the block product, ungated: what was fastest of the grids timed, or within a few percent of it.
+    A matrix beyond 16,384 rows had run as one range of tiles of 128 whatever its width: 37,888 x 3,584 in two rounds,
+    up to 1.3 times as slow as the kernels before."""
+    plan = Planner()._block_few_plan
+    for m in (17, 24, 32, 64, 100, 128):
+        assert plan(m, 18944, 3584, None)[1:3] == (2, 5) and plan(m, 20480, 5120, None)[1:3] == (2, 5)
+        assert plan(m, 32768, 4096, None)[1:3] == (1, 4)
+        assert plan(m, 34944, 3584, None)[1:3] == (1, 5) and plan(m, 37888, 3584, None)[1:3] == (1, 5)
+        assert plan(m, 55296, 5120, None)[1:3] == (1, 8)
+        assert plan(m, 3584, 18944, None)[1:3] == (9, 4) and plan(m, 2048, 2048, None)[1:3] == (8, 2)
+        assert (plan(m, 24576, 4096, None) is None) == (m == 64)
+        for max_splits in (1, None):  # tiles of 256 over a long K
+            assert (plan(m, 59136, 8192, max_splits) is None) == (m <= 64)
+        assert plan(m, 59136, 7168, 1)[1:3] == (1, 8) and plan(m, 37888, 3584, 1)[1:3] == (1, 5)
+    assert plan(64, 8192, 2048, None)[1:3] == (4, 4) and plan(128, 8192, 2048, None)[1:3] == (2, 2)
+    assert plan(128, 16384, 2048, None)[1:3] == (1, 2) and plan(64, 16384, 2048, None)[1:3] == (2, 4)
+    assert plan(128, 10304, 2048, None)[1:3] == (3, 4)
+
+
+@pytest.mark.parametrize("m", [17, 32, 64, 65, 128])
+def test_grids_of_17_to_128_rows_cover_k(m):
+    """Whatever the sizes and the ranges allowed, the ranges cover K without an empty one."""
+    ops = Planner()
+    for n in (16, 272, 2048, 3584, 8192, 16400, 20480, 20496, 24576, 33000, 40960, 41000, 65536, 65552, 152064):
+        for k in (64, 128, 384, 448, 2048, 3584, 4160, 8192, 18944):
+            for max_splits in (None, 1, 2, 5):
+                plan = ops._block_few_plan(m, n, k, max_splits)
+                if plan is not None:
+                    per_split, splits, tn, tm = plan
+                    assert splits == -(-(k // 64) // per_split) and 1 <= splits <= (max_splits or 12)
+                    assert (tn, tm) in {(a, b) for a in (2, 4, 5, 8) for b in (1, 2, 4)} and m <= 32 * tm

@@ -2191,26 +2191,46 @@ class Ops:
     _BLOCK_ONE_RANGE = {2: 0.50, 4: 0.66, 5: 0.72, 8: 0.93}
 
     def _block_few_plan(self, m: int, n: int, k: int, max_splits: int | None) -> tuple[int, int, int, int] | None:
-        """The block product's grid for a decode step of 17 to 128 rows, or None where ``gemm_wide``
-        stays: one tile of activation rows.  As one range of K the tile of weight rows whose rounds
-        of workgroups are over first, if its last round is nine tenths full or the rows are more
-        than 64 (at 64 rows 27,648 x 5,120, 216 workgroups, 56 against 55 us; 37,888 x 3,584, 237, 44
-        against 47.5; at 128 rows 70 against 77 and 50 against 60); else tiles of 128 weight rows
-        and as many ranges as give every compute unit a workgroup, of six iterations at least,
-        or tiles of 64 where that would be fewer (2,048 x 2,048 at 64 rows 6.1 against 7.5)."""
+        """The block product's grid for a decode step of 17 to 128 rows, or None where ``gemm_wide`` (up to 32 rows the tiled
+        product) stays: one tile of activation rows.
+
+        As one range of K (``max_splits`` 1) the tile of weight rows whose rounds of workgroups are over first, if its last round
+        is nine tenths full or the rows are more than 64 (at 64 rows 27,648 x 5,120, 216 workgroups, 56 against 55 us;
+        37,888 x 3,584, 237, 44 against 47.5; at 128 rows 70 against 77 and 50 against 60).
+
+        Else tiles of 128 weight rows and as many ranges as give every compute unit a workgroup; tiles of 64
+        where a range would be shorter than six iterations (2,048 x 2,048 at 64 rows 6.1 against 7.5 us), and above 64 rows
+        where K is short and their grid fills the device (8,192 x 2,048 at 128 rows 19.4 against 23.9, gemm_wide 23.1; 3,584 x 18,944
+        42.6 against 38.7).  A matrix too wide for two ranges of tiles of 128 takes two of tiles of 160 where those run at
+        once (18,944 x 3,584 at 24 / 64 / 128 rows 27.6 / 32.8 / 39.4 against 30.8 / 37.4 / 50 as one range of 128), else one
+        range with the smallest tile whose workgroups do (37,888 x 3,584: 47.0 / 55.5 / 65.1 with tiles of 160 against 62 / 72 / 91 with
+        128, in two rounds; 55,296 x 5,120: 91 / 102 / 117 with 256 against 96 / 121 / 143); at 33 to 64 rows five sixths
+        of the units must have one (24,576 x 4,096, 192, 49.1 against gemm_wide's 49.0; 45,056 x 4,096, 176, 82 against 86).  Tiles of 256
+        over a K of 8,192 or more read slower than gemm_wide up to 64 rows (59,136 x 8,192 at 32 / 64 rows 169 against 157 / 162)."""
         key = (m, n, k, max_splits)
         if key in self._block_plans:
             return self._block_plans[key]
         units, iters, tm = self.compute_units, k // 64, 1 if m <= 32 else 2 if m <= 64 else 4
+        tiles = {tn: -(-n // (32 * tn)) for tn in self._BLOCK_ONE_RANGE}
+        soonest = min(tiles, key=lambda tn: -(-tiles[tn] // units) * self._BLOCK_ONE_RANGE[tn])
+        ranges = {tn: max(1, min(12, max_splits or 12, units // tiles[tn])) for tn in tiles}
+        stays = False
         if max_splits == 1:
-            tn = min(self._BLOCK_ONE_RANGE, key=lambda t: -(-(-(-n // (32 * t))) // units) * self._BLOCK_ONE_RANGE[t])
-            workgroups = -(-n // (32 * tn))
-            filled = m > 64 or 10 * workgroups >= 9 * units * -(-workgroups // units)
-            plan = (iters, 1, tn, tm) if filled else None
+            tn, want = soonest, 1
+            stays = m <= 64 and 10 * tiles[tn] < 9 * units * -(-tiles[tn] // units)
+        elif iters // ranges[4] < 6 or (ranges[4] > 1 and m > 64 and k <= (4096 if ranges[2] > 1 else 2048)
+                                      and 4 * tiles[2] * ranges[2] >= 3 * units):
+            tn, want = 2, ranges[2]
+        elif ranges[4] > 1:
+            tn, want = 4, ranges[4]
+        elif ranges[5] > 1:
+            tn, want = 5, 2
         else:
-            tn, want = 4, max(1, min(12, max_splits or 12, units // -(-n // 128)))
-            if iters // want < 6:
-                tn, want = 2, max(1, min(12, max_splits or 12, units // -(-n // 64)))
+            tn, want = next((t for t in (4, 5, 8) if tiles[t] <= units), soonest), 1
+            stays = 32 < m <= 64 and 6 * tiles[tn] < 5 * units
+        if stays or (tn == 8 and want == 1 and m <= 64 and k >= 8192):
+            plan = None
+        else:
             per_split = -(-iters // min(want, iters))
             plan = (per_split, -(-iters // per_split), tn, tm)
         self._block_plans[key] = plan
