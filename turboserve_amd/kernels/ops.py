@@ -2426,12 +2426,12 @@ class Ops:
 
     def _stream_plan(self, n: int, k: int, max_splits: int | None) -> tuple[int, int, int] | None:
         """(slices of 64 per wavefront, ranges of K, tile) of the streaming product: the fewest
-        ranges that keep the memory busy.  What a compute unit reads takes 36 bytes a nanosecond
-        where few units read and all of them together get 6.6 TB/s; a range more costs 0.12 us (its
-        sums, here and in the kernel that adds them up).  (us at one row: 3,584 x 3,584 as 1 / 2 / 4 ranges 8.1 / 6.2 / 7.2, 2,048 x
+        ranges that keep the memory busy (``_stream_cost``).  (us at one row: 3,584 x 3,584 as 1 / 2 / 4 ranges 8.1 / 6.2 / 7.2, 2,048 x
         8,192 as 1 / 2 / 4 14 / 10 / 7.7, 8,192 x 2,048 as 1 / 2 7.3 / 7.6.)  None where one range
-        leaves the last round of workgroups so empty that the tiled product is as fast
-        (27,648 x 5,120 at eight rows 48 against 46 us; 37,888 x 3,584, a last round two thirds full, 41.7 against 43.9)."""
+        leaves the last round of workgroups so empty that the tiled product is as fast or faster: always where one range is
+        asked for (27,648 x 5,120 at eight rows 48 against 46 us; 37,888 x 3,584, a last round two thirds full, 41.7 against
+        43.9), where it is only the cheapest over a long K (at one / 16 rows 20,480 x 5,120 37.9 / 43.6 against 38.5 / 38.8, but
+        18,944 x 3,584 26.7 / 29.4 against 27.5 / 28.5)."""
         key = (n, k, max_splits)
         if key in self._stream_plans:
             return self._stream_plans[key]
@@ -2442,15 +2442,21 @@ class Ops:
             splits = -(-slices // (4 * per_wave))
             if splits != want:
                 continue
-            rounds = -(-tiles * splits // units)
-            cost = max(2.0 * n * k / 6.6e6, rounds * 64.0 * k / splits / 36e3) + 0.12 * splits
+            cost = self._stream_cost(n, k, splits)
             if best is None or cost < best[0]:
                 best = (cost, per_wave, splits, 2)
         plan = best[1:]
-        if max_splits == 1 and tiles > 2 * units and 10 * units * -(-tiles // units) > 11 * tiles:
+        if plan[1] == 1 and (max_splits == 1 or k > 4096) and tiles > 2 * units and 10 * units * -(-tiles // units) > 11 * tiles:
             plan = None
         self._stream_plans[key] = plan
         return plan
+
+    def _stream_cost(self, n: int, k: int, splits: int) -> float:
+        """What the streaming product takes as ``splits`` ranges, in microseconds beyond its start:
+        what a compute unit reads takes 36 bytes a nanosecond where few units read and all of them
+        together get 6.6 TB/s; a range more costs 0.12 us (its sums, here and in the kernel that adds them up)."""
+        rounds = -(-(-(-n // 32) * splits) // self.compute_units)
+        return max(2.0 * n * k / 6.6e6, rounds * 64.0 * k / splits / 36e3) + 0.12 * splits
 
     def _stream_runs(self, x: torch.Tensor, weight: torch.Tensor, max_splits: int | None) -> tuple[int, int, int] | None:
         """The streaming product's grid where it runs a decode-sized product (up to 16 rows)."""
@@ -2709,6 +2715,13 @@ class Ops:
                 return self.gemm_wide(x, weight, bias, plan=wide, gated=True, rule=rule)
             stream = self._stream_runs(x, weight, 1) if weight.shape[0] % 2 == 0 else None
             if stream is not None:
+                n, k = weight.shape
+                shared = self._stream_plan(n, k, None)
+                # One range of a long K on few units: several ranges and the unit's own launch are sooner (us at 16 rows: 3,584 x
+                # 18,944 38.6 against 26.5, 5,120 x 13,824 31.3 against 27.7, 1,024 x 4,096 9.7 against 7.2; 3,584 x 3,584, 2.4 us
+                # apart by the model, 9.7 against 9.6).
+                if shared is not None and self._stream_cost(n, k, 1) > self._stream_cost(n, k, shared[1]) + 2.6:
+                    return self.swiglu(self.gemm_stream(x, weight, bias, plan=shared), x.dtype, paired=True, rule=rule)
                 return self.gemm_stream(x, weight, bias, plan=stream, gated=True, rule=rule)
             plan = self._tiled_plan(x.shape[0], weight.shape[0], weight.shape[1], None)
             if plan[1] == 1 and weight.shape[0] % 2 == 0 and weight.is_contiguous() and x.stride(1) == 1:
