@@ -160,9 +160,8 @@ def test_gemm_plain(ops, dtype, m, n, k):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("k", [200, 64, 131, 1])
 def test_gemm_plain_rows_do_not_depend_on_the_batch(ops, dtype, k):
-    """The same bits for a row whatever the batch: alone, among a few rows (the layout for up to
-    32 rows, one output a thread), among many (tiles of 64 x 64): every output is the same chain
-    of fused multiply-adds in the order of k in both layouts."""
+    """The same bits for a row whatever the batch: alone, among a few rows (tiles of 16 rows, a wavefront a range of K),
+    among many (tiles of 64 x 64 and 128 x 128): every output is the same chains of fused multiply-adds in all layouts."""
     g = torch.Generator().manual_seed(9)
     x = torch.randn(300, k, generator=g).to(dtype)
     w = torch.randn(150, k, generator=g).to(dtype)
@@ -200,6 +199,22 @@ def test_gemm_plain_layouts(ops, dtype, n, k, most):
         assert bool(got[:, n // 2].isnan().all())
         got[:, n // 2] = whole[:m, n // 2]
         assert torch.equal(got, whole[:m]), m
+
+
+def test_gemm_plain_of_very_many_rows(ops):
+    """2,097,121 rows against a narrow matrix, one more than tiles of 32 rows have places in a grid: a layout of larger tiles
+    takes them.  Beyond 65,535 tiles of 64 rows the product refuses, as it always has."""
+    from turboserve_amd.kernels.ops import KernelError
+
+    rows = 32 * 65535 + 1
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(rows, 4, generator=g, device=DEV)
+    w = torch.randn(3, 4, generator=g, device=DEV)
+    got = ops.gemm_plain(x, w)
+    assert float((got.double() - x.double() @ w.double().T).abs().max()) < 1e-5
+    assert torch.equal(got[-70:], ops.gemm_plain(x[-70:], w))
+    with pytest.raises(KernelError):
+        ops.gemm_plain(x[:1].expand(64 * 65535 + 1, 4).contiguous(), w)
 
 
 @pytest.mark.parametrize("m", [1, 5, 16, 17, 33, 64, 65, 100, 128])

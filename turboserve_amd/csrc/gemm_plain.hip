@@ -619,6 +619,7 @@ inline PlainKind plain_kind(int m, int n, bool stream_reads) {
   PlainKind best = TILES_128;
   long least = -1;
   for (const auto& l : layouts) {
+    if (l.cols < 64 && ceil_of(m, l.rows) > 65535) continue;  // more tiles of rows than their grids take
     const long cost = l.start[stream_reads] + l.round[stream_reads] * ceil_of(ceil_of(m, l.rows) * ceil_of(n, l.cols), GP_UNITS);
     if (least < 0 || cost < least) best = l.kind, least = cost;
   }
@@ -645,7 +646,6 @@ int launch_plain(void* y, const void* x, const void* w, const void* bias, int m,
 #define TS_PLAIN_FEW(MT, NT, AHEAD)                                                                                   \
   do {                                                                                                               \
     dim3 grid((unsigned)ceil_of(n, 16 * NT), (unsigned)ceil_of(m, 16 * MT));                                         \
-    if (grid.y > 65535) return TS_ERR_SHAPE;                                                                         \
     if (stream_reads)                                                                                                \
       return grid.y == 1 ? launch_stream<MT, NT, true>(y, x, w, bias, m, n, k, x_stride, y_stride, grid, stream)     \
                          : launch_stream<MT, NT, false>(y, x, w, bias, m, n, k, x_stride, y_stride, grid, stream);   \
@@ -690,6 +690,7 @@ extern "C" int ts_gemm_plain(void* y, const void* x, const void* w, const void* 
                              hipStream_t stream) {
   if (m == 0 || n == 0) return TS_OK;
   if (!y || !x || !w || k < 1 || x_stride < k || y_stride < n) return TS_ERR_ARG;
+  if (ceil_of(m, 64) > 65535) return TS_ERR_SHAPE;
   if (dtype == TS_F32) return launch_plain<float, float>(y, x, w, bias, m, n, k, x_stride, y_stride, stream);
   if (dtype != TS_BF16) return TS_ERR_DTYPE;
   if (out_f32) return launch_plain<bf16_t, float>(y, x, w, bias, m, n, k, x_stride, y_stride, stream);
