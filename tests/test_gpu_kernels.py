@@ -201,6 +201,60 @@ def test_gemm_plain_layouts(ops, dtype, n, k, most):
         assert torch.equal(got, whole[:m]), m
 
 
+def chains_of_fused_multiply_adds(x, w, bias):
+    """One output as the 32-bit product defines it: a chain of the C library's fmaf in the order of k per range of K (a
+    quarter of K rounded up to 64), the ranges' sums added in order, then the bias."""
+    import ctypes
+    import ctypes.util
+
+    import numpy as np
+
+    fmaf = ctypes.CDLL(ctypes.util.find_library("m")).fmaf
+    fmaf.restype, fmaf.argtypes = ctypes.c_float, [ctypes.c_float] * 3
+    k, span = len(x), -(-(-(-len(x) // 4)) // 64) * 64
+    total = np.float32(0.0)
+    for start in range(0, k, span):
+        acc = 0.0
+        for a, b in zip(x[start: start + span], w[start: start + span]):
+            acc = fmaf(a, b, acc)
+        total = np.float32(total + np.float32(acc))
+    return np.float32(total + np.float32(bias))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [5, 64, 260, 515])
+@pytest.mark.parametrize("values", ["random", "spread", "tiny", "cancelling"])
+def test_gemm_plain_is_chains_of_fused_multiply_adds(ops, dtype, k, values):
+    """The matrix instructions give the bits of a loop of fmaf, in every layout: random operands, exponents over 2^-60 .. 2^60,
+    products and operands among the denormals (kept, not flushed), sums that cancel to the roundings of their terms."""
+    g = torch.Generator().manual_seed(k)
+    m, n = 200, 300
+    x, w, b = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g), torch.randn(n, generator=g)
+    if values == "spread":
+        x, w = (torch.ldexp(t, torch.randint(-30, 31, t.shape, generator=g)) for t in (x, w))
+    elif values == "tiny":
+        x = torch.ldexp(x, torch.randint(-70, -64, x.shape, generator=g))
+        w = torch.ldexp(w, torch.randint(-72, -65, w.shape, generator=g))
+        x[:, ::7] = torch.ldexp(x[:, ::7], torch.tensor(-63))  # denormal operands
+        b = torch.zeros(n)
+    elif values == "cancelling":
+        half = k // 2
+        x[:, half: 2 * half], w[:, half: 2 * half] = -x[:, :half], w[:, :half]
+        b = b * 2.0**-24
+    x, w, b = x.to(dtype), w.to(dtype), b.to(dtype)
+    if values == "tiny":
+        assert bool(((x != 0) & (x.double().abs() < 2.0**-126)).any())
+    picked = [(0, 0), (0, 299), (17, 31), (33, 64), (100, 128), (199, 150)]
+    want = {(i, j): chains_of_fused_multiply_adds(x[i].tolist(), w[j].tolist(), b[j].item()) for i, j in picked}
+    assert values != "tiny" or any(0 < abs(float(v)) < 2.0**-126 for v in want.values())
+    for rows in (1, 18, 34, 101, 200):
+        for cols in (300, 64):
+            got = ops.gemm_plain(x[:rows].to(DEV), w[:cols].to(DEV), b[:cols].to(DEV), out_float32=True).cpu()
+            for (i, j), value in want.items():
+                if i < rows and j < cols:
+                    assert got[i, j].item() == float(value), (rows, cols, i, j)
+
+
 def test_gemm_plain_of_very_many_rows(ops):
     """2,097,121 rows against a narrow matrix, one more than tiles of 32 rows have places in a grid: a layout of larger tiles
     takes them.  Beyond 65,535 tiles of 64 rows the product refuses, as it always has."""
