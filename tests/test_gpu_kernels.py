@@ -499,9 +499,14 @@ def test_gemm_stream_every_tile_and_grid(ops, tile, m, n, k):
     assert bool(((picked.double().sum(0).cpu() - want).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("tn,tm", [(8, 8), (8, 6), (8, 5), (5, 10), (5, 8), (4, 8), (4, 5), (4, 4)] + [(a, b) for b in (1, 2) for a in (8, 5, 4, 2)]
-                         + [(8, 4), (5, 4), (2, 4)])
-@pytest.mark.parametrize("m,n,k,splits", [(1, 16, 64, 1), (17, 304, 448, 3), (33, 272, 128, 2), (65, 1040, 192, 1), (128, 528, 320, 5), (129, 272, 64, 1), (257, 48, 128, 2), (321, 528, 192, 3), (700, 1040, 448, 2)])
+BLOCK_TILES = [(8, 8), (8, 6), (8, 5), (5, 10), (5, 8), (4, 8), (4, 5), (4, 4)]
+BLOCK_ONE_TILES = [(a, b) for b in (1, 2) for a in (8, 5, 4, 2)] + [(8, 4), (5, 4), (2, 4)]  # one tile of activation rows
+BLOCK_SIZES = [(1, 16, 64, 1), (17, 304, 448, 3), (33, 272, 128, 2), (65, 1040, 192, 1), (128, 528, 320, 5), (129, 272, 64, 1), (257, 48, 128, 2),
+               (321, 528, 192, 3), (700, 1040, 448, 2)]
+
+
+@pytest.mark.parametrize("tn,tm,m,n,k,splits", [(*tile, *size) for tile in BLOCK_TILES + BLOCK_ONE_TILES for size in BLOCK_SIZES
+                                                if tile in BLOCK_TILES or size[0] <= 32 * tile[1]])
 def test_gemm_block_every_tile(ops, tn, tm, m, n, k, splits):
     """Blocks of the largest product, one tile short and one over in both directions, ranges of K
     of one to seven iterations, rows of x apart, a bias, the three results and rules of the gated unit; against
@@ -510,8 +515,6 @@ def test_gemm_block_every_tile(ops, tn, tm, m, n, k, splits):
     gated one what the unit makes of its operands' bounds (its slope in the gate stays below 1.2 for these rules)."""
     from turboserve_amd.kernels.ops import GELU_TANH_RULE
 
-    if m > 32 * tm and (tm < 4 or (tn, tm) in ((8, 4), (5, 4), (2, 4))):
-        pytest.skip("one tile of activation rows here")
     g = torch.Generator().manual_seed(100 * tn + tm + m)
     x = torch.randn(m, k + 8, generator=g).bfloat16()[:, :k]
     w = (torch.randn(n, k, generator=g) * 0.3).bfloat16()
@@ -541,6 +544,30 @@ def test_gemm_block_every_tile(ops, tn, tm, m, n, k, splits):
         assert fused.shape == (m, n // 2) and bool(((fused.double().cpu() - exact).abs() <= slack).all()), rule
     # a row does not depend on the rows beside it, nor a result on what stood in its memory
     assert torch.equal(ops.gemm_block(xd[m // 2:], wd, bd, plan=(iters, 1, tn, tm)), one[m // 2:])
+
+
+@pytest.mark.parametrize("m", [1, 7, 9, 16, 17, 32])
+@pytest.mark.parametrize("n,k", [(40, 264), (512, 2048), (8200, 4104)])
+@pytest.mark.parametrize("x_shift,w_shift", [(4, 0), (0, 4), (4, 4)])
+def test_gemm_skinny_of_operands_between_16_bytes(ops, m, n, k, x_shift, w_shift):
+    """Activations or weights that begin 8 bytes off a multiple of 16 go to the kernels that load them with plain loads (up
+    to 16 rows the resident one, for large matrices the tiled one): within the bound of k + 1 roundings of the exact product, and
+    the unit of gate and up as everywhere."""
+    g = torch.Generator().manual_seed(m + n)
+    x, w, b = torch.randn(m, k, generator=g).bfloat16(), (torch.randn(n, k, generator=g) * 0.1).bfloat16(), torch.randn(n, generator=g).bfloat16()
+    xd = torch.empty(m * k + 8, dtype=torch.bfloat16, device=DEV)[x_shift: x_shift + m * k].view(m, k).copy_(x)
+    wd = torch.empty(n * k + 8, dtype=torch.bfloat16, device=DEV)[w_shift: w_shift + n * k].view(n, k).copy_(w)
+    assert xd.data_ptr() % 16 == 2 * x_shift and wd.data_ptr() % 16 == 2 * w_shift
+    want = x.double() @ w.double().T + b.double()
+    bound = (k + 1) * 2.0**-24 * (x.double().abs() @ w.double().abs().T + b.double().abs())
+    if m <= 16:
+        assert ops._stream_runs(xd, wd, None) is None
+    got = ops.gemm_skinny(xd, wd, b.to(DEV)).double().sum(0).cpu()
+    assert bool(((got - want).abs() <= bound).all())
+    gate, up = want[:, 0::2], want[:, 1::2]
+    exact = gate * torch.sigmoid(gate) * up
+    slack = 2.0**-8 * exact.abs() + 1.2 * (bound[:, 0::2] + 2.0**-20 * gate.abs()) * up.abs() + (gate * torch.sigmoid(gate)).abs() * bound[:, 1::2] + 1e-30
+    assert bool(((ops.linear_swiglu(xd, wd, None, b.to(DEV)).double().cpu() - exact).abs() <= slack).all())
 
 
 @pytest.mark.parametrize("m,tn,tm", [(1, 8, 8), (20, 5, 1), (257, 4, 5)])
