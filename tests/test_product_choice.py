@@ -158,3 +158,34 @@ def test_one_range_with_a_nearly_empty_last_round_is_left_to_the_tiled_product()
     assert ops._stream_plan(20480, 5120, None) is None and ops._stream_plan(27648, 5120, 1) is None and ops._stream_plan(17408, 2048, 1) is None
     for n, k in ((18944, 3584), (37888, 3584), (17408, 2048), (55296, 5120), (8192, 8192), (5120, 5120)):
         assert ops._stream_plan(n, k, None) is not None, (n, k)
+
+
+def test_a_steps_estimate_holds_what_its_products_and_attention_leave():
+    """No plan's partial sums are larger than what the sizing of the cache leaves room for, and a 32-bit model's estimate holds the
+    scratch of its single tokens' attention."""
+    from turboserve_amd.weights.random_init import describe_model
+
+    ops = Planner()
+    for n in (512, 2048, 3584, 5120, 7168, 8192, 16384):
+        for k in (512, 2048, 3584, 8192, 18944, 29568, 65536):
+            for m in (1, 16, 17, 64, 128, 129, 257, 640, 641, 1024, 1788, 2048, 2500, 4096, 8192, 16384):
+                splits = [1]
+                if m <= 128:
+                    splits += [ops._tiled_plan(m, n, k, None)[1], ops._wide_plan_few_rows(m, n, k, None)[1]]
+                    few = ops._block_few_plan(m, n, k, None) if m > 16 else ops._stream_plan(n, k, None)
+                    splits += [few[1] if few else 1]
+                else:
+                    splits += [ops._block_plan(m, n, k, "sums")[1]] + ([ops._wide_plan(m, n, k, False)[1]] if m <= 640 else [])
+                assert 4 * max(splits) * m * n <= Ops.partial_sums_bytes(m, n), (m, n, k, splits)
+    config = {
+        "architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "hidden_size": 3584, "num_hidden_layers": 2, "num_attention_heads": 28,
+        "num_key_value_heads": 4, "head_dim": 128, "intermediate_size": 18944, "vocab_size": 1000, "rope_theta": 1e6, "rms_norm_eps": 1e-6,
+        "tie_word_embeddings": False, "use_sliding_window": False, "max_position_embeddings": 32768,
+    }
+    _, model = describe_model(config)
+    sums = max(4 * ops._block_plan(m, 3584, 18944, "sums")[1] * m * 3584 for m in range(129, 2049))
+    assert sums > 100 << 20  # 122 MB at 1,788 rows
+    stream = 2 * 2048 * 3584 * 8
+    products = 2048 * (3 * 18944 * 2 + 3584 * 4)  # gate|up, its units, what the stream waits for
+    assert model.activation_bytes(2048, 64, 2) >= stream + products + sums
+    assert model.activation_bytes(64, 64, 4) >= Ops.float32_attention_scratch

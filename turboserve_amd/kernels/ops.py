@@ -2342,6 +2342,18 @@ class Ops:
         self._wide_plans[key] = best[1:]
         return best[1:]
 
+    #: What the partial sums of one product take at most: a grid has as many ranges of K as give the compute units a
+    #: workgroup or a few, so the sums of a long step are two or three rounds of blocks of 256 x 256 outputs (7,168 x 65,536 at 2,500 rows
+    #: 547 MB; the 7B shape's down projection at 1,788 rows 122 MB).
+    partial_sums_limit = 640 << 20
+
+    @classmethod
+    def partial_sums_bytes(cls, rows: int, n: int) -> int:
+        """Bytes that the 32-bit partial sums of a product of up to ``rows`` rows with ``n`` outputs take at
+        most, whatever the step's own rows and K are: up to 32 ranges, or, in a step of up to 128 rows, as many as
+        256 workgroups of 128 outputs make."""
+        return max(4 * rows * n, min(32 * 4 * rows * n, cls.partial_sums_limit), 4 * min(rows, 128) * 256 * 128)
+
     def _wide_runs(self, rows: int, n: int, k: int, kind: str, untimed: bool, own, library) -> bool:
         """Whether this engine's own product, not the BLAS library's, runs a product of ``rows``
         rows (more than the decode products take): what a timing found, or ``untimed``

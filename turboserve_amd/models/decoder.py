@@ -16,6 +16,7 @@ from dataclasses import dataclass
 
 import torch
 
+from turboserve_amd.kernels.ops import Ops
 from turboserve_amd.parts.base import (
     Block,
     CacheNeed,
@@ -145,14 +146,16 @@ class DecoderModel:
         """Room a step of ``tokens`` rows that wants logits for ``requests`` of them takes beside
         weights and cache: the 32-bit residual stream and the output waiting to be added to it,
         the neediest layer (norm output plus its largest part), twice over because the caching
-        allocator keeps freed blocks of other sizes, and the 32-bit logits with the sampler's
+        allocator keeps freed blocks of other sizes, the partial sums in which a bfloat16 product may leave its
+        result (``Ops.partial_sums_bytes``; one product's at a time), and the 32-bit logits with the sampler's
         working copy (the reference's estimate has the same terms from Qwen2's sizes,
         src/turboserve/engine/runtime/memory.py:208-242)."""
         plan = self.plan
         stream = tokens * plan.hidden_size * (4 + 4 + (4 if self.keeps_origin else 0))
         layer = max((block.activation_bytes(tokens, itemsize) for block in self.blocks), default=0)
         layer += self.head.activation_bytes(tokens, itemsize)
-        return 2 * (stream + layer) + requests * plan.vocab_size * 4 * 2
+        sums = Ops.partial_sums_bytes(tokens, plan.hidden_size) if itemsize == 2 else 0
+        return 2 * (stream + layer) + sums + requests * plan.vocab_size * 4 * 2
 
     # -- caches -------------------------------------------------------------------------------
 

@@ -7,7 +7,7 @@ from collections.abc import Mapping
 
 import torch
 
-from turboserve_amd.kernels.ops import attention_geometry_error
+from turboserve_amd.kernels.ops import Ops, attention_geometry_error
 from turboserve_amd.parts.base import CacheNeed, FixedState, Mixer, PagedKV, PagedKVView, PartSpec, Runtime, SharedKV, TensorSpec
 from turboserve_amd.parts.registry import build_part, register_mixer
 
@@ -204,9 +204,10 @@ class GroupedQueryAttention(Mixer):
 
     def activation_bytes(self, tokens: int, itemsize: int) -> int:
         """The fused projection, the attention output and the output projection (32-bit: it is
-        added to the residual stream) of a step."""
+        added to the residual stream) of a step, and what a 32-bit step's single tokens leave side by side."""
         fused = (self.q_size + self.kv_size + self.v_size) * (2 if self.conv_taps is not None else 1)
-        return tokens * ((fused + self.out_size) * itemsize + self.hidden_size * 4)
+        scratch = Ops.float32_attention_scratch if itemsize == 4 else 0
+        return tokens * ((fused + self.out_size) * itemsize + self.hidden_size * 4) + scratch
 
     def tensor_specs(self) -> dict[str, TensorSpec]:
         sizes = {"q": self.q_size, "k": self.kv_size, "v": self.v_size}
