@@ -19,8 +19,8 @@
 // (attention.py:196-199).  Online softmax over tiles of 64 keys, as the reference's decode
 // kernel does over blocks (src/turboserve/engine/model/triton_attention.py:127-166).
 //
-// This is the kernel of the true 32-bit path and the one every faster kernel is checked
-// against: its result for a token is a function of (p, lo, the request's keys) only, so it is
+// This is the kernel every faster one is checked against, and the one that takes any geometry (32-bit layers that
+// attention_f32.hip does not take among them): its result for a token is a function of (p, lo, the request's keys) only, so it is
 // bitwise independent of how the request was cut into steps and of the batch around it.
 #include "common.hpp"
 

@@ -98,7 +98,10 @@ typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 
 // The body, with two names for the workgroup's LDS: `to` for the loads that write it, `from` for the reads.  __restrict__
 // tells the compiler that they are not the same memory; otherwise it would wait for every load in flight before
-// every read.  What orders them is block_wait, which no access crosses.
+// every read.  They are, so what orders them is said in other ways, all of which an edit has to keep: the slot of every
+// read has come through an asm behind the wait for its loads (ws, xs; a value the compiler cannot follow, so no read moves above
+// it, nor is one read taken for another), what is read of a slot is in registers that an asm before the wait takes (xf[1], wf)
+// or that matrix instructions pinned ahead of it have used (xf[0]), and every slot is filled again behind that wait.
 // out: bfloat16 [m, n] (mode 0), partial: float [splits, m, n] (mode 1), out: bfloat16 [m, n / 2] (mode 2; 3: any rule
 // of the gated unit.  Two kernels: with both epilogues behind one loop the compiler moved the sums between registers in it).
 template <int TN, int TM, int MODE, bool ONCE>

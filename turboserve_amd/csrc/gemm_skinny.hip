@@ -4,9 +4,9 @@
 // them (F.linear's layout, src/turboserve/engine/model/layers.py:142), 32-bit accumulation on
 // the matrix cores and 32-bit partial sums out.  The consumer (norm, rotary/cache write,
 // SwiGLU, or nobody when splits == 1) adds the splits up, so no rounding happens between the
-// product and its consumer.  (gemm_tiled.hip holds the product for up to 64 rows; this one
-// serves small matrices, whose product lasts a few microseconds and gains from many small
-// workgroups that start quickly, and the widest matrices at up to eight rows.)
+// product and its consumer.  (gemm_stream.hip holds the product for up to 16 rows; this one
+// serves the small matrices that it does not take, operands between 16 bytes and a single range of
+// K whose last round of workgroups would be nearly empty: many small workgroups that start quickly.)
 //
 // The product is bound by reading W once from HBM.  Layout of the work:
 //   * a workgroup of 4 or 8 wavefronts owns 64 or 128 consecutive weight rows (16 per

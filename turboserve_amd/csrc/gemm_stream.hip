@@ -36,7 +36,9 @@ struct Ring {
 };
 
 // `to` and `from` are the same memory: __restrict__ keeps the compiler from waiting for every load in flight before every
-// read, so it must not see that two reads have one address either: the slot that this wait lets be read is a new value to it.
+// read, so it must not see that two reads have one address either: the slot that this wait lets be read is a new value to it
+// (no read moves above it), and a slot's fragments go through an asm that waits for them before it is filled again.  An edit
+// has to keep both.
 template <int LEFT>
 __device__ __forceinline__ void stream_wait(int& slot) {
   asm volatile("s_waitcnt vmcnt(%1)" : "+s"(slot) : "n"(LEFT) : "memory");

@@ -2030,7 +2030,8 @@ class Ops:
         waves = self.skinny_resident_wg or (8 if (splits == limit or -(-n // 128) * splits >= 4 * self.compute_units) else 4)
         return per_split, splits, waves, self.skinny_stage_chunks[0 if m <= 8 else 1]
 
-    #: Matrices smaller than this many bytes stay with the resident kernel up to 16 rows: the product
+    #: Of the matrices that the streaming product does not take, those smaller than this many bytes go to the resident
+    #: kernel up to 16 rows, the others to the tiled one: the product
     #: lasts a few microseconds and the resident kernel's many small workgroups start faster.
     resident_small_bytes = 64 << 20
 
@@ -2558,9 +2559,9 @@ class Ops:
         return self._block_few_plan(x.shape[0], weight.shape[0], weight.shape[1], max_splits)
 
     def _few_rows_wide(self, m: int, n: int, k: int, max_splits: int | None) -> bool:
-        """Whether a decode-sized product runs the kernel of the steps of many rows
-        (``gemm_wide``: eight wavefronts, an iteration's staging between the halves of the one
-        before's products) instead of the tiled one: above 32 rows always (7B shape, alone, at 64
+        """Whether a decode-sized product that the block kernel leaves (``_block_few_runs``) runs ``gemm_wide``
+        (eight wavefronts, an iteration's staging between the halves of the one
+        before's products) instead of the tiled kernel: above 32 rows always (7B shape, alone, at 64
         rows: gate|up 46.7 against 50.1 us, down 27.6 against 29.3, q|k|v 10.7 against 14.4, o 9.5
         against 10.6, the head 209 against 221; at 128 rows: 59 against 72, 35 against 39, 14
         against 16, 246 against 282), from 17 rows for a matrix that runs as one range of K and
@@ -2618,9 +2619,9 @@ class Ops:
         return per_split, -(-iters // per_split), 4, x_rows, 8, depth
 
     def _resident_runs(self, m: int, n: int, k: int) -> bool:
-        """Whether the resident kernel, not the tiled one, runs a decode-sized product: small
-        matrices up to 16 rows.  (Before the weights were read with non-temporal loads it also
-        ran the widest matrices at up to eight rows; now the tiled kernel is faster there: the
+        """Whether the resident kernel, not the tiled one, runs a decode-sized product that the
+        streaming kernel leaves (``_stream_runs``): small matrices up to 16 rows.  (Before the weights were read with
+        non-temporal loads it also ran the widest matrices at up to eight rows; now the tiled kernel is faster there: the
         head of the 7B shape at eight rows in 173 against 189 us.)"""
         return m <= self.skinny_resident_rows and 2 * n * k < self.resident_small_bytes
 
