@@ -259,7 +259,7 @@ gemm_plain_kernel(TOut* __restrict__ y, const TIn* __restrict__ x, const TIn* __
 }
 
 // ---------------------------------------------------------------------------------------------
-// Few rows of bfloat16, or of rows that 16-byte loads do not divide: a workgroup owns 16 MT activation rows by 16 NT weight rows, each of its four wavefronts one range of
+// Few rows of bfloat16 (up to 32 rows: that four elements divide), or of 32-bit rows that 16-byte loads do not divide: a workgroup owns 16 MT activation rows by 16 NT weight rows, each of its four wavefronts one range of
 // K; both operands go straight from memory into registers, AHEAD slices of 64 k in flight, without LDS
 // or a barrier before the ranges' sums meet at the end: bound by reading W.
 // Lane (r, g) = (lane % 16, lane / 16) loads 16 bytes of row r: elements 4 g .. 4 g + 3 of every 16, 64 bytes of each of
@@ -403,6 +403,71 @@ gemm_plain_few_rows_kernel(TOut* __restrict__ y, const TIn* __restrict__ x, cons
       }
     }
   }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Up to 32 rows of bfloat16 whose K or strides four elements do not divide: what bounds them is the number of 2-byte loads, and
+// with a wavefront a range of K each of them touches sixteen rows.  Here a workgroup owns 16 x 16 outputs, one a thread, and
+// walks K in slices of 64 that travel memory -> registers -> LDS (two buffers, one barrier a slice, two slices of loads
+// ahead): a row's slice is 128 bytes of sixteen neighbouring lanes.  The same chains, by vector fused multiply-adds.  The
+// layout above -> this one, us at 1 / 16 / 32 rows: 18,944 x 3,583 140 / 226 / 260 -> 104 / 104 / 180, 4,608 x 2,049 60 / 66 / 85
+// -> 31 / 31 / 41, 3,584 x 9,001 195 / 192 / 308 -> 104 / 104 / 116, 512 x 511 9.4 / 11.3 / 11.5 -> 7.7 / 8.0 / 8.1.
+constexpr int UNEVEN_TILE = 16, UNEVEN_SLICE = 64, UNEVEN_MOST_ROWS = 32;
+
+template <typename TOut>
+__global__ void __launch_bounds__(256)
+gemm_plain_uneven_kernel(TOut* __restrict__ y, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                         const bf16_t* __restrict__ bias, int m, int n, int k, long x_stride, long y_stride) {
+  __shared__ __attribute__((aligned(16))) float lds[2][2][UNEVEN_TILE][UNEVEN_SLICE + 4];  // buffer, operand: x, w
+  const int row = threadIdx.x / 16, lane_k = threadIdx.x % 16 * 4;  // of both operands: what this thread fetches of a slice
+  const int m0 = blockIdx.y * UNEVEN_TILE, n0 = blockIdx.x * UNEVEN_TILE;
+  const bf16_t* const xrow = x + (size_t)min(m0 + row, m - 1) * x_stride;
+  const bf16_t* const wrow = w + (size_t)min(n0 + row, n - 1) * k;
+  float xr[2][4], wr[2][4];  // set j: a slice whose number is j modulo 2
+  auto fetch = [&](int j, int slice) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // past the end the last element again, counted as zero
+      const int at = slice * UNEVEN_SLICE + lane_k + i;
+      const float a = to_float(xrow[min(at, k - 1)]), b = to_float(wrow[min(at, k - 1)]);
+      xr[j][i] = at < k ? a : 0.f;
+      wr[j][i] = at < k ? b : 0.f;
+    }
+  };
+  auto stage = [&](int j) __attribute__((always_inline)) {
+    *reinterpret_cast<gp_f32x4*>(&lds[j][0][row][lane_k]) = gp_f32x4{xr[j][0], xr[j][1], xr[j][2], xr[j][3]};
+    *reinterpret_cast<gp_f32x4*>(&lds[j][1][row][lane_k]) = gp_f32x4{wr[j][0], wr[j][1], wr[j][2], wr[j][3]};
+  };
+  const int slices = (k + UNEVEN_SLICE - 1) / UNEVEN_SLICE, range = range_of(k) / UNEVEN_SLICE;
+  const int out_m = threadIdx.x % 16, out_n = threadIdx.x / 16;  // the output this thread owns
+  float acc = 0.f, sum = 0.f;  // the range's chain, the ranges before it
+  int range_end = min(range, slices);
+  fetch(0, 0);
+  fetch(1, 1);
+  stage(0);
+  __syncthreads();
+  auto round = [&](int s, int j) __attribute__((always_inline)) {  // slice s lies in buffer j; every thread walks the same slices
+    fetch(j, s + 2);
+    const float* a = lds[j][0][out_m];
+    const float* b = lds[j][1][out_n];
+#pragma unroll 1  // in one piece the compiler reads the whole slice into registers first: 148 of them, three wavefronts a SIMD
+    for (int part = 0; part < UNEVEN_SLICE; part += 16) {
+#pragma unroll
+      for (int kk = part; kk < part + 16; ++kk) acc = fmaf(a[kk], b[kk], acc);  // in the order of k
+    }
+    if (s + 1 == range_end) {
+      sum += acc;
+      acc = 0.f;
+      range_end = min(range_end + range, slices);
+    }
+    stage(j ^ 1);  // that buffer was last read in the slice before this one, which every thread has left
+    __syncthreads();
+  };
+  for (int s = 0; s < slices; s += 2) {
+    round(s, 0);
+    if (s + 1 < slices) round(s + 1, 1);
+  }
+  const int gm = m0 + out_m, gn = n0 + out_n;
+  if (gm < m && gn < n) y[(size_t)gm * y_stride + gn] = from_float<TOut>(bias ? sum + to_float(bias[gn]) : sum);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -657,6 +722,13 @@ int launch_plain(void* y, const void* x, const void* w, const void* bias, int m,
       hipLaunchKernelGGL((gemm_plain_few_rows_kernel<MT, NT, 2, false, TIn, TOut>), grid, dim3(256), 0, stream,      \
                          TS_PLAIN_ARGS);                                                                             \
   } while (0)
+  if constexpr (sizeof(TIn) == 2) {  // (32-bit: 3,584 x 3,583 at 16 rows 41 us by the layouts below, 51 by this one)
+    if (!vec && m <= UNEVEN_MOST_ROWS) {
+      const dim3 grid((unsigned)ceil_of(n, UNEVEN_TILE), (unsigned)ceil_of(m, UNEVEN_TILE));
+      hipLaunchKernelGGL((gemm_plain_uneven_kernel<TOut>), grid, dim3(256), 0, stream, TS_PLAIN_ARGS);
+      return ts_launch_status();
+    }
+  }
   switch (plain_kind(m, n, stream_reads)) {
     case FEW_1_1:
       TS_PLAIN_FEW(1, 1, 3);
