@@ -1078,10 +1078,11 @@ def test_attention_float32_stays_inside_its_scratch(ops, monkeypatch):
     assert torch.equal(got[1], case.run(ops, [1])[0]) and bool(got.isfinite().all())
 
 
-def test_attention_float32_keeps_values_apart(ops):
+@pytest.mark.parametrize("heads,kv_heads,dim", [(6, 2, 64), (4, 1, 256)])
+def test_attention_float32_keeps_values_apart(ops, heads, kv_heads, dim):
     """A value that is no finite number reaches the rows that see its key and no other: a token's own, in the middle of a
     block of rows; and what lies in a page behind a request's last token reaches nobody."""
-    heads, kv_heads, dim, page, seqs = 6, 2, 64, 16, [(70, 40), (21, 21), (150, 1)]
+    page, seqs = 16, [(70, 40), (21, 21), (150, 1)]
     case = PagedCase(torch.float32, heads, kv_heads, dim, page, seqs, None, seed=5)
     run = lambda: ops.attention_float32(
         case.dev(case.q), heads * dim, case.dev(case.kp), case.dev(case.vp), case.dev(case.table), case.ints(case.token_seq),
