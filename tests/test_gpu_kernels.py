@@ -1078,6 +1078,21 @@ def test_attention_float32_stays_inside_its_scratch(ops, monkeypatch):
     assert torch.equal(got[1], case.run(ops, [1])[0]) and bool(got.isfinite().all())
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim", [(6, 2, 16), (28, 4, 128), (2, 2, 256)])
+def test_attention_float32_of_many_short_prompts(ops, heads, kv_heads, dim):
+    """Rows of up to sixteen requests in one block of 16, walked by one wavefront or shared among up to sixteen: the same bits, every
+    row written."""
+    seqs = [(3, 3), (1, 1), (70, 2), (40, 1), (5, 5), *[(64 + i, 1) for i in range(17)], (90, 20), (2, 2), (33, 15), (130, 3)]
+    case = PagedCase(torch.float32, heads, kv_heads, dim, 16, seqs, None, seed=dim)
+    args = (case.dev(case.q), heads * dim, case.dev(case.kp), case.dev(case.vp), case.dev(case.table), case.ints(case.token_seq),
+            case.ints(case.positions), heads, dim ** -0.5, 30)
+    want = ops.attention_float32(*args, num_single=0, max_single_context=1)
+    torch.testing.assert_close(want, ops.paged_attention_generic(*args), **tol(torch.float32))
+    for prompts in (2, 5, len(seqs), 1000):
+        room = torch.full_like(want, float("nan"))
+        assert torch.equal(ops.attention_float32(*args, num_single=0, max_single_context=1, num_prompts=prompts, out=(room, 0)), want), prompts
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim", [(6, 2, 64), (4, 1, 256)])
 def test_attention_float32_keeps_values_apart(ops, heads, kv_heads, dim):
     """A value that is no finite number reaches the rows that see its key and no other: a token's own, in the middle of a

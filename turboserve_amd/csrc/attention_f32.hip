@@ -139,13 +139,24 @@ attention_f32_kernel(float* __restrict__ out, long out_stride, float out_scale, 
   float m_run = rule.sinks > 0.f ? (rule.sink_scores ? rule.sink_scores[row_head] : 0.f) : -INFINITY;
   float l_run = rule.sinks > 0.f ? rule.sinks : 0.f;
 
-  // Stretches of rows of one request (heads: one stretch).
+  // Stretches of rows of one request (heads: one stretch).  Rows that are tokens: the workgroups of blockIdx.z take them in turn.
+  bool row_walked = by_head;
+  int turn = by_head ? 0 : blockIdx.z;
   for (int first = 0; first < rows;) {
     const int seq = __builtin_amdgcn_readlane(row_seq, first);
     int last_row = rows - 1;
     if (!by_head) {
       const unsigned same = (unsigned)__ballot(row_seq == seq && row_valid) & 0xffffu;
       last_row = 31 - __builtin_clz(same);  // a request's tokens follow one another
+    }
+    if (!by_head) {
+      const bool taken = turn == 0;
+      turn = turn == 0 ? gridDim.z - 1 : turn - 1;
+      if (!taken) {
+        first = last_row + 1;
+        continue;
+      }
+      row_walked = row_walked || (r >= first && r <= last_row);
     }
     const int p_first = __builtin_amdgcn_readlane(row_p, first), p_last = __builtin_amdgcn_readlane(row_p, last_row);
     const int lo_first = lowest_key(p_first, rule), lo_last = lowest_key(p_last, rule);
@@ -318,7 +329,7 @@ attention_f32_kernel(float* __restrict__ out, long out_stride, float out_scale, 
       for (int b = 0; b < F32_BLOCKS; ++b) pages[b] = next_pages[b];
     }
   }
-  if (TILES || !row_valid) return;
+  if (TILES || !row_valid || !row_walked) return;
   const float inv = out_scale / l_run;
   float* to = out + (size_t)row_token * out_stride + (size_t)row_head * dim + 4 * g;
 #pragma unroll
@@ -353,7 +364,8 @@ attention_f32_combine_kernel(float* __restrict__ out, long out_stride, float out
 }  // namespace
 
 // The arguments of ts_paged_attention_generic for `tokens` tokens from first_token on (q, out, token_seq and positions are
-// the whole step's).  mode 0: rows are 16 consecutive tokens of a head; 1: the heads of one token, folded in place; 2: the
+// the whole step's).  mode 0: rows are 16 consecutive tokens of a head, whose requests max_tiles (0: one) wavefronts walk
+// side by side; 1: the heads of one token, folded in place; 2: the
 // heads of one token, the tiles side by side: partial [tokens, heads, max_tiles, dim] and ml [tokens, heads, max_tiles, 2]
 // (32-bit), max_tiles no smaller than any token's tiles: ceil((keys it can see, kept first ones apart) / 64) + 1 + ceil(keep_first / 64)
 // (a token that has more is cut there: nothing is read or written outside the scratch).
@@ -381,7 +393,7 @@ extern "C" int ts_attention_f32(void* out, const void* q, long q_stride, const v
   if (mode == 0) {
     const int waves = group < 4 ? group : 4;  // heads of one KV head side by side: they read the same keys
     block = dim3(64 * waves);
-    grid = dim3((tokens + 15) / 16, kv_heads * ((group + waves - 1) / waves));
+    grid = dim3((tokens + 15) / 16, kv_heads * ((group + waves - 1) / waves), max_tiles < 1 ? 1 : max_tiles > 16 ? 16 : max_tiles);
   } else {
     // Single tokens: no more workgroups than some thousands; one whose first tile lies past the end leaves.
     long side = mode == 2 ? max_tiles : 1;

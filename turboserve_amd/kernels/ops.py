@@ -1635,12 +1635,13 @@ class Ops:
         slopes: torch.Tensor | None = None, softcap: float = 0.0, *, num_single: int, max_single_context: int,
         chunk: int | None = None, sinks: float = 0.0, sink_scores: torch.Tensor | None = None,
         distance_bias: torch.Tensor | None = None, keep_first: int = 0, out_scale: float = 1.0,
-        out: tuple[torch.Tensor, int] | None = None,
+        out: tuple[torch.Tensor, int] | None = None, num_prompts: int = 1,
     ) -> torch.Tensor:
         """What :meth:`paged_attention_generic` computes, in 32-bit throughout, on the matrix cores' 32-bit
         instructions (:meth:`float32_attention_supported` says for which layers).  The last ``num_single`` tokens of the
         step are one request's each, holding ``max_single_context`` tokens at most; those before them
-        may be any.  A token's result does not depend on which of the two it is among: its keys are taken in tiles of 64,
+        may be any, of about ``num_prompts`` requests (which decides only how many wavefronts share
+        a tile of rows).  A token's result does not depend on which of the two it is among: its keys are taken in tiles of 64,
         folded in order, by one wavefront for 16 tokens of a head, or, for single tokens, tile by tile side by side."""
         _gpu(q, k_pages, v_pages, block_table, token_seq, positions)
         self._score_tables(heads, sinks, sink_scores, distance_bias)
@@ -1669,7 +1670,11 @@ class Ops:
                 0 if distance_bias is None else distance_bias.shape[1], int(keep_first), out_stride, float(out_scale), mode,
                 _ptr(partial), _ptr(ml), max_tiles, self.stream()), "ts_attention_f32")
 
-        launch(0, tokens - num_single, 0)
+        # Rows of several requests: 16 rows hold the last of one and some more, each a walk of its own, and a walk is as long
+        # for 3 tokens as for 16.  As many wavefronts as that comes to on average walk them side by side (60 prompts of 3 tokens, us
+        # one after the other / side by side: 28 heads of 128 on 4 63 / 32, 16 of 64 40 / 13.5, 12 of 16 27 / 9.2).
+        shares = min(16, max(1, num_prompts), 1 + round(16 * num_prompts / max(1, tokens - num_single)))
+        launch(0, tokens - num_single, 0, max_tiles=shares)
         if num_single > 0:
             seen = min(max_single_context, window or max_single_context, chunk or max_single_context)
             max_tiles = min(-(-max_single_context // 64), -(-seen // 64) + 1 + -(-keep_first // 64))

@@ -386,7 +386,7 @@ class GroupedQueryAttention(Mixer):
         if ops.float32_attention_supported(qkv, q_stride, cache.k, cache.v, out):
             return ops.attention_float32(
                 qkv, q_stride, cache.k, cache.v, table, ctx.token_seq, ctx.positions, self.num_heads, self.scale, self.window, slopes,
-                self.softcap, num_single=ctx.num_decode_seqs,
+                self.softcap, num_single=ctx.num_decode_seqs, num_prompts=ctx.num_prefill_seqs,
                 max_single_context=min(ctx.max_decode_context_len, table.shape[1] * cache.block_size), **rule)
         return ops.paged_attention_generic(
             qkv, q_stride, cache.k, cache.v, table, ctx.token_seq, ctx.positions,
