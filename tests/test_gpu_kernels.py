@@ -1054,6 +1054,20 @@ def test_attention_float32_of_many_long_requests(ops, monkeypatch, heads, kv_hea
         assert modes == 1 or all(m[1] * token <= scratch for m in launched)
 
 
+@pytest.mark.parametrize("dim,longest,mode", [(64, 64, 1), (64, 65, 2), (128, 40, 1), (256, 64, 2)])
+def test_attention_float32_of_one_tile_is_folded_in_place(ops, monkeypatch, dim, longest, mode):
+    """Single tokens that see one tile of keys leave nothing to combine: one launch, the bits of the tiles side by side."""
+    case = LongSingles([1, 2, 16, 17, 40, longest], 6, 2, dim, 16, seed=dim)
+    noting = Modes(ops.core)
+    monkeypatch.setattr(ops, "core", noting)
+    every = list(range(6))
+    got = case.run(ops, every)
+    assert [m for m in noting.seen if m[1]] == [(mode, 6)]
+    torch.testing.assert_close(got, case.run(ops, every, generic=True), **tol(torch.float32))
+    case.contexts.append(100)  # the longest request of another step's: two tiles
+    assert torch.equal(case.run(ops, every), got) and noting.seen[-1][0] == 2
+
+
 def test_attention_float32_stays_inside_its_scratch(ops, monkeypatch):
     """A caller that understates the longest context gets that many tiles' keys and no access outside the scratch, whose
     neighbours stay as they are."""

@@ -1681,6 +1681,11 @@ class Ops:
             fit = self.float32_attention_scratch // (4 * heads * max_tiles * (head_dim + 2))
             if fit < num_single and num_single * kv_heads * -(-(heads // kv_heads) // 16) > 2 * self.compute_units:
                 fit = 0
+            # One tile a token is folded where it is made, without a launch to combine (us, up to 64 keys, combined / folded: 1 and 64
+            # requests of 28 heads of 128 on 4 11.9 / 9.9 and 12.3 / 9.9, of 16 of 64 9.8 / 7.9 and 10.9 / 8.9; 256-wide heads, whose
+            # folding kernel spills some registers, 16.0 / 17.1 and 17.4 / 19.7).
+            if max_tiles == 1 and head_dim <= 128:
+                fit = 0
             most = min(num_single, fit or num_single, 65535)  # tokens of a launch: what the scratch holds and a grid takes
             group = -(-num_single // -(-num_single // most))
             partial = ml = None
