@@ -17,7 +17,7 @@ class Planner(Ops):
         self._tiled_plans, self._wide_plans, self._stream_plans, self._block_plans = {}, {}, {}, {}
         self.wide_choices, self.wide_timings = {}, {}
 
-    def gemm_block(self, x, weight, bias=None, *, plan, gated=False, sums=False, rule=None):
+    def _block_product(self, x, weight, bias, *, plan, gated, sums, rule):
         return "block", plan, plan[1] > 1 or sums
 
     def gemm_stream(self, x, weight, bias=None, *, plan, gated=False, rule=None):
@@ -151,6 +151,24 @@ def test_gated_products_of_up_to_16_rows(monkeypatch):
         kernel, plan, gated = ops.linear_swiglu(*operands(1, n, k))
         assert kernel == "stream" and plan[1] == 1 and gated, (n, k)
     assert ops.linear_swiglu(*operands(8, 27648, 5120))[0] == "tiled"
+
+
+@pytest.mark.parametrize("m", [17, 64, 128, 129, 300, 1000])
+@pytest.mark.parametrize("kind", ["sums", "one", "gated"])
+def test_a_product_looks_at_its_operands_once(monkeypatch, m, kind):
+    """Choosing the block product asks whether it takes the operands; launching it does not ask again, and the choice is worked out
+    once for all products of the same sizes: the host's share of a short prompt's step."""
+    monkeypatch.setattr("turboserve_amd.kernels.ops._gpu", lambda *tensors: None)
+    ops, asked, planned = Planner(), [], []
+    ops.time_wide_choices = False
+    monkeypatch.setattr(ops, "block_supported", lambda x, w: asked.append(1) or Ops.block_supported(x, w), raising=False)
+    for name in ("_block_plan", "_wide_plan"):
+        monkeypatch.setattr(ops, name, lambda *a, plan=getattr(ops, name): planned.append(1) or plan(*a), raising=False)
+    x, w = operands(m, 37888, 3584)
+    product = {"sums": lambda: ops.linear(x, w, for_residual=True), "one": lambda: ops.linear(x, w), "gated": lambda: ops.linear_swiglu(x, w)}[kind]
+    assert product()[0] == "block" and len(asked) == 1
+    planned.clear()
+    assert product()[0] == "block" and len(asked) == 2 and not planned
 
 
 def test_one_range_with_a_nearly_empty_last_round_is_left_to_the_tiled_product():

@@ -2021,14 +2021,16 @@ class Ops:
     @staticmethod
     def skinny_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
         """bfloat16, at most 128 rows, K a multiple of 8."""
-        return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[0] <= 128
-                and x.shape[1] % 8 == 0 and x.stride(0) % 8 == 0)
+        rows, k = x.shape[:2]
+        return (x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and rows <= 128
+                and k % 8 == 0 and x.stride(0) % 8 == 0)
 
     @staticmethod
     def skinny_supported_any_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
         """bfloat16 and K a multiple of 8: what this engine's matrix-core products take, whatever the rows."""
-        return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[1] % 8 == 0
-                and x.stride(0) % 8 == 0 and x.stride(1) == 1 and weight.is_contiguous())
+        row, one = x.stride()[:2]
+        return (x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and x.shape[1] % 8 == 0
+                and row % 8 == 0 and one == 1 and weight.is_contiguous())
 
     def _resident_plan(self, m: int, n: int, chunks: int, max_splits: int | None) -> tuple[int, int, int, int]:
         """(chunks per split, splits, wavefronts per workgroup, chunks staged at a time) of the
@@ -2163,10 +2165,12 @@ class Ops:
         """Whether ``csrc/gemm_block.hip`` takes a product: bfloat16, K a multiple of 64 (whole
         lines of 128 bytes), N of 16 (whole tiles), rows of 16-byte pieces, a block's rows within
         the 31 bits of a buffer's offsets."""
-        n, k = weight.shape
-        return (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and k % 64 == 0 and k > 0 and n % 16 == 0
-                and x.stride(1) == 1 and k <= x.stride(0) < 1 << 21 and x.stride(0) % 8 == 0 and n < 1 << 20
-                and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+        if x.dim() != 2:
+            return False
+        (n, k), (row, one) = weight.shape, x.stride()
+        return (x.shape[1] == k and k % 64 == 0 and k > 0 and n % 16 == 0 and one == 1 and k <= row < 1 << 21 and row % 8 == 0 and n < 1 << 20
+                and x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and weight.is_contiguous()
+                and (x.data_ptr() | weight.data_ptr()) % 16 == 0)
 
     def _block_plan(self, m: int, n: int, k: int, kind: str) -> tuple[int, int, int, int]:
         """(iterations of 64 per range of K, ranges, tile of weight rows, of activation rows) of the
@@ -2256,6 +2260,13 @@ class Ops:
         _gpu(x, weight, bias)
         _need(x.dim() == 2 and weight.dim() == 2 and x.shape[1] == weight.shape[1], "x must be [M, K], weight [N, K]")
         _need(self.block_supported(x, weight), "the block product takes bfloat16 rows of 16-byte pieces, K % 64 == 0 and N % 16 == 0")
+        return self._block_product(x, weight, bias, plan=plan, gated=gated, sums=sums, rule=rule)
+
+    def _block_product(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, *, plan: tuple[int, int, int, int],
+                       gated: bool, sums: bool, rule: tuple[float, float, float]) -> torch.Tensor:
+        """:meth:`gemm_block` of operands on the GPU that ``block_supported`` has been asked about: the choice of
+        a kernel asks it anyway, and a prompt of a small model is bound by the host (8 layers 2,048 wide, 33 to 256
+        tokens: asked twice and the choice worked out for every product, a step took 1,020 to 1,275 us, now 970 to 1,180)."""
         m, k = x.shape
         n = weight.shape[0]
         if bias is not None:
@@ -2268,8 +2279,9 @@ class Ops:
             out = self.rows_buffer(m, n // 2 if gated else n, torch.bfloat16, x.device)
         else:
             partial = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+        unit = glu_rule(rule) if gated else (1.0, 0.0, 0.0, 0.0)
         _check(self.core.ts_gemm_block(_ptr(partial), _ptr(out), _ptr(x), x.stride(0), _ptr(weight), _ptr(bias), m, n, k, per_split,
-                                       splits, tn, tm, 2 if gated else 1 if out is None else 0, *glu_rule(rule), self.stream()),
+                                       splits, tn, tm, 2 if gated else 1 if out is None else 0, *unit, self.stream()),
                "ts_gemm_block")
         return partial if out is None else out
 
@@ -2285,11 +2297,22 @@ class Ops:
         that adds them up, wide / block: 2,048 x 2,048 at 512 rows 20.8 / 23.9, 1,024 x 4,096 at 400 18.0 / 20.1, 1,536 x 2,048 at
         640 21.4 / 23.5; over 13 such shapes at 129 to 640 rows 4% on average)."""
         m, (n, k) = x.shape[0], weight.shape
+        block_takes = self.block_supported(x, weight) and (bias is None or bias.data_ptr() % 8 == 0)
+        block, plan, sums, runs = self._own_choice(m, n, k, kind, block_takes)
+        product = self._block_product if block else self.gemm_wide
+        return lambda: product(x, weight, bias, plan=plan, gated=kind == "gated", sums=sums, rule=rule), runs
+
+    def _own_choice(self, m: int, n: int, k: int, kind: str, block_takes: bool) -> tuple[bool, tuple[int, ...], bool, bool]:
+        """(the block product, not the wide one; its plan; whether one range stays 32-bit; whether it
+        runs untimed) of ``_own_product``.  Kept by the sizes: a prompt of a small model is bound by the host, which asks once a product."""
+        key = ("own", m, n, k, kind, block_takes, self.wide_default_rows, self.library_residual_float32)
+        known = self._block_plans.get(key)
+        if known is not None:
+            return known
         float32 = kind == "sums" and self.library_residual_float32
         wide = self._wide_plan(m, n, k, kind != "sums")
         workgroups = -(-n // (32 * wide[2])) * -(-m // wide[3]) * wide[1]
         runs = m <= self.wide_default_rows and (2 * workgroups >= self.compute_units or m * n * k < self.library_tuning_min_work)
-        block_takes = self.block_supported(x, weight) and (bias is None or bias.data_ptr() % 8 == 0)
         short = block_takes and kind == "sums" and m <= self.wide_default_rows and wide[0] <= 11
         if block_takes and not short:
             block = self._block_plan(m, n, k, kind)
@@ -2298,8 +2321,11 @@ class Ops:
             sums = float32 or (kind == "sums" and m <= self.wide_default_rows)
             workgroups = -(-n // (32 * block[2])) * -(-m // (32 * block[3])) * block[1]
             runs = runs or (self.wide_default_rows > 0 and workgroups >= self._block_fill(k, kind) * self.compute_units)
-            return lambda: self.gemm_block(x, weight, bias, plan=block, gated=kind == "gated", sums=sums, rule=rule), runs
-        return lambda: self.gemm_wide(x, weight, bias, plan=wide, gated=kind == "gated", sums=float32 or short, rule=rule), runs or short
+            choice = True, block, sums, runs
+        else:
+            choice = False, wide, float32 or short, runs or short
+        self._block_plans[key] = choice
+        return choice
 
     @staticmethod
     def _block_fill(k: int, kind: str) -> float:
@@ -2371,6 +2397,8 @@ class Ops:
         (``_own_product``).  With ``time_wide_choices`` an unknown product that is worth timing
         runs both ways here (``own()`` and ``library()``), four launches each behind a warm-up, each
         waited for, the best by device events that see the device's time alone."""
+        if not self.wide_choices and not self.time_wide_choices:
+            return untimed
         key = (self.library_rows(rows), n, k, kind)
         known = self.wide_choices.get(key)
         if known is not None:
@@ -2419,17 +2447,17 @@ class Ops:
         projection whose rows alternate gate, up, and the result is ``silu(gate) * up`` as
         bfloat16 ``[M, N / 2]`` (one range of K)."""
         _gpu(x, weight, bias)
-        _need(x.dim() == 2 and x.stride(1) == 1 and weight.dim() == 2 and weight.is_contiguous()
-              and x.shape[1] == weight.shape[1], "x must be [M, K] with unit inner stride, weight contiguous [N, K]")
-        _need(x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.shape[1] % 8 == 0 and x.stride(0) % 8 == 0,
+        shapes = "x must be [M, K] with unit inner stride, weight contiguous [N, K]"
+        _need(x.dim() == 2 and weight.dim() == 2, shapes)
+        (m, k), (row, one), (n, weight_k) = x.shape, x.stride(), weight.shape
+        _need(one == 1 and weight.is_contiguous() and k == weight_k, shapes)
+        _need(x.dtype is torch.bfloat16 and weight.dtype is torch.bfloat16 and k % 8 == 0 and row % 8 == 0,
               "the wide product takes bfloat16 and K % 8 == 0")
-        m, k = x.shape
-        n = weight.shape[0]
         if bias is not None:
             _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous(), "bias must be bfloat16 [N]")
         per_split, splits, tile, x_rows, waves = plan[:5]
         depth = plan[5] if len(plan) > 5 else 64
-        x_stride = x.stride(0) if m > 1 else max(k, x.stride(0))
+        x_stride = row if m > 1 else max(k, row)
         if gated:
             _need(splits == 1 and n % 2 == 0, "the gated result needs one range of K and an even number of weight rows")
             out = self.rows_buffer(m, n // 2, torch.bfloat16, x.device)
@@ -2547,14 +2575,15 @@ class Ops:
         rows the streaming kernel (``_stream_plan`` says where not), above the block product
         (``_block_few_plan``), else the tiled or the wide one; operands that are not 16-byte aligned go to the tiled or the resident one."""
         m, (n, k) = x.shape[0], weight.shape
-        stream = self._stream_runs(x, weight, max_splits)
+        stream = self._stream_runs(x, weight, max_splits) if m <= self.stream_max_rows else None
         if stream is not None:
             return self.gemm_stream(x, weight, bias, plan=stream)
-        if self._resident_runs(m, n, k):
+        if m <= self.skinny_resident_rows and self._resident_runs(m, n, k):
             return self.gemm_resident(x, weight, bias, max_splits=max_splits)
         block = self._block_few_runs(x, weight, bias, max_splits)
         if block is not None:
-            return self.gemm_block(x, weight, bias, plan=block, sums=True)
+            _gpu(x, weight, bias)
+            return self._block_product(x, weight, bias, plan=block, gated=False, sums=True, rule=(1.0, 0.0, 0.0))
         if self._few_rows_wide(m, n, k, max_splits):
             return self.gemm_wide(x, weight, bias, plan=self._wide_plan_few_rows(m, n, k, max_splits), sums=True)
         return self.gemm_tiled(x, weight, bias, max_splits=max_splits)
@@ -2667,7 +2696,9 @@ class Ops:
     def rows_buffer(self, rows: int, width: int, dtype: torch.dtype, device) -> torch.Tensor:
         """``[rows, width]`` for a step's activations, with room behind it up to the size a
         library product of these rows is run at."""
-        return torch.empty((self.library_rows(rows), width), dtype=dtype, device=device)[:rows]
+        size = self.library_rows(rows)
+        room = torch.empty((size, width), dtype=dtype, device=device)
+        return room if size == rows else room[:rows]
 
     @staticmethod
     def _with_room(x: torch.Tensor, rows: int) -> torch.Tensor | None:
@@ -2731,7 +2762,7 @@ class Ops:
             _gpu(x, weight, bias)
             block = self._block_few_runs(x, weight, bias, 1)
             if block is not None:
-                return self.gemm_block(x, weight, bias, plan=block, gated=True, rule=rule)
+                return self._block_product(x, weight, bias, plan=block, gated=True, sums=False, rule=rule)
             if (self._few_rows_wide(x.shape[0], weight.shape[0], weight.shape[1], 1) and weight.shape[0] % 2 == 0
                     and weight.is_contiguous() and x.stride(1) == 1):
                 wide = self._wide_plan_few_rows(x.shape[0], weight.shape[0], weight.shape[1], 1)
@@ -2776,11 +2807,11 @@ class Ops:
         the stream then gets the same unrounded addend from a prompt's step as from a decode step's."""
         if x.dtype == torch.float32:
             return self.gemm_plain(x, weight, bias)
-        _gpu(x, weight, bias)
         if x.shape[0] <= self.skinny_max_rows:
             if self.skinny_supported(x, weight):
                 return self.gemm_skinny(x, weight, bias)
             return self.gemm_plain(x, weight, bias)  # a K that 16-byte loads do not divide
+        _gpu(x, weight, bias)
         if self.skinny_supported_any_rows(x, weight):
             m, (n, k) = x.shape[0], weight.shape
             # What goes into the residual stream may stay partial sums (the norm adds them up);
