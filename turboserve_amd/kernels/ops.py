@@ -2266,7 +2266,7 @@ class Ops:
                        gated: bool, sums: bool, rule: tuple[float, float, float]) -> torch.Tensor:
         """:meth:`gemm_block` of operands on the GPU that ``block_supported`` has been asked about: the choice of
         a kernel asks it anyway, and a prompt of a small model is bound by the host (8 layers 2,048 wide, 33 to 256
-        tokens: asked twice and the choice worked out for every product, a step took 1,020 to 1,275 us, now 970 to 1,180)."""
+        tokens: asked twice and the choice worked out for every product, a step took 1,070 to 1,275 us, now 970 to 1,170)."""
         m, k = x.shape
         n = weight.shape[0]
         if bias is not None:
