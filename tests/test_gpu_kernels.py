@@ -1177,6 +1177,40 @@ def test_attention_decode_mfma(ops, heads, kv_heads, dim, page, window):
     torch.testing.assert_close(out.float().cpu(), case.expected, **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,page", ATTENTION_GEOMETRIES)
+@pytest.mark.parametrize("window,splits", [(None, 1), (None, 3), (20, 2), (300, 1)])
+def test_attention_decode_from_projected_sums(ops, monkeypatch, heads, kv_heads, dim, page, window, splits):
+    """Adding up, rotating, storing and attending in one launch against the store's launch and the attention's behind it: the
+    same bits in the pages (a token without a slot stores nothing), the same rows up to the order of the sums; contexts at the
+    edges of windows and pages, keys divided over one to three workgroups, one to nine partial sums."""
+    contexts = [70, 1, 33, 600, 129, 32, 31, 257, 1000]
+    monkeypatch.setattr(type(ops), "_decode_splits", lambda self, pairs, span: splits)
+    case = PagedCase(torch.bfloat16, heads, kv_heads, dim, page, [(c, 1) for c in contexts], window, seed=dim + 2)
+    g = torch.Generator().manual_seed(dim)
+    sums = torch.randn((1, 3, 9)[splits % 3], len(contexts), (heads + 2 * kv_heads) * dim, generator=g).to(DEV)
+    cos, sin = (t.to(DEV) for t in rotary_pair(1024, dim))
+    positions = case.ints([c - 1 for c in contexts])
+    slots = [int(case.table[s, (c - 1) // page]) * page + (c - 1) % page for s, c in enumerate(contexts)]
+    slots[1] = -1  # a padding row of a recorded step
+    slots = case.ints(slots)
+    pages = [(case.dev(case.kp).clone(), case.dev(case.vp).clone()) for _ in range(2)]
+    common = (case.dev(case.table), case.ints(case.qsl), case.ints(contexts), 0, len(contexts), heads, dim ** -0.5, window, max(contexts))
+    want = torch.zeros(len(contexts), heads * dim, dtype=torch.bfloat16, device=DEV)
+    q, stride = ops.rope_store(sums, *pages[0], cos, sin, positions, slots, heads, kv_heads, dim, page, 1023, torch.bfloat16)
+    ops.attention_decode(want, q, stride, *pages[0], *common)
+    got = torch.zeros_like(want)
+    ops.attention_decode(got, sums, 0, *pages[1], *common, projected=(cos, sin, slots, 1023))
+    for a, b in zip(*pages):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    stored = [i for i in range(len(contexts)) if i != 1]
+    torch.testing.assert_close(got[stored].float(), want[stored].float(), rtol=2.0**-7, atol=1e-6)
+
+
+def rotary_pair(capacity, dim):
+    angles = torch.outer(torch.arange(capacity).double(), 10000.0 ** (-torch.arange(dim // 2).double() * 2 / dim))
+    return angles.cos().float(), angles.sin().float()
+
+
 def prefill_blocks_of(ops, case, heads, kv_heads, dim, seqs, shuffle=None):
     """(rows per block the kernel for this geometry takes, its work list for ``seqs``)."""
     rows = ops.prefill_block_rows(dim, heads, kv_heads)

@@ -213,11 +213,10 @@ struct WindowFrags : KeyFrags, ValueFrags {};
 // 23.4).
 constexpr int DECODE_ONCE = 2;
 template <int ONCE = 0>
-__device__ __forceinline__ void load_window(WindowFrags& f, const PageGeometry& g, int w, int lo, int last,
+__device__ __forceinline__ void load_window(WindowFrags& f, const PageGeometry& g, const WindowPages& wp, int w, int lo, int last,
                                             int lane16, int group) {
   auto load8 = [](const uint16_t* p) -> Frag8 { return (ONCE & 1) ? load_once16(p) : *reinterpret_cast<const u32x4*>(p); };
   auto load8v = [](const uint16_t* p) -> Frag8 { return (ONCE & 2) ? load_once16(p) : *reinterpret_cast<const u32x4*>(p); };
-  const WindowPages wp = window_pages(g, w);
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     const int key = w + 8 * (lane16 >> 2) + 4 * t + (lane16 & 3);
@@ -232,6 +231,11 @@ __device__ __forceinline__ void load_window(WindowFrags& f, const PageGeometry& 
 #pragma unroll
   for (int n = 0; n < NT; ++n)
     f.v[n] = load8v(vp + ((long long)(16 * n + lane16) << g.block_shift));
+}
+
+template <int ONCE = 0>
+__device__ __forceinline__ void load_window(WindowFrags& f, const PageGeometry& g, int w, int lo, int last, int lane16, int group) {
+  load_window<ONCE>(f, g, window_pages(g, w), w, lo, last, lane16, group);
 }
 
 // Values of keys beyond `last` are whatever an earlier owner of the page left: clear them, so
@@ -374,78 +378,242 @@ __device__ __forceinline__ void attend(ColumnState& st, const WindowFrags& f, co
 __device__ __forceinline__ float column_sum(float l) { return groups_sum(l); }
 
 // ---------------------------------------------------------------------------------------------
-// decode: grid (splits, kv_heads * head_tiles, requests); one wavefront each.
+// decode: grid (splits, kv_heads * head_tiles, requests), DECODE_WAVES wavefronts a workgroup.  A request's windows go to its
+// workgroups in turn, a workgroup's to its wavefronts in turn (so the first ones do not depend on the context's length); the
+// wavefronts' sums meet in LDS.
+// splits == 1: the rows of `out`; otherwise
 // partial_acc [requests, heads, splits, D] float; partial_ml [requests, heads, splits, 2] float.
+// What bounds it is a chain of trips to memory before the first window's scores (lengths and pages, then sums and keys) and what a
+// launch costs beside it: so wavefronts join their sums here instead of in a second launch where one workgroup
+// takes a request, and the rotation and the store have no launch of their own.  A layer of a recorded step (us: store,
+// attention, combination before -> now, heads of 128, 7 to a KV head): one request of 640 keys 14.8 -> 11.2, of 300 (4 to a KV head) 12.5
+// -> 9.9, 8 of 8,191 34.9 -> 31.4, 64 of 128 to 1,535 40.7 -> 31.0.
 // ---------------------------------------------------------------------------------------------
-template <int ONCE>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TS_WAVES_PER_SIMD, TS_WAVES_PER_SIMD)))
-decode_kernel(float* __restrict__ partial_acc, float* __restrict__ partial_ml,
-              const uint16_t* __restrict__ q, long q_stride, const uint16_t* __restrict__ k_pages,
-              const uint16_t* __restrict__ v_pages, const int* __restrict__ block_table, int table_width,
-              const int* __restrict__ query_start_loc, const int* __restrict__ context_lens,
-              int seq_begin, int heads, int kv_heads, int block_shift, ScoreRule scale_log2, int window,
-              int keys_per_split, int splits, const int* __restrict__ max_context) {
-  // A recorded launch serves growing contexts: the longest context of the step is then read
-  // from device memory and the keys are divided evenly over the fixed number of splits.
-  if (max_context) {
-    int span = *max_context;
-    if (window > 0 && span > window + WINDOW_KEYS - 1) span = window + WINDOW_KEYS - 1;
-    const int per = (span + WINDOW_KEYS - 1 + splits - 1) / splits;
-    keys_per_split = ((per + WINDOW_KEYS - 1) / WINDOW_KEYS) * WINDOW_KEYS;
+constexpr int DECODE_WAVES = 4 * TS_WAVES_PER_SIMD;
+constexpr int DECODE_THREADS = DECODE_WAVES * TS_WAVE;
+constexpr int SUM_ROW = D + 4;    // LDS stride of a column's sums: the columns start in different banks
+constexpr int QUERY_ROW = D + 8;  // of a query (bfloat16)
+
+// The step's tokens as the projection left them: `splits` 32-bit partial sums of [tokens, (heads + 2 kv_heads) D], `stride`
+// elements apart.  A workgroup adds up and rotates its queries and its KV head's new key itself (as rope_store_kernel does, bit
+// for bit), one workgroup a KV head writes the new key and value into the pages.
+struct Projected {
+  const float* sums;
+  size_t stride;
+  int splits;
+  const float* cos_table;  // [positions, D / 2]
+  const float* sin_table;
+  const int* slots;
+};
+
+// Piece `item` of what a workgroup takes from the projection: four pairs of a query head or of the key head, or four
+// elements of the value head (`second` is `first` then).
+struct Piece {
+  int head;  // of the projection's heads
+  int at;
+  int second;
+};
+
+__device__ __forceinline__ Piece piece_of(int item, int columns, int first_head, int heads, int kv_heads, int kvh) {
+  const int row = item / (D / 8), turned = columns + 1;
+  if (row < turned) {
+    const int at = 4 * (item % (D / 8));
+    return Piece{row < columns ? first_head + row : heads + kvh, at, at + D / 2};
   }
-  const int lane = threadIdx.x;
-  const int lane16 = lane & 15;
-  const int group = lane >> 4;
-  const int split = blockIdx.x;
-  const int gsize = heads / kv_heads;
-  const int head_tiles = (gsize + 15) / 16;
-  const int kvh = blockIdx.y / head_tiles;
-  const int head_in_group = (blockIdx.y % head_tiles) * 16 + lane16;
-  const bool head_valid = head_in_group < gsize;
-  const int head = kvh * gsize + head_in_group;
-  const int seq = seq_begin + blockIdx.z;
-  const int ctx = context_lens[seq];
-  const int token = query_start_loc[seq];
-  const int p = ctx - 1;
-  const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
-  const int begin = (lo & ~(WINDOW_KEYS - 1)) + split * keys_per_split;
-  const int end = min(begin + keys_per_split, ctx);
+  const int at = 4 * min(item - turned * (D / 8), D / 4 - 1);
+  return Piece{heads + kv_heads + kvh, at, at};
+}
 
-  PageGeometry geo{k_pages, v_pages, block_table + (size_t)seq * table_width, table_width, kv_heads, kvh, block_shift,
-                   (1 << block_shift) - 1};
-  ColumnState st;
-  init_state(st);
-
-  if (begin < end) {
-    QueryFrags qf;
-    load_query(qf, head_valid ? q + (size_t)token * q_stride + (size_t)head * D : nullptr, group);
-    WindowFrags fa, fb;
-    load_window<ONCE>(fa, geo, begin, lo, p, lane16, group);
-    int w = begin;
-    while (true) {
-      if (w + WINDOW_KEYS < end) load_window<ONCE>(fb, geo, w + WINDOW_KEYS, lo, p, lane16, group);
-      if (w < lo || w + WINDOW_KEYS > ctx) clear_stale_values(fa, w, lo, p, group);
-      attend_window<true>(st, fa, qf, w, group, lo, p, scale_log2);
-      w += WINDOW_KEYS;
-      if (w >= end) break;
-      if (w + WINDOW_KEYS < end) load_window<ONCE>(fa, geo, w + WINDOW_KEYS, lo, p, lane16, group);
-      if (w < lo || w + WINDOW_KEYS > ctx) clear_stale_values(fb, w, lo, p, group);
-      attend_window<true>(st, fb, qf, w, group, lo, p, scale_log2);
-      w += WINDOW_KEYS;
-      if (w >= end) break;
+// Key p of the window at w lies in LDS, not in its page yet: its row of the scores' operand and its value in the lanes'
+// chunks.
+__device__ __forceinline__ void put_new_key(WindowFrags& f, const uint16_t* key, const uint16_t* value, int w, int p, int lane16,
+                                            int group) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (w + 8 * (lane16 >> 2) + 4 * t + (lane16 & 3) == p) {
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) f.k[t][j] = load8(key + 32 * j + 8 * group);
+      if (KTAIL && group < 2) f.ktail[t] = load8(key + 32 * KJ + 8 * group);
     }
   }
+  const int e = p - (w + 8 * group);  // 0..7 in the lanes whose chunk holds the key
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const uint32_t v = value[16 * n + lane16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (e == 2 * i) f.v[n][i] = (f.v[n][i] & 0xffff0000u) | v;
+      if (e == 2 * i + 1) f.v[n][i] = (f.v[n][i] & 0x0000ffffu) | (v << 16);
+    }
+  }
+}
 
+template <bool PROJECTED>
+__global__ void __launch_bounds__(DECODE_THREADS) __attribute__((amdgpu_waves_per_eu(TS_WAVES_PER_SIMD, TS_WAVES_PER_SIMD)))
+decode_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const int* __restrict__ context_lens,
+              const int* __restrict__ query_start_loc, const int* __restrict__ block_table, int table_width, int seq_begin,
+              int heads, int kv_heads, int splits, long q_stride, uint16_t* __restrict__ k_pages, uint16_t* __restrict__ v_pages,
+              int block_shift, int window, ScoreRule scale_log2, float* __restrict__ partial_acc, float* __restrict__ partial_ml,
+              Projected token_sums) {
+  extern __shared__ __attribute__((aligned(16))) float decode_lds[];
+  uint16_t* const queries = reinterpret_cast<uint16_t*>(decode_lds);  // [16][QUERY_ROW]
+  uint16_t* const new_key = queries + 16 * QUERY_ROW;                  // [D]
+  uint16_t* const new_value = new_key + D;                             // [D]
+  float* const ml = reinterpret_cast<float*>(new_value + D);           // [DECODE_WAVES][16][2]
+  float* const sums = ml + DECODE_WAVES * 32;                          // [DECODE_WAVES][columns][SUM_ROW]
+
+  const int lane = threadIdx.x & (TS_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TS_WAVE);
+  const int lane16 = lane & 15, group = lane >> 4;
+  const int gsize = heads / kv_heads, head_tiles = (gsize + 15) / 16;
+  const int kvh = blockIdx.y / head_tiles, tile = blockIdx.y % head_tiles;
+  const int columns = min(16, gsize - 16 * tile), first_head = kvh * gsize + 16 * tile;
+  const int seq = seq_begin + blockIdx.z;
+  // The first window's pages without a window do not wait for the context's length.
+  PageGeometry geo{k_pages, v_pages, block_table + (size_t)seq * table_width, table_width, kv_heads, kvh, block_shift,
+                   (1 << block_shift) - 1};
+  WindowPages first_pages = window_pages(geo, WINDOW_KEYS * (blockIdx.x + splits * wave));
+  const int ctx = context_lens[seq], token = query_start_loc[seq];
+  const int p = ctx - 1;
+  const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
+  const int lo_window = lo & ~(WINDOW_KEYS - 1);
+  int w = lo_window + WINDOW_KEYS * (blockIdx.x + splits * wave);
+  const int step = WINDOW_KEYS * DECODE_WAVES * splits;
+  if (window > 0) first_pages = window_pages(geo, w);
+  QueryFrags qf;
+  WindowFrags fa, fb;
+  if (PROJECTED) {
+    // What a token's heads need is asked for, then the first window; the heads are put together while the window travels.
+    // (Every load unconditional: the compiler then counts them and waits for the first ones alone.)
+    constexpr int PASSES = (17 * (D / 8) + D / 4 + DECODE_THREADS - 1) / DECODE_THREADS, BATCH = D > 128 ? 2 : 4;
+    const int items = (columns + 1) * (D / 8) + D / 4;
+    const float* row = token_sums.sums + (size_t)token * (heads + 2 * kv_heads) * D;
+    f32x4 a[PASSES][BATCH], b[PASSES][BATCH], c[PASSES], s[PASSES];
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+      const Piece piece = piece_of(threadIdx.x + i * DECODE_THREADS, columns, first_head, heads, kv_heads, kvh);
+      const float* at = row + (size_t)piece.head * D;
+#pragma unroll
+      for (int j = 0; j < BATCH; ++j) {
+        const size_t split = (size_t)min(j, token_sums.splits - 1) * token_sums.stride;
+        a[i][j] = *reinterpret_cast<const f32x4*>(at + split + piece.at);
+        b[i][j] = *reinterpret_cast<const f32x4*>(at + split + piece.second);
+      }
+      const size_t angle = (size_t)p * (D / 2) + piece.at % (D / 2);
+      c[i] = *reinterpret_cast<const f32x4*>(token_sums.cos_table + angle);
+      s[i] = *reinterpret_cast<const f32x4*>(token_sums.sin_table + angle);
+    }
+    auto put_together = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < PASSES; ++i) {
+        const int item = threadIdx.x + i * DECODE_THREADS;
+        const Piece piece = piece_of(item, columns, first_head, heads, kv_heads, kvh);
+        f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) {
+          if (j < token_sums.splits) {
+            x += a[i][j];
+            y += b[i][j];
+          }
+        }
+        for (int j = BATCH; j < token_sums.splits; ++j) {
+          const float* at = row + (size_t)piece.head * D + j * token_sums.stride;
+          x += *reinterpret_cast<const f32x4*>(at + piece.at);
+          y += *reinterpret_cast<const f32x4*>(at + piece.second);
+        }
+        if (item >= items) continue;
+        uint16_t lo4[4], hi4[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float r1 = x[e], r2 = y[e];
+          if (piece.second != piece.at) rotate_pair(x[e], y[e], c[i][e], s[i][e], r1, r2);
+          lo4[e] = (uint16_t)bf16_bits(r1);
+          hi4[e] = (uint16_t)bf16_bits(r2);
+        }
+        const u32x2 low = {lo4[0] | ((uint32_t)lo4[1] << 16), lo4[2] | ((uint32_t)lo4[3] << 16)};
+        const u32x2 high = {hi4[0] | ((uint32_t)hi4[1] << 16), hi4[2] | ((uint32_t)hi4[3] << 16)};
+        uint16_t* to = piece.head < heads ? queries + (piece.head - first_head) * QUERY_ROW : piece.head < heads + kv_heads ? new_key : new_value;
+        *reinterpret_cast<u32x2*>(to + piece.second) = high;
+        *reinterpret_cast<u32x2*>(to + piece.at) = low;
+        if (piece.head >= heads && blockIdx.x == 0 && tile == 0) {
+          const int slot = token_sums.slots[token];
+          if (slot >= 0) {
+            const size_t page = (((size_t)(slot >> block_shift) * kv_heads + kvh) << block_shift) * D;
+            const int offset = slot & geo.block_mask;
+            if (piece.head < heads + kv_heads) {
+              *reinterpret_cast<u32x2*>(k_pages + page + (size_t)offset * D + piece.at) = low;
+              *reinterpret_cast<u32x2*>(k_pages + page + (size_t)offset * D + piece.second) = high;
+            } else {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v_pages[page + ((size_t)(piece.at + e) << block_shift) + offset] = lo4[e];
+            }
+          }
+        }
+      }
+    };
+    if (w < ctx) {  // (the count of loads on their way is then known where they are waited for)
+      load_window<DECODE_ONCE>(fa, geo, first_pages, w, lo, p, lane16, group);
+      put_together();
+    } else {
+      put_together();
+    }
+    __syncthreads();
+    load_query(qf, lane16 < columns ? queries + lane16 * QUERY_ROW : nullptr, group);
+  } else if (w < ctx) {
+    load_query(qf, lane16 < columns ? q + (size_t)token * q_stride + (size_t)(first_head + lane16) * D : nullptr, group);
+    load_window<DECODE_ONCE>(fa, geo, first_pages, w, lo, p, lane16, group);
+  }
+
+  ColumnState st;
+  init_state(st);
+  auto take = [&](WindowFrags& f) __attribute__((always_inline)) {
+    if (w < lo || w + WINDOW_KEYS > ctx) clear_stale_values(f, w, lo, p, group);
+    if (PROJECTED && w + WINDOW_KEYS > p) put_new_key(f, new_key, new_value, w, p, lane16, group);
+    attend_window<true>(st, f, qf, w, group, lo, p, scale_log2);
+    w += step;
+  };
+  while (w < ctx) {
+    if (w + step < ctx) load_window<DECODE_ONCE>(fb, geo, w + step, lo, p, lane16, group);
+    take(fa);
+    if (w >= ctx) break;
+    if (w + step < ctx) load_window<DECODE_ONCE>(fa, geo, w + step, lo, p, lane16, group);
+    take(fb);
+  }
+
+  // The wavefronts' sums, each against the largest maximum of its column.
   const float l_total = column_sum(st.l);
-  if (head_valid) {
-    const size_t slot = ((size_t)blockIdx.z * heads + head) * splits + split;
-    float* acc_out = partial_acc + slot * D;
+  if (group == 0) *reinterpret_cast<f32x2*>(ml + (wave * 16 + lane16) * 2) = f32x2{st.m, l_total};
+  __syncthreads();
+  float m_max = -INFINITY;
+#pragma unroll
+  for (int v = 0; v < DECODE_WAVES; ++v) m_max = fmaxf(m_max, ml[(v * 16 + lane16) * 2]);
+  const float by = st.m == -INFINITY ? 0.f : exp2f(st.m - m_max);
+  if (lane16 < columns) {
 #pragma unroll
     for (int n = 0; n < NT; ++n)
-      *reinterpret_cast<f32x4*>(acc_out + 16 * n + 4 * group) = st.acc[n];
-    if (group == 0) {
-      partial_ml[slot * 2] = st.m;
-      partial_ml[slot * 2 + 1] = l_total;
+      *reinterpret_cast<f32x4*>(sums + (wave * columns + lane16) * SUM_ROW + 16 * n + 4 * group) = st.acc[n] * by;
+  }
+  __syncthreads();
+  for (int item = threadIdx.x; item < columns * (D / 4); item += DECODE_THREADS) {
+    const int column = item / (D / 4), d = 4 * (item % (D / 4));
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    float top = -INFINITY, den = 0.f;
+#pragma unroll
+    for (int v = 0; v < DECODE_WAVES; ++v) {
+      acc += *reinterpret_cast<const f32x4*>(sums + (v * columns + column) * SUM_ROW + d);
+      top = fmaxf(top, ml[(v * 16 + column) * 2]);
+    }
+#pragma unroll
+    for (int v = 0; v < DECODE_WAVES; ++v) {
+      const float m = ml[(v * 16 + column) * 2];
+      if (m != -INFINITY) den += ml[(v * 16 + column) * 2 + 1] * exp2f(m - top);
+    }
+    if (splits == 1) {
+      const u32x2 word = {bf16_bits(acc[0] / den) | (bf16_bits(acc[1] / den) << 16), bf16_bits(acc[2] / den) | (bf16_bits(acc[3] / den) << 16)};
+      *reinterpret_cast<u32x2*>(out + ((size_t)token * heads + first_head + column) * D + d) = word;
+    } else {
+      const size_t slot = ((size_t)blockIdx.z * heads + first_head + column) * splits + blockIdx.x;
+      *reinterpret_cast<f32x4*>(partial_acc + slot * D + d) = acc;
+      if (d == 0) *reinterpret_cast<f32x2*>(partial_ml + slot * 2) = f32x2{top, den};
     }
   }
 }
@@ -1615,39 +1783,54 @@ static void prefill_wide_shape(int heads, int kv_heads, int shift, int* per_bloc
 }  // namespace
 
 // Decode attention for the requests seq_begin .. seq_begin + requests - 1 of the step, each of
-// which brings one token.  `splits` wavefronts share each request's keys, `keys_per_split`
-// (a multiple of 32) each; partial buffers must hold requests * heads * splits entries.
-// max_context (device, may be null): the step's longest context; when given, keys_per_split is
-// derived from it on the device so that `splits * keys_per_split` covers it.
+// which brings one token, a request's windows of 32 keys divided evenly over `splits` workgroups.  With one, partial_acc and
+// partial_ml may be null; otherwise they hold requests * heads * splits entries.
+// The queries are rows of `q`, the new keys and values lie in their pages; or q is null and `sums` are the projection's
+// `sum_splits` partial sums [tokens, (heads + 2 kv_heads) D], `sum_stride` elements apart, which are added up, rotated by the
+// angles of the requests' last positions in cos_table and sin_table [.., D / 2], and stored at `slots` (negative: not stored).
+template <bool PROJECTED>
+static int launch_decode(uint16_t* out, float* partial_acc, float* partial_ml, const uint16_t* q, long q_stride, uint16_t* k_pages,
+                         uint16_t* v_pages, const int* block_table, int table_width, const int* query_start_loc,
+                         const int* context_lens, int seq_begin, int requests, int heads, int kv_heads, int shift, ScoreRule rule,
+                         int window, int splits, const Projected& token_sums, hipStream_t stream) {
+  const int gsize = heads / kv_heads, head_tiles = (gsize + 15) / 16, columns = gsize < 16 ? gsize : 16;
+  const size_t lds = (16 * QUERY_ROW + 2 * D) * 2 + (DECODE_WAVES * 32 + (size_t)DECODE_WAVES * columns * SUM_ROW) * 4;
+  static const bool raised = hipFuncSetAttribute((const void*)decode_kernel<PROJECTED>, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) == hipSuccess;
+  if (!raised) return TS_ERR_LAUNCH;
+  hipLaunchKernelGGL(decode_kernel<PROJECTED>, dim3(splits, kv_heads * head_tiles, requests), dim3(DECODE_THREADS), lds, stream, out, q,
+                     context_lens, query_start_loc, block_table, table_width, seq_begin, heads, kv_heads, splits, q_stride, k_pages,
+                     v_pages, shift, window, rule, partial_acc, partial_ml, token_sums);
+  if (splits == 1) return ts_launch_status();
+  if (hipGetLastError() != hipSuccess) return TS_ERR_LAUNCH;
+  hipLaunchKernelGGL(decode_reduce_kernel, dim3(requests, heads), dim3(REDUCE_THREADS), 0, stream, out, partial_acc, partial_ml,
+                     query_start_loc, seq_begin, heads, splits);
+  return ts_launch_status();
+}
+
 extern "C" int TS_SYM(ts_attention_decode_d)(
-    void* out, void* partial_acc, void* partial_ml, const void* q, long q_stride, const void* k_pages,
-    const void* v_pages, const int* block_table, int table_width, const int* query_start_loc,
+    void* out, void* partial_acc, void* partial_ml, const void* q, long q_stride, void* k_pages,
+    void* v_pages, const int* block_table, int table_width, const int* query_start_loc,
     const int* context_lens, int seq_begin, int requests, int heads, int kv_heads, int block_size,
-    float scale, float softcap, int window, int keys_per_split, int splits, const int* max_context, hipStream_t stream) {
+    float scale, float softcap, int window, int splits, const float* sums, long sum_stride, int sum_splits, const float* cos_table,
+    const float* sin_table, const int* slots, hipStream_t stream) {
   if (requests == 0) return TS_OK;
-  if (!out || !partial_acc || !partial_ml || !q || !k_pages || !v_pages || !block_table ||
-      !query_start_loc || !context_lens)
+  if (!out || !k_pages || !v_pages || !block_table || !query_start_loc || !context_lens || (q == nullptr) == (sums == nullptr))
     return TS_ERR_ARG;
+  if (splits > 1 && (!partial_acc || !partial_ml)) return TS_ERR_ARG;
+  if (sums && (!cos_table || !sin_table || !slots || sum_splits < 1)) return TS_ERR_ARG;
+  if (sums && (((uintptr_t)sums | (uintptr_t)cos_table | (uintptr_t)sin_table) % 16 != 0 || sum_stride % 4 != 0)) return TS_ERR_SHAPE;
   if (heads < 1 || kv_heads < 1 || heads % kv_heads != 0) return TS_ERR_SHAPE;
   if (block_size < 8 || (block_size & (block_size - 1))) return TS_ERR_SHAPE;
-  if (keys_per_split < WINDOW_KEYS || keys_per_split % WINDOW_KEYS != 0 || splits < 1 || splits > DECODE_MAX_SPLITS)
-    return TS_ERR_SHAPE;
-  if (requests > 65535) return TS_ERR_SHAPE;
+  if (splits < 1 || splits > DECODE_MAX_SPLITS || requests > 65535) return TS_ERR_SHAPE;
   int shift = 0;
   while ((1 << shift) < block_size) ++shift;
   const int head_tiles = (heads / kv_heads + 15) / 16;
   if (kv_heads * head_tiles > 65535) return TS_ERR_SHAPE;
-  dim3 grid(splits, kv_heads * head_tiles, requests);
-  // The values are read with non-temporal loads, the keys with plain ones (DECODE_ONCE).
-  hipLaunchKernelGGL(decode_kernel<DECODE_ONCE>, grid, dim3(64), 0, stream, (float*)partial_acc, (float*)partial_ml,
-                     (const uint16_t*)q, q_stride, (const uint16_t*)k_pages, (const uint16_t*)v_pages,
-                     block_table, table_width, query_start_loc, context_lens, seq_begin, heads, kv_heads,
-                     shift, score_rule(scale, softcap), window, keys_per_split, splits, max_context);
-  if (hipGetLastError() != hipSuccess) return TS_ERR_LAUNCH;
-  hipLaunchKernelGGL(decode_reduce_kernel, dim3(requests, heads), dim3(REDUCE_THREADS), 0, stream, (uint16_t*)out,
-                     (const float*)partial_acc, (const float*)partial_ml, query_start_loc, seq_begin, heads,
-                     splits);
-  return ts_launch_status();
+  const Projected token_sums = {sums, (size_t)sum_stride, sum_splits, cos_table, sin_table, slots};
+  auto launch = sums ? launch_decode<true> : launch_decode<false>;
+  return launch((uint16_t*)out, (float*)partial_acc, (float*)partial_ml, (const uint16_t*)q, q_stride, (uint16_t*)k_pages,
+                (uint16_t*)v_pages, block_table, table_width, query_start_loc, context_lens, seq_begin, requests, heads, kv_heads,
+                shift, score_rule(scale, softcap), window, splits, token_sums, stream);
 }
 
 // Prefill attention for `num_blocks` blocks of `block_rows` consecutive rows (16 or 32: what

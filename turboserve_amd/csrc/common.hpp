@@ -143,4 +143,10 @@ __device__ __forceinline__ float gated_unit(float g, float u, GluRule rule) {
   return g / (1.f + expf(-(rule.steepness * inner))) * (u + rule.up_shift);
 }
 
+// One rotation, written out so that every kernel rounds it the same way.
+__device__ __forceinline__ void rotate_pair(float x1, float x2, float c, float s, float& o1, float& o2) {
+  o1 = __builtin_fmaf(x1, c, -(x2 * s));
+  o2 = __builtin_fmaf(x2, c, x1 * s);
+}
+
 static inline int ts_launch_status() { return hipGetLastError() == hipSuccess ? TS_OK : TS_ERR_LAUNCH; }

@@ -542,12 +542,6 @@ extern "C" int ts_swiglu(void* out, const void* gate_up, int in_f32, int splits,
 // 16-byte load.  rotate == 0 skips the rotation (a position encoding that only stores).
 // slots == nullptr or a negative slot: nothing is stored for that token.
 // ---------------------------------------------------------------------------------------------
-// One rotation, written out so that every kernel rounds it the same way.
-__device__ __forceinline__ void rotate_pair(float x1, float x2, float c, float s, float& o1, float& o2) {
-  o1 = __builtin_fmaf(x1, c, -(x2 * s));
-  o2 = __builtin_fmaf(x2, c, x1 * s);
-}
-
 template <typename T, typename P>
 __global__ void rope_store_kernel(T* q_out, long q_stride, const P* proj, int splits,
                                   size_t split_stride, T* __restrict__ k_pages, T* __restrict__ v_pages,

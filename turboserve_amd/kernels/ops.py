@@ -164,7 +164,8 @@ def _attention_signatures(head_dim: int) -> dict[str, list]:
     return {
         f"ts_attention_decode_d{head_dim}": [c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p,
                                              c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
-                                             c_int, c_float, c_float, c_int, c_int, c_int, c_void_p, c_void_p],
+                                             c_int, c_float, c_float, c_int, c_int, c_void_p, c_long, c_int, c_void_p,
+                                             c_void_p, c_void_p, c_void_p],
         f"ts_attention_prefill_d{head_dim}": [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int,
                                               c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float,
                                               c_float, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
@@ -393,14 +394,6 @@ class Ops:
         self.time_wide_choices = False
         #: Compute units of the device (256 on an MI355X): the launch plans below size their grids by it.
         self.compute_units = int(torch.cuda.get_device_properties(self.device).multi_processor_count)
-        #: Wavefronts a decode attention launch aims for (each keeps two windows of loads in
-        #: flight): two per compute unit while the step has few requests x KV heads, one per SIMD
-        #: from half as many of those as there are compute units.  Measured through the engine at
-        #: the 7B shape (4 KV heads), context 8,192, two per unit against four: 3.78 against 3.83
-        #: ms a step with 4 requests, 4.11 against 4.15 with 8, 4.19 against 4.23 with 16 (context
-        #: 4,096), 6.27 against 6.28 with 32, 9.43 against 9.29 with 64.
-        self.decode_waves_few_pairs = 2 * self.compute_units
-        self.decode_waves_many_pairs = 4 * self.compute_units
         #: Wavefronts (16 weight rows x one range of K each) the resident product aims for: 16 per compute unit.
         self.skinny_resident_waves = 16 * self.compute_units
 
@@ -1839,12 +1832,17 @@ class Ops:
         max_context: int,
         max_context_dev: torch.Tensor | None = None,
         softcap: float = 0.0,
+        projected: tuple | None = None,
     ) -> None:
         """Matrix-core attention for the single-token requests ``seq_begin .. seq_begin +
         requests - 1`` of the step; writes their rows of ``out [T, heads * D]``.  ``max_context``
-        (host-known) bounds their context lengths and fixes the number of splits of the keys;
-        ``max_context_dev`` (one int32 on the device, at most ``max_context``) is the step's
-        true longest context, from which a recorded launch sizes each split."""
+        (host-known) bounds their context lengths and fixes over how many workgroups a request's keys are
+        divided; ``max_context_dev`` (one int32 on the device, at most ``max_context``) may name the step's true
+        longest context (every request divides its own keys, read from the device).
+
+        ``projected = (cos, sin, slots, max_position)``: ``q`` is the fused projection's partial sums ``[S, T, (heads + 2
+        kv_heads) D]`` (32-bit); the launch adds them up, rotates queries and keys, stores the new keys and values at
+        ``slots`` and attends, in place of :meth:`rope_store` before it (the same bits in the pages)."""
         _gpu(out, q, k_pages, v_pages, block_table, query_start_loc, context_lens, max_context_dev)
         _i32(max_context_dev, "max_context_dev")
         _i32(block_table, "block_table")
@@ -1852,29 +1850,54 @@ class Ops:
         _i32(context_lens, "context_lens")
         _check_pages(k_pages, v_pages, torch.bfloat16)
         _, kv_heads, block_size, head_dim = k_pages.shape
-        _need(self.mfma_attention_supported(q.dtype, head_dim, block_size), "geometry not taken by the matrix-core kernels")
+        _need(self.mfma_attention_supported(out.dtype, head_dim, block_size), "geometry not taken by the matrix-core kernels")
         _need(out.dtype == torch.bfloat16 and out.is_contiguous() and out.shape[1] == heads * head_dim,
               "out must be contiguous bfloat16 [T, heads * D]")
-        _need(q.is_contiguous() and q_stride >= heads * head_dim, "q does not hold [T, q_stride] rows")
         _need(heads % kv_heads == 0 and block_table.dim() == 2, "heads / block table do not fit")
         _need(seq_begin >= 0 and seq_begin + requests <= context_lens.numel() and requests <= block_table.shape[0],
               "request range outside the step")
         _need(max_context <= block_table.shape[1] * block_size, "block table does not cover the context")
+        if projected is None:
+            _need(q.dtype == torch.bfloat16 and q.is_contiguous() and q_stride >= heads * head_dim, "q does not hold [T, q_stride] rows")
+            new = (None, 0, 0, None, None, None)
+        else:
+            cos, sin, slots, max_position = projected
+            _gpu(cos, sin, slots)
+            _i32(slots, "slots")
+            tokens = slots.numel()
+            is_f32, sum_splits, stride = self._partials(q, tokens, (heads + 2 * kv_heads) * head_dim, torch.bfloat16, "projection")
+            _need(bool(is_f32) and q.dim() == 3, "the projection must be 32-bit partial sums")
+            _need(out.shape[0] >= tokens, "one row of out per token")
+            _need(cos.shape == sin.shape and cos.dim() == 2 and cos.shape[1] == head_dim // 2 and cos.dtype == sin.dtype == torch.float32
+                  and cos.is_contiguous() and sin.is_contiguous(), "cos/sin must be float32 [capacity, D/2]")
+            _need(max_position < cos.shape[0], f"position {max_position} is beyond the rotary tables ({cos.shape[0]})")
+            new = (_ptr(q), stride, sum_splits, _ptr(cos), _ptr(sin), _ptr(slots))
         span = max_context if not window else min(max_context, window + 31)
-        head_tiles = -(-(heads // kv_heads) // 16)
-        pairs = requests * kv_heads * head_tiles
-        waves = self.decode_waves_few_pairs if 2 * pairs <= self.compute_units else self.decode_waves_many_pairs
-        splits = max(1, min(-(-waves // pairs), -(-span // self.decode_min_keys), 256))
-        keys_per_split = -(-(-(-(span + 31) // splits)) // 32) * 32
-        splits = -(-(span + 31) // keys_per_split)
-        partial_acc = torch.empty((requests * heads * splits, head_dim), dtype=torch.float32, device=q.device)
-        partial_ml = torch.empty((requests * heads * splits, 2), dtype=torch.float32, device=q.device)
+        splits = self._decode_splits(requests * kv_heads * -(-(heads // kv_heads) // 16), span)
+        partial_acc = partial_ml = None
+        if splits > 1:
+            partial_acc = torch.empty((requests * heads * splits, head_dim), dtype=torch.float32, device=out.device)
+            partial_ml = torch.empty((requests * heads * splits, 2), dtype=torch.float32, device=out.device)
         lib = load_module(build.attention_module(head_dim))
         fn = getattr(lib, f"ts_attention_decode_d{head_dim}")
-        _check(fn(_ptr(out), _ptr(partial_acc), _ptr(partial_ml), _ptr(q), q_stride, _ptr(k_pages), _ptr(v_pages),
+        _check(fn(_ptr(out), _ptr(partial_acc), _ptr(partial_ml), None if projected else _ptr(q), q_stride, _ptr(k_pages), _ptr(v_pages),
                   _ptr(block_table), block_table.shape[1], _ptr(query_start_loc), _ptr(context_lens), seq_begin,
-                  requests, heads, kv_heads, block_size, float(scale), float(softcap), int(window or 0), keys_per_split, splits,
-                  _ptr(max_context_dev), self.stream()), "ts_attention_decode")
+                  requests, heads, kv_heads, block_size, float(scale), float(softcap), int(window or 0), splits,
+                  *new, self.stream()), "ts_attention_decode")
+
+    def _decode_splits(self, pairs: int, span: int) -> int:
+        """Over how many workgroups of the decode attention a request's keys are divided: ``pairs`` of request and KV head, at
+        most ``span`` keys each.
+
+        As many as give every compute unit one workgroup (a second one on a unit waits for the first: its wavefronts
+        hold all registers), none with fewer than ``decode_min_keys`` keys; spans of up to 512 keys stay whole, which saves the
+        launch that combines.  Microseconds a layer with the rotation and the store, heads of 128, 7 to a KV head, by number of
+        workgroups: one request of 300 keys 9.1 (1) 9.9 (3), of 640 13.4 (1) 10.5 (6), of 8,192 11.6 (32) 12.5 (64); 8
+        requests of 640 11.4 (4) 12.3 (2), of 8,192 29.6 (8) 33.6 (16); 32 of 2,048 31.3 (2) 38.7 (1) 35.9 (4); 64 of 129 to
+        1,525 32.1 (1) 38.4 (2)."""
+        if span <= self.decode_whole_keys:
+            return 1
+        return max(1, min(self.compute_units // pairs, -(-span // self.decode_min_keys), 256))
 
     def prefill_block_rows(self, head_dim: int, heads: int, kv_heads: int) -> int:
         """Consecutive rows of one request that a wavefront of the prefill attention kernel
@@ -1975,8 +1998,9 @@ class Ops:
                   self.stream()),
                "ts_attention_prefill")
 
-    #: Fewest keys worth a wavefront of its own.
+    #: Fewest keys worth a workgroup of the decode attention of its own; longest span that is never divided.
     decode_min_keys = 128
+    decode_whole_keys = 512
 
     # -- products -----------------------------------------------------------------------------
 

@@ -328,6 +328,10 @@ class GroupedQueryAttention(Mixer):
                 more["values"] = {"keep": kept}
             else:
                 more["values"] = {"blend": (ctx.carried[key], self.mix_weight)}
+        if not more and self.gate_name is None and scale == 1.0 and out is None:
+            attended = self._attend_projected(qkv, ctx, cache)
+            if attended is not None:
+                return attended
         q, q_stride = self.position.encode_and_store(
             qkv, self.num_heads, self.projected_kv_heads, self.head_dim, ctx, cache, **more
         )
@@ -337,6 +341,25 @@ class GroupedQueryAttention(Mixer):
         # Every head's output times the sigmoid of its gate (the projection's last columns), rounded once.
         return ops.head_gate(attended, proj, self.q_size + self.kv_size + self.v_size, self.num_heads, self.runtime.dtype,
                              scale=scale, out=out)
+
+    def _attend_projected(self, qkv: torch.Tensor, ctx, cache: PagedKVView) -> torch.Tensor | None:
+        """A step of single tokens whose projection came as 32-bit partial sums: one launch adds them up, rotates, stores and
+        attends.  ``None`` where the layer or the step asks for more than that launch does."""
+        ops = self.runtime.ops
+        if (qkv.dim() != 3 or ctx.num_prefill_seqs != 0 or ctx.num_decode_seqs != ctx.num_tokens or not self._plain_rule()
+                or not self.own_keys or not cache.writable
+                or not ops.mfma_attention_supported(self.runtime.dtype, self.head_dim, cache.block_size)):
+            return None
+        tables = self.position.rotation(self.head_dim, ctx)
+        if tables is None:
+            return None
+        table = ctx.block_tables[cache.group]
+        out = ops.rows_buffer(ctx.num_tokens, self.out_size, self.runtime.dtype, qkv.device)
+        ops.attention_decode(
+            out, qkv, 0, cache.k, cache.v, table, ctx.query_start_loc, ctx.context_lens, 0, ctx.num_decode_seqs, self.num_heads,
+            self.scale, self.window, min(ctx.max_decode_context_len, table.shape[1] * cache.block_size), ctx.max_decode_context_dev,
+            softcap=self.softcap, projected=(*tables, ctx.slot_mapping[cache.group], ctx.max_context_len - 1))
+        return out
 
     def attend(self, qkv: torch.Tensor, q_stride: int, ctx, cache: PagedKVView, *, scale: float = 1.0,
                out: tuple | None = None) -> torch.Tensor:

@@ -284,6 +284,12 @@ class PositionEncoding(Part):
         only has ``num_kv_heads = 0``: nothing is stored."""
         raise NotImplementedError
 
+    def rotation(self, head_dim: int, ctx: "StepContext") -> tuple[torch.Tensor, torch.Tensor] | None:
+        """``(cos, sin)``, 32-bit ``[positions, D / 2]``, where all :meth:`encode_and_store` does to queries and keys of
+        ``head_dim`` elements is to turn the pairs ``(i, i + D/2)`` by them: an attention kernel may then do that and the
+        store itself.  ``None``: only :meth:`encode_and_store` encodes."""
+        return None
+
     def score_slopes(self, num_heads: int) -> torch.Tensor | None:
         """An encoding may (also, or instead) act inside the scores: ``[num_heads]`` 32-bit
         slopes ``m`` on the device, for which the score of key ``j`` for the query at position

@@ -180,6 +180,13 @@ class RotaryEncoding(PositionEncoding):
         self.sin = sin.to(self.runtime.device)
         self.capacity = target
 
+    def rotation(self, head_dim, ctx):
+        # (Not for an encoding that inherits the tables and encodes in a way of its own.)
+        if self.neighbours or self.head_dim != head_dim or type(self).encode_and_store is not RotaryEncoding.encode_and_store:
+            return None
+        self.ensure_capacity(ctx.max_context_len)
+        return self.cos, self.sin
+
     def encode_and_store(self, qkv, num_heads, num_kv_heads, head_dim, ctx, cache: PagedKVView, *,
                          value_dim: int | None = None, head_norm: tuple | None = None, span_norm: tuple | None = None,
                          values: Mapping | None = None, shape: Mapping | None = None):
