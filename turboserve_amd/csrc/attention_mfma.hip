@@ -61,6 +61,9 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 
 // Matrix-core operands are kept as raw 32-bit words (two bfloat16 each) and reinterpreted with
 // __builtin_bit_cast where an instruction wants its own vector type; no unions, no aliasing.
@@ -241,7 +244,7 @@ __device__ __forceinline__ void load_window(WindowFrags& f, const PageGeometry& 
 // Values of keys beyond `last` are whatever an earlier owner of the page left: clear them, so
 // that a stale non-finite value cannot meet a zero probability.  Needed only for a window that
 // is not wholly inside lo..last.
-__device__ __forceinline__ void clear_stale_values(WindowFrags& f, int w, int lo, int last, int group) {
+__device__ __forceinline__ void clear_stale_values(ValueFrags& f, int w, int lo, int last, int group) {
   const int chunk = w + 8 * group;
   const bool live = chunk + 7 >= lo && chunk <= last;
   // Word i of a fragment holds keys chunk + 2 i (low half) and chunk + 2 i + 1 (high half).
@@ -378,16 +381,17 @@ __device__ __forceinline__ void attend(ColumnState& st, const WindowFrags& f, co
 __device__ __forceinline__ float column_sum(float l) { return groups_sum(l); }
 
 // ---------------------------------------------------------------------------------------------
-// decode: grid (splits, kv_heads * head_tiles, requests), DECODE_WAVES wavefronts a workgroup.  A request's windows go to its
+// decode: grid (splits, head_tiles * kv_heads, requests), DECODE_WAVES wavefronts a workgroup.  A request's windows go to its
 // workgroups in turn, a workgroup's to its wavefronts in turn (so the first ones do not depend on the context's length); the
 // wavefronts' sums meet in LDS.
 // splits == 1: the rows of `out`; otherwise
 // partial_acc [requests, heads, splits, D] float; partial_ml [requests, heads, splits, 2] float.
 // What bounds it is a chain of trips to memory before the first window's scores (lengths and pages, then sums and keys) and what a
 // launch costs beside it: so wavefronts join their sums here instead of in a second launch where one workgroup
-// takes a request, and the rotation and the store have no launch of their own.  A layer of a recorded step (us: store,
-// attention, combination before -> now, heads of 128, 7 to a KV head): one request of 640 keys 14.8 -> 11.2, of 300 (4 to a KV head) 12.5
-// -> 9.9, 8 of 8,191 34.9 -> 31.4, 64 of 128 to 1,535 40.7 -> 31.0.
+// takes a request, and the rotation and the store have no launch of their own.  A layer of a recorded step (us; a wavefront per
+// stretch of keys with the store and the combination launched apart -> joined in LDS -> windows staged in whole lines; heads of 128, 7 to a
+// KV head): one request of 640 keys 14.8 -> 11.2 -> 11.3, of 300 (4 to a KV head) 12.5 -> 9.9 -> 9.4, 8 of 8,191 34.9 -> 31.4 -> 30.0, 64 of
+// 128 to 1,535 40.7 -> 31.0 -> 27.0.
 // ---------------------------------------------------------------------------------------------
 constexpr int DECODE_WAVES = 4 * TS_WAVES_PER_SIMD;
 constexpr int DECODE_THREADS = DECODE_WAVES * TS_WAVE;
@@ -424,18 +428,19 @@ __device__ __forceinline__ Piece piece_of(int item, int columns, int first_head,
   return Piece{heads + kv_heads + kvh, at, at};
 }
 
-// Key p of the window at w lies in LDS, not in its page yet: its row of the scores' operand and its value in the lanes'
+// Key p of the window at w lies in LDS, not in its page yet: its row of the scores' operand, and its value in the lanes'
 // chunks.
-__device__ __forceinline__ void put_new_key(WindowFrags& f, const uint16_t* key, const uint16_t* value, int w, int p, int lane16,
-                                            int group) {
+__device__ __forceinline__ void put_new_key(KeyFrags& f, const lds_u16* key, int w, int p, int lane16, int group) {
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     if (w + 8 * (lane16 >> 2) + 4 * t + (lane16 & 3) == p) {
 #pragma unroll
-      for (int j = 0; j < KJ; ++j) f.k[t][j] = load8(key + 32 * j + 8 * group);
-      if (KTAIL && group < 2) f.ktail[t] = load8(key + 32 * KJ + 8 * group);
+      for (int j = 0; j < KJ; ++j) f.k[t][j] = *(const lds_u32x4*)(key + 32 * j + 8 * group);
+      if (KTAIL && group < 2) f.ktail[t] = *(const lds_u32x4*)(key + 32 * KJ + 8 * group);
     }
   }
+}
+__device__ __forceinline__ void put_new_value(ValueFrags& f, const lds_u16* value, int w, int p, int lane16, int group) {
   const int e = p - (w + 8 * group);  // 0..7 in the lanes whose chunk holds the key
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
@@ -448,26 +453,257 @@ __device__ __forceinline__ void put_new_key(WindowFrags& f, const uint16_t* key,
   }
 }
 
+// What a workgroup takes from the projection, on its way to registers (`ask`: every load unconditional, so that the compiler
+// counts them and waits for these alone when others are behind them) and from there (`put`) into LDS.
+struct TokenPieces {
+  static constexpr int PASSES = (17 * (D / 8) + D / 4 + DECODE_THREADS - 1) / DECODE_THREADS, BATCH = D > 128 ? 2 : 4;
+  f32x4 a[PASSES][BATCH], b[PASSES][BATCH], c[PASSES], s[PASSES];
+
+  __device__ __forceinline__ void ask(const Projected& from, const float* row, int position, int columns, int first_head, int heads,
+                                      int kv_heads, int kvh) {
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+      const Piece piece = piece_of(threadIdx.x + i * DECODE_THREADS, columns, first_head, heads, kv_heads, kvh);
+      const float* at = row + (size_t)piece.head * D;
+#pragma unroll
+      for (int j = 0; j < BATCH; ++j) {
+        const size_t split = (size_t)min(j, from.splits - 1) * from.stride;
+        a[i][j] = *reinterpret_cast<const f32x4*>(at + split + piece.at);
+        b[i][j] = *reinterpret_cast<const f32x4*>(at + split + piece.second);
+      }
+      const size_t angle = (size_t)position * (D / 2) + piece.at % (D / 2);
+      c[i] = *reinterpret_cast<const f32x4*>(from.cos_table + angle);
+      s[i] = *reinterpret_cast<const f32x4*>(from.sin_table + angle);
+    }
+  }
+
+  __device__ __forceinline__ void put(const Projected& from, const float* row, int columns, int first_head, int heads, int kv_heads,
+                                      int kvh, lds_u16* queries, lds_u16* new_key, lds_u16* new_value) {
+    const int items = (columns + 1) * (D / 8) + D / 4;
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+      const int item = threadIdx.x + i * DECODE_THREADS;
+      const Piece piece = piece_of(item, columns, first_head, heads, kv_heads, kvh);
+      f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
+#pragma unroll
+      for (int j = 0; j < BATCH; ++j) {
+        if (j < from.splits) {
+          x += a[i][j];
+          y += b[i][j];
+        }
+      }
+      for (int j = BATCH; j < from.splits; ++j) {
+        const float* at = row + (size_t)piece.head * D + j * from.stride;
+        x += *reinterpret_cast<const f32x4*>(at + piece.at);
+        y += *reinterpret_cast<const f32x4*>(at + piece.second);
+      }
+      if (item >= items) continue;
+      const bool turned = piece.second != piece.at;
+      f32x4 first, second;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float r1, r2;
+        rotate_pair(x[e], y[e], c[i][e], s[i][e], r1, r2);
+        first[e] = turned ? r1 : x[e];
+        second[e] = turned ? r2 : y[e];
+      }
+      const u32x2 low = {pack2(first[0], first[1]), pack2(first[2], first[3])};
+      const u32x2 high = {pack2(second[0], second[1]), pack2(second[2], second[3])};
+      lds_u16* to = piece.head < heads ? queries + (piece.head - first_head) * QUERY_ROW : piece.head < heads + kv_heads ? new_key : new_value;
+      *(lds_u32x2*)(to + piece.second) = high;
+      *(lds_u32x2*)(to + piece.at) = low;
+    }
+  }
+};
+
+// A window on its way to LDS in whole lines, one per wavefront (D = 64: two) beside the one in registers.  Loaded as matrix-core
+// operands an instruction takes 64 bytes of each of sixteen rows, lane by lane out of order, and a compute unit that has a
+// request to itself gets 45 GB/s; this way 58.  (Head sizes that 64 does not divide, whose pages an instruction would
+// straddle, are still loaded as operands.)
+// Keys: row r of the window, piece (r's 16 bytes) P at position (P + key(r)) % PIECES of the row, so that a piece of eight rows
+// touches every bank once.  Values: chunks of eight keys as the pages hold them, page by page.
+constexpr bool DECODE_STAGED = D % 64 == 0;
+struct Stage {
+  static constexpr int PIECES = D / 8, LOADS = D / 16, KEYS = WINDOW_KEYS * D;  // of a key row; of a window's keys (values: as many)
+  static constexpr int SLOTS = D <= 64 ? 2 : 1;
+  static constexpr int WAVE = SLOTS * 2 * KEYS;  // elements of a wavefront's ring
+  uint32_t key_off[LOADS];
+  uint32_t value_off;
+  int chunk_shift;  // log2 of the chunks of a row of values that lie side by side: 1, 2 or 4 (pages of 8, 16, more keys)
+
+  static __device__ __forceinline__ int turn(int row) { return PIECES >= 16 ? row : row / (16 / PIECES); }
+
+  __device__ __forceinline__ void init(int lane, int block_shift) {
+    chunk_shift = min(block_shift - 3, 2);
+    const int rows_mask = (1 << min(block_shift, 5)) - 1;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int at = 64 * i + lane, r = at / PIECES, piece = (at % PIECES + 4 * PIECES - turn(r)) % PIECES;
+      key_off[i] = (r & rows_mask) * (2 * D) + 16 * piece;
+    }
+    value_off = (((uint32_t)lane >> chunk_shift) << (block_shift + 1)) + 16 * (lane & ((1 << chunk_shift) - 1));
+  }
+
+  // Where the groups of eight keys of window w lie: offsets of their pages' KV head in the pools.  Pages that hold none of the
+  // keys lo..last are replaced by the nearest that does.
+  struct Place {
+    long long page[4];
+    int bytes;
+    int inside;  // of the window in pages of more than 32 keys
+  };
+  static __device__ __forceinline__ Place place(const PageGeometry& g, const WindowPages& wp, int w, int lo, int last) {
+    const int first_live = (max(w, lo) - w) >> g.block_shift, last_live = (min(w + WINDOW_KEYS - 1, last) - w) >> g.block_shift;
+    const int row = D << g.block_shift;
+    Place at;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int index = min(max((8 * i) >> g.block_shift, first_live), last_live);
+      const int low = (index & 1) ? wp.page[1] : wp.page[0], high = (index & 1) ? wp.page[3] : wp.page[2];
+      at.page[i] = ((long long)((index & 2) ? high : low) * g.kv_heads + g.kvh) * row;
+    }
+    at.bytes = row * 2;
+    at.inside = w & g.block_mask & ~(WINDOW_KEYS - 1);
+    return at;
+  }
+
+  // The window's keys or values into `to`.
+  template <bool VALUES>
+  __device__ __forceinline__ void fetch(lds_u16* to, const PageGeometry& g, const Place& place) const {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint16_t* page = (VALUES ? g.v_pages : g.k_pages) + place.page[i];
+      const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(page), 0, place.bytes, 0x00027000);
+#pragma unroll
+      for (int j = i * (LOADS / 4); j < (i + 1) * (LOADS / 4); ++j) {
+        const int off = VALUES ? (int)value_off : (int)key_off[j];
+        const int base = VALUES ? ((((64 * j) >> chunk_shift) % D) << (g.block_shift + 1)) + place.inside * 2 : place.inside * (2 * D);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, to + 512 * j, 16, off, base, 0, 2);  // non-temporal
+      }
+    }
+  }
+
+  __device__ __forceinline__ void read_keys(KeyFrags& f, const lds_u16* from, int lane16, int group) const {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int r = 8 * (lane16 >> 2) + 4 * t + (lane16 & 3);
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) f.k[t][j] = *(const lds_u32x4*)(from + r * D + 8 * ((4 * j + group + turn(r)) % PIECES));
+    }
+  }
+  __device__ __forceinline__ void read_values(ValueFrags& f, const lds_u16* from, int lane16, int group) const {
+    const int chunk = ((group >> chunk_shift) * D + lane16) << chunk_shift | (group & ((1 << chunk_shift) - 1));
+#pragma unroll
+    for (int n = 0; n < NT; ++n) f.v[n] = *(const lds_u32x4*)(from + 8 * (chunk + ((16 * n) << chunk_shift)));
+  }
+};
+
+// A wavefront's windows w, w + step, .. of a request.  `to` and `from` are its ring, the same memory: __restrict__ keeps the compiler from
+// waiting for every load in flight before every access to LDS.  So it must not see that two reads have one address: the slot that
+// a wait lets be read is a new value to it, and a slot's fragments go through an asm that waits for them before the slot is
+// filled again.  An edit has to keep both.
+template <int LEFT>
+__device__ __forceinline__ void stage_wait(int& slot) {
+  asm volatile("s_waitcnt vmcnt(%1)" : "+s"(slot) : "n"(LEFT) : "memory");
+}
+
+template <bool PROJECTED>
+__device__ __forceinline__ void decode_staged(ColumnState& st, lds_u16* __restrict__ to, const lds_u16* __restrict__ from,
+                                              lds_u16* __restrict__ queries, lds_u16* __restrict__ new_key,
+                                              lds_u16* __restrict__ new_value, const PageGeometry& geo, WindowPages pages,
+                                              const uint16_t* q_row, const Projected& token_sums, const float* sum_row, int w, int step,
+                                              int lo, int ctx, int columns, int first_head, int heads, ScoreRule rule) {
+  const int lane = threadIdx.x & (TS_WAVE - 1), lane16 = lane & 15, group = lane >> 4, p = ctx - 1;
+  Stage stage;
+  stage.init(lane, geo.block_shift);
+  QueryFrags qf;
+  TokenPieces pieces;
+  if (PROJECTED) pieces.ask(token_sums, sum_row, p, columns, first_head, heads, geo.kv_heads, geo.kvh);
+  else load_query(qf, lane16 < columns ? q_row : nullptr, group);
+  // (No load is issued for a window past the context: it would bring nothing and still pass through the unit, a microsecond for
+  // a workgroup's.  Where a branch leaves it open how many are on their way, the newest are waited for too.)
+  auto put = [&]() __attribute__((always_inline)) {
+    if (!PROJECTED) return;
+    pieces.put(token_sums, sum_row, columns, first_head, heads, geo.kv_heads, geo.kvh, queries, new_key, new_value);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  if (w >= ctx) {
+    put();
+    return;
+  }
+  int ahead = w;
+#pragma unroll
+  for (int i = 0; i < Stage::SLOTS; ++i) {
+    if (i == 0 || ahead < ctx) {
+      const Stage::Place place = Stage::place(geo, pages, ahead, lo, p);
+      stage.fetch<false>(to + i * 2 * Stage::KEYS, geo, place);
+      stage.fetch<true>(to + (i * 2 + 1) * Stage::KEYS, geo, place);
+    }
+    ahead += step;
+    pages = window_pages(geo, ahead);
+  }
+  put();
+  if (PROJECTED) {
+#pragma unroll
+    for (int j = 0; j < KJ; ++j)
+      qf.main[j] = lane16 < columns ? (Frag8) * (const lds_u32x4*)(queries + lane16 * QUERY_ROW + 32 * j + 8 * group) : Frag8{0u, 0u, 0u, 0u};
+  }
+  constexpr int LEFT = (2 * Stage::SLOTS - 1) * Stage::LOADS;  // all but the oldest keys or values
+  int slot = 0;
+  for (; w < ctx; w += step) {
+    KeyFrags keys;
+    ValueFrags values;
+    if (Stage::SLOTS == 1 || ahead - step < ctx) stage_wait<LEFT>(slot);
+    else stage_wait<0>(slot);
+    stage.read_keys(keys, from + slot * 2 * Stage::KEYS, lane16, group);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int j = 0; j < KJ; ++j) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(keys.k[t][j])::"memory");
+    }
+    const bool more = ahead < ctx;
+    const Stage::Place place = Stage::place(geo, pages, ahead, lo, p);
+    ahead += step;
+    pages = window_pages(geo, ahead);
+    if (more) stage.fetch<false>(to + slot * 2 * Stage::KEYS, geo, place);
+    if (PROJECTED && w + WINDOW_KEYS > p) put_new_key(keys, new_key, w, p, lane16, group);
+    const f32x4 s0 = score_tile(keys, 0, qf), s1 = score_tile(keys, 1, qf);
+    float alpha;
+    const Frag8 weights = softmax_window<true>(st, s0, s1, w, group, lo, p, rule, alpha);
+    if (more) stage_wait<LEFT>(slot);
+    else stage_wait<0>(slot);
+    stage.read_values(values, from + (slot * 2 + 1) * Stage::KEYS, lane16, group);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(values.v[n])::"memory");
+    if (more) stage.fetch<true>(to + (slot * 2 + 1) * Stage::KEYS, geo, place);
+    slot = slot + 1 == Stage::SLOTS ? 0 : slot + 1;
+    if (w < lo || w + WINDOW_KEYS > ctx) clear_stale_values(values, w, lo, p, group);
+    if (PROJECTED && w + WINDOW_KEYS > p) put_new_value(values, new_value, w, p, lane16, group);
+    accumulate(st, values, weights, alpha);
+  }
+}
+
 template <bool PROJECTED>
 __global__ void __launch_bounds__(DECODE_THREADS) __attribute__((amdgpu_waves_per_eu(TS_WAVES_PER_SIMD, TS_WAVES_PER_SIMD)))
 decode_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const int* __restrict__ context_lens,
               const int* __restrict__ query_start_loc, const int* __restrict__ block_table, int table_width, int seq_begin,
-              int heads, int kv_heads, int splits, long q_stride, uint16_t* __restrict__ k_pages, uint16_t* __restrict__ v_pages,
+              int kv_heads, int gsize, int splits, long q_stride, uint16_t* __restrict__ k_pages, uint16_t* __restrict__ v_pages,
               int block_shift, int window, ScoreRule scale_log2, float* __restrict__ partial_acc, float* __restrict__ partial_ml,
               Projected token_sums) {
   extern __shared__ __attribute__((aligned(16))) float decode_lds[];
-  uint16_t* const queries = reinterpret_cast<uint16_t*>(decode_lds);  // [16][QUERY_ROW]
-  uint16_t* const new_key = queries + 16 * QUERY_ROW;                  // [D]
-  uint16_t* const new_value = new_key + D;                             // [D]
-  float* const ml = reinterpret_cast<float*>(new_value + D);           // [DECODE_WAVES][16][2]
-  float* const sums = ml + DECODE_WAVES * 32;                          // [DECODE_WAVES][columns][SUM_ROW]
+  lds_u16* const queries = (lds_u16*)decode_lds;         // [16][QUERY_ROW]
+  lds_u16* const new_key = queries + 16 * QUERY_ROW;     // [D]
+  lds_u16* const new_value = new_key + D;                // [D]
+  float* const tops = decode_lds + (16 * QUERY_ROW + 2 * D) / 2;  // [DECODE_WAVES][16]
+  float* const weights = tops + DECODE_WAVES * 16;                // [DECODE_WAVES][16]
+  float* const sums = weights + DECODE_WAVES * 16;                // [DECODE_WAVES][columns][SUM_ROW], or the rings of a staged walk
 
   const int lane = threadIdx.x & (TS_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TS_WAVE);
   const int lane16 = lane & 15, group = lane >> 4;
-  const int gsize = heads / kv_heads, head_tiles = (gsize + 15) / 16;
-  const int kvh = blockIdx.y / head_tiles, tile = blockIdx.y % head_tiles;
+  const int tile = gsize > 16 ? blockIdx.y / kv_heads : 0, kvh = blockIdx.y - tile * kv_heads;
   const int columns = min(16, gsize - 16 * tile), first_head = kvh * gsize + 16 * tile;
-  const int seq = seq_begin + blockIdx.z;
+  const int heads = kv_heads * gsize, seq = seq_begin + blockIdx.z;
   // The first window's pages without a window do not wait for the context's length.
   PageGeometry geo{k_pages, v_pages, block_table + (size_t)seq * table_width, table_width, kv_heads, kvh, block_shift,
                    (1 << block_shift) - 1};
@@ -479,114 +715,71 @@ decode_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const 
   int w = lo_window + WINDOW_KEYS * (blockIdx.x + splits * wave);
   const int step = WINDOW_KEYS * DECODE_WAVES * splits;
   if (window > 0) first_pages = window_pages(geo, w);
-  QueryFrags qf;
-  WindowFrags fa, fb;
-  if (PROJECTED) {
-    // What a token's heads need is asked for, then the first window; the heads are put together while the window travels.
-    // (Every load unconditional: the compiler then counts them and waits for the first ones alone.)
-    constexpr int PASSES = (17 * (D / 8) + D / 4 + DECODE_THREADS - 1) / DECODE_THREADS, BATCH = D > 128 ? 2 : 4;
-    const int items = (columns + 1) * (D / 8) + D / 4;
-    const float* row = token_sums.sums + (size_t)token * (heads + 2 * kv_heads) * D;
-    f32x4 a[PASSES][BATCH], b[PASSES][BATCH], c[PASSES], s[PASSES];
-#pragma unroll
-    for (int i = 0; i < PASSES; ++i) {
-      const Piece piece = piece_of(threadIdx.x + i * DECODE_THREADS, columns, first_head, heads, kv_heads, kvh);
-      const float* at = row + (size_t)piece.head * D;
-#pragma unroll
-      for (int j = 0; j < BATCH; ++j) {
-        const size_t split = (size_t)min(j, token_sums.splits - 1) * token_sums.stride;
-        a[i][j] = *reinterpret_cast<const f32x4*>(at + split + piece.at);
-        b[i][j] = *reinterpret_cast<const f32x4*>(at + split + piece.second);
-      }
-      const size_t angle = (size_t)p * (D / 2) + piece.at % (D / 2);
-      c[i] = *reinterpret_cast<const f32x4*>(token_sums.cos_table + angle);
-      s[i] = *reinterpret_cast<const f32x4*>(token_sums.sin_table + angle);
-    }
-    auto put_together = [&]() __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < PASSES; ++i) {
-        const int item = threadIdx.x + i * DECODE_THREADS;
-        const Piece piece = piece_of(item, columns, first_head, heads, kv_heads, kvh);
-        f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
-#pragma unroll
-        for (int j = 0; j < BATCH; ++j) {
-          if (j < token_sums.splits) {
-            x += a[i][j];
-            y += b[i][j];
-          }
-        }
-        for (int j = BATCH; j < token_sums.splits; ++j) {
-          const float* at = row + (size_t)piece.head * D + j * token_sums.stride;
-          x += *reinterpret_cast<const f32x4*>(at + piece.at);
-          y += *reinterpret_cast<const f32x4*>(at + piece.second);
-        }
-        if (item >= items) continue;
-        uint16_t lo4[4], hi4[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float r1 = x[e], r2 = y[e];
-          if (piece.second != piece.at) rotate_pair(x[e], y[e], c[i][e], s[i][e], r1, r2);
-          lo4[e] = (uint16_t)bf16_bits(r1);
-          hi4[e] = (uint16_t)bf16_bits(r2);
-        }
-        const u32x2 low = {lo4[0] | ((uint32_t)lo4[1] << 16), lo4[2] | ((uint32_t)lo4[3] << 16)};
-        const u32x2 high = {hi4[0] | ((uint32_t)hi4[1] << 16), hi4[2] | ((uint32_t)hi4[3] << 16)};
-        uint16_t* to = piece.head < heads ? queries + (piece.head - first_head) * QUERY_ROW : piece.head < heads + kv_heads ? new_key : new_value;
-        *reinterpret_cast<u32x2*>(to + piece.second) = high;
-        *reinterpret_cast<u32x2*>(to + piece.at) = low;
-        if (piece.head >= heads && blockIdx.x == 0 && tile == 0) {
-          const int slot = token_sums.slots[token];
-          if (slot >= 0) {
-            const size_t page = (((size_t)(slot >> block_shift) * kv_heads + kvh) << block_shift) * D;
-            const int offset = slot & geo.block_mask;
-            if (piece.head < heads + kv_heads) {
-              *reinterpret_cast<u32x2*>(k_pages + page + (size_t)offset * D + piece.at) = low;
-              *reinterpret_cast<u32x2*>(k_pages + page + (size_t)offset * D + piece.second) = high;
-            } else {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) v_pages[page + ((size_t)(piece.at + e) << block_shift) + offset] = lo4[e];
-            }
-          }
-        }
-      }
-    };
-    if (w < ctx) {  // (the count of loads on their way is then known where they are waited for)
-      load_window<DECODE_ONCE>(fa, geo, first_pages, w, lo, p, lane16, group);
-      put_together();
-    } else {
-      put_together();
-    }
-    __syncthreads();
-    load_query(qf, lane16 < columns ? queries + lane16 * QUERY_ROW : nullptr, group);
-  } else if (w < ctx) {
-    load_query(qf, lane16 < columns ? q + (size_t)token * q_stride + (size_t)(first_head + lane16) * D : nullptr, group);
-    load_window<DECODE_ONCE>(fa, geo, first_pages, w, lo, p, lane16, group);
-  }
-
+  const uint16_t* q_row = PROJECTED ? nullptr : q + (size_t)token * q_stride + (size_t)(first_head + lane16) * D;
+  const float* sum_row = PROJECTED ? token_sums.sums + (size_t)token * (heads + 2 * kv_heads) * D : nullptr;
+  const int slot = PROJECTED && blockIdx.x == 0 && tile == 0 ? token_sums.slots[token] : -1;
   ColumnState st;
   init_state(st);
-  auto take = [&](WindowFrags& f) __attribute__((always_inline)) {
-    if (w < lo || w + WINDOW_KEYS > ctx) clear_stale_values(f, w, lo, p, group);
-    if (PROJECTED && w + WINDOW_KEYS > p) put_new_key(f, new_key, new_value, w, p, lane16, group);
-    attend_window<true>(st, f, qf, w, group, lo, p, scale_log2);
-    w += step;
-  };
-  while (w < ctx) {
-    if (w + step < ctx) load_window<DECODE_ONCE>(fb, geo, w + step, lo, p, lane16, group);
-    take(fa);
-    if (w >= ctx) break;
-    if (w + step < ctx) load_window<DECODE_ONCE>(fa, geo, w + step, lo, p, lane16, group);
-    take(fb);
+  if constexpr (DECODE_STAGED) {
+    lds_u16* ring = (lds_u16*)sums + wave * Stage::WAVE;
+    decode_staged<PROJECTED>(st, ring, ring, queries, new_key, new_value, geo, first_pages, q_row, token_sums, sum_row, w, step, lo,
+                             ctx, columns, first_head, heads, scale_log2);
+  } else {
+    QueryFrags qf;
+    WindowFrags fa, fb;
+    if (PROJECTED) {
+      // What a token's heads need is asked for, then the first window; the heads are put together while the window travels.
+      TokenPieces pieces;
+      pieces.ask(token_sums, sum_row, p, columns, first_head, heads, kv_heads, kvh);
+      auto put = [&]() __attribute__((always_inline)) {
+        pieces.put(token_sums, sum_row, columns, first_head, heads, kv_heads, kvh, queries, new_key, new_value);
+      };
+      if (w < ctx) {  // (the count of loads on their way is then known where they are waited for)
+        load_window<DECODE_ONCE>(fa, geo, first_pages, w, lo, p, lane16, group);
+        put();
+      } else {
+        put();
+      }
+      __syncthreads();
+      load_query(qf, lane16 < columns ? (const uint16_t*)(queries + lane16 * QUERY_ROW) : nullptr, group);
+    } else if (w < ctx) {
+      load_query(qf, lane16 < columns ? q_row : nullptr, group);
+      load_window<DECODE_ONCE>(fa, geo, first_pages, w, lo, p, lane16, group);
+    }
+    auto take = [&](WindowFrags& f) __attribute__((always_inline)) {
+      if (w < lo || w + WINDOW_KEYS > ctx) clear_stale_values(f, w, lo, p, group);
+  if (PROJECTED && w + WINDOW_KEYS > p) {
+        put_new_key(f, new_key, w, p, lane16, group);
+        put_new_value(f, new_value, w, p, lane16, group);
+      }
+      attend_window<true>(st, f, qf, w, group, lo, p, scale_log2);
+      w += step;
+    };
+    while (w < ctx) {
+      if (w + step < ctx) load_window<DECODE_ONCE>(fb, geo, w + step, lo, p, lane16, group);
+      take(fa);
+      if (w >= ctx) break;
+      if (w + step < ctx) load_window<DECODE_ONCE>(fa, geo, w + step, lo, p, lane16, group);
+      take(fb);
+    }
   }
 
+  // The new key and value into their page (not before the walk, whose waits would wait for the stores as well).
+  if (PROJECTED && slot >= 0) {
+    const size_t page = (((size_t)(slot >> block_shift) * kv_heads + kvh) << block_shift) * D;
+    const int offset = slot & geo.block_mask, at = threadIdx.x;
+    if (at < D / 8) *reinterpret_cast<u32x4*>(k_pages + page + (size_t)offset * D + 8 * at) = *(const lds_u32x4*)(new_key + 8 * at);
+    if (at < D) v_pages[page + ((size_t)at << block_shift) + offset] = new_value[at];
+  }
   // The wavefronts' sums, each against the largest maximum of its column.
   const float l_total = column_sum(st.l);
-  if (group == 0) *reinterpret_cast<f32x2*>(ml + (wave * 16 + lane16) * 2) = f32x2{st.m, l_total};
+  if (group == 0) tops[wave * 16 + lane16] = st.m;
   __syncthreads();
   float m_max = -INFINITY;
 #pragma unroll
-  for (int v = 0; v < DECODE_WAVES; ++v) m_max = fmaxf(m_max, ml[(v * 16 + lane16) * 2]);
+  for (int v = 0; v < DECODE_WAVES; ++v) m_max = fmaxf(m_max, tops[v * 16 + lane16]);
   const float by = st.m == -INFINITY ? 0.f : exp2f(st.m - m_max);
+  if (group == 0) weights[wave * 16 + lane16] = l_total * by;
   if (lane16 < columns) {
 #pragma unroll
     for (int n = 0; n < NT; ++n)
@@ -596,24 +789,24 @@ decode_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const 
   for (int item = threadIdx.x; item < columns * (D / 4); item += DECODE_THREADS) {
     const int column = item / (D / 4), d = 4 * (item % (D / 4));
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    float top = -INFINITY, den = 0.f;
+    float den = 0.f;
 #pragma unroll
     for (int v = 0; v < DECODE_WAVES; ++v) {
       acc += *reinterpret_cast<const f32x4*>(sums + (v * columns + column) * SUM_ROW + d);
-      top = fmaxf(top, ml[(v * 16 + column) * 2]);
-    }
-#pragma unroll
-    for (int v = 0; v < DECODE_WAVES; ++v) {
-      const float m = ml[(v * 16 + column) * 2];
-      if (m != -INFINITY) den += ml[(v * 16 + column) * 2 + 1] * exp2f(m - top);
+      den += weights[v * 16 + column];
     }
     if (splits == 1) {
-      const u32x2 word = {bf16_bits(acc[0] / den) | (bf16_bits(acc[1] / den) << 16), bf16_bits(acc[2] / den) | (bf16_bits(acc[3] / den) << 16)};
+      const u32x2 word = {pack2(acc[0] / den, acc[1] / den), pack2(acc[2] / den, acc[3] / den)};
       *reinterpret_cast<u32x2*>(out + ((size_t)token * heads + first_head + column) * D + d) = word;
     } else {
-      const size_t slot = ((size_t)blockIdx.z * heads + first_head + column) * splits + blockIdx.x;
-      *reinterpret_cast<f32x4*>(partial_acc + slot * D + d) = acc;
-      if (d == 0) *reinterpret_cast<f32x2*>(partial_ml + slot * 2) = f32x2{top, den};
+      const size_t at = ((size_t)blockIdx.z * heads + first_head + column) * splits + blockIdx.x;
+      *reinterpret_cast<f32x4*>(partial_acc + at * D + d) = acc;
+      if (d == 0) {
+        float top = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < DECODE_WAVES; ++v) top = fmaxf(top, tops[v * 16 + column]);
+        *reinterpret_cast<f32x2*>(partial_ml + at * 2) = f32x2{top, den};
+      }
     }
   }
 }
@@ -1794,11 +1987,12 @@ static int launch_decode(uint16_t* out, float* partial_acc, float* partial_ml, c
                          const int* context_lens, int seq_begin, int requests, int heads, int kv_heads, int shift, ScoreRule rule,
                          int window, int splits, const Projected& token_sums, hipStream_t stream) {
   const int gsize = heads / kv_heads, head_tiles = (gsize + 15) / 16, columns = gsize < 16 ? gsize : 16;
-  const size_t lds = (16 * QUERY_ROW + 2 * D) * 2 + (DECODE_WAVES * 32 + (size_t)DECODE_WAVES * columns * SUM_ROW) * 4;
-  static const bool raised = hipFuncSetAttribute((const void*)decode_kernel<PROJECTED>, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) == hipSuccess;
+  const size_t joined = (size_t)DECODE_WAVES * columns * SUM_ROW * 4, rings = DECODE_STAGED ? (size_t)DECODE_WAVES * Stage::WAVE * 2 : 0;
+  const size_t lds = (16 * QUERY_ROW + 2 * D) * 2 + DECODE_WAVES * 32 * 4 + (joined > rings ? joined : rings);
+  static const bool raised = hipFuncSetAttribute((const void*)decode_kernel<PROJECTED>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
   if (!raised) return TS_ERR_LAUNCH;
   hipLaunchKernelGGL(decode_kernel<PROJECTED>, dim3(splits, kv_heads * head_tiles, requests), dim3(DECODE_THREADS), lds, stream, out, q,
-                     context_lens, query_start_loc, block_table, table_width, seq_begin, heads, kv_heads, splits, q_stride, k_pages,
+                     context_lens, query_start_loc, block_table, table_width, seq_begin, kv_heads, gsize, splits, q_stride, k_pages,
                      v_pages, shift, window, rule, partial_acc, partial_ml, token_sums);
   if (splits == 1) return ts_launch_status();
   if (hipGetLastError() != hipSuccess) return TS_ERR_LAUNCH;

@@ -1892,9 +1892,9 @@ class Ops:
         As many as give every compute unit one workgroup (a second one on a unit waits for the first: its wavefronts
         hold all registers), none with fewer than ``decode_min_keys`` keys; spans of up to 512 keys stay whole, which saves the
         launch that combines.  Microseconds a layer with the rotation and the store, heads of 128, 7 to a KV head, by number of
-        workgroups: one request of 300 keys 9.1 (1) 9.9 (3), of 640 13.4 (1) 10.5 (6), of 8,192 11.6 (32) 12.5 (64); 8
-        requests of 640 11.4 (4) 12.3 (2), of 8,192 29.6 (8) 33.6 (16); 32 of 2,048 31.3 (2) 38.7 (1) 35.9 (4); 64 of 129 to
-        1,525 32.1 (1) 38.4 (2)."""
+        workgroups: one request of 300 keys 8.5 (1) 8.9 (3), of 640 10.6 (1) 8.9 (6), of 8,192 10.7 (32) 11.3 (64); 8
+        requests of 640 10.2 (4) 11.4 (2), of 8,192 26.6 (8) 29.8 (16); 32 of 2,048 28.6 (2) 30.7 (1) 31.7 (4); 64 of 129 to
+        1,525 26.2 (1) 32.0 (2)."""
         if span <= self.decode_whole_keys:
             return 1
         return max(1, min(self.compute_units // pairs, -(-span // self.decode_min_keys), 256))
