@@ -12,6 +12,8 @@
 // through registers and meet at a barrier every 128 of K; with the SwiGLU where that is in the result): 2,048 x 2,048 4.4 -> 4.0, 2,048 x
 // 8,192 12.2 -> 7.7, 8,192 x 2,048 12.3 -> 7.3, q|k|v [4608, 3584] 8.6 -> 7.9, o [3584, 3584] 8.4 -> 6.2, down [3584, 18944]
 // 24.5 -> 22.0, gate|up [16384, 2048] 17.7 -> 13.4, [37888, 3584] 46.9 -> 41.0, the head [152064, 3584] 178 -> 153 (7.1 TB/s).
+// Without loads past the end and past the eighth row, and with the bias asked for at the start: q|k|v 7.8 -> 7.4, [10304, 2048]
+// 10.9 -> 10.4, 2,048 x 8,192 8.15 -> 7.97, gate|up [16384, 2048] 13.3 -> 13.0, the long ones within 1%.
 #include "common.hpp"
 
 namespace {
@@ -25,11 +27,13 @@ typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 
 constexpr int STREAM_WAVES = 4;
 
-template <int NT>
+// NT tiles of sixteen weight rows, XT of eight activation rows.
+template <int NT, int XT>
 struct Ring {
-  static constexpr int SLICE = 64, TILE = 16 * SLICE, LOADS = 2 * (NT + 1);  // of a tile of sixteen rows; of a slice
-  static constexpr int SLOTS = 80 * 1024 / (STREAM_WAVES * (NT + 1) * TILE * 2);  // two workgroups a compute unit
-  static constexpr int WAVE = SLOTS * (NT + 1) * TILE;                          // elements of a wavefront's ring
+  static constexpr int SLICE = 64, TILE = 16 * SLICE, HALF = 8 * SLICE, LOADS = 2 * NT + XT;  // of sixteen rows; of eight; of a slice
+  static constexpr int SLOT = NT * TILE + XT * HALF;
+  static constexpr int SLOTS = 80 * 1024 / (STREAM_WAVES * SLOT * 2);  // two workgroups a compute unit
+  static constexpr int WAVE = SLOTS * SLOT;                            // elements of a wavefront's ring
   static constexpr size_t BYTES = (size_t)STREAM_WAVES * WAVE * 2;
   static_assert(SLOTS >= 2 && (SLOTS - 1) * LOADS < 64 && 2 * BYTES <= 160 * 1024, "a ring of at least two slices, counted by vmcnt");
   static_assert(WAVE * 2 >= NT * 1024, "a wavefront's sums fit its ring");
@@ -43,14 +47,23 @@ template <int LEFT>
 __device__ __forceinline__ void stream_wait(int& slot) {
   asm volatile("s_waitcnt vmcnt(%1)" : "+s"(slot) : "n"(LEFT) : "memory");
 }
+// With `left` (at most MOST) slices of LOADS loads each still on their way behind the one that is waited for.
+template <int LOADS, int MOST>
+__device__ __forceinline__ void stream_wait_for(int left, int& slot) {
+  if constexpr (MOST > 0) {
+    if (left < MOST) return stream_wait_for<LOADS, MOST - 1>(left, slot);
+  }
+  stream_wait<MOST * LOADS>(slot);
+}
 
-// acc[t][i]: weight row n0 + 16 t + 4 (lane / 16) + i, activation row lane % 16, over slices first .. last - 1 of 64 k.
-template <int NT, int SLOTS>
+// acc[t][i]: weight row n0 + 16 t + 4 (lane / 16) + i, activation row lane % 16 (lane % 8 with XT = 1), over slices first .. last - 1
+// of 64 k.
+template <int NT, int XT>
 __device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, const uint16_t* __restrict__ x,
                                              const uint16_t* __restrict__ w, int m, int n, int k, long x_stride, int n0, int first,
                                              int last, f32x4* acc) {
-  typedef Ring<NT> R;
-  constexpr int SLICE = R::SLICE, TILE = R::TILE;
+  typedef Ring<NT, XT> R;
+  constexpr int SLICE = R::SLICE, TILE = R::TILE, HALF = R::HALF, SLOTS = R::SLOTS;
   const int count = last - first;
   if (count <= 0) return;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
@@ -61,33 +74,32 @@ __device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds
   const size_t wbytes = (size_t)min(n - n0, 16 * NT) * k * 2, xbytes = ((size_t)(m - 1) * x_stride + k) * 2;
   const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w + (size_t)n0 * k), 0, (int)wbytes, 0x00027000);
   const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, (int)xbytes, 0x00027000);
-  uint32_t woff[2 * NT], xoff[2];
+  uint32_t woff[2 * NT], xoff[XT];
 #pragma unroll
   for (int j = 0; j < 2 * NT; ++j) woff[j] = ((uint32_t)(8 * j + row8) * (uint32_t)k + first * SLICE + 8 * (piece ^ (j & 1 ? 4 : 0))) * 2;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) xoff[j] = ((uint32_t)(8 * j + row8) * (uint32_t)x_stride + first * SLICE + 8 * (piece ^ (j & 1 ? 4 : 0))) * 2;
+  for (int j = 0; j < XT; ++j) xoff[j] = ((uint32_t)(8 * j + row8) * (uint32_t)x_stride + first * SLICE + 8 * (piece ^ (j & 1 ? 4 : 0))) * 2;
   auto fetch = [&](int i, int slot) __attribute__((always_inline)) {
-    const uint32_t at = i < count ? (uint32_t)i * (SLICE * 2) : 0x80000000u;  // past the end: outside the buffers, nothing is fetched
-    lds_u16* base = to + slot * (NT + 1) * TILE;
+    const uint32_t at = (uint32_t)i * (SLICE * 2);
+    lds_u16* base = to + slot * R::SLOT;
 #pragma unroll
     for (int j = 0; j < 2 * NT; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, base + j * (TILE / 2), 16, (int)(woff[j] + at), 0, 0, 2);  // non-temporal
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, base + j * HALF, 16, (int)(woff[j] + at), 0, 0, 2);  // non-temporal
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, base + NT * TILE + j * (TILE / 2), 16, (int)(xoff[j] + at), 0, 0, 0);
+    for (int j = 0; j < XT; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, base + NT * TILE + j * HALF, 16, (int)(xoff[j] + at), 0, 0, 0);
   };
   struct Frags {
     u32x4 x[2], w[NT][2];
   };
-  const int key = (r >> 1) & 7;
+  const int key = (r >> 1) & 7, x_row = r & (8 * XT - 1);
   auto read = [&](Frags& f, int slot) __attribute__((always_inline)) {
-    const lds_u16* base = from + slot * (NT + 1) * TILE + r * SLICE;
+    const lds_u16* base = from + slot * R::SLOT;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      const int at = 8 * ((4 * c + g) ^ key);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) f.w[t][c] = *(const lds_u32x4*)(base + t * TILE + at);
-      f.x[c] = *(const lds_u32x4*)(base + NT * TILE + at);
+      for (int t = 0; t < NT; ++t) f.w[t][c] = *(const lds_u32x4*)(base + t * TILE + r * SLICE + 8 * ((4 * c + g) ^ key));
+      f.x[c] = *(const lds_u32x4*)(base + NT * TILE + x_row * SLICE + 8 * ((4 * c + g) ^ (x_row >> 1)));
     }
   };
   auto consume = [&](Frags& f, int left) __attribute__((always_inline)) {  // left: elements of the slice inside the row
@@ -103,56 +115,78 @@ __device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds
       }
     }
   };
-#pragma unroll
-  for (int j = 0; j < SLOTS; ++j) fetch(j, j);
-  int slot = 0;
-  stream_wait<(SLOTS - 1) * R::LOADS>(slot);
-  Frags f[2];
-  read(f[0], slot);
-  auto round = [&](int i, Frags& now, Frags& next) __attribute__((always_inline)) {
-    // `now` is in registers: its slot is free.
+  auto arrived = [&](Frags& f) __attribute__((always_inline)) {  // in registers: the slot is free
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(now.w[t][c])::"memory");
-      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(now.x[c])::"memory");
+      for (int t = 0; t < NT; ++t) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f.w[t][c])::"memory");
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f.x[c])::"memory");
     }
+  };
+  // No load is issued past the end: one that brings nothing still takes its turn in the unit's memory path, and a ring's worth
+  // of them behind every wavefront made a short product's end (or the next workgroup's start) a microsecond longer.
+#pragma unroll
+  for (int j = 0; j < SLOTS; ++j)
+    if (j < count) fetch(j, j);
+  int slot = 0;
+  stream_wait_for<R::LOADS, SLOTS - 1>(count - 1, slot);
+  Frags f[2];
+  read(f[0], slot);
+  auto round = [&](int i, Frags& now, Frags& next) __attribute__((always_inline)) {
+    arrived(now);
     fetch(i + SLOTS, slot);
     slot = slot + 1 == SLOTS ? 0 : slot + 1;
     stream_wait<(SLOTS - 1) * R::LOADS>(slot);
     read(next, slot);
     consume(now, SLICE);
   };
-  int i = 0;  // the last slice alone may be cut short
-  for (; i + 2 < count; i += 2) {
+  int i = 0;
+  for (; i + SLOTS + 1 < count; i += 2) {
     round(i, f[0], f[1]);
     round(i + 1, f[1], f[0]);
   }
-  const int left = k - (last - 1) * SLICE;
-  if (i + 1 < count) {
+  if (i + SLOTS < count) {
     round(i, f[0], f[1]);
-    consume(f[1], left);
-  } else {
-    consume(f[0], left);
+    arrived(f[1]);
+    f[0] = f[1];
+    ++i;
   }
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // loads past the end
+  // What is left lies in the ring or is on its way there: slice i in f[0].
+  for (; i + 1 < count; ++i) {
+    arrived(f[0]);
+    f[1] = f[0];
+    slot = slot + 1 == SLOTS ? 0 : slot + 1;
+    stream_wait_for<R::LOADS, SLOTS - 2>(count - i - 2, slot);
+    read(f[0], slot);
+    consume(f[1], SLICE);
+  }
+  consume(f[0], k - (last - 1) * SLICE);  // the last slice alone may be cut short
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
 // partial: float [splits, m, n], or, GATED, out: bfloat16 [m, n / 2], the gated unit (common.hpp) of rows that alternate gate, up.
-template <int NT, bool GATED>
+template <int NT, int XT, bool GATED>
 __global__ void __launch_bounds__(64 * STREAM_WAVES)
 gemm_stream_kernel(float* __restrict__ partial, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, long x_stride,
                    const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int m, int n, int k, int per_wave, GluRule rule) {
   extern __shared__ __attribute__((aligned(16))) uint16_t ring[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n0 = blockIdx.x * 16 * NT, split = blockIdx.y;
-  const int total = (k + Ring<NT>::SLICE - 1) / Ring<NT>::SLICE;
+  typedef Ring<NT, XT> R;
+  const int total = (k + R::SLICE - 1) / R::SLICE;
   const int first = (split * STREAM_WAVES + wave) * per_wave, last = min(first + per_wave, total);
   f32x4 acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  lds_u16* mine = (lds_u16*)ring + wave * Ring<NT>::WAVE;
-  stream_range<NT, Ring<NT>::SLOTS>(mine, mine, x, w, m, n, k, x_stride, n0, first, last, acc);
+  // The bias is asked for with the first slices, not behind the last.
+  const int col = n0 + 16 * min(wave, NT - 1) + 4 * (lane >> 4);
+  uint16_t shift[4] = {0, 0, 0, 0};
+  if (bias && split == 0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) shift[i] = bias[min(col + i, n - 1)];
+  }
+  lds_u16* mine = (lds_u16*)ring + wave * R::WAVE;
+  stream_range<NT, XT>(mine, mine, x, w, m, n, k, x_stride, n0, first, last, acc);
   // The quarters' sums meet in the rings; wavefront v adds up and stores tile v.
 #pragma unroll
   for (int t = 0; t < NT; ++t) ((lds_f32x4*)mine)[t * 64 + lane] = acc[t];
@@ -160,12 +194,12 @@ gemm_stream_kernel(float* __restrict__ partial, uint16_t* __restrict__ out, cons
   if (wave >= NT) return;
   f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int v = 0; v < STREAM_WAVES; ++v) sum += ((lds_f32x4*)((lds_u16*)ring + v * Ring<NT>::WAVE))[wave * 64 + lane];
-  const int row = lane & 15, col = n0 + 16 * wave + 4 * (lane >> 4);
+  for (int v = 0; v < STREAM_WAVES; ++v) sum += ((lds_f32x4*)((lds_u16*)ring + v * R::WAVE))[wave * 64 + lane];
+  const int row = lane & 15;
   if (row >= m || col >= n) return;
   if (bias && split == 0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sum[i] += to_float(bf16_t{bias[min(col + i, n - 1)]});
+    for (int i = 0; i < 4; ++i) sum[i] += to_float(bf16_t{shift[i]});
   }
   if (GATED) {  // n is even: the first pair lies inside
     uint16_t* at = out + (size_t)row * (n / 2) + col / 2;
@@ -183,18 +217,18 @@ gemm_stream_kernel(float* __restrict__ partial, uint16_t* __restrict__ out, cons
   }
 }
 
-template <int NT, bool GATED>
+template <int NT, int XT, bool GATED>
 int launch_stream(float* partial, void* out, const void* x, long x_stride, const void* w, const void* bias, int m, int n, int k,
                   int per_wave, int splits, GluRule rule, hipStream_t stream) {
+  constexpr size_t BYTES = Ring<NT, XT>::BYTES;
   static bool raised = false;  // per process; the attribute belongs to the kernel
   if (!raised) {
-    if (hipFuncSetAttribute((const void*)gemm_stream_kernel<NT, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)Ring<NT>::BYTES) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)gemm_stream_kernel<NT, XT, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)BYTES) != hipSuccess)
       return TS_ERR_LAUNCH;
     raised = true;
   }
-  hipLaunchKernelGGL((gemm_stream_kernel<NT, GATED>), dim3((n + 16 * NT - 1) / (16 * NT), splits), dim3(64 * STREAM_WAVES),
-                     Ring<NT>::BYTES, stream, partial, (uint16_t*)out, (const uint16_t*)x, x_stride, (const uint16_t*)w,
+  hipLaunchKernelGGL((gemm_stream_kernel<NT, XT, GATED>), dim3((n + 16 * NT - 1) / (16 * NT), splits), dim3(64 * STREAM_WAVES),
+                     BYTES, stream, partial, (uint16_t*)out, (const uint16_t*)x, x_stride, (const uint16_t*)w,
                      (const uint16_t*)bias, m, n, k, per_wave, rule);
   return ts_launch_status();
 }
@@ -216,7 +250,10 @@ extern "C" int ts_gemm_stream(float* partial, void* out, const void* x, long x_s
   if (splits != ((k + 63) / 64 + 4L * per_wave - 1) / (4L * per_wave)) return TS_ERR_SHAPE;
   if (out && (splits != 1 || n % 2 != 0)) return TS_ERR_ARG;
   const GluRule rule = {steepness, limit, up_shift, cubic};
-#define TS_STREAM(NT, GATED) return launch_stream<NT, GATED>(partial, out, x, x_stride, w, bias, m, n, k, per_wave, splits, rule, stream)
+  // Up to eight rows are one load a slice instead of two, and leave room for a slice more in the ring.
+#define TS_STREAM(NT, GATED)                                                                                                                  \
+  return m <= 8 ? launch_stream<NT, 1, GATED>(partial, out, x, x_stride, w, bias, m, n, k, per_wave, splits, rule, stream)                   \
+                : launch_stream<NT, 2, GATED>(partial, out, x, x_stride, w, bias, m, n, k, per_wave, splits, rule, stream)
   if (tile == 1) {
     if (out) TS_STREAM(1, true);
     TS_STREAM(1, false);
