@@ -28,6 +28,8 @@
 // (11.1); at 128 rows 50 (60), 33 (37), 14.5 (15.3), 13.7 (14.1).
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -88,10 +90,32 @@ struct BlockRing {
   static constexpr int ROWS = 160 * 1024 / (BLOCK_DEPTH * 2);
   static constexpr bool fits(int w, int x) { return 32 * (w * TN + x * TM) <= ROWS; }
   static constexpr int W = fits(6, 5) ? 6 : fits(5, 4) ? 5 : fits(4, 3) ? 4 : 3, X = fits(W, W) ? W : W - 1;
-  static constexpr int LEFT = (W - 2) * TN + (X - 2) * TM;
+  // Loads of w iterations of the weights and x of the activations behind the one that is waited for, as far as they are asked for.
+  static constexpr int left(int w, int x) { return (w < W - 2 ? w : W - 2) * TN + (x < X - 2 ? x : X - 2) * TM; }
+  static constexpr int left_first(int behind) { return (behind < W - 2 ? behind : W - 2) * TN + (behind < X - 1 ? behind : X - 1) * TM; }
+  static constexpr int LEFT = left(W, X);
   static constexpr size_t BYTES = (size_t)32 * (W * TN + X * TM) * BLOCK_DEPTH * 2;
   static_assert(fits(W, X) && LEFT + TM < 64, "the rings must fit the LDS of a compute unit, their loads vmcnt");
 };
+
+// The wait of an iteration behind which only `behind` more than the next one's loads have been issued: theirs may be on
+// their way.
+template <typename Ring, int MOST>
+__device__ __forceinline__ void block_wait_for(int behind) {
+  if constexpr (MOST > 0) {
+    if (behind < MOST) return block_wait_for<Ring, MOST - 1>(behind);
+  }
+  block_wait<Ring::left(MOST, MOST)>();
+}
+// The first iteration's wait: `behind` more iterations have been asked for, of the newest the activations alone where the weights' ring
+// has no slot for it yet.
+template <typename Ring, int MOST>
+__device__ __forceinline__ void block_wait_first(int behind) {
+  if constexpr (MOST > 0) {
+    if (behind < MOST) return block_wait_first<Ring, MOST - 1>(behind);
+  }
+  block_wait<Ring::left_first(MOST)>();
+}
 
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
@@ -184,17 +208,16 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
 
   // Iteration i of the range: its weight rows lie in slot i % RW of their ring, its activation rows in slot i % RX of theirs.
   const int count = last - first;
-  auto step = [&](int i) __attribute__((always_inline)) { return first + min(i, count - 1); };
-  const int outside = (int)0x80000000;  // past every buffer's end: nothing is fetched for an iteration past the range's
 #pragma unroll
   for (int s = 0; s < RX; ++s) {
+    if (s >= count) continue;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-      if (s < RW - 1) load_w(j, s < count ? woff : outside, step(s), s);
+      if (s < RW - 1) load_w(j, woff, first + s, s);
 #pragma unroll
-    for (int j = 0; j < TM; ++j) load_x(j, s < count ? xoff : outside, step(s), s);
+    for (int j = 0; j < TM; ++j) load_x(j, xoff, first + s, s);
   }
-  block_wait<Ring::LEFT + TM>();
+  block_wait_first<Ring, RX - 1>(count - 1);
 #pragma unroll
   for (int b = 0; b < TM; ++b) xf[0][b] = read_x(0, 0, b);
 #pragma unroll
@@ -208,16 +231,16 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   constexpr int FREE = TN > 4 ? 2 : 1;              // the barrier stands before this tile of step 1
   constexpr int BEHIND = TM + FREE;                 // fragments of the next iteration read behind it, with those of each tile done
   int ws = 0, xs = 0;
-  for (int it = 0; it < count; ++it) {
+  // W_LOADS, X_LOADS: there is an iteration it + RW - 1, it + RX.
+  auto iteration = [&](int it, auto W_LOADS, auto X_LOADS) __attribute__((always_inline)) {
     // The offsets of the other rows are added up in each iteration: kept, they would take registers that the sums need.
     asm volatile("" : "+v"(woff), "+v"(xoff));
-    const int next_w = step(it + RW - 1), next_x = step(it + RX);
-    const int from_w_at = it + RW - 1 < count ? woff : outside, from_x_at = it + RX < count ? xoff : outside;
+    const int next_w = first + it + RW - 1, next_x = first + it + RX;
     const int free_w = ws == 0 ? RW - 1 : ws - 1, free_x = xs;
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
       TS_PIN;
-      load_w(a, from_w_at, next_w, free_w);
+      if constexpr (W_LOADS) load_w(a, woff, next_w, free_w);
       TS_PIN;
       tile(0, a, 0, TM / 2);
       TS_PIN;
@@ -238,7 +261,8 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
         for (int b = 0; b < TM; ++b) asm volatile("" : "+v"(xf[1][b]));
 #pragma unroll
         for (int j = FREE; j < TN; ++j) asm volatile("" : "+v"(wf[j]));
-        block_wait<Ring::LEFT>();
+        if constexpr (X_LOADS) block_wait<Ring::LEFT>();
+        else block_wait_for<Ring, Ring::W - 2>(count - 2 - it);
         ws = ws + 1 == RW ? 0 : ws + 1;
         xs = xs + 1 == RX ? 0 : xs + 1;
         asm volatile("" : "+s"(ws), "+s"(xs));  // the compiler, for which no load writes what it reads, sees new addresses
@@ -250,16 +274,21 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
           else xf[0][j - FREE] = read_x(xs, 0, j - FREE);
         }
 #pragma unroll
-        for (int j = (a - FREE) * TM / (TN - FREE); j < (a - FREE + 1) * TM / (TN - FREE); ++j) load_x(j, from_x_at, next_x, free_x);
+        for (int j = (a - FREE) * TM / (TN - FREE); j < (a - FREE + 1) * TM / (TN - FREE); ++j)
+          if constexpr (X_LOADS) load_x(j, xoff, next_x, free_x);
       }
       TS_PIN;
       tile(1, a, 0, TM);
       TS_PIN;
       if (a >= FREE) wf[a] = read_w(ws, 0, a);
     }
-  }
+  };
 #undef TS_PIN
-  block_wait<0>();  // loads past the end
+  // No load is issued past the end: one that brings nothing still takes its turn in the unit's memory path.
+  int it = 0;
+  for (; it + RX < count; ++it) iteration(it, std::true_type{}, std::true_type{});
+  if (RX == RW && it + RW - 1 < count) iteration(it++, std::true_type{}, std::false_type{});
+  for (; it < count; ++it) iteration(it, std::false_type{}, std::false_type{});
   // The sums leave the loop where they were: without this the compiler rotated them through other registers in some of the
   // loops (a third of all instructions).
 #pragma unroll
