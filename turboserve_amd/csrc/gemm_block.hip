@@ -207,17 +207,26 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   };
 
   // Iteration i of the range: its weight rows lie in slot i % RW of their ring, its activation rows in slot i % RX of theirs.
+  // No load is issued past the end: one that brings nothing still takes its turn in the unit's memory path.  But a loop of their own
+  // for the last iterations costs the compiler its registers where the sums take more than 160: it moved them about in the main
+  // loop as well (2,048 rows, 7,168 x 5,120 with 256 x 256 115 -> 129 us, 27,648 x 5,120 gated with 256 x 192 467 -> 474).  There the
+  // loads go out in every iteration, those past the end past the buffers' ends too.
+  constexpr bool PEELED = TN * TM <= 40;
+  const int outside = (int)0x80000000;
   const int count = last - first;
+  auto step = [&](int i) __attribute__((always_inline)) { return first + (PEELED ? i : min(i, count - 1)); };
+  auto at = [&](int off, int i) __attribute__((always_inline)) { return PEELED || i < count ? off : outside; };
 #pragma unroll
   for (int s = 0; s < RX; ++s) {
-    if (s >= count) continue;
+    if (PEELED && s >= count) continue;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-      if (s < RW - 1) load_w(j, woff, first + s, s);
+      if (s < RW - 1) load_w(j, at(woff, s), step(s), s);
 #pragma unroll
-    for (int j = 0; j < TM; ++j) load_x(j, xoff, first + s, s);
+    for (int j = 0; j < TM; ++j) load_x(j, at(xoff, s), step(s), s);
   }
-  block_wait_first<Ring, RX - 1>(count - 1);
+  if (PEELED) block_wait_first<Ring, RX - 1>(count - 1);
+  else block_wait<Ring::left_first(RX)>();
 #pragma unroll
   for (int b = 0; b < TM; ++b) xf[0][b] = read_x(0, 0, b);
 #pragma unroll
@@ -235,12 +244,13 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   auto iteration = [&](int it, auto W_LOADS, auto X_LOADS) __attribute__((always_inline)) {
     // The offsets of the other rows are added up in each iteration: kept, they would take registers that the sums need.
     asm volatile("" : "+v"(woff), "+v"(xoff));
-    const int next_w = first + it + RW - 1, next_x = first + it + RX;
+    const int next_w = step(it + RW - 1), next_x = step(it + RX);
+    const int from_w_at = at(woff, it + RW - 1), from_x_at = at(xoff, it + RX);
     const int free_w = ws == 0 ? RW - 1 : ws - 1, free_x = xs;
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
       TS_PIN;
-      if constexpr (W_LOADS) load_w(a, woff, next_w, free_w);
+      if constexpr (W_LOADS) load_w(a, from_w_at, next_w, free_w);
       TS_PIN;
       tile(0, a, 0, TM / 2);
       TS_PIN;
@@ -275,7 +285,7 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
         }
 #pragma unroll
         for (int j = (a - FREE) * TM / (TN - FREE); j < (a - FREE + 1) * TM / (TN - FREE); ++j)
-          if constexpr (X_LOADS) load_x(j, xoff, next_x, free_x);
+          if constexpr (X_LOADS) load_x(j, from_x_at, next_x, free_x);
       }
       TS_PIN;
       tile(1, a, 0, TM);
@@ -284,11 +294,15 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
     }
   };
 #undef TS_PIN
-  // No load is issued past the end: one that brings nothing still takes its turn in the unit's memory path.
   int it = 0;
-  for (; it + RX < count; ++it) iteration(it, std::true_type{}, std::true_type{});
-  if (RX == RW && it + RW - 1 < count) iteration(it++, std::true_type{}, std::false_type{});
-  for (; it < count; ++it) iteration(it, std::false_type{}, std::false_type{});
+  if constexpr (PEELED) {
+    for (; it + RX < count; ++it) iteration(it, std::true_type{}, std::true_type{});
+    if (RX == RW && it + RW - 1 < count) iteration(it++, std::true_type{}, std::false_type{});
+    for (; it < count; ++it) iteration(it, std::false_type{}, std::false_type{});
+  } else {
+    for (; it < count; ++it) iteration(it, std::true_type{}, std::true_type{});
+    block_wait<0>();  // loads past the end
+  }
   // The sums leave the loop where they were: without this the compiler rotated them through other registers in some of the
   // loops (a third of all instructions).
 #pragma unroll
