@@ -340,6 +340,72 @@ __global__ void add_rmsnorm_vec4_kernel(T* __restrict__ y, float* __restrict__ r
   }
 }
 
+// The same bits where there is no second addend, no norm on the pending output and `splits` is at most BATCH: what a step of one token
+// launches 57 times and more.  What bounds such a launch beside one trip to memory is its own code, which the
+// step's other kernels have put out of the instruction cache: the general kernel jumps through 27 KB, each jump a trip; this
+// one is 1 to 4 KB and straight.  Recorded steps, us: one token of the 7B shape, 57 of
+// them, 2,864 -> 2,713; 64 ragged tokens 4,029 -> 3,924; one token of eight layers 2,048 wide 405 -> 373.
+template <typename T, typename P, int THREADS, int ITEMS, int BATCH>
+__global__ void __launch_bounds__(THREADS)
+add_rmsnorm_few_kernel(const P* pending, float* residual, const T* w, const int* rows, T* y, int splits, int hidden,
+                       size_t split_stride, float eps, float gain_offset, int one_rounding) {
+  __shared__ __attribute__((aligned(16))) float scratch[THREADS / TS_WAVE];
+  const int src = rows ? rows[blockIdx.x] : blockIdx.x;
+  const size_t in_base = (size_t)src * hidden;
+  const int quads = hidden / 4;
+  float s[ITEMS][4], g[ITEMS][4], part[ITEMS][BATCH][4];
+  float ss = 0.f;
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int i = 4 * min((int)threadIdx.x + it * THREADS, quads - 1);
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) Vec4Of<P>::load(pending + (size_t)min(j, splits - 1) * split_stride + in_base + i, part[it][j]);
+    Vec4Of<float>::load(residual + in_base + i, s[it]);
+    Vec4Of<T>::load(w + i, g[it]);
+  }
+  asm volatile("" ::: "memory");  // all of them on their way here
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int qd = threadIdx.x + it * THREADS;
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[it][e] = j < splits ? s[it][e] + part[it][j][e] : s[it][e];
+    }
+    if (qd < quads) {
+      if (!rows) Vec4Of<float>::store(residual + in_base + 4 * qd, s[it]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) add_square<T>(ss, s[it][e]);
+    }
+  }
+  const float rstd = rsqrtf(block_sum_of<THREADS>(ss, scratch) / (float)hidden + eps);
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int qd = threadIdx.x + it * THREADS;
+    if (qd < quads) {
+      float o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = with_gain<T>(s[it][e] * rstd, g[it][e], gain_offset, one_rounding);
+      Vec4Of<T>::store(y + (size_t)blockIdx.x * hidden + 4 * qd, o);
+    }
+  }
+}
+
+template <typename T, typename P, int THREADS, int ITEMS>
+static void launch_add_rmsnorm_few(void* y, float* residual, const void* pending, int splits, long split_stride, const void* w,
+                                   const int* rows, float eps, int out_rows, int hidden, float gain_offset, int one_rounding,
+                                   hipStream_t stream) {
+#define TS_NORM_FEW(BATCH)                                                                                                      \
+  hipLaunchKernelGGL((add_rmsnorm_few_kernel<T, P, THREADS, ITEMS, BATCH>), dim3(out_rows), dim3(THREADS), 0, stream, (const P*)pending, \
+                     residual, (const T*)w, rows, (T*)y, splits, hidden, (size_t)split_stride, eps, gain_offset, one_rounding)
+  if (splits == 1) TS_NORM_FEW(1);
+  else if (splits == 2) TS_NORM_FEW(2);
+  else if (splits <= 4) TS_NORM_FEW(4);
+  else if (splits <= 8) TS_NORM_FEW(8);
+  else TS_NORM_FEW(ITEMS * THREADS == 2048 ? 8 : 16);
+#undef TS_NORM_FEW
+}
+
 template <typename T, typename P>
 static void launch_add_rmsnorm(void* y, float* residual, const void* pending, int splits, long split_stride,
                                const void* w, const int* rows, float eps, int out_rows, int hidden,
@@ -359,6 +425,22 @@ static void launch_add_rmsnorm(void* y, float* residual, const void* pending, in
   if (out_rows <= 512 && threads <= (FLOAT32 ? 128 : 256)) threads *= 2;
   else if (out_rows <= 1024 && hidden > 1024 && threads < 256) threads = 256;
   if (out_rows <= 256 && threads < 1024) threads = 1024;
+  // (32-bit rows of fewer threads add their squares in the order of 1,024: TS_NORM_SUMS.  Steps of more than 512 rows fetch a
+  // kernel's code once for several rows a unit, and memory bounds them.)
+  const int items = (hidden / 4 + threads - 1) / threads;
+  if (hidden % 4 == 0 && pending && !also && !post_gain &&
+      ((threads == 1024 && items <= 2 && splits <= 16 / items) || (!FLOAT32 && threads == 512 && items == 2 && splits <= 16))) {
+#define TS_NORM_ITEMS(THREADS, ITEMS) \
+  launch_add_rmsnorm_few<T, P, THREADS, ITEMS>(y, residual, pending, splits, split_stride, w, rows, eps, out_rows, hidden, gain_offset, one_rounding, stream)
+    // (Wavefronts past the row's end would add zeros to its sum, and load.)
+    if (threads == 512) TS_NORM_ITEMS(512, 2);
+    else if (hidden <= 1024) TS_NORM_ITEMS(256, 1);
+    else if (hidden <= 2048) TS_NORM_ITEMS(512, 1);
+    else if (items == 1) TS_NORM_ITEMS(1024, 1);
+    else TS_NORM_ITEMS(1024, 2);
+#undef TS_NORM_ITEMS
+    return;
+  }
   const PostNorm<T> post = {(const T*)post_gain, post_eps, post_scale};
 #define TS_NORM(POST, SUMS)                                                                                                   \
   hipLaunchKernelGGL((add_rmsnorm_vec4_kernel<T, P, POST, SUMS>), dim3(out_rows), dim3(threads), 0, stream, (T*)y, residual,   \
