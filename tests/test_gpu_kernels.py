@@ -56,6 +56,29 @@ def test_rmsnorm_and_fused_residual(ops, dtype, tokens, hidden):
     torch.testing.assert_close(got, plain.rms_norm(total, w.float(), eps)[[tokens - 1, 0]], **tol(dtype))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,hidden", [(1, 4), (63, 1024), (3, 1028), (256, 2048), (2, 2052), (1, 4096), (5, 4100), (257, 2052), (512, 4096), (2, 8192)])
+def test_short_norms_have_the_bits_of_the_general_ones(ops, dtype, rows, hidden):
+    """A step's own norm kernels take up to 16 (8) partial sums at the edges of their threads; as many again that are zero, more than they
+    take, go to the general kernels, which add them up in the same order."""
+    g = torch.Generator().manual_seed(rows + hidden)
+    residual = torch.randn(rows, hidden, generator=g).to(DEV)
+    w, b = ((1 + 0.1 * torch.randn(2, hidden, generator=g)).to(dtype).to(DEV))
+    picked = torch.tensor([rows - 1, 0], dtype=torch.int32, device=DEV)
+    layer_norms = [{"norm": (w, b, 1e-5)}, {"norm": (w, None, 1e-5)}, {"pending_norm": (w, b, 1e-5, 0.5)}]
+    for splits in (1, 2, 3, 5, 8, 9, 16):
+        some = torch.randn(splits, rows, hidden, generator=g).to(DEV)
+        more = torch.cat([some, torch.zeros(17 - splits, rows, hidden, device=DEV)])
+        calls = [lambda into, parts, at: ops.add_rmsnorm(into, parts, w, 1e-6, at)]
+        if rows < 64 and splits <= 8 and hidden <= 4096:
+            calls += [lambda into, parts, at, rule=rule: ops.add_layer_norm(into, parts, dtype, at, **rule) for rule in layer_norms]
+        for call in calls:
+            for at in (None, picked):
+                into, want_into = residual.clone(), residual.clone()
+                got, want = call(into, some, at), call(want_into, more, at)
+                assert torch.equal(got, want) and torch.equal(into, want_into)
+
+
 @pytest.mark.parametrize("rows,hidden,splits", [(256, 2052, 3), (257, 2052, 3), (512, 4100, 1), (513, 2048, 1), (513, 2052, 2), (700, 5120, 1),
                                                 (514, 8196, 9), (300, 16384, 1), (600, 16, 17), (513, 16388, 2)])
 def test_add_rmsnorm_at_the_edges_of_its_blocks(ops, rows, hidden, splits):

@@ -111,6 +111,67 @@ add_layer_norm_kernel(T* __restrict__ y, float* __restrict__ residual, const P* 
   }
 }
 
+// The same bits for a step of few rows with one of the two norms (LAST: the sum's, else the pending output's) and at most BATCH
+// partial sums, four elements a thread: everything a row needs is asked for at once and the code is short and straight.  (In the general
+// kernel the other partial sums, then the gain wait for what came before them, and the code, which a recorded step's other kernels have put out
+// of the instruction cache, is fetched a jump at a time.)
+template <typename T, typename P, int THREADS, int BATCH, bool LAST>
+__global__ void __launch_bounds__(THREADS)
+add_layer_norm_few_kernel(const P* pending, float* residual, const T* w, const T* b, const int* rows, int splits, int hidden,
+                          size_t split_stride, T* y, float eps, float scale) {
+  __shared__ __attribute__((aligned(16))) float scratch[2][THREADS / TS_WAVE];
+  const int src = rows ? rows[blockIdx.x] : blockIdx.x;
+  const size_t in_base = (size_t)src * hidden;
+  const bool in = 4 * (int)threadIdx.x < hidden;
+  const int i = min(4 * (int)threadIdx.x, hidden - 4);
+  float part[BATCH][4], held[4], gain[4], shift[4], s[4];
+#pragma unroll
+  for (int j = 0; j < BATCH; ++j) load_vec<P, 4>(pending + (size_t)min(j, splits - 1) * split_stride + in_base + i, part[j]);
+  load_vec<float, 4>(residual + in_base + i, held);
+  load_vec<T, 4>(w + i, gain);
+  load_vec<T, 4>((b ? b : w) + i, shift);
+  asm volatile("" ::: "memory");  // all of them on their way here
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    s[e] = part[0][e];
+#pragma unroll
+    for (int j = 1; j < BATCH; ++j) s[e] = j < splits ? s[e] + part[j][e] : s[e];
+    if (LAST) s[e] = held[e] + s[e];
+    if (!in) s[e] = 0.f;
+  }
+  if (LAST && in && !rows) store_vec<float, 4>(residual + in_base + i, s);
+  float sum = 0.f, ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) sum += s[e];
+  const float mean = block_sum_of<THREADS>(sum, scratch[0]) / (float)hidden;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    s[e] -= mean;
+    if (in) ss = fmaf(s[e], s[e], ss);
+  }
+  const float rstd = rsqrtf(block_sum_of<THREADS>(ss, scratch[1]) / (float)hidden + eps);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    s[e] = scale * fmaf(s[e] * rstd, gain[e], b ? shift[e] : 0.f);
+    if (!LAST) s[e] = held[e] + s[e];
+  }
+  if (!in) return;
+  if (!LAST && !rows) store_vec<float, 4>(residual + in_base + i, s);
+  store_vec<T, 4>(y + (size_t)blockIdx.x * hidden + i, s);
+}
+
+template <typename T, typename P, int THREADS, bool LAST>
+static void launch_add_layer_norm_few(void* y, float* residual, const void* pending, int splits, long split_stride, const void* w,
+                                      const void* b, float eps, float scale, const int* rows, int out_rows, int hidden, hipStream_t stream) {
+#define LN_FEW(BATCH)                                                                                                               \
+  hipLaunchKernelGGL((add_layer_norm_few_kernel<T, P, THREADS, BATCH, LAST>), dim3(out_rows), dim3(THREADS), 0, stream, (const P*)pending, \
+                     residual, (const T*)w, (const T*)b, rows, splits, hidden, (size_t)split_stride, (T*)y, eps, scale)
+  if (splits == 1) LN_FEW(1);
+  else if (splits <= 4) LN_FEW(4);
+  else LN_FEW(8);
+#undef LN_FEW
+}
+
 template <typename T, typename P>
 static int launch_add_layer_norm(void* y, float* residual, const void* pending, int splits, long split_stride, const void* post_w,
                                  const void* post_b, float post_eps, float post_scale, const void* w, const void* b, float eps,
@@ -126,6 +187,19 @@ static int launch_add_layer_norm(void* y, float* residual, const void* pending, 
     // Steps of few rows spread a row over as many wavefronts as it has pieces for; prompts keep 256 threads a row.
     const int pieces = hidden / 4;
     const bool few = out_rows < 64;
+    if (few && pieces <= 1024 && pending && splits <= 8 && (!post_w || !w) && (post_w || w)) {
+      // (Wavefronts past the row's end add zeros to its sums.)
+#define LN_FEW(THREADS)                                                                                                              \
+  do {                                                                                                                               \
+    if (w) launch_add_layer_norm_few<T, P, THREADS, true>(y, residual, pending, splits, split_stride, w, b, eps, 1.f, rows, out_rows, hidden, stream); \
+    else launch_add_layer_norm_few<T, P, THREADS, false>(y, residual, pending, splits, split_stride, post_w, post_b, post_eps, post_scale, rows, out_rows, hidden, stream); \
+  } while (0)
+      if (pieces <= 256) LN_FEW(256);
+      else if (pieces <= 512) LN_FEW(512);
+      else LN_FEW(1024);
+#undef LN_FEW
+      return ts_launch_status();
+    }
     if (pieces <= 256) LN_GO(4, 1, (pieces + 63) / 64 * 64);
     else if (few && pieces <= 1024) LN_GO(4, 1, (pieces + 63) / 64 * 64);
     else if (pieces <= 512) LN_GO(4, 2, 256);
