@@ -368,9 +368,10 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
 
 template <int TN, int TM, int MODE, bool ONCE>
 __global__ void __launch_bounds__(256, 1)
-gemm_block_kernel(float* __restrict__ partial, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, long x_stride,
-                  const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int m, int n, int k,
-                  int iters_per_split, int splits, int n_tiles, int m_tiles, GluRule rule) {
+gemm_block_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int x_stride, int m, int n, int k, int iters_per_split,
+                  int splits, int n_tiles, int m_tiles, const uint16_t* __restrict__ bias, float* __restrict__ partial,
+                  uint16_t* __restrict__ out, GluRule rule) {
+  // (Fourteen words of arguments lie in registers at the start: those that the first loads want come first.)
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];  // the rings: weight rows, activation rows
   gemm_block<TN, TM, MODE, ONCE>((lds_u16*)lds, (const lds_u16*)lds, partial, out, x, x_stride, w, bias, m, n, k, iters_per_split,
                                  splits, n_tiles, m_tiles, rule);
@@ -392,8 +393,8 @@ int launch_block_kernel(float* partial, uint16_t* out, const uint16_t* x, long x
   const long units = (long)n_tiles * splits;
   const long ids = (units * m_tiles + BLOCK_DIES - 1) / BLOCK_DIES * BLOCK_DIES;
   if (ids > 0x7fffffffL) return TS_ERR_SHAPE;
-  hipLaunchKernelGGL((gemm_block_kernel<TN, TM, MODE, ONCE>), dim3((unsigned)ids), dim3(256), lds_bytes, stream, partial, out, x,
-                     x_stride, w, bias, m, n, k, iters_per_split, splits, n_tiles, m_tiles, rule);
+  hipLaunchKernelGGL((gemm_block_kernel<TN, TM, MODE, ONCE>), dim3((unsigned)ids), dim3(256), lds_bytes, stream, x, w,
+                     (int)x_stride, m, n, k, iters_per_split, splits, n_tiles, m_tiles, bias, partial, out, rule);
   return ts_launch_status();
 }
 

@@ -167,8 +167,9 @@ __device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds
 // partial: float [splits, m, n], or, GATED, out: bfloat16 [m, n / 2], the gated unit (common.hpp) of rows that alternate gate, up.
 template <int NT, int XT, bool GATED>
 __global__ void __launch_bounds__(64 * STREAM_WAVES)
-gemm_stream_kernel(float* __restrict__ partial, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, long x_stride,
-                   const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int m, int n, int k, int per_wave, GluRule rule) {
+gemm_stream_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int x_stride, int m,
+                   int n, int k, int per_wave, float* __restrict__ partial, uint16_t* __restrict__ out, GluRule rule) {
+  // (Fourteen words of arguments lie in registers at the start: those that the first loads want come first.)
   extern __shared__ __attribute__((aligned(16))) uint16_t ring[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n0 = blockIdx.x * 16 * NT, split = blockIdx.y;
@@ -178,9 +179,9 @@ gemm_stream_kernel(float* __restrict__ partial, uint16_t* __restrict__ out, cons
   f32x4 acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // The bias is asked for with the first slices, not behind the last.
+  // The bias is asked for with the first slices, not behind the last (a register each: packed in pairs they were waited for at once).
   const int col = n0 + 16 * min(wave, NT - 1) + 4 * (lane >> 4);
-  uint16_t shift[4] = {0, 0, 0, 0};
+  uint32_t shift[4] = {0, 0, 0, 0};
   if (bias && split == 0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) shift[i] = bias[min(col + i, n - 1)];
@@ -199,7 +200,7 @@ gemm_stream_kernel(float* __restrict__ partial, uint16_t* __restrict__ out, cons
   if (row >= m || col >= n) return;
   if (bias && split == 0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sum[i] += to_float(bf16_t{shift[i]});
+    for (int i = 0; i < 4; ++i) sum[i] += __uint_as_float(shift[i] << 16);
   }
   if (GATED) {  // n is even: the first pair lies inside
     uint16_t* at = out + (size_t)row * (n / 2) + col / 2;
@@ -228,8 +229,8 @@ int launch_stream(float* partial, void* out, const void* x, long x_stride, const
     raised = true;
   }
   hipLaunchKernelGGL((gemm_stream_kernel<NT, XT, GATED>), dim3((n + 16 * NT - 1) / (16 * NT), splits), dim3(64 * STREAM_WAVES),
-                     BYTES, stream, partial, (uint16_t*)out, (const uint16_t*)x, x_stride, (const uint16_t*)w,
-                     (const uint16_t*)bias, m, n, k, per_wave, rule);
+                     BYTES, stream, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (int)x_stride, m, n, k, per_wave,
+                     partial, (uint16_t*)out, rule);
   return ts_launch_status();
 }
 
