@@ -686,11 +686,11 @@ __device__ __forceinline__ void decode_staged(ColumnState& st, lds_u16* __restri
 
 template <bool PROJECTED>
 __global__ void __launch_bounds__(DECODE_THREADS) __attribute__((amdgpu_waves_per_eu(TS_WAVES_PER_SIMD, TS_WAVES_PER_SIMD)))
-decode_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const int* __restrict__ context_lens,
-              const int* __restrict__ query_start_loc, const int* __restrict__ block_table, int table_width, int seq_begin,
-              int kv_heads, int gsize, int splits, long q_stride, uint16_t* __restrict__ k_pages, uint16_t* __restrict__ v_pages,
-              int block_shift, int window, ScoreRule scale_log2, float* __restrict__ partial_acc, float* __restrict__ partial_ml,
-              Projected token_sums) {
+decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ query_start_loc, const int* __restrict__ block_table,
+              int table_width, int seq_begin, int kv_heads, int gsize, int splits, int block_shift, int window, long q_stride,
+              uint16_t* __restrict__ k_pages, uint16_t* __restrict__ v_pages, const uint16_t* __restrict__ q, Projected token_sums,
+              ScoreRule scale_log2, uint16_t* __restrict__ out, float* __restrict__ partial_acc, float* __restrict__ partial_ml) {
+  // (Fourteen words of arguments lie in registers at the start: what the first lookups want comes first.)
   extern __shared__ __attribute__((aligned(16))) float decode_lds[];
   lds_u16* const queries = (lds_u16*)decode_lds;         // [16][QUERY_ROW]
   lds_u16* const new_key = queries + 16 * QUERY_ROW;     // [D]
@@ -708,7 +708,11 @@ decode_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const 
   PageGeometry geo{k_pages, v_pages, block_table + (size_t)seq * table_width, table_width, kv_heads, kvh, block_shift,
                    (1 << block_shift) - 1};
   WindowPages first_pages = window_pages(geo, WINDOW_KEYS * (blockIdx.x + splits * wave));
-  const int ctx = context_lens[seq], token = query_start_loc[seq];
+  int ctx = context_lens[seq], token = query_start_loc[seq];
+  // (One wait for the three and the other arguments; the compiler asked for some behind a wait for the others.)
+  asm volatile("" ::"s"(token_sums.sums), "s"(token_sums.stride), "s"(token_sums.splits), "s"(token_sums.cos_table),
+               "s"(token_sums.sin_table), "s"(token_sums.slots), "s"(k_pages), "s"(v_pages), "s"(q), "s"(q_stride));
+  asm volatile("" : "+s"(ctx), "+s"(token), "+s"(first_pages.page[0]), "+s"(first_pages.page[1]), "+s"(first_pages.page[2]), "+s"(first_pages.page[3]));
   const int p = ctx - 1;
   const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
   const int lo_window = lo & ~(WINDOW_KEYS - 1);
@@ -717,7 +721,12 @@ decode_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const 
   if (window > 0) first_pages = window_pages(geo, w);
   const uint16_t* q_row = PROJECTED ? nullptr : q + (size_t)token * q_stride + (size_t)(first_head + lane16) * D;
   const float* sum_row = PROJECTED ? token_sums.sums + (size_t)token * (heads + 2 * kv_heads) * D : nullptr;
-  const int slot = PROJECTED && blockIdx.x == 0 && tile == 0 ? token_sums.slots[token] : -1;
+  int slot = -1;
+  if (PROJECTED && blockIdx.x == 0 && tile == 0) {
+    int at = token;  // a vector load: scalar ones come back in any order, and what waits for another would wait for this one
+    asm volatile("" : "+v"(at));
+    slot = token_sums.slots[at];
+  }
   ColumnState st;
   init_state(st);
   if constexpr (DECODE_STAGED) {
@@ -765,6 +774,7 @@ decode_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, const 
   }
 
   // The new key and value into their page (not before the walk, whose waits would wait for the stores as well).
+  if (PROJECTED) slot = __builtin_amdgcn_readfirstlane(slot);
   if (PROJECTED && slot >= 0) {
     const size_t page = (((size_t)(slot >> block_shift) * kv_heads + kvh) << block_shift) * D;
     const int offset = slot & geo.block_mask, at = threadIdx.x;
@@ -1991,9 +2001,9 @@ static int launch_decode(uint16_t* out, float* partial_acc, float* partial_ml, c
   const size_t lds = (16 * QUERY_ROW + 2 * D) * 2 + DECODE_WAVES * 32 * 4 + (joined > rings ? joined : rings);
   static const bool raised = hipFuncSetAttribute((const void*)decode_kernel<PROJECTED>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
   if (!raised) return TS_ERR_LAUNCH;
-  hipLaunchKernelGGL(decode_kernel<PROJECTED>, dim3(splits, kv_heads * head_tiles, requests), dim3(DECODE_THREADS), lds, stream, out, q,
-                     context_lens, query_start_loc, block_table, table_width, seq_begin, kv_heads, gsize, splits, q_stride, k_pages,
-                     v_pages, shift, window, rule, partial_acc, partial_ml, token_sums);
+  hipLaunchKernelGGL(decode_kernel<PROJECTED>, dim3(splits, kv_heads * head_tiles, requests), dim3(DECODE_THREADS), lds, stream,
+                     context_lens, query_start_loc, block_table, table_width, seq_begin, kv_heads, gsize, splits, shift, window, q_stride,
+                     k_pages, v_pages, q, token_sums, rule, out, partial_acc, partial_ml);
   if (splits == 1) return ts_launch_status();
   if (hipGetLastError() != hipSuccess) return TS_ERR_LAUNCH;
   hipLaunchKernelGGL(decode_reduce_kernel, dim3(requests, heads), dim3(REDUCE_THREADS), 0, stream, out, partial_acc, partial_ml,
