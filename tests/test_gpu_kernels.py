@@ -820,6 +820,30 @@ def test_rope_store(ops, dtype, heads, kv_heads, dim, page, theta, factor):
         ops.rope_store(dev, kp, vp, cos.to(DEV), sin.to(DEV), positions.to(DEV), None, heads, kv_heads, dim, page, 128)
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,page", [(4, 2, 64, 16), (7, 1, 128, 8), (3, 3, 48, 32)])
+@pytest.mark.parametrize("tokens,splits", [(129, 1), (130, 3), (136, 4), (300, 5), (135, 9)])
+def test_rope_store_of_a_prompts_partial_sums_equals_token_by_token(ops, heads, kv_heads, dim, page, tokens, splits):
+    """Groups of eight tokens (from 129 on) against the kernel of few tokens: the same bits in queries and pages, slots in runs and not."""
+    g = torch.Generator().manual_seed(tokens + dim)
+    sums = torch.randn(splits, tokens, (heads + 2 * kv_heads) * dim, generator=g)
+    cos, sin = (t.to(DEV) for t in rotary_pair(512, dim))
+    positions = torch.randint(0, 512, (tokens,), generator=g, dtype=torch.int32)
+    pages = -(-2 * tokens // page)
+    slots = torch.arange(8, 8 + tokens, dtype=torch.int32)
+    slots[40:80] = torch.randperm(tokens, generator=g)[:40].to(torch.int32) + tokens + 8
+    slots[90] = -1
+    cuts = [(0, tokens)], [(at, min(at + 100, tokens)) for at in range(0, tokens, 100)]
+    got = []
+    for parts in cuts:
+        kp = torch.zeros(pages + 2, kv_heads, page, dim, dtype=torch.bfloat16, device=DEV)
+        vp = torch.zeros(pages + 2, kv_heads, dim, page, dtype=torch.bfloat16, device=DEV)
+        rows = [ops.rope_store(sums[:, a:b].contiguous().to(DEV), kp, vp, cos, sin, positions[a:b].to(DEV), slots[a:b].to(DEV), heads, kv_heads, dim,
+                               page, 511, torch.bfloat16)[0] for a, b in parts]
+        got.append((torch.cat(rows).view(torch.int16), kp.view(torch.int16), vp.view(torch.int16)))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,page", [(7, 1, 128, 16), (3, 3, 48, 8), (4, 2, 32, 4), (2, 1, 96, 32)])
 def test_rope_store_of_many_tokens_equals_token_by_token(ops, heads, kv_heads, dim, page):
     """Prompt portions of 32 tokens or more go through a kernel that handles 8 tokens per block

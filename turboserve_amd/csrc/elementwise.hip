@@ -677,7 +677,37 @@ __global__ void rope_store_kernel(T* q_out, long q_stride, const P* proj, int sp
   }
 }
 
-// The same for many tokens at once (prompt portions): bfloat16 in and out, no partial sums, head
+// N neighbouring elements of a projection as numbers: its own, or `splits` partial sums added up in their order, four on their way at once.
+template <int N>
+__device__ __forceinline__ void rope_input(const bf16_t* p, int, size_t, float (&v)[N]) {
+  typedef uint16_t u16xN __attribute__((ext_vector_type(N)));
+  const u16xN raw = *reinterpret_cast<const u16xN*>(p);
+#pragma unroll
+  for (int e = 0; e < N; ++e) v[e] = to_float(bf16_t{raw[e]});
+}
+template <int N>
+__device__ __forceinline__ void rope_input(const float* p, int splits, size_t stride, float (&v)[N]) {
+  typedef float f32xP __attribute__((ext_vector_type(N < 4 ? N : 4)));
+  constexpr int EACH = N < 4 ? N : 4;
+#pragma unroll
+  for (int e = 0; e < N; ++e) v[e] = 0.f;
+  for (int first = 0; first < splits; first += 4) {
+    f32xP part[4][N / EACH];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int e = 0; e < N / EACH; ++e)
+        part[j][e] = *reinterpret_cast<const f32xP*>(p + (size_t)min(first + j, splits - 1) * stride + EACH * e);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) v[e] = first + j < splits ? v[e] + part[j][e / EACH][e % EACH] : v[e];
+    }
+  }
+}
+
+// The same for many tokens at once (prompt portions): a bfloat16 projection or 32-bit partial sums, bfloat16 out, head
 // size a multiple of 16.  One block per (group of 8 consecutive tokens, head).  q and k heads: a
 // thread rotates 8 pairs with 16-byte loads and stores.  v heads: a thread collects one head
 // dimension of the 8 tokens; when the group's slots are 8 consecutive ones starting at a multiple
@@ -685,9 +715,10 @@ __global__ void rope_store_kernel(T* q_out, long q_stride, const P* proj, int sp
 // that is one 16-byte store into the transposed value page, else one 2-byte store per token.
 constexpr int ROPE_GROUP = 8;
 
+template <typename P>
 __global__ void __launch_bounds__(64)
-rope_store_group_kernel(bf16_t* q_out, long q_stride, const bf16_t* proj, bf16_t* __restrict__ k_pages,
-                        bf16_t* __restrict__ v_pages, const float* __restrict__ cos_table,
+rope_store_group_kernel(bf16_t* q_out, long q_stride, const P* proj, int splits, size_t split_stride,
+                        bf16_t* __restrict__ k_pages, bf16_t* __restrict__ v_pages, const float* __restrict__ cos_table,
                         const float* __restrict__ sin_table, const int* __restrict__ positions,
                         const int* __restrict__ slots, int tokens, int heads, int kv_heads, int dim,
                         int block_size, int rotate) {
@@ -706,10 +737,16 @@ rope_store_group_kernel(bf16_t* q_out, long q_stride, const bf16_t* proj, bf16_t
       const int j = item / vectors, i = (item % vectors) * 8;
       if (j >= count) continue;
       const int t = t0 + j;
-      const bf16_t* row = proj + (size_t)t * width + (size_t)h * dim;
-      const u16x8 a = *reinterpret_cast<const u16x8*>(row + i);
-      const u16x8 b = *reinterpret_cast<const u16x8*>(row + i + half);
-      u16x8 o1 = a, o2 = b;
+      const P* row = proj + (size_t)t * width + (size_t)h * dim;
+      float a[8], b[8];
+      rope_input<8>(row + i, splits, split_stride, a);
+      rope_input<8>(row + i + half, splits, split_stride, b);
+      u16x8 o1, o2;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        o1[e] = from_float<bf16_t>(a[e]).bits;
+        o2[e] = from_float<bf16_t>(b[e]).bits;
+      }
       if (rotate) {
         const float* c = cos_table + (size_t)positions[t] * half + i;
         const float* s = sin_table + (size_t)positions[t] * half + i;
@@ -719,7 +756,7 @@ rope_store_group_kernel(bf16_t* q_out, long q_stride, const bf16_t* proj, bf16_t
         for (int e = 0; e < 8; ++e) {
           const float cv = e < 4 ? c0[e & 3] : c1[e & 3], sv = e < 4 ? s0[e & 3] : s1[e & 3];
           float r1, r2;
-          rotate_pair(to_float(bf16_t{a[e]}), to_float(bf16_t{b[e]}), cv, sv, r1, r2);
+          rotate_pair(a[e], b[e], cv, sv, r1, r2);
           o1[e] = from_float<bf16_t>(r1).bits;
           o2[e] = from_float<bf16_t>(r2).bits;
         }
@@ -746,11 +783,15 @@ rope_store_group_kernel(bf16_t* q_out, long q_stride, const bf16_t* proj, bf16_t
   bool run = count == ROPE_GROUP && slot[0] >= 0 && (slot[0] & 7) == 0 && (block_size & 7) == 0;
 #pragma unroll
   for (int j = 1; j < ROPE_GROUP; ++j) run = run && slot[j] == slot[0] + j;
-  const bf16_t* column = proj + (size_t)t0 * width + (size_t)h * dim;
+  const P* column = proj + (size_t)t0 * width + (size_t)h * dim;
   for (int d = threadIdx.x; d < dim; d += blockDim.x) {
     u16x8 v;
 #pragma unroll
-    for (int j = 0; j < ROPE_GROUP; ++j) v[j] = j < count ? column[(size_t)j * width + d].bits : (uint16_t)0;
+    for (int j = 0; j < ROPE_GROUP; ++j) {
+      float one[1];
+      rope_input<1>(column + (size_t)min(j, count - 1) * width + d, splits, split_stride, one);
+      v[j] = j < count ? from_float<bf16_t>(one[0]).bits : (uint16_t)0;
+    }
     if (run) {
       bf16_t* dst = v_pages + (((size_t)(slot[0] / block_size) * kv_heads + kvh) * dim + d) * block_size + slot[0] % block_size;
       *reinterpret_cast<u16x8*>(dst) = v;
@@ -778,9 +819,16 @@ extern "C" int ts_rope_store(void* q_out, long q_stride, const void* proj, int i
   dim3 grid(tokens, heads + 2 * kv_heads), block(64);
   const bool aligned = ((uintptr_t)q_out | (uintptr_t)proj | (uintptr_t)k_pages | (uintptr_t)v_pages |
                         (uintptr_t)cos_table | (uintptr_t)sin_table) % 16 == 0 && q_stride % 8 == 0;
-  if (dtype == TS_BF16 && !in_f32 && splits == 1 && dim % 16 == 0 && tokens >= 4 * ROPE_GROUP && aligned) {
+  const bool sums_in_groups = in_f32 && split_stride % 4 == 0 && tokens > 128;
+  if (dtype == TS_BF16 && ((!in_f32 && splits == 1) || sums_in_groups) && dim % 16 == 0 && tokens >= 4 * ROPE_GROUP && aligned) {
     dim3 groups((tokens + ROPE_GROUP - 1) / ROPE_GROUP, heads + 2 * kv_heads);
-    hipLaunchKernelGGL(rope_store_group_kernel, groups, block, 0, stream, (bf16_t*)q_out, q_stride, (const bf16_t*)proj, (bf16_t*)k_pages, (bf16_t*)v_pages, cos_table, sin_table, positions, slots, tokens, heads, kv_heads, dim, block_size, rotate);
+#define TS_ROPE_GROUP(P)                                                                                                       \
+  hipLaunchKernelGGL(rope_store_group_kernel<P>, groups, block, 0, stream, (bf16_t*)q_out, q_stride, (const P*)proj, splits,   \
+                     (size_t)split_stride, (bf16_t*)k_pages, (bf16_t*)v_pages, cos_table, sin_table, positions, slots, tokens, \
+                     heads, kv_heads, dim, block_size, rotate)
+    if (in_f32) TS_ROPE_GROUP(float);
+    else TS_ROPE_GROUP(bf16_t);
+#undef TS_ROPE_GROUP
     return ts_launch_status();
   }
   if (dtype == TS_F32)

@@ -2203,27 +2203,32 @@ class Ops:
         result the unit's time, and partial sums of several ranges their way to the norm, 3.6
         bytes per nanosecond.  Against every tile with 1 to 16 ranges, timed for the matrices of six shapes (K 2,048 to 18,944) at 144 to
         2,048 rows, the plan's grid takes 1% more than the fastest on average.
-        ``kind``: "sums" (partial sums may stay), "one" (one bfloat16 result), "gated"."""
+        ``kind``: "sums" (partial sums may stay), "store" (up to four of them, what the store of heads asks for at once), "one"
+        (one bfloat16 result), "gated"."""
         key = (m, n, k, kind)
         known = self._block_plans.get(key)
         if known is not None:
             return known
         iters = k // 64
         best = None
-        for (tn, tm), pace in self._BLOCK_TILES.items():
-            tiles = -(-n // (32 * tn)) * -(-m // (32 * tm))
-            for want in range(1, (min(iters, 16) if kind == "sums" else 1) + 1):
+        for tn, tm in self._BLOCK_TILES:
+            for want in range(1, min(iters, {"sums": 16, "store": 4}.get(kind, 1)) + 1):
                 per_split = -(-iters // want)
                 splits = -(-iters // per_split)
                 if splits != want:
                     continue
-                cost = -(-tiles * splits // self.compute_units) * ((per_split + 6) * pace + (0.18 * tn * tm if kind == "gated" else 0.0))
-                if splits > 1:
-                    cost += splits * m * n * 4 / 3.6e6
+                cost = self._block_cost(m, n, k, (per_split, splits, tn, tm), kind == "gated")
                 if best is None or cost < best[0]:
                     best = (cost, per_split, splits, tn, tm)
         self._block_plans[key] = best[1:]
         return best[1:]
+
+    def _block_cost(self, m: int, n: int, k: int, plan: tuple[int, int, int, int], gated: bool = False) -> float:
+        """What :meth:`_block_plan` compares, in microseconds."""
+        per_split, splits, tn, tm = plan
+        workgroups = -(-n // (32 * tn)) * -(-m // (32 * tm)) * splits
+        cost = -(-workgroups // self.compute_units) * ((per_split + 6) * self._BLOCK_TILES[tn, tm] + (0.18 * tn * tm if gated else 0.0))
+        return cost + (splits * m * n * 4 / 3.6e6 if splits > 1 else 0.0)
 
     #: What an iteration of 64 of K takes with one tile of activation rows, one workgroup a compute unit, by tile of weight
     #: rows, in microseconds (at 64 rows; 16,384 to 152,064 weight rows).
@@ -2815,8 +2820,25 @@ class Ops:
             return self.swiglu(self._library_product(x, weight, bias, None), x.dtype, paired=True, rule=rule)
         return self.swiglu(self.linear(x, weight, bias), x.dtype, paired=True, rule=rule)
 
+    def _sums_plan(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> tuple[int, int, int, int] | None:
+        """The block product's grid for a prompt of few rows whose consumer adds up partial sums as well as it takes one result
+        (the store of rotated heads), or None where one result is as soon there.  A narrow product as one range of K leaves most
+        units idle: several ranges where the model puts them, their way to the consumer included, at seven tenths of one
+        range's time (us with the store, one result by the library or here / sums: 4,608 x 3,584 at 200 / 256 / 299 / 350 rows 36 / 39 /
+        33.9 / 33.4 against 26 / 28 / 29.9 / 31.5, at 400 31.6 against 33.0; 7,168 x 5,120 at 200 / 299 42 / 47 against 38 / 45, at
+        400 46 against 50)."""
+        m, (n, k) = x.shape[0], weight.shape
+        if not self.skinny_max_rows < m <= self.wide_default_rows or not self.block_supported(x, weight) or (bias is not None and bias.data_ptr() % 8):
+            return None
+        key = ("sums for the store", m, n, k)
+        if key not in self._block_plans:
+            sums, one = self._block_plan(m, n, k, "store"), self._block_plan(m, n, k, "one")
+            soon = sums[1] > 1 and 10 * self._block_cost(m, n, k, sums) <= 7 * self._block_cost(m, n, k, one)
+            self._block_plans[key] = sums if soon else None
+        return self._block_plans[key]
+
     def linear(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *,
-               for_residual: bool = False) -> torch.Tensor:
+               for_residual: bool = False, for_store: bool = False) -> torch.Tensor:
         """The projection of the serving path.  32-bit runs use :meth:`gemm_plain` (no reduced
         matrix mode).  bfloat16 runs with decode-sized batches (up to ``skinny_max_rows`` rows) use
         :meth:`gemm_skinny` and return ``[S, M, N]`` 32-bit partial sums for the consumer to add
@@ -2828,7 +2850,8 @@ class Ops:
         timed (``_wide_runs``; untimed: ``_own_product``).  ``for_residual``: the result is what a
         norm adds to the 32-bit residual stream, so it may stay 32-bit partial sums ``[S, M, N]``, and
         with ``library_residual_float32`` it always does (as ``[1, M, N]`` where it is one range):
-        the stream then gets the same unrounded addend from a prompt's step as from a decode step's."""
+        the stream then gets the same unrounded addend from a prompt's step as from a decode step's.  ``for_store``: the result goes to
+        :meth:`rope_store`, which takes either; a prompt of few rows may leave partial sums (``_sums_plan``)."""
         if x.dtype == torch.float32:
             return self.gemm_plain(x, weight, bias)
         if x.shape[0] <= self.skinny_max_rows:
@@ -2836,6 +2859,9 @@ class Ops:
                 return self.gemm_skinny(x, weight, bias)
             return self.gemm_plain(x, weight, bias)  # a K that 16-byte loads do not divide
         _gpu(x, weight, bias)
+        plan = self._sums_plan(x, weight, bias) if for_store else None
+        if plan is not None:
+            return self._block_product(x, weight, bias, plan=plan, gated=False, sums=True, rule=(1.0, 0.0, 0.0))
         if self.skinny_supported_any_rows(x, weight):
             m, (n, k) = x.shape[0], weight.shape
             # What goes into the residual stream may stay partial sums (the norm adds them up);

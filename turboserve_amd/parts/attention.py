@@ -284,6 +284,12 @@ class GroupedQueryAttention(Mixer):
         do the attention kernels that take any rule (the ones that only take plain causal or windowed attention do not)."""
         return self.gate_name is not None or not self._plain_rule()
 
+    def _plain_store(self) -> bool:
+        """Whether the projection goes to the plain rotation and store (:meth:`Ops.rope_store`) as it is."""
+        return (self.conv_taps is None and self.gate_name is None and not self.values_are_keys and self.query_temperature is None
+                and self.value_dim == self.head_dim and self.head_norm_eps is None and self.span_norm_eps is None
+                and self.value_mix is None and self.own_keys and self.position.plain_store(self.head_dim))
+
     def _plain_rule(self) -> bool:
         """Whether the head-size-specialised attention kernels take this layer's rule."""
         return (not self.position.biases_scores and self.value_dim == self.head_dim and self.chunk is None and self.sinks == 0.0
@@ -295,7 +301,7 @@ class GroupedQueryAttention(Mixer):
         = (buffer, col0)``): a caller that adds this mixer's output to another's can then run both output matrices as
         one product."""
         ops = self.runtime.ops
-        qkv = proj = ops.linear(x, self.qkv_weight, self.qkv_bias_tensor)
+        qkv = proj = ops.linear(x, self.qkv_weight, self.qkv_bias_tensor, for_store=self._plain_store())
         more, shape = {}, {}
         if self.conv_taps is not None:
             cache, held = cache

@@ -290,6 +290,11 @@ class PositionEncoding(Part):
         store itself.  ``None``: only :meth:`encode_and_store` encodes."""
         return None
 
+    def plain_store(self, head_dim: int) -> bool:
+        """Whether :meth:`encode_and_store` of plain heads (no norms, no shapes) is one call of ``Ops.rope_store``, which takes a prompt's
+        projection as partial sums too."""
+        return False
+
     def score_slopes(self, num_heads: int) -> torch.Tensor | None:
         """An encoding may (also, or instead) act inside the scores: ``[num_heads]`` 32-bit
         slopes ``m`` on the device, for which the score of key ``j`` for the query at position

@@ -180,9 +180,12 @@ class RotaryEncoding(PositionEncoding):
         self.sin = sin.to(self.runtime.device)
         self.capacity = target
 
+    def plain_store(self, head_dim):
+        return not self.neighbours and self.head_dim == head_dim and type(self).encode_and_store is RotaryEncoding.encode_and_store
+
     def rotation(self, head_dim, ctx):
         # (Not for an encoding that inherits the tables and encodes in a way of its own.)
-        if self.neighbours or self.head_dim != head_dim or type(self).encode_and_store is not RotaryEncoding.encode_and_store:
+        if not self.plain_store(head_dim):
             return None
         self.ensure_capacity(ctx.max_context_len)
         return self.cos, self.sin
