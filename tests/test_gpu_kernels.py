@@ -622,6 +622,23 @@ def test_gemm_block_gates_of_every_size(ops, m, tn, tm):
     assert bool(lowest.isnan().all() and none.isnan().all())  # as -inf / (1 + expf(inf)) is
 
 
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("m,n,first,tiles,rest", [(300, 1040, 512, (8, 8), (5, 8)), (33, 784, 768, (8, 6), (4, 4)), (129, 528, 16, (8, 5), (5, 10)),
+                                                  (257, 2064, 1792, (8, 8), (4, 5))])
+def test_a_product_in_two_launches_is_the_product_in_one(ops, m, n, first, tiles, rest, gated):
+    """Whole rounds of one tile and another tile for the rest of the weight rows write, bit for bit, what one tile writes, and
+    nothing beside it; the plan of a long prompt's product has such a rest and covers it."""
+    g = torch.Generator().manual_seed(m + n)
+    x = torch.randn(m, 192, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(n, 192, generator=g) / 14).bfloat16().to(DEV)
+    bias = torch.randn(n, generator=g).bfloat16().to(DEV)
+    for b in (None, bias):
+        want = ops.gemm_block(x, w, b, plan=(3, 1, 4, 4), gated=gated)
+        assert torch.equal(ops.gemm_block(x, w, b, plan=(3, 1, *tiles, first, *rest), gated=gated), want)
+    plan = ops._block_rounds(2048, 27648, 5120, True, ops._block_plan(2048, 27648, 5120, "gated"))
+    assert len(plan) == 7 and plan[4] % 32 == 0 and 0 < plan[4] < 27648
+
+
 @pytest.mark.parametrize("m,n,k,offset", [(17, 4608, 3584, 0), (32, 2048, 2048, 0), (33, 2064, 576, 0), (64, 512, 64, 0), (65, 528, 640, 0), (128, 272, 1088, 4),
                                           (100, 1000, 264, 0), (129, 16, 64, 0), (300, 2064, 1088, 0), (200, 500, 264, 0), (200, 512, 264, 0), (200, 520, 256, 0),
                                           (200, 512, 256, 4), (150, 256, 192, 0)])

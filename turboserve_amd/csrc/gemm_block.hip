@@ -132,7 +132,7 @@ template <int TN, int TM, int MODE, bool ONCE>
 __device__ __forceinline__ void
 gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __restrict__ partial, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, long x_stride,
                   const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int m, int n, int k,
-                  int iters_per_split, int splits, int n_tiles, int m_tiles, GluRule rule) {
+                  int iters_per_split, int splits, int n_tiles, int m_tiles, int whole_n, GluRule rule) {
   constexpr int NT = 32 * TN, XR = 32 * TM, ROW = BLOCK_DEPTH;
   typedef BlockRing<TN, TM> Ring;
   constexpr int RW = Ring::W, RX = Ring::X;
@@ -317,9 +317,9 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   // columns of every tile, and exchange them until one holds eight of one of two tiles (gated: all of one of four).
   // Rows beyond M lie past the buffer's end, tiles beyond N are sent there.
   constexpr int BYTES = MODE == 1 ? 4 : 2, PER = MODE >= 2 ? 2 : 1;  // of an output element; weight rows of one
-  const int row_bytes = n / PER * BYTES;
-  char* base = MODE == 1 ? (char*)(partial + ((size_t)split * m + m_base) * n) : (char*)out + (size_t)m_base * row_bytes;
-  const __amdgpu_buffer_rsrc_t ybuf = block_buffer(base, (size_t)min(m - m_base, XR) * row_bytes);
+  const int row_bytes = whole_n / PER * BYTES;
+  char* base = MODE == 1 ? (char*)(partial + ((size_t)split * m + m_base) * whole_n) : (char*)out + (size_t)m_base * row_bytes;
+  const __amdgpu_buffer_rsrc_t ybuf = block_buffer(base, (size_t)(min(m - m_base, XR) - 1) * row_bytes + n / PER * BYTES);
   const int tiles = (n - n_base) / 16 - wave_n * TN;  // of this wavefront's, those that exist
   const int OUTSIDE = (int)0x80000000;
   const int tile_bytes = 16 / PER * BYTES;
@@ -370,16 +370,16 @@ template <int TN, int TM, int MODE, bool ONCE>
 __global__ void __launch_bounds__(256, 1)
 gemm_block_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int x_stride, int m, int n, int k, int iters_per_split,
                   int splits, int n_tiles, int m_tiles, const uint16_t* __restrict__ bias, float* __restrict__ partial,
-                  uint16_t* __restrict__ out, GluRule rule) {
+                  uint16_t* __restrict__ out, int whole_n, GluRule rule) {
   // (Fourteen words of arguments lie in registers at the start: those that the first loads want come first.)
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];  // the rings: weight rows, activation rows
   gemm_block<TN, TM, MODE, ONCE>((lds_u16*)lds, (const lds_u16*)lds, partial, out, x, x_stride, w, bias, m, n, k, iters_per_split,
-                                 splits, n_tiles, m_tiles, rule);
+                                 splits, n_tiles, m_tiles, whole_n, rule);
 }
 
 template <int TN, int TM, int MODE, bool ONCE>
 int launch_block_kernel(float* partial, uint16_t* out, const uint16_t* x, long x_stride, const uint16_t* w, const uint16_t* bias,
-                        int m, int n, int k, int iters_per_split, int splits, GluRule rule, hipStream_t stream) {
+                        int m, int n, int k, int iters_per_split, int splits, int whole_n, GluRule rule, hipStream_t stream) {
   constexpr int NT = 32 * TN, XR = 32 * TM;
   constexpr size_t lds_bytes = BlockRing<TN, TM>::BYTES;
   static bool raised = false;  // per process; the attribute belongs to the kernel
@@ -394,7 +394,7 @@ int launch_block_kernel(float* partial, uint16_t* out, const uint16_t* x, long x
   const long ids = (units * m_tiles + BLOCK_DIES - 1) / BLOCK_DIES * BLOCK_DIES;
   if (ids > 0x7fffffffL) return TS_ERR_SHAPE;
   hipLaunchKernelGGL((gemm_block_kernel<TN, TM, MODE, ONCE>), dim3((unsigned)ids), dim3(256), lds_bytes, stream, x, w,
-                     (int)x_stride, m, n, k, iters_per_split, splits, n_tiles, m_tiles, bias, partial, out, rule);
+                     (int)x_stride, m, n, k, iters_per_split, splits, n_tiles, m_tiles, bias, partial, out, whole_n, rule);
   return ts_launch_status();
 }
 
@@ -404,16 +404,19 @@ int launch_block_kernel(float* partial, uint16_t* out, const uint16_t* x, long x
 // 0: out = bfloat16 [m, n] (splits must be 1); mode 1: partial = float [splits, m, n]; mode 2: out = bfloat16 [m, n / 2] =
 // the gated unit (common.hpp) of a w whose rows alternate gate, up (splits 1).  iters_per_split iterations of 64 of k go to
 // each of `splits` = ceil(k / 64 / iters_per_split) ranges.  tn, tm: 32 tn weight rows by 32 tm activation rows a
-// workgroup.
+// workgroup.  w, bias and out may be a run of weight rows of a larger product: whole_n is its n, the length of out's rows
+// (out points at the run's first column).
 extern "C" int ts_gemm_block(float* partial, void* out, const void* x, long x_stride, const void* w, const void* bias,
-                             int m, int n, int k, int iters_per_split, int splits, int tn, int tm, int mode,
+                             int m, int n, int k, int iters_per_split, int splits, int tn, int tm, int mode, int whole_n,
                              float steepness, float limit, float up_shift, float cubic, hipStream_t stream) {
   if (m == 0 || n == 0) return TS_OK;
   if (!x || !w || m < 0 || n < 0 || k < 1 || mode < 0 || mode > 2) return TS_ERR_ARG;
   if ((mode == 1) != (partial != nullptr) || (mode != 1) != (out != nullptr)) return TS_ERR_ARG;
   if (k % BLOCK_DEPTH != 0 || n % 16 != 0 || x_stride < k || x_stride % 8 != 0 || (uintptr_t)x % 16 != 0 || (uintptr_t)w % 16 != 0)
     return TS_ERR_SHAPE;
+  if (whole_n < n || whole_n % 16 != 0) return TS_ERR_SHAPE;
   // A block's rows are addressed by 31-bit byte offsets from its first one.
+  if (whole_n >= (1 << 20)) return TS_ERR_SHAPE;
   if (x_stride >= (1L << 21) || k >= (1 << 21) || n >= (1 << 20)) return TS_ERR_SHAPE;
   const int total = k / BLOCK_DEPTH;
   if (iters_per_split < 1 || splits != (total + iters_per_split - 1) / iters_per_split) return TS_ERR_SHAPE;
@@ -422,7 +425,7 @@ extern "C" int ts_gemm_block(float* partial, void* out, const void* x, long x_st
   const bool plain = limit <= 0.f && cubic == 0.f;
 #define TS_BLOCK_MODE(TN, TM, MODE, ONCE)                                                                                    \
   return launch_block_kernel<TN, TM, MODE, ONCE>(partial, (uint16_t*)out, (const uint16_t*)x, x_stride, (const uint16_t*)w,  \
-                                                 (const uint16_t*)bias, m, n, k, iters_per_split, splits, rule, stream)
+                                                 (const uint16_t*)bias, m, n, k, iters_per_split, splits, whole_n, rule, stream)
 #define TS_BLOCK(TN, TM, ONCE)                       \
   if (tn == TN && tm == TM && once == ONCE) {        \
     if (mode == 0) TS_BLOCK_MODE(TN, TM, 0, ONCE);   \

@@ -147,7 +147,7 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "ts_gemm_wide": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                          c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_block": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
-                          c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
+                          c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_stream": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                            c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_skinny_resident": [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
@@ -2223,6 +2223,27 @@ class Ops:
         self._block_plans[key] = best[1:]
         return best[1:]
 
+    def _block_rounds(self, m: int, n: int, k: int, gated: bool, plan: tuple[int, int, int, int]) -> tuple[int, ...]:
+        """``plan`` (one range of K), or, where its last round of workgroups is better spent, whole rounds of one tile over the first weight
+        rows and another tile over the rest, a launch each: ``(iterations, 1, tile of weight rows, of activation rows, first rows,
+        the rest's tiles)``.  By the model of :meth:`_block_plan` and 3 us for the second launch, and only where that saves
+        2% (us at 2,048 rows, one tile / whole rounds and the rest: 27,648 x 5,120 gated 459 to 480 / 437, 37,888 x 3,584 434 to 442 / 423 to
+        434; at 509 rows, where the model sees no gain, 127 to 134 / 128)."""
+        iters, units = k // 64, self.compute_units
+        best = 0.98 * self._block_cost(m, n, k, plan, gated), plan
+        for tn, tm in self._BLOCK_TILES:
+            m_tiles = -(-m // (32 * tm))
+            for rounds in range(1, -(-n // (32 * tn)) * m_tiles // units + 1):
+                first = rounds * units // m_tiles * 32 * tn
+                if not 0 < first < n:
+                    continue
+                head = self._block_cost(m, first, k, (iters, 1, tn, tm), gated) + 3.0
+                for rest in self._BLOCK_TILES:
+                    cost = head + self._block_cost(m, n - first, k, (iters, 1, *rest), gated)
+                    if cost < best[0]:
+                        best = cost, (iters, 1, tn, tm, first, *rest)
+        return best[1]
+
     def _block_cost(self, m: int, n: int, k: int, plan: tuple[int, int, int, int], gated: bool = False) -> float:
         """What :meth:`_block_plan` compares, in microseconds."""
         per_split, splits, tn, tm = plan
@@ -2291,7 +2312,7 @@ class Ops:
         _need(self.block_supported(x, weight), "the block product takes bfloat16 rows of 16-byte pieces, K % 64 == 0 and N % 16 == 0")
         return self._block_product(x, weight, bias, plan=plan, gated=gated, sums=sums, rule=rule)
 
-    def _block_product(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, *, plan: tuple[int, int, int, int],
+    def _block_product(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, *, plan: tuple[int, ...],
                        gated: bool, sums: bool, rule: tuple[float, float, float]) -> torch.Tensor:
         """:meth:`gemm_block` of operands on the GPU that ``block_supported`` has been asked about: the choice of
         a kernel asks it anyway, and a prompt of a small model is bound by the host (8 layers 2,048 wide, 33 to 256
@@ -2301,17 +2322,23 @@ class Ops:
         if bias is not None:
             _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 8 == 0,
                   "bias must be bfloat16 [N]")
-        per_split, splits, tn, tm = plan
+        per_split, splits, tn, tm, *tail = plan
         _need(not gated or splits == 1, "the gated result needs one range of K")
+        _need(not tail or (splits == 1 and not sums and 0 < tail[0] < n and tail[0] % 16 == 0), "a tail is for one range of K and one result")
         partial = out = None
         if gated or (splits == 1 and not sums):
             out = self.rows_buffer(m, n // 2 if gated else n, torch.bfloat16, x.device)
         else:
             partial = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
         unit = glu_rule(rule) if gated else (1.0, 0.0, 0.0, 0.0)
-        _check(self.core.ts_gemm_block(_ptr(partial), _ptr(out), _ptr(x), x.stride(0), _ptr(weight), _ptr(bias), m, n, k, per_split,
-                                       splits, tn, tm, 2 if gated else 1 if out is None else 0, *unit, self.stream()),
-               "ts_gemm_block")
+        mode = 2 if gated else 1 if out is None else 0
+        runs = [(0, n, tn, tm)] if not tail else [(0, tail[0], tn, tm), (tail[0], n - tail[0], *tail[1:])]
+        for first, rows, tile_n, tile_m in runs:
+            at = None if out is None else out.data_ptr() + 2 * (first // 2 if gated else first)
+            _check(self.core.ts_gemm_block(_ptr(partial), at, _ptr(x), x.stride(0), weight.data_ptr() + 2 * first * k,
+                                           None if bias is None else bias.data_ptr() + 2 * first, m, rows, k, per_split, splits,
+                                           tile_n, tile_m, mode, n, *unit, self.stream()),
+                   "ts_gemm_block")
         return partial if out is None else out
 
     def _own_product(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, kind: str,
@@ -2345,6 +2372,8 @@ class Ops:
         short = block_takes and kind == "sums" and m <= self.wide_default_rows and wide[0] <= 11
         if block_takes and not short:
             block = self._block_plan(m, n, k, kind)
+            if kind != "sums":
+                block = self._block_rounds(m, n, k, kind == "gated", block)
             # One range too stays 32-bit up to the rows at which gemm_wide's ranges leave partial sums (a plan of one range
             # there is wide: 16,384 x 16,384), above as the library's result is.
             sums = float32 or (kind == "sums" and m <= self.wide_default_rows)
