@@ -691,3 +691,29 @@ def test_the_command_line_serves_the_design(tmp_path, capsys):
     sizing = capsys.readouterr().out
     sizing = json.loads(sizing[sizing.index("{"):])
     assert sizing["bytes_per_block"] == [2 * (16 + 24) * 2 * page] and sizing["activation_bytes"] > 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("splits", [1, 2, 4, 5, 8])
+@pytest.mark.parametrize("tokens,channels,parts,silu,bias", [(1, 4, 1, True, True), (3, 260, 1, False, False), (8, 1024, 4, True, False), (63, 516, 3, True, True)])
+def test_a_steps_short_kernels_have_the_bits_of_the_general_ones(ops, dtype, splits, tokens, channels, parts, silu, bias):
+    """Convolution (channels past the last block's, shuffled slots) and gated norm of single tokens from up to eight partial sums; as
+    many more that are zero go to the general kernels, which add them up in the same order."""
+    g = torch.Generator().manual_seed(splits + channels)
+    width = channels + 8
+    some = torch.randn(splits, tokens, width, generator=g).to(DEV)
+    more = torch.cat([some, torch.zeros(9 - splits, tokens, width, device=DEV)])
+    taps = torch.randn(channels, 4, generator=g).to(dtype).to(DEV)
+    add = torch.randn(channels, generator=g).to(dtype).to(DEV) if bias else None
+    slots = torch.randperm(tokens + 2, generator=g)[:tokens].to(torch.int32).to(DEV)
+    held = torch.randn(tokens + 2, 3, channels, generator=g).to(DEV)
+    each = torch.arange(tokens + 1, dtype=torch.int32, device=DEV)
+    got = []
+    for parts_of in (some, more):
+        state = held.clone()
+        out = ops.short_conv(parts_of, 4, taps, state, slots, each[:-1], each, tokens=tokens, num_seqs=tokens, dtype=dtype, silu=silu, bias=add)
+        got.append((out, state))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    y, gain = torch.randn(tokens, channels, generator=g).to(DEV), torch.randn(channels, generator=g).to(dtype).to(DEV)
+    short, general = (ops.gated_group_norm(y, parts_of, 4, gain, 1e-5, parts, dtype) for parts_of in (some, more))
+    assert torch.equal(short, general)

@@ -881,6 +881,40 @@ gated_group_norm_kernel(T* __restrict__ out, const float* __restrict__ y, const 
   }
 }
 
+// The same bits for a step of few parts of up to 1,024 elements, at most BATCH partial sums: everything a part needs is asked for at once,
+// and the code is short and straight (other kernels of a recorded step have put it out of the instruction cache).
+template <typename T, typename P, int THREADS, int BATCH>
+__global__ void __launch_bounds__(THREADS)
+gated_group_norm_few_kernel(const P* proj, const float* y, const T* gain, T* out, int splits, int width, size_t split_stride, int z_at,
+                            int parts, int size, float eps) {
+  __shared__ __attribute__((aligned(16))) float scratch[(THREADS / TS_WAVE + 3) / 4 * 4];
+  const int t = blockIdx.x, part = blockIdx.y;
+  const size_t row = ((size_t)t * parts + part) * size;
+  const bool in = 4 * (int)threadIdx.x < size;
+  const int i = min(4 * (int)threadIdx.x, size - 4);
+  const P* z = proj + (size_t)t * width + z_at + (size_t)part * size + i;
+  float gates[BATCH][4], v[4], w[4];
+#pragma unroll
+  for (int j = 0; j < BATCH; ++j) load_vec<P, 4>(z + (size_t)min(j, splits - 1) * split_stride, gates[j]);
+  load_vec<float, 4>(y + row + i, v);
+  load_vec<T, 4>(gain + (size_t)part * size + i, w);
+  asm volatile("" ::: "memory");  // all of them on their way here
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float gate = gates[0][e];
+#pragma unroll
+    for (int j = 1; j < BATCH; ++j) gate = j < splits ? gate + gates[j][e] : gate;
+    v[e] *= gate / (1.f + expf(-gate));
+    ss = in ? fmaf(v[e], v[e], ss) : ss;
+  }
+  const float by = rsqrtf(block_sum_of<THREADS>(ss, scratch) / (float)size + eps);
+  if (!in) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] *= by * w[e];
+  store_vec<T, 4>(out + row + i, v);
+}
+
 // ---------------------------------------------------------------------------------------------
 // the finish
 // ---------------------------------------------------------------------------------------------
@@ -1146,6 +1180,23 @@ static int launch_gated_group_norm(void* out, const float* y, const void* proj, 
   if (wide) {
     const int pieces = size / 4;
     const bool few = (long)tokens * parts < 256;
+    if (few && pieces <= 256 && splits <= 8) {
+#define GN_FEW(THREADS, BATCH)                                                                                                      \
+  hipLaunchKernelGGL((gated_group_norm_few_kernel<T, P, THREADS, BATCH>), dim3(tokens, parts), dim3(THREADS), 0, stream,            \
+                     (const P*)proj, y, (const T*)gain, (T*)out, splits, width, (size_t)split_stride, z_at, parts, size, eps)
+#define GN_BATCH(THREADS)                     \
+  do {                                        \
+    if (splits == 1) GN_FEW(THREADS, 1);      \
+    else if (splits <= 4) GN_FEW(THREADS, 4); \
+    else GN_FEW(THREADS, 8);                  \
+  } while (0)
+      if (pieces <= 64) GN_BATCH(64);
+      else if (pieces <= 128) GN_BATCH(128);
+      else GN_BATCH(256);
+#undef GN_BATCH
+#undef GN_FEW
+      return ts_launch_status();
+    }
     if (pieces <= 256 || (few && pieces <= 1024)) GN_GO(4, 1, (pieces + 63) / 64 * 64);
     else if (pieces <= 1024) GN_GO(4, 4, 256);
     else if (pieces <= 4096) GN_GO(4, 4, 1024);

@@ -65,6 +65,43 @@ short_conv_kernel(O* __restrict__ out, const P* __restrict__ proj, int splits, s
   out[(size_t)t * channels + c] = from_float<O>(y);
 }
 
+// The same bits for a step of single tokens with four taps and at most BATCH partial sums: everything a channel needs is asked for at
+// once.  (In the general kernel each tap's loads wait for the state's of the tap before, and the code is
+// fetched a jump at a time: other kernels of a recorded step have put it out of the instruction cache.)
+template <typename T, typename P, typename O, int BATCH>
+__global__ void __launch_bounds__(256)
+short_conv_single_kernel(const P* proj, const T* taps, const int* state_slots, float* state, int splits, int width, size_t split_stride,
+                         int first_col, int channels, const T* bias, O* out, int activation) {
+  const int c = blockIdx.y * 256 + threadIdx.x, t = blockIdx.x, at = min(c, channels - 1);
+  const P* row = proj + (size_t)t * width + first_col + at;
+  float* held = state + (size_t)state_slots[t] * 3 * channels + at;
+  P part[BATCH];
+  T w[4], add = {};
+  float old[3];
+#pragma unroll
+  for (int j = 0; j < BATCH; ++j) part[j] = row[(size_t)min(j, splits - 1) * split_stride];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) w[j] = taps[(size_t)at * 4 + j];
+  if (bias) add = bias[at];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) old[j] = held[(size_t)j * channels];
+  asm volatile("" ::: "memory");  // all of them on their way here
+  float mine = splits == 1 ? to_float(part[0]) : 0.f + to_float(part[0]);
+#pragma unroll
+  for (int j = 1; j < BATCH; ++j) mine = j < splits ? mine + to_float(part[j]) : mine;
+  float y = 0.f;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) y = fmaf(to_float(w[j]), old[j], y);
+  y = fmaf(to_float(w[3]), mine, y);
+  if (bias) y += to_float(add);
+  if (activation == 1) y = y / (1.f + expf(-y));
+  if (c >= channels) return;
+  held[0] = old[1];
+  held[channels] = old[2];
+  held[(size_t)2 * channels] = mine;
+  out[(size_t)t * channels + c] = from_float<O>(y);
+}
+
 // Prompt portions: bfloat16 in, four neighbouring channels by SC_TILE consecutive rows a thread, 8-byte
 // accesses; every input row is read once for all the taps that want it (and the taps of a thread's channels once).  A
 // row's request is the same for all threads of a block, so the cases below are uniform branches.  Per element the
@@ -175,6 +212,23 @@ extern "C" int ts_short_conv(void* out, int out_f32, const void* proj, int in_f3
       SC_ROWS(1) SC_ROWS(2) SC_ROWS(3) SC_ROWS(4) SC_ROWS(5) SC_ROWS(6) SC_ROWS(7) SC_ROWS(8)
     }
 #undef SC_ROWS
+    return ts_launch_status();
+  }
+  if (single && k == 4 && splits <= 8 && (dtype == TS_F32 || (dtype == TS_BF16 && in_f32))) {
+#define SC_SINGLE(T, O, BATCH)                                                                                                      \
+  hipLaunchKernelGGL((short_conv_single_kernel<T, float, O, BATCH>), grid, block, 0, stream, (const float*)proj, (const T*)taps, state_slots, \
+                     state, splits, width, (size_t)split_stride, first_col, channels, (const T*)bias, (O*)out, activation)
+#define SC_SINGLES(T, O)                       \
+  do {                                         \
+    if (splits == 1) SC_SINGLE(T, O, 1);       \
+    else if (splits <= 4) SC_SINGLE(T, O, 4);  \
+    else SC_SINGLE(T, O, 8);                   \
+  } while (0)
+    if (dtype == TS_F32) SC_SINGLES(float, float);
+    else if (out_f32) SC_SINGLES(bf16_t, float);
+    else SC_SINGLES(bf16_t, bf16_t);
+#undef SC_SINGLES
+#undef SC_SINGLE
     return ts_launch_status();
   }
 #define SC_GO(T, P, O)                                                                                                   \
