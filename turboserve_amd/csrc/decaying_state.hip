@@ -152,10 +152,11 @@ __device__ __forceinline__ void ss_log_gates(const P* proj, const SsGates& gates
 // workgroup; BATCH: tokens staged in LDS at a time.  norm [T, H, 2] (gated): n . C and the running maximum.
 template <typename U, typename P, int RULE, int NR, int BATCH, int COLS>
 __global__ void __launch_bounds__(SS_PARTS * COLS, NR <= 32 ? 5 : 2)
-decaying_walk_kernel(float* __restrict__ y, float* __restrict__ norm, float* __restrict__ state, float* __restrict__ sums,
+decaying_walk_kernel(float* __restrict__ state, const int* __restrict__ state_slots, const int* __restrict__ query_start_loc, int first_seq,
+                     int heads, int groups, int n, int p, float* __restrict__ y, float* __restrict__ norm, float* __restrict__ sums,
                      const float* __restrict__ tops, const U* __restrict__ u, SsRows rows, const P* __restrict__ proj, SsGates gates,
-                     const float* __restrict__ skip, float scale, const int* __restrict__ state_slots,
-                     const int* __restrict__ query_start_loc, int first_seq, int heads, int groups, int n, int p) {
+                     const float* __restrict__ skip, float scale) {
+  // (Fourteen words of arguments lie in registers at the start: what the state's loads want comes first.)
   constexpr int ROWS = SS_PARTS * NR, THREADS = SS_PARTS * COLS;
   __shared__ __attribute__((aligned(16))) float bs[BATCH][ROWS];
   __shared__ __attribute__((aligned(16))) float cs[BATCH][ROWS];
@@ -166,43 +167,50 @@ decaying_walk_kernel(float* __restrict__ y, float* __restrict__ norm, float* __r
   const int c0 = blockIdx.z * COLS, c = c0 + col_in;
   const bool summing = RULE == SS_GATED && c == p;  // the column of n
   const bool live = c < p || summing;
-  const int row0 = query_start_loc[seq], count = query_start_loc[seq + 1] - row0;
+  int row0 = query_start_loc[seq], row_end = query_start_loc[seq + 1];
   const size_t b_at = (size_t)rows.b_at + (size_t)g * n, c_at = (size_t)rows.c_at + (size_t)g * n, x_at = (size_t)rows.x_at + (size_t)h * p;
-  const size_t owner = (size_t)state_slots[seq] * heads + h;
+  int slot = state_slots[seq];
+  // The other arguments, the rows and the slot come with one wait.
+  asm volatile("" : "+s"(slot), "+s"(row0), "+s"(row_end) : "s"(u), "s"(proj), "s"(gates.one), "s"(gates.two), "s"(skip), "s"(rows.stride), "s"(rows.width), "s"(gates.stride), "s"(gates.width));
+  const int count = row_end - row0;
+  const size_t owner = (size_t)slot * heads + h;
   float* held = summing ? sums + owner * n : state + (owner * p + (live ? c : 0)) * n;
   const bool quads = n % 4 == 0;
   float s[NR];
+  // The loads are unconditional (rows past N, columns past P: others of the same state, dropped below), so that they are on their way
+  // together: with a branch about each the compiler waited for one before it asked for the next.
+  if (quads) {
 #pragma unroll
-  for (int x = 0; x < NR / 4; ++x) {
-    const int d = x * 4 * SS_PARTS + part * 4;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (live && quads) {
-      if (d < n) v = *reinterpret_cast<const float4*>(held + d);
-    } else if (live) {
-      if (d < n) v.x = held[d];
-      if (d + 1 < n) v.y = held[d + 1];
-      if (d + 2 < n) v.z = held[d + 2];
-      if (d + 3 < n) v.w = held[d + 3];
+    for (int x = 0; x < NR / 4; ++x) {
+      const int d = x * 4 * SS_PARTS + part * 4;
+      const float4 v = *reinterpret_cast<const float4*>(held + (d < n ? d : 0));
+      s[4 * x] = v.x; s[4 * x + 1] = v.y; s[4 * x + 2] = v.z; s[4 * x + 3] = v.w;
     }
-    s[4 * x] = v.x; s[4 * x + 1] = v.y; s[4 * x + 2] = v.z; s[4 * x + 3] = v.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < NR; ++e) {
+      const int d = e / 4 * 4 * SS_PARTS + part * 4 + e % 4;
+      s[e] = held[d < n ? d : 0];
+    }
   }
-  float rate = 0.f, bias = 0.f, d_skip = 0.f, top = 0.f;
-  if (RULE == SS_SELECTIVE) {
-    rate = expf(gates.two[h]);
-    bias = gates.one[h];
-    d_skip = skip[h];
+  if (n < ROWS) {
+#pragma unroll
+    for (int e = 0; e < NR; ++e) s[e] = e / 4 * 4 * SS_PARTS + part * 4 + e % 4 < n ? s[e] : 0.f;
   }
+  float rate = 0.f, d_skip = 0.f, top = 0.f;
+  if (RULE == SS_SELECTIVE) d_skip = skip[h];
   if (RULE == SS_FIXED) rate = gates.one[h];
   if (RULE == SS_GATED) top = tops[owner];
   for (int base = 0; base < count; base += BATCH) {
     const int batch = min(BATCH, count - base);
     if (base > 0) __syncthreads();  // the batch before is done with what is staged
-    // The gates are the second wavefront's, x the last ones': a step of one token waits for them side by side.
-    const int lane = tid - TS_WAVE;
+    // The gates are the third wavefront's, x the last ones', B and C begin with the first: a step of one token waits for them side by side.
+    const int lane = tid - 2 * TS_WAVE;
     if (RULE == SS_SELECTIVE && lane >= 0 && lane < batch) {
-      const float dt = ss_softplus(ss_input(proj + (size_t)(row0 + base + lane) * gates.width + gates.first + h, gates.splits, gates.stride) + bias);
+      const float one = gates.one[h], two = gates.two[h];  // beside the gates' inputs: asked for before, they were waited for first
+      const float dt = ss_softplus(ss_input(proj + (size_t)(row0 + base + lane) * gates.width + gates.first + h, gates.splits, gates.stride) + one);
       ws[lane] = dt;
-      as[lane] = expf(-rate * dt);
+      as[lane] = expf(-expf(two) * dt);
     }
     if (RULE == SS_FIXED && lane >= 0 && lane < batch) {
       ws[lane] = 1.f;
@@ -1021,8 +1029,8 @@ extern "C" int ts_decaying_walk(float* y, float* norm, float* state, float* sums
   const int columns = rule == SS_GATED ? p + 1 : p;
 #define SS_GO(U, P, RULE, NR, BATCH, COLS)                                                                                            \
   hipLaunchKernelGGL((decaying_walk_kernel<U, P, RULE, NR, BATCH, COLS>), dim3(num_seqs, heads, (columns + COLS - 1) / COLS),         \
-                     dim3(SS_PARTS * COLS), 0, stream, y, norm, state, sums, tops, (const U*)u, rows, (const P*)proj, gates, skip,   \
-                     scale, state_slots, query_start_loc, first_seq, heads, groups, n, p)
+                     dim3(SS_PARTS * COLS), 0, stream, state, state_slots, query_start_loc, first_seq, heads, groups, n, p, y, norm,  \
+                     sums, tops, (const U*)u, rows, (const P*)proj, gates, skip, scale)
 #define SS_SIZES(U, P, RULE)                                     \
   do {                                                           \
     if (n <= 32) SS_GO(U, P, RULE, 4, 8, 32);                    \
