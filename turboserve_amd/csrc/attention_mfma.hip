@@ -14,9 +14,9 @@
 // bfloat16 for the second product.
 //
 // Decode kernel: the 16 columns are the query heads of one KV head (G of them, the rest
-// padding), for one request whose step brings a single token.  The keys lo..ctx-1 are split
-// over `splits` wavefronts (flash-decoding); each writes an unnormalised partial (m, l, acc)
-// and a second kernel combines them.  Equals the reference's decode kernel
+// padding), for one request whose step brings a single token.  The windows of its keys lo..ctx-1 go to the wavefronts of one
+// workgroup, which joins their sums, or of `splits` workgroups; each then writes an unnormalised partial (m, l, acc) and a second
+// kernel combines them.  Equals the reference's decode kernel
 // (src/turboserve/engine/model/triton_attention.py:110-174) and, with a window, keeps only
 // the keys p - window + 1 .. p.
 //
