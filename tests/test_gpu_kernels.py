@@ -57,10 +57,11 @@ def test_rmsnorm_and_fused_residual(ops, dtype, tokens, hidden):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows,hidden", [(1, 4), (63, 1024), (3, 1028), (256, 2048), (2, 2052), (1, 4096), (5, 4100), (257, 2052), (512, 4096), (2, 8192)])
+@pytest.mark.parametrize("rows,hidden", [(1, 4), (63, 1024), (3, 1028), (256, 2048), (2, 2052), (1, 4096), (5, 4100), (257, 2052), (512, 4096), (2, 8192),
+                                         (513, 2052), (600, 3584), (600, 5120), (1025, 1024), (1025, 1028), (1025, 2048), (513, 8192)])
 def test_short_norms_have_the_bits_of_the_general_ones(ops, dtype, rows, hidden):
-    """A step's own norm kernels take up to 16 (8) partial sums at the edges of their threads; as many again that are zero, more than they
-    take, go to the general kernels, which add them up in the same order."""
+    """The short norm kernels take up to 16 (8; 4 in a long step) partial sums at the edges of their threads and items; as many again that are
+    zero, more than they take, go to the general kernels, which add them up in the same order."""
     g = torch.Generator().manual_seed(rows + hidden)
     residual = torch.randn(rows, hidden, generator=g).to(DEV)
     w, b = ((1 + 0.1 * torch.randn(2, hidden, generator=g)).to(dtype).to(DEV))

@@ -398,11 +398,12 @@ static void launch_add_rmsnorm_few(void* y, float* residual, const void* pending
 #define TS_NORM_FEW(BATCH)                                                                                                      \
   hipLaunchKernelGGL((add_rmsnorm_few_kernel<T, P, THREADS, ITEMS, BATCH>), dim3(out_rows), dim3(THREADS), 0, stream, (const P*)pending, \
                      residual, (const T*)w, rows, (T*)y, splits, hidden, (size_t)split_stride, eps, gain_offset, one_rounding)
+  constexpr int MOST = ITEMS * THREADS == 2048 && THREADS == 1024 ? 8 : ITEMS == 1 || (THREADS == 512 && ITEMS == 2) ? 16 : 4;
   if (splits == 1) TS_NORM_FEW(1);
   else if (splits == 2) TS_NORM_FEW(2);
   else if (splits <= 4) TS_NORM_FEW(4);
-  else if (splits <= 8) TS_NORM_FEW(8);
-  else TS_NORM_FEW(ITEMS * THREADS == 2048 ? 8 : 16);
+  else if (splits <= 8) TS_NORM_FEW(MOST < 8 ? MOST : 8);
+  else TS_NORM_FEW(MOST);
 #undef TS_NORM_FEW
 }
 
@@ -425,22 +426,38 @@ static void launch_add_rmsnorm(void* y, float* residual, const void* pending, in
   if (out_rows <= 512 && threads <= (FLOAT32 ? 128 : 256)) threads *= 2;
   else if (out_rows <= 1024 && hidden > 1024 && threads < 256) threads = 256;
   if (out_rows <= 256 && threads < 1024) threads = 1024;
-  // (32-bit rows of fewer threads add their squares in the order of 1,024: TS_NORM_SUMS.  Steps of more than 512 rows fetch a
-  // kernel's code once for several rows a unit, and memory bounds them.)
+  // (32-bit rows of fewer threads add their squares in the order of 1,024: TS_NORM_SUMS.)
   const int items = (hidden / 4 + threads - 1) / threads;
-  if (hidden % 4 == 0 && pending && !also && !post_gain &&
-      ((threads == 1024 && items <= 2 && splits <= 16 / items) || (!FLOAT32 && threads == 512 && items == 2 && splits <= 16))) {
+  const bool plain = hidden % 4 == 0 && pending && !also && !post_gain;
 #define TS_NORM_ITEMS(THREADS, ITEMS) \
   launch_add_rmsnorm_few<T, P, THREADS, ITEMS>(y, residual, pending, splits, split_stride, w, rows, eps, out_rows, hidden, gain_offset, one_rounding, stream)
+  if (plain && threads == 1024 && items <= 2 && splits <= 16 / items) {
     // (Wavefronts past the row's end would add zeros to its sum, and load.)
-    if (threads == 512) TS_NORM_ITEMS(512, 2);
-    else if (hidden <= 1024) TS_NORM_ITEMS(256, 1);
+    if (hidden <= 1024) TS_NORM_ITEMS(256, 1);
     else if (hidden <= 2048) TS_NORM_ITEMS(512, 1);
     else if (items == 1) TS_NORM_ITEMS(1024, 1);
     else TS_NORM_ITEMS(1024, 2);
-#undef TS_NORM_ITEMS
     return;
   }
+  if constexpr (!FLOAT32) {
+    // A prompt's rows: in the general kernel a thread's items are behind a branch each, and the compiler waits for the loads of one
+    // before it asks for the next's.  (Steps, us: 2,048 tokens, 56 norms of rows of 3,584, 24,090 -> 23,708; 2,048 rows of 5,120, 96 norms,
+    // 50,260 -> 49,040.)
+    if (plain && threads < 1024 && items >= 2 && splits <= (threads == 512 && items == 2 ? 16 : 4)) {
+#define TS_NORM_THREADS(THREADS)                  \
+  do {                                            \
+    if (items == 2) TS_NORM_ITEMS(THREADS, 2);    \
+    else if (items == 3) TS_NORM_ITEMS(THREADS, 3); \
+    else TS_NORM_ITEMS(THREADS, 4);               \
+  } while (0)
+      if (threads == 128) TS_NORM_THREADS(128);
+      else if (threads == 256) TS_NORM_THREADS(256);
+      else TS_NORM_THREADS(512);
+#undef TS_NORM_THREADS
+      return;
+    }
+  }
+#undef TS_NORM_ITEMS
   const PostNorm<T> post = {(const T*)post_gain, post_eps, post_scale};
 #define TS_NORM(POST, SUMS)                                                                                                   \
   hipLaunchKernelGGL((add_rmsnorm_vec4_kernel<T, P, POST, SUMS>), dim3(out_rows), dim3(threads), 0, stream, (T*)y, residual,   \
