@@ -636,8 +636,23 @@ def test_a_product_in_two_launches_is_the_product_in_one(ops, m, n, first, tiles
     for b in (None, bias):
         want = ops.gemm_block(x, w, b, plan=(3, 1, 4, 4), gated=gated)
         assert torch.equal(ops.gemm_block(x, w, b, plan=(3, 1, *tiles, first, *rest), gated=gated), want)
+        if not gated:
+            want = ops.gemm_block(x, w, b, plan=(3, 1, 4, 4), sums=True)
+            assert torch.equal(ops.gemm_block(x, w, b, plan=(3, 1, *tiles, first, *rest), sums=True), want)
     plan = ops._block_rounds(2048, 27648, 5120, True, ops._block_plan(2048, 27648, 5120, "gated"))
     assert len(plan) == 7 and plan[4] % 32 == 0 and 0 < plan[4] < 27648
+
+
+@pytest.mark.parametrize("m", [17, 33, 100])
+def test_a_wide_head_in_two_launches_is_the_product(ops, m):
+    """At 17 to 128 rows: two rounds of 256 tiles of 256 weight rows and a rest of 144 in tiles of 128, the same bits as one launch."""
+    g = torch.Generator().manual_seed(m)
+    n, k = 131072 + 144, 64
+    x, w = torch.randn(m, k, generator=g).bfloat16().to(DEV), (torch.randn(n, k, generator=g) / 8).bfloat16().to(DEV)
+    plan = ops._block_few_runs(x, w, None, 1)
+    tm = 1 if m <= 32 else 2 if m <= 64 else 4
+    assert plan == (1, 1, 8, tm, 131072, 4, tm)
+    assert torch.equal(ops.linear_float32_out(x, w), ops.gemm_block(x, w, plan=(1, 1, 4, tm), sums=True)[0])
 
 
 @pytest.mark.parametrize("m,n,k,offset", [(17, 4608, 3584, 0), (32, 2048, 2048, 0), (33, 2064, 576, 0), (64, 512, 64, 0), (65, 528, 640, 0), (128, 272, 1088, 4),

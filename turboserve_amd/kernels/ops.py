@@ -2324,7 +2324,7 @@ class Ops:
                   "bias must be bfloat16 [N]")
         per_split, splits, tn, tm, *tail = plan
         _need(not gated or splits == 1, "the gated result needs one range of K")
-        _need(not tail or (splits == 1 and not sums and 0 < tail[0] < n and tail[0] % 16 == 0), "a tail is for one range of K and one result")
+        _need(not tail or (splits == 1 and 0 < tail[0] < n and tail[0] % 16 == 0), "a tail is for one range of K")
         partial = out = None
         if gated or (splits == 1 and not sums):
             out = self.rows_buffer(m, n // 2 if gated else n, torch.bfloat16, x.device)
@@ -2335,7 +2335,8 @@ class Ops:
         runs = [(0, n, tn, tm)] if not tail else [(0, tail[0], tn, tm), (tail[0], n - tail[0], *tail[1:])]
         for first, rows, tile_n, tile_m in runs:
             at = None if out is None else out.data_ptr() + 2 * (first // 2 if gated else first)
-            _check(self.core.ts_gemm_block(_ptr(partial), at, _ptr(x), x.stride(0), weight.data_ptr() + 2 * first * k,
+            sums_at = None if partial is None else partial.data_ptr() + 4 * first
+            _check(self.core.ts_gemm_block(sums_at, at, _ptr(x), x.stride(0), weight.data_ptr() + 2 * first * k,
                                            None if bias is None else bias.data_ptr() + 2 * first, m, rows, k, per_split, splits,
                                            tile_n, tile_m, mode, n, *unit, self.stream()),
                    "ts_gemm_block")
@@ -2647,13 +2648,29 @@ class Ops:
         return self.gemm_tiled(x, weight, bias, max_splits=max_splits)
 
     def _block_few_runs(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
-                        max_splits: int | None) -> tuple[int, int, int, int] | None:
+                        max_splits: int | None) -> tuple[int, ...] | None:
         """The block product's grid where it runs a decode-sized product (17 to 128 rows)."""
         if not self.stream_max_rows < x.shape[0] <= self.skinny_max_rows or not self.block_supported(x, weight):
             return None
         if bias is not None and bias.data_ptr() % 8:
             return None
-        return self._block_few_plan(x.shape[0], weight.shape[0], weight.shape[1], max_splits)
+        m, (n, k) = x.shape[0], weight.shape
+        return (self._block_few_rounds(m, n, k) if max_splits == 1 else None) or self._block_few_plan(m, n, k, max_splits)
+
+    def _block_few_rounds(self, m: int, n: int, k: int) -> tuple[int, ...] | None:
+        """A matrix of more than 65,536 rows (a head) as one range of K for a decode step: whole rounds of tiles of 256 and the rest in one
+        round of tiles of 128, a launch each (as :meth:`_block_rounds` has it), where that is 3% sooner than one tile's rounds, or None
+        (us, 152,064 x 3,584 at 24 / 64 / 128 rows 177 / 194 / 220 against 197 / 211 / 229 by gemm_wide and the tiled kernel, 152,064 x 5,120 248 / 276 /
+        308 against 268 / 305 / 323).  Not over a K of 8,192 or more, where tiles of 256 read slowly (:meth:`_block_few_plan`)."""
+        units, pace = self.compute_units, self._BLOCK_ONE_RANGE
+        rounds = -(-n // 256) // units
+        rest = n - rounds * units * 256
+        if rounds == 0 or not 0 < rest <= 128 * units or k >= 8192:
+            return None
+        if rounds * pace[8] + pace[4] >= 0.97 * min(-(-(-(-n // (32 * tn))) // units) * pace[tn] for tn in pace):
+            return None
+        tm = 1 if m <= 32 else 2 if m <= 64 else 4
+        return k // 64, 1, 8, tm, n - rest, 4, tm
 
     def _few_rows_wide(self, m: int, n: int, k: int, max_splits: int | None) -> bool:
         """Whether a decode-sized product that the block kernel leaves (``_block_few_runs``) runs ``gemm_wide``
