@@ -1,0 +1,97 @@
+"""Which launches a decode step's attention layer takes, decided on the host: the launch that also rotates and stores is for plain
+attention of a plain rotation alone."""
+
+from __future__ import annotations
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from turboserve_amd.kernels.ops import Ops
+from turboserve_amd.parts.attention import GroupedQueryAttention
+from turboserve_amd.parts.base import PartSpec, Runtime
+from turboserve_amd.parts.registry import POSITION_ENCODINGS, register_position_encoding
+from turboserve_amd.parts.rope import RotaryEncoding
+
+
+class Launches:
+    """The operations an attention layer asks for, by name."""
+
+    mfma_attention_supported = staticmethod(Ops.mfma_attention_supported)
+
+    def __init__(self):
+        self.names = []
+
+    def linear(self, x, weight, bias, **more):
+        return torch.zeros(3, x.shape[0], weight.shape[0])
+
+    def rows_buffer(self, rows, width, dtype, device):
+        return torch.zeros(rows, width, dtype=dtype)
+
+    def tiled_attention_supported(self, *geometry):
+        return False
+
+    def float32_attention_supported(self, *operands):
+        return False
+
+    def rope_store(self, proj, k, v, cos, sin, positions, slots, heads, *more):
+        self.names.append("store")
+        return torch.zeros(proj.shape[1], heads * k.shape[3], dtype=torch.bfloat16), heads * k.shape[3]
+
+    def attention_decode(self, out, q, *more, projected=None, **rest):
+        self.names.append("attention" if projected is None else "all in one")
+
+    def paged_attention_generic(self, *more, **rest):
+        self.names.append("generic")
+
+
+class RotaryAndSlopes(RotaryEncoding):
+    """A rotation whose scores also fall with the distance."""
+
+    def score_slopes(self, num_heads):
+        return torch.full((num_heads,), 0.5)
+
+
+class RotaryAndTable(RotaryEncoding):
+    def score_bias_table(self, num_heads):
+        return torch.zeros(num_heads, 4)
+
+
+class OwnAttention(GroupedQueryAttention):
+    """Attends in a way of its own."""
+
+    def attend(self, qkv, q_stride, ctx, cache, **more):
+        self.runtime.ops.names.append("own")
+        return qkv
+
+
+@pytest.fixture
+def encodings(monkeypatch):
+    for name, part in (("rope_slopes", RotaryAndSlopes), ("rope_table", RotaryAndTable)):
+        monkeypatch.delitem(POSITION_ENCODINGS, name, raising=False)
+        register_position_encoding(name)(part)
+    yield
+    for name in ("rope_slopes", "rope_table"):
+        POSITION_ENCODINGS.pop(name, None)
+
+
+@pytest.mark.parametrize("kind,encoding,launches", [
+    (GroupedQueryAttention, "rope", ["all in one"]),
+    (GroupedQueryAttention, "rope_slopes", ["store", "generic"]),
+    (GroupedQueryAttention, "rope_table", ["store", "generic"]),
+    (OwnAttention, "rope", ["store", "own"]),
+])
+def test_a_decode_step_attends_by_the_layers_rule(encodings, kind, encoding, launches):
+    ops = Launches()
+    runtime = Runtime(device=torch.device("cpu"), dtype=torch.bfloat16, ops=ops)
+    layer = kind("layer", runtime, hidden_size=64, num_heads=4, num_kv_heads=2, head_dim=32, scale=32 ** -0.5, qkv_bias=False, out_bias=False,
+                 window=None, position=PartSpec(encoding, {"head_dim": 32, "theta": 1e4, "max_positions": 64}))
+    layer.qkv_weight = torch.zeros(8 * 32, 64)
+    cache = SimpleNamespace(group=0, writable=True, block_size=16, k=torch.zeros(4, 2, 16, 32), v=torch.zeros(4, 2, 32, 16))
+    ints = torch.zeros(3, dtype=torch.int32)
+    ctx = SimpleNamespace(num_tokens=3, num_seqs=3, num_prefill_seqs=0, num_decode_seqs=3, max_context_len=20, max_decode_context_len=20,
+                          block_tables=[torch.zeros(3, 4, dtype=torch.int32)], slot_mapping=[ints], positions=ints, token_seq=ints,
+                          query_start_loc=ints, context_lens=ints, max_decode_context_dev=ints[:1], carried={})
+    layer.heads_out(torch.zeros(3, 64), ctx, cache)
+    assert ops.names == launches

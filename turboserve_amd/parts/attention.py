@@ -356,6 +356,10 @@ class GroupedQueryAttention(Mixer):
                 or not self.own_keys or not cache.writable
                 or not ops.mfma_attention_supported(self.runtime.dtype, self.head_dim, cache.block_size)):
             return None
+        # What attends in a way of its own is asked (`attend`), and so is an encoding that also acts inside the scores.
+        if (type(self).attend is not GroupedQueryAttention.attend or self.position.score_slopes(self.num_heads) is not None
+                or self.position.score_bias_table(self.num_heads) is not None):
+            return None
         tables = self.position.rotation(self.head_dim, ctx)
         if tables is None:
             return None
