@@ -95,3 +95,13 @@ def test_a_decode_step_attends_by_the_layers_rule(encodings, kind, encoding, lau
                           query_start_loc=ints, context_lens=ints, max_decode_context_dev=ints[:1], carried={})
     layer.heads_out(torch.zeros(3, 64), ctx, cache)
     assert ops.names == launches
+
+
+@pytest.mark.parametrize("workgroups,span,head_dim,waves", [
+    (256, 128, 128, 8), (257, 1024, 128, 4), (1023, 512, 128, 4), (1024, 512, 128, 2), (1024, 1024, 128, 4), (257, 1025, 128, 8),
+    (320, 2048, 80, 4), (320, 2049, 80, 8), (512, 64, 64, 4), (2048, 64, 64, 2), (257, 2048, 256, 2), (256, 2048, 256, 8), (2048, 4096, 256, 8),
+])
+def test_more_workgroups_than_units_over_short_spans_share_units(workgroups, span, head_dim, waves):
+    """A workgroup of eight wavefronts has a unit to itself: 64 requests of 100 keys with 32 KV heads took eight turns of starts, 55 us
+    where a wavefront per stretch of keys had taken 34."""
+    assert Ops._decode_waves(SimpleNamespace(compute_units=256), workgroups, span, head_dim) == waves

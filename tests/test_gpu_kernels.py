@@ -1286,6 +1286,33 @@ def test_attention_decode_from_projected_sums(ops, monkeypatch, heads, kv_heads,
     torch.testing.assert_close(got[stored].float(), want[stored].float(), rtol=2.0**-7, atol=1e-6)
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,page", [(14, 2, 128, 8), (7, 1, 128, 64), (4, 4, 64, 32), (20, 1, 80, 16), (6, 2, 256, 8), (2, 2, 32, 64)])
+@pytest.mark.parametrize("waves", [8, 4, 2])
+@pytest.mark.parametrize("splits,window", [(1, None), (3, None), (1, 300)])
+def test_attention_decode_with_fewer_wavefronts(ops, monkeypatch, heads, kv_heads, dim, page, waves, splits, window):
+    """Eight, four or two wavefronts a workgroup, from encoded queries and from the projection's sums: plain attention's rows either
+    way, the new keys and values in their pages."""
+    contexts = [70, 1, 33, 600, 129, 32, 31, 257, 1000]
+    monkeypatch.setattr(type(ops), "_decode_splits", lambda self, pairs, span: splits)
+    monkeypatch.setattr(type(ops), "_decode_waves", lambda self, workgroups, span, head_dim: waves)
+    case = PagedCase(torch.bfloat16, heads, kv_heads, dim, page, [(c, 1) for c in contexts], window, seed=dim + page)
+    common = (case.dev(case.table), case.ints(case.qsl), case.ints(contexts), 0, len(contexts), heads, dim ** -0.5, window, max(contexts))
+    out = torch.zeros(len(contexts), heads * dim, dtype=torch.bfloat16, device=DEV)
+    ops.attention_decode(out, case.dev(case.q), heads * dim, case.dev(case.kp), case.dev(case.vp), *common)
+    torch.testing.assert_close(out.float().cpu(), case.expected, **tol(torch.bfloat16))
+    sums = torch.randn(5, len(contexts), (heads + 2 * kv_heads) * dim, generator=torch.Generator().manual_seed(dim)).to(DEV)
+    cos, sin = (t.to(DEV) for t in rotary_pair(1024, dim))
+    slots = case.ints([int(case.table[s, (c - 1) // page]) * page + (c - 1) % page for s, c in enumerate(contexts)])
+    pages = [(case.dev(case.kp).clone(), case.dev(case.vp).clone()) for _ in range(2)]
+    want, got = torch.zeros_like(out), torch.zeros_like(out)
+    q, stride = ops.rope_store(sums, *pages[0], cos, sin, case.ints([c - 1 for c in contexts]), slots, heads, kv_heads, dim, page, 1023, torch.bfloat16)
+    ops.attention_decode(want, q, stride, *pages[0], *common)
+    ops.attention_decode(got, sums, 0, *pages[1], *common, projected=(cos, sin, slots, 1023))
+    for a, b in zip(*pages):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    torch.testing.assert_close(got.float(), want.float(), rtol=2.0**-7, atol=1e-6)
+
+
 def rotary_pair(capacity, dim):
     angles = torch.outer(torch.arange(capacity).double(), 10000.0 ** (-torch.arange(dim // 2).double() * 2 / dim))
     return angles.cos().float(), angles.sin().float()

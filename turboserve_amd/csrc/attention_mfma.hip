@@ -381,7 +381,8 @@ __device__ __forceinline__ void attend(ColumnState& st, const WindowFrags& f, co
 __device__ __forceinline__ float column_sum(float l) { return groups_sum(l); }
 
 // ---------------------------------------------------------------------------------------------
-// decode: grid (splits, head_tiles * kv_heads, requests), DECODE_WAVES wavefronts a workgroup.  A request's windows go to its
+// decode: grid (splits, head_tiles * kv_heads, requests), WAVES wavefronts a workgroup: DECODE_WAVES, which have a compute unit to
+// themselves, or fewer where more workgroups than units have little to do (Ops._decode_waves).  A request's windows go to its
 // workgroups in turn, a workgroup's to its wavefronts in turn (so the first ones do not depend on the context's length); the
 // wavefronts' sums meet in LDS.
 // splits == 1: the rows of `out`; otherwise
@@ -393,8 +394,7 @@ __device__ __forceinline__ float column_sum(float l) { return groups_sum(l); }
 // KV head): one request of 640 keys 14.8 -> 11.2 -> 11.3, of 300 (4 to a KV head) 12.5 -> 9.9 -> 9.4, 8 of 8,191 34.9 -> 31.4 -> 30.0, 64 of
 // 128 to 1,535 40.7 -> 31.0 -> 27.0.
 // ---------------------------------------------------------------------------------------------
-constexpr int DECODE_WAVES = 4 * TS_WAVES_PER_SIMD;
-constexpr int DECODE_THREADS = DECODE_WAVES * TS_WAVE;
+constexpr int DECODE_WAVES = 4 * TS_WAVES_PER_SIMD;  // of the largest workgroup
 constexpr int SUM_ROW = D + 4;    // LDS stride of a column's sums: the columns start in different banks
 constexpr int QUERY_ROW = D + 8;  // of a query (bfloat16)
 
@@ -455,15 +455,16 @@ __device__ __forceinline__ void put_new_value(ValueFrags& f, const lds_u16* valu
 
 // What a workgroup takes from the projection, on its way to registers (`ask`: every load unconditional, so that the compiler
 // counts them and waits for these alone when others are behind them) and from there (`put`) into LDS.
+template <int THREADS>
 struct TokenPieces {
-  static constexpr int PASSES = (17 * (D / 8) + D / 4 + DECODE_THREADS - 1) / DECODE_THREADS, BATCH = D > 128 ? 2 : 4;
+  static constexpr int PASSES = (17 * (D / 8) + D / 4 + THREADS - 1) / THREADS, BATCH = D > 128 ? 2 : 4;
   f32x4 a[PASSES][BATCH], b[PASSES][BATCH], c[PASSES], s[PASSES];
 
   __device__ __forceinline__ void ask(const Projected& from, const float* row, int position, int columns, int first_head, int heads,
                                       int kv_heads, int kvh) {
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
-      const Piece piece = piece_of(threadIdx.x + i * DECODE_THREADS, columns, first_head, heads, kv_heads, kvh);
+      const Piece piece = piece_of(threadIdx.x + i * THREADS, columns, first_head, heads, kv_heads, kvh);
       const float* at = row + (size_t)piece.head * D;
 #pragma unroll
       for (int j = 0; j < BATCH; ++j) {
@@ -482,7 +483,7 @@ struct TokenPieces {
     const int items = (columns + 1) * (D / 8) + D / 4;
 #pragma unroll
     for (int i = 0; i < PASSES; ++i) {
-      const int item = threadIdx.x + i * DECODE_THREADS;
+      const int item = threadIdx.x + i * THREADS;
       const Piece piece = piece_of(item, columns, first_head, heads, kv_heads, kvh);
       f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
 #pragma unroll
@@ -606,7 +607,7 @@ __device__ __forceinline__ void stage_wait(int& slot) {
   asm volatile("s_waitcnt vmcnt(%1)" : "+s"(slot) : "n"(LEFT) : "memory");
 }
 
-template <bool PROJECTED>
+template <int WAVES, bool PROJECTED>
 __device__ __forceinline__ void decode_staged(ColumnState& st, lds_u16* __restrict__ to, const lds_u16* __restrict__ from,
                                               lds_u16* __restrict__ queries, lds_u16* __restrict__ new_key,
                                               lds_u16* __restrict__ new_value, const PageGeometry& geo, WindowPages pages,
@@ -616,7 +617,7 @@ __device__ __forceinline__ void decode_staged(ColumnState& st, lds_u16* __restri
   Stage stage;
   stage.init(lane, geo.block_shift);
   QueryFrags qf;
-  TokenPieces pieces;
+  TokenPieces<WAVES * TS_WAVE> pieces;
   if (PROJECTED) pieces.ask(token_sums, sum_row, p, columns, first_head, heads, geo.kv_heads, geo.kvh);
   else load_query(qf, lane16 < columns ? q_row : nullptr, group);
   // (No load is issued for a window past the context: it would bring nothing and still pass through the unit, a microsecond for
@@ -684,8 +685,8 @@ __device__ __forceinline__ void decode_staged(ColumnState& st, lds_u16* __restri
   }
 }
 
-template <bool PROJECTED>
-__global__ void __launch_bounds__(DECODE_THREADS) __attribute__((amdgpu_waves_per_eu(TS_WAVES_PER_SIMD, TS_WAVES_PER_SIMD)))
+template <int WAVES, bool PROJECTED, bool STAGED>
+__global__ void __launch_bounds__(WAVES * TS_WAVE) __attribute__((amdgpu_waves_per_eu(TS_WAVES_PER_SIMD, TS_WAVES_PER_SIMD)))
 decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ query_start_loc, const int* __restrict__ block_table,
               int table_width, int seq_begin, int kv_heads, int gsize, int splits, int block_shift, int window, long q_stride,
               uint16_t* __restrict__ k_pages, uint16_t* __restrict__ v_pages, const uint16_t* __restrict__ q, Projected token_sums,
@@ -695,9 +696,9 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
   lds_u16* const queries = (lds_u16*)decode_lds;         // [16][QUERY_ROW]
   lds_u16* const new_key = queries + 16 * QUERY_ROW;     // [D]
   lds_u16* const new_value = new_key + D;                // [D]
-  float* const tops = decode_lds + (16 * QUERY_ROW + 2 * D) / 2;  // [DECODE_WAVES][16]
-  float* const weights = tops + DECODE_WAVES * 16;                // [DECODE_WAVES][16]
-  float* const sums = weights + DECODE_WAVES * 16;                // [DECODE_WAVES][columns][SUM_ROW], or the rings of a staged walk
+  float* const tops = decode_lds + (16 * QUERY_ROW + 2 * D) / 2;  // [WAVES][16]
+  float* const weights = tops + WAVES * 16;                // [WAVES][16]
+  float* const sums = weights + WAVES * 16;                // [WAVES][columns][SUM_ROW], or the rings of a staged walk
 
   const int lane = threadIdx.x & (TS_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TS_WAVE);
   const int lane16 = lane & 15, group = lane >> 4;
@@ -717,7 +718,7 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
   const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
   const int lo_window = lo & ~(WINDOW_KEYS - 1);
   int w = lo_window + WINDOW_KEYS * (blockIdx.x + splits * wave);
-  const int step = WINDOW_KEYS * DECODE_WAVES * splits;
+  const int step = WINDOW_KEYS * WAVES * splits;
   if (window > 0) first_pages = window_pages(geo, w);
   const uint16_t* q_row = PROJECTED ? nullptr : q + (size_t)token * q_stride + (size_t)(first_head + lane16) * D;
   const float* sum_row = PROJECTED ? token_sums.sums + (size_t)token * (heads + 2 * kv_heads) * D : nullptr;
@@ -729,16 +730,16 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
   }
   ColumnState st;
   init_state(st);
-  if constexpr (DECODE_STAGED) {
+  if constexpr (STAGED) {
     lds_u16* ring = (lds_u16*)sums + wave * Stage::WAVE;
-    decode_staged<PROJECTED>(st, ring, ring, queries, new_key, new_value, geo, first_pages, q_row, token_sums, sum_row, w, step, lo,
+    decode_staged<WAVES, PROJECTED>(st, ring, ring, queries, new_key, new_value, geo, first_pages, q_row, token_sums, sum_row, w, step, lo,
                              ctx, columns, first_head, heads, scale_log2);
   } else {
     QueryFrags qf;
     WindowFrags fa, fb;
     if (PROJECTED) {
       // What a token's heads need is asked for, then the first window; the heads are put together while the window travels.
-      TokenPieces pieces;
+      TokenPieces<WAVES * TS_WAVE> pieces;
       pieces.ask(token_sums, sum_row, p, columns, first_head, heads, kv_heads, kvh);
       auto put = [&]() __attribute__((always_inline)) {
         pieces.put(token_sums, sum_row, columns, first_head, heads, kv_heads, kvh, queries, new_key, new_value);
@@ -779,7 +780,8 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
     const size_t page = (((size_t)(slot >> block_shift) * kv_heads + kvh) << block_shift) * D;
     const int offset = slot & geo.block_mask, at = threadIdx.x;
     if (at < D / 8) *reinterpret_cast<u32x4*>(k_pages + page + (size_t)offset * D + 8 * at) = *(const lds_u32x4*)(new_key + 8 * at);
-    if (at < D) v_pages[page + ((size_t)at << block_shift) + offset] = new_value[at];
+#pragma unroll
+    for (int d = at; d < D; d += WAVES * TS_WAVE) v_pages[page + ((size_t)d << block_shift) + offset] = new_value[d];
   }
   // The wavefronts' sums, each against the largest maximum of its column.
   const float l_total = column_sum(st.l);
@@ -787,7 +789,7 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
   __syncthreads();
   float m_max = -INFINITY;
 #pragma unroll
-  for (int v = 0; v < DECODE_WAVES; ++v) m_max = fmaxf(m_max, tops[v * 16 + lane16]);
+  for (int v = 0; v < WAVES; ++v) m_max = fmaxf(m_max, tops[v * 16 + lane16]);
   const float by = st.m == -INFINITY ? 0.f : exp2f(st.m - m_max);
   if (group == 0) weights[wave * 16 + lane16] = l_total * by;
   if (lane16 < columns) {
@@ -796,12 +798,12 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
       *reinterpret_cast<f32x4*>(sums + (wave * columns + lane16) * SUM_ROW + 16 * n + 4 * group) = st.acc[n] * by;
   }
   __syncthreads();
-  for (int item = threadIdx.x; item < columns * (D / 4); item += DECODE_THREADS) {
+  for (int item = threadIdx.x; item < columns * (D / 4); item += WAVES * TS_WAVE) {
     const int column = item / (D / 4), d = 4 * (item % (D / 4));
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     float den = 0.f;
 #pragma unroll
-    for (int v = 0; v < DECODE_WAVES; ++v) {
+    for (int v = 0; v < WAVES; ++v) {
       acc += *reinterpret_cast<const f32x4*>(sums + (v * columns + column) * SUM_ROW + d);
       den += weights[v * 16 + column];
     }
@@ -814,7 +816,7 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
       if (d == 0) {
         float top = -INFINITY;
 #pragma unroll
-        for (int v = 0; v < DECODE_WAVES; ++v) top = fmaxf(top, tops[v * 16 + column]);
+        for (int v = 0; v < WAVES; ++v) top = fmaxf(top, tops[v * 16 + column]);
         *reinterpret_cast<f32x2*>(partial_ml + at * 2) = f32x2{top, den};
       }
     }
@@ -1988,24 +1990,25 @@ static void prefill_wide_shape(int heads, int kv_heads, int shift, int* per_bloc
 }  // namespace
 
 // Decode attention for the requests seq_begin .. seq_begin + requests - 1 of the step, each of
-// which brings one token, a request's windows of 32 keys divided evenly over `splits` workgroups.  With one, partial_acc and
+// which brings one token, a request's windows of 32 keys divided evenly over `splits` workgroups of `waves` wavefronts (8, 4 or 2; heads
+// of more than 128: 4, for 8 as well, or 2).  With one workgroup a request, partial_acc and
 // partial_ml may be null; otherwise they hold requests * heads * splits entries.
 // The queries are rows of `q`, the new keys and values lie in their pages; or q is null and `sums` are the projection's
 // `sum_splits` partial sums [tokens, (heads + 2 kv_heads) D], `sum_stride` elements apart, which are added up, rotated by the
 // angles of the requests' last positions in cos_table and sin_table [.., D / 2], and stored at `slots` (negative: not stored).
-template <bool PROJECTED>
+template <int WAVES, bool PROJECTED, bool STAGED>
 static int launch_decode(uint16_t* out, float* partial_acc, float* partial_ml, const uint16_t* q, long q_stride, uint16_t* k_pages,
                          uint16_t* v_pages, const int* block_table, int table_width, const int* query_start_loc,
                          const int* context_lens, int seq_begin, int requests, int heads, int kv_heads, int shift, ScoreRule rule,
                          int window, int splits, const Projected& token_sums, hipStream_t stream) {
   const int gsize = heads / kv_heads, head_tiles = (gsize + 15) / 16, columns = gsize < 16 ? gsize : 16;
-  const size_t joined = (size_t)DECODE_WAVES * columns * SUM_ROW * 4, rings = DECODE_STAGED ? (size_t)DECODE_WAVES * Stage::WAVE * 2 : 0;
-  const size_t lds = (16 * QUERY_ROW + 2 * D) * 2 + DECODE_WAVES * 32 * 4 + (joined > rings ? joined : rings);
-  static const bool raised = hipFuncSetAttribute((const void*)decode_kernel<PROJECTED>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
+  const size_t joined = (size_t)WAVES * columns * SUM_ROW * 4, rings = STAGED ? (size_t)WAVES * Stage::WAVE * 2 : 0;
+  const size_t lds = (16 * QUERY_ROW + 2 * D) * 2 + WAVES * 32 * 4 + (joined > rings ? joined : rings);
+  static const bool raised = hipFuncSetAttribute((const void*)decode_kernel<WAVES, PROJECTED, STAGED>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
   if (!raised) return TS_ERR_LAUNCH;
-  hipLaunchKernelGGL(decode_kernel<PROJECTED>, dim3(splits, kv_heads * head_tiles, requests), dim3(DECODE_THREADS), lds, stream,
-                     context_lens, query_start_loc, block_table, table_width, seq_begin, kv_heads, gsize, splits, shift, window, q_stride,
-                     k_pages, v_pages, q, token_sums, rule, out, partial_acc, partial_ml);
+  hipLaunchKernelGGL((decode_kernel<WAVES, PROJECTED, STAGED>), dim3(splits, kv_heads * head_tiles, requests), dim3(WAVES * TS_WAVE), lds,
+                     stream, context_lens, query_start_loc, block_table, table_width, seq_begin, kv_heads, gsize, splits, shift, window,
+                     q_stride, k_pages, v_pages, q, token_sums, rule, out, partial_acc, partial_ml);
   if (splits == 1) return ts_launch_status();
   if (hipGetLastError() != hipSuccess) return TS_ERR_LAUNCH;
   hipLaunchKernelGGL(decode_reduce_kernel, dim3(requests, heads), dim3(REDUCE_THREADS), 0, stream, out, partial_acc, partial_ml,
@@ -2017,7 +2020,7 @@ extern "C" int TS_SYM(ts_attention_decode_d)(
     void* out, void* partial_acc, void* partial_ml, const void* q, long q_stride, void* k_pages,
     void* v_pages, const int* block_table, int table_width, const int* query_start_loc,
     const int* context_lens, int seq_begin, int requests, int heads, int kv_heads, int block_size,
-    float scale, float softcap, int window, int splits, const float* sums, long sum_stride, int sum_splits, const float* cos_table,
+    float scale, float softcap, int window, int splits, int waves, const float* sums, long sum_stride, int sum_splits, const float* cos_table,
     const float* sin_table, const int* slots, hipStream_t stream) {
   if (requests == 0) return TS_OK;
   if (!out || !k_pages || !v_pages || !block_table || !query_start_loc || !context_lens || (q == nullptr) == (sums == nullptr))
@@ -2028,12 +2031,15 @@ extern "C" int TS_SYM(ts_attention_decode_d)(
   if (heads < 1 || kv_heads < 1 || heads % kv_heads != 0) return TS_ERR_SHAPE;
   if (block_size < 8 || (block_size & (block_size - 1))) return TS_ERR_SHAPE;
   if (splits < 1 || splits > DECODE_MAX_SPLITS || requests > 65535) return TS_ERR_SHAPE;
+  if (waves != 8 && waves != 4 && waves != 2) return TS_ERR_SHAPE;
   int shift = 0;
   while ((1 << shift) < block_size) ++shift;
   const int head_tiles = (heads / kv_heads + 15) / 16;
   if (kv_heads * head_tiles > 65535) return TS_ERR_SHAPE;
   const Projected token_sums = {sums, (size_t)sum_stride, sum_splits, cos_table, sin_table, slots};
-  auto launch = sums ? launch_decode<true> : launch_decode<false>;
+  auto launch = sums ? launch_decode<DECODE_WAVES, true, DECODE_STAGED> : launch_decode<DECODE_WAVES, false, DECODE_STAGED>;
+  if (waves == 4 && DECODE_WAVES > 4) launch = sums ? launch_decode<4, true, DECODE_STAGED> : launch_decode<4, false, DECODE_STAGED>;
+  if (waves == 2) launch = sums ? launch_decode<2, true, DECODE_STAGED> : launch_decode<2, false, DECODE_STAGED>;
   return launch((uint16_t*)out, (float*)partial_acc, (float*)partial_ml, (const uint16_t*)q, q_stride, (uint16_t*)k_pages,
                 (uint16_t*)v_pages, block_table, table_width, query_start_loc, context_lens, seq_begin, requests, heads, kv_heads,
                 shift, score_rule(scale, softcap), window, splits, token_sums, stream);

@@ -164,7 +164,7 @@ def _attention_signatures(head_dim: int) -> dict[str, list]:
     return {
         f"ts_attention_decode_d{head_dim}": [c_void_p, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p,
                                              c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
-                                             c_int, c_float, c_float, c_int, c_int, c_void_p, c_long, c_int, c_void_p,
+                                             c_int, c_float, c_float, c_int, c_int, c_int, c_void_p, c_long, c_int, c_void_p,
                                              c_void_p, c_void_p, c_void_p],
         f"ts_attention_prefill_d{head_dim}": [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int,
                                               c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float,
@@ -1873,7 +1873,8 @@ class Ops:
             _need(max_position < cos.shape[0], f"position {max_position} is beyond the rotary tables ({cos.shape[0]})")
             new = (_ptr(q), stride, sum_splits, _ptr(cos), _ptr(sin), _ptr(slots))
         span = max_context if not window else min(max_context, window + 31)
-        splits = self._decode_splits(requests * kv_heads * -(-(heads // kv_heads) // 16), span)
+        pairs = requests * kv_heads * -(-(heads // kv_heads) // 16)
+        splits = self._decode_splits(pairs, span)
         partial_acc = partial_ml = None
         if splits > 1:
             partial_acc = torch.empty((requests * heads * splits, head_dim), dtype=torch.float32, device=out.device)
@@ -1883,7 +1884,7 @@ class Ops:
         _check(fn(_ptr(out), _ptr(partial_acc), _ptr(partial_ml), None if projected else _ptr(q), q_stride, _ptr(k_pages), _ptr(v_pages),
                   _ptr(block_table), block_table.shape[1], _ptr(query_start_loc), _ptr(context_lens), seq_begin,
                   requests, heads, kv_heads, block_size, float(scale), float(softcap), int(window or 0), splits,
-                  *new, self.stream()), "ts_attention_decode")
+                  self._decode_waves(pairs * splits, span, head_dim), *new, self.stream()), "ts_attention_decode")
 
     def _decode_splits(self, pairs: int, span: int) -> int:
         """Over how many workgroups of the decode attention a request's keys are divided: ``pairs`` of request and KV head, at
@@ -1898,6 +1899,18 @@ class Ops:
         if span <= self.decode_whole_keys:
             return 1
         return max(1, min(self.compute_units // pairs, -(-span // self.decode_min_keys), 256))
+
+    def _decode_waves(self, workgroups: int, span: int, head_dim: int) -> int:
+        """Wavefronts of a workgroup of the decode attention: eight (heads of more than 128: four) hold a compute unit alone.  More
+        workgroups than units over short spans take turns that are mostly starts: with half or a quarter of the wavefronts two or four
+        share a unit.  Over longer spans a long request among short ones wants them all.  Microseconds a layer, eight / four / two,
+        heads of 128: 64 requests of 100 keys with 32 KV heads 55.5 / 34.1 / 30.8 (a wavefront per stretch of keys, as it was: 33.9),
+        33 of 300 60.4 / 43.7 / 39.6 (45.0), 128 of 100 with 8 16.7 / 12.3 / 11.8, 64 of 1,000 with 8 50.4 / 46.4 / 48.4 (59.5), 100 of
+        128 to 1,535 with 8 66.5 / 69.6 / 71.8; of 80, 64 of 2,048 with 5 50.1 / 44.5 / 52.9 (46.9); of 256, four / two, 65 of 100 with
+        4 23.4 / 17.2 (20.8), of 1,000 71.9 / 65.9 (70.8)."""
+        if workgroups <= self.compute_units or span > (1024 if head_dim == 128 else 2048):
+            return 8
+        return 2 if head_dim > 128 or (workgroups >= 4 * self.compute_units and span <= 512) else 4
 
     def prefill_block_rows(self, head_dim: int, heads: int, kv_heads: int) -> int:
         """Consecutive rows of one request that a wavefront of the prefill attention kernel
