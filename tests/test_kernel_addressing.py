@@ -5,9 +5,9 @@ the kernels whose launches the host plans most freely is restated here in Python
 over shapes, plans and cache states on the CPU: the tiled product (``csrc/gemm_tiled.hip``:
 what a thread fetches, where it stages it in LDS, which fragments a wavefront reads, where the
 sums go), the product of steps of many rows (``csrc/gemm_wide.hip``: the same, with its
-numbering of workgroups over weight tiles, ranges of K and tiles of activation rows), the decode attention (``csrc/attention_mfma.hip``, ``decode_kernel``: which page and
-key every lane reads for every split, with pages given back below a window and table entries
-that are padding) and the 32-row prefill attention (``prefill_wide_kernel``: the block-table
+numbering of workgroups over weight tiles, ranges of K and tiles of activation rows), the decode attention (``csrc/attention_mfma.hip``, ``decode_kernel``: which windows
+a wavefront walks, which page every lane reads, and, for staged windows, which bytes of it, where in LDS they are put and what is read there, with
+pages given back below a window and table entries that are padding) and the 32-row prefill attention (``prefill_wide_kernel``: the block-table
 look-ups of its pipeline, five windows ahead, self-fed and fed, whole blocks and shares of a
 block, and the slots the shares' partial sums go to).  The models follow the kernels line by
 line and must be changed with them.
@@ -108,61 +108,117 @@ def test_tiled_product_stays_inside_its_buffers(m):
 WINDOW_KEYS = 32  # attention_mfma.hip
 
 
-def check_decode(ctx, window, shift, table, splits, keys_per_split, device_context=None):
-    """Every page a lane of ``decode_kernel`` selects is a live one, and the splits cover the
-    keys lo..ctx-1 exactly."""
-    if device_context is not None:  # a recorded launch sizes the splits on the device
-        span = device_context
-        if window and span > window + WINDOW_KEYS - 1:
-            span = window + WINDOW_KEYS - 1
-        per = (span + WINDOW_KEYS - 1 + splits - 1) // splits
-        keys_per_split = -(-per // WINDOW_KEYS) * WINDOW_KEYS
+def decode_places(table, kv_heads, shift, dim, w, lo, p):
+    """``Stage::place`` and ``Stage::fetch``: for every 16-byte piece of the window's keys and values where it is read (page, byte of the
+    page's KV head) and where in the wavefront's ring it is put."""
+    pages = [table[min((w >> shift) + i, len(table) - 1)] for i in range(4)]
+    first_live, last_live = (max(w, lo) - w) >> shift, (min(w + 31, p) - w) >> shift
+    page_of = [pages[min(max((8 * i) >> shift, first_live), last_live)] for i in range(4)]
+    size, inside, pieces, loads = 2 * (dim << shift), w & ((1 << shift) - 1) & ~31, dim // 8, dim // 16
+    chunk_shift, rows_mask = min(shift - 3, 2), (1 << min(shift, 5)) - 1
+    turn = lambda r: r if pieces >= 16 else r // (16 // pieces)
+    keys, values = {}, {}
+    for i in range(4):
+        assert page_of[i] >= 0, (w, lo, p, shift)
+        for j in range(i * (loads // 4), (i + 1) * (loads // 4)):
+            for lane in range(64):
+                at = 64 * j + lane
+                r, piece = at // pieces, (at % pieces + 4 * pieces - turn(at // pieces)) % pieces
+                byte = (r & rows_mask) * 2 * dim + 16 * piece + inside * 2 * dim
+                assert 0 <= byte and byte + 16 <= size
+                keys[512 * j + 8 * lane] = (page_of[i], byte)
+                byte = ((lane >> chunk_shift) << (shift + 1)) + 16 * (lane & ((1 << chunk_shift) - 1))
+                byte += ((((64 * j) >> chunk_shift) % dim) << (shift + 1)) + inside * 2
+                assert 0 <= byte and byte + 16 <= size
+                values[512 * j + 8 * lane] = (page_of[i], byte)
+    return keys, values, turn, chunk_shift
+
+
+def check_decode_stage(table, kv_heads, shift, dim, w, lo, p):
+    """What the lanes of a staged window read from the ring is their keys and values (``Stage::read_keys``, ``read_values``)."""
+    keys, values, turn, chunk_shift = decode_places(table, kv_heads, shift, dim, w, lo, p)
+    assert len(keys) == len(values) == 4 * dim and max(keys) + 8 == 32 * dim  # the slot's keys, then its values, each filled once
+    page_at = lambda key: (table[key >> shift], key & ((1 << shift) - 1))
+    pieces = dim // 8
+    for lane16 in range(16):
+        for group in range(4):
+            for t in range(2):
+                r = 8 * (lane16 >> 2) + 4 * t + (lane16 & 3)
+                for j in range(dim // 32):
+                    got = keys[r * dim + 8 * ((4 * j + group + turn(r)) % pieces)]
+                    if lo <= w + r <= p:
+                        page, row = page_at(w + r)
+                        assert got == (page, row * 2 * dim + 2 * (32 * j + 8 * group))
+            chunk = ((group >> chunk_shift) * dim + lane16) << chunk_shift | (group & ((1 << chunk_shift) - 1))
+            for n in range(dim // 16):
+                got = values[8 * (chunk + ((16 * n) << chunk_shift))]
+                if w + 8 * group + 7 >= lo and w + 8 * group <= p:
+                    page, row = page_at(max(w + 8 * group, 0))
+                    assert got == (page, ((16 * n + lane16) << (shift + 1)) + 2 * row)
+
+
+def check_decode(ctx, window, shift, table, splits, waves, staged):
+    """Every page a lane of ``decode_kernel`` reads is a live one, no wavefront walks a window without a live key, and the wavefronts of a
+    request's workgroups cover the keys lo..ctx-1 exactly."""
     p = ctx - 1
     lo = max(0, p - window + 1) if window else 0
     covered = set()
-    for split in range(splits):
-        begin = (lo & ~31) + split * keys_per_split
-        end = min(begin + keys_per_split, ctx)
-        for w in range(begin, end, WINDOW_KEYS):
-            first = w >> shift
-            pages = [table[min(first + i, len(table) - 1)] for i in range(4)]
-            for lane16 in range(16):
-                for t in range(2):
-                    key = w + 8 * (lane16 >> 2) + 4 * t + (lane16 & 3)
-                    live = min(max(key, max(w, lo)), min(w + 31, p))
-                    assert pages[(live - w) >> shift] >= 0, (ctx, window, 1 << shift, split, w, key)
-                    if lo <= key <= p:
-                        assert key not in covered
-                        covered.add(key)
-            for group in range(4):
-                chunk = w + 8 * group
-                live = chunk + 7 >= lo and chunk <= p
-                key = chunk if live else (min(max(chunk, max(w, lo)), min(w + 31, p)) & ~7)
-                assert pages[(key - w) >> shift] >= 0, (ctx, window, 1 << shift, split, w, chunk)
-    assert covered == set(range(lo, ctx)), (ctx, window, splits, keys_per_split)
+    for x in range(splits):
+        for wave in range(waves):
+            first = 32 * (x + splits * wave)
+            # The first window's pages are looked up before the context is known (with a window: again).
+            assert all(0 <= min((first >> shift) + i, len(table) - 1) < len(table) for i in range(4))
+            w, step = (lo & ~31) + first, 32 * waves * splits
+            while w < ctx:
+                assert w + 31 >= lo and w not in covered
+                covered.add(w)
+                pages = [table[min((w >> shift) + i, len(table) - 1)] for i in range(4)]
+                if not staged:  # operands straight from the pages
+                    for lane16 in range(16):
+                        for t in range(2):
+                            key = w + 8 * (lane16 >> 2) + 4 * t + (lane16 & 3)
+                            live = min(max(key, max(w, lo)), min(w + 31, p))
+                            assert pages[(live - w) >> shift] >= 0, (ctx, window, 1 << shift, x, w, key)
+                    for group in range(4):
+                        chunk = w + 8 * group
+                        live = chunk + 7 >= lo and chunk <= p
+                        key = chunk if live else (min(max(chunk, max(w, lo)), min(w + 31, p)) & ~7)
+                        assert pages[(key - w) >> shift] >= 0, (ctx, window, 1 << shift, x, w, chunk)
+                w += step
+    assert covered == set(range(lo & ~31, ctx, 32)), (ctx, window, splits, waves)
+
+
+def decode_request(rng):
+    """(context, window, page shift, block table): pages wholly below the window given back, entries past the context padding."""
+    shift = rng.choice([3, 4, 5, 6, 7])
+    page = 1 << shift
+    ctx = rng.choice([1, 2, 31, 32, 33, 63, 64, 65, 100, 257, 600, 1000, rng.randint(1, 5000)])
+    window = rng.choice([0, 0, 1, 12, 16, 33, 70, 300, 1025])
+    needed = -(-ctx // page)
+    table = [rng.randint(0, 500) for _ in range(needed)] + [-1] * rng.choice([0, 1, 5])
+    if window:
+        for i in range(max(0, ctx - window) // page):
+            table[i] = -1
+    return ctx, window, shift, table
 
 
 def test_decode_attention_reads_live_pages_only():
     rng = random.Random(2)
-    for _ in range(3000):
-        shift = rng.choice([3, 4, 5, 6])
-        page = 1 << shift
-        ctx = rng.choice([1, 2, 31, 32, 33, 63, 64, 65, 100, 257, 600, 1000, rng.randint(1, 5000)])
-        window = rng.choice([0, 0, 1, 12, 16, 33, 70, 300, 1025])
-        needed = -(-ctx // page)
-        width = needed + rng.choice([0, 1, 5])
-        table = [rng.randint(0, 500) for _ in range(needed)] + [-1] * (width - needed)
-        if window:  # pages wholly below the window's lower bound were given back
-            for i in range(max(0, ctx - window) // page):
-                table[i] = -1
-        bound = rng.choice([ctx, min(ctx + 50, width * page), width * page])  # what the host knows of the longest context
-        span = bound if not window else min(bound, window + 31)
-        for splits_wanted in (1, 2, rng.randint(1, 64), 256):
-            splits = max(1, min(splits_wanted, -(-span // 32)))
-            keys_per_split = -(-(-(-(span + 31) // splits)) // 32) * 32
-            splits = -(-(span + 31) // keys_per_split)
-            check_decode(ctx, window, shift, table, splits, keys_per_split)
-            check_decode(ctx, window, shift, table, splits, keys_per_split, device_context=ctx)
+    for _ in range(1500):
+        ctx, window, shift, table = decode_request(rng)
+        for splits in (1, rng.choice([2, 4, 256]), rng.randint(3, 64)):
+            check_decode(ctx, window, shift, table, splits, rng.choice([2, 4, 8]), staged=rng.random() < 0.5)
+
+
+@pytest.mark.parametrize("dim", [64, 128, 192, 256])
+def test_staged_decode_windows_hold_their_keys_and_values(dim):
+    rng = random.Random(dim)
+    for _ in range(15):
+        ctx, window, shift, table = decode_request(rng)
+        p = ctx - 1
+        lo = max(0, p - window + 1) if window else 0
+        for w in sorted({lo & ~31, (p & ~31), rng.randrange(lo & ~31, ctx, 32)}):
+            check_decode_stage(table, 1, shift, dim, w, lo, p)
 
 
 def check_prefill_wide(pos0, cols, window, shift, table, fed, share=None):
