@@ -19,6 +19,7 @@ class Launches:
     """The operations an attention layer asks for, by name."""
 
     mfma_attention_supported = staticmethod(Ops.mfma_attention_supported)
+    decode_shared_keys = Ops.decode_shared_keys
 
     def __init__(self):
         self.names = []
@@ -105,3 +106,42 @@ def test_more_workgroups_than_units_over_short_spans_share_units(workgroups, spa
     """A workgroup of eight wavefronts has a unit to itself: 64 requests of 100 keys with 32 KV heads took eight turns of starts, 55 us
     where a wavefront per stretch of keys had taken 34."""
     assert Ops._decode_waves(SimpleNamespace(compute_units=256), workgroups, span, head_dim) == waves
+
+
+def shares(lengths, rows, pairs, head_dim=128, window=None):
+    ops = SimpleNamespace(compute_units=256, decode_shared_keys=Ops.decode_shared_keys)
+    return Ops.decode_shares(ops, lengths, rows, pairs, head_dim, window)
+
+
+@pytest.mark.parametrize("lengths,rows,pairs,parts", [
+    ([16384] + [600] * 40, 64, 4, 4),                        # a long request ends last, alone
+    ([16384] + [600] * 16, 32, 8, 4),
+    ([8192] * 65, 128, 4, 4), ([8192] * 33, 64, 8, 4),       # a few workgroups more than a round
+    ([8192] * 64, 64, 4, 1), ([8192] * 128, 128, 4, 1), ([8192] * 33, 64, 4, 1),
+    ([2048] * 65, 128, 4, 1), ([16384] + [600] * 16, 32, 4, 1), ([16384], 1, 4, 1), ([], 64, 4, 1),
+])
+def test_long_requests_among_short_ones_are_divided(lengths, rows, pairs, parts):
+    """From half the compute units on, a request was one workgroup's whatever the others brought: 151 us a layer for 16,384 keys among 40
+    short requests where 131 had been enough."""
+    assert shares(lengths, rows, pairs) == parts
+    assert shares(lengths, rows, pairs, window=1024) == 1
+
+
+def test_a_recorded_step_is_for_lengths_that_divide_alike():
+    """Uneven lengths are another recorded shape; the layers find their parts in its context."""
+    from turboserve_amd.engine.decode_graph import DecodeGraphs
+
+    geometry, windowed = (4, 128, None), (4, 128, 1024)
+    ops = SimpleNamespace(compute_units=256, decode_shared_keys=Ops.decode_shared_keys)
+    ops.decode_shares = lambda *of: Ops.decode_shares(ops, *of)
+    model = SimpleNamespace(runtime=SimpleNamespace(device=torch.device("cpu"), ops=ops, decode_geometries={geometry, windowed}))
+    graphs = DecodeGraphs(model, [], page_size=16, num_groups=1, pad_state_slot=0)
+    entries = lambda lengths: [SimpleNamespace(start=n - 1, tables=[[0] * -(-n // 16)]) for n in lengths]
+    uneven, even = graphs._key(entries([16384] + [600] * 40)), graphs._key(entries([16384] * 41))
+    assert uneven[:2] == even[:2] and even[2] == () and dict(uneven[2]) == {geometry: 4}
+    assert graphs._key(entries([600] * 41))[2] == ()
+    layer = SimpleNamespace(decode_geometry=geometry, runtime=model.runtime)
+    step = SimpleNamespace(recorded=True, max_decode_context_len=16384, decode_shares=dict(uneven[2]))
+    assert GroupedQueryAttention._decode_shares(layer, step) == 4
+    step.decode_shares = {}
+    assert GroupedQueryAttention._decode_shares(layer, step) == 1

@@ -256,6 +256,38 @@ def test_recorded_steps_survive_the_growth_of_the_rotary_tables(tmp_path):
         assert torch.equal(results[False][step], results[True][step]), f"step {step}: recorded differs from eager"
 
 
+def test_recorded_steps_of_uneven_requests_divide_their_keys(tmp_path, monkeypatch):
+    """A request of some 2,100 tokens among 40 short ones of a model with four KV heads: its keys are divided over several workgroups, in
+    a recorded step as in an eager one, and the logits are those of steps that leave every request whole, up to the order of
+    the sums."""
+    from turboserve_amd.engine.replay import TraceReplayer
+    from turboserve_amd.kernels.ops import Ops
+
+    config = {**tiny.CONFIG_A, "num_key_value_heads": 4, "max_position_embeddings": 4096}
+    folder = tiny.make_model_dir(tmp_path / "m", config, 12, torch.bfloat16, std=tiny.std_for(torch.bfloat16, 64))
+    requests = {"long": tiny.random_tokens(256, 2104, 1), **{f"r{i}": tiny.random_tokens(256, 5 + i, 2 + i) for i in range(40)}}
+    asked = []
+    whole = Ops.attention_decode
+    monkeypatch.setattr(Ops, "attention_decode", lambda self, *a, shares=1, **more: (asked.append(shares), whole(self, *a, shares=shares, **more))[1])
+    results = {}
+    for kind in ("eager", "recorded", "whole"):
+        monkeypatch.setattr(Ops, "decode_shares", lambda self, lengths, *more: 3 if max(lengths) > 2048 and kind != "whole" else 1)
+        replayer = TraceReplayer(folder, dtype="bfloat16", max_tokens=64 * 40 + 2304, page_size=16, max_live=48)
+        if kind != "recorded":
+            replayer.runner.graphs = None
+        asked.clear()
+        steps = [{"entries": [{"id": rid, "tokens": tokens[:-3], "want": []}], "end": []} for rid, tokens in requests.items()]
+        for back in (3, 2, 1):
+            steps.append({"entries": [{"id": rid, "tokens": [tokens[-back]], "want": [0]} for rid, tokens in requests.items()], "end": []})
+        for index, record in enumerate(steps):
+            record["step"] = index
+        results[kind] = torch.stack([replayer.run_step(record).float().cpu() for record in steps][-3:])
+        assert set(asked) == {1 if kind == "whole" else 3}
+    assert torch.equal(results["eager"], results["recorded"])
+    bound = 2e-2 * float(results["whole"].abs().max())
+    assert float((results["eager"] - results["whole"]).abs().max()) <= bound
+
+
 _TIMED_WIDTHS = itertools.count()
 
 

@@ -345,6 +345,9 @@ class StepContext:
     #: A recorded step: replayed with other data than it was recorded with, so a part may use
     #: nothing about the step but its shape, the fields above and what ``derive`` refuses there.
     recorded: bool = False
+    #: In a recorded step: ``Ops.decode_shares`` by the attention geometry it was asked for (``Runtime.decode_geometries``), 1 where
+    #: it is not named; the steps that replay it have the same.
+    decode_shares: dict = field(default_factory=dict)
     #: The fields the model's parts asked for (``Part.step_fields``), by name: int32 device views.
     extras: dict = field(default_factory=dict)
     #: Device tensors one layer makes in this step for a later layer of the same step (by a key the

@@ -9,7 +9,8 @@ shape's layout), copies it to the device and launches the graph.
 Shapes are bucketed so that few graphs serve every batch: the number of requests is rounded up
 to a power of two (the extra rows are padding: position 0, context 1, no cache write, results
 dropped) and each cache group's block-table width to a power of two.  The kernels read the
-true context lengths from the device, so one graph serves every length up to its width.  What
+true context lengths from the device, so one graph serves every length up to its width; only how the decode
+attention divides the requests' keys (``Ops.decode_shares``: long requests among short ones) is part of the shape too.  What
 the engine's own parts launch in such a step are this engine's kernels only (no BLAS call, no
 memset node): products of up to 128 rows are the weight-streaming kernels, or, where K is no
 multiple of 8, the plain fused-multiply-add kernel.  A part from elsewhere may record torch
@@ -62,6 +63,8 @@ class DecodeGraphs:
         self.limits = limits
         #: Fields the model's parts add to the packed buffer (``Part.step_fields``).
         self.extra_fields = tuple(extra_fields)
+        #: Attention geometries whose launches the requests' lengths have a say in.
+        self.geometries = sorted(model.runtime.decode_geometries, key=repr)
         self.device = model.runtime.device
         self._graphs: dict[tuple, _Graph] = {}
         self._pool = None
@@ -77,12 +80,21 @@ class DecodeGraphs:
         widths = tuple(
             max(4, next_power_of_two(max(len(e.tables[g]) for e in entries))) for g in range(self.num_groups)
         )
-        return batch, widths
+        return batch, widths, self._shares(entries, batch)
+
+    def _shares(self, entries: Sequence[StepEntry], batch: int) -> tuple:
+        """What the requests' lengths make of the decode attention's launches, by geometry (where it is not 1)."""
+        ops = self.model.runtime.ops
+        lengths = [e.start + 1 for e in entries]
+        if max(lengths) <= ops.decode_shared_keys:
+            return ()
+        shares = ((geometry, ops.decode_shares(lengths, batch, *geometry)) for geometry in self.geometries)
+        return tuple((geometry, parts) for geometry, parts in shares if parts > 1)
 
     # -- buffers ---------------------------------------------------------------------------------
 
     def _build(self, key: tuple) -> _Graph:
-        batch, widths = key
+        batch, widths, shares = key
         shape = _Graph(batch, widths, self.extra_fields)
         total = shape.layout.total
         shape.device_ints = torch.zeros(total, dtype=torch.int32, device=self.device)
@@ -103,6 +115,7 @@ class DecodeGraphs:
             max_prefill_context_len=0,
             max_decode_context_len=max_context,
             recorded=True,
+            decode_shares=dict(shares),
         )
         # Harmless contents for the eager warm-up and the recording: every row is padding.
         shape.device_ints.copy_(self._fill(shape, []))

@@ -7,6 +7,7 @@ the library cannot be built or loaded, or a tensor is not on a GPU, the op raise
 from __future__ import annotations
 
 import ctypes
+from collections.abc import Sequence
 from ctypes import c_float, c_int, c_long, c_void_p
 from dataclasses import dataclass
 
@@ -1833,6 +1834,7 @@ class Ops:
         max_context_dev: torch.Tensor | None = None,
         softcap: float = 0.0,
         projected: tuple | None = None,
+        shares: int = 1,
     ) -> None:
         """Matrix-core attention for the single-token requests ``seq_begin .. seq_begin +
         requests - 1`` of the step; writes their rows of ``out [T, heads * D]``.  ``max_context``
@@ -1842,7 +1844,10 @@ class Ops:
 
         ``projected = (cos, sin, slots, max_position)``: ``q`` is the fused projection's partial sums ``[S, T, (heads + 2
         kv_heads) D]`` (32-bit); the launch adds them up, rotates queries and keys, stores the new keys and values at
-        ``slots`` and attends, in place of :meth:`rope_store` before it (the same bits in the pages)."""
+        ``slots`` and attends, in place of :meth:`rope_store` before it (the same bits in the pages).
+
+        ``shares`` (:meth:`decode_shares`): what the requests' own lengths, which ``max_context`` does not tell, make of a
+        request's keys where requests and KV heads alone give every compute unit a workgroup."""
         _gpu(out, q, k_pages, v_pages, block_table, query_start_loc, context_lens, max_context_dev)
         _i32(max_context_dev, "max_context_dev")
         _i32(block_table, "block_table")
@@ -1875,6 +1880,8 @@ class Ops:
         span = max_context if not window else min(max_context, window + 31)
         pairs = requests * kv_heads * -(-(heads // kv_heads) // 16)
         splits = self._decode_splits(pairs, span)
+        if splits == 1 and span > self.decode_shared_keys and 2 * pairs > self.compute_units:
+            splits = min(max(1, shares), 256)
         partial_acc = partial_ml = None
         if splits > 1:
             partial_acc = torch.empty((requests * heads * splits, head_dim), dtype=torch.float32, device=out.device)
@@ -1899,6 +1906,37 @@ class Ops:
         if span <= self.decode_whole_keys:
             return 1
         return max(1, min(self.compute_units // pairs, -(-span // self.decode_min_keys), 256))
+
+    #: Spans up to this are not divided where requests and KV heads are more than half the compute units.
+    decode_shared_keys = 2048
+
+    def decode_shares(self, lengths: Sequence[int], rows: int, pairs: int, head_dim: int, window: int | None = None) -> int:
+        """Into how many workgroups (1, 2 or 4) the decode attention divides the keys of requests that see ``lengths`` of them, in a launch
+        of ``rows`` requests (some may be padding) with ``pairs`` workgroups each, where these alone are more than half the compute
+        units: more than one where a long request would end last and alone, or where the long requests just miss a whole round of
+        workgroups.  By what a workgroup takes alone (55 bytes a nanosecond) and among many (6.2 TB/s shared), 4.7 us to start it
+        and 5 us for the launch that combines, where that saves 4% (us a layer, whole / in the parts chosen / before workgroups had a
+        unit to themselves; heads of 128): 16,384 keys among 40 requests of 200 to 1,000, 4 KV heads, 151 / 50 / 131, 8 heads with
+        16 others 154 / 50 / 129; 65 of 8,192 235 / 202 / 212, 80 255 / 238 / 241, 33 with 8 heads 238 / 203 / 210.  64 and 128 of 8,192
+        stay whole (175 and 337; in four 177 and 368)."""
+        if window:
+            lengths = [min(n, window + 31) for n in lengths]
+        longest = max(lengths, default=0)
+        if longest <= self.decode_shared_keys or 2 * rows * pairs <= self.compute_units:
+            return 1
+        key, start, units = 4 * head_dim, 4.7, self.compute_units
+        read, longs = sum(lengths) * pairs * key / 6.2e6, pairs * sum(1 for n in lengths if 2 * n > longest)
+        best = None
+        for parts in (1, 2, 4):
+            alone = longest / parts * key / 55e3 + start
+            last = longs * parts % units / units  # how full the long requests' last round of workgroups is
+            tail = (1 - last) * alone if longs * parts > units and 0 < last <= 0.5 else 0.0
+            cost = max(read + len(lengths) * pairs * parts * start / units + tail, alone) + (5.0 if parts > 1 else 0.0)
+            if best is None or cost < 0.96 * whole and cost < best[0]:
+                best = cost, parts
+            if parts == 1:
+                whole = cost
+        return best[1]
 
     def _decode_waves(self, workgroups: int, span: int, head_dim: int) -> int:
         """Wavefronts of a workgroup of the decode attention: eight (heads of more than 128: four) hold a compute unit alone.  More

@@ -172,6 +172,10 @@ class GroupedQueryAttention(Mixer):
         self.kv_size = self.projected_kv_heads * self.head_dim
         self.v_size = 0 if self.values_are_keys else self.projected_kv_heads * self.value_dim
         self.out_size = self.num_heads * self.value_dim
+        #: See ``Runtime.decode_geometries``.
+        self.decode_geometry = (self.num_kv_heads * -(-(self.num_heads // self.num_kv_heads) // 16), self.head_dim, self.window)
+        if runtime.dtype == torch.bfloat16 and self._plain_rule():
+            runtime.decode_geometries.add(self.decode_geometry)
         self.conv_weight: torch.Tensor | None = None
         self.q_gain: torch.Tensor | None = None
         self.k_gain: torch.Tensor | None = None
@@ -368,8 +372,17 @@ class GroupedQueryAttention(Mixer):
         ops.attention_decode(
             out, qkv, 0, cache.k, cache.v, table, ctx.query_start_loc, ctx.context_lens, 0, ctx.num_decode_seqs, self.num_heads,
             self.scale, self.window, min(ctx.max_decode_context_len, table.shape[1] * cache.block_size), ctx.max_decode_context_dev,
-            softcap=self.softcap, projected=(*tables, ctx.slot_mapping[cache.group], ctx.max_context_len - 1))
+            softcap=self.softcap, projected=(*tables, ctx.slot_mapping[cache.group], ctx.max_context_len - 1), shares=self._decode_shares(ctx))
         return out
+
+    def _decode_shares(self, ctx) -> int:
+        """Into how many workgroups the decode attention divides the requests' keys (``Ops.decode_shares``)."""
+        if ctx.max_decode_context_len <= self.runtime.ops.decode_shared_keys:
+            return 1
+        if ctx.recorded:
+            return ctx.decode_shares.get(self.decode_geometry, 1)
+        return ctx.derive(("decode_shares", self.decode_geometry), lambda step: self.runtime.ops.decode_shares(
+            step.context_lens_host[step.num_prefill_seqs:], step.num_decode_seqs, *self.decode_geometry))
 
     def attend(self, qkv: torch.Tensor, q_stride: int, ctx, cache: PagedKVView, *, scale: float = 1.0,
                out: tuple | None = None) -> torch.Tensor:
@@ -407,7 +420,7 @@ class GroupedQueryAttention(Mixer):
                     out, qkv, q_stride, cache.k, cache.v, table, ctx.query_start_loc, ctx.context_lens,
                     ctx.num_prefill_seqs, ctx.num_decode_seqs, self.num_heads, self.scale, self.window,
                     min(ctx.max_decode_context_len, table.shape[1] * cache.block_size),
-                    ctx.max_decode_context_dev, softcap=self.softcap,
+                    ctx.max_decode_context_dev, softcap=self.softcap, shares=self._decode_shares(ctx),
                 )
             return out
         if ops.tiled_attention_supported(qkv.dtype, self.head_dim, self.value_dim, cache.block_size, q_stride):

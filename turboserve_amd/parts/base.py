@@ -147,6 +147,8 @@ class Runtime:
     dtype: torch.dtype
     ops: Any  # turboserve_amd.kernels.ops.Ops
     shared: dict = field(default_factory=dict)
+    #: ``(workgroups a request, head size, window)`` of the layers that run the matrix-core decode attention.
+    decode_geometries: set = field(default_factory=set)
 
 
 @dataclass
