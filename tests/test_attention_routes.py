@@ -145,3 +145,14 @@ def test_a_recorded_step_is_for_lengths_that_divide_alike():
     assert GroupedQueryAttention._decode_shares(layer, step) == 4
     step.decode_shares = {}
     assert GroupedQueryAttention._decode_shares(layer, step) == 1
+
+
+@pytest.mark.parametrize("pairs,span,head_dim,shares,parts", [
+    (4, 512, 128, 1, 1), (4, 513, 128, 1, 5), (4, 256, 256, 1, 1), (4, 300, 256, 1, 5), (1, 500, 256, 1, 5), (132, 300, 256, 1, 1),
+    (64, 8192, 128, 4, 4), (128, 8192, 128, 4, 2), (132, 8192, 128, 4, 4), (132, 2048, 128, 4, 1), (512, 8192, 128, 1, 1),
+])
+def test_spans_that_are_divided(pairs, span, head_dim, shares, parts):
+    """Four wavefronts of heads of more than 128 took four turns over 512 keys in one workgroup."""
+    ops = object.__new__(Ops)
+    ops.compute_units = 256
+    assert ops._decode_parts(pairs, span, head_dim, shares) == parts

@@ -1879,9 +1879,7 @@ class Ops:
             new = (_ptr(q), stride, sum_splits, _ptr(cos), _ptr(sin), _ptr(slots))
         span = max_context if not window else min(max_context, window + 31)
         pairs = requests * kv_heads * -(-(heads // kv_heads) // 16)
-        splits = self._decode_splits(pairs, span)
-        if splits == 1 and span > self.decode_shared_keys and 2 * pairs > self.compute_units:
-            splits = min(max(1, shares), 256)
+        splits = self._decode_parts(pairs, span, head_dim, shares)
         partial_acc = partial_ml = None
         if splits > 1:
             partial_acc = torch.empty((requests * heads * splits, head_dim), dtype=torch.float32, device=out.device)
@@ -1893,14 +1891,25 @@ class Ops:
                   requests, heads, kv_heads, block_size, float(scale), float(softcap), int(window or 0), splits,
                   self._decode_waves(pairs * splits, span, head_dim), *new, self.stream()), "ts_attention_decode")
 
+    def _decode_parts(self, pairs: int, span: int, head_dim: int, shares: int) -> int:
+        """How many workgroups a request and KV head get: :meth:`_decode_splits`, or ``shares`` where that leaves long spans whole.  Heads of
+        more than 128 are divided from 256 keys on, which their four wavefronts walk in two turns (us a layer, 256-wide heads, 300 / 500 keys
+        of one request whole 14.0 / 18.5, divided 11.9 / 13.8, and 13.4 / 16.1 when every 128 keys were a wavefront's; 33 of 300 17.1, 15.3
+        and 16.1)."""
+        splits = self._decode_splits(pairs, max(span, self.decode_whole_keys + 1) if head_dim > 128 and span > 256 else span)
+        if splits == 1 and span > self.decode_shared_keys and 2 * pairs > self.compute_units:
+            return min(max(1, shares), 256)
+        return splits
+
     def _decode_splits(self, pairs: int, span: int) -> int:
         """Over how many workgroups of the decode attention a request's keys are divided: ``pairs`` of request and KV head, at
         most ``span`` keys each.
 
         As many as give every compute unit one workgroup (a second one on a unit waits for the first: its wavefronts
-        hold all registers), none with fewer than ``decode_min_keys`` keys; spans of up to 512 keys stay whole, which saves the
+        hold all registers), at most one for every ``decode_min_keys`` keys of the span (a recorded step's is its shape's bound, of which a request may
+        have less); spans of up to 512 keys stay whole, which saves the
         launch that combines.  Microseconds a layer with the rotation and the store, heads of 128, 7 to a KV head, by number of
-        workgroups: one request of 300 keys 8.5 (1) 8.9 (3), of 640 10.6 (1) 8.9 (6), of 8,192 10.7 (32) 11.3 (64); 8
+        workgroups: one request of 300 keys 8.5 (1) 8.9 (3), of 640 10.6 (1) 8.9 (6), of 8,192 17.7 (8) 11.2 (32) 11.3 (64); 8
         requests of 640 10.2 (4) 11.4 (2), of 8,192 26.6 (8) 29.8 (16); 32 of 2,048 28.6 (2) 30.7 (1) 31.7 (4); 64 of 129 to
         1,525 26.2 (1) 32.0 (2)."""
         if span <= self.decode_whole_keys:
