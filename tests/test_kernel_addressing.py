@@ -165,7 +165,7 @@ def check_decode(ctx, window, shift, table, splits, waves, staged):
     covered = set()
     for x in range(splits):
         for wave in range(waves):
-            first = 32 * (x + splits * wave)
+            first = 32 * (2 * (x + splits * (wave >> 1)) + (wave & 1) if shift > 5 else x + splits * wave)
             # The first window's pages are looked up before the context is known (with a window: again).
             assert all(0 <= min((first >> shift) + i, len(table) - 1) < len(table) for i in range(4))
             w, step = (lo & ~31) + first, 32 * waves * splits
