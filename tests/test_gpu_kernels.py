@@ -1313,6 +1313,18 @@ def test_attention_decode_with_fewer_wavefronts(ops, monkeypatch, heads, kv_head
     torch.testing.assert_close(got.float(), want.float(), rtol=2.0**-7, atol=1e-6)
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,splits", [(20, 1, 80, 1), (34, 2, 128, 3), (40, 1, 32, 5)])
+def test_attention_decode_of_many_requests_and_heads(ops, monkeypatch, heads, kv_heads, dim, splits):
+    """33 requests (not whole groups of eight workgroups) of two and three tiles of query heads a KV head: every workgroup finds its place."""
+    contexts = [1 + (37 * i) % 200 for i in range(33)]
+    monkeypatch.setattr(type(ops), "_decode_splits", lambda self, pairs, span: splits)
+    case = PagedCase(torch.bfloat16, heads, kv_heads, dim, 16, [(c, 1) for c in contexts], None, seed=heads)
+    out = torch.zeros(len(contexts), heads * dim, dtype=torch.bfloat16, device=DEV)
+    ops.attention_decode(out, case.dev(case.q), heads * dim, case.dev(case.kp), case.dev(case.vp), case.dev(case.table), case.ints(case.qsl),
+                         case.ints(contexts), 0, len(contexts), heads, dim ** -0.5, None, max(contexts))
+    torch.testing.assert_close(out.float().cpu(), case.expected, **tol(torch.bfloat16))
+
+
 def rotary_pair(capacity, dim):
     angles = torch.outer(torch.arange(capacity).double(), 10000.0 ** (-torch.arange(dim // 2).double() * 2 / dim))
     return angles.cos().float(), angles.sin().float()

@@ -221,6 +221,26 @@ def test_staged_decode_windows_hold_their_keys_and_values(dim):
             check_decode_stage(table, 1, shift, dim, w, lo, p)
 
 
+@pytest.mark.parametrize("tiles", [2, 3, 8])
+def test_decode_tiles_of_a_kv_head_lie_on_one_die(tiles):
+    """``tiled_place``: every (part, KV head, request, tile) once, the tiles of one eight workgroups apart (in whole groups of eight)."""
+    for splits, kv_heads, requests in ((1, 1, 1), (4, 1, 32), (3, 1, 7), (1, 2, 5), (8, 1, 3), (5, 3, 2), (1, 1, 65)):
+        units, seen = splits * kv_heads * requests, {}
+        for place in range(units * tiles):  # x + splits (y + kv_heads tiles z)
+            group, at = divmod(place, 8 * tiles)
+            width = min(8, units - 8 * group)
+            tile, unit = at // width, 8 * group + at % width
+            part, rest = unit % splits, unit // splits
+            key = (part, rest % kv_heads, rest // kv_heads, tile)
+            assert key not in seen and rest // kv_heads < requests and tile < tiles
+            seen[key] = place
+        assert len(seen) == units * tiles
+        whole = units // 8 * 8
+        for (part, kvh, request, tile), place in seen.items():
+            if part + splits * (kvh + kv_heads * request) < whole:
+                assert place == seen[part, kvh, request, 0] + 8 * tile
+
+
 def check_prefill_wide(pos0, cols, window, shift, table, fed, share=None):
     """``prefill_wide_kernel``'s block-table look-ups for one block of ``cols`` rows whose first
     row is at ``pos0``: every index lies inside the row, every page a load is formed from is a

@@ -685,12 +685,31 @@ __device__ __forceinline__ void decode_staged(ColumnState& st, lds_u16* __restri
   }
 }
 
+// The place of a workgroup where a KV head's query heads are several tiles of sixteen.  The tiles read the same keys, so they are eight
+// workgroups apart in the order of the grid, which deals workgroups to the eight dies in turn: the second finds the keys
+// in its die's L2 (us a layer, 32 heads on one KV head, 32 / 64 requests of 8,192 keys: 45.5 / 91.2 when a wavefront had a stretch of keys and
+// eight splits happened to place them so, 49.9 / 94.1 on different dies, 35.4 / 66.0 here).  A grid whose tiles lie so anyway, and a step of few
+// requests, to which the divisions are 0.2 us and no gain, stay as they are (launch_decode).
+constexpr int DECODE_DIES = 8;
+__device__ __forceinline__ void tiled_place(int splits, int kv_heads, int tiles, int requests, int& part, int& kvh, int& request, int& tile) {
+  const unsigned units = (unsigned)splits * kv_heads * requests, id = blockIdx.x + splits * (blockIdx.y + (unsigned)kv_heads * tiles * blockIdx.z);
+  const unsigned group = id / (DECODE_DIES * tiles), in = id - group * (DECODE_DIES * tiles);
+  const unsigned width = min((unsigned)DECODE_DIES, units - DECODE_DIES * group);  // the last group may be narrower
+  tile = in / width;
+  unsigned unit = DECODE_DIES * group + in - tile * width;
+  part = unit % splits;
+  unit /= splits;
+  kvh = unit % kv_heads;
+  request = unit / kv_heads;
+}
+
 template <int WAVES, bool PROJECTED, bool STAGED>
 __global__ void __launch_bounds__(WAVES * TS_WAVE) __attribute__((amdgpu_waves_per_eu(TS_WAVES_PER_SIMD, TS_WAVES_PER_SIMD)))
 decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ query_start_loc, const int* __restrict__ block_table,
-              int table_width, int seq_begin, int kv_heads, int gsize, int splits, int block_shift, int window, long q_stride,
+              int table_width, int seq_begin, int kv_heads, int gsize, int splits, int block_shift, int window, int placed_tiles, long q_stride,
               uint16_t* __restrict__ k_pages, uint16_t* __restrict__ v_pages, const uint16_t* __restrict__ q, Projected token_sums,
-              ScoreRule scale_log2, uint16_t* __restrict__ out, float* __restrict__ partial_acc, float* __restrict__ partial_ml) {
+              ScoreRule scale_log2, uint16_t* __restrict__ out, float* __restrict__ partial_acc, float* __restrict__ partial_ml,
+              int requests) {
   // (Fourteen words of arguments lie in registers at the start: what the first lookups want comes first.)
   extern __shared__ __attribute__((aligned(16))) float decode_lds[];
   lds_u16* const queries = (lds_u16*)decode_lds;         // [16][QUERY_ROW]
@@ -702,15 +721,16 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
 
   const int lane = threadIdx.x & (TS_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TS_WAVE);
   const int lane16 = lane & 15, group = lane >> 4;
-  const int tile = gsize > 16 ? blockIdx.y / kv_heads : 0, kvh = blockIdx.y - tile * kv_heads;
+  int part = blockIdx.x, tile = gsize > 16 ? blockIdx.y / kv_heads : 0, kvh = blockIdx.y - tile * kv_heads, request = blockIdx.z;
+  if (placed_tiles > 0) tiled_place(splits, kv_heads, placed_tiles, requests, part, kvh, request, tile);
   const int columns = min(16, gsize - 16 * tile), first_head = kvh * gsize + 16 * tile;
-  const int heads = kv_heads * gsize, seq = seq_begin + blockIdx.z;
+  const int heads = kv_heads * gsize, seq = seq_begin + request;
   // The first window's pages without a window do not wait for the context's length.
   PageGeometry geo{k_pages, v_pages, block_table + (size_t)seq * table_width, table_width, kv_heads, kvh, block_shift,
                    (1 << block_shift) - 1};
   // (Windows that share a page's lines of values, of pages of 64 keys and more, are one workgroup's: dealt to two, each line was
   // read twice, a layer of 32 requests of 2,048 keys 39.4 us.)
-  const int first_turn = block_shift > 5 ? 2 * (blockIdx.x + splits * (wave >> 1)) + (wave & 1) : blockIdx.x + splits * wave;
+  const int first_turn = block_shift > 5 ? 2 * (part + splits * (wave >> 1)) + (wave & 1) : part + splits * wave;
   WindowPages first_pages = window_pages(geo, WINDOW_KEYS * first_turn);
   int ctx = context_lens[seq], token = query_start_loc[seq];
   // (One wait for the three and the other arguments; the compiler asked for some behind a wait for the others.)
@@ -726,7 +746,7 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
   const uint16_t* q_row = PROJECTED ? nullptr : q + (size_t)token * q_stride + (size_t)(first_head + lane16) * D;
   const float* sum_row = PROJECTED ? token_sums.sums + (size_t)token * (heads + 2 * kv_heads) * D : nullptr;
   int slot = -1;
-  if (PROJECTED && blockIdx.x == 0 && tile == 0) {
+  if (PROJECTED && part == 0 && tile == 0) {
     int at = token;  // a vector load: scalar ones come back in any order, and what waits for another would wait for this one
     asm volatile("" : "+v"(at));
     slot = token_sums.slots[at];
@@ -814,7 +834,7 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
       const u32x2 word = {pack2(acc[0] / den, acc[1] / den), pack2(acc[2] / den, acc[3] / den)};
       *reinterpret_cast<u32x2*>(out + ((size_t)token * heads + first_head + column) * D + d) = word;
     } else {
-      const size_t at = ((size_t)blockIdx.z * heads + first_head + column) * splits + blockIdx.x;
+      const size_t at = ((size_t)request * heads + first_head + column) * splits + part;
       *reinterpret_cast<f32x4*>(partial_acc + at * D + d) = acc;
       if (d == 0) {
         float top = -INFINITY;
@@ -2007,11 +2027,12 @@ static int launch_decode(uint16_t* out, float* partial_acc, float* partial_ml, c
   const int gsize = heads / kv_heads, head_tiles = (gsize + 15) / 16, columns = gsize < 16 ? gsize : 16;
   const size_t joined = (size_t)WAVES * columns * SUM_ROW * 4, rings = STAGED ? (size_t)WAVES * Stage::WAVE * 2 : 0;
   const size_t lds = (16 * QUERY_ROW + 2 * D) * 2 + WAVES * 32 * 4 + (joined > rings ? joined : rings);
+  const bool placed = head_tiles > 1 && requests >= 32 && splits * kv_heads % DECODE_DIES != 0;
   static const bool raised = hipFuncSetAttribute((const void*)decode_kernel<WAVES, PROJECTED, STAGED>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
   if (!raised) return TS_ERR_LAUNCH;
   hipLaunchKernelGGL((decode_kernel<WAVES, PROJECTED, STAGED>), dim3(splits, kv_heads * head_tiles, requests), dim3(WAVES * TS_WAVE), lds,
                      stream, context_lens, query_start_loc, block_table, table_width, seq_begin, kv_heads, gsize, splits, shift, window,
-                     q_stride, k_pages, v_pages, q, token_sums, rule, out, partial_acc, partial_ml);
+                     placed ? head_tiles : 0, q_stride, k_pages, v_pages, q, token_sums, rule, out, partial_acc, partial_ml, requests);
   if (splits == 1) return ts_launch_status();
   if (hipGetLastError() != hipSuccess) return TS_ERR_LAUNCH;
   hipLaunchKernelGGL(decode_reduce_kernel, dim3(requests, heads), dim3(REDUCE_THREADS), 0, stream, out, partial_acc, partial_ml,
