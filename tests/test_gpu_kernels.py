@@ -877,6 +877,28 @@ def test_rope_store_of_a_prompts_partial_sums_equals_token_by_token(ops, heads, 
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,page,rotate", [(2, 1, 256, 16, True), (3, 2, 16, 4, True), (5, 1, 80, 8, True), (2, 1, 64, 32, False)])
+@pytest.mark.parametrize("tokens,splits", [(129, 2), (137, 4), (131, 1)])
+def test_rope_store_of_a_prompts_partial_sums_of_any_head(ops, heads, kv_heads, dim, page, rotate, tokens, splits):
+    """Heads wider and narrower than a wavefront's pieces, pages of fewer than eight keys, no rotation, no slots: as token by token."""
+    g = torch.Generator().manual_seed(tokens + dim)
+    sums = torch.randn(splits, tokens, (heads + 2 * kv_heads) * dim, generator=g)
+    tables = tuple(t.to(DEV) for t in rotary_pair(512, dim)) if rotate else (None, None)
+    positions = torch.randint(0, 512, (tokens,), generator=g, dtype=torch.int32)
+    slots = (torch.randperm(tokens, generator=g) + 3).to(torch.int32)
+    slots[64:96] = torch.arange(200, 232)
+    pages = -(-240 // page)
+    got = []
+    for parts in ([(0, tokens)], [(at, min(at + 100, tokens)) for at in range(0, tokens, 100)]):
+        kp = torch.zeros(pages, kv_heads, page, dim, dtype=torch.bfloat16, device=DEV)
+        vp = torch.zeros(pages, kv_heads, dim, page, dtype=torch.bfloat16, device=DEV)
+        rows = [[ops.rope_store(sums[:, a:b].contiguous().to(DEV), kp, vp, *tables, positions[a:b].to(DEV), at, heads, kv_heads, dim, page, 511,
+                                torch.bfloat16)[0] for at in (None, slots[a:b].to(DEV))] for a, b in parts]
+        got.append(tuple(torch.cat(r).view(torch.int16) for r in zip(*rows)) + (kp.view(torch.int16), vp.view(torch.int16)))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,page", [(7, 1, 128, 16), (3, 3, 48, 8), (4, 2, 32, 4), (2, 1, 96, 32)])
 def test_rope_store_of_many_tokens_equals_token_by_token(ops, heads, kv_heads, dim, page):
     """Prompt portions of 32 tokens or more go through a kernel that handles 8 tokens per block

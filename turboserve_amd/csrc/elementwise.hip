@@ -694,37 +694,7 @@ __global__ void rope_store_kernel(T* q_out, long q_stride, const P* proj, int sp
   }
 }
 
-// N neighbouring elements of a projection as numbers: its own, or `splits` partial sums added up in their order, four on their way at once.
-template <int N>
-__device__ __forceinline__ void rope_input(const bf16_t* p, int, size_t, float (&v)[N]) {
-  typedef uint16_t u16xN __attribute__((ext_vector_type(N)));
-  const u16xN raw = *reinterpret_cast<const u16xN*>(p);
-#pragma unroll
-  for (int e = 0; e < N; ++e) v[e] = to_float(bf16_t{raw[e]});
-}
-template <int N>
-__device__ __forceinline__ void rope_input(const float* p, int splits, size_t stride, float (&v)[N]) {
-  typedef float f32xP __attribute__((ext_vector_type(N < 4 ? N : 4)));
-  constexpr int EACH = N < 4 ? N : 4;
-#pragma unroll
-  for (int e = 0; e < N; ++e) v[e] = 0.f;
-  for (int first = 0; first < splits; first += 4) {
-    f32xP part[4][N / EACH];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-      for (int e = 0; e < N / EACH; ++e)
-        part[j][e] = *reinterpret_cast<const f32xP*>(p + (size_t)min(first + j, splits - 1) * stride + EACH * e);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-      for (int e = 0; e < N; ++e) v[e] = first + j < splits ? v[e] + part[j][e / EACH][e % EACH] : v[e];
-    }
-  }
-}
-
-// The same for many tokens at once (prompt portions): a bfloat16 projection or 32-bit partial sums, bfloat16 out, head
+// The same for many tokens at once (prompt portions): bfloat16 in and out, no partial sums, head
 // size a multiple of 16.  One block per (group of 8 consecutive tokens, head).  q and k heads: a
 // thread rotates 8 pairs with 16-byte loads and stores.  v heads: a thread collects one head
 // dimension of the 8 tokens; when the group's slots are 8 consecutive ones starting at a multiple
@@ -732,10 +702,9 @@ __device__ __forceinline__ void rope_input(const float* p, int splits, size_t st
 // that is one 16-byte store into the transposed value page, else one 2-byte store per token.
 constexpr int ROPE_GROUP = 8;
 
-template <typename P>
 __global__ void __launch_bounds__(64)
-rope_store_group_kernel(bf16_t* q_out, long q_stride, const P* proj, int splits, size_t split_stride,
-                        bf16_t* __restrict__ k_pages, bf16_t* __restrict__ v_pages, const float* __restrict__ cos_table,
+rope_store_group_kernel(bf16_t* q_out, long q_stride, const bf16_t* proj, bf16_t* __restrict__ k_pages,
+                        bf16_t* __restrict__ v_pages, const float* __restrict__ cos_table,
                         const float* __restrict__ sin_table, const int* __restrict__ positions,
                         const int* __restrict__ slots, int tokens, int heads, int kv_heads, int dim,
                         int block_size, int rotate) {
@@ -754,16 +723,10 @@ rope_store_group_kernel(bf16_t* q_out, long q_stride, const P* proj, int splits,
       const int j = item / vectors, i = (item % vectors) * 8;
       if (j >= count) continue;
       const int t = t0 + j;
-      const P* row = proj + (size_t)t * width + (size_t)h * dim;
-      float a[8], b[8];
-      rope_input<8>(row + i, splits, split_stride, a);
-      rope_input<8>(row + i + half, splits, split_stride, b);
-      u16x8 o1, o2;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        o1[e] = from_float<bf16_t>(a[e]).bits;
-        o2[e] = from_float<bf16_t>(b[e]).bits;
-      }
+      const bf16_t* row = proj + (size_t)t * width + (size_t)h * dim;
+      const u16x8 a = *reinterpret_cast<const u16x8*>(row + i);
+      const u16x8 b = *reinterpret_cast<const u16x8*>(row + i + half);
+      u16x8 o1 = a, o2 = b;
       if (rotate) {
         const float* c = cos_table + (size_t)positions[t] * half + i;
         const float* s = sin_table + (size_t)positions[t] * half + i;
@@ -773,7 +736,7 @@ rope_store_group_kernel(bf16_t* q_out, long q_stride, const P* proj, int splits,
         for (int e = 0; e < 8; ++e) {
           const float cv = e < 4 ? c0[e & 3] : c1[e & 3], sv = e < 4 ? s0[e & 3] : s1[e & 3];
           float r1, r2;
-          rotate_pair(a[e], b[e], cv, sv, r1, r2);
+          rotate_pair(to_float(bf16_t{a[e]}), to_float(bf16_t{b[e]}), cv, sv, r1, r2);
           o1[e] = from_float<bf16_t>(r1).bits;
           o2[e] = from_float<bf16_t>(r2).bits;
         }
@@ -800,15 +763,11 @@ rope_store_group_kernel(bf16_t* q_out, long q_stride, const P* proj, int splits,
   bool run = count == ROPE_GROUP && slot[0] >= 0 && (slot[0] & 7) == 0 && (block_size & 7) == 0;
 #pragma unroll
   for (int j = 1; j < ROPE_GROUP; ++j) run = run && slot[j] == slot[0] + j;
-  const P* column = proj + (size_t)t0 * width + (size_t)h * dim;
+  const bf16_t* column = proj + (size_t)t0 * width + (size_t)h * dim;
   for (int d = threadIdx.x; d < dim; d += blockDim.x) {
     u16x8 v;
 #pragma unroll
-    for (int j = 0; j < ROPE_GROUP; ++j) {
-      float one[1];
-      rope_input<1>(column + (size_t)min(j, count - 1) * width + d, splits, split_stride, one);
-      v[j] = j < count ? from_float<bf16_t>(one[0]).bits : (uint16_t)0;
-    }
+    for (int j = 0; j < ROPE_GROUP; ++j) v[j] = j < count ? column[(size_t)j * width + d].bits : (uint16_t)0;
     if (run) {
       bf16_t* dst = v_pages + (((size_t)(slot[0] / block_size) * kv_heads + kvh) * dim + d) * block_size + slot[0] % block_size;
       *reinterpret_cast<u16x8*>(dst) = v;
@@ -817,6 +776,109 @@ rope_store_group_kernel(bf16_t* q_out, long q_stride, const P* proj, int splits,
       for (int j = 0; j < ROPE_GROUP; ++j) {
         if (slot[j] < 0) continue;
         v_pages[(((size_t)(slot[j] / block_size) * kv_heads + kvh) * dim + d) * block_size + slot[j] % block_size] = bf16_t{v[j]};
+      }
+    }
+  }
+}
+
+// The same for a prompt's projection as up to BATCH 32-bit partial sums: what a thread adds up (eight pairs of a q or k head, two neighbouring
+// dimensions of a v head of the eight tokens) is all on its way before any of it is added, in the order of the sums.  One token's
+// behind the other's it was eight trips to memory a thread (us behind the product: 299 rows of the 7B shape as three sums 10.3 -> 6.2, 256
+// of 7,168 columns as two 10.1 -> 5.1; a bfloat16 projection 4).
+template <int BATCH>
+__global__ void __launch_bounds__(64)
+rope_store_sums_kernel(const float* proj, const int* __restrict__ positions, const int* __restrict__ slots, int splits, int tokens,
+                       size_t split_stride, int heads, int kv_heads, int dim, int block_size, int rotate, long q_stride,
+                       const float* __restrict__ cos_table, const float* __restrict__ sin_table, bf16_t* q_out,
+                       bf16_t* __restrict__ k_pages, bf16_t* __restrict__ v_pages) {
+  typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+  typedef float f32x2v __attribute__((ext_vector_type(2)));
+  typedef float f32x4v __attribute__((ext_vector_type(4)));
+  const int t0 = blockIdx.x * ROPE_GROUP, h = blockIdx.y, half = dim / 2;
+  const int width = (heads + 2 * kv_heads) * dim, count = min(ROPE_GROUP, tokens - t0);
+  if (h < heads + kv_heads) {
+    const int vectors = half / 8;
+    for (int item = threadIdx.x; item < count * vectors; item += 64) {
+      const int t = t0 + item / vectors, i = (item % vectors) * 8;
+      const float* row = proj + (size_t)t * width + (size_t)h * dim + i;
+      f32x4v part[BATCH][4], turn[4];
+#pragma unroll
+      for (int j = 0; j < BATCH; ++j) {
+        const float* at = row + (size_t)min(j, splits - 1) * split_stride;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) part[j][q] = *reinterpret_cast<const f32x4v*>(at + (q >> 1) * half + 4 * (q & 1));
+      }
+      int slot = h >= heads && slots ? slots[t] : -1;
+      if (rotate) {
+        const size_t angle = (size_t)positions[t] * half + i;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) turn[q] = *reinterpret_cast<const f32x4v*>((q < 2 ? cos_table : sin_table) + angle + 4 * (q & 1));
+      }
+      asm volatile("" : "+v"(slot)::"memory");  // all of them on their way here
+      u16x8 o1, o2;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float a = 0.f, b = 0.f;
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) {
+          a = j < splits ? a + part[j][e / 4][e % 4] : a;
+          b = j < splits ? b + part[j][2 + e / 4][e % 4] : b;
+        }
+        float r1 = a, r2 = b;
+        if (rotate) rotate_pair(a, b, turn[e / 4][e % 4], turn[2 + e / 4][e % 4], r1, r2);
+        o1[e] = from_float<bf16_t>(r1).bits;
+        o2[e] = from_float<bf16_t>(r2).bits;
+      }
+      bf16_t* to = q_out + (size_t)t * q_stride + (size_t)h * dim;
+      if (h >= heads) {
+        if (slot < 0) continue;
+        to = k_pages + (((size_t)(slot / block_size) * kv_heads + h - heads) * block_size + slot % block_size) * dim;
+      }
+      *reinterpret_cast<u16x8*>(to + i) = o1;
+      *reinterpret_cast<u16x8*>(to + i + half) = o2;
+    }
+    return;
+  }
+  if (!slots) return;
+  const int kvh = h - heads - kv_heads;
+  const float* column = proj + (size_t)t0 * width + (size_t)h * dim;
+  for (int d = 2 * threadIdx.x; d < dim; d += 128) {
+    f32x2v part[ROPE_GROUP][BATCH];
+#pragma unroll
+    for (int t = 0; t < ROPE_GROUP; ++t) {
+#pragma unroll
+      for (int j = 0; j < BATCH; ++j)
+        part[t][j] = *reinterpret_cast<const f32x2v*>(column + (size_t)min(j, splits - 1) * split_stride + (size_t)min(t, count - 1) * width + d);
+    }
+    int slot[ROPE_GROUP];
+#pragma unroll
+    for (int t = 0; t < ROPE_GROUP; ++t) slot[t] = t < count ? slots[t0 + t] : -1;
+    asm volatile("" ::: "memory");
+    bool run = count == ROPE_GROUP && slot[0] >= 0 && (slot[0] & 7) == 0 && (block_size & 7) == 0;
+#pragma unroll
+    for (int t = 1; t < ROPE_GROUP; ++t) run = run && slot[t] == slot[0] + t;
+    u16x8 v[2];
+#pragma unroll
+    for (int t = 0; t < ROPE_GROUP; ++t) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        float x = 0.f;
+#pragma unroll
+        for (int j = 0; j < BATCH; ++j) x = j < splits ? x + part[t][j][e] : x;
+        v[e][t] = from_float<bf16_t>(x).bits;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      if (run) {
+        bf16_t* dst = v_pages + (((size_t)(slot[0] / block_size) * kv_heads + kvh) * dim + d + e) * block_size + slot[0] % block_size;
+        *reinterpret_cast<u16x8*>(dst) = v[e];
+      } else {
+#pragma unroll
+        for (int t = 0; t < ROPE_GROUP; ++t) {
+          if (slot[t] < 0) continue;
+          v_pages[(((size_t)(slot[t] / block_size) * kv_heads + kvh) * dim + d + e) * block_size + slot[t] % block_size] = bf16_t{v[e][t]};
+        }
       }
     }
   }
@@ -836,16 +898,20 @@ extern "C" int ts_rope_store(void* q_out, long q_stride, const void* proj, int i
   dim3 grid(tokens, heads + 2 * kv_heads), block(64);
   const bool aligned = ((uintptr_t)q_out | (uintptr_t)proj | (uintptr_t)k_pages | (uintptr_t)v_pages |
                         (uintptr_t)cos_table | (uintptr_t)sin_table) % 16 == 0 && q_stride % 8 == 0;
-  const bool sums_in_groups = in_f32 && split_stride % 4 == 0 && tokens > 128;
-  if (dtype == TS_BF16 && ((!in_f32 && splits == 1) || sums_in_groups) && dim % 16 == 0 && tokens >= 4 * ROPE_GROUP && aligned) {
-    dim3 groups((tokens + ROPE_GROUP - 1) / ROPE_GROUP, heads + 2 * kv_heads);
-#define TS_ROPE_GROUP(P)                                                                                                       \
-  hipLaunchKernelGGL(rope_store_group_kernel<P>, groups, block, 0, stream, (bf16_t*)q_out, q_stride, (const P*)proj, splits,   \
-                     (size_t)split_stride, (bf16_t*)k_pages, (bf16_t*)v_pages, cos_table, sin_table, positions, slots, tokens, \
-                     heads, kv_heads, dim, block_size, rotate)
-    if (in_f32) TS_ROPE_GROUP(float);
-    else TS_ROPE_GROUP(bf16_t);
-#undef TS_ROPE_GROUP
+  const dim3 groups((tokens + ROPE_GROUP - 1) / ROPE_GROUP, heads + 2 * kv_heads);
+  if (dtype == TS_BF16 && in_f32 && splits <= 4 && split_stride % 4 == 0 && dim % 16 == 0 && tokens > 128 && aligned) {
+#define TS_ROPE_SUMS(BATCH)                                                                                                                  \
+  hipLaunchKernelGGL(rope_store_sums_kernel<BATCH>, groups, block, 0, stream, (const float*)proj, positions, slots, splits, tokens,           \
+                     (size_t)split_stride, heads, kv_heads, dim, block_size, rotate, q_stride, cos_table, sin_table, (bf16_t*)q_out,         \
+                     (bf16_t*)k_pages, (bf16_t*)v_pages)
+    if (splits == 1) TS_ROPE_SUMS(1);
+    else if (splits == 2) TS_ROPE_SUMS(2);
+    else TS_ROPE_SUMS(4);
+#undef TS_ROPE_SUMS
+    return ts_launch_status();
+  }
+  if (dtype == TS_BF16 && !in_f32 && splits == 1 && dim % 16 == 0 && tokens >= 4 * ROPE_GROUP && aligned) {
+    hipLaunchKernelGGL(rope_store_group_kernel, groups, block, 0, stream, (bf16_t*)q_out, q_stride, (const bf16_t*)proj, (bf16_t*)k_pages, (bf16_t*)v_pages, cos_table, sin_table, positions, slots, tokens, heads, kv_heads, dim, block_size, rotate);
     return ts_launch_status();
   }
   if (dtype == TS_F32)
