@@ -19,6 +19,7 @@ class Launches:
     """The operations an attention layer asks for, by name."""
 
     mfma_attention_supported = staticmethod(Ops.mfma_attention_supported)
+    decode_projected_supported = staticmethod(Ops.decode_projected_supported)
     decode_shared_keys = Ops.decode_shared_keys
 
     def __init__(self):
@@ -83,13 +84,17 @@ def encodings(monkeypatch):
     (GroupedQueryAttention, "rope_table", ["store", "generic"]),
     (OwnAttention, "rope", ["store", "own"]),
 ])
-def test_a_decode_step_attends_by_the_layers_rule(encodings, kind, encoding, launches):
+@pytest.mark.parametrize("offset", [0, 4])
+def test_a_decode_step_attends_by_the_layers_rule(encodings, kind, encoding, launches, offset):
     ops = Launches()
     runtime = Runtime(device=torch.device("cpu"), dtype=torch.bfloat16, ops=ops)
     layer = kind("layer", runtime, hidden_size=64, num_heads=4, num_kv_heads=2, head_dim=32, scale=32 ** -0.5, qkv_bias=False, out_bias=False,
                  window=None, position=PartSpec(encoding, {"head_dim": 32, "theta": 1e4, "max_positions": 64}))
     layer.qkv_weight = torch.zeros(8 * 32, 64)
-    cache = SimpleNamespace(group=0, writable=True, block_size=16, k=torch.zeros(4, 2, 16, 32), v=torch.zeros(4, 2, 32, 16))
+    pages = [torch.zeros(4 * 1024 + 4, dtype=torch.bfloat16)[offset:offset + 4096] for _ in range(2)]
+    cache = SimpleNamespace(group=0, writable=True, block_size=16, k=pages[0].view(4, 2, 16, 32), v=pages[1].view(4, 2, 32, 16))
+    if offset and launches == ["all in one"]:  # the launch that stores wants pages on 16 bytes
+        launches = ["store", "attention"]
     ints = torch.zeros(3, dtype=torch.int32)
     ctx = SimpleNamespace(num_tokens=3, num_seqs=3, num_prefill_seqs=0, num_decode_seqs=3, max_context_len=20, max_decode_context_len=20,
                           block_tables=[torch.zeros(3, 4, dtype=torch.int32)], slot_mapping=[ints], positions=ints, token_seq=ints,

@@ -1335,6 +1335,26 @@ def test_attention_decode_with_fewer_wavefronts(ops, monkeypatch, heads, kv_head
     torch.testing.assert_close(got.float(), want.float(), rtol=2.0**-7, atol=1e-6)
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim", [(14, 2, 128), (8, 1, 64), (6, 2, 256), (4, 2, 80)])
+def test_attention_decode_of_pages_between_16_bytes(ops, heads, kv_heads, dim):
+    """Pages 8 bytes off: transfers to LDS are not for them, plain loads are; the launch that stores refuses them."""
+    from turboserve_amd.kernels.ops import KernelError
+
+    contexts = [70, 1, 33, 600, 129]
+    case = PagedCase(torch.bfloat16, heads, kv_heads, dim, 16, [(c, 1) for c in contexts], None, seed=dim)
+    off = lambda t: torch.cat([t.new_zeros(4), t.flatten(), t.new_zeros(4)]).to(DEV)[4:4 + t.numel()].view(t.shape)
+    kp, vp = off(case.kp), off(case.vp)
+    assert kp.data_ptr() % 16 == 8
+    out = torch.zeros(len(contexts), heads * dim, dtype=torch.bfloat16, device=DEV)
+    common = (case.dev(case.table), case.ints(case.qsl), case.ints(contexts), 0, len(contexts), heads, dim ** -0.5, None, max(contexts))
+    ops.attention_decode(out, case.dev(case.q), heads * dim, kp, vp, *common)
+    torch.testing.assert_close(out.float().cpu(), case.expected, **tol(torch.bfloat16))
+    sums = torch.zeros(1, len(contexts), (heads + 2 * kv_heads) * dim, device=DEV)
+    cos, sin = (t.to(DEV) for t in rotary_pair(1024, dim))
+    with pytest.raises(KernelError):
+        ops.attention_decode(out, sums, 0, kp, vp, *common, projected=(cos, sin, case.ints(contexts), 1023))
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,splits", [(20, 1, 80, 1), (34, 2, 128, 3), (40, 1, 32, 5)])
 def test_attention_decode_of_many_requests_and_heads(ops, monkeypatch, heads, kv_heads, dim, splits):
     """33 requests (not whole groups of eight workgroups) of two and three tiles of query heads a KV head: every workgroup finds its place."""

@@ -2051,6 +2051,7 @@ extern "C" int TS_SYM(ts_attention_decode_d)(
     return TS_ERR_ARG;
   if (splits > 1 && (!partial_acc || !partial_ml)) return TS_ERR_ARG;
   if (sums && (!cos_table || !sin_table || !slots || sum_splits < 1)) return TS_ERR_ARG;
+  if (sums && (((uintptr_t)k_pages | (uintptr_t)v_pages) % 16 != 0 || block_size > (1 << 20))) return TS_ERR_SHAPE;
   if (sums && (((uintptr_t)sums | (uintptr_t)cos_table | (uintptr_t)sin_table) % 16 != 0 || sum_stride % 4 != 0)) return TS_ERR_SHAPE;
   if (heads < 1 || kv_heads < 1 || heads % kv_heads != 0) return TS_ERR_SHAPE;
   if (block_size < 8 || (block_size & (block_size - 1))) return TS_ERR_SHAPE;
@@ -2064,6 +2065,8 @@ extern "C" int TS_SYM(ts_attention_decode_d)(
   auto launch = sums ? launch_decode<DECODE_WAVES, true, DECODE_STAGED> : launch_decode<DECODE_WAVES, false, DECODE_STAGED>;
   if (waves == 4 && DECODE_WAVES > 4) launch = sums ? launch_decode<4, true, DECODE_STAGED> : launch_decode<4, false, DECODE_STAGED>;
   if (waves == 2) launch = sums ? launch_decode<2, true, DECODE_STAGED> : launch_decode<2, false, DECODE_STAGED>;
+  // Transfers to LDS want pages on 16 bytes that 31-bit offsets reach; plain loads take any.
+  if (DECODE_STAGED && (((uintptr_t)k_pages | (uintptr_t)v_pages) % 16 != 0 || shift > 20)) launch = launch_decode<DECODE_WAVES, false, false>;
   return launch((uint16_t*)out, (float*)partial_acc, (float*)partial_ml, (const uint16_t*)q, q_stride, (uint16_t*)k_pages,
                 (uint16_t*)v_pages, block_table, table_width, query_start_loc, context_lens, seq_begin, requests, heads, kv_heads,
                 shift, score_rule(scale, softcap), window, splits, token_sums, stream);

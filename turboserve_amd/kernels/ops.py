@@ -1815,6 +1815,11 @@ class Ops:
         kernel."""
         return dtype == torch.bfloat16 and head_dim % 16 == 0 and 16 <= head_dim <= 256 and block_size >= 8
 
+    @staticmethod
+    def decode_projected_supported(k_pages: torch.Tensor, v_pages: torch.Tensor) -> bool:
+        """Whether :meth:`attention_decode` stores into these pages itself (``projected``)."""
+        return (k_pages.data_ptr() | v_pages.data_ptr()) % 16 == 0 and k_pages.shape[2] <= 1 << 20
+
     def attention_decode(
         self,
         out: torch.Tensor,
@@ -1872,6 +1877,7 @@ class Ops:
             tokens = slots.numel()
             is_f32, sum_splits, stride = self._partials(q, tokens, (heads + 2 * kv_heads) * head_dim, torch.bfloat16, "projection")
             _need(bool(is_f32) and q.dim() == 3, "the projection must be 32-bit partial sums")
+            _need(self.decode_projected_supported(k_pages, v_pages), "the new keys and values go to pages on 16 bytes")
             _need(out.shape[0] >= tokens, "one row of out per token")
             _need(cos.shape == sin.shape and cos.dim() == 2 and cos.shape[1] == head_dim // 2 and cos.dtype == sin.dtype == torch.float32
                   and cos.is_contiguous() and sin.is_contiguous(), "cos/sin must be float32 [capacity, D/2]")

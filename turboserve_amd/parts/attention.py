@@ -358,7 +358,8 @@ class GroupedQueryAttention(Mixer):
         ops = self.runtime.ops
         if (qkv.dim() != 3 or ctx.num_prefill_seqs != 0 or ctx.num_decode_seqs != ctx.num_tokens or not self._plain_rule()
                 or not self.own_keys or not cache.writable
-                or not ops.mfma_attention_supported(self.runtime.dtype, self.head_dim, cache.block_size)):
+                or not ops.mfma_attention_supported(self.runtime.dtype, self.head_dim, cache.block_size)
+                or not ops.decode_projected_supported(cache.k, cache.v)):
             return None
         # What attends in a way of its own is asked (`attend`), and so is an encoding that also acts inside the scores.
         if (type(self).attend is not GroupedQueryAttention.attend or self.position.score_slopes(self.num_heads) is not None
