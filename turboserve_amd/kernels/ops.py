@@ -2932,21 +2932,14 @@ class Ops:
             return self.swiglu(self._library_product(x, weight, bias, None), x.dtype, paired=True, rule=rule)
         return self.swiglu(self.linear(x, weight, bias), x.dtype, paired=True, rule=rule)
 
-    #: Fewest elements of a matrix whose product may leave partial sums for the store of heads.
-    store_sums_min_weights = 12 << 20
-
     def _sums_plan(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> tuple[int, int, int, int] | None:
         """The block product's grid for a prompt of few rows whose consumer adds up partial sums as well as it takes one result
         (the store of rotated heads), or None where one result is as soon there.  A narrow product as one range of K leaves most
         units idle: several ranges where the model puts them, their way to the consumer included, at seven tenths of one
-        range's time (us with the store, one result by the library or here / sums: 4,608 x 3,584 at 150 / 200 / 256 / 299 / 350 rows 26.1 / 36.2 /
-        41.1 / 29.0 / 32.3 against 23.1 / 22.3 / 24.9 / 27.2 / 28.3; 7,168 x 5,120 at 150 / 200 / 299 38.2 / 44.6 / 50.7 against 32.2 / 35.6 /
-        43.1; the library's kernels timed for the shape: 22.5 / 26.6 / 28.8 / 29.3 / 31.2, 37.0 / 43.2 / 47.8).  Smaller matrices keep one
-        result: the sums' way to the store is long beside the product (3,072 x 2,048 at 150 / 256 / 400 rows 17.7 / 17.4 / 19.4 against 16.9 / 21.4 /
-        22.4, 2,048 x 1,536 at 256 14.0 against 17.2; 6,144 x 2,048 at 150 / 256 26.9 / 29.2 against 21.0 / 21.4)."""
+        range's time (us with the store, one result by the library or here / sums: 4,608 x 3,584 at 200 / 256 / 299 / 350 rows 36 / 39 /
+        33.9 / 33.4 against 26 / 28 / 29.9 / 31.5, at 400 31.6 against 33.0; 7,168 x 5,120 at 200 / 299 42 / 47 against 38 / 45, at
+        400 46 against 50)."""
         m, (n, k) = x.shape[0], weight.shape
-        if n * k < self.store_sums_min_weights:
-            return None
         if not self.skinny_max_rows < m <= self.wide_default_rows or not self.block_supported(x, weight) or (bias is not None and bias.data_ptr() % 8):
             return None
         key = ("sums for the store", m, n, k)
