@@ -99,8 +99,13 @@ def test_a_decode_step_attends_by_the_layers_rule(encodings, kind, encoding, lau
     ctx = SimpleNamespace(num_tokens=3, num_seqs=3, num_prefill_seqs=0, num_decode_seqs=3, max_context_len=20, max_decode_context_len=20,
                           block_tables=[torch.zeros(3, 4, dtype=torch.int32)], slot_mapping=[ints], positions=ints, token_seq=ints,
                           query_start_loc=ints, context_lens=ints, max_decode_context_dev=ints[:1], carried={})
+    asked, plain_store = [], layer.position.plain_store
+    layer.position.plain_store = lambda head_dim: asked.append(head_dim) or plain_store(head_dim)
     layer.heads_out(torch.zeros(3, 64), ctx, cache)
     assert ops.names == launches
+    ctx.num_prefill_seqs, ctx.num_decode_seqs = 1, 2  # a step with a prompt never goes to the launch that stores
+    assert layer._attend_projected(torch.zeros(3, 3, 256), ctx, cache) is None
+    assert layer._plain_store == plain_store(32) and len(asked) <= (2 if launches == ["all in one"] else 1)  # worked out once
 
 
 @pytest.mark.parametrize("workgroups,span,head_dim,waves", [

@@ -207,3 +207,15 @@ def test_a_steps_estimate_holds_what_its_products_and_attention_leave():
     products = 2048 * (3 * 18944 * 2 + 3584 * 4)  # gate|up, its units, what the stream waits for
     assert model.activation_bytes(2048, 64, 2) >= stream + products + sums
     assert model.activation_bytes(64, 64, 4) >= Ops.float32_attention_scratch
+
+
+def test_only_a_head_is_asked_for_rounds(monkeypatch):
+    """A decode-sized product knows its grid; only a matrix of more weight rows than a round of tiles of 256 is looked at for whole rounds
+    and a rest (asked for every gated product, with a loop over one launch in each product: 2% of a short prompt of eight layers 2,048 wide)."""
+    monkeypatch.setattr("turboserve_amd.kernels.ops._gpu", lambda *tensors: None)
+    ops, asked = Planner(), []
+    monkeypatch.setattr(ops, "_block_few_rounds", lambda *of: asked.append(of) or Ops._block_few_rounds(ops, *of), raising=False)
+    for n, k in ((16384, 2048), (37888, 3584), (65280, 2048)):
+        ops._block_few_runs(*operands(31, n, k), None, 1)
+    assert not asked
+    assert len(ops._block_few_runs(*operands(64, 152064, 3584), None, 1)) == 7 and asked == [(64, 152064, 3584)]

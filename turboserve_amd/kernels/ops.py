@@ -2388,9 +2388,8 @@ class Ops:
         if bias is not None:
             _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 8 == 0,
                   "bias must be bfloat16 [N]")
-        per_split, splits, tn, tm, *tail = plan
+        per_split, splits, tn, tm = plan[:4]
         _need(not gated or splits == 1, "the gated result needs one range of K")
-        _need(not tail or (splits == 1 and 0 < tail[0] < n and tail[0] % 16 == 0), "a tail is for one range of K")
         partial = out = None
         if gated or (splits == 1 and not sums):
             out = self.rows_buffer(m, n // 2 if gated else n, torch.bfloat16, x.device)
@@ -2398,14 +2397,18 @@ class Ops:
             partial = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
         unit = glu_rule(rule) if gated else (1.0, 0.0, 0.0, 0.0)
         mode = 2 if gated else 1 if out is None else 0
-        runs = [(0, n, tn, tm)] if not tail else [(0, tail[0], tn, tm), (tail[0], n - tail[0], *tail[1:])]
-        for first, rows, tile_n, tile_m in runs:
-            at = None if out is None else out.data_ptr() + 2 * (first // 2 if gated else first)
-            sums_at = None if partial is None else partial.data_ptr() + 4 * first
-            _check(self.core.ts_gemm_block(sums_at, at, _ptr(x), x.stride(0), weight.data_ptr() + 2 * first * k,
-                                           None if bias is None else bias.data_ptr() + 2 * first, m, rows, k, per_split, splits,
-                                           tile_n, tile_m, mode, n, *unit, self.stream()),
-                   "ts_gemm_block")
+        rows = n
+        sums_at, at, weight_at, bias_at = _ptr(partial), _ptr(out), weight.data_ptr(), _ptr(bias)
+        if len(plan) > 4:  # whole rounds first, the rest of the weight rows in other tiles
+            first = plan[4]
+            _need(splits == 1 and 0 < first < n and first % 16 == 0, "a rest is for one range of K")
+            _check(self.core.ts_gemm_block(sums_at, at, _ptr(x), x.stride(0), weight_at, bias_at, m, first, k, per_split, splits, tn, tm,
+                                           mode, n, *unit, self.stream()), "ts_gemm_block")
+            rows, tn, tm = n - first, *plan[5:]
+            sums_at, at = sums_at and sums_at + 4 * first, at and at + (first if gated else 2 * first)
+            weight_at, bias_at = weight_at + 2 * first * k, bias_at and bias_at + 2 * first
+        _check(self.core.ts_gemm_block(sums_at, at, _ptr(x), x.stride(0), weight_at, bias_at, m, rows, k, per_split, splits, tn, tm,
+                                       mode, n, *unit, self.stream()), "ts_gemm_block")
         return partial if out is None else out
 
     def _own_product(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, kind: str,
@@ -2721,7 +2724,8 @@ class Ops:
         if bias is not None and bias.data_ptr() % 8:
             return None
         m, (n, k) = x.shape[0], weight.shape
-        return (self._block_few_rounds(m, n, k) if max_splits == 1 else None) or self._block_few_plan(m, n, k, max_splits)
+        rounds = self._block_few_rounds(m, n, k) if max_splits == 1 and n > 256 * (self.compute_units - 1) else None
+        return rounds or self._block_few_plan(m, n, k, max_splits)
 
     def _block_few_rounds(self, m: int, n: int, k: int) -> tuple[int, ...] | None:
         """A matrix of more than 65,536 rows (a head) as one range of K for a decode step: whole rounds of tiles of 256 and the rest in one

@@ -3,6 +3,7 @@ src/turboserve/engine/model/attention.py:213-295)."""
 
 from __future__ import annotations
 
+import functools
 from collections.abc import Mapping
 
 import torch
@@ -288,6 +289,7 @@ class GroupedQueryAttention(Mixer):
         do the attention kernels that take any rule (the ones that only take plain causal or windowed attention do not)."""
         return self.gate_name is not None or not self._plain_rule()
 
+    @functools.cached_property
     def _plain_store(self) -> bool:
         """Whether the projection goes to the plain rotation and store (:meth:`Ops.rope_store`) as it is."""
         return (self.conv_taps is None and self.gate_name is None and not self.values_are_keys and self.query_temperature is None
@@ -305,7 +307,7 @@ class GroupedQueryAttention(Mixer):
         = (buffer, col0)``): a caller that adds this mixer's output to another's can then run both output matrices as
         one product."""
         ops = self.runtime.ops
-        qkv = proj = ops.linear(x, self.qkv_weight, self.qkv_bias_tensor, for_store=self._plain_store())
+        qkv = proj = ops.linear(x, self.qkv_weight, self.qkv_bias_tensor, for_store=self._plain_store)
         more, shape = {}, {}
         if self.conv_taps is not None:
             cache, held = cache
@@ -338,7 +340,7 @@ class GroupedQueryAttention(Mixer):
                 more["values"] = {"keep": kept}
             else:
                 more["values"] = {"blend": (ctx.carried[key], self.mix_weight)}
-        if not more and self.gate_name is None and scale == 1.0 and out is None:
+        if ctx.num_prefill_seqs == 0 and not more and self.gate_name is None and scale == 1.0 and out is None:
             attended = self._attend_projected(qkv, ctx, cache)
             if attended is not None:
                 return attended
@@ -356,7 +358,7 @@ class GroupedQueryAttention(Mixer):
         """A step of single tokens whose projection came as 32-bit partial sums: one launch adds them up, rotates, stores and
         attends.  ``None`` where the layer or the step asks for more than that launch does."""
         ops = self.runtime.ops
-        if (qkv.dim() != 3 or ctx.num_prefill_seqs != 0 or ctx.num_decode_seqs != ctx.num_tokens or not self._plain_rule()
+        if (qkv.dim() != 3 or ctx.num_decode_seqs != ctx.num_tokens or not self._plain_rule()
                 or not self.own_keys or not cache.writable
                 or not ops.mfma_attention_supported(self.runtime.dtype, self.head_dim, cache.block_size)
                 or not ops.decode_projected_supported(cache.k, cache.v)):
