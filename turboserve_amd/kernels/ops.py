@@ -2940,9 +2940,12 @@ class Ops:
         """The block product's grid for a prompt of few rows whose consumer adds up partial sums as well as it takes one result
         (the store of rotated heads), or None where one result is as soon there.  A narrow product as one range of K leaves most
         units idle: several ranges where the model puts them, their way to the consumer included, at seven tenths of one
-        range's time (us with the store, one result by the library or here / sums: 4,608 x 3,584 at 200 / 256 / 299 / 350 rows 36 / 39 /
-        33.9 / 33.4 against 26 / 28 / 29.9 / 31.5, at 400 31.6 against 33.0; 7,168 x 5,120 at 200 / 299 42 / 47 against 38 / 45, at
-        400 46 against 50)."""
+        range's time (us with the store, one result by the library or here / sums: 4,608 x 3,584 at 150 / 200 / 256 / 299 / 350 rows 26.1 / 36.2 /
+        41.1 / 29.0 / 32.3 against 23.1 / 22.3 / 24.9 / 27.2 / 28.3; 7,168 x 5,120 at 150 / 200 / 299 38.2 / 44.6 / 50.7 against 32.2 / 35.6 /
+        43.1; the library's kernels timed for the shape 22.5 / 26.6 / 28.8 / 29.3 / 31.2 and 37.0 / 43.2 / 47.8).  Of a matrix as small as 3,072 x
+        2,048 the sums' way to the store is long beside the product (at 150 / 256 / 400 rows 17.7 / 17.4 / 19.4 against 16.9 / 21.4 / 22.4), but the
+        host, which bounds a short prompt of such a model, is done with them sooner than with the library's call (a step of eight such layers, 222 /
+        300 tokens, 1,155 / 1,165 us with the library, 1,000 / 1,011 with sums)."""
         m, (n, k) = x.shape[0], weight.shape
         if not self.skinny_max_rows < m <= self.wide_default_rows or not self.block_supported(x, weight) or (bias is not None and bias.data_ptr() % 8):
             return None
