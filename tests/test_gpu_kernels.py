@@ -1028,6 +1028,10 @@ def test_attention_generic(ops, dtype, heads, kv_heads, dim, page, window):
     torch.testing.assert_close(got, case.expected, **tol(dtype))
 
 
+#: What the decode kernel's staged windows differ by: 24 pieces a key row, pages of a quarter of a window, of one, of two.
+DECODE_GEOMETRIES = [*ATTENTION_GEOMETRIES, (6, 2, 192, 16), (4, 1, 192, 64), (14, 2, 128, 8), (5, 1, 128, 32), (7, 1, 128, 64), (2, 2, 64, 128)]
+
+
 FLOAT32_RULES = {
     "causal": {},
     "window": {"window": 20},
@@ -1266,7 +1270,7 @@ def test_attention_generic_with_a_bias_by_distance(ops, dtype, window):
     torch.testing.assert_close(got[:, 0].reshape(-1), case.expected.view(-1, heads, dim)[:, 0].reshape(-1), **tol(dtype))
 
 
-@pytest.mark.parametrize("heads,kv_heads,dim,page", ATTENTION_GEOMETRIES)
+@pytest.mark.parametrize("heads,kv_heads,dim,page", DECODE_GEOMETRIES)
 @pytest.mark.parametrize("window", [None, 20, 300])
 def test_attention_decode_mfma(ops, heads, kv_heads, dim, page, window):
     contexts = [70, 1, 33, 600, 129, 32, 31, 257]
@@ -1279,7 +1283,7 @@ def test_attention_decode_mfma(ops, heads, kv_heads, dim, page, window):
     torch.testing.assert_close(out.float().cpu(), case.expected, **tol(torch.bfloat16))
 
 
-@pytest.mark.parametrize("heads,kv_heads,dim,page", ATTENTION_GEOMETRIES)
+@pytest.mark.parametrize("heads,kv_heads,dim,page", DECODE_GEOMETRIES)
 @pytest.mark.parametrize("window,splits", [(None, 1), (None, 3), (20, 2), (300, 1)])
 def test_attention_decode_from_projected_sums(ops, monkeypatch, heads, kv_heads, dim, page, window, splits):
     """Adding up, rotating, storing and attending in one launch against the store's launch and the attention's behind it: the

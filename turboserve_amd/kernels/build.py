@@ -60,7 +60,7 @@ MODULES: dict[str, tuple[str, ...]] = {
 #: Head sizes whose matrix-core attention module ``build_all`` compiles ahead of time: the
 #: common ones and those of the test configurations.  Any other multiple of 16 up to 256 is
 #: compiled when a model with that head size is first loaded.
-PREBUILT_HEAD_DIMS = (16, 32, 48, 64, 80, 96, 128, 256)
+PREBUILT_HEAD_DIMS = (16, 32, 48, 64, 80, 96, 128, 192, 256)
 
 
 def attention_module(head_dim: int) -> str:
