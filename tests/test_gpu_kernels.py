@@ -56,18 +56,46 @@ def test_rmsnorm_and_fused_residual(ops, dtype, tokens, hidden):
     torch.testing.assert_close(got, plain.rms_norm(total, w.float(), eps)[[tokens - 1, 0]], **tol(dtype))
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows,hidden", [(1, 4), (63, 1024), (3, 1028), (256, 2048), (2, 2052), (1, 4096), (5, 4100), (257, 2052), (512, 4096), (2, 8192),
-                                         (513, 2052), (600, 3584), (600, 5120), (1025, 1024), (1025, 1028), (1025, 2048), (513, 8192)])
+def short_norm_sums(dtype, rows, hidden):
+    """How many partial sums ``ts_add_rmsnorm``'s short kernels take of such rows (0: none, the general kernel does)."""
+    threads = 128
+    while threads < -(-hidden // 16):
+        threads *= 2
+    if rows <= 256:
+        threads = 1024
+    elif rows <= 512 and threads <= (128 if dtype == torch.float32 else 256):
+        threads *= 2
+    elif rows <= 1024 and hidden > 1024 and threads < 256:
+        threads = 256
+    items = -(-hidden // (4 * threads))
+    if threads == 1024:
+        return 16 // items if items <= 2 else 0
+    if dtype == torch.float32 or items < 2:
+        return 0
+    return 16 if (threads, items) == (512, 2) else 4
+
+
+SHORT_NORMS = [(torch.float32, 1, 4), (torch.float32, 63, 1024), (torch.float32, 3, 1028), (torch.float32, 256, 2048), (torch.float32, 2, 2052),
+               (torch.float32, 5, 4100), (torch.float32, 2, 8192)]
+SHORT_NORMS += [(torch.bfloat16, rows, hidden) for rows, hidden in (
+    (1, 4), (63, 1024), (3, 1028), (256, 2048), (2, 2052), (1, 4096), (5, 4100), (257, 2052), (512, 4096), (2, 8192), (300, 1028), (400, 2048), (300, 5120),
+    (513, 2052), (600, 3584), (600, 5120), (1025, 1024), (1025, 1028), (1025, 2048), (513, 8192))]
+
+
+@pytest.mark.parametrize("dtype,rows,hidden", SHORT_NORMS)
 def test_short_norms_have_the_bits_of_the_general_ones(ops, dtype, rows, hidden):
-    """The short norm kernels take up to 16 (8; 4 in a long step) partial sums at the edges of their threads and items; as many again that are
+    """The short norm kernels take up to 16 (8, 4) partial sums at the edges of their threads and items; as many again that are
     zero, more than they take, go to the general kernels, which add them up in the same order."""
+    most = short_norm_sums(dtype, rows, hidden)
+    assert most > 0
     g = torch.Generator().manual_seed(rows + hidden)
     residual = torch.randn(rows, hidden, generator=g).to(DEV)
     w, b = ((1 + 0.1 * torch.randn(2, hidden, generator=g)).to(dtype).to(DEV))
     picked = torch.tensor([rows - 1, 0], dtype=torch.int32, device=DEV)
     layer_norms = [{"norm": (w, b, 1e-5)}, {"norm": (w, None, 1e-5)}, {"pending_norm": (w, b, 1e-5, 0.5)}]
     for splits in (1, 2, 3, 5, 8, 9, 16):
+        if splits > most:
+            break
         some = torch.randn(splits, rows, hidden, generator=g).to(DEV)
         more = torch.cat([some, torch.zeros(17 - splits, rows, hidden, device=DEV)])
         calls = [lambda into, parts, at: ops.add_rmsnorm(into, parts, w, 1e-6, at)]

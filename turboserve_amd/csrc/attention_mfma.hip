@@ -207,13 +207,14 @@ struct ValueFrags {
 struct WindowFrags : KeyFrags, ValueFrags {};
 
 // Issue the loads of window `w` (keys outside lo..last: see live_key).  ONCE: bit 0, the keys,
-// bit 1, the values are read with non-temporal loads (by this wavefront alone: a decode step
-// reads every cached key once).  A decode step wants that for the values only (DECODE_ONCE): an
+// bit 1, the values are read with non-temporal loads (a decode step reads every cached key once, or
+// once for each sixteen query heads of its KV head).  Loaded as operands, which the decode kernel does for head
+// sizes that 64 does not divide and for pages between 16 bytes, the values alone want it (DECODE_ONCE): an
 // instruction of theirs reads runs of 512 bytes, one of the keys' 64 bytes of each of 16 rows, so
 // two instructions share every 128-byte line, and marking those costs more than it gains
-// (7B heads, attention and combine, plain / keys / values / both: 8 requests at 8,192 tokens
-// 30.7 / 30.5 / 29.3 / 29.5 us, 64 at 8,192 188 / 177 / 172 / 171, 64 at 640 22.8 / 23.4 / 21.8 /
-// 23.4).
+// (measured where all heads were loaded so, a wavefront per stretch of keys: 7B heads, attention and combine, plain / keys / values /
+// both: 8 requests at 8,192 tokens 30.7 / 30.5 / 29.3 / 29.5 us, 64 at 8,192 188 / 177 / 172 / 171, 64 at 640 22.8 / 23.4 / 21.8 /
+// 23.4).  Staged windows (Stage::fetch) read whole lines of both.
 constexpr int DECODE_ONCE = 2;
 template <int ONCE = 0>
 __device__ __forceinline__ void load_window(WindowFrags& f, const PageGeometry& g, const WindowPages& wp, int w, int lo, int last,
@@ -567,7 +568,9 @@ struct Stage {
     return at;
   }
 
-  // The window's keys or values into `to`.
+  // The window's keys or values into `to`: whole lines, each read by one instruction of this workgroup, so keys and values alike are
+  // marked non-temporal (which leaves them in the die's L2 long enough for another tile of query heads that reads them at the
+  // same time: tiled_place).
   template <bool VALUES>
   __device__ __forceinline__ void fetch(lds_u16* to, const PageGeometry& g, const Place& place) const {
 #pragma unroll
@@ -781,7 +784,7 @@ decode_kernel(const int* __restrict__ context_lens, const int* __restrict__ quer
     }
     auto take = [&](WindowFrags& f) __attribute__((always_inline)) {
       if (w < lo || w + WINDOW_KEYS > ctx) clear_stale_values(f, w, lo, p, group);
-  if (PROJECTED && w + WINDOW_KEYS > p) {
+      if (PROJECTED && w + WINDOW_KEYS > p) {
         put_new_key(f, new_key, w, p, lane16, group);
         put_new_value(f, new_value, w, p, lane16, group);
       }
