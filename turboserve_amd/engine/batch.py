@@ -340,7 +340,8 @@ class StepContext:
     max_prefill_context_len: int = 0
     max_decode_context_len: int = 0
     #: The longest context of the single-token requests as a one-element device tensor.  In a
-    #: recorded step the host lengths above are upper bounds (the shape's) and this is the truth.
+    #: recorded step the host lengths above are upper bounds (the shape's) and this is the truth, for a part whose kernels
+    #: size their launch's shares by it (this engine's attention kernels divide each request by its own length).
     max_decode_context_dev: torch.Tensor | None = None
     #: A recorded step: replayed with other data than it was recorded with, so a part may use
     #: nothing about the step but its shape, the fields above and what ``derive`` refuses there.

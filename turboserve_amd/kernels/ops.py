@@ -1836,7 +1836,6 @@ class Ops:
         scale: float,
         window: int | None,
         max_context: int,
-        max_context_dev: torch.Tensor | None = None,
         softcap: float = 0.0,
         projected: tuple | None = None,
         shares: int = 1,
@@ -1844,8 +1843,7 @@ class Ops:
         """Matrix-core attention for the single-token requests ``seq_begin .. seq_begin +
         requests - 1`` of the step; writes their rows of ``out [T, heads * D]``.  ``max_context``
         (host-known) bounds their context lengths and fixes over how many workgroups a request's keys are
-        divided; ``max_context_dev`` (one int32 on the device, at most ``max_context``) may name the step's true
-        longest context (every request divides its own keys, read from the device).
+        divided (every request divides its own keys, by its length on the device).
 
         ``projected = (cos, sin, slots, max_position)``: ``q`` is the fused projection's partial sums ``[S, T, (heads + 2
         kv_heads) D]`` (32-bit); the launch adds them up, rotates queries and keys, stores the new keys and values at
@@ -1853,8 +1851,7 @@ class Ops:
 
         ``shares`` (:meth:`decode_shares`): what the requests' own lengths, which ``max_context`` does not tell, make of a
         request's keys where requests and KV heads alone give every compute unit a workgroup."""
-        _gpu(out, q, k_pages, v_pages, block_table, query_start_loc, context_lens, max_context_dev)
-        _i32(max_context_dev, "max_context_dev")
+        _gpu(out, q, k_pages, v_pages, block_table, query_start_loc, context_lens)
         _i32(block_table, "block_table")
         _i32(query_start_loc, "query_start_loc")
         _i32(context_lens, "context_lens")

@@ -374,7 +374,7 @@ class GroupedQueryAttention(Mixer):
         out = ops.rows_buffer(ctx.num_tokens, self.out_size, self.runtime.dtype, qkv.device)
         ops.attention_decode(
             out, qkv, 0, cache.k, cache.v, table, ctx.query_start_loc, ctx.context_lens, 0, ctx.num_decode_seqs, self.num_heads,
-            self.scale, self.window, min(ctx.max_decode_context_len, table.shape[1] * cache.block_size), ctx.max_decode_context_dev,
+            self.scale, self.window, min(ctx.max_decode_context_len, table.shape[1] * cache.block_size),
             softcap=self.softcap, projected=(*tables, ctx.slot_mapping[cache.group], ctx.max_context_len - 1), shares=self._decode_shares(ctx))
         return out
 
@@ -423,7 +423,7 @@ class GroupedQueryAttention(Mixer):
                     out, qkv, q_stride, cache.k, cache.v, table, ctx.query_start_loc, ctx.context_lens,
                     ctx.num_prefill_seqs, ctx.num_decode_seqs, self.num_heads, self.scale, self.window,
                     min(ctx.max_decode_context_len, table.shape[1] * cache.block_size),
-                    ctx.max_decode_context_dev, softcap=self.softcap, shares=self._decode_shares(ctx),
+                    softcap=self.softcap, shares=self._decode_shares(ctx),
                 )
             return out
         if ops.tiled_attention_supported(qkv.dtype, self.head_dim, self.value_dim, cache.block_size, q_stride):
