@@ -442,9 +442,9 @@ static void launch_add_rmsnorm(void* y, float* residual, const void* pending, in
   if constexpr (!FLOAT32) {
     // A prompt's rows: in the general kernel a thread's items are behind a branch each, and the compiler waits for the loads of one
     // before it asks for the next's.  (Steps, us: 2,048 tokens, 56 norms of rows of 3,584, 24,090 -> 23,708; 2,048 rows of 5,120, 96 norms,
-    // 50,260 -> 49,040.)  512 threads of two items hold sixteen sums' pieces in 128 registers; steps of more rows, whose products leave four
-    // sums and fewer, need no more than four.  (Three and four items of rows at 257 to 512 with more sums than that stay general:
-    // not built, not measured.)
+    // 50,260 -> 49,040.)  512 threads of two items hold sixteen sums' pieces in 128 registers; the other forms are built for four sums,
+    // which most products of more rows leave.  (More, of a long K over a narrow matrix, 3,584 x 18,944 at 641 to 768 rows six, and of three
+    // and four items at 257 to 512 rows, stay general: not built, not measured.)
     if (plain && threads < 1024 && items >= 2 && splits <= (threads == 512 && items == 2 ? 16 : 4)) {
 #define TS_NORM_THREADS(THREADS)                  \
   do {                                            \
