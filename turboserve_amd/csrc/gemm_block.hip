@@ -15,14 +15,14 @@
 // With one wavefront on a SIMD nothing hides its waits, so nothing waits: a step's activation fragments are
 // read from LDS during the step before it, its weight fragments a tile's instructions after the last use of
 // their registers, and the first ones of the next iteration behind the barrier that ends this one's reads,
-// while most of its second step is still to be multiplied; loads are issued two to five iterations ahead, one beside each tile's
-// instructions (issued in one go they held the matrix instructions up).
+// while most of its second step is still to be multiplied; loads are issued two to five iterations ahead.  Loads and reads stand one
+// by one between matrix instructions (in one go they held them up).
 // Measured, microseconds, against the better of gemm_wide and the library's default kernel (with the kernel that reads or
 // makes the result: SwiGLU, or the norm that takes the partial sums), at 299 / 509 / 2,048 rows: gate|up [37888, 3584] 85 / 139 /
 // 441 against 126 / 158 / 560 (1.26 PFLOP/s), down [3584, 18944] 58 / 79 / 246 against 111 / 90 / 291, o [3584, 3584] 26 / 30 / 73
-// against 35 / 34 / 77, q|k|v [4608, 3584] 27 / 28 / 59 against 23 / 31 / 62.  An iteration of 256 x 256 takes 1.15 us where
-// half the compute units have a workgroup and 1.4 where all do (the matrix instructions 0.85 at the full clock); a
-// workgroup's start takes 2 us and its stores 4 (gated 9).
+// against 35 / 34 / 77, q|k|v [4608, 3584] 27 / 28 / 59 against 23 / 31 / 62.  An iteration of 256 x 256 takes 1.01 us where
+// half the compute units have a workgroup and 1.32 where all do (the matrix instructions 0.85 at the full clock of 2.4 GHz; with every unit
+// at work the card holds 1.7 to 1.8); a workgroup's start takes 2 us and its stores 4 (gated 9).
 // A decode step's product is bound by reading the weights; 160 weight rows by 64 activation rows a workgroup, the weights
 // non-temporal, take gate|up at 64 rows in 44.1 us (gemm_wide 47.5), 128 rows down in 26.6 (28.6), q|k|v in 11.5 (12.0), o in 10.4
 // (11.1); at 128 rows 50 (60), 33 (37), 14.5 (15.3), 13.7 (14.1).
@@ -158,18 +158,29 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   // once.  Wavefront v takes the eights v, v + 4, ... of the weight rows and of the activation rows (so a lane's key is
   // the same for all of them).  Loads beyond a buffer's end (rows beyond N or M, whose results are not stored) bring zeros.
   const int row0 = 8 * wave + (lane >> 3), piece = (lane & 7) ^ ((row0 >> 1) & 7);
-  const __amdgpu_buffer_rsrc_t wbuf = block_buffer(w + (size_t)n_base * k, ((size_t)(min(n - n_base, NT) - 1) * k + k) * 2);
-  const __amdgpu_buffer_rsrc_t xbuf = block_buffer(x + (size_t)m_base * x_stride, ((size_t)(min(m - m_base, XR) - 1) * x_stride + k) * 2);
-  // A row's place is in the lane's offset, the place in K in the wavefront's: what is compared with the buffer's size is
-  // the first against the size less the second, which is never below 0.
-  int woff = (row0 * k + 8 * piece) * 2, xoff = (row0 * (int)x_stride + 8 * piece) * 2;
-  auto load_w = [&](int j, int off, int it, int slot) __attribute__((always_inline)) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, to + (slot * NT + 32 * j + 8 * wave) * ROW, 16, off + j * 64 * k, it * (BLOCK_DEPTH * 2), 0,
+  const uint16_t *const w_rows = w + (size_t)n_base * k, *const x_rows = x + (size_t)m_base * x_stride;
+  const size_t w_bytes = ((size_t)(min(n - n_base, NT) - 1) * k + k) * 2, x_bytes = ((size_t)(min(m - m_base, XR) - 1) * x_stride + k) * 2;
+  // A row's place is in the lane's offsets, one for every eight rows that it takes part in, the place in K in the wavefront's:
+  // what is compared with the buffer's size is the first against the size less the second, which is never below 0.  The offsets stay
+  // in registers (the asm hides that they could be added up again: a load with its addition took 28 cycles of a wavefront that the matrix
+  // cores had nothing to do in, without it 14).
+  int woff[TN], xoff[TM];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    woff[j] = ((row0 + 32 * j) * k + 8 * piece) * 2;
+    asm volatile("" : "+v"(woff[j]));
+  }
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    xoff[j] = ((row0 + 32 * j) * (int)x_stride + 8 * piece) * 2;
+    asm volatile("" : "+v"(xoff[j]));
+  }
+  auto load_w = [&](int j, __amdgpu_buffer_rsrc_t buf, int at, int slot) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, to + (slot * NT + 32 * j + 8 * wave) * ROW, 16, woff[j], at, 0,
                                              ONCE ? 2 : 0);  // non-temporal where one tile of activation rows reads them
   };
-  auto load_x = [&](int j, int off, int it, int slot) __attribute__((always_inline)) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(xbuf, to + (RW * NT + slot * XR + 32 * j + 8 * wave) * ROW, 16, off + j * 64 * (int)x_stride, it * (BLOCK_DEPTH * 2),
-                                             0, 0);
+  auto load_x = [&](int j, __amdgpu_buffer_rsrc_t buf, int at, int slot) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, to + (RW * NT + slot * XR + 32 * j + 8 * wave) * ROW, 16, xoff[j], at, 0, 0);
   };
 
   // This lane's piece of step s (32 of K) in every row it reads.
@@ -200,10 +211,8 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
     for (int b = 0; b < TM; ++b) acc[a][b] = start;
   }
   u32x4 xf[2][TM], wf[TN];
-  auto tile = [&](int s, int a, int from, int end) __attribute__((always_inline)) {
-#pragma unroll
-    for (int b = from; b < end; ++b)
-      acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(block_bf16x8(wf[a]), block_bf16x8(xf[s][b]), acc[a][b], 0, 0, 0);
+  auto multiply = [&](int s, int a, int b) __attribute__((always_inline)) {
+    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(block_bf16x8(wf[a]), block_bf16x8(xf[s][b]), acc[a][b], 0, 0, 0);
   };
 
   // Iteration i of the range: its weight rows lie in slot i % RW of their ring, its activation rows in slot i % RX of theirs.
@@ -212,18 +221,19 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   // loop as well (2,048 rows, 7,168 x 5,120 with 256 x 256 115 -> 129 us, 27,648 x 5,120 gated with 256 x 192 467 -> 474).  There the
   // loads go out in every iteration, those past the end past the buffers' ends too.
   constexpr bool PEELED = TN * TM <= 40;
-  const int outside = (int)0x80000000;
   const int count = last - first;
-  auto step = [&](int i) __attribute__((always_inline)) { return first + (PEELED ? i : min(i, count - 1)); };
-  auto at = [&](int off, int i) __attribute__((always_inline)) { return PEELED || i < count ? off : outside; };
+  // The buffers and the place in them that iteration i reads from: an empty buffer past the end.
+  auto from_w_rows = [&](int i) __attribute__((always_inline)) { return block_buffer(w_rows, PEELED || i < count ? w_bytes : 0); };
+  auto from_x_rows = [&](int i) __attribute__((always_inline)) { return block_buffer(x_rows, PEELED || i < count ? x_bytes : 0); };
+  auto place_of = [&](int i) __attribute__((always_inline)) { return PEELED || i < count ? (first + i) * (BLOCK_DEPTH * 2) : 0; };
 #pragma unroll
   for (int s = 0; s < RX; ++s) {
     if (PEELED && s >= count) continue;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-      if (s < RW - 1) load_w(j, at(woff, s), step(s), s);
+      if (s < RW - 1) load_w(j, from_w_rows(s), place_of(s), s);
 #pragma unroll
-    for (int j = 0; j < TM; ++j) load_x(j, at(xoff, s), step(s), s);
+    for (int j = 0; j < TM; ++j) load_x(j, from_x_rows(s), place_of(s), s);
   }
   if (PEELED) block_wait_first<Ring, RX - 1>(count - 1);
   else block_wait<Ring::left_first(RX)>();
@@ -233,37 +243,48 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   for (int a = 0; a < TN; ++a) wf[a] = read_w(0, 0, a);
 
   // Top of a round: slots ws and xs hold iteration `it` complete, xf[0] and wf its step 0; the loads of the iterations
-  // behind it are on their way.  The order below is the one that is issued: a few accesses, then matrix
-  // instructions, which run while the next accesses issue.
+  // behind it are on their way.  The order below is the one that is issued: matrix instructions with at most one access or two between
+  // them.  A matrix instruction lasts as long as four others take to issue, so what stands alone behind one costs nothing; a
+  // read, a load and their addresses in one go between the tiles did (an iteration of 256 x 256: 2,650 cycles, 2,450 one by one, 2,320
+  // with the offsets kept, of which the matrix instructions are 2,048; microseconds where half of the compute units have a workgroup
+  // 1.11 -> 1.01, where all do, on a clock that falls the more the busier they are, 1.39 -> 1.32).
 #define TS_PIN __builtin_amdgcn_sched_barrier(0)
   constexpr int EARLY = TN / 2;                     // tiles of step 0 beside which step 1's activations are read
   constexpr int FREE = TN > 4 ? 2 : 1;              // the barrier stands before this tile of step 1
   constexpr int BEHIND = TM + FREE;                 // fragments of the next iteration read behind it, with those of each tile done
   int ws = 0, xs = 0;
+  // Access i of n beside a tile's TM instructions stands behind this one of them.
+  auto behind = [](int i, int n) __attribute__((always_inline)) { return (2 * i + 1) * TM / (2 * n); };
   // W_LOADS, X_LOADS: there is an iteration it + RW - 1, it + RX.
   auto iteration = [&](int it, auto W_LOADS, auto X_LOADS) __attribute__((always_inline)) {
-    // The offsets of the other rows are added up in each iteration: kept, they would take registers that the sums need.
-    asm volatile("" : "+v"(woff), "+v"(xoff));
-    const int next_w = step(it + RW - 1), next_x = step(it + RX);
-    const int from_w_at = at(woff, it + RW - 1), from_x_at = at(xoff, it + RX);
+    const __amdgpu_buffer_rsrc_t wbuf = from_w_rows(it + RW - 1), xbuf = from_x_rows(it + RX);
+    const int next_w = place_of(it + RW - 1), next_x = place_of(it + RX);
     const int free_w = ws == 0 ? RW - 1 : ws - 1, free_x = xs;
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
-      TS_PIN;
-      if constexpr (W_LOADS) load_w(a, from_w_at, next_w, free_w);
-      TS_PIN;
-      tile(0, a, 0, TM / 2);
-      TS_PIN;
+      // A load amid the reads of step 1's activations.
+      const int x_first = min(a * TM / EARLY, TM), x_last = min((a + 1) * TM / EARLY, TM), n = 1 + x_last - x_first;
 #pragma unroll
-      for (int b = a * TM / EARLY; b < (a + 1) * TM / EARLY && b < TM; ++b) xf[1][b] = read_x(xs, 1, b);
-      TS_PIN;
-      tile(0, a, TM / 2, TM);
-      TS_PIN;
+      for (int b = 0; b < TM; ++b) {
+        multiply(0, a, b);
+        TS_PIN;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+          if (behind(i, n) != b) continue;
+          if (i == n / 2) {
+            if constexpr (W_LOADS) load_w(a, wbuf, next_w, free_w);
+          } else {
+            const int j = x_first + i - (i > n / 2);
+            xf[1][j] = read_x(xs, 1, j);
+          }
+          TS_PIN;
+        }
+      }
       wf[a] = read_w(ws, 1, a);
+      TS_PIN;
     }
 #pragma unroll
     for (int a = 0; a < TN; ++a) {
-      TS_PIN;
       if (a == FREE) {
         // This wavefront has read all of iteration `it` (its fragments are in registers) and its loads of it + 1 have landed;
         // behind the barrier both hold for the workgroup.
@@ -276,21 +297,32 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
         ws = ws + 1 == RW ? 0 : ws + 1;
         xs = xs + 1 == RX ? 0 : xs + 1;
         asm volatile("" : "+s"(ws), "+s"(xs));  // the compiler, for which no load writes what it reads, sees new addresses
+        TS_PIN;
       }
-      if (a >= FREE) {
+      // Reads and loads in turn.
+      const int tiles = TN - FREE, done = a < FREE ? 0 : a - FREE, end = a < FREE ? 0 : done + 1;
+      const int r_first = done * BEHIND / tiles, l_first = done * TM / tiles, loads = end * TM / tiles - l_first;
+      const int n = end * BEHIND / tiles - r_first + loads;
 #pragma unroll
-        for (int j = (a - FREE) * BEHIND / (TN - FREE); j < (a - FREE + 1) * BEHIND / (TN - FREE); ++j) {
-          if (j < FREE) wf[j] = read_w(ws, 0, j);
-          else xf[0][j - FREE] = read_x(xs, 0, j - FREE);
+      for (int b = 0; b < TM; ++b) {
+        multiply(1, a, b);
+        TS_PIN;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+          if (behind(i, n) != b) continue;
+          const int l = i * loads / n;
+          if ((i + 1) * loads / n > l) {
+            if constexpr (X_LOADS) load_x(l_first + l, xbuf, next_x, free_x);
+          } else {
+            const int j = r_first + i - l;
+            if (j < FREE) wf[j] = read_w(ws, 0, j);
+            else xf[0][j - FREE] = read_x(xs, 0, j - FREE);
+          }
+          TS_PIN;
         }
-#pragma unroll
-        for (int j = (a - FREE) * TM / (TN - FREE); j < (a - FREE + 1) * TM / (TN - FREE); ++j)
-          if constexpr (X_LOADS) load_x(j, from_x_at, next_x, free_x);
       }
-      TS_PIN;
-      tile(1, a, 0, TM);
-      TS_PIN;
       if (a >= FREE) wf[a] = read_w(ws, 0, a);
+      TS_PIN;
     }
   };
 #undef TS_PIN
