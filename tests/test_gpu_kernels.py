@@ -551,7 +551,7 @@ def test_gemm_stream_every_tile_and_grid(ops, tile, m, n, k):
     assert bool(((picked.double().sum(0).cpu() - want).abs() <= bound).all())
 
 
-BLOCK_TILES = [(8, 8), (8, 6), (8, 5), (5, 10), (5, 8), (4, 8), (4, 5), (4, 4)]
+BLOCK_TILES = [(8, 8), (8, 6), (8, 5), (5, 10), (5, 8), (4, 8), (4, 5), (4, 4), (7, 8), (6, 8), (7, 4)]
 BLOCK_ONE_TILES = [(a, b) for b in (1, 2) for a in (8, 5, 4, 2)] + [(8, 4), (5, 4), (2, 4)]  # one tile of activation rows
 BLOCK_SIZES = [(1, 16, 64, 1), (17, 304, 448, 3), (33, 272, 128, 2), (65, 1040, 192, 1), (128, 528, 320, 5), (129, 272, 64, 1), (257, 48, 128, 2),
                (321, 528, 192, 3), (700, 1040, 448, 2)]
@@ -653,7 +653,7 @@ def test_gemm_block_gates_of_every_size(ops, m, tn, tm):
 
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("m,n,first,tiles,rest", [(300, 1040, 512, (8, 8), (5, 8)), (33, 784, 768, (8, 6), (4, 4)), (129, 528, 16, (8, 5), (5, 10)),
-                                                  (257, 2064, 1792, (8, 8), (4, 5))])
+                                                  (257, 2064, 1792, (8, 8), (4, 5)), (270, 912, 448, (7, 8), (6, 8)), (140, 1008, 768, (6, 8), (7, 4))])
 def test_a_product_in_two_launches_is_the_product_in_one(ops, m, n, first, tiles, rest, gated):
     """Whole rounds of one tile and another tile for the rest of the weight rows write, bit for bit, what one tile writes, and
     nothing beside it; the plan of a long prompt's product has such a rest and covers it."""

@@ -89,6 +89,20 @@ def test_short_ranges_of_partial_sums_run_the_wide_product():
         assert picked(m, n, k) == "block", (m, n, k)
 
 
+def test_tiles_of_224_weight_rows_fill_the_rounds_of_several_ranges():
+    """Where a plan of several ranges takes them, nine tenths of its rounds of workgroups are full; at 2,048 rows they take the narrow matrices
+    that 16 tiles of 224 cover."""
+    ops = Planner()
+    assert ops._block_plan(2048, 3584, 18944, "sums") == (148, 2, 7, 8) and ops._block_plan(2048, 3584, 3584, "sums") == (56, 1, 7, 4)
+    assert ops._block_plan(2048, 7168, 5120, "one") == (80, 1, 7, 8)
+    for n, k in ((3584, 18944), (3584, 3584), (5120, 13824), (2048, 8192), (7168, 5120), (4608, 3584)):
+        for m in range(129, 2049, 31):
+            for kind in ("sums", "store"):
+                _, splits, tn, tm = ops._block_plan(m, n, k, kind)
+                workgroups = -(-n // 224) * -(-m // (32 * tm)) * splits
+                assert tn != 7 or splits == 1 or 10 * workgroups >= 9 * 256 * -(-workgroups // 256), (m, n, k, kind)
+
+
 def test_32_bit_attention_is_asked_only_for_what_it_takes():
     """Pages of 24 keys and pages or rows that 16-byte accesses do not fit stay with the kernel that takes any geometry."""
     ops = Planner()

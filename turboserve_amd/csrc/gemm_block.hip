@@ -465,10 +465,13 @@ extern "C" int ts_gemm_block(float* partial, void* out, const void* x, long x_st
     if (plain) TS_BLOCK_MODE(TN, TM, 2, ONCE);       \
     TS_BLOCK_MODE(TN, TM, 3, ONCE);                  \
   }
-  const bool once = m <= 32 * tm && tm <= 4;
+  const bool once = m <= 32 * tm && tm <= 4 && tn != 7;
   TS_BLOCK(8, 8, false)
   TS_BLOCK(8, 6, false)
   TS_BLOCK(8, 5, false)
+  TS_BLOCK(7, 8, false)
+  TS_BLOCK(7, 4, false)
+  TS_BLOCK(6, 8, false)
   TS_BLOCK(5, 10, false)
   TS_BLOCK(5, 8, false)
   TS_BLOCK(4, 8, false)

@@ -2245,7 +2245,8 @@ class Ops:
     #: The block product's tiles (in 32 weight rows, 32 activation rows) and what an iteration of
     #: 64 of K takes a compute unit with each, in microseconds: the slope over K of products at 144
     #: to 2,048 rows that give every compute unit a workgroup.
-    _BLOCK_TILES = {(8, 8): 1.24, (8, 6): 0.99, (8, 5): 0.86, (5, 10): 1.07, (5, 8): 0.88, (4, 8): 0.76, (4, 5): 0.54, (4, 4): 0.50}
+    _BLOCK_TILES = {(8, 8): 1.24, (7, 8): 1.14, (8, 6): 0.99, (6, 8): 1.01, (8, 5): 0.86, (5, 10): 1.07, (5, 8): 0.88, (4, 8): 0.76, (7, 4): 0.73, (4, 5): 0.54,
+                    (4, 4): 0.50}
 
     @staticmethod
     def block_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -2265,7 +2266,10 @@ class Ops:
         its iterations and six more (first loads, stores) at the tile's pace, a gated
         result the unit's time, and partial sums of several ranges their way to the norm, 3.6
         bytes per nanosecond.  Against every tile with 1 to 16 ranges, timed for the matrices of six shapes (K 2,048 to 18,944) at 144 to
-        2,048 rows, the plan's grid takes 1% more than the fastest on average.
+        2,048 rows, the plan's grid takes 1% more than the fastest on average.  The tiles of 192 and 224 weight rows fill rounds that the others
+        leave in part empty (us: 3,584 x 18,944 at 2,048 rows, two ranges, 256 workgroups of 224 x 256 195 against 224 of 256 x 256 210, 3,584 x
+        3,584 of 224 x 128 45 against 224 of 128 x 256 47, 7,168 x 5,120 107 against 113; 57 of 14 matrices' grids at 129 to 2,048 rows changed with
+        them, 5% sooner on average); as several ranges those of 224 are taken only where they do fill them, to nine tenths.
         ``kind``: "sums" (partial sums may stay), "store" (up to four of them, what the store of heads asks for at once), "one"
         (one bfloat16 result), "gated"."""
         key = (m, n, k, kind)
@@ -2279,6 +2283,9 @@ class Ops:
                 per_split = -(-iters // want)
                 splits = -(-iters // per_split)
                 if splits != want:
+                    continue
+                workgroups = -(-n // (32 * tn)) * -(-m // (32 * tm)) * splits
+                if tn == 7 and splits > 1 and 10 * workgroups < 9 * self.compute_units * -(-workgroups // self.compute_units):
                     continue
                 cost = self._block_cost(m, n, k, (per_split, splits, tn, tm), kind == "gated")
                 if best is None or cost < best[0]:
