@@ -307,6 +307,36 @@ def test_gemm_plain_is_chains_of_fused_multiply_adds(ops, dtype, k, values):
                     assert got[i, j].item() == float(value), (rows, cols, i, j)
 
 
+@pytest.mark.parametrize("tile", [2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("m,k", [(1, 32), (64, 64), (65, 96), (130, 288), (527, 1056)])
+def test_gemm_plain_block_every_tile(ops, tile, m, k):
+    """Tiles of 64 x 16 tile outputs of a 32-bit product, weight rows one tile short of whole, whole, and four beyond, one slice of K to four ranges
+    of nine, rows apart: the bits of the layout that takes sixteen rows, the bits of a loop of fmaf also among denormals, and nothing
+    of what lies behind a row of x or in another row of the weights."""
+    from turboserve_amd.kernels.ops import KernelError
+
+    g = torch.Generator().manual_seed(tile + m)
+    x = torch.full((m, k + 8), float("nan"), device=DEV)[:, :k].copy_(torch.randn(m, k, generator=g))
+    for n in (16 * tile - 12, 32 * tile, 32 * tile + 4):
+        w, b = torch.randn(n, k, generator=g).to(DEV), torch.randn(n, generator=g).to(DEV)
+        want = torch.cat([ops.gemm_plain(rows, w, b) for rows in x.split(16)])
+        assert torch.equal(ops.gemm_plain(x, w, b, tile=tile), want)
+        assert torch.equal(ops.gemm_plain(x, w, tile=tile), torch.cat([ops.gemm_plain(rows, w) for rows in x.split(16)]))
+        w[n // 2] = float("nan")
+        got = ops.gemm_plain(x, w, b, tile=tile)
+        assert bool(got[:, n // 2].isnan().all())
+        got[:, n // 2] = want[:, n // 2]
+        assert torch.equal(got, want)
+    x = torch.ldexp(torch.randn(m, k, generator=g), torch.randint(-70, -64, (m, k), generator=g))
+    w = torch.ldexp(torch.randn(16, k, generator=g), torch.randint(-72, -65, (16, k), generator=g))
+    got = ops.gemm_plain(x.to(DEV), w.to(DEV), tile=tile).cpu()
+    for i, j in ((0, 0), (m - 1, 15), (m // 2, 7)):
+        assert got[i, j].item() == float(chains_of_fused_multiply_adds(x[i].tolist(), w[j].tolist(), 0.0))
+    for refused in (x[:, :-1], x[:, 4:]):  # a K that is not whole slices
+        with pytest.raises(KernelError):
+            ops.gemm_plain(refused.contiguous().to(DEV), w[:, : refused.shape[1]].contiguous().to(DEV), tile=tile)
+
+
 def test_gemm_plain_of_very_many_rows(ops):
     """2,097,121 rows against a narrow matrix, one more than tiles of 32 rows have places in a grid: a layout of larger tiles
     takes them.  Beyond 65,535 tiles of 64 rows the product refuses, as it always has."""

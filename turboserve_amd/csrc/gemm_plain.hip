@@ -13,9 +13,11 @@
 // multiply-adds allow, and a few rows against a long K get four times the wavefronts one chain would.
 //
 // Microseconds at the 7B shape, one chain of vector multiply-adds (64 x 64 tiles; up to 32 rows one output a thread)
-// -> these: gate|up at 8 / 64 / 500 rows 194 -> 88, 765 -> 208, 3,048 -> 1,142 (119 TFLOP/s); down 220 -> 47, 3,402 -> 155,
-// 3,365 -> 724; o 35 -> 13, 581 -> 29, 581 -> 139; q|k|v 41 -> 18, 579 -> 43, 638 -> 195; the head at 8 rows 637 -> 330.
+// -> these: gate|up at 8 / 64 / 500 rows 194 -> 88, 765 -> 152, 3,048 -> 961 (141 TFLOP/s); down 220 -> 47, 3,402 -> 119,
+// 3,365 -> 486; o 35 -> 12, 581 -> 25, 581 -> 98; q|k|v 41 -> 16, 579 -> 32, 638 -> 121; the head at 8 rows 637 -> 320.
 #include "common.hpp"
+
+#include <type_traits>
 
 namespace {
 
@@ -51,6 +53,8 @@ struct Quad<bf16_t> {
                     __uint_as_float(hi & 0xffff0000u)};
   }
 };
+
+inline long ceil_of(long a, long b) { return (a + b - 1) / b; }
 
 // The length of a range of K, the same for every layout: a function of K alone.
 __host__ __device__ constexpr int range_of(int k) { return (((k + 3) / 4 + 63) / 64) * 64; }
@@ -667,34 +671,249 @@ int launch_stream(void* y, const void* x, const void* w, const void* bias, int m
   return ts_launch_status();
 }
 
-inline long ceil_of(long a, long b) { return (a + b - 1) / b; }
+// ---------------------------------------------------------------------------------------------
+// Many 32-bit rows whose K is a multiple of 32: a workgroup of four wavefronts owns 64 activation rows by 16 NT weight rows, a
+// wavefront NT tiles of v_mfma_f32_16x16x4_f32.  Bound by the matrix cores, and by everything that a wavefront has its vector unit do
+// meanwhile: a 32-bit matrix instruction holds it (32 cycles alone, 51 with two vector instructions behind each, 70 with seven, where a
+// bfloat16 one takes three beside it).  So the loop has none: operands go straight from memory to LDS, SLOTS slices of 32 k ahead, their
+// offsets kept; a fragment is read from LDS in the order of k, an element of one k of sixteen rows a time (two tiles an instruction), through eight kept
+// addresses; slots are numbers known to the compiler.
+// Piece p (16 bytes) of row r lies at position p ^ (r / 2 % 8) of the row's eight: the elements that an instruction reads of sixteen rows touch
+// every bank once.  The same chains, bit for bit.
+template <int NT>
+struct PlainRing {
+  static constexpr int SLICE = 32, ROWS = 16 * NT + 64, SLOT = ROWS * SLICE;  // floats of a slice
+  static constexpr int WLOADS = (NT + 1) / 2, XLOADS = 2, LOADS = WLOADS + XLOADS;  // of a wavefront, eight rows each
+  static constexpr int SLOTS = 4;
+  static constexpr size_t BYTES = (size_t)SLOTS * SLOT * 4;
+  static_assert(NT >= 2 && (SLOTS - 1) * LOADS < 64 && BYTES <= 160 * 1024, "the ring must fit the LDS of a compute unit, its loads vmcnt");
+};
+
+// `to` and `from` are the same memory: __restrict__ keeps the compiler from waiting for every load in flight before every
+// read.  What orders them: every read's address has come through the asm behind the wait for its loads (at), and a slot is filled again behind the
+// barrier before which every wavefront has what it reads of it in registers.  An edit has to keep both.
+template <int NT>
+__device__ __forceinline__ void plain_block(lds_f32* __restrict__ to, const lds_f32* __restrict__ from, float* __restrict__ y,
+                                            const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, int m,
+                                            int n, int k, long x_stride, long y_stride, int m_tiles, int n_tiles) {
+  typedef PlainRing<NT> R;
+  constexpr int SLICE = R::SLICE, SLOT = R::SLOT, SLOTS = R::SLOTS, WLOADS = R::WLOADS, XLOADS = R::XLOADS, FRAGS = NT + 1;
+  // Workgroup id -> tile: ids go to the eight dies in turn; a die takes an eighth of the tiles, which follow one another over eight tiles of
+  // activation rows (512 rows) and then over the weight tiles, so that what runs on a die at once, 8 by 4 tiles, shares both in its L2.
+  const int mine = (n_tiles * m_tiles + GP_DIES - 1) / GP_DIES;
+  const int place = blockIdx.x % GP_DIES * mine + blockIdx.x / GP_DIES;
+  if (place >= n_tiles * m_tiles) return;  // the whole workgroup leaves together
+  const int band = place / (8 * n_tiles), in_band = place % (8 * n_tiles), high = min(8, m_tiles - 8 * band);
+  const int m0 = (8 * band + in_band % high) * 64, n0 = in_band / high * 16 * NT;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+
+  // A load takes eight rows' slices, a lane piece (lane % 8) ^ key of row lane / 8.  Wavefront v takes the eights v, v + 4, ...; where there is none
+  // it loads its last one again.  What lies past the last row's end (rows beyond N or M) brings zeros, which are not stored.
+  const int row8 = lane >> 3, piece = (lane & 7) ^ (4 * (wave & 1) + (row8 >> 1));
+  const float *const w_rows = w + (size_t)n0 * k, *const x_rows = x + (size_t)m0 * x_stride;
+  const size_t w_bytes = ((size_t)(min(n - n0, 16 * NT) - 1) * k + k) * 4, x_bytes = ((size_t)(min(m - m0, 64) - 1) * x_stride + k) * 4;
+  int woff[WLOADS], xoff[XLOADS], eight[WLOADS];
+#pragma unroll
+  for (int j = 0; j < WLOADS; ++j) {
+    eight[j] = wave + 4 * j < 2 * NT ? wave + 4 * j : wave + 4 * j - 4;
+    woff[j] = ((8 * eight[j] + row8) * k + 4 * piece) * 4;
+    asm volatile("" : "+v"(woff[j]));  // kept, not added up again
+  }
+#pragma unroll
+  for (int j = 0; j < XLOADS; ++j) {
+    xoff[j] = ((8 * (wave + 4 * j) + row8) * (int)x_stride + 4 * piece) * 4;
+    asm volatile("" : "+v"(xoff[j]));
+  }
+  const int count = k / SLICE;
+  // Slice i: its buffers (empty past the end) and its place in them.
+  auto buffer = [&](const float* rows, size_t bytes, int i) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(rows), 0, i < count ? (int)bytes : 0, 0x00027000);
+  };
+  auto place_of = [&](int i) __attribute__((always_inline)) { return i < count ? i * (SLICE * 4) : 0; };
+  auto load = [&](int j, int i, int slot) __attribute__((always_inline)) {
+    if (j < WLOADS)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer(w_rows, w_bytes, i), to + slot * SLOT + 8 * eight[j] * SLICE, 16, woff[j], place_of(i), 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer(x_rows, x_bytes, i), to + slot * SLOT + (16 * NT + 8 * (wave + 4 * (j - WLOADS))) * SLICE,
+                                               16, xoff[j - WLOADS], place_of(i), 0, 0);
+  };
+  // Where this lane's element of four k lies, piece q of the slice, in bytes: of a weight tile's row r, and of its activation rows; in the first two
+  // slots and in the last two (an instruction reaches 64 KB beyond its address).
+  constexpr int FAR = SLOTS / 2;
+  unsigned at[2][2][8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const unsigned base = (unsigned)(uintptr_t)from + 4 * (r * SLICE + 4 * (q ^ ((r >> 1) & 7)) + g);
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      at[f][0][q] = base + 4 * f * FAR * SLOT;
+      at[f][1][q] = at[f][0][q] + 4 * (16 * NT + 16 * wave) * SLICE;
+    }
+  }
+  float f[2][4][FRAGS];  // of sixteen k, in steps of four: the weights' fragments, the activations'
+  auto read = [&](int half, int e, int t, int slot) __attribute__((always_inline)) {
+    const unsigned base = at[slot / FAR][t < NT ? 0 : 1][4 * half + e];
+    f[half][e][t] = ((const lds_f32*)(uintptr_t)base)[slot % FAR * SLOT + 16 * (t < NT ? t : 0) * SLICE];
+  };
+  gp_f32x4 acc[NT], sum[NT];  // the range's chain, the ranges before it
+#pragma unroll
+  for (int b = 0; b < NT; ++b) acc[b] = sum[b] = gp_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < SLOTS; ++i) {
+#pragma unroll
+    for (int j = 0; j < R::LOADS; ++j) load(j, i, i);
+  }
+  auto renew = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) asm volatile("" : "+v"(at[i][0][q]), "+v"(at[i][1][q])::"memory");
+    }
+  };
+  auto arrive = [&](auto LEFT) __attribute__((always_inline)) {  // with LEFT loads still on their way
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(LEFT)::value) : "memory");
+    renew();
+  };
+  auto held = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0), one wait instead of one for each
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+      for (int t = 0; t < FRAGS; ++t) asm volatile("" : "+v"(f[1][e][t]));
+    }
+  };
+  arrive(std::integral_constant<int, (SLOTS - 1) * R::LOADS>{});
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+#pragma unroll
+    for (int t = 0; t < FRAGS; ++t) read(0, e, t, 0);
+  }
+  const int range_slices = range_of(k) / SLICE;
+  int range_end = min(range_slices, count);
+  // 4 NT instructions over one half's fragments, the other half's read beside them in the order in which they are wanted.
+  auto multiply = [&](int half, int read_slot, auto LOADING, int i, int free) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+      for (int b = 0; b < NT; ++b) {
+        acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[half][e][b], f[half][e][NT], acc[b], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < FRAGS; ++t)
+          if (t / 2 * NT / ((FRAGS + 1) / 2) == b) read(half ^ 1, e, t, read_slot);
+        if constexpr (decltype(LOADING)::value) {
+#pragma unroll
+          for (int j = 0; j < R::LOADS; ++j)
+            if (j * 4 * NT / R::LOADS == e * NT + b) load(j, i, free);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  // Slice `it` lies in slot SLOT_NOW, its first half's fragments are in registers.
+  auto round = [&](int it, auto SLOT_NOW) __attribute__((always_inline)) {
+    constexpr int slot = decltype(SLOT_NOW)::value, next = (slot + 1) % SLOTS;
+    multiply(0, slot, std::false_type{}, 0, 0);
+    // This wavefront has all of slice `it` in registers, and its loads of it + 1 have landed; behind the barrier both hold for the workgroup.
+    held();
+    arrive(std::integral_constant<int, (SLOTS - 2) * R::LOADS>{});
+    multiply(1, next, std::true_type{}, it + SLOTS, slot);
+    if (it + 1 == range_end) {  // the same for every thread
+#pragma unroll
+      for (int b = 0; b < NT; ++b) sum[b] += acc[b], acc[b] = gp_f32x4{0.f, 0.f, 0.f, 0.f};
+      range_end = min(range_end + range_slices, count);
+    }
+  };
+  static_assert(SLOTS == 4, "a turn of the loop goes once round the ring");
+  for (int it = 0; it < count; it += SLOTS) {
+    round(it, std::integral_constant<int, 0>{});
+    if (it + 1 >= count) break;
+    round(it + 1, std::integral_constant<int, 1>{});
+    if (it + 2 >= count) break;
+    round(it + 2, std::integral_constant<int, 2>{});
+    if (it + 3 >= count) break;
+    round(it + 3, std::integral_constant<int, 3>{});
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // loads past the end
+
+  // sum[b][i]: activation row 16 wave + r, weight row 16 b + 4 g + i.
+  const int row = m0 + 16 * wave + r;
+  if (row >= m) return;
+#pragma unroll
+  for (int b = 0; b < NT; ++b) {
+    const int col = n0 + 16 * b + 4 * g;
+    if (col >= n) continue;
+    if (bias) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[b][i] += bias[col + i];
+    }
+    *reinterpret_cast<gp_f32x4*>(y + (size_t)row * y_stride + col) = sum[b];
+  }
+}
+
+template <int NT>
+__global__ void __launch_bounds__(256, 2)
+gemm_plain_block_kernel(const float* __restrict__ x, const float* __restrict__ w, int x_stride, int m, int n, int k, int m_tiles, int n_tiles,
+                        float* __restrict__ y, const float* __restrict__ bias, long y_stride) {
+  extern __shared__ __attribute__((aligned(16))) float block_ring[];
+  plain_block<NT>((lds_f32*)block_ring, (const lds_f32*)block_ring, y, x, w, bias, m, n, k, x_stride, y_stride, m_tiles, n_tiles);
+}
+
+template <int NT>
+int launch_plain_block(void* y, const void* x, const void* w, const void* bias, int m, int n, int k, long x_stride, long y_stride,
+                       hipStream_t stream) {
+  static bool raised = false;  // per process; the attribute belongs to the kernel
+  if (!raised) {
+    if (hipFuncSetAttribute((const void*)gemm_plain_block_kernel<NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)PlainRing<NT>::BYTES) != hipSuccess)
+      return TS_ERR_LAUNCH;
+    raised = true;
+  }
+  const long m_tiles = ceil_of(m, 64), n_tiles = ceil_of(n, 16 * NT), ids = ceil_of(m_tiles * n_tiles, GP_DIES) * GP_DIES;
+  if (ids > 0x7fffffffL) return TS_ERR_SHAPE;
+  hipLaunchKernelGGL((gemm_plain_block_kernel<NT>), dim3((unsigned)ids), dim3(256), (PlainRing<NT>::BYTES), stream, (const float*)x,
+                     (const float*)w, (int)x_stride, m, n, k, (int)m_tiles, (int)n_tiles, (float*)y, (const float*)bias, y_stride);
+  return ts_launch_status();
+}
 
 // Which layout runs a product: the one whose workgroups are through soonest, a round of one on every compute unit at a time.
 // Half microseconds at K = 3,584, measured over q|k|v, o, gate|up and the head of the 7B shape at 1 to 2,048 rows (all
 // grow with K alike): a round of workgroups of 16 x 16 outputs whose operands go through LDS takes 9.5 us (read straight from
 // memory 13), of 16 x 32 17.5 (24), 32 x 16 15 (22), 32 x 32 24.5 (37) (more weight rows a wavefront read the
-// activations less often, fewer give more workgroups), of 64 x 64 70, of 128 x 128 240, and the first round a little more.
-enum PlainKind { FEW_1_1, FEW_1_2, FEW_2_1, FEW_2_2, TILES_64, TILES_128 };
+// activations less often, fewer give more workgroups), of 64 x 64 70, of 128 x 128 240, and the first round a little more.  Where the block
+// layout takes the operands: a round of 64 x 16 NT 13 NT, 3 more where a compute unit holds one (NT 7 and more); 64 x 64 and 128 x 128
+// are not asked for there (500 rows, us, before -> NT: gate|up 1,145 -> 961, down 671 -> 486, o 131 -> 99, q|k|v 187 -> 121; 128 rows of o 42 -> 31).
+enum PlainKind { FEW_1_1, FEW_1_2, FEW_2_1, FEW_2_2, TILES_64, TILES_128, BLOCK };  // BLOCK + NT
 
-inline PlainKind plain_kind(int m, int n, bool stream_reads) {
+inline int plain_kind(int m, int n, bool stream_reads, bool block) {
   static const struct {
     PlainKind kind;
     int rows, cols, start[2], round[2];  // straight from memory, through LDS
   } layouts[] = {{FEW_1_1, 16, 16, {6, 6}, {26, 19}}, {FEW_1_2, 16, 32, {0, 2}, {48, 35}}, {FEW_2_1, 32, 16, {6, 8}, {44, 30}},
                  {FEW_2_2, 32, 32, {0, 4}, {74, 49}}, {TILES_64, 64, 64, {24, 10}, {130, 140}}, {TILES_128, 128, 128, {0, 0}, {470, 480}}};
-  PlainKind best = TILES_128;
-  long least = -1;
+  int best = TILES_128;
+  long least = -1, filled = 1L << 40;
   for (const auto& l : layouts) {
-    if (l.cols < 64 && ceil_of(m, l.rows) > 65535) continue;  // more tiles of rows than their grids take
-    const long cost = l.start[stream_reads] + l.round[stream_reads] * ceil_of(ceil_of(m, l.rows) * ceil_of(n, l.cols), GP_UNITS);
-    if (least < 0 || cost < least) best = l.kind, least = cost;
+    if (l.cols < 64 ? ceil_of(m, l.rows) > 65535 : block) continue;  // more tiles of rows than their grids take
+    const long workgroups = ceil_of(m, l.rows) * ceil_of(n, l.cols);
+    const long cost = l.start[stream_reads] + l.round[stream_reads] * ceil_of(workgroups, GP_UNITS);
+    if (least < 0 || cost < least) best = l.kind, least = cost, filled = l.start[1] + l.round[1] * max(workgroups, (long)GP_UNITS) / GP_UNITS;
+  }
+  // A last round of the few rows' layouts that is nearly empty is nearly over at once (48 rows of 4,608, 432 workgroups of 16 x 32: 26 us, one
+  // round of 64 x 32 32).  No tile of the block layout is through before 64, so what is sooner is not compared.
+  for (int nt = 2; block && nt <= 9 && filled > 64; ++nt) {
+    const long rounds = ceil_of(ceil_of(ceil_of(m, 64) * ceil_of(n, 16 * nt), GP_DIES), GP_UNITS / GP_DIES);
+    const long cost = 8 + rounds * (26 * nt + (nt == 2 ? 4 : nt < 7 ? 0 : 6));
+    if (cost < filled) best = BLOCK + nt, filled = cost;
   }
   return best;
 }
 
 template <typename TIn, typename TOut>
 int launch_plain(void* y, const void* x, const void* w, const void* bias, int m, int n, int k, long x_stride,
-                 long y_stride, hipStream_t stream) {
+                 long y_stride, int tile, hipStream_t stream) {
   const size_t quad = 4 * sizeof(TIn);
   const bool vec = k % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)x % quad == 0 && (uintptr_t)w % quad == 0 &&
                    x_stride < (1L << 25) && k < (1 << 25);
@@ -729,7 +948,25 @@ int launch_plain(void* y, const void* x, const void* w, const void* bias, int m,
       return ts_launch_status();
     }
   }
-  switch (plain_kind(m, n, stream_reads)) {
+  // The block layout's stores and loads are 16 bytes, its slices whole, its tiles' rows within 31 bits of the first one.
+  const bool block = stream_reads && k % 32 == 0 && n % 4 == 0 && y_stride % 4 == 0 && (uintptr_t)y % 16 == 0 && x_stride < (1L << 21) &&
+                     k < (1 << 21);
+  if (tile != 0 && (!block || tile < 2 || tile > 9)) return TS_ERR_SHAPE;
+  const int kind = tile ? BLOCK + tile : plain_kind(m, n, stream_reads, block);
+  if constexpr (sizeof(TIn) == 4 && sizeof(TOut) == 4) {
+#define TS_PLAIN_BLOCK(NT) \
+  if (kind == BLOCK + NT) return launch_plain_block<NT>(y, x, w, bias, m, n, k, x_stride, y_stride, stream)
+    TS_PLAIN_BLOCK(2);
+    TS_PLAIN_BLOCK(3);
+    TS_PLAIN_BLOCK(4);
+    TS_PLAIN_BLOCK(5);
+    TS_PLAIN_BLOCK(6);
+    TS_PLAIN_BLOCK(7);
+    TS_PLAIN_BLOCK(8);
+    TS_PLAIN_BLOCK(9);
+#undef TS_PLAIN_BLOCK
+  }
+  switch (kind) {
     case FEW_1_1:
       TS_PLAIN_FEW(1, 1, 3);
       break;
@@ -757,15 +994,17 @@ int launch_plain(void* y, const void* x, const void* w, const void* bias, int m,
 
 }  // namespace
 
-// dtype: type of x, w and bias.  out_f32 != 0: y is float whatever dtype is.
+// dtype: type of x, w and bias.  out_f32 != 0: y is float whatever dtype is.  tile: 0, or 2 to 9, tiles of 64 x 16 tile outputs by the block
+// layout, where it takes the operands.
 extern "C" int ts_gemm_plain(void* y, const void* x, const void* w, const void* bias, int m, int n,
-                             int k, long x_stride, long y_stride, int dtype, int out_f32,
+                             int k, long x_stride, long y_stride, int dtype, int out_f32, int tile,
                              hipStream_t stream) {
   if (m == 0 || n == 0) return TS_OK;
   if (!y || !x || !w || k < 1 || x_stride < k || y_stride < n) return TS_ERR_ARG;
   if (ceil_of(m, 64) > 65535) return TS_ERR_SHAPE;
-  if (dtype == TS_F32) return launch_plain<float, float>(y, x, w, bias, m, n, k, x_stride, y_stride, stream);
+  if (dtype == TS_F32) return launch_plain<float, float>(y, x, w, bias, m, n, k, x_stride, y_stride, tile, stream);
   if (dtype != TS_BF16) return TS_ERR_DTYPE;
-  if (out_f32) return launch_plain<bf16_t, float>(y, x, w, bias, m, n, k, x_stride, y_stride, stream);
-  return launch_plain<bf16_t, bf16_t>(y, x, w, bias, m, n, k, x_stride, y_stride, stream);
+  if (tile != 0) return TS_ERR_SHAPE;
+  if (out_f32) return launch_plain<bf16_t, float>(y, x, w, bias, m, n, k, x_stride, y_stride, 0, stream);
+  return launch_plain<bf16_t, bf16_t>(y, x, w, bias, m, n, k, x_stride, y_stride, 0, stream);
 }

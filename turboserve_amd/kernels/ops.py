@@ -142,7 +142,7 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "ts_moe_combine": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_long, c_void_p, c_int, c_int, c_int,
                            c_int, c_void_p, c_int, c_void_p, c_void_p],
         "ts_gemm_plain": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long,
-                          c_int, c_int, c_void_p],
+                          c_int, c_int, c_int, c_void_p],
         "ts_gemm_tiled": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                           c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_wide": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -2074,8 +2074,10 @@ class Ops:
         bias: torch.Tensor | None = None,
         *,
         out_float32: bool = False,
+        tile: int = 0,
     ) -> torch.Tensor:
-        """``x [M, K] @ weight [N, K]^T (+ bias)`` by 32-bit fused multiply-adds."""
+        """``x [M, K] @ weight [N, K]^T (+ bias)`` by 32-bit fused multiply-adds, in the layout that is through soonest.  ``tile`` (2 to 9): in tiles
+        of 64 rows by 16 ``tile`` outputs, where the operands are 32-bit and 16-byte accesses, a K of whole slices of 32 and 31-bit offsets fit."""
         _gpu(x, weight, bias)
         _need(x.dim() == 2 and x.stride(1) == 1 and weight.dim() == 2 and weight.is_contiguous(),
               "x must be [M, K] with unit inner stride, weight contiguous [N, K]")
@@ -2088,7 +2090,7 @@ class Ops:
         y = torch.empty((m, n), dtype=out_dtype, device=x.device)
         _check(self.core.ts_gemm_plain(_ptr(y), _ptr(x), _ptr(weight), _ptr(bias), m, n, k,
                                        x.stride(0) if m > 1 else max(k, x.stride(0)), n,
-                                       dtype_code(x.dtype), 1 if out_float32 else 0, self.stream()),
+                                       dtype_code(x.dtype), 1 if out_float32 else 0, tile, self.stream()),
                "ts_gemm_plain")
         return y
 
