@@ -103,6 +103,29 @@ def test_tiles_of_224_weight_rows_fill_the_rounds_of_several_ranges():
                 assert tn != 7 or splits == 1 or 10 * workgroups >= 9 * 256 * -(-workgroups // 256), (m, n, k, kind)
 
 
+def test_a_norm_waits_for_a_product_that_makes_it(monkeypatch):
+    """One row up to 6,144 wide and two up to 3,072, as 32-bit sums of up to four ranges, for a matrix that the streaming product takes; every
+    other norm runs by itself."""
+    monkeypatch.setattr("turboserve_amd.kernels.ops._gpu", lambda *tensors: None)
+    ops = Planner()
+
+    def waits(rows, n, k, gated=False, sums=2, dtype=torch.bfloat16, pending=True):
+        parts = torch.empty(sums, rows, k, device="meta") if pending else None
+        gain, matrix = torch.empty(k, dtype=dtype, device="meta"), torch.empty(n, k, dtype=dtype, device="meta")
+        residual = torch.empty(rows, k, device="meta")
+        norm = ops.waiting_norm(residual, parts, gain, 1e-6, matrix, gated=gated)
+        assert norm is None or (norm.after.shape == residual.shape and norm.after is not residual)
+        return norm is not None
+
+    assert waits(1, 4608, 3584) and waits(1, 37888, 3584, gated=True) and waits(2, 16384, 2048, gated=True) and waits(1, 9216, 6144) and waits(2, 6144, 3072)
+    assert not waits(2, 4608, 3584) and not waits(3, 3072, 2048) and not waits(1, 8192, 8192) and not waits(1, 4608, 3584, sums=5)
+    assert not waits(1, 4608, 3584, pending=False) and not waits(1, 4608, 3584, dtype=torch.float32) and not waits(1, 4608, 3592) and not waits(1, 96, 3584)
+    assert not waits(1, 27648, 5120, gated=True) and not waits(1, 3584, 18944, gated=True)  # tiles or several ranges are sooner
+    parts = torch.empty(1, 3584, dtype=torch.bfloat16, device="meta")  # one result of the run's type
+    gain, matrix = torch.empty(3584, dtype=torch.bfloat16, device="meta"), torch.empty(4608, 3584, dtype=torch.bfloat16, device="meta")
+    assert ops.waiting_norm(torch.empty(1, 3584, device="meta"), parts, gain, 1e-6, matrix, gated=False) is None
+
+
 def test_32_bit_attention_is_asked_only_for_what_it_takes():
     """Pages of 24 keys and pages or rows that 16-byte accesses do not fit stay with the kernel that takes any geometry."""
     ops = Planner()

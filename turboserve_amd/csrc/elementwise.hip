@@ -40,22 +40,6 @@ extern "C" int ts_embed(void* residual, const void* table, const int* ids, int t
   return ts_launch_status();
 }
 
-// ---------------------------------------------------------------------------------------------
-// RMSNorm.  y = w * round_T(x * rsqrt(mean(x^2) + eps)): the normalised value is rounded to the
-// storage type before the gain, as the reference does (layers.py:208).
-//
-// add_rmsnorm: s = residual + pending (32-bit); residual = s; y = norm(s).  With `rows` the
-// kernel reads rows[i] and writes y[i] only (residual untouched): the final norm at the wanted
-// positions.
-// ---------------------------------------------------------------------------------------------
-// The gain: `one_rounding == 0` is the rule above, w * round_T(n); otherwise the whole norm is
-// 32-bit arithmetic with one rounding at the end, round_T(n * (gain_offset + w)) (a gain stored
-// around zero has gain_offset 1).
-template <typename T>
-__device__ __forceinline__ float with_gain(float normalised, float gain, float gain_offset, int one_rounding) {
-  return one_rounding ? normalised * (gain_offset + gain) : gain * round_to<T>(normalised);
-}
-
 template <typename T>
 __global__ void rmsnorm_kernel(T* __restrict__ y, const T* __restrict__ x, const T* __restrict__ w,
                                float eps, int hidden, float gain_offset, int one_rounding) {

@@ -16,26 +16,31 @@
 // 10.9 -> 10.4, 2,048 x 8,192 8.15 -> 7.97, gate|up [16384, 2048] 13.3 -> 13.0, the long ones within 1%.
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 
 constexpr int STREAM_WAVES = 4;
 
-// NT tiles of sixteen weight rows, XT of eight activation rows.
+constexpr int NORMED_MOST = 6144, NORMED_ROOM = NORMED_MOST + 64;  // elements of normalised rows in LDS (XT = 0), and their wavefronts' sums
+
+// NT tiles of sixteen weight rows, XT of eight activation rows (0: they lie in LDS as a whole).
 template <int NT, int XT>
 struct Ring {
   static constexpr int SLICE = 64, TILE = 16 * SLICE, HALF = 8 * SLICE, LOADS = 2 * NT + XT;  // of sixteen rows; of eight; of a slice
   static constexpr int SLOT = NT * TILE + XT * HALF;
-  static constexpr int SLOTS = 80 * 1024 / (STREAM_WAVES * SLOT * 2);  // two workgroups a compute unit
+  static constexpr int SLOTS = (80 * 1024 - (XT ? 0 : NORMED_ROOM * 2)) / (STREAM_WAVES * SLOT * 2);  // two workgroups a compute unit
   static constexpr int WAVE = SLOTS * SLOT;                            // elements of a wavefront's ring
   static constexpr size_t BYTES = (size_t)STREAM_WAVES * WAVE * 2;
-  static_assert(SLOTS >= 2 && (SLOTS - 1) * LOADS < 64 && 2 * BYTES <= 160 * 1024, "a ring of at least two slices, counted by vmcnt");
+  static_assert(SLOTS >= 2 && (SLOTS - 1) * LOADS < 64 && 2 * (BYTES + (XT ? 0 : NORMED_ROOM * 2)) <= 160 * 1024, "a ring of at least two slices, counted by vmcnt");
   static_assert(WAVE * 2 >= NT * 1024, "a wavefront's sums fit its ring");
 };
 
@@ -57,24 +62,25 @@ __device__ __forceinline__ void stream_wait_for(int left, int& slot) {
 }
 
 // acc[t][i]: weight row n0 + 16 t + 4 (lane / 16) + i, activation row lane % 16 (lane % 8 with XT = 1), over slices first .. last - 1
-// of 64 k.
-template <int NT, int XT>
-__device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, const uint16_t* __restrict__ x,
-                                             const uint16_t* __restrict__ w, int m, int n, int k, long x_stride, int n0, int first,
-                                             int last, f32x4* acc) {
+// of 64 k.  XT = 0: activation row lane % ROWS of `held`, rows of k elements in LDS (k whole slices); `meanwhile` runs when the first slices
+// have been asked for and puts them there, its own loads before those of any slice; it is called by every wavefront.
+template <int NT, int XT, int ROWS, typename Meanwhile>
+__device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, const lds_u16* __restrict__ held,
+                                             const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int m, int n, int k,
+                                             long x_stride, int n0, int first, int last, f32x4* acc, Meanwhile meanwhile) {
   typedef Ring<NT, XT> R;
   constexpr int SLICE = R::SLICE, TILE = R::TILE, HALF = R::HALF, SLOTS = R::SLOTS;
   const int count = last - first;
-  if (count <= 0) return;
+  if (XT != 0 && count <= 0) return;
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   // A lane loads 16 bytes, piece (lane % 8) ^ key of row lane / 8 of eight, key = row / 2 % 8: a piece of sixteen rows
   // touches every bank once.  (The second eight rows of a tile have keys four further on: piece ^ 4.)  What lies past the last
   // row's end (rows beyond N or M) brings zeros, what lies past another row's end (a K that is no multiple of 64) is cleared.
   const int row8 = lane >> 3, piece = (lane & 7) ^ (row8 >> 1);
   const size_t wbytes = (size_t)min(n - n0, 16 * NT) * k * 2, xbytes = ((size_t)(m - 1) * x_stride + k) * 2;
-  const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w + (size_t)n0 * k), 0, (int)wbytes, 0x00027000);
+  const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w + (size_t)n0 * k), 0, XT == 0 && count <= 0 ? 0 : (int)wbytes, 0x00027000);
   const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, (int)xbytes, 0x00027000);
-  uint32_t woff[2 * NT], xoff[XT];
+  uint32_t woff[2 * NT], xoff[XT ? XT : 1];
 #pragma unroll
   for (int j = 0; j < 2 * NT; ++j) woff[j] = ((uint32_t)(8 * j + row8) * (uint32_t)k + first * SLICE + 8 * (piece ^ (j & 1 ? 4 : 0))) * 2;
 #pragma unroll
@@ -92,14 +98,16 @@ __device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds
   struct Frags {
     u32x4 x[2], w[NT][2];
   };
-  const int key = (r >> 1) & 7, x_row = r & (8 * XT - 1);
-  auto read = [&](Frags& f, int slot) __attribute__((always_inline)) {
+  const int key = (r >> 1) & 7, x_row = XT ? r & (8 * XT - 1) : r & (ROWS - 1);
+  int held_at = x_row * k + first * SLICE + 8 * g;
+  auto read = [&](Frags& f, int i, int slot) __attribute__((always_inline)) {
     const lds_u16* base = from + slot * R::SLOT;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) f.w[t][c] = *(const lds_u32x4*)(base + t * TILE + r * SLICE + 8 * ((4 * c + g) ^ key));
-      f.x[c] = *(const lds_u32x4*)(base + NT * TILE + x_row * SLICE + 8 * ((4 * c + g) ^ (x_row >> 1)));
+      if (XT) f.x[c] = *(const lds_u32x4*)(base + NT * TILE + x_row * SLICE + 8 * ((4 * c + g) ^ (x_row >> 1)));
+      else f.x[c] = *(const lds_u32x4*)(held + held_at + i * SLICE + 32 * c);
     }
   };
   auto consume = [&](Frags& f, int left) __attribute__((always_inline)) {  // left: elements of the slice inside the row
@@ -125,19 +133,34 @@ __device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds
   };
   // No load is issued past the end: one that brings nothing still takes its turn in the unit's memory path, and a ring's worth
   // of them behind every wavefront made a short product's end (or the next workgroup's start) a microsecond longer.
-#pragma unroll
-  for (int j = 0; j < SLOTS; ++j)
-    if (j < count) fetch(j, j);
   int slot = 0;
-  stream_wait_for<R::LOADS, SLOTS - 1>(count - 1, slot);
+  if (XT) {
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j)
+      if (j < count) fetch(j, j);
+    stream_wait_for<R::LOADS, SLOTS - 1>(count - 1, slot);
+  } else {
+    // (Without a branch, so that the compiler can count them behind the loads of `meanwhile`; those past the end lie outside the buffer.)
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j) {
+#pragma unroll
+      for (int t = 0; t < 2 * NT; ++t)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, to + j * R::SLOT + t * HALF, 16, j < count ? (int)(woff[t] + j * (SLICE * 2)) : (int)0x80000000, 0, 0, 2);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    meanwhile();
+    asm volatile("" : "+v"(held_at)::"memory");  // what `meanwhile` wrote is read at addresses that are new to the compiler
+    if (count <= 0) return;
+    stream_wait<(SLOTS - 1) * R::LOADS>(slot);
+  }
   Frags f[2];
-  read(f[0], slot);
+  read(f[0], 0, slot);
   auto round = [&](int i, Frags& now, Frags& next) __attribute__((always_inline)) {
     arrived(now);
     fetch(i + SLOTS, slot);
     slot = slot + 1 == SLOTS ? 0 : slot + 1;
     stream_wait<(SLOTS - 1) * R::LOADS>(slot);
-    read(next, slot);
+    read(next, i + 1, slot);
     consume(now, SLICE);
   };
   int i = 0;
@@ -157,11 +180,46 @@ __device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds
     f[1] = f[0];
     slot = slot + 1 == SLOTS ? 0 : slot + 1;
     stream_wait_for<R::LOADS, SLOTS - 2>(count - i - 2, slot);
-    read(f[0], slot);
+    read(f[0], i + 1, slot);
     consume(f[1], SLICE);
   }
   consume(f[0], k - (last - 1) * SLICE);  // the last slice alone may be cut short
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
+// What a workgroup does with its wavefronts' sums: the quarters meet in the rings; wavefront v adds up and stores tile v, `shift` its bias.
+template <int NT, int XT, bool GATED>
+__device__ __forceinline__ void stream_finish(lds_u16* ring, const f32x4* acc, const uint32_t (&shift)[4], bool shifted, int m, int n, int col, int split,
+                                              float* __restrict__ partial, uint16_t* __restrict__ out, GluRule rule) {
+  typedef Ring<NT, XT> R;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+  for (int t = 0; t < NT; ++t) ((lds_f32x4*)(ring + wave * R::WAVE))[t * 64 + lane] = acc[t];
+  __syncthreads();
+  if (wave >= NT) return;
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int v = 0; v < STREAM_WAVES; ++v) sum += ((lds_f32x4*)(ring + v * R::WAVE))[wave * 64 + lane];
+  const int row = lane & 15;
+  if (row >= m || col >= n) return;
+  if (shifted) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] += __uint_as_float(shift[i] << 16);
+  }
+  if (GATED) {  // n is even: the first pair lies inside
+    uint16_t* at = out + (size_t)row * (n / 2) + col / 2;
+    at[0] = from_float<bf16_t>(gated_unit(sum[0], sum[1], rule)).bits;
+    if (col + 2 < n) at[1] = from_float<bf16_t>(gated_unit(sum[2], sum[3], rule)).bits;
+  } else {
+    float* at = partial + ((size_t)split * m + row) * n + col;
+    if (n % 4 == 0) {
+      *reinterpret_cast<f32x4*>(at) = sum;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (col + i < n) at[i] = sum[i];
+    }
+  }
 }
 
 // partial: float [splits, m, n], or, GATED, out: bfloat16 [m, n / 2], the gated unit (common.hpp) of rows that alternate gate, up.
@@ -187,35 +245,8 @@ gemm_stream_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
     for (int i = 0; i < 4; ++i) shift[i] = bias[min(col + i, n - 1)];
   }
   lds_u16* mine = (lds_u16*)ring + wave * R::WAVE;
-  stream_range<NT, XT>(mine, mine, x, w, m, n, k, x_stride, n0, first, last, acc);
-  // The quarters' sums meet in the rings; wavefront v adds up and stores tile v.
-#pragma unroll
-  for (int t = 0; t < NT; ++t) ((lds_f32x4*)mine)[t * 64 + lane] = acc[t];
-  __syncthreads();
-  if (wave >= NT) return;
-  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int v = 0; v < STREAM_WAVES; ++v) sum += ((lds_f32x4*)((lds_u16*)ring + v * R::WAVE))[wave * 64 + lane];
-  const int row = lane & 15;
-  if (row >= m || col >= n) return;
-  if (bias && split == 0) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sum[i] += __uint_as_float(shift[i] << 16);
-  }
-  if (GATED) {  // n is even: the first pair lies inside
-    uint16_t* at = out + (size_t)row * (n / 2) + col / 2;
-    at[0] = from_float<bf16_t>(gated_unit(sum[0], sum[1], rule)).bits;
-    if (col + 2 < n) at[1] = from_float<bf16_t>(gated_unit(sum[2], sum[3], rule)).bits;
-  } else {
-    float* at = partial + ((size_t)split * m + row) * n + col;
-    if (n % 4 == 0) {
-      *reinterpret_cast<f32x4*>(at) = sum;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (col + i < n) at[i] = sum[i];
-    }
-  }
+  stream_range<NT, XT, 0>(mine, mine, mine, x, w, m, n, k, x_stride, n0, first, last, acc, [] {});
+  stream_finish<NT, XT, GATED>((lds_u16*)ring, acc, shift, bias && split == 0, m, n, col, split, partial, out, rule);
 }
 
 template <int NT, int XT, bool GATED>
@@ -231,6 +262,134 @@ int launch_stream(float* partial, void* out, const void* x, long x_stride, const
   hipLaunchKernelGGL((gemm_stream_kernel<NT, XT, GATED>), dim3((n + 16 * NT - 1) / (16 * NT), splits), dim3(64 * STREAM_WAVES),
                      BYTES, stream, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (int)x_stride, m, n, k, per_wave,
                      partial, (uint16_t*)out, rule);
+  return ts_launch_status();
+}
+
+// The same for one or two rows that are the norm of the residual stream, which is not stored: every workgroup adds up the pending partial sums and
+// normalises the whole row for itself while its first weights travel.  The norm's own launch, some 4.5 us of a
+// recorded step of which one trip to memory and the launch are most, falls away; what comes instead is 50 KB a row from L2 for every workgroup.
+// The sum goes to `after` (not to `residual`, which other workgroups are still to read): of 1,024 elements by one workgroup each.
+template <int NT, int ROWS, int ITEMS, int SUMS, bool GATED>
+__global__ void __launch_bounds__(64 * STREAM_WAVES)
+gemm_stream_normed_kernel(const float* __restrict__ residual, const float* __restrict__ pending, const uint16_t* __restrict__ gain,
+                          const uint16_t* __restrict__ w, int n, int k, int per_wave, float eps, float* __restrict__ after,
+                          const uint16_t* __restrict__ bias, float* __restrict__ partial, uint16_t* __restrict__ out, float gain_offset,
+                          int one_rounding, GluRule rule) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t ring[];
+  constexpr int THREADS = 64 * STREAM_WAVES;
+  typedef Ring<NT, 0> R;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * 16 * NT, split = blockIdx.y, quads = k / 4;
+  float s[ROWS][ITEMS][4], part[ROWS][ITEMS][SUMS][4];
+  u32x2 g[ITEMS];
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int quad = threadIdx.x + it * THREADS, at = 4 * (it + 1 < ITEMS ? quad : min(quad, quads - 1));
+#pragma unroll
+    for (int row = 0; row < ROWS; ++row) {
+#pragma unroll
+      for (int j = 0; j < SUMS; ++j) *(f32x4*)part[row][it][j] = *(const f32x4*)(pending + ((size_t)j * ROWS + row) * k + at);
+      *(f32x4*)s[row][it] = *(const f32x4*)(residual + (size_t)row * k + at);
+    }
+    g[it] = *(const u32x2*)(gain + at);
+  }
+  const int col = n0 + 16 * min(wave, NT - 1) + 4 * (lane >> 4);
+  uint32_t shift[4] = {0, 0, 0, 0};
+  if (bias && split == 0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) shift[i] = bias[min(col + i, n - 1)];
+  }
+  asm volatile("" ::: "memory");  // all of them on their way here
+  __builtin_amdgcn_sched_barrier(0);
+  uint16_t* const held = ring + STREAM_WAVES * R::WAVE;
+  float(*const sums)[STREAM_WAVES] = reinterpret_cast<float(*)[STREAM_WAVES]>(held + NORMED_ROOM - 2 * ROWS * STREAM_WAVES);  // behind the rows
+  auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };  // (the fence of __syncthreads would wait for the weights)
+  // The workgroup's range of K is all it needs normalised.
+  const int from_quad = split * STREAM_WAVES * per_wave * (R::SLICE / 4), to_quad = min(quads, from_quad + STREAM_WAVES * per_wave * (R::SLICE / 4));
+  auto normalise = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int row = 0; row < ROWS; ++row) {
+      float ss = 0.f;
+#pragma unroll
+      for (int it = 0; it < ITEMS; ++it) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+          for (int j = 0; j < SUMS; ++j) s[row][it][e] += part[row][it][j][e];
+        }
+        const float one = (int)threadIdx.x + it * THREADS < quads ? 1.f : 0.f;
+        float four = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) four = fmaf(s[row][it][e], s[row][it][e], four);
+        ss += it + 1 < ITEMS || one != 0.f ? four : 0.f;  // all but the last item lie inside the row
+      }
+      ss = wave_sum(ss);
+      if (lane == 0) sums[row][wave] = ss;
+    }
+    meet();
+    float rstd[ROWS];
+#pragma unroll
+    for (int row = 0; row < ROWS; ++row) {
+      float ss = 0.f;
+#pragma unroll
+      for (int v = 0; v < STREAM_WAVES; ++v) ss += sums[row][v];
+      rstd[row] = rsqrtf(ss / (float)k + eps);
+    }
+    auto write = [&](auto ONE_ROUNDING) __attribute__((always_inline)) {
+#pragma unroll
+      for (int it = 0; it < ITEMS; ++it) {
+        const int quad = threadIdx.x + it * THREADS;
+        if (quad < from_quad || quad >= to_quad) continue;
+#pragma unroll
+        for (int row = 0; row < ROWS; ++row) {
+          float n[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float gained = __uint_as_float(e & 1 ? g[it][e / 2] & 0xffff0000u : g[it][e / 2] << 16);
+            n[e] = with_gain<bf16_t>(s[row][it][e] * rstd[row], gained, gain_offset, decltype(ONE_ROUNDING)::value);
+          }
+          *(u32x2*)(held + row * k + 4 * quad) = u32x2{(uint32_t)from_float<bf16_t>(n[0]).bits | (uint32_t)from_float<bf16_t>(n[1]).bits << 16,
+                                                       (uint32_t)from_float<bf16_t>(n[2]).bits | (uint32_t)from_float<bf16_t>(n[3]).bits << 16};
+        }
+      }
+    };
+    if (one_rounding) write(std::true_type{});
+    else write(std::false_type{});
+    meet();
+    if (split == 0 && (int)blockIdx.x < ITEMS) {
+#pragma unroll
+      for (int it = 0; it < ITEMS; ++it) {
+        const int quad = threadIdx.x + it * THREADS;
+#pragma unroll
+        for (int row = 0; row < ROWS; ++row)
+          if ((int)blockIdx.x == it && quad < quads) *(f32x4*)(after + (size_t)row * k + 4 * quad) = *(const f32x4*)s[row][it];
+      }
+    }
+  };
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int total = k / R::SLICE, first = (split * STREAM_WAVES + wave) * per_wave, last = min(first + per_wave, total);
+  lds_u16* mine = (lds_u16*)ring + wave * R::WAVE;
+  stream_range<NT, 0, ROWS>(mine, mine, (const lds_u16*)held, nullptr, w, ROWS, n, k, 0, n0, first, last, acc, normalise);
+  stream_finish<NT, 0, GATED>((lds_u16*)ring, acc, shift, bias && split == 0, ROWS, n, col, split, partial, out, rule);
+}
+
+template <int ROWS, int ITEMS, int SUMS, bool GATED>
+int launch_stream_normed(float* partial, void* out, const float* residual, const float* pending, float* after, const void* gain,
+                         float eps, float gain_offset, int one_rounding, const void* w, const void* bias, int n, int k, int per_wave, int splits,
+                         GluRule rule, hipStream_t stream) {
+  constexpr size_t BYTES = Ring<2, 0>::BYTES + NORMED_ROOM * 2;
+  static bool raised = false;  // per process; the attribute belongs to the kernel
+  if (!raised) {
+    if (hipFuncSetAttribute((const void*)gemm_stream_normed_kernel<2, ROWS, ITEMS, SUMS, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)BYTES) !=
+        hipSuccess)
+      return TS_ERR_LAUNCH;
+    raised = true;
+  }
+  hipLaunchKernelGGL((gemm_stream_normed_kernel<2, ROWS, ITEMS, SUMS, GATED>), dim3((n + 31) / 32, splits), dim3(64 * STREAM_WAVES), BYTES, stream,
+                     residual, pending, (const uint16_t*)gain, (const uint16_t*)w, n, k, per_wave, eps, after, (const uint16_t*)bias,
+                     partial, (uint16_t*)out, gain_offset, one_rounding, rule);
   return ts_launch_status();
 }
 
@@ -264,5 +423,40 @@ extern "C" int ts_gemm_stream(float* partial, void* out, const void* x, long x_s
     TS_STREAM(2, false);
   }
 #undef TS_STREAM
+  return TS_ERR_SHAPE;
+}
+
+// The product of norm(residual + pending) as add_rmsnorm makes it (elementwise.hip), bfloat16, which is not stored: residual [m, k] float, m 1 or 2, pending
+// float [sums, m, k], up to 4, gain [k] bfloat16, k a multiple of 64 and m k at most 6,144; after [m, k] float, other memory than residual, takes
+// the sum.  All 16-byte aligned.  n more than 32 (ceil(k / 1024) - 1): a workgroup for every 1,024 elements of `after`.  The rest as ts_gemm_stream's.
+extern "C" int ts_gemm_stream_normed(float* partial, void* out, const float* residual, const float* pending, int sums, float* after, const void* gain,
+                                     float eps, float gain_offset, int one_rounding, const void* w, const void* bias, int m, int n, int k,
+                                     int per_wave, int splits, float steepness, float limit, float up_shift, float cubic, hipStream_t stream) {
+  if (!residual || !pending || !after || after == residual || !gain || !w || (partial == nullptr) == (out == nullptr)) return TS_ERR_ARG;
+  if (m < 1 || m > 2 || k < 64 || k % 64 != 0 || m * (long)k > NORMED_MOST || sums < 1 || sums > 4 || n < 1) return TS_ERR_SHAPE;
+  if (n <= 32 * ((k + 1023) / 1024 - 1)) return TS_ERR_SHAPE;
+  if (((uintptr_t)residual | (uintptr_t)pending | (uintptr_t)after | (uintptr_t)gain | (uintptr_t)w) % 16 != 0) return TS_ERR_SHAPE;
+  if (per_wave < 1 || splits < 1 || splits > 65535 || splits != (k / 64 + 4L * per_wave - 1) / (4L * per_wave)) return TS_ERR_SHAPE;
+  if (out && (splits != 1 || n % 2 != 0)) return TS_ERR_ARG;
+  const GluRule rule = {steepness, limit, up_shift, cubic};
+  const int items = (k + 1023) / 1024;
+#define TS_NORMED(ROWS, ITEMS, SUMS)                                                                                                               \
+  if (m == ROWS && items == ITEMS && sums == SUMS)                                                                                                 \
+    return out ? launch_stream_normed<ROWS, ITEMS, SUMS, true>(partial, out, residual, pending, after, gain, eps, gain_offset, one_rounding, w,    \
+                                                               bias, n, k, per_wave, splits, rule, stream)                                         \
+               : launch_stream_normed<ROWS, ITEMS, SUMS, false>(partial, out, residual, pending, after, gain, eps, gain_offset, one_rounding, w,   \
+                                                                bias, n, k, per_wave, splits, rule, stream);
+#define TS_NORMED_SUMS(ROWS, ITEMS) TS_NORMED(ROWS, ITEMS, 1) TS_NORMED(ROWS, ITEMS, 2) TS_NORMED(ROWS, ITEMS, 3) TS_NORMED(ROWS, ITEMS, 4)
+  TS_NORMED_SUMS(1, 1)
+  TS_NORMED_SUMS(1, 2)
+  TS_NORMED_SUMS(1, 3)
+  TS_NORMED_SUMS(1, 4)
+  TS_NORMED_SUMS(1, 5)
+  TS_NORMED_SUMS(1, 6)
+  TS_NORMED_SUMS(2, 1)
+  TS_NORMED_SUMS(2, 2)
+  TS_NORMED_SUMS(2, 3)
+#undef TS_NORMED_SUMS
+#undef TS_NORMED
   return TS_ERR_SHAPE;
 }

@@ -149,6 +149,8 @@ _SIGNATURES: dict[str, dict[str, list]] = {
                          c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_block": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                           c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
+        "ts_gemm_stream_normed": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_float, c_float, c_int, c_void_p, c_void_p,
+                                  c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_stream": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                            c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_skinny_resident": [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
@@ -366,6 +368,29 @@ class PrefillWork:
     ranges: torch.Tensor | None = None   # int32 [n, 3]: first window, windows, slot; None: whole blocks only
     combine: torch.Tensor | None = None  # int32 [c, 4]: first row, rows, first slot, shares
     slots: int = 0
+
+
+@dataclass(frozen=True)
+class WaitingNorm:
+    """One or two rows that are ``norm(residual + pending)`` (:meth:`Ops.add_rmsnorm`'s), which the product that reads them makes for
+    itself; the sum goes to ``after``.  :meth:`Ops.waiting_norm` makes one for a matrix, :meth:`Ops.linear` or :meth:`Ops.linear_swiglu` of
+    that matrix takes it in the place of the rows."""
+
+    residual: torch.Tensor
+    pending: torch.Tensor
+    gain: torch.Tensor
+    eps: float
+    gain_offset: float
+    one_rounding: bool
+    after: torch.Tensor
+
+    @property
+    def dtype(self) -> torch.dtype:
+        return self.gain.dtype
+
+    @property
+    def device(self) -> torch.device:
+        return self.gain.device
 
 
 class Ops:
@@ -2680,6 +2705,54 @@ class Ops:
                                         splits, tile, *glu_rule(rule), self.stream()), "ts_gemm_stream")
         return out if gated else partial
 
+    #: Rows up to which a product makes the norm that it reads (``csrc/gemm_stream.hip``).
+    normed_max_rows = 2
+
+    def waiting_norm(self, residual: torch.Tensor, pending: torch.Tensor | None, gain: torch.Tensor, eps: float, matrix: torch.Tensor, *,
+                     gated: bool, gain_offset: float = 0.0, one_rounding: bool = False) -> WaitingNorm | None:
+        """``norm(residual + pending)`` for the product by ``matrix`` (``gated``: :meth:`linear_swiglu`'s) to make, or None where the
+        streaming product does not take it: one or two bfloat16 rows of whole slices of 64, in all at most 6,144 elements, that up to
+        four 32-bit partial sums are to be added to.  The launch of the norm falls away.  ``residual`` keeps its
+        values; ``after`` of the result is the sum once that product has run."""
+        rows, hidden = residual.shape
+        if (rows > self.normed_max_rows or pending is None or pending.dim() != 3 or pending.shape[0] > 4 or rows * hidden > 6144 or hidden % 64
+                or gain.dtype is not torch.bfloat16 or matrix.dtype is not torch.bfloat16 or matrix.shape[1] != hidden
+                or not pending.is_contiguous() or not residual.is_contiguous() or not gain.is_contiguous() or not matrix.is_contiguous()
+                or (residual.data_ptr() | pending.data_ptr() | gain.data_ptr() | matrix.data_ptr()) % 16):
+            return None
+        n = matrix.shape[0]
+        if n <= 32 * (-(-hidden // 1024) - 1) or (gated and n % 2):
+            return None
+        plan = self._stream_plan(n, hidden, 1 if gated else None)
+        if plan is None:
+            return None
+        if gated:
+            shared = self._stream_plan(n, hidden, None)
+            if shared is not None and self._stream_cost(n, hidden, 1) > self._stream_cost(n, hidden, shared[1]) + 2.6:
+                return None  # linear_swiglu takes several ranges and the unit's own launch
+        _gpu(residual, pending, gain, matrix)
+        _need(pending.dtype == torch.float32 and pending.shape[1:] == (rows, hidden), f"pending: partial sums must be float32 [S, {rows}, {hidden}]")
+        _need(residual.dtype == torch.float32 and gain.shape == (hidden,), "residual must be float32 [T, H], the gain [H]")
+        return WaitingNorm(residual, pending, gain, float(eps), float(gain_offset), bool(one_rounding), torch.empty_like(residual))
+
+    def _normed_product(self, norm: WaitingNorm, weight: torch.Tensor, bias: torch.Tensor | None, *, gated: bool,
+                        rule: tuple[float, ...] = (1.0, 0.0, 0.0)) -> torch.Tensor:
+        """:meth:`gemm_stream` of the rows that ``norm`` stands for, which the same launch makes."""
+        (m, k), n = norm.residual.shape, weight.shape[0]
+        if bias is not None:
+            _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous(), "bias must be bfloat16 [N]")
+        per_wave, splits, _ = self._stream_plan(n, k, 1 if gated else None)
+        partial = out = None
+        if gated:
+            out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=weight.device)
+        else:
+            partial = torch.empty((splits, m, n), dtype=torch.float32, device=weight.device)
+        _check(self.core.ts_gemm_stream_normed(_ptr(partial), _ptr(out), _ptr(norm.residual), _ptr(norm.pending), norm.pending.shape[0],
+                                               _ptr(norm.after), _ptr(norm.gain), norm.eps, norm.gain_offset, 1 if norm.one_rounding else 0,
+                                               _ptr(weight), _ptr(bias), m, n, k, per_wave, splits, *glu_rule(rule), self.stream()),
+               "ts_gemm_stream_normed")
+        return out if gated else partial
+
     def gemm_resident(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
                       *, max_splits: int | None = None) -> torch.Tensor:
         """The same partial sums by the kernel that keeps a split's activations resident in LDS and
@@ -2901,7 +2974,7 @@ class Ops:
     #: 0.62% instead of 0.66%).
     library_residual_float32 = False
 
-    def linear_swiglu(self, x: torch.Tensor, weight: torch.Tensor,
+    def linear_swiglu(self, x: torch.Tensor | WaitingNorm, weight: torch.Tensor,
                       rule: tuple[float, float, float] | None = None, bias: torch.Tensor | None = None) -> torch.Tensor:
         """The gated unit of the projection of ``x`` by a gate|up matrix ``[2 I, K]`` whose rows
         alternate gate, up (and a bias ``[2 I]`` that alternates likewise) -> ``[T, I]`` in the dtype of ``x``: ``silu(gate) * up``, or another
@@ -2909,6 +2982,8 @@ class Ops:
         apply the unit in the product's own kernel; every other case is the projection followed
         by :meth:`swiglu`."""
         rule = (1.0, 0.0, 0.0) if rule is None else tuple(float(v) for v in rule)
+        if isinstance(x, WaitingNorm):
+            return self._normed_product(x, weight, bias, gated=True, rule=rule)
         if x.dtype == torch.bfloat16 and self.skinny_supported(x, weight) and x.shape[0] <= self.skinny_max_rows:
             _gpu(x, weight, bias)
             block = self._block_few_runs(x, weight, bias, 1)
@@ -2962,7 +3037,7 @@ class Ops:
             self._block_plans[key] = sums if soon else None
         return self._block_plans[key]
 
-    def linear(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *,
+    def linear(self, x: torch.Tensor | WaitingNorm, weight: torch.Tensor, bias: torch.Tensor | None = None, *,
                for_residual: bool = False, for_store: bool = False) -> torch.Tensor:
         """The projection of the serving path.  32-bit runs use :meth:`gemm_plain` (no reduced
         matrix mode).  bfloat16 runs with decode-sized batches (up to ``skinny_max_rows`` rows) use
@@ -2976,7 +3051,10 @@ class Ops:
         norm adds to the 32-bit residual stream, so it may stay 32-bit partial sums ``[S, M, N]``, and
         with ``library_residual_float32`` it always does (as ``[1, M, N]`` where it is one range):
         the stream then gets the same unrounded addend from a prompt's step as from a decode step's.  ``for_store``: the result goes to
-        :meth:`rope_store`, which takes either; a prompt of few rows may leave partial sums (``_sums_plan``)."""
+        :meth:`rope_store`, which takes either; a prompt of few rows may leave partial sums (``_sums_plan``).  ``x`` may be a
+        :class:`WaitingNorm` that was made for ``weight``."""
+        if isinstance(x, WaitingNorm):
+            return self._normed_product(x, weight, bias, gated=False)
         if x.dtype == torch.float32:
             return self.gemm_plain(x, weight, bias)
         if x.shape[0] <= self.skinny_max_rows:

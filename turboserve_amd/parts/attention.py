@@ -276,6 +276,9 @@ class GroupedQueryAttention(Mixer):
             self.mix_weight = float(tensors[self.name(self.value_mix["name"])].float().item())
         self.position.load(tensors)
 
+    def first_matrix(self) -> tuple[torch.Tensor, bool]:
+        return self.qkv_weight, False
+
     def forward(self, x: torch.Tensor, ctx, cache) -> torch.Tensor:
         return self.runtime.ops.linear(self.heads_out(x, ctx, cache), self.o_weight, self.o_bias_tensor, for_residual=True)
 

@@ -228,6 +228,11 @@ class Part:
         alike.  The part finds them as ``ctx.extras[name]``."""
         return ()
 
+    def first_matrix(self) -> "tuple[torch.Tensor, bool] | None":
+        """The matrix (and whether :meth:`Ops.linear_swiglu` multiplies it) whose product is all that this part reads of its input in the
+        run's own kernels: its input may then be a ``WaitingNorm``.  None: it reads the rows."""
+        return None
+
     def activation_bytes(self, tokens: int, itemsize: int) -> int:
         """Bytes of the transient tensors this part holds at once in a step of ``tokens`` rows
         (``itemsize``: bytes of a run-dtype element).  The engine sums these over the model to
@@ -247,6 +252,11 @@ class Norm(Part):
         sum in the run dtype.  With ``rows`` only those rows are read and returned, and the
         stream is left as it is."""
         raise NotImplementedError
+
+    def waiting(self, stream: ResidualStream, matrix: torch.Tensor, gated: bool) -> "WaitingNorm | None":
+        """What :meth:`forward_residual` returns, for the product by ``matrix`` to make (``Ops.waiting_norm``), the stream left as behind
+        it; or None, the stream untouched, where the norm runs by itself."""
+        return None
 
     def pending_rule(self, scale: float) -> "tuple | PendingLayerNorm":
         """This norm as the rule of a pending output (``ResidualStream.pending_norm``): ``(gain, eps,

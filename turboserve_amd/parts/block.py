@@ -66,12 +66,21 @@ class PreNormBlock(Block):
         for part in self.parts():
             part.load(tensors)
 
+    def _normed(self, norm, part: Part, stream: ResidualStream):
+        """The norm of the stream for ``part``: its rows, or, in a step of one or two, what its first product makes them from."""
+        if stream.residual.shape[0] <= self.runtime.ops.normed_max_rows:
+            first = part.first_matrix()
+            waiting = None if first is None else norm.waiting(stream, *first)
+            if waiting is not None:
+                return waiting
+        return norm.forward_residual(stream)
+
     def forward(self, stream: ResidualStream, ctx, cache: CacheView) -> ResidualStream:
-        x = self.mixer_norm.forward_residual(stream)
+        x = self._normed(self.mixer_norm, self.mixer, stream)
         stream.pending = self.mixer.forward(x, ctx, cache)
         if self.feed_forward is None:
             return stream
-        x = self.ff_norm.forward_residual(stream)
+        x = self._normed(self.ff_norm, self.feed_forward, stream)
         stream.pending = self.feed_forward.forward(x, ctx)
         return stream
 

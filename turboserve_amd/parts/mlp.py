@@ -62,6 +62,9 @@ class SwiGLU(FeedForward):
             gate, up, self.down_bias = (tensors[self.name(f"{n}.b")].contiguous() for n in (self.gate_name, self.up_name, self.down_name))
             self.gate_up_bias = torch.stack([gate, up], dim=1).reshape(-1).contiguous()
 
+    def first_matrix(self) -> tuple[torch.Tensor, bool]:
+        return self.gate_up_weight, True
+
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         ops = self.runtime.ops
         units = ops.linear_swiglu(x, self.gate_up_weight, self.rule, self.gate_up_bias)
@@ -99,6 +102,9 @@ class ActivatedMLP(FeedForward):
     def load(self, tensors: Mapping[str, torch.Tensor]) -> None:
         self.up_weight = tensors[self.name(self.up_name)].contiguous()
         self.down_weight = tensors[self.name(self.down_name)].contiguous()
+
+    def first_matrix(self) -> tuple[torch.Tensor, bool]:
+        return self.up_weight, False
 
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         ops = self.runtime.ops

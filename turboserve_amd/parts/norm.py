@@ -55,6 +55,15 @@ class RMSNorm(Norm):
             stream.pending = stream.also = stream.pending_norm = None
         return y
 
+    def waiting(self, stream: ResidualStream, matrix: torch.Tensor, gated: bool):
+        if stream.also is not None or stream.pending_norm is not None:
+            return None
+        norm = self.runtime.ops.waiting_norm(stream.residual, stream.pending, self.weight, self.eps, matrix, gated=gated,
+                                             gain_offset=self.gain_offset, one_rounding=self.one_rounding)
+        if norm is not None:
+            stream.residual, stream.pending = norm.after, None
+        return norm
+
     def pending_rule(self, scale: float) -> tuple:
         if self.gain_offset != 0.0:
             raise ValueError(f"{self.prefix}: a norm on a pending output takes its gain as stored (no offset)")
