@@ -2272,7 +2272,7 @@ class Ops:
     #: The block product's tiles (in 32 weight rows, 32 activation rows) and what an iteration of
     #: 64 of K takes a compute unit with each, in microseconds: the slope over K of products at 144
     #: to 2,048 rows that give every compute unit a workgroup.
-    _BLOCK_TILES = {(8, 8): 1.24, (7, 8): 1.14, (8, 6): 0.99, (6, 8): 1.01, (8, 5): 0.86, (5, 10): 1.07, (5, 8): 0.88, (4, 8): 0.76, (7, 4): 0.73, (4, 5): 0.54,
+    _BLOCK_TILES = {(8, 8): 1.24, (7, 8): 1.14, (8, 6): 0.99, (6, 8): 1.01, (8, 5): 0.86, (5, 10): 1.07, (5, 8): 0.88, (4, 8): 0.76, (7, 4): 0.755, (4, 5): 0.54,
                     (4, 4): 0.50}
 
     @staticmethod
@@ -2295,7 +2295,7 @@ class Ops:
         bytes per nanosecond.  Against every tile with 1 to 16 ranges, timed for the matrices of six shapes (K 2,048 to 18,944) at 144 to
         2,048 rows, the plan's grid takes 1% more than the fastest on average.  The tiles of 192 and 224 weight rows fill rounds that the others
         leave in part empty (us: 3,584 x 18,944 at 2,048 rows, two ranges, 256 workgroups of 224 x 256 195 against 224 of 256 x 256 210, 3,584 x
-        3,584 of 224 x 128 45 against 224 of 128 x 256 47, 7,168 x 5,120 107 against 113; 57 of 14 matrices' grids at 129 to 2,048 rows changed with
+        3,584 of 224 x 128 45 against 224 of 128 x 256 47, 7,168 x 5,120 107 against 113; some 60 of 14 matrices' grids at 129 to 2,048 rows changed with
         them, 5% sooner on average); as several ranges those of 224 are taken only where they do fill them, to nine tenths.
         ``kind``: "sums" (partial sums may stay), "store" (up to four of them, what the store of heads asks for at once), "one"
         (one bfloat16 result), "gated"."""
