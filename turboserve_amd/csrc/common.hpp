@@ -140,13 +140,40 @@ struct GluRule {
   float cubic;
 };
 
-__device__ __forceinline__ float gated_unit(float g, float u, GluRule rule) {
+// g * sigmoid(x) for |x| up to GATE_NEAR: 2^t of the hardware with t = -x log2(e) rounded, and the quotient by 1 + 2^t of the hardware's reciprocal,
+// corrected once by its remainder, into which goes what the rounding of t left (-x - t ln 2, ln 2 in two parts).  Twelve instructions where
+// expf and a division of any numbers are 24; relative to 64 bits 3.1e-8 to 3.6e-8 (root mean square over gates of 1 to 80) where those
+// were 3.7e-8 to 4.0e-8.  No factor, divisor or quotient is beyond the normal numbers there, but for those of a denormal g.
+constexpr float GATE_NEAR = 80.f;
+__device__ __forceinline__ float gated_near(float g, float x) {
+  const float t = x * -1.44269502f;
+  const float left = fmaf(t, 1.90465432e-9f, fmaf(t, -0.693147182f, -x));
+  const float e = __builtin_amdgcn_exp2f(t), r = __builtin_amdgcn_rcpf(1.f + e), q = g * r;
+  return fmaf(fmaf(-(q * e), left, fmaf(-q, e, g) - q), r, q);
+}
+
+// The same beyond (and for NaN): the sigmoid is 1, or e^x, 2^64 times which is a normal number where the result is not 0.
+__device__ __forceinline__ float gated_far(float g, float x) {
+#pragma clang fp contract(off)  // t is rounded, t + 64 then exact where the sum is below t
+  const float y = fmaxf(x, -4000.f), t = y * 1.44269502f;
+  const float left = fmaf(t, 1.90465432e-9f, fmaf(t, -0.693147182f, y));
+  const float e = __builtin_amdgcn_exp2f(t + 64.f), p = g * e;
+  return x > 0.f ? g : (p + fmaf(p, left, fmaf(g, e, -p))) * 5.42101086e-20f;
+}
+
+// The operands within the rule's limits, and what the sigmoid is taken of.
+__device__ __forceinline__ void glu_limits(float& g, float& u, float& x, GluRule rule) {
   if (rule.limit > 0.f) {
     g = fminf(g, rule.limit);
     u = fminf(fmaxf(u, -rule.limit), rule.limit);
   }
-  const float inner = rule.cubic != 0.f ? fmaf(rule.cubic * g * g, g, g) : g;
-  return g / (1.f + expf(-(rule.steepness * inner))) * (u + rule.up_shift);
+  x = rule.steepness * (rule.cubic != 0.f ? fmaf(rule.cubic * g * g, g, g) : g);
+}
+
+__device__ __forceinline__ float gated_unit(float g, float u, GluRule rule) {
+  float x;
+  glu_limits(g, u, x, rule);
+  return (fabsf(x) <= GATE_NEAR ? gated_near(g, x) : gated_far(g, x)) * (u + rule.up_shift);
 }
 
 // One rotation, written out so that every kernel rounds it the same way.

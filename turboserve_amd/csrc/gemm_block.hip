@@ -55,14 +55,28 @@ __device__ __forceinline__ uint32_t block_pack(float lo, float hi) {
   return both;
 }
 
-// The two outputs that a lane holds of a tile, whose rows alternate gate, up: gated_unit as every kernel computes it.  (The
-// hardware's 2^x and reciprocal alone take 5 us less over a block of 256 x 256, gate|up at 2,048 rows 425 us instead of 438, but
-// their error is a tenth larger and gates below -87.3, whose reciprocal is a denormal, come out as 0.)  PLAIN: a rule
-// without limit and cubic.
-template <bool PLAIN>
-__device__ __forceinline__ uint32_t block_units(f32x4 v, GluRule rule) {
-  if (PLAIN) rule.limit = 0.f, rule.cubic = 0.f;
-  return block_pack(gated_unit(v[0], v[1], rule), gated_unit(v[2], v[3], rule));
+// The outputs that a lane holds of COUNT tiles, two of each, whose rows alternate gate, up: gated_unit's bits, by the form for gates up to
+// GATE_NEAR alone where the wavefront has no other.  SILU: the rule is g sigmoid(g) u.
+template <bool SILU, int COUNT>
+__device__ __forceinline__ void block_units(const f32x4 (&v)[COUNT], GluRule rule, uint32_t (&units)[COUNT]) {
+  float g[2 * COUNT], u[2 * COUNT], x[2 * COUNT], most = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2 * COUNT; ++i) {
+    g[i] = v[i / 2][2 * (i % 2)], u[i] = v[i / 2][2 * (i % 2) + 1];
+    if (SILU) x[i] = g[i];
+    else glu_limits(g[i], u[i], x[i], rule);
+    most = fmaxf(most, fabsf(x[i]));  // (a NaN stays one either way)
+  }
+  if (__ballot(most > GATE_NEAR) == 0) {
+#pragma unroll
+    for (int i = 0; i < 2 * COUNT; ++i) g[i] = gated_near(g[i], x[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2 * COUNT; ++i) g[i] = fabsf(x[i]) <= GATE_NEAR ? gated_near(g[i], x[i]) : gated_far(g[i], x[i]);
+  }
+#pragma unroll
+  for (int t = 0; t < COUNT; ++t)
+    units[t] = block_pack(g[2 * t] * (SILU ? u[2 * t] : u[2 * t] + rule.up_shift), g[2 * t + 1] * (SILU ? u[2 * t + 1] : u[2 * t + 1] + rule.up_shift));
 }
 
 // Odd rows of sixteen lanes of a against even rows of b; the upper 32 lanes of a against the lower 32 of b.
@@ -126,7 +140,7 @@ typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 // read has come through an asm behind the wait for its loads (ws, xs; a value the compiler cannot follow, so no read moves above
 // it, nor is one read taken for another), what is read of a slot is in registers that an asm before the wait takes (xf[1], wf)
 // or that matrix instructions pinned ahead of it have used (xf[0]), and every slot is filled again behind that wait.
-// out: bfloat16 [m, n] (mode 0), partial: float [splits, m, n] (mode 1), out: bfloat16 [m, n / 2] (mode 2; 3: any rule
+// out: bfloat16 [m, n] (mode 0), partial: float [splits, m, n] (mode 1), out: bfloat16 [m, n / 2] (mode 2: silu; 3: any rule
 // of the gated unit.  Two kernels: with both epilogues behind one loop the compiler moved the sums between registers in it).
 template <int TN, int TM, int MODE, bool ONCE>
 __device__ __forceinline__ void
@@ -377,9 +391,9 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
         }
       } else {
         mine += group;
+        const f32x4 four[4] = {acc[a][b], acc[a + 1 % SHARE][b], acc[a + 2 % SHARE][b], acc[a + 3 % SHARE][b]};
         uint32_t u[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) u[t] = block_units<MODE == 2>(acc[a + t % SHARE][b], rule);
+        block_units<MODE == 2>(four, rule, u);
         const u32x2 even = block_swap32(u[0], u[2]), odd = block_swap32(u[1], u[3]);
         const u32x2 low = block_swap16(even[0], odd[0]), high = block_swap16(even[1], odd[1]);
         v = u32x4{low[0], low[1], high[0], high[1]};
@@ -390,10 +404,14 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
 #pragma unroll
     for (int a = TN / SHARE * SHARE; a < TN; ++a) {
       const int at = a < tiles ? row_at + a * tile_bytes + tile_bytes / 4 * group : OUTSIDE;
-      if (MODE == 0)
+      if (MODE == 0) {
         __builtin_amdgcn_raw_buffer_store_b64(u32x2{block_pack(acc[a][b][0], acc[a][b][1]), block_pack(acc[a][b][2], acc[a][b][3])}, ybuf, at, 0, 0);
-      else
-        __builtin_amdgcn_raw_buffer_store_b32(block_units<MODE == 2>(acc[a][b], rule), ybuf, at, 0, 0);
+      } else {
+        const f32x4 one[1] = {acc[a][b]};
+        uint32_t u[1];
+        block_units<MODE == 2>(one, rule, u);
+        __builtin_amdgcn_raw_buffer_store_b32(u[0], ybuf, at, 0, 0);
+      }
     }
   }
 }
@@ -454,7 +472,7 @@ extern "C" int ts_gemm_block(float* partial, void* out, const void* x, long x_st
   if (iters_per_split < 1 || splits != (total + iters_per_split - 1) / iters_per_split) return TS_ERR_SHAPE;
   if (mode != 1 && splits != 1) return TS_ERR_ARG;
   const GluRule rule = {steepness, limit, up_shift, cubic};
-  const bool plain = limit <= 0.f && cubic == 0.f;
+  const bool plain = steepness == 1.f && limit <= 0.f && up_shift == 0.f && cubic == 0.f;
 #define TS_BLOCK_MODE(TN, TM, MODE, ONCE)                                                                                    \
   return launch_block_kernel<TN, TM, MODE, ONCE>(partial, (uint16_t*)out, (const uint16_t*)x, x_stride, (const uint16_t*)w,  \
                                                  (const uint16_t*)bias, m, n, k, iters_per_split, splits, whole_n, rule, stream)
