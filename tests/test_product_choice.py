@@ -126,6 +126,21 @@ def test_a_norm_waits_for_a_product_that_makes_it(monkeypatch):
     assert ops.waiting_norm(torch.empty(1, 3584, device="meta"), parts, gain, 1e-6, matrix, gated=False) is None
 
 
+def test_the_store_of_heads_adds_up_what_few_rows_leave():
+    """A prompt's q|k|v as two to four 32-bit sums wherever those are the model's cheapest grid (up to ``wide_default_rows`` rows), one result elsewhere."""
+    ops = Planner()
+
+    def ranges(m, n, k):
+        plan = ops._sums_plan(*operands(m, n, k), None)
+        return plan and plan[1]
+
+    for n, k in ((4608, 3584), (7168, 5120), (3072, 2048), (1536, 1024)):
+        for m in range(129, 513, 19):
+            assert 2 <= ranges(m, n, k) <= 4, (m, n, k)
+        assert ranges(128, n, k) is None and ranges(641, n, k) is None and ranges(2048, n, k) is None
+    assert ranges(640, 4608, 3584) is None and ranges(509, 12288, 4096) is None and ranges(640, 3072, 2048) == 2
+
+
 def test_32_bit_attention_is_asked_only_for_what_it_takes():
     """Pages of 24 keys and pages or rows that 16-byte accesses do not fit stay with the kernel that takes any geometry."""
     ops = Planner()

@@ -2272,7 +2272,7 @@ class Ops:
     #: The block product's tiles (in 32 weight rows, 32 activation rows) and what an iteration of
     #: 64 of K takes a compute unit with each, in microseconds: the slope over K of products at 144
     #: to 2,048 rows that give every compute unit a workgroup.
-    _BLOCK_TILES = {(8, 8): 1.24, (7, 8): 1.14, (8, 6): 0.99, (6, 8): 1.01, (8, 5): 0.86, (5, 10): 1.07, (5, 8): 0.88, (4, 8): 0.76, (7, 4): 0.755, (4, 5): 0.54,
+    _BLOCK_TILES = {(8, 8): 1.24, (7, 8): 1.14, (8, 6): 0.99, (6, 8): 1.01, (8, 5): 0.86, (5, 10): 1.07, (5, 8): 0.88, (4, 8): 0.76, (7, 4): 0.745, (4, 5): 0.54,
                     (4, 4): 0.50}
 
     @staticmethod
@@ -3020,21 +3020,18 @@ class Ops:
     def _sums_plan(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> tuple[int, int, int, int] | None:
         """The block product's grid for a prompt of few rows whose consumer adds up partial sums as well as it takes one result
         (the store of rotated heads), or None where one result is as soon there.  A narrow product as one range of K leaves most
-        units idle: several ranges where the model puts them, their way to the consumer included, at seven tenths of one
-        range's time (us with the store, one result by the library or here / sums: 4,608 x 3,584 at 150 / 200 / 256 / 299 / 350 rows 26.1 / 36.2 /
-        41.1 / 29.0 / 32.3 against 23.1 / 22.3 / 24.9 / 27.2 / 28.3; 7,168 x 5,120 at 150 / 200 / 299 38.2 / 44.6 / 50.7 against 32.2 / 35.6 /
-        43.1; the library's kernels timed for the shape 22.5 / 26.6 / 28.8 / 29.3 / 31.2 and 37.0 / 43.2 / 47.8).  Of a matrix as small as 3,072 x
-        2,048 the sums' way to the store is long beside the product (at 150 / 256 / 400 rows 17.7 / 17.4 / 19.4 against 16.9 / 21.4 / 22.4), but the
-        host, which bounds a short prompt of such a model, is done with them sooner than with the library's call (a step of eight such layers, 222 /
-        300 tokens, 1,155 / 1,165 us with the library, 1,000 / 1,011 with sums)."""
+        units idle, and what few units have on its way to them does not keep a memory busy that the weights come from for the first time:
+        several ranges where the model has them as the cheapest, their way to the consumer included (us with the store, the weights not in any cache, one result by the library or here / sums: 4,608 x 3,584 at 150 / 230 / 299 / 400 / 509 / 640 rows
+        30.8 / 30.0 / 29.6 / 30.9 / 38.4 / 35.5 against 22.1 / 23.5 / 25.8 / 27.4 / 31.5 / 36.5; 7,168 x 5,120 at 230 / 299 / 400 / 509 / 640 43.1 / 48.9 /
+        46.4 / 58.5 / 63.4 against 34.5 / 41.4 / 44.1 / 48.7 / 58.0; 3,072 x 2,048 at 299 / 400 / 509 / 640 21.7 / 21.3 / 25.5 / 25.0 against 18.7 / 21.2 / 24.3 /
+        23.7)."""
         m, (n, k) = x.shape[0], weight.shape
         if not self.skinny_max_rows < m <= self.wide_default_rows or not self.block_supported(x, weight) or (bias is not None and bias.data_ptr() % 8):
             return None
         key = ("sums for the store", m, n, k)
         if key not in self._block_plans:
-            sums, one = self._block_plan(m, n, k, "store"), self._block_plan(m, n, k, "one")
-            soon = sums[1] > 1 and 10 * self._block_cost(m, n, k, sums) <= 7 * self._block_cost(m, n, k, one)
-            self._block_plans[key] = sums if soon else None
+            sums = self._block_plan(m, n, k, "store")
+            self._block_plans[key] = sums if sums[1] > 1 else None
         return self._block_plans[key]
 
     def linear(self, x: torch.Tensor | WaitingNorm, weight: torch.Tensor, bias: torch.Tensor | None = None, *,
