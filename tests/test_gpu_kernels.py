@@ -341,6 +341,31 @@ def test_a_product_that_makes_its_norm(ops, rows, k, sums, one_rounding):
     assert bool(((got - exact @ w.double().T).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("m", [1, 8, 16, 17, 33, 70, 300])
+@pytest.mark.parametrize("n,k", [(4, 32), (36, 96), (1028, 512), (16384, 256)])
+def test_gemm_plain_gated(ops, m, n, k):
+    """A 32-bit gate|up product that applies its unit: the bits of the product followed by the unit's own kernel, in every layout that row counts
+    choose and every tile of the block layout, rows apart; a K that is not whole slices goes the long way."""
+    from turboserve_amd.kernels.ops import GELU_TANH_RULE, KernelError
+
+    g = torch.Generator().manual_seed(m + n)
+    x = torch.full((m, k + 8), float("nan"), device=DEV)[:, :k].copy_(torch.randn(m, k, generator=g))
+    w, b = torch.randn(n, k, generator=g).to(DEV), torch.randn(n, generator=g).to(DEV)
+    for rule, bias in (((1.0, 0.0, 0.0), None), ((1.702, 7.0, 1.0), b), (GELU_TANH_RULE, b)):
+        assert ops._plain_gates(x, w)
+        want = ops.swiglu(ops.gemm_plain(x, w, bias), torch.float32, paired=True, rule=rule)
+        assert torch.equal(ops.linear_swiglu(x, w, rule, bias), want), rule
+        for tile in (2, 3, 7) if m > 64 else ():
+            assert torch.equal(ops.gemm_plain(x, w, bias, tile=tile, gated=rule), want), (tile, rule)
+    for short in (x[:, : k - 4], x[:, 1:]):
+        rows = w[:, : short.shape[1]].contiguous()
+        assert not ops._plain_gates(short, rows)
+        got = ops.linear_swiglu(short, rows)
+        assert torch.equal(got, ops.swiglu(ops.gemm_plain(short, rows), torch.float32, paired=True))
+        with pytest.raises(KernelError):
+            ops.gemm_plain(short, rows, gated=(1.0, 0.0, 0.0))
+
+
 @pytest.mark.parametrize("tile", [2, 3, 4, 5, 6, 7, 8, 9])
 @pytest.mark.parametrize("m,k", [(1, 32), (64, 64), (65, 96), (130, 288), (527, 1056)])
 def test_gemm_plain_block_every_tile(ops, tile, m, k):

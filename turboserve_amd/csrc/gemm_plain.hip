@@ -25,6 +25,12 @@ typedef float gp_f32x4 __attribute__((ext_vector_type(4)));
 typedef float gp_f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int gp_u32x2 __attribute__((ext_vector_type(2)));
 
+// A product whose weight rows alternate gate, up and that leaves the gated unit of each two (32-bit, the layouts that stage through LDS).
+struct PlainGlu {
+  int gated;
+  GluRule rule;
+};
+
 constexpr int GP_DIES = 8;
 constexpr int GP_UNITS = 256;  // compute units of an MI355X
 
@@ -616,7 +622,7 @@ __device__ __forceinline__ void stream_ranges(lds_f32* __restrict__ to, const ld
 template <int MT, int NT, bool ONCE>
 __global__ void __launch_bounds__(256)
 gemm_plain_stream_kernel(float* __restrict__ y, const float* __restrict__ x, const float* __restrict__ w,
-                         const float* __restrict__ bias, int m, int n, int k, long x_stride, long y_stride) {
+                         const float* __restrict__ bias, int m, int n, int k, long x_stride, long y_stride, PlainGlu glu) {
   typedef Stream<MT, NT> S;
   extern __shared__ __attribute__((aligned(16))) float ring[];
   const int lane = threadIdx.x & 63;
@@ -651,14 +657,20 @@ gemm_plain_stream_kernel(float* __restrict__ y, const float* __restrict__ x, con
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = blockIdx.y * 16 * MT + 16 * (t / NT) + 4 * g + i;
-      if (row < m) y[(size_t)row * y_stride + col] = bias ? sum[i] + bv : sum[i];
+      const float v = bias ? sum[i] + bv : sum[i];
+      if (glu.gated) {  // the up value is the next lane's
+        const float up = lanes_moved<0xB1, 0xF>(v, v);  // quad_perm [1,0,3,2]
+        if (row < m && r % 2 == 0) y[(size_t)row * y_stride + col / 2] = gated_unit(v, up, glu.rule);
+      } else if (row < m) {
+        y[(size_t)row * y_stride + col] = v;
+      }
     }
   }
 }
 
 template <int MT, int NT, bool ONCE>
 int launch_stream(void* y, const void* x, const void* w, const void* bias, int m, int n, int k, long x_stride, long y_stride,
-                  dim3 grid, hipStream_t stream) {
+                  dim3 grid, PlainGlu glu, hipStream_t stream) {
   static bool raised = false;  // per process; the attribute belongs to the kernel
   if (!raised) {
     if (hipFuncSetAttribute((const void*)gemm_plain_stream_kernel<MT, NT, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -667,7 +679,7 @@ int launch_stream(void* y, const void* x, const void* w, const void* bias, int m
     raised = true;
   }
   hipLaunchKernelGGL((gemm_plain_stream_kernel<MT, NT, ONCE>), grid, dim3(256), (Stream<MT, NT>::BYTES), stream, (float*)y,
-                     (const float*)x, (const float*)w, (const float*)bias, m, n, k, x_stride, y_stride);
+                     (const float*)x, (const float*)w, (const float*)bias, m, n, k, x_stride, y_stride, glu);
   return ts_launch_status();
 }
 
@@ -695,7 +707,7 @@ struct PlainRing {
 template <int NT>
 __device__ __forceinline__ void plain_block(lds_f32* __restrict__ to, const lds_f32* __restrict__ from, float* __restrict__ y,
                                             const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, int m,
-                                            int n, int k, long x_stride, long y_stride, int m_tiles, int n_tiles) {
+                                            int n, int k, long x_stride, long y_stride, int m_tiles, int n_tiles, PlainGlu glu) {
   typedef PlainRing<NT> R;
   constexpr int SLICE = R::SLICE, SLOT = R::SLOT, SLOTS = R::SLOTS, WLOADS = R::WLOADS, XLOADS = R::XLOADS, FRAGS = NT + 1;
   // Workgroup id -> tile: ids go to the eight dies in turn; a die takes an eighth of the tiles, which follow one another over eight tiles of
@@ -849,21 +861,26 @@ __device__ __forceinline__ void plain_block(lds_f32* __restrict__ to, const lds_
 #pragma unroll
       for (int i = 0; i < 4; ++i) sum[b][i] += bias[col + i];
     }
-    *reinterpret_cast<gp_f32x4*>(y + (size_t)row * y_stride + col) = sum[b];
+    if (glu.gated) {
+      *reinterpret_cast<float2*>(y + (size_t)row * y_stride + col / 2) =
+          make_float2(gated_unit(sum[b][0], sum[b][1], glu.rule), gated_unit(sum[b][2], sum[b][3], glu.rule));
+    } else {
+      *reinterpret_cast<gp_f32x4*>(y + (size_t)row * y_stride + col) = sum[b];
+    }
   }
 }
 
 template <int NT>
 __global__ void __launch_bounds__(256, 2)
 gemm_plain_block_kernel(const float* __restrict__ x, const float* __restrict__ w, int x_stride, int m, int n, int k, int m_tiles, int n_tiles,
-                        float* __restrict__ y, const float* __restrict__ bias, long y_stride) {
+                        float* __restrict__ y, const float* __restrict__ bias, long y_stride, PlainGlu glu) {
   extern __shared__ __attribute__((aligned(16))) float block_ring[];
-  plain_block<NT>((lds_f32*)block_ring, (const lds_f32*)block_ring, y, x, w, bias, m, n, k, x_stride, y_stride, m_tiles, n_tiles);
+  plain_block<NT>((lds_f32*)block_ring, (const lds_f32*)block_ring, y, x, w, bias, m, n, k, x_stride, y_stride, m_tiles, n_tiles, glu);
 }
 
 template <int NT>
 int launch_plain_block(void* y, const void* x, const void* w, const void* bias, int m, int n, int k, long x_stride, long y_stride,
-                       hipStream_t stream) {
+                       PlainGlu glu, hipStream_t stream) {
   static bool raised = false;  // per process; the attribute belongs to the kernel
   if (!raised) {
     if (hipFuncSetAttribute((const void*)gemm_plain_block_kernel<NT>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -874,7 +891,7 @@ int launch_plain_block(void* y, const void* x, const void* w, const void* bias, 
   const long m_tiles = ceil_of(m, 64), n_tiles = ceil_of(n, 16 * NT), ids = ceil_of(m_tiles * n_tiles, GP_DIES) * GP_DIES;
   if (ids > 0x7fffffffL) return TS_ERR_SHAPE;
   hipLaunchKernelGGL((gemm_plain_block_kernel<NT>), dim3((unsigned)ids), dim3(256), (PlainRing<NT>::BYTES), stream, (const float*)x,
-                     (const float*)w, (int)x_stride, m, n, k, (int)m_tiles, (int)n_tiles, (float*)y, (const float*)bias, y_stride);
+                     (const float*)w, (int)x_stride, m, n, k, (int)m_tiles, (int)n_tiles, (float*)y, (const float*)bias, y_stride, glu);
   return ts_launch_status();
 }
 
@@ -913,7 +930,7 @@ inline int plain_kind(int m, int n, bool stream_reads, bool block) {
 
 template <typename TIn, typename TOut>
 int launch_plain(void* y, const void* x, const void* w, const void* bias, int m, int n, int k, long x_stride,
-                 long y_stride, int tile, hipStream_t stream) {
+                 long y_stride, int tile, PlainGlu glu, hipStream_t stream) {
   const size_t quad = 4 * sizeof(TIn);
   const bool vec = k % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)x % quad == 0 && (uintptr_t)w % quad == 0 &&
                    x_stride < (1L << 25) && k < (1 << 25);
@@ -932,8 +949,8 @@ int launch_plain(void* y, const void* x, const void* w, const void* bias, int m,
   do {                                                                                                               \
     dim3 grid((unsigned)ceil_of(n, 16 * NT), (unsigned)ceil_of(m, 16 * MT));                                         \
     if (stream_reads)                                                                                                \
-      return grid.y == 1 ? launch_stream<MT, NT, true>(y, x, w, bias, m, n, k, x_stride, y_stride, grid, stream)     \
-                         : launch_stream<MT, NT, false>(y, x, w, bias, m, n, k, x_stride, y_stride, grid, stream);   \
+      return grid.y == 1 ? launch_stream<MT, NT, true>(y, x, w, bias, m, n, k, x_stride, y_stride, grid, glu, stream)     \
+                         : launch_stream<MT, NT, false>(y, x, w, bias, m, n, k, x_stride, y_stride, grid, glu, stream);   \
     if (vec && sizeof(TIn) == 2)                                                                                     \
       hipLaunchKernelGGL((gemm_plain_few_rows_kernel<MT, NT, AHEAD, sizeof(TIn) == 2, TIn, TOut>), grid, dim3(256),  \
                          0, stream, TS_PLAIN_ARGS);                                                                  \
@@ -949,13 +966,13 @@ int launch_plain(void* y, const void* x, const void* w, const void* bias, int m,
     }
   }
   // The block layout's stores and loads are 16 bytes, its slices whole, its tiles' rows within 31 bits of the first one.
-  const bool block = stream_reads && k % 32 == 0 && n % 4 == 0 && y_stride % 4 == 0 && (uintptr_t)y % 16 == 0 && x_stride < (1L << 21) &&
+  const bool block = stream_reads && k % 32 == 0 && n % 4 == 0 && y_stride % (glu.gated ? 2 : 4) == 0 && (uintptr_t)y % 16 == 0 && x_stride < (1L << 21) &&
                      k < (1 << 21);
-  if (tile != 0 && (!block || tile < 2 || tile > 9)) return TS_ERR_SHAPE;
+  if ((tile != 0 && (!block || tile < 2 || tile > 9)) || (glu.gated && !block)) return TS_ERR_SHAPE;
   const int kind = tile ? BLOCK + tile : plain_kind(m, n, stream_reads, block);
   if constexpr (sizeof(TIn) == 4 && sizeof(TOut) == 4) {
 #define TS_PLAIN_BLOCK(NT) \
-  if (kind == BLOCK + NT) return launch_plain_block<NT>(y, x, w, bias, m, n, k, x_stride, y_stride, stream)
+  if (kind == BLOCK + NT) return launch_plain_block<NT>(y, x, w, bias, m, n, k, x_stride, y_stride, glu, stream)
     TS_PLAIN_BLOCK(2);
     TS_PLAIN_BLOCK(3);
     TS_PLAIN_BLOCK(4);
@@ -996,15 +1013,18 @@ int launch_plain(void* y, const void* x, const void* w, const void* bias, int m,
 
 // dtype: type of x, w and bias.  out_f32 != 0: y is float whatever dtype is.  tile: 0, or 2 to 9, tiles of 64 x 16 tile outputs by the block
 // layout, where it takes the operands.
+// gated != 0 (32-bit, n and k multiples of 4 and 32, operands and strides on 16 bytes): y is [m, n / 2], the gated unit (common.hpp) of rows that
+// alternate gate, up.
 extern "C" int ts_gemm_plain(void* y, const void* x, const void* w, const void* bias, int m, int n,
-                             int k, long x_stride, long y_stride, int dtype, int out_f32, int tile,
-                             hipStream_t stream) {
+                             int k, long x_stride, long y_stride, int dtype, int out_f32, int tile, int gated, float steepness, float limit,
+                             float up_shift, float cubic, hipStream_t stream) {
   if (m == 0 || n == 0) return TS_OK;
-  if (!y || !x || !w || k < 1 || x_stride < k || y_stride < n) return TS_ERR_ARG;
+  if (!y || !x || !w || k < 1 || x_stride < k || y_stride < (gated ? n / 2 : n)) return TS_ERR_ARG;
   if (ceil_of(m, 64) > 65535) return TS_ERR_SHAPE;
-  if (dtype == TS_F32) return launch_plain<float, float>(y, x, w, bias, m, n, k, x_stride, y_stride, tile, stream);
+  const PlainGlu glu = {gated != 0, {steepness, limit, up_shift, cubic}};
+  if (dtype == TS_F32) return launch_plain<float, float>(y, x, w, bias, m, n, k, x_stride, y_stride, tile, glu, stream);
   if (dtype != TS_BF16) return TS_ERR_DTYPE;
-  if (tile != 0) return TS_ERR_SHAPE;
-  if (out_f32) return launch_plain<bf16_t, float>(y, x, w, bias, m, n, k, x_stride, y_stride, 0, stream);
-  return launch_plain<bf16_t, bf16_t>(y, x, w, bias, m, n, k, x_stride, y_stride, 0, stream);
+  if (tile != 0 || gated) return TS_ERR_SHAPE;
+  if (out_f32) return launch_plain<bf16_t, float>(y, x, w, bias, m, n, k, x_stride, y_stride, 0, glu, stream);
+  return launch_plain<bf16_t, bf16_t>(y, x, w, bias, m, n, k, x_stride, y_stride, 0, glu, stream);
 }

@@ -142,7 +142,7 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "ts_moe_combine": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_long, c_void_p, c_int, c_int, c_int,
                            c_int, c_void_p, c_int, c_void_p, c_void_p],
         "ts_gemm_plain": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_long, c_long,
-                          c_int, c_int, c_int, c_void_p],
+                          c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_tiled": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                           c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_wide": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -2100,9 +2100,11 @@ class Ops:
         *,
         out_float32: bool = False,
         tile: int = 0,
+        gated: tuple[float, ...] | None = None,
     ) -> torch.Tensor:
         """``x [M, K] @ weight [N, K]^T (+ bias)`` by 32-bit fused multiply-adds, in the layout that is through soonest.  ``tile`` (2 to 9): in tiles
-        of 64 rows by 16 ``tile`` outputs, where the operands are 32-bit and 16-byte accesses, a K of whole slices of 32 and 31-bit offsets fit."""
+        of 64 rows by 16 ``tile`` outputs, where the operands are 32-bit and 16-byte accesses, a K of whole slices of 32 and 31-bit offsets fit.
+        ``gated``: the rule of :meth:`swiglu`; the weight rows alternate gate, up and the result is ``[M, N / 2]``, where the same fits."""
         _gpu(x, weight, bias)
         _need(x.dim() == 2 and x.stride(1) == 1 and weight.dim() == 2 and weight.is_contiguous(),
               "x must be [M, K] with unit inner stride, weight contiguous [N, K]")
@@ -2112,10 +2114,12 @@ class Ops:
         if bias is not None:
             _need(bias.shape == (n,) and bias.dtype == x.dtype and bias.is_contiguous(), "bias must be [N]")
         out_dtype = torch.float32 if out_float32 else x.dtype
-        y = torch.empty((m, n), dtype=out_dtype, device=x.device)
+        width = n // 2 if gated else n
+        y = torch.empty((m, width), dtype=out_dtype, device=x.device)
         _check(self.core.ts_gemm_plain(_ptr(y), _ptr(x), _ptr(weight), _ptr(bias), m, n, k,
-                                       x.stride(0) if m > 1 else max(k, x.stride(0)), n,
-                                       dtype_code(x.dtype), 1 if out_float32 else 0, tile, self.stream()),
+                                       x.stride(0) if m > 1 else max(k, x.stride(0)), width,
+                                       dtype_code(x.dtype), 1 if out_float32 else 0, tile, 1 if gated else 0,
+                                       *glu_rule(gated or (1.0, 0.0, 0.0)), self.stream()),
                "ts_gemm_plain")
         return y
 
@@ -3015,7 +3019,16 @@ class Ops:
                                lambda: self.swiglu(self._library_product(x, weight, bias, None), x.dtype, paired=True, rule=rule)):
                 return own()
             return self.swiglu(self._library_product(x, weight, bias, None), x.dtype, paired=True, rule=rule)
+        if self._plain_gates(x, weight):
+            return self.gemm_plain(x, weight, bias, gated=rule)
         return self.swiglu(self.linear(x, weight, bias), x.dtype, paired=True, rule=rule)
+
+    @staticmethod
+    def _plain_gates(x: torch.Tensor, weight: torch.Tensor) -> bool:
+        """Whether the 32-bit product applies the gated unit itself (``csrc/gemm_plain.hip``: the layouts that stage whole slices through LDS)."""
+        (n, k), (row, one) = weight.shape, x.stride()
+        return (x.dtype is torch.float32 and one == 1 and weight.is_contiguous() and k % 32 == 0 and n % 4 == 0 and row % 4 == 0
+                and k < 1 << 21 and row < 1 << 21 and (x.data_ptr() | weight.data_ptr()) % 16 == 0)
 
     def _sums_plan(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> tuple[int, int, int, int] | None:
         """The block product's grid for a prompt of few rows whose consumer adds up partial sums as well as it takes one result
