@@ -1429,6 +1429,36 @@ def test_attention_decode_from_projected_sums(ops, monkeypatch, heads, kv_heads,
     torch.testing.assert_close(got[stored].float(), want[stored].float(), rtol=2.0**-7, atol=1e-6)
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim", [(14, 2, 128), (28, 4, 128), (4, 4, 64), (2, 2, 32), (16, 4, 80), (6, 2, 256)])
+@pytest.mark.parametrize("parts", [2, 3, 5, 8])
+@pytest.mark.parametrize("window", [None, 300])
+def test_a_product_that_puts_a_tokens_attention_together(ops, monkeypatch, heads, kv_heads, dim, parts, window):
+    """One request's keys divided over two to eight workgroups, put together by the product that reads the row: the bits of the combining launch and the
+    streaming product of its row where that launch adds up a workgroup's sums one by one (a thread for every workgroup: 1,024 / D of them), else
+    within one bfloat16 unit of every element (2^-8 of its size); workgroups without keys count for nothing, `out` stays as it was."""
+    monkeypatch.setattr(type(ops), "_decode_parts", lambda self, pairs, span, head_dim, shares: parts)
+    for context in (1000, 40):
+        case = PagedCase(torch.bfloat16, heads, kv_heads, dim, 16, [(context, 1)], window, seed=dim + parts)
+        common = (case.dev(case.q), heads * dim, case.dev(case.kp), case.dev(case.vp), case.dev(case.table), case.ints(case.qsl), case.ints([context]), 0, 1,
+                  heads, dim ** -0.5, window, context)
+        g = torch.Generator().manual_seed(dim)
+        row = torch.full((1, heads * dim), float("nan"), dtype=torch.bfloat16, device=DEV)
+        for n in (336, 2060):
+            w, b = (torch.randn(n, heads * dim, generator=g) / 8).bfloat16().to(DEV), torch.randn(n, generator=g).bfloat16().to(DEV)
+            waiting = ops.attention_decode(row, *common, waits_for=w)
+            assert waiting is not None and bool(row.isnan().all())
+            whole = torch.zeros_like(row)
+            assert ops.attention_decode(whole, *common) is None
+            for bias in (None, b):
+                got, want = ops.linear(waiting, w, bias), ops.linear(whole, w, bias)
+                if parts <= 1024 // dim:
+                    assert torch.equal(got, want)
+                room = 2.0**-8 * (whole.double().abs() @ w.double().abs().T)
+                assert bool(((got.double() - want.double()).sum(0).abs() <= room).all())
+    for refused in (w[:, :-8], w.float()):  # another width, another type
+        assert ops.attention_decode(whole, *common, waits_for=refused.contiguous()) is None
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,page", [(14, 2, 128, 8), (7, 1, 128, 64), (4, 4, 64, 32), (20, 1, 80, 16), (6, 2, 256, 8), (2, 2, 32, 64)])
 @pytest.mark.parametrize("waves", [8, 4, 2])
 @pytest.mark.parametrize("splits,window", [(1, None), (3, None), (1, 300)])

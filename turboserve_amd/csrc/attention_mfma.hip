@@ -2018,7 +2018,7 @@ static void prefill_wide_shape(int heads, int kv_heads, int shift, int* per_bloc
 // Decode attention for the requests seq_begin .. seq_begin + requests - 1 of the step, each of
 // which brings one token, a request's windows of 32 keys divided evenly over `splits` workgroups of `waves` wavefronts (8, 4 or 2; heads
 // of more than 128: 4, for 8 as well, or 2).  With one workgroup a request, partial_acc and
-// partial_ml may be null; otherwise they hold requests * heads * splits entries.
+// partial_ml may be null; otherwise they hold requests * heads * splits entries, and are left as they are where `out` is null.
 // The queries are rows of `q`, the new keys and values lie in their pages; or q is null and `sums` are the projection's
 // `sum_splits` partial sums [tokens, (heads + 2 kv_heads) D], `sum_stride` elements apart, which are added up, rotated by the
 // angles of the requests' last positions in cos_table and sin_table [.., D / 2], and stored at `slots` (negative: not stored).
@@ -2036,7 +2036,7 @@ static int launch_decode(uint16_t* out, float* partial_acc, float* partial_ml, c
   hipLaunchKernelGGL((decode_kernel<WAVES, PROJECTED, STAGED>), dim3(splits, kv_heads * head_tiles, requests), dim3(WAVES * TS_WAVE), lds,
                      stream, context_lens, query_start_loc, block_table, table_width, seq_begin, kv_heads, gsize, splits, shift, window,
                      placed ? head_tiles : 0, q_stride, k_pages, v_pages, q, token_sums, rule, out, partial_acc, partial_ml, requests);
-  if (splits == 1) return ts_launch_status();
+  if (splits == 1 || !out) return ts_launch_status();
   if (hipGetLastError() != hipSuccess) return TS_ERR_LAUNCH;
   hipLaunchKernelGGL(decode_reduce_kernel, dim3(requests, heads), dim3(REDUCE_THREADS), 0, stream, out, partial_acc, partial_ml,
                      query_start_loc, seq_begin, heads, splits);
@@ -2050,7 +2050,7 @@ extern "C" int TS_SYM(ts_attention_decode_d)(
     float scale, float softcap, int window, int splits, int waves, const float* sums, long sum_stride, int sum_splits, const float* cos_table,
     const float* sin_table, const int* slots, hipStream_t stream) {
   if (requests == 0) return TS_OK;
-  if (!out || !k_pages || !v_pages || !block_table || !query_start_loc || !context_lens || (q == nullptr) == (sums == nullptr))
+  if ((!out && splits == 1) || !k_pages || !v_pages || !block_table || !query_start_loc || !context_lens || (q == nullptr) == (sums == nullptr))
     return TS_ERR_ARG;
   if (splits > 1 && (!partial_acc || !partial_ml)) return TS_ERR_ARG;
   if (sums && (!cos_table || !sin_table || !slots || sum_splits < 1)) return TS_ERR_ARG;

@@ -393,6 +393,96 @@ int launch_stream_normed(float* partial, void* out, const float* residual, const
   return ts_launch_status();
 }
 
+// The same for the one row that is a token's attention, whose workgroups have left their sums (attention_mfma.hip: partial_acc [heads, splits, d], partial_ml
+// [heads, splits] of reference and sum): every workgroup puts its range of K together, as decode_reduce_kernel does, while its first weights
+// travel (weights below 2^-126 count for nothing here).  That launch took 4.9 us of a layer; 3,584 elements of eight workgroups are 57 KB from L2 for
+// every workgroup of two ranges, and their exponentials and quotients 3: a token of the 7B shape 2,603 -> 2,574 us.
+template <int NT, int ITEMS, int PARTS>
+__global__ void __launch_bounds__(64 * STREAM_WAVES)
+gemm_stream_heads_kernel(const float* __restrict__ partial_acc, const float* __restrict__ partial_ml, const uint16_t* __restrict__ w, int splits_in,
+                         int d, int n, int k, int per_wave, const uint16_t* __restrict__ bias, float* __restrict__ partial) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t ring[];
+  constexpr int THREADS = 64 * STREAM_WAVES;
+  typedef Ring<NT, 0> R;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * 16 * NT, split = blockIdx.y;
+  const int from_quad = split * STREAM_WAVES * per_wave * (R::SLICE / 4), to_quad = min(k / 4, from_quad + STREAM_WAVES * per_wave * (R::SLICE / 4));
+  float part[ITEMS][PARTS][4], m[ITEMS][PARTS], l[ITEMS][PARTS];
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int at = 4 * min(from_quad + (int)threadIdx.x + it * THREADS, to_quad - 1), head = at / d;
+    const size_t base = (size_t)head * splits_in;
+#pragma unroll
+    for (int s = 0; s < PARTS; ++s) {
+      const size_t entry = base + min(s, splits_in - 1);
+      const float2 ml = *(const float2*)(partial_ml + 2 * entry);
+      m[it][s] = ml.x, l[it][s] = ml.y;
+      *(f32x4*)part[it][s] = *(const f32x4*)(partial_acc + entry * d + (at - head * d));
+    }
+  }
+  const int col = n0 + 16 * min(wave, NT - 1) + 4 * (lane >> 4);
+  uint32_t shift[4] = {0, 0, 0, 0};
+  if (bias && split == 0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) shift[i] = bias[min(col + i, n - 1)];
+  }
+  asm volatile("" ::: "memory");  // all of them on their way here
+  __builtin_amdgcn_sched_barrier(0);
+  uint16_t* const held = ring + STREAM_WAVES * R::WAVE;
+  auto combine = [&]() __attribute__((always_inline)) {
+#pragma clang fp contract(off)  // the products rounded before they are added up, as between that kernel's threads
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+      const int quad = from_quad + threadIdx.x + it * THREADS;
+      float most = -INFINITY, weight[PARTS];
+#pragma unroll
+      for (int s = 0; s < PARTS; ++s) most = fmaxf(most, m[it][s]);  // (a share past the last is the last one again)
+#pragma unroll
+      for (int s = 0; s < PARTS; ++s) weight[s] = s >= splits_in || m[it][s] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[it][s] - most);  // no keys
+      float sum[PARTS];
+#pragma unroll
+      for (int s = 0; s < PARTS; ++s) sum[s] = l[it][s] * weight[s];
+#pragma unroll
+      for (int step = 1; step < PARTS; step *= 2) {
+#pragma unroll
+        for (int s = 0; s < PARTS; s += 2 * step) sum[s] += sum[s + step];
+      }
+      uint32_t two[2] = {0, 0};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float num = 0.f;
+#pragma unroll
+        for (int s = 0; s < PARTS; ++s) num += part[it][s][e] * weight[s];
+        two[e / 2] |= (uint32_t)from_float<bf16_t>(num / sum[0]).bits << 16 * (e & 1);
+      }
+      if (quad < to_quad) *(u32x2*)(held + 4 * quad) = u32x2{two[0], two[1]};
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the fence of __syncthreads would wait for the weights)
+  };
+  f32x4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int total = k / R::SLICE, first = (split * STREAM_WAVES + wave) * per_wave, last = min(first + per_wave, total);
+  lds_u16* mine = (lds_u16*)ring + wave * R::WAVE;
+  stream_range<NT, 0, 1>(mine, mine, (const lds_u16*)held, nullptr, w, 1, n, k, 0, n0, first, last, acc, combine);
+  stream_finish<NT, 0, false>((lds_u16*)ring, acc, shift, bias && split == 0, 1, n, col, split, partial, nullptr, GluRule{1.f, 0.f, 0.f, 0.f});
+}
+
+template <int ITEMS, int PARTS>
+int launch_stream_heads(float* partial, const float* partial_acc, const float* partial_ml, int splits_in, int d, const void* w, const void* bias,
+                        int n, int k, int per_wave, int splits, hipStream_t stream) {
+  constexpr size_t BYTES = Ring<2, 0>::BYTES + NORMED_ROOM * 2;
+  static bool raised = false;  // per process; the attribute belongs to the kernel
+  if (!raised) {
+    if (hipFuncSetAttribute((const void*)gemm_stream_heads_kernel<2, ITEMS, PARTS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)BYTES) != hipSuccess)
+      return TS_ERR_LAUNCH;
+    raised = true;
+  }
+  hipLaunchKernelGGL((gemm_stream_heads_kernel<2, ITEMS, PARTS>), dim3((n + 31) / 32, splits), dim3(64 * STREAM_WAVES), BYTES, stream, partial_acc,
+                     partial_ml, (const uint16_t*)w, splits_in, d, n, k, per_wave, (const uint16_t*)bias, partial);
+  return ts_launch_status();
+}
+
 }  // namespace
 
 // x [m, k] bfloat16 (m up to 16, k a multiple of 8) with row stride x_stride; w [n, k] bfloat16 contiguous; bias [n] bfloat16 or
@@ -458,5 +548,30 @@ extern "C" int ts_gemm_stream_normed(float* partial, void* out, const float* res
   TS_NORMED_SUMS(2, 3)
 #undef TS_NORMED_SUMS
 #undef TS_NORMED
+  return TS_ERR_SHAPE;
+}
+
+// The product of one token's attention as its workgroups left it: partial_acc float [heads, parts, d], partial_ml float [heads, parts, 2] (parts 2 to
+// 8), k = heads d, a multiple of 64 and at most 6,144, d of 4; per_wave up to 16.  partial = float [splits, 1, n]; the rest as ts_gemm_stream's.
+extern "C" int ts_gemm_stream_heads(float* partial, const float* partial_acc, const float* partial_ml, int parts, int heads, int d, const void* w,
+                                    const void* bias, int n, int per_wave, int splits, hipStream_t stream) {
+  if (!partial || !partial_acc || !partial_ml || !w) return TS_ERR_ARG;
+  if (parts < 2 || parts > 8 || heads < 1 || d < 4 || d % 4 != 0 || heads > NORMED_MOST || d > NORMED_MOST || n < 1) return TS_ERR_SHAPE;
+  const int k = heads * d;
+  if (k % 64 != 0 || k > NORMED_MOST || ((uintptr_t)partial_acc | (uintptr_t)w) % 16 != 0 || (uintptr_t)partial_ml % 8 != 0) return TS_ERR_SHAPE;
+  if (per_wave < 1 || per_wave > 16 || splits < 1 || splits > 65535 || splits != (k / 64 + 4L * per_wave - 1) / (4L * per_wave)) return TS_ERR_SHAPE;
+  const int items = (per_wave + 3) / 4;
+#define TS_HEADS(ITEMS, PARTS)           \
+  if (items == ITEMS && parts <= PARTS) \
+    return launch_stream_heads<ITEMS, PARTS>(partial, partial_acc, partial_ml, parts, d, w, bias, n, k, per_wave, splits, stream);
+  TS_HEADS(1, 4)
+  TS_HEADS(1, 8)
+  TS_HEADS(2, 4)
+  TS_HEADS(2, 8)
+  TS_HEADS(3, 4)
+  TS_HEADS(3, 8)
+  TS_HEADS(4, 4)
+  TS_HEADS(4, 8)
+#undef TS_HEADS
   return TS_ERR_SHAPE;
 }

@@ -149,6 +149,7 @@ _SIGNATURES: dict[str, dict[str, list]] = {
                          c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_block": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                           c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
+        "ts_gemm_stream_heads": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
         "ts_gemm_stream_normed": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_float, c_float, c_int, c_void_p, c_void_p,
                                   c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_stream": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
@@ -391,6 +392,15 @@ class WaitingNorm:
     @property
     def device(self) -> torch.device:
         return self.gain.device
+
+
+@dataclass(frozen=True)
+class WaitingHeads:
+    """One token's attention as the workgroups that divided its keys have left it, which the product by the output matrix puts together
+    (:meth:`Ops.attention_decode`, :meth:`Ops.linear`): their sums ``[heads, parts, D]``, references and weights ``[heads, parts, 2]``."""
+
+    sums: torch.Tensor
+    weights: torch.Tensor
 
 
 class Ops:
@@ -1864,7 +1874,8 @@ class Ops:
         softcap: float = 0.0,
         projected: tuple | None = None,
         shares: int = 1,
-    ) -> None:
+        waits_for: torch.Tensor | None = None,
+    ) -> WaitingHeads | None:
         """Matrix-core attention for the single-token requests ``seq_begin .. seq_begin +
         requests - 1`` of the step; writes their rows of ``out [T, heads * D]``.  ``max_context``
         (host-known) bounds their context lengths and fixes over how many workgroups a request's keys are
@@ -1873,6 +1884,9 @@ class Ops:
         ``projected = (cos, sin, slots, max_position)``: ``q`` is the fused projection's partial sums ``[S, T, (heads + 2
         kv_heads) D]`` (32-bit); the launch adds them up, rotates queries and keys, stores the new keys and values at
         ``slots`` and attends, in place of :meth:`rope_store` before it (the same bits in the pages).
+
+        ``waits_for``: the matrix ``[N, heads * D]`` whose product (:meth:`linear`) is all that reads ``out``: where that product puts one request's
+        workgroups together itself, ``out`` is left alone and what it takes instead is returned (else None).
 
         ``shares`` (:meth:`decode_shares`): what the requests' own lengths, which ``max_context`` does not tell, make of a
         request's keys where requests and KV heads alone give every compute unit a workgroup."""
@@ -1912,12 +1926,38 @@ class Ops:
         if splits > 1:
             partial_acc = torch.empty((requests * heads * splits, head_dim), dtype=torch.float32, device=out.device)
             partial_ml = torch.empty((requests * heads * splits, 2), dtype=torch.float32, device=out.device)
+        waiting = None
+        if waits_for is not None and requests == 1 and self._heads_wait(splits, heads * head_dim, waits_for):
+            waiting = WaitingHeads(partial_acc.view(heads, splits, head_dim), partial_ml.view(heads, splits, 2))
         lib = load_module(build.attention_module(head_dim))
         fn = getattr(lib, f"ts_attention_decode_d{head_dim}")
-        _check(fn(_ptr(out), _ptr(partial_acc), _ptr(partial_ml), None if projected else _ptr(q), q_stride, _ptr(k_pages), _ptr(v_pages),
+        _check(fn(None if waiting else _ptr(out), _ptr(partial_acc), _ptr(partial_ml), None if projected else _ptr(q), q_stride, _ptr(k_pages), _ptr(v_pages),
                   _ptr(block_table), block_table.shape[1], _ptr(query_start_loc), _ptr(context_lens), seq_begin,
                   requests, heads, kv_heads, block_size, float(scale), float(softcap), int(window or 0), splits,
                   self._decode_waves(pairs * splits, span, head_dim), *new, self.stream()), "ts_attention_decode")
+        return waiting
+
+    def _heads_wait(self, parts: int, k: int, matrix: torch.Tensor) -> bool:
+        """Whether the product by ``matrix [N, K]`` puts together what ``parts`` workgroups left of one request's keys: up to eight (a
+        range of K reads them all, once for every 32 weight rows), of up to 6,144 elements, where the streaming product runs."""
+        if not (2 <= parts <= 8 and k % 64 == 0 and k <= 6144 and matrix.dtype is torch.bfloat16 and matrix.shape[1] == k
+                and matrix.is_contiguous() and matrix.data_ptr() % 16 == 0):
+            return False
+        plan = self._stream_plan(matrix.shape[0], k, None)
+        return plan is not None and plan[0] <= 16
+
+    def _heads_product(self, heads: WaitingHeads, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
+        """:meth:`gemm_stream` of the row that ``heads`` stands for."""
+        _gpu(heads.sums, heads.weights, weight, bias)
+        (count, parts, dim), (n, k) = heads.sums.shape, weight.shape
+        _need(count * dim == k, "heads of another width than the matrix")
+        if bias is not None:
+            _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous(), "bias must be bfloat16 [N]")
+        per_wave, splits, _ = self._stream_plan(n, k, None)
+        partial = torch.empty((splits, 1, n), dtype=torch.float32, device=weight.device)
+        _check(self.core.ts_gemm_stream_heads(_ptr(partial), _ptr(heads.sums), _ptr(heads.weights), parts, count, dim, _ptr(weight), _ptr(bias), n,
+                                              per_wave, splits, self.stream()), "ts_gemm_stream_heads")
+        return partial
 
     def _decode_parts(self, pairs: int, span: int, head_dim: int, shares: int) -> int:
         """How many workgroups a request and KV head get: :meth:`_decode_splits`, or ``shares`` where that leaves long spans whole.  Heads of
@@ -3047,7 +3087,7 @@ class Ops:
             self._block_plans[key] = sums if sums[1] > 1 else None
         return self._block_plans[key]
 
-    def linear(self, x: torch.Tensor | WaitingNorm, weight: torch.Tensor, bias: torch.Tensor | None = None, *,
+    def linear(self, x: torch.Tensor | WaitingNorm | WaitingHeads, weight: torch.Tensor, bias: torch.Tensor | None = None, *,
                for_residual: bool = False, for_store: bool = False) -> torch.Tensor:
         """The projection of the serving path.  32-bit runs use :meth:`gemm_plain` (no reduced
         matrix mode).  bfloat16 runs with decode-sized batches (up to ``skinny_max_rows`` rows) use
@@ -3062,9 +3102,11 @@ class Ops:
         with ``library_residual_float32`` it always does (as ``[1, M, N]`` where it is one range):
         the stream then gets the same unrounded addend from a prompt's step as from a decode step's.  ``for_store``: the result goes to
         :meth:`rope_store`, which takes either; a prompt of few rows may leave partial sums (``_sums_plan``).  ``x`` may be a
-        :class:`WaitingNorm` that was made for ``weight``."""
+        :class:`WaitingNorm` or :class:`WaitingHeads` that was made for ``weight``."""
         if isinstance(x, WaitingNorm):
             return self._normed_product(x, weight, bias, gated=False)
+        if isinstance(x, WaitingHeads):
+            return self._heads_product(x, weight, bias)
         if x.dtype == torch.float32:
             return self.gemm_plain(x, weight, bias)
         if x.shape[0] <= self.skinny_max_rows:

@@ -280,7 +280,7 @@ class GroupedQueryAttention(Mixer):
         return self.qkv_weight, False
 
     def forward(self, x: torch.Tensor, ctx, cache) -> torch.Tensor:
-        return self.runtime.ops.linear(self.heads_out(x, ctx, cache), self.o_weight, self.o_bias_tensor, for_residual=True)
+        return self.runtime.ops.linear(self.heads_out(x, ctx, cache, waits_for=self.o_weight), self.o_weight, self.o_bias_tensor, for_residual=True)
 
     @property
     def out_features(self) -> int:
@@ -304,8 +304,10 @@ class GroupedQueryAttention(Mixer):
         return (not self.position.biases_scores and self.value_dim == self.head_dim and self.chunk is None and self.sinks == 0.0
                 and self.keep_first == 0)
 
-    def heads_out(self, x: torch.Tensor, ctx, cache, *, scale: float = 1.0, out: tuple | None = None) -> torch.Tensor:
-        """Everything but the output matrix: ``[T, Hq Dv]`` of the run dtype, what that matrix multiplies.  Where
+    def heads_out(self, x: torch.Tensor, ctx, cache, *, scale: float = 1.0, out: tuple | None = None,
+                  waits_for: torch.Tensor | None = None) -> torch.Tensor:
+        """Everything but the output matrix: ``[T, Hq Dv]`` of the run dtype, what that matrix multiplies; or, ``waits_for`` being that
+        matrix and its product (``Ops.linear``) all that reads them, what that product makes a single token's row from (``WaitingHeads``).  Where
         :meth:`scales_its_heads` the result may be multiplied by ``scale`` and written into columns of a wider buffer (``out
         = (buffer, col0)``): a caller that adds this mixer's output to another's can then run both output matrices as
         one product."""
@@ -344,7 +346,7 @@ class GroupedQueryAttention(Mixer):
             else:
                 more["values"] = {"blend": (ctx.carried[key], self.mix_weight)}
         if ctx.num_prefill_seqs == 0 and not more and self.gate_name is None and scale == 1.0 and out is None:
-            attended = self._attend_projected(qkv, ctx, cache)
+            attended = self._attend_projected(qkv, ctx, cache, waits_for)
             if attended is not None:
                 return attended
         q, q_stride = self.position.encode_and_store(
@@ -357,7 +359,7 @@ class GroupedQueryAttention(Mixer):
         return ops.head_gate(attended, proj, self.q_size + self.kv_size + self.v_size, self.num_heads, self.runtime.dtype,
                              scale=scale, out=out)
 
-    def _attend_projected(self, qkv: torch.Tensor, ctx, cache: PagedKVView) -> torch.Tensor | None:
+    def _attend_projected(self, qkv: torch.Tensor, ctx, cache: PagedKVView, waits_for: torch.Tensor | None = None) -> torch.Tensor | None:
         """A step of single tokens whose projection came as 32-bit partial sums: one launch adds them up, rotates, stores and
         attends.  ``None`` where the layer or the step asks for more than that launch does."""
         ops = self.runtime.ops
@@ -375,11 +377,12 @@ class GroupedQueryAttention(Mixer):
             return None
         table = ctx.block_tables[cache.group]
         out = ops.rows_buffer(ctx.num_tokens, self.out_size, self.runtime.dtype, qkv.device)
-        ops.attention_decode(
+        waiting = ops.attention_decode(
             out, qkv, 0, cache.k, cache.v, table, ctx.query_start_loc, ctx.context_lens, 0, ctx.num_decode_seqs, self.num_heads,
             self.scale, self.window, min(ctx.max_decode_context_len, table.shape[1] * cache.block_size),
-            softcap=self.softcap, projected=(*tables, ctx.slot_mapping[cache.group], ctx.max_context_len - 1), shares=self._decode_shares(ctx))
-        return out
+            softcap=self.softcap, projected=(*tables, ctx.slot_mapping[cache.group], ctx.max_context_len - 1), shares=self._decode_shares(ctx),
+            waits_for=waits_for)
+        return out if waiting is None else waiting
 
     def _decode_shares(self, ctx) -> int:
         """Into how many workgroups the decode attention divides the requests' keys (``Ops.decode_shares``)."""
