@@ -17,12 +17,11 @@
 // their registers, and the first ones of the next iteration behind the barrier that ends this one's reads,
 // while most of its second step is still to be multiplied; loads are issued two to five iterations ahead.  Loads and reads stand one
 // by one between matrix instructions (in one go they held them up).
-// Measured, microseconds, against the better of gemm_wide and the library's default kernel (with the kernel that reads or
-// makes the result: SwiGLU, or the norm that takes the partial sums), at 299 / 509 / 2,048 rows: gate|up [37888, 3584] 85 / 139 /
-// 441 against 126 / 158 / 560 (1.26 PFLOP/s), down [3584, 18944] 58 / 79 / 246 against 111 / 90 / 291, o [3584, 3584] 26 / 30 / 73
-// against 35 / 34 / 77, q|k|v [4608, 3584] 27 / 28 / 59 against 23 / 31 / 62.  An iteration of 256 x 256 takes 1.01 us where
+// Measured, microseconds, with the kernel that reads or makes the result (the gated unit, the norm that takes the partial sums, the store of heads),
+// weights that no cache holds, at 299 / 509 / 2,048 rows: gate|up [37888, 3584] 81 / 120 / 407 (1.37 PFLOP/s), down [3584, 18944] 56 / 72 /
+// 218, o [3584, 3584] 23 / 29 / 65, q|k|v [4608, 3584] 26 / 32 / 67.  An iteration of 256 x 256 takes 1.01 us where
 // half the compute units have a workgroup and 1.32 where all do (the matrix instructions 0.85 at the full clock of 2.4 GHz; with every unit
-// at work the card holds 1.7 to 1.8); a workgroup's start takes 2 us and its stores 4 (gated 9).
+// at work the card holds 1.7 to 1.8); a workgroup's start takes 2 us and its stores 4 (gated 7).
 // A decode step's product is bound by reading the weights; 160 weight rows by 64 activation rows a workgroup, the weights
 // non-temporal, take gate|up at 64 rows in 44.1 us (gemm_wide 47.5), 128 rows down in 26.6 (28.6), q|k|v in 11.5 (12.0), o in 10.4
 // (11.1); at 128 rows 50 (60), 33 (37), 14.5 (15.3), 13.7 (14.1).
