@@ -53,6 +53,25 @@ def test_an_addend_of_the_residual_stream_keeps_its_32_bits(n, k):
         assert ops._own_product(x, w[:, :-8], None, "sums")[0]()[2], "the wide product too"
 
 
+@pytest.mark.parametrize("n,k,first,last", [(3584, 3584, 1574, 1690), (4608, 3584, 1224, 1314), (3072, 3072, 1601, 1661), (5120, 8192, 1281, 1321),
+                                            (6144, 16384, 1921, 2048)])
+def test_a_wider_tile_takes_no_bits_from_the_residual_stream(n, k, first, last):
+    """Rows at which the tiles of 128, 160 and 256 weight rows are cheapest as several ranges of K, whose sums are 32-bit: the addend stays 32-bit where
+    one range of 192 or 224 weight rows is sooner, too.  Beside them one range is rounded once."""
+    for m in range(first, last + 1):
+        assert Planner()._own_product(*operands(m, n, k), None, "sums")[0]()[2], m
+    assert not Planner()._own_product(*operands(2048, 3584, 3584), None, "sums")[0]()[2]
+
+
+@pytest.mark.parametrize("n,k", [(3584, 18944), (3584, 3584), (5120, 13824), (5120, 5120), (2048, 8192), (2048, 2048), (4096, 14336), (6144, 6144),
+                                 (8192, 29568)])
+def test_an_addend_is_32_bit_wherever_the_first_tiles_leave_it_so(n, k):
+    first = tuple(tile for tile in Ops._BLOCK_TILES if tile[0] in (4, 5, 8))
+    for m in range(641, 2049, 32):
+        ops = Planner()
+        assert ops._own_product(*operands(m, n, k), None, "sums")[0]()[2] >= (ops._block_cheapest(m, n, k, "sums", first)[1] > 1), m
+
+
 def test_one_result_of_a_narrow_product_is_left_to_the_library():
     """A product as one range of K runs the block kernel only from a grid on that fills enough of the device.
     The shapes on the left were up to 2.4 times as slow with it as with the library, those on the right up to 1.5 times as fast."""

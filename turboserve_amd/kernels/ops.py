@@ -2347,9 +2347,29 @@ class Ops:
         known = self._block_plans.get(key)
         if known is not None:
             return known
+        plan = self._block_cheapest(m, n, k, kind, tuple(self._BLOCK_TILES))
+        if kind == "sums" and plan[1] == 1 and m > self.wide_default_rows:
+            ranges = self._block_ranges(m, n, k)
+            if ranges is not None and self._block_cost(m, n, k, ranges) <= self._block_cost(m, n, k, plan) + m * n * 4 / 3.6e6:
+                plan = ranges
+        self._block_plans[key] = plan
+        return plan
+
+    def _block_ranges(self, m: int, n: int, k: int) -> tuple[int, int, int, int] | None:
+        """The plan of several ranges of K, 32-bit sums, that an addend of the residual stream has without the tiles of 192 and 224 weight rows, or None
+        where it is one range, rounded to bfloat16 above ``wide_default_rows`` rows, without them too.  One range of theirs that is sooner takes no
+        bits from the stream: it stays 32-bit there, and its way to the norm counts as the others' does (us with the norm, one range rounded / one
+        range of 32 bits / several: 3,584 x 3,584 at 1,574 to 1,690 rows 55 to 58 / 59 to 62 / 57 to 58, 3,072 x 3,072 at 1,601 to 1,661 49 to 50 /
+        53 to 54 / 48, 5,120 x 8,192 at 1,281 to 1,321 105 to 108 / 110 to 114 / 112 to 113, 6,144 x 16,384 at 1,921 to 2,048 312 to 321 / 320 to
+        330 / 348 to 360)."""
+        plan = self._block_cheapest(m, n, k, "sums", tuple(tile for tile in self._BLOCK_TILES if tile[0] not in (6, 7)))
+        return plan if plan[1] > 1 else None
+
+    def _block_cheapest(self, m: int, n: int, k: int, kind: str, tiles: tuple[tuple[int, int], ...]) -> tuple[int, int, int, int]:
+        """:meth:`_block_plan` among ``tiles``."""
         iters = k // 64
         best = None
-        for tn, tm in self._BLOCK_TILES:
+        for tn, tm in tiles:
             for want in range(1, min(iters, {"sums": 16, "store": 4}.get(kind, 1)) + 1):
                 per_split = -(-iters // want)
                 splits = -(-iters // per_split)
@@ -2361,7 +2381,6 @@ class Ops:
                 cost = self._block_cost(m, n, k, (per_split, splits, tn, tm), kind == "gated")
                 if best is None or cost < best[0]:
                     best = (cost, per_split, splits, tn, tm)
-        self._block_plans[key] = best[1:]
         return best[1:]
 
     def _block_rounds(self, m: int, n: int, k: int, gated: bool, plan: tuple[int, int, int, int]) -> tuple[int, ...]:
@@ -2520,8 +2539,8 @@ class Ops:
             if kind != "sums":
                 block = self._block_rounds(m, n, k, kind == "gated", block)
             # One range too stays 32-bit up to the rows at which gemm_wide's ranges leave partial sums (a plan of one range
-            # there is wide: 16,384 x 16,384), above as the library's result is.
-            sums = float32 or (kind == "sums" and m <= self.wide_default_rows)
+            # there is wide: 16,384 x 16,384), and above where it stands for several (_block_ranges); else it is as the library's result is.
+            sums = float32 or (kind == "sums" and (m <= self.wide_default_rows or (block[1] == 1 and self._block_ranges(m, n, k) is not None)))
             workgroups = -(-n // (32 * block[2])) * -(-m // (32 * block[3])) * block[1]
             runs = runs or (self.wide_default_rows > 0 and workgroups >= self._block_fill(k, kind) * self.compute_units)
             choice = True, block, sums, runs
