@@ -307,15 +307,15 @@ def test_gemm_plain_is_chains_of_fused_multiply_adds(ops, dtype, k, values):
                     assert got[i, j].item() == float(value), (rows, cols, i, j)
 
 
-@pytest.mark.parametrize("rows,k,sums", [(1, 64, 1), (1, 1024, 4), (1, 1088, 2), (2, 2048, 3), (2, 3072, 2), (1, 3584, 2), (1, 5120, 4), (1, 6144, 3)])
+@pytest.mark.parametrize("rows,k,sums", [(1, 64, 1), (1, 1024, 4), (1, 1088, 2), (2, 64, 3), (2, 576, 1), (2, 1024, 2), (2, 1088, 4), (2, 2048, 3), (2, 2624, 1),
+                                         (2, 3072, 2), (1, 2624, 4), (1, 3584, 2), (1, 4096, 1), (1, 4160, 3), (1, 5120, 4), (1, 6144, 3)])
 @pytest.mark.parametrize("one_rounding", [False, True])
 def test_a_product_that_makes_its_norm(ops, rows, k, sums, one_rounding):
-    """One or two rows normalised by the product that reads them: residual and partial sums are small whole numbers, whose squares add up exactly in
-    any order, so the sum, the rows and the product are the bits of the norm's own launch and the streaming product of its rows; as partial sums
-    with a bias, and gated; weight rows that fill no tile; what was in the results before is not read."""
+    """One or two rows normalised by the product that reads them: the sum, the rows and the product are the bits of the norm's own launch and
+    the streaming product of its rows, as partial sums with a bias and gated, so that a row of a step has the same bits beside any others; weight
+    rows that fill no tile; what was in the results before is not read."""
     g = torch.Generator().manual_seed(k + sums)
-    whole = lambda *shape: torch.randint(-3, 4, shape, generator=g).float().to(DEV)  # noqa: E731
-    residual, pending = whole(rows, k), whole(sums, rows, k)
+    residual, pending = torch.randn(rows, k, generator=g).to(DEV), torch.randn(sums, rows, k, generator=g).to(DEV)
     gain, offset = torch.randn(k, generator=g).bfloat16().to(DEV), 1.0 if one_rounding else 0.0
     for n, gated in ((336, False), (214, True), (2064, False), (2064, True)):
         w, b = (torch.randn(n, k, generator=g) / 8).bfloat16().to(DEV), torch.randn(n, generator=g).bfloat16().to(DEV)
@@ -331,8 +331,7 @@ def test_a_product_that_makes_its_norm(ops, rows, k, sums, one_rounding):
         else:
             got, want = ops.linear(norm, w, b), ops.linear(x, w, b)
         assert torch.equal(got, want) and torch.equal(norm.after, after), n
-    # In general the order of the squares differs: half a unit in the last place of each of two bfloat16 roundings, and of the sums.
-    residual, pending = torch.randn(rows, k, generator=g).to(DEV), torch.randn(sums, rows, k, generator=g).to(DEV)
+    # Against 64 bits: half a unit in the last place of each of two bfloat16 roundings, and of the sums.
     norm = ops.waiting_norm(residual, pending, gain, 1e-5, w, gated=False, gain_offset=offset, one_rounding=one_rounding)
     total = residual.double() + pending.double().sum(0)
     exact = total / (total.square().mean(-1, keepdim=True) + 1e-5).sqrt() * (gain.double() + offset)

@@ -69,6 +69,23 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), TS_WAVE - 1));
 }
 
+// The same of N values, step by step beside one another; the last lane holds the sums.
+template <int N>
+__device__ __forceinline__ void wave_sums(float (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += lanes_moved<0xB1, 0xF>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += lanes_moved<0x4E, 0xF>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += lanes_moved<0x141, 0xF>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += lanes_moved<0x140, 0xF>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += lanes_moved<0x142, 0xA>(0.f, v[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] += lanes_moved<0x143, 0xC>(0.f, v[i]);
+}
+
 __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, lanes_moved<0xB1, 0xF>(v, v));
   v = fmaxf(v, lanes_moved<0x4E, 0xF>(v, v));

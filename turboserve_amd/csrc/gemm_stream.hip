@@ -303,14 +303,19 @@ gemm_stream_normed_kernel(const float* __restrict__ residual, const float* __res
   asm volatile("" ::: "memory");  // all of them on their way here
   __builtin_amdgcn_sched_barrier(0);
   uint16_t* const held = ring + STREAM_WAVES * R::WAVE;
-  float(*const sums)[STREAM_WAVES] = reinterpret_cast<float(*)[STREAM_WAVES]>(held + NORMED_ROOM - 2 * ROWS * STREAM_WAVES);  // behind the rows
+  constexpr int CHAINS = ITEMS < 4 ? ITEMS : 4;
+  typedef float chains __attribute__((ext_vector_type(4)));
+  chains(*const sums)[STREAM_WAVES] = reinterpret_cast<chains(*)[STREAM_WAVES]>(held + NORMED_ROOM - 8 * ROWS * STREAM_WAVES);  // behind the rows
+  static_assert(NORMED_MOST + 8 * ROWS * STREAM_WAVES <= NORMED_ROOM, "the wavefronts' sums lie behind the rows");
   auto meet = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };  // (the fence of __syncthreads would wait for the weights)
   // The workgroup's range of K is all it needs normalised.
   const int from_quad = split * STREAM_WAVES * per_wave * (R::SLICE / 4), to_quad = min(quads, from_quad + STREAM_WAVES * per_wave * (R::SLICE / 4));
   auto normalise = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int row = 0; row < ROWS; ++row) {
-      float ss = 0.f;
+      // The squares in add_rmsnorm's order (elementwise.hip, add_rmsnorm_few_kernel), so that a row has its bits in steps of any number of rows: chain
+      // c of this thread is what thread (threadIdx.x + 256 c) of 1,024 adds up, its wavefront's sum the one in place 4 c + wave.
+      float ss[CHAINS];
 #pragma unroll
       for (int it = 0; it < ITEMS; ++it) {
 #pragma unroll
@@ -318,14 +323,14 @@ gemm_stream_normed_kernel(const float* __restrict__ residual, const float* __res
 #pragma unroll
           for (int j = 0; j < SUMS; ++j) s[row][it][e] += part[row][it][j][e];
         }
-        const float one = (int)threadIdx.x + it * THREADS < quads ? 1.f : 0.f;
-        float four = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) four = fmaf(s[row][it][e], s[row][it][e], four);
-        ss += it + 1 < ITEMS || one != 0.f ? four : 0.f;  // all but the last item lie inside the row
+        const float(&v)[4] = s[row][it];
+        const float two = it < CHAINS ? fmaf(v[0], v[0], v[1] * v[1]) : fmaf(v[1], v[1], fmaf(v[0], v[0], ss[it % CHAINS]));
+        const float four = fmaf(v[3], v[3], fmaf(v[2], v[2], two));
+        // All but the last item lie inside the row.
+        ss[it % CHAINS] = it + 1 < ITEMS || (int)threadIdx.x + it * THREADS < quads ? four : it < CHAINS ? 0.f : ss[it % CHAINS];
       }
-      ss = wave_sum(ss);
-      if (lane == 0) sums[row][wave] = ss;
+      wave_sums(ss);
+      if (lane == TS_WAVE - 1) sums[row][wave] = chains{ss[0], ss[1 % CHAINS], ss[2 % CHAINS], ss[3 % CHAINS]};
     }
     meet();
     float rstd[ROWS];
@@ -333,7 +338,7 @@ gemm_stream_normed_kernel(const float* __restrict__ residual, const float* __res
     for (int row = 0; row < ROWS; ++row) {
       float ss = 0.f;
 #pragma unroll
-      for (int v = 0; v < STREAM_WAVES; ++v) ss += sums[row][v];
+      for (int v = 0; v < CHAINS * STREAM_WAVES; ++v) ss += sums[row][v % STREAM_WAVES][v / STREAM_WAVES];
       rstd[row] = rsqrtf(ss / (float)k + eps);
     }
     auto write = [&](auto ONE_ROUNDING) __attribute__((always_inline)) {
