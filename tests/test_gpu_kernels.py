@@ -1458,6 +1458,27 @@ def test_a_product_that_puts_a_tokens_attention_together(ops, monkeypatch, heads
         assert ops.attention_decode(whole, *common, waits_for=refused.contiguous()) is None
 
 
+@pytest.mark.parametrize("parts", [2, 5, 8])
+def test_a_share_of_denormal_weight_counts(ops, parts):
+    """Workgroups whose references lie 127 to 149 below the largest: their weights are denormal numbers, and their values large enough to be all
+    that the row is made of.  Every number is a power of two, so the product is exact."""
+    from turboserve_amd.kernels.ops import WaitingHeads
+
+    heads, dim, n = 4, 64, 336
+    sums, weights = torch.zeros(heads, parts, dim), torch.ones(heads, parts, 2)
+    weights[:, :, 0] = 0.0
+    want = torch.zeros(heads, dim)
+    for h, below in enumerate((127, 130, 140, 149)):
+        weights[h, parts - 1] = torch.tensor([-float(below), 2.0**20])
+        weights[h, 1 : parts - 1, 0] = -float("inf")
+        sums[h, parts - 1] = 2.0**100
+        want[h] = 2.0 ** (100 - below)
+    w = torch.ones(n, heads * dim)
+    w[:, 1::2] = -0.5
+    got = ops.linear(WaitingHeads(sums.to(DEV), weights.to(DEV)), w.bfloat16().to(DEV)).double().sum(0)[0].cpu()
+    assert torch.equal(got, w.double() @ want.double().view(-1))
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,page", [(14, 2, 128, 8), (7, 1, 128, 64), (4, 4, 64, 32), (20, 1, 80, 16), (6, 2, 256, 8), (2, 2, 32, 64)])
 @pytest.mark.parametrize("waves", [8, 4, 2])
 @pytest.mark.parametrize("splits,window", [(1, None), (3, None), (1, 300)])

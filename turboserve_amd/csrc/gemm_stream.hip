@@ -401,8 +401,9 @@ int launch_stream_normed(float* partial, void* out, const float* residual, const
 
 // The same for the one row that is a token's attention, whose workgroups have left their sums (attention_mfma.hip: partial_acc [heads, splits, d], partial_ml
 // [heads, splits] of reference and sum): every workgroup puts its range of K together, as decode_reduce_kernel does, while its first weights
-// travel (weights below 2^-126 count for nothing here).  That launch took 4.9 us of a layer; 3,584 elements of eight workgroups are 57 KB from L2 for
-// every workgroup of two ranges, and their exponentials and quotients 3: a token of the 7B shape 2,603 -> 2,574 us.
+// travel.  That launch took 4.9 us of a layer; 3,584 elements of eight workgroups are 57 KB from L2 for
+// every workgroup of two ranges, and their exponentials and quotients 3: a token of the 7B shape 2,603 -> 2,579 us, 5 of which
+// weights below 2^-126 take (exp2f; the hardware's 2^x clears them, and a branch around it for those without was no sooner).
 template <int NT, int ITEMS, int PARTS>
 __global__ void __launch_bounds__(64 * STREAM_WAVES)
 gemm_stream_heads_kernel(const float* __restrict__ partial_acc, const float* __restrict__ partial_ml, const uint16_t* __restrict__ w, int splits_in,
@@ -444,7 +445,7 @@ gemm_stream_heads_kernel(const float* __restrict__ partial_acc, const float* __r
 #pragma unroll
       for (int s = 0; s < PARTS; ++s) most = fmaxf(most, m[it][s]);  // (a share past the last is the last one again)
 #pragma unroll
-      for (int s = 0; s < PARTS; ++s) weight[s] = s >= splits_in || m[it][s] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[it][s] - most);  // no keys
+      for (int s = 0; s < PARTS; ++s) weight[s] = s >= splits_in || m[it][s] == -INFINITY ? 0.f : exp2f(m[it][s] - most);  // no keys
       float sum[PARTS];
 #pragma unroll
       for (int s = 0; s < PARTS; ++s) sum[s] = l[it][s] * weight[s];
