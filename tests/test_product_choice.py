@@ -145,6 +145,30 @@ def test_a_norm_waits_for_a_product_that_makes_it(monkeypatch):
     assert ops.waiting_norm(torch.empty(1, 3584, device="meta"), parts, gain, 1e-6, matrix, gated=False) is None
 
 
+@pytest.mark.parametrize("gated", [False, True])
+def test_what_waits_is_for_the_matrix_it_was_made_for(monkeypatch, gated):
+    """A norm or heads that wait are not multiplied by a matrix that the launch would read past its end or by the wrong type; a step without rows has a
+    norm of its own."""
+    from turboserve_amd.kernels.ops import KernelError, WaitingHeads
+
+    monkeypatch.setattr("turboserve_amd.kernels.ops._gpu", lambda *tensors: None)
+    ops, k = Planner(), 2048
+    gain, residual, pending = torch.ones(k, dtype=torch.bfloat16), torch.zeros(1, k), torch.zeros(2, 1, k)
+    norm = ops.waiting_norm(residual, pending, gain, 1e-6, torch.zeros(256, k, dtype=torch.bfloat16), gated=gated)
+    heads = WaitingHeads(torch.zeros(16, 4, 128), torch.zeros(16, 4, 2))
+    refused = [torch.zeros(256, k - 64, dtype=torch.bfloat16), torch.zeros(256, k), torch.zeros(k, 256, dtype=torch.bfloat16).t(),
+               torch.zeros(256 * k + 4, dtype=torch.bfloat16)[4:].view(256, k), torch.zeros(256 * k, dtype=torch.bfloat16)]
+    assert refused[3].data_ptr() % 16
+    for matrix in refused:
+        with pytest.raises(KernelError):
+            (ops.linear_swiglu if gated else ops.linear)(norm, matrix)
+        with pytest.raises(KernelError):
+            ops.linear(heads, matrix)
+    with pytest.raises(KernelError):  # no workgroup for the last elements of the sum
+        (ops.linear_swiglu if gated else ops.linear)(norm, torch.zeros(32, k, dtype=torch.bfloat16))
+    assert ops.waiting_norm(residual[:0], pending[:, :0], gain, 1e-6, torch.zeros(256, k, dtype=torch.bfloat16), gated=gated) is None
+
+
 def test_the_store_of_heads_adds_up_what_few_rows_leave():
     """A prompt's q|k|v as two to four 32-bit sums wherever those are the model's cheapest grid (up to ``wide_default_rows`` rows), one result elsewhere."""
     ops = Planner()

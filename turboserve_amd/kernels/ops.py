@@ -1949,8 +1949,9 @@ class Ops:
     def _heads_product(self, heads: WaitingHeads, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
         """:meth:`gemm_stream` of the row that ``heads`` stands for."""
         _gpu(heads.sums, heads.weights, weight, bias)
-        (count, parts, dim), (n, k) = heads.sums.shape, weight.shape
-        _need(count * dim == k, "heads of another width than the matrix")
+        count, parts, dim = heads.sums.shape
+        _need(weight.dim() == 2 and self._heads_wait(parts, count * dim, weight), "waiting heads are for the matrix that they were made for")
+        n, k = weight.shape
         if bias is not None:
             _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous(), "bias must be bfloat16 [N]")
         per_wave, splits, _ = self._stream_plan(n, k, None)
@@ -2778,19 +2779,12 @@ class Ops:
         four 32-bit partial sums are to be added to.  The launch of the norm falls away.  ``residual`` keeps its
         values; ``after`` of the result is the sum once that product has run."""
         rows, hidden = residual.shape
-        if (rows > self.normed_max_rows or pending is None or pending.dim() != 3 or pending.shape[0] > 4 or rows * hidden > 6144 or hidden % 64
-                or gain.dtype is not torch.bfloat16 or matrix.dtype is not torch.bfloat16 or matrix.shape[1] != hidden
-                or not pending.is_contiguous() or not residual.is_contiguous() or not gain.is_contiguous() or not matrix.is_contiguous()
-                or (residual.data_ptr() | pending.data_ptr() | gain.data_ptr() | matrix.data_ptr()) % 16):
-            return None
-        n = matrix.shape[0]
-        if n <= 32 * (-(-hidden // 1024) - 1) or (gated and n % 2):
-            return None
-        plan = self._stream_plan(n, hidden, 1 if gated else None)
-        if plan is None:
+        if (pending is None or pending.dim() != 3 or not 1 <= pending.shape[0] <= 4 or gain.dtype is not torch.bfloat16
+                or not pending.is_contiguous() or not residual.is_contiguous() or not gain.is_contiguous()
+                or (residual.data_ptr() | pending.data_ptr() | gain.data_ptr()) % 16 or self._normed_plan(rows, hidden, matrix, gated) is None):
             return None
         if gated:
-            shared = self._stream_plan(n, hidden, None)
+            n, shared = matrix.shape[0], self._stream_plan(matrix.shape[0], hidden, None)
             if shared is not None and self._stream_cost(n, hidden, 1) > self._stream_cost(n, hidden, shared[1]) + 2.6:
                 return None  # linear_swiglu takes several ranges and the unit's own launch
         _gpu(residual, pending, gain, matrix)
@@ -2798,13 +2792,26 @@ class Ops:
         _need(residual.dtype == torch.float32 and gain.shape == (hidden,), "residual must be float32 [T, H], the gain [H]")
         return WaitingNorm(residual, pending, gain, float(eps), float(gain_offset), bool(one_rounding), torch.empty_like(residual))
 
+    def _normed_plan(self, rows: int, k: int, matrix: torch.Tensor, gated: bool) -> tuple[int, int, int] | None:
+        """The streaming product's grid for ``rows`` rows of ``k`` elements that it normalises itself, or None where it does not take them or
+        ``matrix``."""
+        n = matrix.shape[0]
+        if (not 1 <= rows <= self.normed_max_rows or rows * k > 6144 or k % 64 or matrix.dim() != 2 or matrix.shape[1] != k
+                or matrix.dtype is not torch.bfloat16 or not matrix.is_contiguous() or matrix.data_ptr() % 16
+                or n <= 32 * (-(-k // 1024) - 1) or (gated and n % 2)):
+            return None
+        return self._stream_plan(n, k, 1 if gated else None)
+
     def _normed_product(self, norm: WaitingNorm, weight: torch.Tensor, bias: torch.Tensor | None, *, gated: bool,
                         rule: tuple[float, ...] = (1.0, 0.0, 0.0)) -> torch.Tensor:
         """:meth:`gemm_stream` of the rows that ``norm`` stands for, which the same launch makes."""
+        _gpu(weight, bias)
         (m, k), n = norm.residual.shape, weight.shape[0]
+        plan = self._normed_plan(m, k, weight, gated)
+        _need(plan is not None, "a waiting norm is for the matrix that it was made for")
         if bias is not None:
             _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous(), "bias must be bfloat16 [N]")
-        per_wave, splits, _ = self._stream_plan(n, k, 1 if gated else None)
+        per_wave, splits, _ = plan
         partial = out = None
         if gated:
             out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=weight.device)
