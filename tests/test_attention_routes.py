@@ -10,7 +10,10 @@ import torch
 
 from turboserve_amd.kernels.ops import Ops
 from turboserve_amd.parts.attention import GroupedQueryAttention
-from turboserve_amd.parts.base import PartSpec, Runtime
+from turboserve_amd.parts.base import PartSpec, ResidualStream, Runtime
+from turboserve_amd.parts.block import PreNormBlock
+from turboserve_amd.parts.mlp import ActivatedMLP, SwiGLU
+from turboserve_amd.parts.norm import RMSNorm
 from turboserve_amd.parts.registry import POSITION_ENCODINGS, register_position_encoding
 from turboserve_amd.parts.rope import RotaryEncoding
 
@@ -106,6 +109,107 @@ def test_a_decode_step_attends_by_the_layers_rule(encodings, kind, encoding, lau
     ctx.num_prefill_seqs, ctx.num_decode_seqs = 1, 2  # a step with a prompt never goes to the launch that stores
     assert layer._attend_projected(torch.zeros(3, 3, 256), ctx, cache) is None
     assert layer._plain_store == plain_store(32) and len(asked) <= (2 if launches == ["all in one"] else 1)  # worked out once
+
+
+class Steps:
+    """What a block of a step of one token asks for, and what its products get."""
+
+    normed_max_rows = Ops.normed_max_rows
+
+    def __init__(self):
+        self.names = []
+
+    def waiting_norm(self, residual, *more, **rest):
+        self.names.append("waits")
+        return SimpleNamespace(after=residual, dtype=torch.bfloat16, device=residual.device)
+
+    def add_rmsnorm(self, residual, *more, **rest):
+        self.names.append("norm")
+        return residual.bfloat16()
+
+    def linear(self, x, weight, bias=None, **more):
+        return torch.zeros(1, 1, weight.shape[0])
+
+    def linear_swiglu(self, x, weight, rule, bias):
+        return torch.zeros(1, weight.shape[0] // 2)
+
+    def activate(self, x, *more):
+        return x[0]
+
+
+class ReadingAttention(GroupedQueryAttention):
+    """An adapter's way: looks at its rows, then runs the layer."""
+
+    def forward(self, x, ctx, cache):
+        assert x.shape == (1, 64)
+        return super().forward(x, ctx, cache)
+
+    def _attend_projected(self, *more):
+        return torch.zeros(1, 128)
+
+
+class ReadingHeads(GroupedQueryAttention):
+    def heads_out(self, x, ctx, cache, *, scale=1.0, out=None):
+        assert x.shape == (1, 64)
+        return torch.zeros(1, 128)
+
+
+class PlainAttention(GroupedQueryAttention):
+    def _attend_projected(self, qkv, ctx, cache, waits_for=None):
+        assert waits_for is self.o_weight
+        return torch.zeros(1, 128)
+
+
+class ReadingSwiGLU(SwiGLU):
+    def forward(self, x, ctx):
+        assert x.shape == (1, 64)
+        return super().forward(x, ctx)
+
+
+class ReadingMLP(ActivatedMLP):
+    def forward(self, x, ctx):
+        assert x.shape == (1, 64)
+        return super().forward(x, ctx)
+
+
+class OwnNorm(RMSNorm):
+    def forward_residual(self, stream, rows=None):
+        self.runtime.ops.names.append("own")
+        return stream.residual.bfloat16()
+
+
+@pytest.mark.parametrize("mixer,feed_forward,norm,asked", [
+    (PlainAttention, SwiGLU, RMSNorm, ["waits", "waits"]),
+    (PlainAttention, ActivatedMLP, RMSNorm, ["waits", "waits"]),
+    (ReadingAttention, ReadingSwiGLU, RMSNorm, ["norm", "norm"]),
+    (ReadingHeads, ReadingMLP, RMSNorm, ["norm", "norm"]),
+    (PlainAttention, SwiGLU, OwnNorm, ["own", "own"]),
+])
+@pytest.mark.parametrize("on_the_instance", [False, True])
+def test_a_part_of_its_own_ways_gets_rows(mixer, feed_forward, norm, asked, on_the_instance):
+    """A norm waits for its product only where the part that reads it is known to read nothing but the product, and the norm is the plain one: a
+    subclass's ways, or those set on an instance, get the rows in a step of one token, too."""
+    runtime = Runtime(device=torch.device("cpu"), dtype=torch.bfloat16, ops=Steps())
+    block = PreNormBlock.__new__(PreNormBlock)
+    block.runtime = runtime
+    block.mixer = mixer("mixer", runtime, hidden_size=64, num_heads=4, num_kv_heads=2, head_dim=32, scale=32 ** -0.5, qkv_bias=False, out_bias=False,
+                        window=None, position=PartSpec("rope", {"head_dim": 32, "theta": 1e4, "max_positions": 64}))
+    block.mixer.qkv_weight, block.mixer.o_weight = torch.zeros(8 * 32, 64), torch.zeros(64, 4 * 32)
+    more = {"activation": "relu"} if issubclass(feed_forward, ActivatedMLP) else {}
+    block.feed_forward = feed_forward("mlp", runtime, hidden_size=64, intermediate_size=32, **more)
+    block.feed_forward.gate_up_weight = block.feed_forward.up_weight = torch.zeros(64, 64)
+    block.feed_forward.down_weight = torch.zeros(64, 32)
+    block.mixer_norm, block.ff_norm = (norm(name, runtime, size=64, eps=1e-6) for name in ("a", "b"))
+    if on_the_instance:
+        for part in (block.mixer, block.feed_forward):
+            def looks(x, *rest, forward=part.forward):
+                assert x.shape == (1, 64)
+                return forward(x, *rest)
+            part.forward = looks
+        asked = [name.replace("waits", "norm") for name in asked]
+    ctx = SimpleNamespace(num_prefill_seqs=0, num_tokens=1)
+    block.forward(ResidualStream(torch.zeros(1, 64), torch.zeros(2, 1, 64)), ctx, None)
+    assert runtime.ops.names == asked
 
 
 @pytest.mark.parametrize("workgroups,span,head_dim,waves", [

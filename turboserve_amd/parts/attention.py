@@ -276,11 +276,12 @@ class GroupedQueryAttention(Mixer):
             self.mix_weight = float(tensors[self.name(self.value_mix["name"])].float().item())
         self.position.load(tensors)
 
-    def first_matrix(self) -> tuple[torch.Tensor, bool]:
-        return self.qkv_weight, False
+    def first_matrix(self) -> tuple[torch.Tensor, bool] | None:
+        return (self.qkv_weight, False) if self.runs(GroupedQueryAttention, "forward", "heads_out") else None
 
     def forward(self, x: torch.Tensor, ctx, cache) -> torch.Tensor:
-        return self.runtime.ops.linear(self.heads_out(x, ctx, cache, waits_for=self.o_weight), self.o_weight, self.o_bias_tensor, for_residual=True)
+        more = {"waits_for": self.o_weight} if self.runs(GroupedQueryAttention, "heads_out") else {}
+        return self.runtime.ops.linear(self.heads_out(x, ctx, cache, **more), self.o_weight, self.o_bias_tensor, for_residual=True)
 
     @property
     def out_features(self) -> int:

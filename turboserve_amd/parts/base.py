@@ -230,8 +230,13 @@ class Part:
 
     def first_matrix(self) -> "tuple[torch.Tensor, bool] | None":
         """The matrix (and whether :meth:`Ops.linear_swiglu` multiplies it) whose product is all that this part reads of its input in the
-        run's own kernels: its input may then be a ``WaitingNorm``.  None: it reads the rows."""
+        run's own kernels: its input may then be a ``WaitingNorm``.  None: it reads the rows, as does a part whose class says otherwise but that
+        runs other methods than that class's (:meth:`runs`)."""
         return None
+
+    def runs(self, cls: type, *methods: str) -> bool:
+        """Whether these methods are ``cls``'s own, not a subclass's and not set on the instance."""
+        return all(getattr(getattr(self, name), "__func__", None) is getattr(cls, name) for name in methods)
 
     def activation_bytes(self, tokens: int, itemsize: int) -> int:
         """Bytes of the transient tensors this part holds at once in a step of ``tokens`` rows

@@ -62,8 +62,8 @@ class SwiGLU(FeedForward):
             gate, up, self.down_bias = (tensors[self.name(f"{n}.b")].contiguous() for n in (self.gate_name, self.up_name, self.down_name))
             self.gate_up_bias = torch.stack([gate, up], dim=1).reshape(-1).contiguous()
 
-    def first_matrix(self) -> tuple[torch.Tensor, bool]:
-        return self.gate_up_weight, True
+    def first_matrix(self) -> tuple[torch.Tensor, bool] | None:
+        return (self.gate_up_weight, True) if self.runs(SwiGLU, "forward") else None
 
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         ops = self.runtime.ops
@@ -103,8 +103,8 @@ class ActivatedMLP(FeedForward):
         self.up_weight = tensors[self.name(self.up_name)].contiguous()
         self.down_weight = tensors[self.name(self.down_name)].contiguous()
 
-    def first_matrix(self) -> tuple[torch.Tensor, bool]:
-        return self.up_weight, False
+    def first_matrix(self) -> tuple[torch.Tensor, bool] | None:
+        return (self.up_weight, False) if self.runs(ActivatedMLP, "forward") else None
 
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         ops = self.runtime.ops

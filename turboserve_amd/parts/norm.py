@@ -56,7 +56,7 @@ class RMSNorm(Norm):
         return y
 
     def waiting(self, stream: ResidualStream, matrix: torch.Tensor, gated: bool):
-        if stream.also is not None or stream.pending_norm is not None:
+        if stream.also is not None or stream.pending_norm is not None or not self.runs(RMSNorm, "forward_residual"):
             return None
         norm = self.runtime.ops.waiting_norm(stream.residual, stream.pending, self.weight, self.eps, matrix, gated=gated,
                                              gain_offset=self.gain_offset, one_rounding=self.one_rounding)
