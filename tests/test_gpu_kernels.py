@@ -1454,6 +1454,8 @@ def test_a_product_that_puts_a_tokens_attention_together(ops, monkeypatch, heads
                     assert torch.equal(got, want)
                 room = 2.0**-8 * (whole.double().abs() @ w.double().abs().T)
                 assert bool(((got.double() - want.double()).sum(0).abs() <= room).all())
+            two = torch.full((2, heads * dim), float("nan"), dtype=torch.bfloat16, device=DEV)  # a step with other rows: all of them are the product's
+            assert ops.attention_decode(two, *common, waits_for=w) is None and torch.equal(two[:1], whole) and bool(two[1].isnan().all())
     for refused in (w[:, :-8], w.float()):  # another width, another type
         assert ops.attention_decode(whole, *common, waits_for=refused.contiguous()) is None
 

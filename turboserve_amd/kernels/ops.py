@@ -1886,7 +1886,7 @@ class Ops:
         ``slots`` and attends, in place of :meth:`rope_store` before it (the same bits in the pages).
 
         ``waits_for``: the matrix ``[N, heads * D]`` whose product (:meth:`linear`) is all that reads ``out``: where that product puts one request's
-        workgroups together itself, ``out`` is left alone and what it takes instead is returned (else None).
+        workgroups together itself and ``out`` has no other rows, it is left alone and what it takes instead is returned (else None).
 
         ``shares`` (:meth:`decode_shares`): what the requests' own lengths, which ``max_context`` does not tell, make of a
         request's keys where requests and KV heads alone give every compute unit a workgroup."""
@@ -1927,7 +1927,7 @@ class Ops:
             partial_acc = torch.empty((requests * heads * splits, head_dim), dtype=torch.float32, device=out.device)
             partial_ml = torch.empty((requests * heads * splits, 2), dtype=torch.float32, device=out.device)
         waiting = None
-        if waits_for is not None and requests == 1 and self._heads_wait(splits, heads * head_dim, waits_for):
+        if waits_for is not None and requests == 1 and out.shape[0] == 1 and self._heads_wait(splits, heads * head_dim, waits_for):
             waiting = WaitingHeads(partial_acc.view(heads, splits, head_dim), partial_ml.view(heads, splits, 2))
         lib = load_module(build.attention_module(head_dim))
         fn = getattr(lib, f"ts_attention_decode_d{head_dim}")
