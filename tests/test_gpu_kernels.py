@@ -307,6 +307,39 @@ def test_gemm_plain_is_chains_of_fused_multiply_adds(ops, dtype, k, values):
                     assert got[i, j].item() == float(value), (rows, cols, i, j)
 
 
+@pytest.mark.parametrize("rule,inner_roundings", [((1.0, 0.0, 0.0), 0), ((1.702, 7.0, 1.0), 1), ("gelu_tanh", 4)])
+def test_the_gated_unit_against_64_bits(ops, rule, inner_roundings):
+    """Gates of every size, on both sides of the 80 up to which the sigmoid's short form goes and of the 88.7 beyond which e^x is no normal number,
+    tiny, denormal and no finite ones.  Relative to 64 bits: two units of 2^-24 for 2^x of the hardware, one each for the rounding of the quotient,
+    of up + shift and of their product, one for what is of second order; and a rounding of the sigmoid's argument for each operation that
+    makes it, which counts for |x| times as much; one unit of the denormal numbers for each of the results that may be one."""
+    from turboserve_amd.kernels.ops import GELU_TANH_RULE
+
+    rule = GELU_TANH_RULE if rule == "gelu_tanh" else rule
+    steepness, limit, shift, cubic = (torch.tensor(v).double().item() for v in (*map(float, rule), 0.0)[:4])
+    g = torch.Generator().manual_seed(7)
+    edges = torch.tensor([0.0, 80.0, 80.00001, 79.99999, 88.7, 88.8, 87.3, 103.9, 104.0, 1e-45, 1e-40, 1.2e-38, 1e-30, 7.0, 6.9999995, 3e4, 1e30])
+    gates = torch.cat([edges, -edges, torch.rand(1 << 18, generator=g) * 208 - 104, torch.randn(1 << 18, generator=g),
+                       torch.exp(torch.rand(1 << 16, generator=g) * 90 - 90) * torch.randn(1 << 16, generator=g).sign()])
+    gates = torch.cat([gates, torch.zeros(-len(gates) % 8)])
+    ups = torch.randn(len(gates), generator=g) * 3
+    rows = torch.stack([gates, ups], -1).view(1, -1).to(DEV)
+    got = ops.swiglu(rows, torch.float32, paired=True, rule=rule)[0].double().cpu()
+    gate, up = gates.double(), ups.double()
+    if limit > 0:
+        gate, up = gate.clamp(max=limit), up.clamp(-limit, limit)
+    x = steepness * (gate + cubic * gate**3)
+    small = torch.exp(-x.abs())
+    sigmoid = torch.where(x >= 0, 1 / (1 + small), small / (1 + small))
+    want = gate * sigmoid * (up + shift)
+    relative = 6 + inner_roundings * x.abs() * torch.where(x >= 0, small / (1 + small), 1 / (1 + small))
+    within = (got - want).abs() <= 2.0**-24 * relative * want.abs() + 2.0**-149 * (2 + (up + shift).abs())
+    assert bool(within.all()), (gates[~within][:8], got[~within][:8], want[~within][:8])
+    odd = torch.tensor([[float("inf"), 2.0, float("inf"), -2.0, -float("inf"), 2.0, float("nan"), 2.0]], device=DEV)
+    got = ops.swiglu(odd, torch.float32, paired=True, rule=rule)[0].tolist()
+    assert got[2] != got[2] and (limit > 0 or (got[0] == float("inf") and got[1] == -float("inf") and got[3] != got[3]))
+
+
 @pytest.mark.parametrize("rows,k,sums", [(1, 64, 1), (1, 1024, 4), (1, 1088, 2), (2, 64, 3), (2, 576, 1), (2, 1024, 2), (2, 1088, 4), (2, 2048, 3), (2, 2624, 1),
                                          (2, 3072, 2), (1, 2624, 4), (1, 3584, 2), (1, 4096, 1), (1, 4160, 3), (1, 5120, 4), (1, 6144, 3)])
 @pytest.mark.parametrize("one_rounding", [False, True])
@@ -1428,13 +1461,15 @@ def test_attention_decode_from_projected_sums(ops, monkeypatch, heads, kv_heads,
     torch.testing.assert_close(got[stored].float(), want[stored].float(), rtol=2.0**-7, atol=1e-6)
 
 
-@pytest.mark.parametrize("heads,kv_heads,dim", [(14, 2, 128), (28, 4, 128), (4, 4, 64), (2, 2, 32), (16, 4, 80), (6, 2, 256)])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(14, 2, 128), (28, 4, 128), (4, 4, 64), (2, 2, 32), (16, 4, 80), (6, 2, 256),
+                                                (20, 4, 128), (32, 8, 128)])
 @pytest.mark.parametrize("parts", [2, 3, 5, 8])
 @pytest.mark.parametrize("window", [None, 300])
 def test_a_product_that_puts_a_tokens_attention_together(ops, monkeypatch, heads, kv_heads, dim, parts, window):
     """One request's keys divided over two to eight workgroups, put together by the product that reads the row: the bits of the combining launch and the
     streaming product of its row where that launch adds up a workgroup's sums one by one (a thread for every workgroup: 1,024 / D of them), else
-    within one bfloat16 unit of every element (2^-8 of its size); workgroups without keys count for nothing, `out` stays as it was."""
+    within one bfloat16 unit of every element (2^-8 of its size); workgroups without keys count for nothing, `out` stays as it was.  Matrices whose grid gives a
+    wavefront one to sixteen slices of 64 (8,192 x 2,560 ten, 8,192 x 4,096 sixteen)."""
     monkeypatch.setattr(type(ops), "_decode_parts", lambda self, pairs, span, head_dim, shares: parts)
     for context in (1000, 40):
         case = PagedCase(torch.bfloat16, heads, kv_heads, dim, 16, [(context, 1)], window, seed=dim + parts)
@@ -1442,7 +1477,7 @@ def test_a_product_that_puts_a_tokens_attention_together(ops, monkeypatch, heads
                   heads, dim ** -0.5, window, context)
         g = torch.Generator().manual_seed(dim)
         row = torch.full((1, heads * dim), float("nan"), dtype=torch.bfloat16, device=DEV)
-        for n in (336, 2060):
+        for n in (8192,) if heads in (20, 32) else (336, 2060):
             w, b = (torch.randn(n, heads * dim, generator=g) / 8).bfloat16().to(DEV), torch.randn(n, generator=g).bfloat16().to(DEV)
             waiting = ops.attention_decode(row, *common, waits_for=w)
             assert waiting is not None and bool(row.isnan().all())
