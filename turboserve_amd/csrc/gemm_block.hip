@@ -232,7 +232,7 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   // No load is issued past the end: one that brings nothing still takes its turn in the unit's memory path.  But a loop of their own
   // for the last iterations costs the compiler its registers where the sums take more than 160: it moved them about in the main
   // loop as well (2,048 rows, 7,168 x 5,120 with 256 x 256 115 -> 129 us, 27,648 x 5,120 gated with 256 x 192 467 -> 474).  There the
-  // loads go out in every iteration, those past the end past the buffers' ends too.
+  // loads go out in every iteration, those past the end to an empty buffer.
   constexpr bool PEELED = TN * TM <= 40;
   const int count = last - first;
   // The buffers and the place in them that iteration i reads from: an empty buffer past the end.

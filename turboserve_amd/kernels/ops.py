@@ -1939,7 +1939,9 @@ class Ops:
 
     def _heads_wait(self, parts: int, k: int, matrix: torch.Tensor) -> bool:
         """Whether the product by ``matrix [N, K]`` puts together what ``parts`` workgroups left of one request's keys: up to eight (a
-        range of K reads them all, once for every 32 weight rows), of up to 6,144 elements, where the streaming product runs."""
+        range of K reads them all, once for every 32 weight rows), of up to 6,144 elements, where the streaming product runs.  A part is at
+        least 128 keys of a bound that is a power of two in a recorded step, so with fewer than 32 KV heads these are bounds of 1,024 keys (513 to 1,024 of the
+        request's); from 1,025 on there are sixteen parts and more, and the launch that combines them."""
         if not (2 <= parts <= 8 and k % 64 == 0 and k <= 6144 and matrix.dtype is torch.bfloat16 and matrix.shape[1] == k
                 and matrix.is_contiguous() and matrix.data_ptr() % 16 == 0):
             return False
@@ -1976,8 +1978,9 @@ class Ops:
 
         As many as give every compute unit one workgroup (a second one on a unit waits for the first: its wavefronts
         hold all registers), at most one for every ``decode_min_keys`` keys of the span (a recorded step's is its shape's bound, of which a request may
-        have less); spans of up to 512 keys stay whole, which saves the
-        launch that combines.  Microseconds a layer with the rotation and the store, heads of 128, 7 to a KV head, by number of
+        have less); spans of up to 512 keys stay whole, which saved the
+        launch that combines (it is in the figures; one request's up to eight parts are since joined by the output product, ``_heads_wait``, for which the line
+        was not drawn anew).  Microseconds a layer with the rotation and the store, heads of 128, 7 to a KV head, by number of
         workgroups: one request of 300 keys 8.5 (1) 8.9 (3), of 640 10.6 (1) 8.9 (6), of 8,192 17.7 (8) 11.2 (32) 11.3 (64); 8
         requests of 640 10.2 (4) 11.4 (2), of 8,192 26.6 (8) 29.8 (16); 32 of 2,048 28.6 (2) 30.7 (1) 31.7 (4); 64 of 129 to
         1,525 26.2 (1) 32.0 (2)."""
@@ -2315,8 +2318,10 @@ class Ops:
     wide_default_rows = 640
 
     #: The block product's tiles (in 32 weight rows, 32 activation rows) and what an iteration of
-    #: 64 of K takes a compute unit with each, in microseconds: the slope over K of products at 144
-    #: to 2,048 rows that give every compute unit a workgroup.
+    #: 64 of K counts for with each when grids are compared, in microseconds.  The slope over K of products that give every
+    #: compute unit a workgroup, those of 256, 160 and 128 weight rows with a loop whose accesses went out in groups, those of 224 and 192 with the
+    #: present one; with it all are, in this order, 1.37, 1.25, 1.10, 1.10, 0.94, 1.15, 0.92, 0.80, 0.68, 0.56 and 0.45 on a card whose clock
+    #: falls when all units are at work, and a workgroup's first loads and stores five to twelve iterations, gated or not.
     _BLOCK_TILES = {(8, 8): 1.24, (7, 8): 1.14, (8, 6): 0.99, (6, 8): 1.01, (8, 5): 0.86, (5, 10): 1.07, (5, 8): 0.88, (4, 8): 0.76, (7, 4): 0.745, (4, 5): 0.54,
                     (4, 4): 0.50}
 
@@ -2337,8 +2342,9 @@ class Ops:
         block product: the cheapest grid, where a round of workgroups (one per compute unit) takes
         its iterations and six more (first loads, stores) at the tile's pace, a gated
         result the unit's time, and partial sums of several ranges their way to the norm, 3.6
-        bytes per nanosecond.  Against every tile with 1 to 16 ranges, timed for the matrices of six shapes (K 2,048 to 18,944) at 144 to
-        2,048 rows, the plan's grid takes 1% more than the fastest on average.  The tiles of 192 and 224 weight rows fill rounds that the others
+        bytes per nanosecond.  Against every tile with 1 to 16 ranges, timed with the kernel that reads the result and weights that no cache holds, for
+        eight matrices (K 2,048 to 18,944) at ten row counts from 144 to 2,048, the plan's grid takes 1.6% more than the fastest on average, up to
+        7% at one, and 10 to 22% for 2,048 x 8,192 at 144 to 299 rows (sixteen and eight ranges against six and four).  The tiles of 192 and 224 weight rows fill rounds that the others
         leave in part empty (us: 3,584 x 18,944 at 2,048 rows, two ranges, 256 workgroups of 224 x 256 195 against 224 of 256 x 256 210, 3,584 x
         3,584 of 224 x 128 45 against 224 of 128 x 256 47, 7,168 x 5,120 107 against 113; some 60 of 14 matrices' grids at 129 to 2,048 rows changed with
         them, 5% sooner on average; 3,584 x 18,944 at 1,729 to 1,792 rows as two ranges of 224 x 256, 224 workgroups, 200 to 205 us with the norm
@@ -2404,7 +2410,8 @@ class Ops:
         return best[1]
 
     def _block_cost(self, m: int, n: int, k: int, plan: tuple[int, int, int, int], gated: bool = False) -> float:
-        """What :meth:`_block_plan` compares, in microseconds."""
+        """What :meth:`_block_plan` compares, in microseconds.  (The gated unit's 0.18 us a tile of 32 x 32 is what it took as ``expf`` and a
+        division; now a gated result's stores and unit take about as long as one result's stores.)"""
         per_split, splits, tn, tm = plan
         workgroups = -(-n // (32 * tn)) * -(-m // (32 * tm)) * splits
         cost = -(-workgroups // self.compute_units) * ((per_split + 6) * self._BLOCK_TILES[tn, tm] + (0.18 * tn * tm if gated else 0.0))
