@@ -165,6 +165,15 @@ def test_what_waits_is_for_the_matrix_it_was_made_for(monkeypatch, gated):
     assert ops.waiting_norm(residual[:0], pending[:, :0], gain, 1e-6, torch.zeros(256, k, dtype=torch.bfloat16), gated=gated) is None
 
 
+def test_a_gated_product_of_other_than_rows_is_refused_as_any_product(monkeypatch):
+    from turboserve_amd.kernels.ops import KernelError
+
+    monkeypatch.setattr("turboserve_amd.kernels.ops._gpu", lambda *tensors: None)
+    for x, w in ((torch.zeros(2, 3, 32), torch.zeros(64, 32)), (torch.zeros(32), torch.zeros(64, 32)), (torch.zeros(3, 32), torch.zeros(2, 64, 32))):
+        with pytest.raises(KernelError):
+            Planner().linear_swiglu(x, w)
+
+
 def test_the_store_of_heads_adds_up_what_few_rows_leave():
     """A prompt's q|k|v as two to four 32-bit sums wherever those are the model's cheapest grid (up to ``wide_default_rows`` rows), one result elsewhere."""
     ops = Planner()

@@ -3097,8 +3097,10 @@ class Ops:
     @staticmethod
     def _plain_gates(x: torch.Tensor, weight: torch.Tensor) -> bool:
         """Whether the 32-bit product applies the gated unit itself (``csrc/gemm_plain.hip``: the layouts that stage whole slices through LDS)."""
+        if x.dtype is not torch.float32 or x.dim() != 2 or weight.dim() != 2:
+            return False
         (n, k), (row, one) = weight.shape, x.stride()
-        return (x.dtype is torch.float32 and one == 1 and weight.is_contiguous() and k % 32 == 0 and n % 4 == 0 and row % 4 == 0
+        return (one == 1 and weight.is_contiguous() and k % 32 == 0 and n % 4 == 0 and row % 4 == 0
                 and k < 1 << 21 and row < 1 << 21 and (x.data_ptr() | weight.data_ptr()) % 16 == 0)
 
     def _sums_plan(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> tuple[int, int, int, int] | None:
