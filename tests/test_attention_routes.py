@@ -270,3 +270,12 @@ def test_spans_that_are_divided(pairs, span, head_dim, shares, parts):
     ops = object.__new__(Ops)
     ops.compute_units = 256
     assert ops._decode_parts(pairs, span, head_dim, shares) == parts
+
+
+@pytest.mark.parametrize("pairs,span,parts", [(4, 64, 1), (4, 65, 2), (4, 128, 2), (4, 256, 4), (4, 300, 4), (4, 512, 4), (4, 513, 5), (4, 1024, 8), (32, 512, 4),
+                                              (100, 512, 2), (129, 512, 1)])
+def test_spans_whose_parts_the_output_product_joins(pairs, span, parts):
+    """No more parts than that product takes, and none without a unit of its own."""
+    ops = object.__new__(Ops)
+    ops.compute_units = 256
+    assert ops._joined_parts(pairs, span) == parts

@@ -1921,13 +1921,16 @@ class Ops:
             new = (_ptr(q), stride, sum_splits, _ptr(cos), _ptr(sin), _ptr(slots))
         span = max_context if not window else min(max_context, window + 31)
         pairs = requests * kv_heads * -(-(heads // kv_heads) // 16)
+        joined = waits_for is not None and requests == 1 and out.shape[0] == 1 and self._heads_wait(2, heads * head_dim, waits_for)
         splits = self._decode_parts(pairs, span, head_dim, shares)
+        if joined and splits == 1:
+            splits = self._joined_parts(pairs, span)
         partial_acc = partial_ml = None
         if splits > 1:
             partial_acc = torch.empty((requests * heads * splits, head_dim), dtype=torch.float32, device=out.device)
             partial_ml = torch.empty((requests * heads * splits, 2), dtype=torch.float32, device=out.device)
         waiting = None
-        if waits_for is not None and requests == 1 and out.shape[0] == 1 and self._heads_wait(splits, heads * head_dim, waits_for):
+        if joined and self._heads_wait(splits, heads * head_dim, waits_for):
             waiting = WaitingHeads(partial_acc.view(heads, splits, head_dim), partial_ml.view(heads, splits, 2))
         lib = load_module(build.attention_module(head_dim))
         fn = getattr(lib, f"ts_attention_decode_d{head_dim}")
@@ -1940,8 +1943,8 @@ class Ops:
     def _heads_wait(self, parts: int, k: int, matrix: torch.Tensor) -> bool:
         """Whether the product by ``matrix [N, K]`` puts together what ``parts`` workgroups left of one request's keys: up to eight (a
         range of K reads them all, once for every 32 weight rows), of up to 6,144 elements, where the streaming product runs.  A part is at
-        least 128 keys of a bound that is a power of two in a recorded step, so with fewer than 32 KV heads these are bounds of 1,024 keys (513 to 1,024 of the
-        request's); from 1,025 on there are sixteen parts and more, and the launch that combines them."""
+        least 64 keys of a bound that is a power of two in a recorded step, so with fewer than 32 KV heads these are bounds of 128 to 1,024 keys (65 to 1,024 of
+        the request's); from 1,025 on there are sixteen parts and more, and the launch that combines them."""
         if not (2 <= parts <= 8 and k % 64 == 0 and k <= 6144 and matrix.dtype is torch.bfloat16 and matrix.shape[1] == k
                 and matrix.is_contiguous() and matrix.data_ptr() % 16 == 0):
             return False
@@ -1962,6 +1965,15 @@ class Ops:
                                               per_wave, splits, self.stream()), "ts_gemm_stream_heads")
         return partial
 
+    def _joined_parts(self, pairs: int, span: int) -> int:
+        """How many workgroups share one request's whole span where the product by the output matrix puts their parts together (:meth:`_heads_wait`),
+        so that dividing costs no launch: one for every 64 keys, up to four; from 512 keys on one for every 128.  A step's
+        microseconds, whole / a part for every 128 keys / for every 64 (bounds are powers of two in a recorded step): 16 heads of 128 on 4 KV
+        heads, 8 layers, 120 keys 319.0 / 319.0 / 317.2, 250 330.8 / 323.1 / 318.0, 300 337.9 / 320.9 / 321.9, 500 348.1 / 322.7 / 321.8,
+        640 - / 324.4 / 333.0 (sixteen parts, and the launch that combines); 28 heads, 28 layers, 250 keys 2,588 / 2,568 / 2,546, 300 2,606 /
+        2,560 / 2,572, 500 2,644 / 2,575 / 2,569."""
+        return max(1, min(max(min(4, -(-span // 64)), -(-span // self.decode_min_keys)), self.compute_units // pairs, 8))
+
     def _decode_parts(self, pairs: int, span: int, head_dim: int, shares: int) -> int:
         """How many workgroups a request and KV head get: :meth:`_decode_splits`, or ``shares`` where that leaves long spans whole.  Heads of
         more than 128 are divided from 256 keys on, which their four wavefronts walk in two turns (us a layer, 256-wide heads, 300 / 500 keys
@@ -1978,9 +1990,8 @@ class Ops:
 
         As many as give every compute unit one workgroup (a second one on a unit waits for the first: its wavefronts
         hold all registers), at most one for every ``decode_min_keys`` keys of the span (a recorded step's is its shape's bound, of which a request may
-        have less); spans of up to 512 keys stay whole, which saved the
-        launch that combines (it is in the figures; one request's up to eight parts are since joined by the output product, ``_heads_wait``, for which the line
-        was not drawn anew).  Microseconds a layer with the rotation and the store, heads of 128, 7 to a KV head, by number of
+        have less); spans of up to 512 keys stay whole, which saves the
+        launch that combines (it is in the figures; where the output product joins the parts the line is another, :meth:`_joined_parts`).  Microseconds a layer with the rotation and the store, heads of 128, 7 to a KV head, by number of
         workgroups: one request of 300 keys 8.5 (1) 8.9 (3), of 640 10.6 (1) 8.9 (6), of 8,192 17.7 (8) 11.2 (32) 11.3 (64); 8
         requests of 640 10.2 (4) 11.4 (2), of 8,192 26.6 (8) 29.8 (16); 32 of 2,048 28.6 (2) 30.7 (1) 31.7 (4); 64 of 129 to
         1,525 26.2 (1) 32.0 (2)."""
