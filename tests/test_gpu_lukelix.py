@@ -197,6 +197,23 @@ def test_the_short_convolution_with_a_bias(ops, dtype, taps, channels, silu, bia
             done[i] += n
 
 
+@pytest.mark.parametrize("taps", [1, 2, 4, 8])
+@pytest.mark.parametrize("lead", [1, 2, 3, 5, 6, 7, 8, 9])
+def test_the_convolution_of_rows_moves_the_state_on(ops, taps, lead):
+    """Requests that begin at every place of a tile of eight rows, as long as the taps look back, shorter and longer: the bits of
+    the kernel that takes a row a workgroup (32-bit sums) with the state moved by a launch of its own, in the rows and in the slots."""
+    g = torch.Generator().manual_seed(10 * taps + lead)
+    lengths, channels, width, first = [lead, 1, taps, 9, max(1, taps - 2), 40], 36, 44, 4
+    slots, starts = ints([4, 0, 6, 2, 1, 5]), [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    seqs = ints([j for j, n in enumerate(lengths) for _ in range(n)])
+    proj = torch.randn(starts[-1], width, generator=g).bfloat16().to(DEV)
+    weight, bias = torch.randn(channels, taps, generator=g).bfloat16().to(DEV), torch.randn(channels, generator=g).bfloat16().to(DEV)
+    states = [torch.randn(8, max(taps - 1, 1), channels, generator=torch.Generator().manual_seed(lead)).to(DEV) for _ in range(2)]
+    outs = [ops.short_conv(given, first, weight, state, slots, seqs, ints(starts), tokens=starts[-1], num_seqs=len(lengths), dtype=torch.bfloat16, bias=bias)
+            for given, state in zip((proj, proj.float().unsqueeze(0)), states)]
+    assert torch.equal(*outs) and torch.equal(*states)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,turned,tokens", [(4, 2, 16, 24, 8, 40), (3, 3, 12, 12, 12, 5), (2, 1, 128, 128, 128, 70),
                                                                    (1, 1, 64, 32, 6, 33), (6, 0, 32, 32, 16, 90), (3, 0, 20, 20, 4, 2), (2, 2, 72, 40, 40, 37)])

@@ -8,11 +8,10 @@
 // holds (state [slots, K - 1, channels] 32-bit, oldest first; zero for a request that starts).  A `bias` [channels],
 // where given, is added; with `activation` 1 the result then goes through silu.  The result is [T, channels] of type T, or 32-bit.
 //
-// ts_short_conv computes every row of the step and leaves the state alone; ts_short_conv_carry, launched
-// behind it, moves each request's last K - 1 inputs into its slot.  In a step whose requests all bring one
-// token (`single`), the thread that computes a channel of a request also moves the channel's state on, and
-// nothing is launched behind it.  Prompt portions in bfloat16 take four channels by eight rows a thread
-// (short_conv_rows_kernel), the same arithmetic.
+// In a step whose requests all bring one token, the thread that computes a channel of a request also moves the channel's state on.  Prompt
+// portions in bfloat16 take four channels by eight rows a thread (short_conv_rows_kernel), the same arithmetic, and move the
+// state on in the same launch, too.  Behind the general kernel a second one (short_conv_carry_kernel) moves each request's last K - 1
+// inputs into its slot.
 #include "vec.hpp"
 
 template <typename P>
@@ -106,21 +105,25 @@ short_conv_single_kernel(const P* proj, const T* taps, const int* state_slots, f
 // accesses; every input row is read once for all the taps that want it (and the taps of a thread's channels once).  A
 // row's request is the same for all threads of a block, so the cases below are uniform branches.  Per element the
 // sums of the kernel above.
+// The thread whose tile holds a request's first row computes all rows that look at the request's state, those behind the
+// tile among them (the next tile leaves them out), and so can move the state on itself: a launch for that alone was 5 us of the 19 that
+// 6,144 channels of 2,000 rows took, and the next kernel waited for it.
 #define SC_TILE 8
 template <typename O, int K>
 __global__ void __launch_bounds__(256)
 short_conv_rows_kernel(O* __restrict__ out, const bf16_t* __restrict__ proj, int width, int first_col, int channels,
-                       const bf16_t* __restrict__ taps, const bf16_t* __restrict__ bias, const float* __restrict__ state,
+                       const bf16_t* __restrict__ taps, const bf16_t* __restrict__ bias, float* __restrict__ state,
                        const int* __restrict__ state_slots, const int* __restrict__ token_seq,
                        const int* __restrict__ query_start_loc, int activation, int tokens) {
   const int c = 4 * (blockIdx.y * blockDim.x + threadIdx.x);
   if (c >= channels) return;
   const int t0 = blockIdx.x * SC_TILE;
+  const bf16_t* const mine = proj + first_col + c;
   uint2 raw[SC_TILE + K - 1];  // rows t0 - (K - 1) .. t0 + SC_TILE - 1 of the projection
 #pragma unroll
   for (int i = 0; i < SC_TILE + K - 1; ++i) {
     const int row = min(max(t0 - (K - 1) + i, 0), tokens - 1);  // (a row outside is never looked at)
-    raw[i] = *reinterpret_cast<const uint2*>(proj + (size_t)row * width + first_col + c);
+    raw[i] = *reinterpret_cast<const uint2*>(mine + (size_t)row * width);
   }
   // The 4 K taps of the thread's channels lie side by side: K loads of four.
   float w[4 * K], add[4] = {0.f, 0.f, 0.f, 0.f};
@@ -132,26 +135,22 @@ short_conv_rows_kernel(O* __restrict__ out, const bf16_t* __restrict__ proj, int
     for (int e = 0; e < 4; ++e) w[4 * f + e] = four[e];
   }
   if (bias) load_vec<bf16_t, 4>(bias + c, add);
-#pragma unroll
-  for (int j = 0; j < SC_TILE; ++j) {
-    const int t = t0 + j;
-    if (t >= tokens) break;
-    const int seq = token_seq[t];
-    const int index = t - query_start_loc[seq];  // the token's place in its request's portion
+  auto wide = [](uint2 r, float (&u)[4]) __attribute__((always_inline)) {
+    u[0] = __uint_as_float(r.x << 16);
+    u[1] = __uint_as_float(r.x & 0xffff0000u);
+    u[2] = __uint_as_float(r.y << 16);
+    u[3] = __uint_as_float(r.y & 0xffff0000u);
+  };
+  auto held = [&](int seq) __attribute__((always_inline)) { return state + (size_t)state_slots[seq] * (K - 1) * channels + c; };
+  // Row t, the `index`-th of its request's portion; input(f): the row that tap f takes, where the step brings it.
+  auto row = [&](int t, int seq, int index, auto input) __attribute__((always_inline)) {
     float y[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int f = 0; f < K; ++f) {
       const int back = index - (K - 1) + f;
       float u[4];
-      if (back >= 0) {
-        const uint2 r = raw[j + f];
-        u[0] = __uint_as_float(r.x << 16);
-        u[1] = __uint_as_float(r.x & 0xffff0000u);
-        u[2] = __uint_as_float(r.y << 16);
-        u[3] = __uint_as_float(r.y & 0xffff0000u);
-      } else {
-        load_vec<float, 4>(state + ((size_t)state_slots[seq] * (K - 1) + K - 1 + back) * channels + c, u);
-      }
+      if (back >= 0) wide(input(f), u);
+      else load_vec<float, 4>(held(seq) + (size_t)(K - 1 + back) * channels, u);
 #pragma unroll
       for (int e = 0; e < 4; ++e) y[e] = fmaf(w[e * K + f], u[e], y[e]);
     }
@@ -162,6 +161,47 @@ short_conv_rows_kernel(O* __restrict__ out, const bf16_t* __restrict__ proj, int
       if (activation == 1) y[e] *= __builtin_amdgcn_rcpf(1.f + __expf(-y[e]));
     }
     store_vec<O, 4>(out + (size_t)t * channels + c, y);
+  };
+  // Most tiles lie inside a request, behind the rows that look at its state: one trip says so, where row after row each waited for two.
+  const int first_seq = token_seq[t0], last_seq = token_seq[min(t0 + SC_TILE, tokens) - 1];
+  if (first_seq == last_seq && t0 + SC_TILE <= tokens && t0 - query_start_loc[first_seq] >= K - 1) {
+#pragma unroll
+    for (int j = 0; j < SC_TILE; ++j) row(t0 + j, first_seq, K - 1, [&](int f) __attribute__((always_inline)) { return raw[j + f]; });
+    return;
+  }
+  int begins = 0;  // bit j: a request begins at row t0 + j
+#pragma unroll
+  for (int j = 0; j < SC_TILE; ++j) {
+    const int t = t0 + j;
+    if (t >= tokens) break;
+    const int seq = token_seq[t];
+    const int index = t - query_start_loc[seq];  // the token's place in its request's portion
+    if (index == 0) begins |= 1 << j;
+    if (index < K - 1 && index > j) continue;  // the tile before computes it
+    row(t, seq, index, [&](int f) __attribute__((always_inline)) { return raw[j + f]; });
+  }
+  if (K == 1 || begins == 0) return;
+  const int begin = query_start_loc[last_seq];
+  if (begin >= t0) {
+    const int end = min(begin + K - 1, query_start_loc[last_seq + 1]);
+    for (int t = t0 + SC_TILE; t < end; ++t)
+      row(t, last_seq, t - begin, [&](int f) __attribute__((always_inline)) {
+        return *reinterpret_cast<const uint2*>(mine + (size_t)(t - (K - 1) + f) * width);
+      });
+  }
+  for (int j = 0; j < SC_TILE; ++j) {
+    if (!(begins >> j & 1)) continue;
+    const int seq = token_seq[t0 + j], count = query_start_loc[seq + 1] - (t0 + j);
+    float* const to = held(seq);
+#pragma unroll
+    for (int i = 0; i < K - 1; ++i) {
+      // As in the kernel below: a place further on, read before it is written.
+      const int from = count - (K - 1) + i;
+      float u[4];
+      if (from >= 0) wide(*reinterpret_cast<const uint2*>(mine + (size_t)(t0 + j + from) * width), u);
+      else load_vec<float, 4>(to + (size_t)(i + count) * channels, u);
+      store_vec<float, 4>(to + (size_t)i * channels, u);
+    }
   }
 }
 
@@ -185,15 +225,25 @@ short_conv_carry_kernel(float* __restrict__ state, const P* __restrict__ proj, i
   }
 }
 
+template <typename P>
+static int launch_short_conv_carry(float* state, const void* proj, int splits, long split_stride, int width, int first_col, int channels,
+                                   int k, const int* state_slots, const int* query_start_loc, int num_seqs, hipStream_t stream) {
+  if (k == 1 || num_seqs == 0) return TS_OK;  // one tap: nothing is carried
+  hipLaunchKernelGGL((short_conv_carry_kernel<P>), dim3(num_seqs, (channels + 255) / 256), dim3(256), 0, stream, state, (const P*)proj,
+                     splits, (size_t)split_stride, width, first_col, channels, k, state_slots, query_start_loc);
+  return ts_launch_status();
+}
+
 // dtype: the run's type (taps, and the projection unless it is partial sums); out_f32: a 32-bit result.
 extern "C" int ts_short_conv(void* out, int out_f32, const void* proj, int in_f32, int splits, long split_stride, int width,
                              int first_col, int channels, const void* taps, const void* bias, int k, float* state,
                              const int* state_slots, const int* token_seq, const int* query_start_loc, int tokens,
-                             int activation, int single, int dtype, hipStream_t stream) {
+                             int num_seqs, int activation, int dtype, hipStream_t stream) {
   if (tokens == 0) return TS_OK;
   if (!out || !proj || !taps || (!state && k > 1) || !state_slots || !token_seq || !query_start_loc) return TS_ERR_ARG;
   if (k < 1 || k > SC_MAX_TAPS || channels < 1 || first_col < 0 || first_col + channels > width || splits < 1) return TS_ERR_SHAPE;
-  if (activation < 0 || activation > 1) return TS_ERR_ARG;
+  if (activation < 0 || activation > 1 || num_seqs < 0) return TS_ERR_ARG;
+  const int single = tokens == num_seqs;  // every request brings one token
   const dim3 grid(tokens, (channels + 255) / 256), block(256);
   if (grid.y > 65535) return TS_ERR_SHAPE;
   if (dtype == TS_BF16 && !in_f32 && !single && tokens >= 32 && channels % 4 == 0 && width % 4 == 0 && first_col % 4 == 0 &&
@@ -241,24 +291,9 @@ extern "C" int ts_short_conv(void* out, int out_f32, const void* proj, int in_f3
   else if (dtype == TS_BF16) SC_GO(bf16_t, bf16_t, bf16_t);
   else return TS_ERR_DTYPE;
 #undef SC_GO
-  return ts_launch_status();
-}
-
-extern "C" int ts_short_conv_carry(float* state, const void* proj, int in_f32, int splits, long split_stride, int width,
-                                   int first_col, int channels, int k, const int* state_slots, const int* query_start_loc,
-                                   int num_seqs, int dtype, hipStream_t stream) {
-  if (num_seqs == 0 || k == 1) return TS_OK;  // one tap: nothing is carried
-  if (!state || !proj || !state_slots || !query_start_loc) return TS_ERR_ARG;
-  if (k < 1 || k > SC_MAX_TAPS || channels < 1 || first_col < 0 || first_col + channels > width || splits < 1) return TS_ERR_SHAPE;
-  const dim3 grid(num_seqs, (channels + 255) / 256), block(256);
-  if (grid.y > 65535) return TS_ERR_SHAPE;
+  const int status = ts_launch_status();
+  if (single || status != TS_OK) return status;
   if (dtype == TS_F32 || in_f32)
-    hipLaunchKernelGGL((short_conv_carry_kernel<float>), grid, block, 0, stream, state, (const float*)proj, splits,
-                       (size_t)split_stride, width, first_col, channels, k, state_slots, query_start_loc);
-  else if (dtype == TS_BF16)
-    hipLaunchKernelGGL((short_conv_carry_kernel<bf16_t>), grid, block, 0, stream, state, (const bf16_t*)proj, splits,
-                       (size_t)split_stride, width, first_col, channels, k, state_slots, query_start_loc);
-  else
-    return TS_ERR_DTYPE;
-  return ts_launch_status();
+    return launch_short_conv_carry<float>(state, proj, splits, split_stride, width, first_col, channels, k, state_slots, query_start_loc, num_seqs, stream);
+  return launch_short_conv_carry<bf16_t>(state, proj, splits, split_stride, width, first_col, channels, k, state_slots, query_start_loc, num_seqs, stream);
 }

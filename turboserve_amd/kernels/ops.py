@@ -99,8 +99,6 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "ts_scale_cap": [c_void_p, c_long, c_float, c_float, c_void_p],
         "ts_short_conv": [c_void_p, c_int, c_void_p, c_int, c_int, c_long, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p,
                           c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
-        "ts_short_conv_carry": [c_void_p, c_void_p, c_int, c_int, c_long, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
-                                c_int, c_int, c_void_p],
         "ts_decaying_walk": [*[c_void_p] * 6, c_int, c_int, c_long, *[c_int] * 4, c_void_p, c_int, c_int, c_long, c_int, c_int, c_void_p,
                              c_void_p, c_float, c_void_p, c_float, c_void_p, c_void_p, *[c_int] * 8, c_void_p],
         "ts_decaying_pieces": [*[c_void_p] * 6, *[c_int] * 4, c_void_p, c_int, c_int, c_long, c_int, c_int, c_void_p, c_void_p, c_float,
@@ -1075,7 +1073,7 @@ class Ops:
         """A short causal convolution over time on the ``C`` columns of ``proj`` from ``first_col`` on (``taps [C,
         K]``: ``y_t = sum_j taps[:, j] u_(t - K + 1 + j)``), continuing every request from the ``K - 1`` inputs its
         state slot holds (``state [slots, max(K - 1, 1), C]`` 32-bit, oldest first) and leaving its last ``K - 1``
-        inputs there (by a second launch; in a step whose requests all bring one token the first launch does it).
+        inputs there.
         ``proj`` is ``[T, W]`` of the run dtype or 32-bit partial sums.  Returns ``[T, C]`` of the run dtype (32-bit
         with ``out_float32``), plus ``bias [C]`` where given, through ``silu`` if asked."""
         _gpu(proj, taps, bias, state, state_slots, token_seq, query_start_loc)
@@ -1097,16 +1095,9 @@ class Ops:
         out = torch.empty((tokens, channels), dtype=torch.float32, device=proj.device) if wide \
             else self.rows_buffer(tokens, channels, dtype, proj.device)
         code = dtype_code(dtype)
-        # Every request brings one token: the launch that convolves also moves the state on.
-        single = tokens == num_seqs
         _check(self.core.ts_short_conv(_ptr(out), 1 if wide else 0, _ptr(proj), is_f32, splits, stride, width, first_col, channels,
                                        _ptr(taps), _ptr(bias), k, _ptr(state), _ptr(state_slots), _ptr(token_seq), _ptr(query_start_loc),
-                                       tokens, 1 if silu else 0, 1 if single else 0, code, self.stream()), "ts_short_conv")
-        if single:
-            return out
-        _check(self.core.ts_short_conv_carry(_ptr(state), _ptr(proj), is_f32, splits, stride, width, first_col, channels, k,
-                                             _ptr(state_slots), _ptr(query_start_loc), num_seqs, code, self.stream()),
-               "ts_short_conv_carry")
+                                       tokens, num_seqs, 1 if silu else 0, code, self.stream()), "ts_short_conv")
         return out
 
     def delta_rule(self, u: torch.Tensor, proj: torch.Tensor, *, beta_at: int, decay_at: int, gate_at: int, a2: torch.Tensor,
