@@ -805,3 +805,42 @@ def test_the_command_line_serves_the_design(tmp_path, capsys):
     sizing = capsys.readouterr().out
     sizing = json.loads(sizing[sizing.index("{"):])
     assert sorted(sizing["bytes_per_block"]) == sorted([2 * 2 * (16 + 24) * 2 * page, (8 + 8) * 2 * page]) and sizing["activation_bytes"] > 0
+
+
+@pytest.mark.parametrize("rule", ["selective", "fixed", "gated"])
+@pytest.mark.parametrize("n,p,heads,groups", [(8, 8, 2, 1), (32, 24, 8, 4), (64, 64, 8, 2), (128, 64, 16, 2), (136, 40, 3, 3), (256, 72, 8, 8)])
+@pytest.mark.parametrize("lengths", [[128], [1, 130, 128, 300], [2179], [4096, 17]])
+def test_the_states_before_the_pieces_two_ways(ops, monkeypatch, rule, n, p, heads, groups, lengths):
+    """A request's pieces one behind the other in one launch against pieces side by side put together by another: the same products summed in the
+    same order, so the same bits, but for the gated rule's sum of keys, which are products here and a chain there (32-bit sums of up to
+    4,096 terms whose weights fall off: 1e-6 of its size).  A piece, two tables of sixteen and more, a last piece of one row; rows that fill no tile."""
+    g = torch.Generator().manual_seed(n + p + len(lengths))
+    tokens = sum(lengths)
+    width = heads * p + 2 * groups * n + 2 * heads
+    width += -width % 8
+    u = torch.randn(tokens, width, generator=g).bfloat16().to(DEV)
+    first = heads * p + 2 * groups * n
+    one, two = torch.rand(heads, generator=g).to(DEV), torch.rand(heads, generator=g).to(DEV)
+    numbers = {"selective": (one - 4.0, two), "fixed": (1.0 - 0.1 * one,), "gated": (one - 3.0, two + 3.0)}[rule]
+    slots = [3 * i + 1 for i in range(len(lengths))]
+    starts = [sum(lengths[:i]) for i in range(len(lengths) + 1)]
+    pieces, carries = ops.linear_state_pieces(lengths, 128)
+    plan = (ops.device_ints(pieces), ops.device_ints(carries), len(pieces), len(carries), max(c[2] for c in carries))
+    results = []
+    for passes in (True, False):
+        monkeypatch.setattr(type(ops), "_decaying_passes", lambda self, *sizes: passes)
+        fresh = torch.Generator().manual_seed(n)
+        state = torch.randn(3 * len(lengths) + 2, heads, p, n, generator=fresh).to(DEV)
+        sums, tops = torch.randn(state.shape[0], heads, n, generator=fresh).to(DEV), torch.rand(state.shape[0], heads, generator=fresh).to(DEV)
+        y, norm = ops.decaying_state(
+            rule, u, (0, heads * p, heads * p + groups * n), state, torch.tensor(slots, dtype=torch.int32, device=DEV),
+            torch.tensor(starts, dtype=torch.int32, device=DEV), num_seqs=len(lengths), heads=heads, groups=groups, state_dim=n, value_dim=p,
+            dtype=torch.bfloat16, proj=None if rule == "fixed" else u, first_gate=0 if rule == "fixed" else first, numbers=numbers, cap=15.0 if rule == "gated" else 0.0,
+            skip=one if rule == "selective" else None, sums=sums if rule == "gated" else None, tops=tops if rule == "gated" else None, plan=plan)
+        results.append((y, state, norm, sums))
+    (y, state, norm, sums), (y2, state2, norm2, sums2) = results
+    assert bool(y.isfinite().all()) and torch.equal(y, y2) and torch.equal(state, state2)
+    if rule == "gated":
+        assert torch.equal(norm[..., 1], norm2[..., 1])
+        for a, b in ((norm[..., 0], norm2[..., 0]), (sums, sums2)):
+            assert float((a - b).norm()) <= 1e-6 * float(b.norm())

@@ -24,9 +24,10 @@
 //     S_end = exp(t_0 - t_last) S_before + sum_j w_j exp(s_j - t_last) B_j x_j^T
 //     y_i   = exp(t_0 - t_i) S_before^T C_i + sum_{j <= i} w_j exp(s_j - t_i) (C_i . B_j) x_j,
 // (the blocked form of Dao and Gu, "Transformers are SSMs: Generalized Models and Efficient Algorithms Through
-// Structured State Space Duality"), in three launches: ts_decaying_pieces mode 0 (every piece's own S_end from a zero
-// state), ts_decaying_carry (the state before each piece, elementwise; the last one goes to the slot),
-// mode 1 (y).  x, B and C are bfloat16 numbers, so C . B is exact products summed in 32-bit; every other factor is a
+// Structured State Space Duality"), in two or three launches: ts_decaying_pass (the state before each piece, a request's
+// pieces one behind the other; what the last one leaves goes to the slot), or where those would be too many rounds of workgroups or too few
+// workgroups ts_decaying_pieces mode 0 (every piece's own S_end from a zero state, the pieces side by side) and ts_decaying_carry (the states
+// before the pieces, elementwise); then ts_decaying_pieces mode 1 (y).  x, B and C are bfloat16 numbers, so C . B is exact products summed in 32-bit; every other factor is a
 // 32-bit number that is cut into three bfloat16 numbers whose sum it is exactly, and the three products are summed
 // in 32-bit: nothing of the recurrence is rounded to 16 bits.
 //
@@ -36,6 +37,8 @@
 // ts_gated_group_norm: y silu(z), every one of `parts` equal parts of a row divided by its own root mean square, times
 // a gain, rounded once.
 #include "vec.hpp"
+
+#include <type_traits>
 
 #define SS_PIECE 128
 #define SS_STRETCH 32
@@ -333,30 +336,68 @@ struct SsSteps {
   __device__ __forceinline__ float passed(int r, int i) const { return (t_top(r) - t_top(i)) + (t_low(r) - t_low(i)); }
 };
 
-// By the first wavefront: lane l takes the tokens 2 l and 2 l + 1 (beyond the piece: nothing decays, nothing is added).
+// What the projection says of a wavefront's two tokens a lane, 2 l and 2 l + 1 (rows beyond the piece: its last one's).
+template <int RULE>
+struct SsInputs {
+  float one[2];                        // d; i'
+  float two[RULE == SS_GATED ? 2 : 1]; // f'
+};
+
+// For several pieces at once, so that their loads are on their way together.
+template <int RULE, int COUNT, typename P>
+__device__ __forceinline__ void ss_inputs(SsInputs<RULE> (&in)[COUNT], const P* proj, const SsGates& gates, int h, int heads, const SsPiece (&pieces)[COUNT]) {
+  if (RULE == SS_FIXED) return;
+  const P* column = proj + gates.first + h;
+  const int lane = threadIdx.x % TS_WAVE;
+  if (gates.splits == 1) {
+    P raw[COUNT][2][RULE == SS_GATED ? 2 : 1];
+#pragma unroll
+    for (int x = 0; x < COUNT; ++x)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const P* row = column + (size_t)(pieces[x].first + min(2 * lane + e, pieces[x].count - 1)) * gates.width;
+        raw[x][e][0] = row[0];
+        if (RULE == SS_GATED) raw[x][e][RULE == SS_GATED ? 1 : 0] = row[heads];
+      }
+#pragma unroll
+    for (int x = 0; x < COUNT; ++x)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        in[x].one[e] = to_float(raw[x][e][0]);
+        if (RULE == SS_GATED) in[x].two[RULE == SS_GATED ? e : 0] = to_float(raw[x][e][RULE == SS_GATED ? 1 : 0]);
+      }
+    return;
+  }
+#pragma unroll
+  for (int x = 0; x < COUNT; ++x)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const P* row = column + (size_t)(pieces[x].first + min(2 * lane + e, pieces[x].count - 1)) * gates.width;
+      if (RULE == SS_GATED) ss_input_two(row, row + heads, gates.splits, gates.stride, in[x].one[e], in[x].two[RULE == SS_GATED ? e : 0]);
+      else in[x].one[e] = ss_input(row, gates.splits, gates.stride);
+    }
+}
+
+// By one wavefront: lane l takes the tokens 2 l and 2 l + 1 (beyond the piece: nothing decays, nothing is added).
 // `floor`: what t starts from (gated).
-template <int RULE, typename P>
-__device__ __forceinline__ void ss_steps(SsSteps<RULE>& at, const P* proj, const SsGates& gates, int h, int heads, double floor, SsPiece piece) {
-  const int lane = threadIdx.x;
+template <int RULE>
+__device__ __forceinline__ void ss_steps(SsSteps<RULE>& at, const SsInputs<RULE>& inputs, const SsGates& gates, int h, double floor, int count) {
+  const int lane = threadIdx.x % TS_WAVE;
   float w[2];
   double gone[2], in[2] = {0., 0.};  // log a; the log input gate
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
-    const int j = 2 * lane + e, t = piece.first + min(j, piece.count - 1);
-    const bool there = j < piece.count;
+    const bool there = 2 * lane + e < count;
     if (RULE == SS_SELECTIVE) {
-      const float z = ss_input(proj + (size_t)t * gates.width + gates.first + h, gates.splits, gates.stride) + gates.one[h];
-      w[e] = there ? ss_softplus(z) : 0.f;
+      w[e] = there ? ss_softplus(inputs.one[e] + gates.one[h]) : 0.f;
       gone[e] = -(double)expf(gates.two[h]) * (double)w[e];
     } else if (RULE == SS_FIXED) {
       w[e] = there ? 1.f : 0.f;
       gone[e] = there ? log((double)gates.one[h]) : 0.;
     } else {
-      float i, f;
-      ss_log_gates(proj, gates, t, h, heads, i, f);
       w[e] = there ? 1.f : 0.f;
-      gone[e] = there ? (double)f : 0.;
-      in[e] = (double)i;
+      gone[e] = there ? (double)ss_log_sigmoid(ss_capped(inputs.two[RULE == SS_GATED ? e : 0] + gates.two[h], gates.cap)) : 0.;
+      in[e] = (double)ss_capped(inputs.one[e] + gates.one[h], gates.cap);
     }
   }
   const double own = gone[0] + gone[1];
@@ -370,7 +411,7 @@ __device__ __forceinline__ void ss_steps(SsSteps<RULE>& at, const P* proj, const
   double s[2] = {-c[0], -c[1]};
   if (RULE == SS_GATED) {
 #pragma unroll
-    for (int e = 0; e < 2; ++e) s[e] = 2 * lane + e < piece.count ? in[e] + s[e] : SS_NEVER;
+    for (int e = 0; e < 2; ++e) s[e] = 2 * lane + e < count ? in[e] + s[e] : SS_NEVER;
     double most = fmax(s[0], s[1]);
 #pragma unroll
     for (int d = 1; d < TS_WAVE; d <<= 1) {
@@ -446,7 +487,12 @@ decaying_piece_state_kernel(float* __restrict__ piece_state, float* __restrict__
   const size_t b_at = (size_t)rows.b_at + (size_t)g * n, x_at = (size_t)rows.x_at + (size_t)h * p + c0;
   const bool summing = RULE == SS_GATED && blockIdx.z == 0;  // this workgroup also makes the piece's n, thread d row d
   float own_sum = 0.f;
-  if (wave == 0) ss_steps<RULE>(steps, proj, gates, h, heads, SS_NEVER, piece);
+  if (wave == 0) {
+    SsInputs<RULE> in[1];
+    const SsPiece one[1] = {piece};
+    ss_inputs<RULE>(in, proj, gates, h, heads, one);
+    ss_steps<RULE>(steps, in[0], gates, h, SS_NEVER, piece.count);
+  }
   const size_t columns = RULE == SS_GATED ? p + 1 : p;
   ss_f32x4 acc[TILES][PT];
 #pragma unroll
@@ -592,6 +638,276 @@ decaying_carry_kernel(float* __restrict__ state, float* __restrict__ sums, const
   *reinterpret_cast<float4*>(slot) = s;
 }
 
+// Four 16-bit numbers of sixteen lanes turned over: lane i reads row i / 4, columns 4 (i % 4) .. + 3 of a tile of 4 x 16 and gets column
+// i, rows 0 .. 3.
+typedef short ss_i16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) ss_i16x4 ss_lds_i16x4;
+typedef __attribute__((address_space(3))) uint16_t ss_lds_u16;
+typedef __attribute__((address_space(3))) uint32_t ss_lds_u32;
+typedef __attribute__((address_space(3))) ts_u32x4 ss_lds_u32x4;
+__device__ __forceinline__ ts_u32x4 ss_read_turned(const ss_lds_u16* first, const ss_lds_u16* second) {
+  const ss_u32x2 a = __builtin_bit_cast(ss_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ss_lds_i16x4*)first));
+  const ss_u32x2 b = __builtin_bit_cast(ss_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((ss_lds_i16x4*)second));
+  return ts_u32x4{a[0], a[1], b[0], b[1]};
+}
+
+// Workgroups go to the eight dies in turn: those of neighbouring heads, which share B and C, to one of them and its L2 (`turn`: a workgroup's
+// number among the heads', which the grid counts first).
+__device__ __forceinline__ int ss_head(int turn, int heads) { return heads % 8 == 0 ? turn % 8 * (heads / 8) + turn / 8 : turn; }
+
+// The state before every piece, and behind the last.  A workgroup takes a request's pieces one behind the other, with ROWS rows by COLS
+// columns of a head's state in the registers of its first four wavefronts: the piece's own S_end^T (rows n, columns p) = sum over j of B^T
+// (exact) times the weighted x (three planes) on the matrix cores, then S = exp(t_0 - t_last) S + S_end.  So the pieces' own ends never go
+// through memory and no launch puts them together.  The other four wavefronts bring the next piece to LDS meanwhile: B straight from
+// memory, as its rows lie (the reads turn it over; LDS takes 30 bytes a cycle from registers, twice that from memory), x weighted and
+// cut; its rows have travelled for two pieces.  The gates of up to sixteen pieces are made at the start.
+// What bounds it is LDS, some 1,200 cycles a piece: so a wavefront multiplies 32 rows, and a workgroup has all rows of few columns, whose x
+// it alone weighs.  16 pieces of 64 heads of 128 x 64, whose states before the pieces are 34 MB: 22.5 us where the pieces' own ends
+// side by side and a launch that puts them together take 32; one piece 6.6 against 12.8 (alone, in a graph).
+// piece_state [pieces][H][P (gated: + 1, n)][N]; piece_top [pieces][H] (gated): m before each piece.  The slot's own m stays until the
+// finish, since every workgroup here reads it.
+// `to` and `lds` are the same memory: B goes there through the one name, all else uses the other, and __restrict__ keeps the compiler from
+// waiting for every load in flight before every read.  So it must not see that two reads have one address: the slots of what is
+// read behind a barrier have come through an asm behind it.  An edit has to keep that.
+#define SS_TABLE 16
+template <typename P, int RULE, int ROWS>
+__device__ __forceinline__ void
+decaying_pass(ss_lds_u16* __restrict__ to, ss_lds_u16* __restrict__ lds, SsSteps<RULE>* steps, float (*ends)[SS_PIECE], float* decay_of, float* most_of,
+              float* __restrict__ state, float* __restrict__ sums, const float* __restrict__ tops, const int* __restrict__ state_slots,
+              const SsCarry* __restrict__ carries, const SsPiece* __restrict__ pieces, float* __restrict__ piece_state,
+              float* __restrict__ piece_top, const bf16_t* __restrict__ u, SsRows rows, const P* __restrict__ proj, SsGates gates, int heads,
+              int groups, int n, int p) {
+  constexpr int WAVES = 8, HALF = 256, COLS = 2048 / ROWS, EACH = SS_TABLE / WAVES;
+  // In LDS: two pieces of x, [3 planes][tokens][COLS], then three of B, [tokens][ROWS].
+  constexpr int X_PLANE = SS_PIECE * COLS, X_PIECE = 3 * X_PLANE, B_PIECE = SS_PIECE * ROWS, CHUNKS = ROWS / 8;
+  constexpr int X_ITEMS = X_PLANE / 8 / HALF, B_LOADS = B_PIECE / 8 / HALF;  // of eight elements, 16 bytes
+  const SsCarry carry = carries[blockIdx.y];
+  if (carry.count < 1) return;
+  // The request's pieces are SS_PIECE rows each, one behind the other, but for the last one's.
+  const int first_row = pieces[carry.first].first, last_count = pieces[carry.first + carry.count - 1].count;
+  auto piece_of = [&](int i) __attribute__((always_inline)) {
+    const int at = min(i, carry.count - 1);
+    return SsPiece{0, first_row + SS_PIECE * at, at == carry.count - 1 ? last_count : SS_PIECE, 0};
+  };
+  const int h = ss_head(blockIdx.x, heads), g = h / (heads / groups), slices = (n + ROWS - 1) / ROWS;
+  const int n0 = (int)blockIdx.z % slices * ROWS, c0 = (int)blockIdx.z / slices * COLS;
+  const int tid = threadIdx.x % HALF, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TS_WAVE), lane = threadIdx.x % TS_WAVE;
+  const int lo = lane % 16, quad = lane / 16;
+  const bool brings = wave >= WAVES / 2;
+  const int u_width = rows.width;
+  const size_t owner = (size_t)state_slots[carry.slot_seq] * heads + h;
+  const int columns = RULE == SS_GATED ? p + 1 : p;
+  // Where a token's row of x and its chunk of eight elements of B lie: the reads of four tokens by sixteen columns of each of four
+  // groups of eight tokens touch every bank twice.
+  auto x_row = [](int t) __attribute__((always_inline)) { return COLS == 16 ? (t & ~12) | (t & 4) << 1 | (t & 8) >> 1 : t; };
+  auto b_chunk = [](int t, int chunk) __attribute__((always_inline)) { return chunk ^ ((((t & 3) | (t >> 1 & 4)) << 1) & (CHUNKS - 1)); };
+
+  // -- the wavefronts that bring: B of a piece on its way to LDS (tokens beyond the piece: zeros), x on its way to registers, and from there
+  int b_off[B_LOADS];
+#pragma unroll
+  for (int y = 0; y < B_LOADS; ++y) {
+    const int item = tid + HALF * y, t = item / CHUNKS, chunk = b_chunk(t, item % CHUNKS);
+    b_off[y] = (t * u_width + (n0 + 8 * chunk < n ? 8 * chunk : 0)) * 2;
+  }
+  const uint16_t* const b_from = reinterpret_cast<const uint16_t*>(u) + rows.b_at + (size_t)g * n + n0;
+  const uint16_t* const x_from = reinterpret_cast<const uint16_t*>(u) + rows.x_at + (size_t)h * p;
+  auto fetch_b = [&](const SsPiece piece, int slot) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(b_from + (size_t)piece.first * u_width), 0,
+                                                                            ((piece.count - 1) * u_width + min(n - n0, ROWS)) * 2, 0x00027000);
+#pragma unroll
+    for (int y = 0; y < B_LOADS; ++y)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, to + 2 * X_PIECE + slot * B_PIECE + (HALF * y + TS_WAVE * (wave % 4)) * 8, 16, b_off[y], 0, 0, 0);
+  };
+  struct Part {
+    ts_u32x4 x[X_ITEMS];
+  };
+  auto fetch_x = [&](Part& part, const SsPiece piece) __attribute__((always_inline)) {
+#pragma unroll
+    for (int y = 0; y < X_ITEMS; ++y) {
+      // (Unconditional, of the piece's last row or the first columns where nothing is there, whose weight is 0 or whose result is not stored.)
+      const int item = tid + HALF * y, t = min(item / (COLS / 8), piece.count - 1), c = c0 + item % (COLS / 8) * 8;
+      part.x[y] = *reinterpret_cast<const ts_u32x4*>(x_from + (size_t)(piece.first + t) * u_width + (c < p ? c : 0));
+    }
+  };
+  auto put = [&](int i, const Part& part) __attribute__((always_inline)) {
+#pragma unroll
+    for (int y = 0; y < X_ITEMS; ++y) {
+      const int item = tid + HALF * y, t = item / (COLS / 8), d = item % (COLS / 8) * 8;
+      const float w = ends[i % SS_TABLE][t];
+      const ts_u32x4 x = RULE == SS_GATED && c0 + d == p ? ts_u32x4{0x3f80u, 0u, 0u, 0u} : part.x[y];  // (n: x is 1)
+      ts_u32x4 planes[3];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t top[2], mid[2], low[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) ss_cut(w * __uint_as_float(k ? x[e] & 0xffff0000u : x[e] << 16), top[k], mid[k], low[k]);
+        planes[0][e] = ss_pair(top[0], top[1]);
+        planes[1][e] = ss_pair(mid[0], mid[1]);
+        planes[2][e] = ss_pair(low[0], low[1]);
+      }
+#pragma unroll
+      for (int plane = 0; plane < 3; ++plane)
+        *(ss_lds_u32x4*)(lds + i % 2 * X_PIECE + plane * X_PLANE + x_row(t) * COLS + d) = planes[plane];
+    }
+  };
+  Part ahead[2];
+  if (brings) {
+    fetch_x(ahead[0], piece_of(0));
+    fetch_b(piece_of(0), 0);
+    fetch_x(ahead[1], piece_of(1));
+    fetch_b(piece_of(1), 1);
+  }
+
+  // -- the wavefronts that multiply: tiles of rows n0 + row0 + 16 a + 4 quad .. + 3, column c
+  const int row0 = 32 * (wave % 4 % (ROWS / 32)), col0 = 16 * (wave % 4 / (ROWS / 32));
+  const int c = c0 + col0 + lo;
+  const size_t step = (size_t)heads * columns * n;
+  ss_f32x4 held[2];
+  bool live[2];
+  float *slot[2], *before[2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    const int d = n0 + row0 + 16 * a + 4 * quad;
+    live[a] = !brings && d < n && c < columns;
+    slot[a] = RULE == SS_GATED && c == p ? sums + owner * n + d : state + (owner * p + c) * n + d;
+    before[a] = piece_state + ((size_t)carry.first * heads + h) * columns * n + (size_t)c * n + d;
+    held[a] = ss_f32x4{0.f, 0.f, 0.f, 0.f};
+    if (live[a]) held[a] = *reinterpret_cast<const ss_f32x4*>(slot[a]);
+  }
+  float top = RULE == SS_GATED ? tops[owner] : 0.f;
+
+  // All LDS accesses done, then the workgroup's barrier (the fence of __syncthreads would wait for the loads, too).
+  auto meet = []() __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // Of piece i, whose x and B lie in LDS.
+  auto multiply = [&](int i, int slot_b) __attribute__((always_inline)) {
+    int x_now = i % 2 * X_PIECE, b_now = 2 * X_PIECE + slot_b * B_PIECE;
+    asm volatile("" : "+s"(x_now), "+s"(b_now));
+    constexpr int STEPS = SS_PIECE / 32;
+    ts_u32x4 bf[STEPS][2], xf[STEPS][3];
+#pragma unroll
+    for (int k = 0; k < STEPS; ++k) {
+      const int t = 32 * k + 8 * quad + lo / 4;
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        const int chunk = row0 / 8 + 2 * a + lo % 4 / 2;
+        const ss_lds_u16* b = lds + b_now + lo % 2 * 4;
+        bf[k][a] = ss_read_turned(b + t * ROWS + 8 * b_chunk(t, chunk), b + (t + 4) * ROWS + 8 * b_chunk(t + 4, chunk));
+      }
+#pragma unroll
+      for (int plane = 0; plane < 3; ++plane) {
+        const ss_lds_u16* x = lds + x_now + plane * X_PLANE + col0 + 4 * (lo % 4);
+        xf[k][plane] = ss_read_turned(x + x_row(t) * COLS, x + x_row(t + 4) * COLS);
+      }
+    }
+    float a_of = decay_of[i % SS_TABLE], w_of = 1.f;
+    const float most = RULE == SS_GATED ? most_of[i % SS_TABLE] : 0.f;
+    ss_f32x4 own[2] = {ss_f32x4{0.f, 0.f, 0.f, 0.f}, ss_f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int k = 0; k < STEPS; ++k)
+#pragma unroll
+      for (int plane = 2; plane >= 0; --plane)  // (the small planes first)
+#pragma unroll
+        for (int a = 0; a < 2; ++a) own[a] = ss_mfma(bf[k][a], xf[k][plane], own[a]);
+    if (RULE == SS_GATED) {
+      if (threadIdx.x == 0 && blockIdx.z == 0) piece_top[(size_t)(carry.first + i) * heads + h] = top;
+      const float decay = a_of, after = fmaxf(decay + top, most);
+      a_of = expf(decay + top - after);
+      w_of = expf(most - after);
+      top = after;
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      if (live[a]) *reinterpret_cast<ss_f32x4*>(before[a]) = held[a];
+      before[a] += step;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) held[a][e] = fmaf(a_of, held[a][e], w_of * own[a][e]);
+    }
+  };
+  int slot_b = 0;  // of the piece whose turn it is
+  for (int i0 = 0; i0 < carry.count; i0 += SS_TABLE) {
+    const int batch = min(SS_TABLE, carry.count - i0);
+    if (i0 > 0) meet();  // the table's readers are done
+    if (wave < batch) {  // pieces wave, wave + 8, ..
+      SsPiece of[EACH];
+      SsInputs<RULE> in[EACH];
+#pragma unroll
+      for (int x = 0; x < EACH; ++x) of[x] = piece_of(i0 + min(wave + WAVES * x, batch - 1));
+      ss_inputs<RULE>(in, proj, gates, h, heads, of);
+#pragma unroll
+      for (int x = 0; x < EACH; ++x) {
+        const int i = wave + WAVES * x;
+        if (i >= batch) break;
+        SsSteps<RULE>& at = steps[wave];
+        __builtin_amdgcn_wave_barrier();  // (a wavefront's accesses to LDS are in order)
+        ss_steps<RULE>(at, in[x], gates, h, SS_NEVER, of[x].count);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int e = 0; e < 2; ++e) ends[i][2 * lane + e] = at.w[2 * lane + e] * expf(at.from(2 * lane + e, SS_PIECE - 1));
+        if (lane == 0) {
+          decay_of[i] = RULE == SS_GATED ? at.total : expf(at.total);
+          most_of[i] = RULE == SS_GATED ? at.m[RULE == SS_GATED ? SS_PIECE - 1 : 0] : 0.f;
+        }
+      }
+    }
+    meet();
+    const int until = i0 + batch;
+    if (brings) {
+      // Behind a piece's barrier the slots of the piece before are free, x and B.  B of piece i has landed when no more than what has been asked
+      // for behind it at least, x and B of one turn, is on its way (what the next turn of the loop takes is not asked for later, and the scheduler
+      // moves nothing over its barriers).
+      auto bring = [&](int i, Part& part) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(B_LOADS + X_ITEMS) : "memory");
+        meet();
+        const int free_b = slot_b == 0 ? 2 : slot_b - 1;
+        slot_b = slot_b == 2 ? 0 : slot_b + 1;
+        fetch_b(piece_of(i + 2), free_b);
+        if (i + 1 < until) {
+          put(i + 1, part);
+          fetch_x(part, piece_of(i + 3));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      put(i0, ahead[0]);
+      fetch_x(ahead[0], piece_of(i0 + 2));
+      __builtin_amdgcn_sched_barrier(0);
+      int i = i0;
+      for (; i + 1 < until; i += 2) {  // (no way out between the two: the compiler would count the loads of one of them alone)
+        bring(i, ahead[1]);
+        bring(i + 1, ahead[0]);
+      }
+      if (i < until) bring(i, ahead[1]);
+    } else {
+      for (int i = i0; i < until; ++i) {
+        meet();
+        multiply(i, slot_b);
+        slot_b = slot_b == 2 ? 0 : slot_b + 1;
+      }
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+    if (live[a]) *reinterpret_cast<ss_f32x4*>(slot[a]) = held[a];
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // what has been asked for past the end must not come into another workgroup's LDS
+}
+
+template <typename P, int RULE, int ROWS>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+decaying_pass_kernel(float* __restrict__ state, float* __restrict__ sums, const float* __restrict__ tops, const int* __restrict__ state_slots,
+                     const SsCarry* __restrict__ carries, const SsPiece* __restrict__ pieces, float* __restrict__ piece_state,
+                     float* __restrict__ piece_top, const bf16_t* __restrict__ u, SsRows rows, const P* __restrict__ proj, SsGates gates,
+                     int heads, int groups, int n, int p) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t ss_lds[];
+  __shared__ SsSteps<RULE> steps[8];
+  __shared__ __attribute__((aligned(16))) float ends[SS_TABLE][SS_PIECE];  // the tokens' weights at their piece's end
+  __shared__ float decay_of[SS_TABLE], most_of[SS_TABLE];
+  decaying_pass<P, RULE, ROWS>((ss_lds_u16*)ss_lds, (ss_lds_u16*)ss_lds, steps, ends, decay_of, most_of, state, sums, tops, state_slots, carries,
+                               pieces, piece_state, piece_top, u, rows, proj, gates, heads, groups, n, p);
+}
+
 // Mode 1.  Wavefront w owns the tokens of the stretches w and 7 - w of sixteen (together they see as many tokens as any
 // other's two).  Everything is computed turned, y^T (rows p, columns i): the weights (C_i . B_j) exp(c_i - c_j) dt_j come
 // out of one product with token i on the lane and four tokens j in its registers, which is what the next product wants of
@@ -623,7 +939,12 @@ decaying_piece_out_kernel(float* __restrict__ y, float* __restrict__ norm, const
   const int tiles[2] = {wave, 7 - wave};
   const bool summing = RULE == SS_GATED && blockIdx.z == 0;
   const float enter = RULE == SS_GATED ? piece_top[(size_t)item * heads + h] : 0.f;  // t before the piece
-  if (wave == 0) ss_steps<RULE>(steps, proj, gates, h, heads, enter, piece);
+  if (wave == 0) {
+    SsInputs<RULE> in[1];
+    const SsPiece one[1] = {piece};
+    ss_inputs<RULE>(in, proj, gates, h, heads, one);
+    ss_steps<RULE>(steps, in[0], gates, h, enter, piece.count);
+  }
   const size_t head_state = ((size_t)item * heads + h) * (RULE == SS_GATED ? p + 1 : p);
   const float* entering = piece_state + (head_state + c0) * n;
   float sum_of[2] = {0.f, 0.f};  // this lane's share of n . C of its tokens
@@ -1085,6 +1406,59 @@ static int ss_pieces_launch(int mode, float* y, float* norm, float* piece_state,
   return ts_launch_status();
 }
 
+template <typename P, int RULE, int ROWS>
+static int ss_pass_launch(float* state, float* sums, const float* tops, const int* state_slots, const void* carries, int requests,
+                          const void* pieces, float* piece_state, float* piece_top, const void* u, SsRows rows, const void* proj, SsGates gates,
+                          int heads, int groups, int n, int p, hipStream_t stream) {
+  constexpr int COLS = 2048 / ROWS, lds = (2 * 3 * COLS + 3 * ROWS) * SS_PIECE * 2;
+  static const bool ready = hipFuncSetAttribute((const void*)decaying_pass_kernel<P, RULE, ROWS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                lds) == hipSuccess;
+  if (!ready) return TS_ERR_LAUNCH;
+  const int columns = RULE == SS_GATED ? p + 1 : p;
+  const dim3 grid(heads, requests, (n + ROWS - 1) / ROWS * ((columns + COLS - 1) / COLS));
+  hipLaunchKernelGGL((decaying_pass_kernel<P, RULE, ROWS>), grid, dim3(512), lds, stream, state, sums, tops, state_slots, (const SsCarry*)carries,
+                     (const SsPiece*)pieces, piece_state, piece_top, (const bf16_t*)u, rows, (const P*)proj, gates, heads, groups, n, p);
+  return ts_launch_status();
+}
+
+// What both launches of a cut portion ask of their operands.
+static int ss_pieces_ok(int rule, const void* u, const SsRows& rows, const SsGates& gates, const void* piece_state, int heads, int groups, int n, int p) {
+  if (!ss_sizes_ok(rule, rows, gates, heads, groups, n, p) || n > 256 || n % 8 != 0 || p % 8 != 0) return TS_ERR_SHAPE;
+  if (rows.width % 8 != 0 || rows.x_at % 8 != 0 || rows.b_at % 8 != 0 || rows.c_at % 8 != 0) return TS_ERR_SHAPE;  // 16-byte accesses
+  return ((uintptr_t)u | (uintptr_t)piece_state) % 16 != 0 ? TS_ERR_ARG : TS_OK;
+}
+
+// bfloat16 runs; the states before the pieces (and in the slots what the last piece leaves), from a request's pieces one behind the other.
+extern "C" int ts_decaying_pass(float* state, float* sums, const float* tops, const int* state_slots, const void* carries, int requests,
+                                const void* pieces, float* piece_state, float* piece_top, const void* u, int u_width, int x_at, int b_at, int c_at,
+                                const void* proj, int in_f32, int splits, long split_stride, int width, int first_gate, const float* one,
+                                const float* two, float cap, int heads, int groups, int n, int p, int rule, hipStream_t stream) {
+  if (requests == 0) return TS_OK;
+  const SsRows rows = {1, 0, u_width, x_at, b_at, c_at};
+  const SsGates gates = {splits, split_stride, width, first_gate, one, two, cap};
+  if (!state || !state_slots || !carries || !pieces || !piece_state || !u || (rule == SS_GATED && !piece_top)) return TS_ERR_ARG;
+  if (!ss_rule_ok(rule, gates, proj, piece_state, piece_state, sums, tops)) return TS_ERR_ARG;  // (no skip and no norm here)
+  const int status = ss_pieces_ok(rule, u, rows, gates, piece_state, heads, groups, n, p);
+  if (status != TS_OK) return status;
+  if (((uintptr_t)state | (uintptr_t)sums) % 16 != 0) return TS_ERR_ARG;
+#define SS_SIZE(P, RULE, ROWS)                                                                                                     \
+  return ss_pass_launch<P, RULE, ROWS>(state, sums, tops, state_slots, carries, requests, pieces, piece_state, piece_top, u, rows, \
+                                       proj, gates, heads, groups, n, p, stream)
+#define SS_GO(P, RULE)                      \
+  do {                                      \
+    if (n <= 32) SS_SIZE(P, RULE, 32);      \
+    if (n <= 64) SS_SIZE(P, RULE, 64);      \
+    SS_SIZE(P, RULE, 128);                  \
+  } while (0)
+  if (rule == SS_SELECTIVE && in_f32) SS_GO(float, SS_SELECTIVE);
+  if (rule == SS_SELECTIVE) SS_GO(bf16_t, SS_SELECTIVE);
+  if (rule == SS_FIXED) SS_GO(bf16_t, SS_FIXED);
+  if (in_f32) SS_GO(float, SS_GATED);
+  SS_GO(bf16_t, SS_GATED);
+#undef SS_GO
+#undef SS_SIZE
+}
+
 // bfloat16 runs; mode 0: every piece's own end state and decay; mode 1: y from the state before each piece.
 extern "C" int ts_decaying_pieces(float* y, float* norm, float* piece_state, float* piece_decay, const float* piece_top, const void* u,
                                   int u_width, int x_at, int b_at, int c_at, const void* proj, int in_f32, int splits, long split_stride,
@@ -1096,9 +1470,9 @@ extern "C" int ts_decaying_pieces(float* y, float* norm, float* piece_state, flo
   const SsGates gates = {splits, split_stride, width, first_gate, one, two, cap};
   if (!piece_state || !piece_decay || !u || !pieces || (mode == 1 && !y) || mode < 0 || mode > 1) return TS_ERR_ARG;
   if (!ss_rule_ok(rule, gates, proj, skip, norm, piece_state, piece_top)) return TS_ERR_ARG;
-  if (!ss_sizes_ok(rule, rows, gates, heads, groups, n, p) || n > 256 || n % 8 != 0 || p % 8 != 0) return TS_ERR_SHAPE;
-  if (u_width % 8 != 0 || x_at % 8 != 0 || b_at % 8 != 0 || c_at % 8 != 0) return TS_ERR_SHAPE;  // 16-byte accesses
-  if (((uintptr_t)u | (uintptr_t)piece_state | (uintptr_t)y) % 16 != 0) return TS_ERR_ARG;
+  const int status = ss_pieces_ok(rule, u, rows, gates, piece_state, heads, groups, n, p);
+  if (status != TS_OK) return status;
+  if ((uintptr_t)y % 16 != 0) return TS_ERR_ARG;
 #define SS_GO(P, RULE, NK, PT)                                                                                                     \
   return ss_pieces_launch<P, RULE, NK, PT>(mode, y, norm, piece_state, piece_decay, piece_top, u, rows, proj, gates, skip, scale,  \
                                            pieces, num_pieces, heads, groups, n, p, stream)

@@ -101,6 +101,8 @@ _SIGNATURES: dict[str, dict[str, list]] = {
                           c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
         "ts_decaying_walk": [*[c_void_p] * 6, c_int, c_int, c_long, *[c_int] * 4, c_void_p, c_int, c_int, c_long, c_int, c_int, c_void_p,
                              c_void_p, c_float, c_void_p, c_float, c_void_p, c_void_p, *[c_int] * 8, c_void_p],
+        "ts_decaying_pass": [*[c_void_p] * 5, c_int, *[c_void_p] * 4, *[c_int] * 4, c_void_p, c_int, c_int, c_long, c_int, c_int, c_void_p,
+                             c_void_p, c_float, *[c_int] * 5, c_void_p],
         "ts_decaying_pieces": [*[c_void_p] * 6, *[c_int] * 4, c_void_p, c_int, c_int, c_long, c_int, c_int, c_void_p, c_void_p, c_float,
                                c_void_p, c_float, c_void_p, *[c_int] * 7, c_void_p],
         "ts_decaying_carry": [*[c_void_p] * 8, *[c_int] * 5, c_void_p],
@@ -1230,9 +1232,21 @@ class Ops:
         def cut(step) -> tuple:  # the requests that bring several tokens come first
             pieces, carries = self.linear_state_pieces(step.query_lens[: step.num_prefill_seqs], self.decaying_piece)
             both = self.device_ints(pieces + carries)
-            return both[: len(pieces)], both[len(pieces):], len(pieces), len(carries)
+            return both[: len(pieces)], both[len(pieces):], len(pieces), len(carries), max(carry[2] for carry in carries)
 
         return ctx.derive(("decaying_pieces", self.decaying_piece), cut)
+
+    def _decaying_passes(self, pieces: int, requests: int, longest: int, heads: int, state_dim: int, columns: int) -> bool:
+        """Whether the states before a step's pieces are made a request's pieces one behind the other (``ts_decaying_pass``), not side by
+        side and put together by a launch of its own.  By a small model, in microseconds: a workgroup has a compute unit to itself and takes 3.5
+        and 1.05 a piece of its request (``longest`` at most), side by side it is 13 and 2.4 for every million elements of a piece's state
+        (side by side / one behind the other, heads x rows x columns: 64 x 128 x 64, one prompt of 128 / 512 / 2,000 tokens 12.8 / 6.6,
+        18.1 / 9.8, 32.2 / 22.5; 8 x 128 x 256, of 2,048 24.2 / 19.1, six of 300 24.9 / 19.3; 8 x 256 x 512 53.4 / 41.7, with the sum of
+        keys, a third round for few, 57.5 / 66.2; 16 x 64 x 64, 32 workgroups, 14.2 / 17.2; 32 x 128 x 128, 20 of 100 tokens, 20 rounds,
+        47.3 / 84.6)."""
+        rows = 32 if state_dim <= 32 else 64 if state_dim <= 64 else 128
+        workgroups = heads * requests * -(-state_dim // rows) * -(-columns // (2048 // rows))
+        return -(-workgroups // self.compute_units) * (3.5 + 1.05 * longest) < 13.0 + 2.4e-6 * pieces * heads * state_dim * columns
 
     def decaying_state(self, rule: str, u: torch.Tensor, columns: tuple[int, int, int], state: torch.Tensor, state_slots: torch.Tensor,
                        query_start_loc: torch.Tensor, *, num_seqs: int, heads: int, groups: int, state_dim: int, value_dim: int,
@@ -1254,8 +1268,8 @@ class Ops:
 
         All in 32-bit; ``numbers`` are 32-bit ``[H]``.  Returns ``(y [T, H P], norm)``, both 32-bit, ``norm [T, H, 2]`` being ``(scale
         n . C, m')`` for the gated rule, else ``None``.  Without a ``plan`` every request is walked; ``plan = (pieces, carries,
-        n_pieces, n_requests)`` (:meth:`decaying_plan`) cuts the first ``n_requests`` into pieces of :attr:`decaying_piece` tokens
-        that run side by side, and the requests behind them are walked."""
+        n_pieces, n_requests[, pieces of the longest])`` (:meth:`decaying_plan`) cuts the first ``n_requests`` into pieces of
+        :attr:`decaying_piece` tokens, the last one of a request what is left, and the requests behind them are walked."""
         _gpu(u, state, state_slots, query_start_loc, proj, skip, sums, tops, *numbers)
         _i32(state_slots, "state_slots")
         _i32(query_start_loc, "query_start_loc")
@@ -1289,23 +1303,32 @@ class Ops:
                  float(cap), _ptr(skip), float(scale))
         first = 0
         if plan is not None:
-            pieces, carries, n_pieces, first = plan
+            pieces, carries, n_pieces, first, *longest = plan
             _i32(pieces, "pieces")
             _i32(carries, "carries")
             _need(self.decaying_pieces_supported(dtype, state_dim, value_dim) and first <= num_seqs, "a geometry that is not cut into pieces")
             rounded = u if u.dim() == 2 else self.dense(u, dtype)
             held = value_dim + (1 if code == 2 else 0)
             piece_state = torch.empty((n_pieces, heads, held, state_dim), dtype=torch.float32, device=u.device)
-            piece_decay = torch.empty((n_pieces, heads, 2), dtype=torch.float32, device=u.device)
             piece_top = torch.empty((n_pieces, heads), dtype=torch.float32, device=u.device) if code == 2 else None
-            for mode in (0, 1):
+
+            def cut(mode: int, decays) -> None:
                 _check(self.core.ts_decaying_pieces(
-                    _ptr(y), _ptr(norm), _ptr(piece_state), _ptr(piece_decay), _ptr(piece_top), _ptr(rounded), *rows, *gates, _ptr(pieces),
+                    _ptr(y), _ptr(norm), _ptr(piece_state), _ptr(decays), _ptr(piece_top), _ptr(rounded), *rows, *gates, _ptr(pieces),
                     n_pieces, heads, groups, state_dim, value_dim, code, mode, self.stream()), "ts_decaying_pieces")
-                if mode == 0:
-                    _check(self.core.ts_decaying_carry(
-                        _ptr(state), _ptr(sums), _ptr(tops), _ptr(state_slots), _ptr(carries), _ptr(piece_state), _ptr(piece_decay),
-                        _ptr(piece_top), first, heads, state_dim, value_dim, code, self.stream()), "ts_decaying_carry")
+
+            if self._decaying_passes(n_pieces, first, longest[0] if longest else n_pieces - first + 1, heads, state_dim, held):
+                _check(self.core.ts_decaying_pass(
+                    _ptr(state), _ptr(sums), _ptr(tops), _ptr(state_slots), _ptr(carries), first, _ptr(pieces), _ptr(piece_state), _ptr(piece_top),
+                    _ptr(rounded), *rows, *gates[:9], heads, groups, state_dim, value_dim, code, self.stream()), "ts_decaying_pass")
+                cut(1, piece_state)  # (no decays there)
+            else:
+                piece_decay = torch.empty((n_pieces, heads, 2), dtype=torch.float32, device=u.device)
+                cut(0, piece_decay)
+                _check(self.core.ts_decaying_carry(
+                    _ptr(state), _ptr(sums), _ptr(tops), _ptr(state_slots), _ptr(carries), _ptr(piece_state), _ptr(piece_decay),
+                    _ptr(piece_top), first, heads, state_dim, value_dim, code, self.stream()), "ts_decaying_carry")
+                cut(1, piece_decay)
         _check(self.core.ts_decaying_walk(
             _ptr(y), _ptr(norm), _ptr(state), _ptr(sums), _ptr(tops), _ptr(u), 1 if u_f32 or dtype == torch.float32 else 0, u_splits, u_stride,
             *rows, *gates, _ptr(state_slots), _ptr(query_start_loc), first, num_seqs - first, heads, groups, state_dim, value_dim, code,
