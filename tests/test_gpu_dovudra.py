@@ -99,6 +99,29 @@ def test_activations_without_a_gate(ops, dtype, kind, inter):
     torch.testing.assert_close(got, want.to(dtype).float(), **tol)
 
 
+@pytest.mark.parametrize("rows,n,k,alone", [
+    (1, 8192, 256, True), (8, 8190, 512, True), (9, 8196, 64, True), (16, 4096, 72, True), (17, 8192, 256, False), (40, 20480, 512, False), (40, 37888, 128, True), (128, 65792, 64, True),
+    (129, 16384, 128, True), (300, 16400, 192, True), (700, 16384, 64, True), (2, 48, 64, False), (5, 100, 36, False), (8, 2048, 8192, False),
+])
+def test_a_product_that_squares_what_is_positive(ops, monkeypatch, rows, n, k, alone):
+    """max(x w, 0)^2 against 64 bits: one rounding to bfloat16 (2^-9 of its size, and half the smallest step) of the square of a 32-bit sum (k
+    roundings of 2^-24 of the terms' sizes).  Odd widths, few and many rows, whole rounds of tiles with a rest; where the product is one range no
+    launch follows it."""
+    g = torch.Generator().manual_seed(rows + n)
+    x, w = torch.randn(rows, k, generator=g).bfloat16().to(DEV), (torch.randn(n, k, generator=g) / 4).bfloat16().to(DEV)
+    calls = []
+    real = type(ops).activate
+    monkeypatch.setattr(type(ops), "activate", lambda self, *rest: calls.append(1) or real(self, *rest))
+    got = ops.linear_relu_squared(x, w)
+    assert got.dtype == torch.bfloat16 and got.shape == (rows, n) and (not alone or not calls)
+    z, size = (x.double() @ w.double().T).clamp(min=0.0), x.double().abs() @ w.double().abs().T
+    off = k * 2.0**-24 * size
+    room = 2.0**-8 * (z + off) ** 2 + 2 * z * off + off**2 + 1e-30
+    if calls:  # a product that is one bfloat16 result is rounded before it is squared, too
+        room = room + 2.0**-7 * (z + off) ** 2
+    assert bool(((got.double() - z * z).abs() <= room).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,vdim", [(3, 12), (1, 20), (8, 64), (5, 7)])
 def test_a_gate_per_head(ops, dtype, heads, vdim):

@@ -193,6 +193,12 @@ __device__ __forceinline__ float gated_unit(float g, float u, GluRule rule) {
   return (fabsf(x) <= GATE_NEAR ? gated_near(g, x) : gated_far(g, x)) * (u + rule.up_shift);
 }
 
+// max(z, 0)^2, the unit of a feed-forward without a gate.
+__device__ __forceinline__ float relu_squared(float z) {
+  const float r = fmaxf(z, 0.f);
+  return r * r;
+}
+
 // One rotation, written out so that every kernel rounds it the same way.
 __device__ __forceinline__ void rotate_pair(float x1, float x2, float c, float s, float& o1, float& o2) {
   o1 = __builtin_fmaf(x1, c, -(x2 * s));

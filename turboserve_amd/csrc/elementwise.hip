@@ -1043,10 +1043,7 @@ extern "C" int ts_copy_f32(float* out, const float* in, long total, hipStream_t 
 //   kind 3: the tanh form of GELU, 0.5 x (1 + tanh(sqrt(2 / pi) (x + 0.044715 x^3)))
 // ---------------------------------------------------------------------------------------------
 __device__ __forceinline__ float activation(float x, int kind) {
-  if (kind == 0) {
-    const float r = fmaxf(x, 0.f);
-    return r * r;
-  }
+  if (kind == 0) return relu_squared(x);
   if (kind == 1) return fmaxf(x, 0.f);
   if (kind == 2) return x / (1.f + expf(-x));
   return x / (1.f + expf(-1.5957691216057308f * fmaf(0.044715f * x * x, x, x)));

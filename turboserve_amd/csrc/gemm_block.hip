@@ -139,8 +139,8 @@ typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 // read has come through an asm behind the wait for its loads (ws, xs; a value the compiler cannot follow, so no read moves above
 // it, nor is one read taken for another), what is read of a slot is in registers that an asm before the wait takes (xf[1], wf)
 // or that matrix instructions pinned ahead of it have used (xf[0]), and every slot is filled again behind that wait.
-// out: bfloat16 [m, n] (mode 0), partial: float [splits, m, n] (mode 1), out: bfloat16 [m, n / 2] (mode 2: silu; 3: any rule
-// of the gated unit.  Two kernels: with both epilogues behind one loop the compiler moved the sums between registers in it).
+// out: bfloat16 [m, n] (mode 0; 4: of relu_squared's values), partial: float [splits, m, n] (mode 1), out: bfloat16 [m, n / 2] (mode 2: silu; 3: any rule
+// of the gated unit.  Kernels of their own: with several epilogues behind one loop the compiler moved the sums between registers in it).
 template <int TN, int TM, int MODE, bool ONCE>
 __device__ __forceinline__ void
 gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __restrict__ partial, uint16_t* __restrict__ out, const uint16_t* __restrict__ x, long x_stride,
@@ -361,7 +361,11 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   // 4 with these).  So every lane writes 16 bytes: the four lanes of a row hold four consecutive
   // columns of every tile, and exchange them until one holds eight of one of two tiles (gated: all of one of four).
   // Rows beyond M lie past the buffer's end, tiles beyond N are sent there.
-  constexpr int BYTES = MODE == 1 ? 4 : 2, PER = MODE >= 2 ? 2 : 1;  // of an output element; weight rows of one
+  constexpr bool WHOLE = MODE == 0 || MODE == 4, GATED = MODE == 2 || MODE == 3;
+  auto pack = [](float lo, float hi) __attribute__((always_inline)) {
+    return MODE == 4 ? block_pack(relu_squared(lo), relu_squared(hi)) : block_pack(lo, hi);
+  };
+  constexpr int BYTES = MODE == 1 ? 4 : 2, PER = GATED ? 2 : 1;  // of an output element; weight rows of one
   const int row_bytes = whole_n / PER * BYTES;
   char* base = MODE == 1 ? (char*)(partial + ((size_t)split * m + m_base) * whole_n) : (char*)out + (size_t)m_base * row_bytes;
   const __amdgpu_buffer_rsrc_t ybuf = block_buffer(base, (size_t)(min(m - m_base, XR) - 1) * row_bytes + n / PER * BYTES);
@@ -371,7 +375,7 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
   int row_at = (wave_m * TM * 16 + lane16) * row_bytes + (n_base / 16 + wave_n * TN) * tile_bytes;
 #pragma unroll
   for (int b = 0; b < TM; ++b, row_at += 16 * row_bytes) {
-    constexpr int SHARE = MODE == 0 ? 2 : MODE >= 2 ? 4 : 1;  // tiles exchanged; what TN leaves over is stored tile by tile
+    constexpr int SHARE = WHOLE ? 2 : GATED ? 4 : 1;  // tiles exchanged; what TN leaves over is stored tile by tile
 #pragma unroll
     for (int c = 0; c < TN / SHARE; ++c) {
       const int a = c * SHARE;
@@ -379,12 +383,12 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
       u32x4 v;
       if (MODE == 1) {
         v = __builtin_bit_cast(u32x4, acc[a][b]);
-      } else if (MODE == 0) {
+      } else if (WHOLE) {
         mine += group & 1;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const u32x2 both = block_swap16(block_pack(acc[a][b][2 * h], acc[a][b][2 * h + 1]),
-                                          block_pack(acc[a + SHARE - 1][b][2 * h], acc[a + SHARE - 1][b][2 * h + 1]));
+          const u32x2 both = block_swap16(pack(acc[a][b][2 * h], acc[a][b][2 * h + 1]),
+                                          pack(acc[a + SHARE - 1][b][2 * h], acc[a + SHARE - 1][b][2 * h + 1]));
           v[h] = both[0];
           v[2 + h] = both[1];
         }
@@ -397,14 +401,14 @@ gemm_block(lds_u16* __restrict__ to, const lds_u16* __restrict__ from, float* __
         const u32x2 low = block_swap16(even[0], odd[0]), high = block_swap16(even[1], odd[1]);
         v = u32x4{low[0], low[1], high[0], high[1]};
       }
-      const int at = row_at + mine * tile_bytes + (MODE == 1 ? 16 * group : MODE == 0 ? 8 * (group & 2) : 0);
+      const int at = row_at + mine * tile_bytes + (MODE == 1 ? 16 * group : WHOLE ? 8 * (group & 2) : 0);
       __builtin_amdgcn_raw_buffer_store_b128(v, ybuf, mine < tiles ? at : OUTSIDE, 0, 0);
     }
 #pragma unroll
     for (int a = TN / SHARE * SHARE; a < TN; ++a) {
       const int at = a < tiles ? row_at + a * tile_bytes + tile_bytes / 4 * group : OUTSIDE;
-      if (MODE == 0) {
-        __builtin_amdgcn_raw_buffer_store_b64(u32x2{block_pack(acc[a][b][0], acc[a][b][1]), block_pack(acc[a][b][2], acc[a][b][3])}, ybuf, at, 0, 0);
+      if (WHOLE) {
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack(acc[a][b][0], acc[a][b][1]), pack(acc[a][b][2], acc[a][b][3])}, ybuf, at, 0, 0);
       } else {
         const f32x4 one[1] = {acc[a][b]};
         uint32_t u[1];
@@ -451,7 +455,7 @@ int launch_block_kernel(float* partial, uint16_t* out, const uint16_t* x, long x
 
 // x [m, k] bfloat16 with row stride x_stride; w [n, k] bfloat16 contiguous; bias [n] bfloat16 or null; k a multiple of 64, n of 16.  mode
 // 0: out = bfloat16 [m, n] (splits must be 1); mode 1: partial = float [splits, m, n]; mode 2: out = bfloat16 [m, n / 2] =
-// the gated unit (common.hpp) of a w whose rows alternate gate, up (splits 1).  iters_per_split iterations of 64 of k go to
+// the gated unit (common.hpp) of a w whose rows alternate gate, up (splits 1); mode 3: out = bfloat16 [m, n] = relu_squared (splits 1).  iters_per_split iterations of 64 of k go to
 // each of `splits` = ceil(k / 64 / iters_per_split) ranges.  tn, tm: 32 tn weight rows by 32 tm activation rows a
 // workgroup.  w, bias and out may be a run of weight rows of a larger product: whole_n is its n, the length of out's rows
 // (out points at the run's first column).
@@ -459,7 +463,7 @@ extern "C" int ts_gemm_block(float* partial, void* out, const void* x, long x_st
                              int m, int n, int k, int iters_per_split, int splits, int tn, int tm, int mode, int whole_n,
                              float steepness, float limit, float up_shift, float cubic, hipStream_t stream) {
   if (m == 0 || n == 0) return TS_OK;
-  if (!x || !w || m < 0 || n < 0 || k < 1 || mode < 0 || mode > 2) return TS_ERR_ARG;
+  if (!x || !w || m < 0 || n < 0 || k < 1 || mode < 0 || mode > 3) return TS_ERR_ARG;
   if ((mode == 1) != (partial != nullptr) || (mode != 1) != (out != nullptr)) return TS_ERR_ARG;
   if (k % BLOCK_DEPTH != 0 || n % 16 != 0 || x_stride < k || x_stride % 8 != 0 || (uintptr_t)x % 16 != 0 || (uintptr_t)w % 16 != 0)
     return TS_ERR_SHAPE;
@@ -479,6 +483,7 @@ extern "C" int ts_gemm_block(float* partial, void* out, const void* x, long x_st
   if (tn == TN && tm == TM && once == ONCE) {        \
     if (mode == 0) TS_BLOCK_MODE(TN, TM, 0, ONCE);   \
     if (mode == 1) TS_BLOCK_MODE(TN, TM, 1, ONCE);   \
+    if (mode == 3) TS_BLOCK_MODE(TN, TM, 4, ONCE);   \
     if (plain) TS_BLOCK_MODE(TN, TM, 2, ONCE);       \
     TS_BLOCK_MODE(TN, TM, 3, ONCE);                  \
   }

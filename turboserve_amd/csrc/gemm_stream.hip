@@ -189,7 +189,8 @@ __device__ __forceinline__ void stream_range(lds_u16* __restrict__ to, const lds
 
 // What a workgroup does with its wavefronts' sums: the quarters meet in the rings; wavefront v adds up and stores tile v, `shift` its bias.
 // (`wave` comes from the caller: asked for again here, with a wait behind the last product, a decode step of 28 products took 495.5 us for 492.7.)
-template <int NT, int XT, bool GATED>
+// UNIT: what is stored of the sums: 0 they themselves, 32-bit, 1 the gated unit, 2 relu_squared, bfloat16.
+template <int NT, int XT, int UNIT>
 __device__ __forceinline__ void stream_finish(lds_u16* ring, int wave, const f32x4* acc, const uint32_t (&shift)[4], bool shifted, int m, int n, int col, int split,
                                               float* __restrict__ partial, uint16_t* __restrict__ out, GluRule rule) {
   typedef Ring<NT, XT> R;
@@ -207,7 +208,17 @@ __device__ __forceinline__ void stream_finish(lds_u16* ring, int wave, const f32
 #pragma unroll
     for (int i = 0; i < 4; ++i) sum[i] += __uint_as_float(shift[i] << 16);
   }
-  if (GATED) {  // n is even: the first pair lies inside
+  if (UNIT == 2) {
+    uint16_t* at = out + (size_t)row * n + col;
+    if (n % 4 == 0) {
+      *reinterpret_cast<u32x2*>(at) = u32x2{from_float<bf16_t>(relu_squared(sum[0])).bits | (uint32_t)from_float<bf16_t>(relu_squared(sum[1])).bits << 16,
+                                            from_float<bf16_t>(relu_squared(sum[2])).bits | (uint32_t)from_float<bf16_t>(relu_squared(sum[3])).bits << 16};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (col + i < n) at[i] = from_float<bf16_t>(relu_squared(sum[i])).bits;
+    }
+  } else if (UNIT == 1) {  // n is even: the first pair lies inside
     uint16_t* at = out + (size_t)row * (n / 2) + col / 2;
     at[0] = from_float<bf16_t>(gated_unit(sum[0], sum[1], rule)).bits;
     if (col + 2 < n) at[1] = from_float<bf16_t>(gated_unit(sum[2], sum[3], rule)).bits;
@@ -223,8 +234,8 @@ __device__ __forceinline__ void stream_finish(lds_u16* ring, int wave, const f32
   }
 }
 
-// partial: float [splits, m, n], or, GATED, out: bfloat16 [m, n / 2], the gated unit (common.hpp) of rows that alternate gate, up.
-template <int NT, int XT, bool GATED>
+// partial: float [splits, m, n], or out: bfloat16 [m, n / 2], the gated unit (common.hpp) of rows that alternate gate, up, or [m, n], relu_squared.
+template <int NT, int XT, int UNIT>
 __global__ void __launch_bounds__(64 * STREAM_WAVES)
 gemm_stream_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias, int x_stride, int m,
                    int n, int k, int per_wave, float* __restrict__ partial, uint16_t* __restrict__ out, GluRule rule) {
@@ -247,20 +258,20 @@ gemm_stream_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
   }
   lds_u16* mine = (lds_u16*)ring + wave * R::WAVE;
   stream_range<NT, XT, 0>(mine, mine, mine, x, w, m, n, k, x_stride, n0, first, last, acc, [] {});
-  stream_finish<NT, XT, GATED>((lds_u16*)ring, wave, acc, shift, bias && split == 0, m, n, col, split, partial, out, rule);
+  stream_finish<NT, XT, UNIT>((lds_u16*)ring, wave, acc, shift, bias && split == 0, m, n, col, split, partial, out, rule);
 }
 
-template <int NT, int XT, bool GATED>
+template <int NT, int XT, int UNIT>
 int launch_stream(float* partial, void* out, const void* x, long x_stride, const void* w, const void* bias, int m, int n, int k,
                   int per_wave, int splits, GluRule rule, hipStream_t stream) {
   constexpr size_t BYTES = Ring<NT, XT>::BYTES;
   static bool raised = false;  // per process; the attribute belongs to the kernel
   if (!raised) {
-    if (hipFuncSetAttribute((const void*)gemm_stream_kernel<NT, XT, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)BYTES) != hipSuccess)
+    if (hipFuncSetAttribute((const void*)gemm_stream_kernel<NT, XT, UNIT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)BYTES) != hipSuccess)
       return TS_ERR_LAUNCH;
     raised = true;
   }
-  hipLaunchKernelGGL((gemm_stream_kernel<NT, XT, GATED>), dim3((n + 16 * NT - 1) / (16 * NT), splits), dim3(64 * STREAM_WAVES),
+  hipLaunchKernelGGL((gemm_stream_kernel<NT, XT, UNIT>), dim3((n + 16 * NT - 1) / (16 * NT), splits), dim3(64 * STREAM_WAVES),
                      BYTES, stream, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (int)x_stride, m, n, k, per_wave,
                      partial, (uint16_t*)out, rule);
   return ts_launch_status();
@@ -378,7 +389,7 @@ gemm_stream_normed_kernel(const float* __restrict__ residual, const float* __res
   const int total = k / R::SLICE, first = (split * STREAM_WAVES + wave) * per_wave, last = min(first + per_wave, total);
   lds_u16* mine = (lds_u16*)ring + wave * R::WAVE;
   stream_range<NT, 0, ROWS>(mine, mine, (const lds_u16*)held, nullptr, w, ROWS, n, k, 0, n0, first, last, acc, normalise);
-  stream_finish<NT, 0, GATED>((lds_u16*)ring, wave, acc, shift, bias && split == 0, ROWS, n, col, split, partial, out, rule);
+  stream_finish<NT, 0, GATED ? 1 : 0>((lds_u16*)ring, wave, acc, shift, bias && split == 0, ROWS, n, col, split, partial, out, rule);
 }
 
 template <int ROWS, int ITEMS, int SUMS, bool GATED>
@@ -472,7 +483,7 @@ gemm_stream_heads_kernel(const float* __restrict__ partial_acc, const float* __r
   const int total = k / R::SLICE, first = (split * STREAM_WAVES + wave) * per_wave, last = min(first + per_wave, total);
   lds_u16* mine = (lds_u16*)ring + wave * R::WAVE;
   stream_range<NT, 0, 1>(mine, mine, (const lds_u16*)held, nullptr, w, 1, n, k, 0, n0, first, last, acc, combine);
-  stream_finish<NT, 0, false>((lds_u16*)ring, wave, acc, shift, bias && split == 0, 1, n, col, split, partial, nullptr, GluRule{1.f, 0.f, 0.f, 0.f});
+  stream_finish<NT, 0, 0>((lds_u16*)ring, wave, acc, shift, bias && split == 0, 1, n, col, split, partial, nullptr, GluRule{1.f, 0.f, 0.f, 0.f});
 }
 
 template <int ITEMS, int PARTS>
@@ -494,10 +505,10 @@ int launch_stream_heads(float* partial, const float* partial_acc, const float* p
 
 // x [m, k] bfloat16 (m up to 16, k a multiple of 8) with row stride x_stride; w [n, k] bfloat16 contiguous; bias [n] bfloat16 or
 // null.  partial = float [splits, m, n], or out = bfloat16 [m, n / 2] (splits 1, n even): the gated unit of a w whose rows
-// alternate gate, up.  Slices of 64 of k: per_wave to each of the four wavefronts of each of `splits` =
+// alternate gate, up, or, `squared`, bfloat16 [m, n]: relu_squared (splits 1; n even or odd).  Slices of 64 of k: per_wave to each of the four wavefronts of each of `splits` =
 // ceil(ceil(k / 64) / (4 per_wave)) ranges.  tile: 1 or 2 (16 or 32 weight rows a workgroup).
 extern "C" int ts_gemm_stream(float* partial, void* out, const void* x, long x_stride, const void* w, const void* bias, int m,
-                              int n, int k, int per_wave, int splits, int tile, float steepness, float limit, float up_shift,
+                              int n, int k, int per_wave, int splits, int tile, int squared, float steepness, float limit, float up_shift,
                               float cubic, hipStream_t stream) {
   if (m == 0 || n == 0) return TS_OK;
   if (!x || !w || m < 0 || n < 0 || k < 8 || (partial == nullptr) == (out == nullptr)) return TS_ERR_ARG;
@@ -505,19 +516,21 @@ extern "C" int ts_gemm_stream(float* partial, void* out, const void* x, long x_s
   if (x_stride >= (1L << 24) || k >= (1 << 24)) return TS_ERR_SHAPE;  // a tile's rows lie within 31 bits of its first one
   if (per_wave < 1 || splits < 1 || splits > 65535) return TS_ERR_SHAPE;
   if (splits != ((k + 63) / 64 + 4L * per_wave - 1) / (4L * per_wave)) return TS_ERR_SHAPE;
-  if (out && (splits != 1 || n % 2 != 0)) return TS_ERR_ARG;
+  if (out && (splits != 1 || (!squared && n % 2 != 0))) return TS_ERR_ARG;
   const GluRule rule = {steepness, limit, up_shift, cubic};
   // Up to eight rows are one load a slice instead of two, and leave room for a slice more in the ring.
-#define TS_STREAM(NT, GATED)                                                                                                                  \
-  return m <= 8 ? launch_stream<NT, 1, GATED>(partial, out, x, x_stride, w, bias, m, n, k, per_wave, splits, rule, stream)                   \
-                : launch_stream<NT, 2, GATED>(partial, out, x, x_stride, w, bias, m, n, k, per_wave, splits, rule, stream)
+#define TS_STREAM(NT, UNIT)                                                                                                                   \
+  return m <= 8 ? launch_stream<NT, 1, UNIT>(partial, out, x, x_stride, w, bias, m, n, k, per_wave, splits, rule, stream)                   \
+                : launch_stream<NT, 2, UNIT>(partial, out, x, x_stride, w, bias, m, n, k, per_wave, splits, rule, stream)
   if (tile == 1) {
-    if (out) TS_STREAM(1, true);
-    TS_STREAM(1, false);
+    if (out && squared) TS_STREAM(1, 2);
+    if (out) TS_STREAM(1, 1);
+    TS_STREAM(1, 0);
   }
   if (tile == 2) {
-    if (out) TS_STREAM(2, true);
-    TS_STREAM(2, false);
+    if (out && squared) TS_STREAM(2, 2);
+    if (out) TS_STREAM(2, 1);
+    TS_STREAM(2, 0);
   }
 #undef TS_STREAM
   return TS_ERR_SHAPE;

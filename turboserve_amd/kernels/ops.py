@@ -152,7 +152,7 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "ts_gemm_stream_heads": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
         "ts_gemm_stream_normed": [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_float, c_float, c_int, c_void_p, c_void_p,
                                   c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_float, c_void_p],
-        "ts_gemm_stream": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
+        "ts_gemm_stream": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                            c_float, c_float, c_float, c_float, c_void_p],
         "ts_gemm_skinny_resident": [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
                                     c_int, c_int, c_int, c_void_p],
@@ -2504,7 +2504,7 @@ class Ops:
         return self._block_product(x, weight, bias, plan=plan, gated=gated, sums=sums, rule=rule)
 
     def _block_product(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, *, plan: tuple[int, ...],
-                       gated: bool, sums: bool, rule: tuple[float, float, float]) -> torch.Tensor:
+                       gated: bool, sums: bool, rule: tuple[float, float, float], squared: bool = False) -> torch.Tensor:
         """:meth:`gemm_block` of operands on the GPU that ``block_supported`` has been asked about: the choice of
         a kernel asks it anyway, and a prompt of a small model is bound by the host (8 layers 2,048 wide, 33 to 256
         tokens: asked twice and the choice worked out for every product, a step took 1,070 to 1,275 us, now 970 to 1,170)."""
@@ -2514,14 +2514,14 @@ class Ops:
             _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.data_ptr() % 8 == 0,
                   "bias must be bfloat16 [N]")
         per_split, splits, tn, tm = plan[:4]
-        _need(not gated or splits == 1, "the gated result needs one range of K")
+        _need(not (gated or squared) or splits == 1, "a unit needs one range of K")
         partial = out = None
-        if gated or (splits == 1 and not sums):
+        if gated or squared or (splits == 1 and not sums):
             out = self.rows_buffer(m, n // 2 if gated else n, torch.bfloat16, x.device)
         else:
             partial = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
         unit = glu_rule(rule) if gated else (1.0, 0.0, 0.0, 0.0)
-        mode = 2 if gated else 1 if out is None else 0
+        mode = 2 if gated else 3 if squared else 1 if out is None else 0
         rows = n
         sums_at, at, weight_at, bias_at = _ptr(partial), _ptr(out), weight.data_ptr(), _ptr(bias)
         if len(plan) > 4:  # whole rounds first, the rest of the weight rows in other tiles
@@ -2774,11 +2774,11 @@ class Ops:
     stream_max_rows = 16
 
     def gemm_stream(self, x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None, *, plan: tuple[int, int, int],
-                    gated: bool = False, rule: tuple[float, float, float] = (1.0, 0.0, 0.0)) -> torch.Tensor:
+                    gated: bool = False, rule: tuple[float, float, float] = (1.0, 0.0, 0.0), squared: bool = False) -> torch.Tensor:
         """``[S, M, N]`` 32-bit partial sums of ``x [M, K] @ weight [N, K]^T`` over ``S`` ranges of
         K (bias in the first) by the kernel that streams whole lines of the weights through LDS
         (``csrc/gemm_stream.hip``): M up to 16, K a multiple of 8.  ``plan`` as
-        :meth:`_stream_plan` gives it; ``gated`` as :meth:`gemm_tiled`'s."""
+        :meth:`_stream_plan` gives it; ``gated`` as :meth:`gemm_tiled`'s; ``squared``: ``max(y, 0)^2`` of the one range, bfloat16 ``[M, N]``."""
         _gpu(x, weight, bias)
         _need(x.dim() == 2 and x.stride(1) == 1 and weight.dim() == 2 and weight.is_contiguous()
               and x.shape[1] == weight.shape[1], "x must be [M, K] with unit inner stride, weight contiguous [N, K]")
@@ -2793,11 +2793,14 @@ class Ops:
         if gated:
             _need(splits == 1 and n % 2 == 0, "the gated result needs one range of K and an even number of weight rows")
             out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
+        elif squared:
+            _need(splits == 1, "the unit needs one range of K")
+            out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
         else:
             partial = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
         _check(self.core.ts_gemm_stream(_ptr(partial), _ptr(out), _ptr(x), x_stride, _ptr(weight), _ptr(bias), m, n, k, per_wave,
-                                        splits, tile, *glu_rule(rule), self.stream()), "ts_gemm_stream")
-        return out if gated else partial
+                                        splits, tile, 1 if squared else 0, *glu_rule(rule), self.stream()), "ts_gemm_stream")
+        return partial if out is None else out
 
     #: Rows up to which a product makes the norm that it reads (``csrc/gemm_stream.hip``).
     normed_max_rows = 2
@@ -3189,6 +3192,30 @@ class Ops:
                 out += bias
             return out.unsqueeze(0)
         return self._library_product(x, weight, bias, None)
+
+    def linear_relu_squared(self, x: torch.Tensor | WaitingNorm, weight: torch.Tensor) -> torch.Tensor:
+        """``max(x @ weight^T, 0)^2`` in the dtype of ``x``: :meth:`linear` and :meth:`activate`, in one launch where the product is one range of
+        K of the streaming or the block kernel, which then square its 32-bit sums and round once (us, 8,192 x 2,048 with 2,000 / 300 / 8 rows, product
+        and activation / one launch: 67.4 / 54.6, 22.6 / 19.3, 9.4 / 7.3)."""
+        if not isinstance(x, WaitingNorm) and x.dtype == torch.bfloat16 and x.dim() == 2:
+            rule, (n, k) = (1.0, 0.0, 0.0), weight.shape
+            if x.shape[0] <= self.skinny_max_rows:
+                if self.skinny_supported(x, weight):
+                    _gpu(x, weight)
+                    block = self._block_few_runs(x, weight, None, None)
+                    if block is not None and block[1] == 1:
+                        return self._block_product(x, weight, None, plan=block, gated=False, sums=False, rule=rule, squared=True)
+                    stream = self._stream_runs(x, weight, None) if block is None else None
+                    if stream is not None and stream[1] == 1:
+                        return self.gemm_stream(x, weight, plan=stream, squared=True)
+            elif self.skinny_supported_any_rows(x, weight):
+                _gpu(x, weight)
+                m = x.shape[0]
+                block, plan, _, untimed = self._own_choice(m, n, k, "one", self.block_supported(x, weight))
+                if block and self._wide_runs(m, n, k, "one", untimed, self._own_product(x, weight, None, "one")[0],
+                                             lambda: self._library_product(x, weight, None, None)):
+                    return self._block_product(x, weight, None, plan=plan, gated=False, sums=False, rule=rule, squared=True)
+        return self.activate(self.linear(x, weight), "relu_squared", x.dtype)
 
     def linear_float32_out(self, x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         """``x @ weight^T`` with a 32-bit result (the head: logits are 32-bit,

@@ -108,5 +108,8 @@ class ActivatedMLP(FeedForward):
 
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         ops = self.runtime.ops
-        hidden = ops.activate(ops.linear(x, self.up_weight), self.activation, x.dtype)
+        if self.activation == "relu_squared":
+            hidden = ops.linear_relu_squared(x, self.up_weight)
+        else:
+            hidden = ops.activate(ops.linear(x, self.up_weight), self.activation, x.dtype)
         return ops.linear(hidden, self.down_weight, for_residual=True)
