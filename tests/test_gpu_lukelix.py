@@ -734,3 +734,36 @@ def test_a_steps_short_kernels_have_the_bits_of_the_general_ones(ops, dtype, spl
     y, gain = torch.randn(tokens, channels, generator=g).to(DEV), torch.randn(channels, generator=g).to(dtype).to(DEV)
     short, general = (ops.gated_group_norm(y, parts_of, 4, gain, 1e-5, parts, dtype) for parts_of in (some, more))
     assert torch.equal(short, general)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,groups,n,p,parts", [(64, 8, 128, 64, 8), (6, 3, 32, 12, 2), (4, 1, 64, 36, 1), (8, 8, 100, 128, 2), (3, 3, 4, 4, 3)])
+@pytest.mark.parametrize("tokens,splits,bias", [(1, 2, True), (8, 1, False), (5, 3, True), (7, 8, True)])
+def test_a_token_from_its_projection_on_in_two_launches(ops, dtype, heads, groups, n, p, parts, tokens, splits, bias):
+    """Convolution, walk and gated norm in two launches: the bits of the three, in the rows and in both states, whose slots are not in row order;
+    columns that fill no workgroup, rows that fill no tile, as many partial sums as there may be."""
+    g = torch.Generator().manual_seed(heads + n + tokens)
+    inner, channels = heads * p, heads * p + 2 * groups * n
+    width = inner + channels + heads + -heads % 4 + 4
+    width += -width % 4
+    proj = torch.randn(splits, tokens, width, generator=g).to(DEV)
+    taps, add = (0.5 * torch.randn(channels, 4, generator=g)).to(dtype).to(DEV), torch.randn(channels, generator=g).to(dtype).to(DEV) if bias else None
+    one, two, skip = (torch.rand(heads, generator=g).to(DEV) for _ in range(3))
+    gain = torch.randn(inner, generator=g).to(dtype).to(DEV)
+    slots, starts = ints([2 * (tokens - i) for i in range(tokens)]), ints(list(range(tokens + 1)))
+    results = []
+    for launches in (2, 3):
+        fresh = torch.Generator().manual_seed(n)
+        held, state = torch.randn(2 * tokens + 1, 3, channels, generator=fresh).to(DEV), torch.randn(2 * tokens + 1, heads, p, n, generator=fresh).to(DEV)
+        if launches == 2:
+            out = ops.selective_token(proj, inner, taps, add, held, inner + channels, one - 4.0, two, skip, state, slots, heads=heads, groups=groups,
+                                      state_dim=n, value_dim=p, z_at=0, gain=gain, eps=1e-6, parts=parts, dtype=dtype)
+            assert out is not None
+        else:
+            u = ops.short_conv(proj, inner, taps, held, slots, starts[:-1], starts, tokens=tokens, num_seqs=tokens, dtype=dtype, silu=True, bias=add)
+            y = ops.selective_state(u, proj, inner + channels, one - 4.0, two, skip, state, slots, starts, num_seqs=tokens, heads=heads, groups=groups,
+                                    state_dim=n, value_dim=p, dtype=dtype)
+            out = ops.gated_group_norm(y, proj, 0, gain, 1e-6, parts, dtype)
+        results.append((out, held, state))
+    for got, want in zip(*results):
+        assert bool(want.isfinite().all()) and torch.equal(got, want)

@@ -291,6 +291,121 @@ decaying_walk_kernel(float* __restrict__ state, const int* __restrict__ state_sl
 }
 
 // ---------------------------------------------------------------------------------------------
+// a step of single tokens with the convolution in front
+// ---------------------------------------------------------------------------------------------
+
+// The selective walk of one token a request whose x, B and C are a convolution of four taps over columns of the projection, with a bias or
+// without, through silu, rounded to T (short_conv.hip: `held` [slots, 3, channels], oldest first; the same bits): every workgroup convolves the
+// channels that it reads, 288 of them at 128 rows, while its part of the state travels, and a launch of 4 us between two that wait for it falls
+// away.  A channel of x belongs to one workgroup, which moves it on in `held`; those of B and C, which all heads of a group read, are
+// moved on by the launch behind this one (gated_group_norm_few_kernel).  proj: `splits` 32-bit partial sums, at most BATCH.
+struct SsConv {
+  const void* taps;  // [channels, 4] of T: x of every head, B of every group, C
+  const void* bias;  // [channels] of T, or null
+  int first;         // their first column of the projection
+  int silu;
+};
+
+template <typename T, int NR, int BATCH>
+__global__ void __launch_bounds__(256)
+selective_token_kernel(float* __restrict__ state, const int* __restrict__ state_slots, const float* __restrict__ proj, float* __restrict__ held, int width,
+                       int heads, int groups, int n, int p, int splits, size_t stride, SsConv conv, int dt_at, const float* __restrict__ dt_bias,
+                       const float* __restrict__ a_log, const float* __restrict__ skip, float* __restrict__ y) {
+  constexpr int THREADS = 256, COLS = THREADS / SS_PARTS, ROWS = SS_PARTS * NR, ITEMS = 2 * ROWS + COLS, ROUNDS = (ITEMS + THREADS - 1) / THREADS;
+  __shared__ __attribute__((aligned(16))) float us[ITEMS];  // B, C, x
+  __shared__ float weight, decay;
+  const int t = blockIdx.x, h = blockIdx.y, g = h / (heads / groups);
+  const int tid = threadIdx.x, part = tid % SS_PARTS, col_in = tid / SS_PARTS;
+  const int c0 = blockIdx.z * COLS, c = c0 + col_in;
+  const bool live = c < p;
+  const int channels = heads * p + 2 * groups * n;
+  const int slot = state_slots[t];
+  float* const own = state + (((size_t)slot * heads + h) * p + (live ? c : 0)) * n;
+  float* const kept = held + (size_t)slot * 3 * channels;
+  const float* const row = proj + (size_t)t * width;
+  // Everything is asked for at once, unconditionally (rows past N, columns past P: others', dropped below).
+  float s[NR];
+#pragma unroll
+  for (int x = 0; x < NR / 4; ++x) {
+    const int d = x * 4 * SS_PARTS + part * 4;
+    const float4 v = *reinterpret_cast<const float4*>(own + (d < n ? d : 0));
+    s[4 * x] = v.x; s[4 * x + 1] = v.y; s[4 * x + 2] = v.z; s[4 * x + 3] = v.w;
+  }
+  float in[ROUNDS][BATCH], old[ROUNDS][3];
+  T taps[ROUNDS][4], add[ROUNDS];
+  int channel[ROUNDS];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int i = tid + THREADS * r;
+    if (i >= ITEMS) break;
+    const int d = i < 2 * ROWS ? i % ROWS : 0;
+    channel[r] = i >= 2 * ROWS ? h * p + min(c0 + i - 2 * ROWS, p - 1) : heads * p + ((i < ROWS ? 0 : groups) + g) * n + min(d, n - 1);
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) in[r][j] = row[(size_t)min(j, splits - 1) * stride + conv.first + channel[r]];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) old[r][j] = kept[(size_t)j * channels + channel[r]];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) taps[r][j] = ((const T*)conv.taps)[(size_t)channel[r] * 4 + j];
+    if (conv.bias) add[r] = ((const T*)conv.bias)[channel[r]];
+  }
+  const float d_skip = skip[h];
+  if (tid == 2 * TS_WAVE) {  // (a wavefront that convolves no x)
+    const float one = dt_bias[h], two = a_log[h];
+    const float dt = ss_softplus(ss_input(row + dt_at + h, splits, stride) + one);
+    weight = dt;
+    decay = expf(-expf(two) * dt);
+  }
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int i = tid + THREADS * r;
+    if (i >= ITEMS) break;
+    float mine = splits == 1 ? in[r][0] : 0.f + in[r][0];
+#pragma unroll
+    for (int j = 1; j < BATCH; ++j) mine = j < splits ? mine + in[r][j] : mine;
+    float v = 0.f;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) v = fmaf(to_float(taps[r][j]), old[r][j], v);
+    v = fmaf(to_float(taps[r][3]), mine, v);
+    if (conv.bias) v += to_float(add[r]);
+    if (conv.silu) v = v / (1.f + expf(-v));
+    us[i] = i < 2 * ROWS && i % ROWS >= n ? 0.f : to_float(from_float<T>(v));
+    if (i >= 2 * ROWS && c0 + i - 2 * ROWS < p) {
+      kept[channel[r]] = old[r][1];
+      kept[(size_t)channels + channel[r]] = old[r][2];
+      kept[(size_t)2 * channels + channel[r]] = mine;
+    }
+  }
+  if (n < ROWS) {
+#pragma unroll
+    for (int e = 0; e < NR; ++e) s[e] = e / 4 * 4 * SS_PARTS + part * 4 + e % 4 < n ? s[e] : 0.f;
+  }
+  __syncthreads();
+  const float a = decay, xv = us[2 * ROWS + col_in], dx = weight * xv;
+  float r[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int x = 0; x < NR / 4; ++x) {
+    const float4 b4 = *reinterpret_cast<const float4*>(&us[x * 4 * SS_PARTS + part * 4]);
+    const float4 c4 = *reinterpret_cast<const float4*>(&us[ROWS + x * 4 * SS_PARTS + part * 4]);
+    const int i = 4 * x;
+    s[i] = fmaf(a, s[i], b4.x * dx); s[i + 1] = fmaf(a, s[i + 1], b4.y * dx);
+    s[i + 2] = fmaf(a, s[i + 2], b4.z * dx); s[i + 3] = fmaf(a, s[i + 3], b4.w * dx);
+    r[0] = fmaf(s[i], c4.x, r[0]); r[1] = fmaf(s[i + 1], c4.y, r[1]);
+    r[2] = fmaf(s[i + 2], c4.z, r[2]); r[3] = fmaf(s[i + 3], c4.w, r[3]);
+  }
+  float sum = (r[0] + r[1]) + (r[2] + r[3]);
+  sum += lanes_moved<0xB1, 0xF>(0.f, sum);
+  sum += lanes_moved<0x4E, 0xF>(0.f, sum);
+  sum += lanes_moved<0x141, 0xF>(0.f, sum);
+  if (!live) return;
+  if (part == 0) y[((size_t)t * heads + h) * p + c] = fmaf(d_skip, xv, sum);
+#pragma unroll
+  for (int x = 0; x < NR / 4; ++x) {
+    const int d = x * 4 * SS_PARTS + part * 4;
+    if (d < n) *reinterpret_cast<float4*>(own + d) = make_float4(s[4 * x], s[4 * x + 1], s[4 * x + 2], s[4 * x + 3]);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // pieces side by side on the matrix cores
 // ---------------------------------------------------------------------------------------------
 
@@ -1212,12 +1327,39 @@ gated_group_norm_kernel(T* __restrict__ out, const float* __restrict__ y, const 
 
 // The same bits for a step of few parts of up to 1,024 elements, at most BATCH partial sums: everything a part needs is asked for at once,
 // and the code is short and straight (other kernels of a recorded step have put it out of the instruction cache).
-template <typename T, typename P, int THREADS, int BATCH>
+// MOVES: the workgroups behind the parts' move the channels on that selective_token_kernel, the launch before, has left as they were:
+// `moved` of them from `from` on, of `channels`.
+struct SsMoves {
+  float* held;  // [slots, 3, channels]
+  const int* state_slots;
+  int channels;
+  int from;
+  int moved;
+  int first;    // the channels' first column of the projection
+};
+template <typename T, typename P, int THREADS, int BATCH, bool MOVES = false>
 __global__ void __launch_bounds__(THREADS)
 gated_group_norm_few_kernel(const P* proj, const float* y, const T* gain, T* out, int splits, int width, size_t split_stride, int z_at,
-                            int parts, int size, float eps) {
+                            int parts, int size, float eps, SsMoves moves) {
   __shared__ __attribute__((aligned(16))) float scratch[(THREADS / TS_WAVE + 3) / 4 * 4];
   const int t = blockIdx.x, part = blockIdx.y;
+  if (MOVES && part >= parts) {
+    const int i = (part - parts) * THREADS + threadIdx.x, channel = moves.from + min(i, moves.moved - 1);
+    const P* in = proj + (size_t)t * width + moves.first + channel;
+    float* kept = moves.held + (size_t)moves.state_slots[t] * 3 * moves.channels + channel;
+    float v[BATCH];
+#pragma unroll
+    for (int j = 0; j < BATCH; ++j) v[j] = to_float(in[(size_t)min(j, splits - 1) * split_stride]);
+    const float one = kept[moves.channels], two = kept[(size_t)2 * moves.channels];
+    float mine = splits == 1 ? v[0] : 0.f + v[0];
+#pragma unroll
+    for (int j = 1; j < BATCH; ++j) mine = j < splits ? mine + v[j] : mine;
+    if (i >= moves.moved) return;
+    kept[0] = one;
+    kept[moves.channels] = two;
+    kept[(size_t)2 * moves.channels] = mine;
+    return;
+  }
   const size_t row = ((size_t)t * parts + part) * size;
   const bool in = 4 * (int)threadIdx.x < size;
   const int i = min(4 * (int)threadIdx.x, size - 4);
@@ -1565,7 +1707,7 @@ static int launch_gated_group_norm(void* out, const float* y, const void* proj, 
     if (few && pieces <= 256 && splits <= 8) {
 #define GN_FEW(THREADS, BATCH)                                                                                                      \
   hipLaunchKernelGGL((gated_group_norm_few_kernel<T, P, THREADS, BATCH>), dim3(tokens, parts), dim3(THREADS), 0, stream,            \
-                     (const P*)proj, y, (const T*)gain, (T*)out, splits, width, (size_t)split_stride, z_at, parts, size, eps)
+                     (const P*)proj, y, (const T*)gain, (T*)out, splits, width, (size_t)split_stride, z_at, parts, size, eps, SsMoves{})
 #define GN_BATCH(THREADS)                     \
   do {                                        \
     if (splits == 1) GN_FEW(THREADS, 1);      \
@@ -1604,5 +1746,72 @@ extern "C" int ts_gated_group_norm(void* out, const float* y, const void* proj, 
     return launch_gated_group_norm<bf16_t, float>(out, y, proj, splits, split_stride, width, z_at, gain, eps, tokens, parts, size, stream);
   if (dtype == TS_BF16)
     return launch_gated_group_norm<bf16_t, bf16_t>(out, y, proj, splits, split_stride, width, z_at, gain, eps, tokens, parts, size, stream);
+  return TS_ERR_DTYPE;
+}
+
+template <typename T>
+static int launch_selective_token(void* out, float* y, float* state, float* held, const int* state_slots, const float* proj, int splits, long stride,
+                                  int width, int z_at, int dt_at, SsConv conv, const float* dt_bias, const float* a_log, const float* skip, const void* gain,
+                                  float eps, int tokens, int heads, int groups, int n, int p, int parts, hipStream_t stream) {
+  const dim3 grid(tokens, heads, (p + 31) / 32);
+#define ST_GO(NR, BATCH)                                                                                                                        \
+  hipLaunchKernelGGL((selective_token_kernel<T, NR, BATCH>), grid, dim3(256), 0, stream, state, state_slots, proj, held, width, heads, groups, n, p, \
+                     splits, (size_t)stride, conv, dt_at, dt_bias, a_log, skip, y)
+#define ST_ROWS(BATCH)                  \
+  do {                                  \
+    if (n <= 32) ST_GO(4, BATCH);       \
+    else if (n <= 64) ST_GO(8, BATCH);  \
+    else ST_GO(16, BATCH);              \
+  } while (0)
+  if (splits == 1) ST_ROWS(1);
+  else if (splits <= 4) ST_ROWS(4);
+  else ST_ROWS(8);
+#undef ST_ROWS
+#undef ST_GO
+  const int status = ts_launch_status();
+  if (status != TS_OK) return status;
+  const int inner = heads * p, moved = 2 * groups * n, size = inner / parts;
+  const SsMoves moves = {held, state_slots, inner + moved, inner, moved, conv.first};
+#define ST_NORM(THREADS, BATCH)                                                                                                          \
+  hipLaunchKernelGGL((gated_group_norm_few_kernel<T, float, THREADS, BATCH, true>), dim3(tokens, parts + (moved + THREADS - 1) / THREADS), \
+                     dim3(THREADS), 0, stream, proj, y, (const T*)gain, (T*)out, splits, width, (size_t)stride, z_at, parts, size, eps, moves)
+#define ST_BATCH(THREADS)                     \
+  do {                                        \
+    if (splits == 1) ST_NORM(THREADS, 1);     \
+    else if (splits <= 4) ST_NORM(THREADS, 4);\
+    else ST_NORM(THREADS, 8);                 \
+  } while (0)
+  if (size <= 256) ST_BATCH(64);
+  else if (size <= 512) ST_BATCH(128);
+  else ST_BATCH(256);
+#undef ST_BATCH
+#undef ST_NORM
+  return ts_launch_status();
+}
+
+// A step of single tokens of a selective state space from its projection on: ts_short_conv (four taps), ts_decaying_walk (selective) and
+// ts_gated_group_norm in two launches, the same bits.  proj: `splits` (at most 8) 32-bit partial sums [tokens, width]; held float [slots, 3,
+// heads p + 2 groups n]; y float [tokens, heads p] (scratch); out [tokens, heads p] of dtype; parts equal parts of a row of up to 1,024 elements;
+// n and p multiples of 4, n at most 128; all on 16 bytes.
+extern "C" int ts_selective_token(void* out, float* y, float* state, float* held, const int* state_slots, const void* proj, int splits, long stride,
+                                  int width, int z_at, int first, int dt_at, const void* taps, const void* bias, int silu, const float* dt_bias,
+                                  const float* a_log, const float* skip, const void* gain, float eps, int tokens, int heads, int groups, int n, int p,
+                                  int parts, int dtype, hipStream_t stream) {
+  if (tokens == 0) return TS_OK;
+  if (!out || !y || !state || !held || !state_slots || !proj || !taps || !dt_bias || !a_log || !skip || !gain) return TS_ERR_ARG;
+  if (heads < 1 || heads > 65535 || groups < 1 || heads % groups != 0 || n < 4 || n > 128 || n % 4 != 0 || p < 4 || p % 4 != 0 || parts < 1 ||
+      splits < 1 || splits > 8 || width % 4 != 0 || z_at % 4 != 0 || stride % 4 != 0)
+    return TS_ERR_SHAPE;
+  const long inner = (long)heads * p;
+  if (inner % parts != 0 || inner / parts > 1024 || inner / parts % 4 != 0 || z_at < 0 || z_at + inner > width || first < 0 ||
+      first + inner + 2L * groups * n > width || dt_at < 0 || dt_at + heads > width || parts + 2L * groups * n / 64 > 65534)
+    return TS_ERR_SHAPE;
+  if (((uintptr_t)out | (uintptr_t)y | (uintptr_t)state | (uintptr_t)held | (uintptr_t)proj | (uintptr_t)gain) % 16 != 0) return TS_ERR_ARG;
+  const SsConv conv = {taps, bias, first, silu};
+#define ST_ARGS out, y, state, held, state_slots, (const float*)proj, splits, stride, width, z_at, dt_at, conv, dt_bias, a_log, skip, gain, eps, tokens, \
+                heads, groups, n, p, parts, stream
+  if (dtype == TS_F32) return launch_selective_token<float>(ST_ARGS);
+  if (dtype == TS_BF16) return launch_selective_token<bf16_t>(ST_ARGS);
+#undef ST_ARGS
   return TS_ERR_DTYPE;
 }

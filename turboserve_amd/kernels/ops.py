@@ -106,6 +106,8 @@ _SIGNATURES: dict[str, dict[str, list]] = {
         "ts_decaying_pieces": [*[c_void_p] * 6, *[c_int] * 4, c_void_p, c_int, c_int, c_long, c_int, c_int, c_void_p, c_void_p, c_float,
                                c_void_p, c_float, c_void_p, *[c_int] * 7, c_void_p],
         "ts_decaying_carry": [*[c_void_p] * 8, *[c_int] * 5, c_void_p],
+        "ts_selective_token": [*[c_void_p] * 6, c_int, c_long, *[c_int] * 4, c_void_p, c_void_p, c_int, *[c_void_p] * 4, c_float, *[c_int] * 7,
+                               c_void_p],
         "ts_heads_finish": [c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int, c_long, c_int, c_int, c_void_p, c_int, c_float,
                             c_float, *[c_void_p] * 4, *[c_int] * 4, c_void_p],
         "ts_gated_group_norm": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_long, c_int, c_int, c_void_p, c_float, c_int, c_int, c_int,
@@ -1349,6 +1351,43 @@ class Ops:
             groups=groups, state_dim=state_dim, value_dim=value_dim, dtype=dtype, proj=proj, first_gate=dt_at, numbers=(dt_bias, a_log),
             skip=skip, plan=plan)
         return y
+
+    def selective_token(self, proj: torch.Tensor, first_col: int, taps: torch.Tensor, bias: torch.Tensor | None, held: torch.Tensor, dt_at: int,
+                        dt_bias: torch.Tensor, a_log: torch.Tensor, skip: torch.Tensor, state: torch.Tensor, state_slots: torch.Tensor, *, heads: int,
+                        groups: int, state_dim: int, value_dim: int, z_at: int, gain: torch.Tensor, eps: float, parts: int,
+                        dtype: torch.dtype) -> torch.Tensor | None:
+        """A step of single tokens of a selective state space, from its projection to what the output matrix multiplies: :meth:`short_conv` (with
+        ``silu``), :meth:`selective_state` and :meth:`gated_group_norm` in two launches, the same bits, or None where they are three: for other
+        than four taps, state rows of more than 128, more than eight partial sums or a plain bfloat16 projection, sizes that four elements do not
+        divide, and from 256 parts of rows on, where the norm is another kernel (us a layer, 64 heads of 128 x 64, eight tokens, three launches 3.8 +
+        9.0 + 3.9, two 9.0 + 4.2; a step of nine such layers 486 / 463)."""
+        tokens, width = proj.shape[-2], proj.shape[-1]
+        inner, channels = heads * value_dim, heads * value_dim + 2 * groups * state_dim
+        if (proj.dtype != torch.float32 or taps.shape[1] != 4 or not 4 <= state_dim <= 128 or state_dim % 4 or value_dim % 4 or inner % parts
+                or inner // parts > 1024 or (inner // parts) % 4 or width % 4 or z_at % 4 or tokens * parts >= 256 or proj.data_ptr() % 16
+                or (proj.dim() == 3 and (proj.shape[0] > 8 or proj.stride(0) % 4))):
+            return None
+        _gpu(proj, taps, bias, held, dt_bias, a_log, skip, state, state_slots, gain)
+        _i32(state_slots, "state_slots")
+        _, splits, stride = self._partials(proj, tokens, width, dtype, "projection")
+        _need(taps.shape == (channels, 4) and taps.dtype == dtype and taps.is_contiguous() and 0 <= first_col and first_col + channels <= width,
+              "taps must be [C, 4] of the run dtype, over columns of the projection")
+        _need(bias is None or (bias.shape == (channels,) and bias.dtype == dtype and bias.is_contiguous()), "the convolution's bias must be [C] of the run dtype")
+        _need(held.dtype == torch.float32 and held.is_contiguous() and held.shape[1:] == (3, channels), "the inputs held must be float32 [slots, 3, C]")
+        _need(state.dtype == torch.float32 and state.is_contiguous() and state.shape[1:] == (heads, value_dim, state_dim),
+              "the state must be float32 [slots, H, P, N]")
+        for t in (dt_bias, a_log, skip):
+            _need(t.shape == (heads,) and t.dtype == torch.float32 and t.is_contiguous(), "a rule's numbers must be float32 [H]")
+        _need(heads % groups == 0 and gain.shape == (inner,) and gain.dtype == dtype and gain.is_contiguous() and gain.data_ptr() % 16 == 0
+              and 0 <= z_at and z_at + inner <= width and 0 <= dt_at and dt_at + heads <= width and state_slots.numel() >= tokens,
+              "the gates' columns inside the projection, a gain [H P] of the run dtype, a slot a token")
+        y = torch.empty((tokens, inner), dtype=torch.float32, device=proj.device)
+        out = self.rows_buffer(tokens, inner, dtype, proj.device)
+        _check(self.core.ts_selective_token(
+            _ptr(out), _ptr(y), _ptr(state), _ptr(held), _ptr(state_slots), _ptr(proj), splits, stride, width, z_at, first_col, dt_at, _ptr(taps), _ptr(bias),
+            1, _ptr(dt_bias), _ptr(a_log), _ptr(skip), _ptr(gain), float(eps), tokens, heads, groups, state_dim, value_dim, parts, dtype_code(dtype),
+            self.stream()), "ts_selective_token")
+        return out
 
     def heads_finish(self, y: torch.Tensor, proj: torch.Tensor, gate_at: int, heads: int, eps: float, dtype: torch.dtype, *,
                      gate: str = "silu", gain: torch.Tensor | None = None, norm: torch.Tensor | None = None,

@@ -109,6 +109,12 @@ class Mamba2(Mixer):
         ops, dtype = self.runtime.ops, self.runtime.dtype
         memory, held = cache
         proj = ops.linear(x, self.in_weight)
+        if ctx.num_tokens == ctx.num_seqs:  # every request brings one token
+            out = ops.selective_token(proj, self.inner, self.conv_weight, self.conv_bias, held.state, self.inner + self.channels, self.dt_bias, self.a_log,
+                                      self.skip, memory.state, ctx.state_slots, heads=self.num_heads, groups=self.groups, state_dim=self.state_dim,
+                                      value_dim=self.value_dim, z_at=0, gain=self.gain, eps=self.norm_eps, parts=self.norm_groups, dtype=dtype)
+            if out is not None:
+                return out
         u = ops.short_conv(proj, self.inner, self.conv_weight, held.state, ctx.state_slots, ctx.token_seq, ctx.query_start_loc,
                            tokens=ctx.num_tokens, num_seqs=ctx.num_seqs, dtype=dtype, silu=True, bias=self.conv_bias)
         plan = ops.decaying_plan(ctx, dtype, self.state_dim, self.value_dim)
