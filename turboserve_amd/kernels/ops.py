@@ -2774,7 +2774,10 @@ class Ops:
         leaves the last round of workgroups so empty that the tiled product is as fast or faster: always where one range is
         asked for (27,648 x 5,120 at eight rows 48 against 46 us; 37,888 x 3,584, a last round two thirds full, 41.7 against
         43.9), where it is only the cheapest over a long K (at one / 16 rows 20,480 x 5,120 37.9 / 43.6 against 38.5 / 38.8, but
-        18,944 x 3,584 26.7 / 29.4 against 27.5 / 28.5)."""
+        18,944 x 3,584 26.7 / 29.4 against 27.5 / 28.5).  Over a short K tiles of 16 weight rows as one range where tiles of 32 leave the last
+        round up to half full (one / eight / 16 rows: 10,304 x 2,048 9.7 / 9.9 / 10.6 against 11.0 / 10.9 / 11.2 as two ranges, 12,288 x 2,048 10.5 / 10.7 /
+        11.4 against 10.7 / 11.3 / 12.3, 18,944 x 2,048 14.2 / 14.8 / 16.0 against 15.4 / 15.8 / 16.6; gated, 10,304 x 2,560 11.1 / 12.0 / 14.2 against 12.5 /
+        13.2 / 14.8; as sums over 2,560 two ranges are the sooner, 10.9 / 11.4 / 12.2 against 11.0 / 12.0 / 14.3, over 1,536 it is the same)."""
         key = (n, k, max_splits)
         if key in self._stream_plans:
             return self._stream_plans[key]
@@ -2791,15 +2794,22 @@ class Ops:
         plan = best[1:]
         if plan[1] == 1 and (max_splits == 1 or k > 4096) and tiles > 2 * units and 10 * units * -(-tiles // units) > 11 * tiles:
             plan = None
+        elif (1024 < k < 3072 if max_splits == 1 else 1536 < k <= 2048) and units < tiles < 3 * units and 0 < tiles % units <= units // 2:
+            plan = (-(-slices // 4), 1, 1)
         self._stream_plans[key] = plan
         return plan
 
     def _stream_cost(self, n: int, k: int, splits: int) -> float:
         """What the streaming product takes as ``splits`` ranges, in microseconds beyond its start:
         what a compute unit reads takes 36 bytes a nanosecond where few units read and all of them
-        together get 6.6 TB/s; a range more costs 0.12 us (its sums, here and in the kernel that adds them up)."""
+        together get 6.6 TB/s; a range more costs 0.12 us (its sums, here and in the kernel that adds them up).  Over a long K it is 31 a nanosecond
+        where some units have two workgroups or more (at 36 grids that give some units two and some one look as soon as finer ones; one / eight
+        rows, 12,288 x 3,584 as one / two ranges 16.5 / 15.6 and 17.8 / 16.1, 18,944 x 3,584 24.9 / 22.3 and 25.1 / 22.7, 12,288 x 5,120
+        23.9 / 21.4 and 25.1 / 21.8, x 6,144 27.6 / 26.1 and 29.9 / 26.8; not of multiples of 4,096, whose ranges lie in the same
+        channels of the memory, x 4,096 17.8 / 20.2 and 18.8 / 20.5; 13,312 x 2,560 13.0 / 14.0 and 14.8 / 14.1)."""
         rounds = -(-(-(-n // 32) * splits) // self.compute_units)
-        return max(2.0 * n * k / 6.6e6, rounds * 64.0 * k / splits / 36e3) + 0.12 * splits
+        rate = 31e3 if rounds > 1 and k > 3072 and k % 4096 else 36e3
+        return max(2.0 * n * k / 6.6e6, rounds * 64.0 * k / splits / rate) + 0.12 * splits
 
     def _stream_runs(self, x: torch.Tensor, weight: torch.Tensor, max_splits: int | None) -> tuple[int, int, int] | None:
         """The streaming product's grid where it runs a decode-sized product (up to 16 rows)."""
