@@ -1285,6 +1285,21 @@ decaying_piece_out_kernel(float* __restrict__ y, float* __restrict__ norm, const
 // ---------------------------------------------------------------------------------------------
 // the gated norm in parts
 // ---------------------------------------------------------------------------------------------
+// y silu(gate) of a thread's COUNT elements (gated_near's arithmetic, common.hpp; the other form only where a wavefront has such gates).
+template <int COUNT>
+__device__ __forceinline__ void ss_gated(float (&y)[COUNT], const float (&gate)[COUNT]) {
+  float most = 0.f;
+#pragma unroll
+  for (int e = 0; e < COUNT; ++e) most = fmaxf(most, fabsf(gate[e]));
+  if (__ballot(!(most <= GATE_NEAR)) == 0) {
+#pragma unroll
+    for (int e = 0; e < COUNT; ++e) y[e] *= gated_near(gate[e], gate[e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < COUNT; ++e) y[e] *= fabsf(gate[e]) <= GATE_NEAR ? gated_near(gate[e], gate[e]) : gated_far(gate[e], gate[e]);
+  }
+}
+
 template <typename T, typename P, int VEC, int CHUNKS>
 __global__ void __launch_bounds__(1024)
 gated_group_norm_kernel(T* __restrict__ out, const float* __restrict__ y, const P* __restrict__ proj, int splits, size_t split_stride,
@@ -1304,11 +1319,9 @@ gated_group_norm_kernel(T* __restrict__ out, const float* __restrict__ y, const 
       float gate[VEC];
       ss_input_vec<P, VEC>(z + i, splits, split_stride, gate);
       load_vec<float, VEC>(y + row + i, v[c]);
+      ss_gated<VEC>(v[c], gate);
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        v[c][e] *= gate[e] / (1.f + expf(-gate[e]));
-        ss = fmaf(v[c][e], v[c][e], ss);
-      }
+      for (int e = 0; e < VEC; ++e) ss = fmaf(v[c][e], v[c][e], ss);
     }
   }
   const float by = rsqrtf(block_sum(ss, scratch) / (float)size + eps);
@@ -1322,6 +1335,46 @@ gated_group_norm_kernel(T* __restrict__ out, const float* __restrict__ y, const 
       for (int e = 0; e < VEC; ++e) v[c][e] *= by * w[e];
       store_vec<T, VEC>(out + row + i, v[c]);
     }
+  }
+}
+
+// The same bits for a prompt's many parts of up to 256 CHUNKS elements: a wavefront a part, four a workgroup, which meet nowhere; a part's quads
+// and their sums lie as a workgroup's wavefronts have them above.  64 MB for 2,000 rows of eight parts of 512: GN_FIGURES us a layer.
+template <typename T, typename P, int CHUNKS>
+__global__ void __launch_bounds__(256)
+gated_group_norm_rows_kernel(T* __restrict__ out, const float* __restrict__ y, const P* __restrict__ proj, int splits, size_t split_stride, int width,
+                             int z_at, const T* __restrict__ gain, float eps, int parts, int size, int items) {
+  const int item = blockIdx.x * 4 + threadIdx.x / TS_WAVE, lane = threadIdx.x % TS_WAVE;
+  if (item >= items) return;
+  const int t = item / parts, part = item - t * parts;
+  const size_t row = (size_t)item * size;
+  const P* z = proj + (size_t)t * width + z_at + (size_t)part * size;
+  float v[CHUNKS][4], gate[CHUNKS][4], w[CHUNKS][4];
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = min(4 * (c * TS_WAVE + lane), size - 4);
+    ss_input_vec<P, 4>(z + i, splits, split_stride, gate[c]);
+    load_vec<float, 4>(y + row + i, v[c]);
+    load_vec<T, 4>(gain + (size_t)part * size + i, w[c]);
+  }
+  float total = 0.f;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const bool in = 4 * (c * TS_WAVE + lane) < size;
+    float ss = 0.f;
+    ss_gated<4>(v[c], gate[c]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = in ? fmaf(v[c][e], v[c][e], ss) : ss;
+    total += wave_sum(ss);
+  }
+  const float by = rsqrtf(total / (float)size + eps);
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = 4 * (c * TS_WAVE + lane);
+    if (i >= size) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[c][e] *= by * w[c][e];
+    store_vec<T, 4>(out + row + i, v[c]);
   }
 }
 
@@ -1370,15 +1423,16 @@ gated_group_norm_few_kernel(const P* proj, const float* y, const T* gain, T* out
   load_vec<float, 4>(y + row + i, v);
   load_vec<T, 4>(gain + (size_t)part * size + i, w);
   asm volatile("" ::: "memory");  // all of them on their way here
-  float ss = 0.f;
+  float ss = 0.f, gate[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    float gate = gates[0][e];
+    gate[e] = gates[0][e];
 #pragma unroll
-    for (int j = 1; j < BATCH; ++j) gate = j < splits ? gate + gates[j][e] : gate;
-    v[e] *= gate / (1.f + expf(-gate));
-    ss = in ? fmaf(v[e], v[e], ss) : ss;
+    for (int j = 1; j < BATCH; ++j) gate[e] = j < splits ? gate[e] + gates[j][e] : gate[e];
   }
+  ss_gated<4>(v, gate);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ss = in ? fmaf(v[e], v[e], ss) : ss;
   const float by = rsqrtf(block_sum_of<THREADS>(ss, scratch) / (float)size + eps);
   if (!in) return;
 #pragma unroll
@@ -1721,7 +1775,14 @@ static int launch_gated_group_norm(void* out, const float* y, const void* proj, 
 #undef GN_FEW
       return ts_launch_status();
     }
-    if (pieces <= 256 || (few && pieces <= 1024)) GN_GO(4, 1, (pieces + 63) / 64 * 64);
+#define GN_ROWS(CHUNKS)                                                                                                                    \
+  hipLaunchKernelGGL((gated_group_norm_rows_kernel<T, P, CHUNKS>), dim3((unsigned)(((long)tokens * parts + 3) / 4)), dim3(256), 0, stream, \
+                     (T*)out, y, (const P*)proj, splits, (size_t)split_stride, width, z_at, (const T*)gain, eps, parts, size, tokens * parts)
+    if (!few && pieces <= 256 && (long)tokens * parts <= 0x7fffffffL) {
+      if (pieces <= 64) GN_ROWS(1);
+      else if (pieces <= 128) GN_ROWS(2);
+      else GN_ROWS(4);
+    } else if (pieces <= 256 || (few && pieces <= 1024)) GN_GO(4, 1, (pieces + 63) / 64 * 64);
     else if (pieces <= 1024) GN_GO(4, 4, 256);
     else if (pieces <= 4096) GN_GO(4, 4, 1024);
     else if (pieces <= 16384) GN_GO(4, 16, 1024);
@@ -1732,6 +1793,7 @@ static int launch_gated_group_norm(void* out, const float* y, const void* proj, 
     else return TS_ERR_SHAPE;
   }
 #undef GN_GO
+#undef GN_ROWS
   return ts_launch_status();
 }
 
