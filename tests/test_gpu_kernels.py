@@ -1683,6 +1683,26 @@ def test_attention_prefill_mfma_every_launch_plan(ops, heads, kv_heads, dim, tok
     torch.testing.assert_close(out.float().cpu(), case.expected, **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("window", [None, 333])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(28, 4, 128), (16, 4, 128), (10, 2, 96), (8, 2, 64), (6, 2, 32)])
+@pytest.mark.parametrize("seqs", [
+    [(1000, 45)], [(417, 417), (701, 13), (33, 1)], [(448, 31), (449, 33), (480, 64), (900, 2)], [(299, 299), (64, 40)],
+    [(300 + i, 33 + i % 31) for i in range(70)],
+])
+def test_attention_prefill_mfma_of_ragged_blocks(ops, heads, kv_heads, dim, seqs, window):
+    """Blocks of fewer rows than a tile behind contexts of many windows, which no column's masks touch; halves of a block's windows in one workgroup (an odd
+    window, a block of one window, a last window of one key), and grids of more workgroups than units, whose blocks stay whole."""
+    case = PagedCase(torch.bfloat16, heads, kv_heads, dim, 16, seqs, window, seed=dim + len(seqs))
+    rows, blocks = prefill_blocks_of(ops, case, heads, kv_heads, dim, seqs)
+    assert rows == 32
+    out = torch.zeros(case.qsl[-1], heads * dim, dtype=torch.bfloat16, device=DEV)
+    ops.attention_prefill(
+        out, case.dev(case.q), heads * dim, case.dev(case.kp), case.dev(case.vp), case.dev(case.table),
+        case.ints(case.qsl), case.ints([c for c, _ in seqs]), case.ints(blocks), heads, dim ** -0.5, window, max(c for c, _ in seqs), rows,
+    )
+    torch.testing.assert_close(out.float().cpu(), case.expected, **tol(torch.bfloat16))
+
+
 def shared_out_work(case, seqs, window, shares_wanted):
     """A work list in which every block of 32 rows with two or more windows of keys is shared out
     over up to ``shares_wanted`` workgroups, written out from the entry point's description."""
