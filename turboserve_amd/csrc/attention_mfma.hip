@@ -1533,8 +1533,14 @@ constexpr int WIDE_PIECES = WINDOW_KEYS / KEYS_PER_WAVE;
 constexpr int FED_MAX_HEADS = 7;
 constexpr int FED_MIN_HEADS = 5;  // fewer heads beside the feeder leave SIMDs with one wavefront
 
-template <bool FED>
-__global__ void __launch_bounds__((FED ? FED_MAX_HEADS + 1 : STAGE_WAVES) * TS_WAVE)
+// PAIRED: eight wavefronts, two for every head: the second four take the later half of the block's windows, with LDS of their own, and leave
+// their sums in LDS for the first.  For grids that leave a workgroup a compute unit to itself: a block's rounds, each of which waits
+// for the one before, are half as many, and no launch puts the halves together.  From thirteen windows on (us, four / eight wavefronts, 28
+// heads of 128 on 4 KV heads: 299 tokens 13.2 / 13.7, 400 15.6 / 15.5, 512 17.8 / 17.2, 768 23.4 / 21.5, 1,000 28.2 / 25.3, 128 behind 512
+// 19.9 / 18.3, 256 behind 512 22.8 / 20.7; twice the wavefronts start later, and the halves' way through LDS takes 1 us).
+constexpr int PAIRED_MIN_KEYS = 13 * WINDOW_KEYS;
+template <bool FED, bool PAIRED>
+__global__ void __launch_bounds__((FED ? FED_MAX_HEADS + 1 : PAIRED ? 2 * STAGE_WAVES : STAGE_WAVES) * TS_WAVE)
     __attribute__((amdgpu_waves_per_eu(2, 2)))
 prefill_wide_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, long q_stride,
                     const uint16_t* __restrict__ k_pages, const uint16_t* __restrict__ v_pages,
@@ -1543,11 +1549,13 @@ prefill_wide_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, 
                     int pair_blocks, int group_heads, int heads, int kv_heads, int block_shift, ScoreRule scale_log2,
                     int window, const int* __restrict__ ranges, float* __restrict__ partial_acc,
                     float* __restrict__ partial_ml) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t staged[];  // [2][K_TILE] then [2][V_TILE]
-  uint16_t* ks = staged;
-  uint16_t* vs = staged + 2 * K_TILE;
+  extern __shared__ __attribute__((aligned(16))) uint16_t staged[];  // [2][K_TILE] then [2][V_TILE] (paired: twice)
   const int lane = threadIdx.x & (TS_WAVE - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TS_WAVE);  // known to be the same in every lane
+  const int place = __builtin_amdgcn_readfirstlane(threadIdx.x / TS_WAVE);  // known to be the same in every lane
+  const bool later = PAIRED && place >= STAGE_WAVES;  // of the second four
+  const int wave = PAIRED ? place % STAGE_WAVES : place;
+  uint16_t* ks = staged + (later ? 2 * (K_TILE + V_TILE) : 0);
+  uint16_t* vs = ks + 2 * K_TILE;
   const int col = lane & 31;
   const int half = lane >> 5;
   const int gsize = heads / kv_heads;
@@ -1598,7 +1606,7 @@ prefill_wide_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, 
   if (begin >= end) {
     // A share that lies past the block's keys (no work list of this library's makes one): it
     // has seen nothing, and says so.  The whole workgroup leaves here, before any barrier.
-    if (slot >= 0 && wave_live) {
+    if (slot >= 0 && wave_live && !later) {
       const size_t entry = ((size_t)slot * heads + kvh * gsize + hg) * WIDE_ROWS + col;
       for (int d = 4 * half; d < D; d += 8) *reinterpret_cast<f32x4*>(partial_acc + entry * D + d) = f32x4{0.f, 0.f, 0.f, 0.f};
       if (half == 0) {
@@ -1609,6 +1617,12 @@ prefill_wide_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, 
     return;
   }
 
+  // The halves of a paired block; the later one may have no window (it then goes through the first rounds' loads, of the last window, alone).
+  const int earlier_rounds = PAIRED ? ((end - begin + WINDOW_KEYS - 1) / WINDOW_KEYS + 1) / 2 : 0;
+  if (PAIRED) {
+    if (later) begin += earlier_rounds * WINDOW_KEYS;
+    else end = min(end, begin + earlier_rounds * WINDOW_KEYS);
+  }
   PageGeometry geo{k_pages, v_pages, block_table + (size_t)seq * table_width, table_width, kv_heads, kvh, block_shift,
                    (1 << block_shift) - 1};
   // The queries as B operands: lane holds, for token `col`, head dimensions 16 j + 8 half .. + 7.
@@ -1637,7 +1651,7 @@ prefill_wide_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, 
   // ago, go to LDS, and the keys of W(i + 3) and the values of W(i + 1) are asked for.  LDS
   // holds two windows of keys and two of values.  Windows past the last are the last again
   // (loads stay unconditional, see prefill_shared_kernel); their scores are computed and dropped.
-  const int rounds = (end - begin + WINDOW_KEYS - 1) / WINDOW_KEYS;
+  const int rounds = max(0, (end - begin + WINDOW_KEYS - 1) / WINDOW_KEYS);
   const int last_window = (end - 1) & ~(WINDOW_KEYS - 1);
   auto window_at = [&](int i) { return min(begin + i * WINDOW_KEYS, last_window); };
   // The pieces this wavefront moves: its own one, or all of them.
@@ -1671,7 +1685,7 @@ prefill_wide_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, 
   }
   // The value windows start as zeros: the first round multiplies one of them by probabilities
   // that are all zero, and what LDS held before could be anything.
-  for (int e = threadIdx.x * 8; e < 2 * V_TILE; e += blockDim.x * 8)
+  for (int e = (PAIRED ? threadIdx.x % (STAGE_WAVES * TS_WAVE) : threadIdx.x) * 8; e < 2 * V_TILE; e += (PAIRED ? STAGE_WAVES * TS_WAVE : blockDim.x) * 8)
     *reinterpret_cast<u32x4*>(vs + e) = u32x4{0u, 0u, 0u, 0u};
   if (feeds) {
 #pragma unroll
@@ -1852,11 +1866,41 @@ prefill_wide_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, 
   } else {
     run(std::false_type{}, std::true_type{});
   }
+  if (PAIRED && rounds < earlier_rounds) __syncthreads();  // the later half is a round shorter where they are odd in all
   // The last window's values are still to be accumulated.
   if (wave_live) accumulate_values(vs + ((rounds - 1) & 1) * V_TILE, pp0, pp1);
 
   float la, lb;
   swap_rows(l, true, la, lb);
+  if constexpr (PAIRED) {
+    // The later half's sums and references through LDS, a lane's side by side with its neighbours'.
+    f32x4* const sums = reinterpret_cast<f32x4*>(staged) + wave * (D / 8) * TS_WAVE + lane;
+    f32x2* const refs = reinterpret_cast<f32x2*>(staged + STAGE_WAVES * (D / 8) * TS_WAVE * 8) + wave * TS_WAVE + lane;
+    __syncthreads();  // the staged windows have been read
+    if (later) {
+#pragma unroll
+      for (int t = 0; t < NT32; ++t)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) sums[(4 * t + a) * TS_WAVE] = f32x4{acc[t][4 * a], acc[t][4 * a + 1], acc[t][4 * a + 2], acc[t][4 * a + 3]};
+      *refs = f32x2{m, la + lb};
+    }
+    __syncthreads();
+    if (later) return;
+    const f32x2 other = *refs;
+    const float top = fmaxf(m, other[0]);
+    const float mine = m == -INFINITY ? 0.f : exp2f(m - top), theirs = other[0] == -INFINITY ? 0.f : exp2f(other[0] - top);
+    la = (la + lb) * mine;
+    lb = other[1] * theirs;
+    m = top;
+#pragma unroll
+    for (int t = 0; t < NT32; ++t)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const f32x4 sum = sums[(4 * t + a) * TS_WAVE];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[t][4 * a + e] = fmaf(sum[e], theirs, acc[t][4 * a + e] * mine);
+      }
+  }
   if (slot >= 0) {
     // A share of a block: the sums as they are, with the reference they were taken against.
     // Columns past the block's rows saw nothing (m = -inf, zeros) and are written like the rest.
@@ -1985,16 +2029,26 @@ static int launch_prefill_wide(hipStream_t stream, uint16_t* out, const uint16_t
   if (fed) {
     // One workgroup fills a compute unit; blocks come heaviest first, so units that finish early
     // take the lighter ones.
-    hipLaunchKernelGGL(prefill_wide_kernel<true>, dim3((unsigned)total), dim3((group_heads + 1) * TS_WAVE), lds, stream,
+    hipLaunchKernelGGL((prefill_wide_kernel<true, false>), dim3((unsigned)total), dim3((group_heads + 1) * TS_WAVE), lds, stream,
                        out, q, q_stride, k_pages, v_pages, block_table, table_width, query_start_loc, context_lens,
                        blocks, num_blocks, 0, group_heads, heads, kv_heads, shift, scale_log2, window, ranges,
                        partial_acc, partial_ml);
   } else {
     const int pair_blocks = (!ranges && total <= 2LL * compute_units) ? 1 : 0;
-    hipLaunchKernelGGL(prefill_wide_kernel<false>, dim3((unsigned)total), dim3(STAGE_WAVES * TS_WAVE), lds, stream, out,
-                       q, q_stride, k_pages, v_pages, block_table, table_width, query_start_loc, context_lens, blocks,
-                       num_blocks, pair_blocks, group_heads, heads, kv_heads, shift, scale_log2, window, ranges,
-                       partial_acc, partial_ml);
+    if (total <= compute_units && max_context > PAIRED_MIN_KEYS) {
+      constexpr size_t joined = (size_t)STAGE_WAVES * TS_WAVE * (D / 8 * 16 + 8), both = 2 * lds > joined ? 2 * lds : joined;
+      static const bool raised = hipFuncSetAttribute((const void*)prefill_wide_kernel<false, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     (int)both) == hipSuccess;
+      if (!raised) return TS_ERR_LAUNCH;
+      hipLaunchKernelGGL((prefill_wide_kernel<false, true>), dim3((unsigned)total), dim3(2 * STAGE_WAVES * TS_WAVE), both, stream, out, q,
+                         q_stride, k_pages, v_pages, block_table, table_width, query_start_loc, context_lens, blocks, num_blocks, 0,
+                         group_heads, heads, kv_heads, shift, scale_log2, window, ranges, partial_acc, partial_ml);
+    } else {
+      hipLaunchKernelGGL((prefill_wide_kernel<false, false>), dim3((unsigned)total), dim3(STAGE_WAVES * TS_WAVE), lds, stream, out,
+                         q, q_stride, k_pages, v_pages, block_table, table_width, query_start_loc, context_lens, blocks,
+                         num_blocks, pair_blocks, group_heads, heads, kv_heads, shift, scale_log2, window, ranges,
+                         partial_acc, partial_ml);
+    }
   }
   const int status = ts_launch_status();
   if (status != TS_OK || num_combine == 0) return status;
