@@ -1340,20 +1340,20 @@ gated_group_norm_kernel(T* __restrict__ out, const float* __restrict__ y, const 
 
 // The same bits for a prompt's many parts of up to 256 CHUNKS elements: a wavefront a part, four a workgroup, which meet nowhere; a part's quads
 // and their sums lie as a workgroup's wavefronts have them above.  64 MB for 2,000 rows of eight parts of 512: 13.5 -> 12.8 us.
-template <typename T, typename P, int CHUNKS>
+template <typename T, int CHUNKS>
 __global__ void __launch_bounds__(256)
-gated_group_norm_rows_kernel(T* __restrict__ out, const float* __restrict__ y, const P* __restrict__ proj, int splits, size_t split_stride, int width,
-                             int z_at, const T* __restrict__ gain, float eps, int parts, int size, int items) {
+gated_group_norm_rows_kernel(T* __restrict__ out, const float* __restrict__ y, const T* __restrict__ proj, int width, int z_at,
+                             const T* __restrict__ gain, float eps, int parts, int size, int items) {
   const int item = blockIdx.x * 4 + threadIdx.x / TS_WAVE, lane = threadIdx.x % TS_WAVE;
   if (item >= items) return;
   const int t = item / parts, part = item - t * parts;
   const size_t row = (size_t)item * size;
-  const P* z = proj + (size_t)t * width + z_at + (size_t)part * size;
+  const T* z = proj + (size_t)t * width + z_at + (size_t)part * size;
   float v[CHUNKS][4], gate[CHUNKS][4], w[CHUNKS][4];
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
     const int i = min(4 * (c * TS_WAVE + lane), size - 4);
-    ss_input_vec<P, 4>(z + i, splits, split_stride, gate[c]);
+    load_vec<T, 4>(z + i, gate[c]);
     load_vec<float, 4>(y + row + i, v[c]);
     load_vec<T, 4>(gain + (size_t)part * size + i, w[c]);
   }
@@ -1775,14 +1775,23 @@ static int launch_gated_group_norm(void* out, const float* y, const void* proj, 
 #undef GN_FEW
       return ts_launch_status();
     }
-#define GN_ROWS(CHUNKS)                                                                                                                    \
-  hipLaunchKernelGGL((gated_group_norm_rows_kernel<T, P, CHUNKS>), dim3((unsigned)(((long)tokens * parts + 3) / 4)), dim3(256), 0, stream, \
-                     (T*)out, y, (const P*)proj, splits, (size_t)split_stride, width, z_at, (const T*)gain, eps, parts, size, tokens * parts)
-    if (!few && pieces <= 256 && (long)tokens * parts <= 0x7fffffffL) {
-      if (pieces <= 64) GN_ROWS(1);
-      else if (pieces <= 128) GN_ROWS(2);
-      else GN_ROWS(4);
-    } else if (pieces <= 256 || (few && pieces <= 1024)) GN_GO(4, 1, (pieces + 63) / 64 * 64);
+    // A wavefront a part where the projection is one of 16 bits and there are parts enough that four a workgroup fill the units (us, a workgroup /
+    // a wavefront a part of 512, eight a row: 32 rows 2.6 / 2.8, 128 2.9 / 3.0, 192 3.3 / 3.2, 512 4.5 / 4.2, 1,024 7.1 / 6.5; of two partial
+    // sums, which a workgroup asks for sooner, 32 rows 2.8 / 3.4, 256 4.0 / 4.2).
+    const long items = (long)tokens * parts;
+    if constexpr (sizeof(P) == 2) {
+#define GN_ROWS(CHUNKS)                                                                                                                     \
+  hipLaunchKernelGGL((gated_group_norm_rows_kernel<T, CHUNKS>), dim3((unsigned)((items + 3) / 4)), dim3(256), 0, stream, (T*)out, y,        \
+                     (const T*)proj, width, z_at, (const T*)gain, eps, parts, size, (int)items)
+      if (pieces <= 256 && items >= 1536 && items <= 0x7fffffffL && splits == 1) {
+        if (pieces <= 64) GN_ROWS(1);
+        else if (pieces <= 128) GN_ROWS(2);
+        else GN_ROWS(4);
+#undef GN_ROWS
+        return ts_launch_status();
+      }
+    }
+    if (pieces <= 256 || (few && pieces <= 1024)) GN_GO(4, 1, (pieces + 63) / 64 * 64);
     else if (pieces <= 1024) GN_GO(4, 4, 256);
     else if (pieces <= 4096) GN_GO(4, 4, 1024);
     else if (pieces <= 16384) GN_GO(4, 16, 1024);
@@ -1793,7 +1802,6 @@ static int launch_gated_group_norm(void* out, const float* y, const void* proj, 
     else return TS_ERR_SHAPE;
   }
 #undef GN_GO
-#undef GN_ROWS
   return ts_launch_status();
 }
 
