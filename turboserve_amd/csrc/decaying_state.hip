@@ -454,6 +454,7 @@ struct SsSteps {
 // What the projection says of a wavefront's two tokens a lane, 2 l and 2 l + 1 (rows beyond the piece: its last one's).
 template <int RULE>
 struct SsInputs {
+  float head_one, head_two;            // the head's own
   float one[2];                        // d; i'
   float two[RULE == SS_GATED ? 2 : 1]; // f'
 };
@@ -461,6 +462,11 @@ struct SsInputs {
 // For several pieces at once, so that their loads are on their way together.
 template <int RULE, int COUNT, typename P>
 __device__ __forceinline__ void ss_inputs(SsInputs<RULE> (&in)[COUNT], const P* proj, const SsGates& gates, int h, int heads, const SsPiece (&pieces)[COUNT]) {
+#pragma unroll
+  for (int x = 0; x < COUNT; ++x) {
+    in[x].head_one = gates.one[h];
+    in[x].head_two = RULE == SS_FIXED ? 0.f : gates.two[h];
+  }
   if (RULE == SS_FIXED) return;
   const P* column = proj + gates.first + h;
   const int lane = threadIdx.x % TS_WAVE;
@@ -493,10 +499,30 @@ __device__ __forceinline__ void ss_inputs(SsInputs<RULE> (&in)[COUNT], const P* 
     }
 }
 
+template <int CONTROL, int ROW_MASK>
+__device__ __forceinline__ double ss_moved(double keep, double v) {  // lanes_moved of 64 bits
+  const uint64_t k = __builtin_bit_cast(uint64_t, keep), b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t low = __builtin_amdgcn_update_dpp((int)(uint32_t)k, (int)(uint32_t)b, CONTROL, ROW_MASK, 0xF, false);
+  const uint32_t high = __builtin_amdgcn_update_dpp((int)(uint32_t)(k >> 32), (int)(uint32_t)(b >> 32), CONTROL, ROW_MASK, 0xF, false);
+  return __builtin_bit_cast(double, (uint64_t)high << 32 | low);
+}
+
+// What `join` makes of a lane's value and those of the lanes before it (`none`: of no lane), in registers: every other wavefront of the
+// workgroup waits for the decays, and each of the six steps through LDS took some 200 clocks.
+template <typename Join>
+__device__ __forceinline__ double ss_running(double v, Join join, double none) {
+  v = join(ss_moved<0x111, 0xF>(none, v), v);  // row_shr 1, 2, 4, 8: the lanes before it in its row of 16
+  v = join(ss_moved<0x112, 0xF>(none, v), v);
+  v = join(ss_moved<0x114, 0xF>(none, v), v);
+  v = join(ss_moved<0x118, 0xF>(none, v), v);
+  v = join(ss_moved<0x142, 0xA>(none, v), v);  // row_bcast15 into rows 1 and 3, row_bcast31 into rows 2 and 3
+  return join(ss_moved<0x143, 0xC>(none, v), v);
+}
+
 // By one wavefront: lane l takes the tokens 2 l and 2 l + 1 (beyond the piece: nothing decays, nothing is added).
 // `floor`: what t starts from (gated).
 template <int RULE>
-__device__ __forceinline__ void ss_steps(SsSteps<RULE>& at, const SsInputs<RULE>& inputs, const SsGates& gates, int h, double floor, int count) {
+__device__ __forceinline__ void ss_steps(SsSteps<RULE>& at, const SsInputs<RULE>& inputs, const SsGates& gates, double floor, int count) {
   const int lane = threadIdx.x % TS_WAVE;
   float w[2];
   double gone[2], in[2] = {0., 0.};  // log a; the log input gate
@@ -504,35 +530,25 @@ __device__ __forceinline__ void ss_steps(SsSteps<RULE>& at, const SsInputs<RULE>
   for (int e = 0; e < 2; ++e) {
     const bool there = 2 * lane + e < count;
     if (RULE == SS_SELECTIVE) {
-      w[e] = there ? ss_softplus(inputs.one[e] + gates.one[h]) : 0.f;
-      gone[e] = -(double)expf(gates.two[h]) * (double)w[e];
+      w[e] = there ? ss_softplus(inputs.one[e] + inputs.head_one) : 0.f;
+      gone[e] = -(double)expf(inputs.head_two) * (double)w[e];
     } else if (RULE == SS_FIXED) {
       w[e] = there ? 1.f : 0.f;
-      gone[e] = there ? log((double)gates.one[h]) : 0.;
+      gone[e] = there ? log((double)inputs.head_one) : 0.;
     } else {
       w[e] = there ? 1.f : 0.f;
-      gone[e] = there ? (double)ss_log_sigmoid(ss_capped(inputs.two[RULE == SS_GATED ? e : 0] + gates.two[h], gates.cap)) : 0.;
-      in[e] = (double)ss_capped(inputs.one[e] + gates.one[h], gates.cap);
+      gone[e] = there ? (double)ss_log_sigmoid(ss_capped(inputs.two[RULE == SS_GATED ? e : 0] + inputs.head_two, gates.cap)) : 0.;
+      in[e] = (double)ss_capped(inputs.one[e] + inputs.head_one, gates.cap);
     }
   }
   const double own = gone[0] + gone[1];
-  double sum = own;
-#pragma unroll
-  for (int d = 1; d < TS_WAVE; d <<= 1) {
-    const double other = __shfl_up(sum, d);
-    if (lane >= d) sum += other;
-  }
+  const double sum = ss_running(own, [](double before, double v) { return before + v; }, 0.);
   const double c[2] = {sum - own + gone[0], sum};
   double s[2] = {-c[0], -c[1]};
   if (RULE == SS_GATED) {
 #pragma unroll
     for (int e = 0; e < 2; ++e) s[e] = 2 * lane + e < count ? in[e] + s[e] : SS_NEVER;
-    double most = fmax(s[0], s[1]);
-#pragma unroll
-    for (int d = 1; d < TS_WAVE; d <<= 1) {
-      const double other = __shfl_up(most, d);
-      if (lane >= d) most = fmax(most, other);
-    }
+    const double most = ss_running(fmax(s[0], s[1]), [](double before, double v) { return fmax(v, before); }, (double)SS_NEVER);
     const double before = __shfl_up(most, 1);
     const double t[2] = {fmax(fmax(lane > 0 ? before : SS_NEVER, s[0]), floor), fmax(most, floor)};
 #pragma unroll
@@ -606,7 +622,7 @@ decaying_piece_state_kernel(float* __restrict__ piece_state, float* __restrict__
     SsInputs<RULE> in[1];
     const SsPiece one[1] = {piece};
     ss_inputs<RULE>(in, proj, gates, h, heads, one);
-    ss_steps<RULE>(steps, in[0], gates, h, SS_NEVER, piece.count);
+    ss_steps<RULE>(steps, in[0], gates, SS_NEVER, piece.count);
   }
   const size_t columns = RULE == SS_GATED ? p + 1 : p;
   ss_f32x4 acc[TILES][PT];
@@ -958,7 +974,7 @@ decaying_pass(ss_lds_u16* __restrict__ to, ss_lds_u16* __restrict__ lds, SsSteps
         if (i >= batch) break;
         SsSteps<RULE>& at = steps[wave];
         __builtin_amdgcn_wave_barrier();  // (a wavefront's accesses to LDS are in order)
-        ss_steps<RULE>(at, in[x], gates, h, SS_NEVER, of[x].count);
+        ss_steps<RULE>(at, in[x], gates, SS_NEVER, of[x].count);
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int e = 0; e < 2; ++e) ends[i][2 * lane + e] = at.w[2 * lane + e] * expf(at.from(2 * lane + e, SS_PIECE - 1));
@@ -1031,6 +1047,9 @@ decaying_pass_kernel(float* __restrict__ state, float* __restrict__ sums, const 
 // the stretch: the first is applied to a stretch's sums once, the second comes from a table that the workgroup makes once
 // (`before`: both exponents are at most zero, so nothing overflows however strong the decays are).
 // n . C (gated) is the same sum without x: of the weights that a lane holds, and of n before the piece against C.
+// Its loads were eight trips to memory one behind the other, and the others waited for what the first wavefront makes of the decays; C and the
+// state go out together, B and x before the last of the state's products (us, 64 heads of 128 x 64: one piece 15.9 -> 12.8, 512 tokens 16.8 ->
+// 14.1, 2,000 30.3 -> 27.2, 4,096 56.6 -> 47.6).  With four workgroups a unit LDS bounds it: 96 KB written and 430 KB read each.
 template <typename P, int RULE, int NK, int PT>
 __global__ void __launch_bounds__(256, NK <= 4 ? 4 : 2)
 decaying_piece_out_kernel(float* __restrict__ y, float* __restrict__ norm, const float* __restrict__ piece_state,
@@ -1054,86 +1073,120 @@ decaying_piece_out_kernel(float* __restrict__ y, float* __restrict__ norm, const
   const int tiles[2] = {wave, 7 - wave};
   const bool summing = RULE == SS_GATED && blockIdx.z == 0;
   const float enter = RULE == SS_GATED ? piece_top[(size_t)item * heads + h] : 0.f;  // t before the piece
-  if (wave == 0) {
-    SsInputs<RULE> in[1];
+  SsInputs<RULE> in[1];
+  // What one wavefront makes of the decays, all wait for: its loads go ahead of the others, whose queue is 4,000 clocks long, and the makers of a
+  // compute unit's workgroups (256 apart) are on different SIMDs.
+  const int maker = (blockIdx.y * gridDim.x + blockIdx.x) / 256 % 4;
+  if (wave == maker) {
     const SsPiece one[1] = {piece};
     ss_inputs<RULE>(in, proj, gates, h, heads, one);
-    ss_steps<RULE>(steps, in[0], gates, h, enter, piece.count);
   }
   const size_t head_state = ((size_t)item * heads + h) * (RULE == SS_GATED ? p + 1 : p);
   const float* entering = piece_state + (head_state + c0) * n;
-  float sum_of[2] = {0.f, 0.f};  // this lane's share of n . C of its tokens
+  auto row_bytes = [&](size_t at, int i, int d) __attribute__((always_inline)) {  // sixteen of a token's row
+    return *reinterpret_cast<const ts_u32x4*>(u + (size_t)(piece.first + min(i, piece.count - 1)) * u_width + at + d);
+  };
+  // What the first products read is asked for at once (whatever lies past the sizes as the last one's, and dropped).
+  constexpr int ITEMS = (PP * (NP / 8) + 255) / 256, B_ITEMS = HALF * (NP / 8) / 256, X_ITEMS = HALF * (PP / 8) / 256;
+  ss_f32x4 raw[ITEMS][2];
+#pragma unroll
+  for (int x = 0; x < ITEMS; ++x) {
+    const int i = tid + 256 * x, c = i / (NP / 8), d = (i % (NP / 8)) * 8;
+    const float* at = entering + (size_t)min(c, p - 1 - c0) * n + (d < n ? d : 0);
+    raw[x][0] = *reinterpret_cast<const ss_f32x4*>(at);
+    raw[x][1] = *reinterpret_cast<const ss_f32x4*>(at + 4);
+  }
   ts_u32x4 cf[2][NK];  // C of the wavefront's tokens: columns i, eight state rows a lane
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      const int i = 16 * tiles[a] + lo, d = 32 * k + 8 * quad;
+      cf[a][k] = row_bytes(c_at, i, d < n ? d : 0);
+    }
+  __builtin_amdgcn_sched_barrier(0);
+  if (wave == maker) ss_steps<RULE>(steps, in[0], gates, enter, piece.count);
+  float sum_of[2] = {0.f, 0.f};  // this lane's share of n . C of its tokens
   ss_f32x4 acc[PT][2];
 #pragma unroll
   for (int b = 0; b < PT; ++b)
 #pragma unroll
     for (int a = 0; a < 2; ++a) acc[b][a] = ss_f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int ITEMS = (PP * (NP / 8) + 255) / 256;
   ts_u32x4 upper[ITEMS];  // the upper plane of what the thread has read of the state, while the lower ones are multiplied
 #pragma unroll
-  for (int turn = 0; turn < 2; ++turn) {  // the two lower planes first, then the upper one in their place
-    if (turn > 0) __syncthreads();
+  for (int x = 0; x < ITEMS; ++x) {
+    const int i = tid + 256 * x, c = i / (NP / 8), d = (i % (NP / 8)) * 8;
+    const bool held = c0 + c < p && d < n;
+    ts_u32x4 middle, lower;
 #pragma unroll
-    for (int x = 0; x < ITEMS; ++x) {
-      const int i = tid + 256 * x;
-      if (i >= PP * (NP / 8)) continue;
-      const int c = i / (NP / 8), d = (i % (NP / 8)) * 8;
-      if (turn > 0) {
-        *reinterpret_cast<ts_u32x4*>(&planes[c * SROW + d]) = upper[x];
-        continue;
-      }
-      float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (c0 + c < p && d < n) {
-        const float4 v0 = *reinterpret_cast<const float4*>(entering + (size_t)c * n + d);
-        const float4 v1 = *reinterpret_cast<const float4*>(entering + (size_t)c * n + d + 4);
-        v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
-        v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
-      }
-      ts_u32x4 middle, lower;
+    for (int e = 0; e < 4; ++e) {
+      uint32_t top[2], mid[2], low[2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        uint32_t top[2], mid[2], low[2];
-        ss_cut(v[2 * e], top[0], mid[0], low[0]);
-        ss_cut(v[2 * e + 1], top[1], mid[1], low[1]);
-        upper[x][e] = ss_pair(top[0], top[1]);
-        middle[e] = ss_pair(mid[0], mid[1]);
-        lower[e] = ss_pair(low[0], low[1]);
-      }
-      *reinterpret_cast<ts_u32x4*>(&planes[c * SROW + d]) = middle;
-      *reinterpret_cast<ts_u32x4*>(&planes[(PP + c) * SROW + d]) = lower;
+      for (int k = 0; k < 2; ++k) ss_cut(held ? raw[x][e / 2][2 * (e % 2) + k] : 0.f, top[k], mid[k], low[k]);
+      upper[x][e] = ss_pair(top[0], top[1]);
+      middle[e] = ss_pair(mid[0], mid[1]);
+      lower[e] = ss_pair(low[0], low[1]);
     }
-    if (turn == 0) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        const int i = 16 * tiles[a] + lo;
-#pragma unroll
-        for (int k = 0; k < NK; ++k) {
-          const int d = 32 * k + 8 * quad;
-          cf[a][k] = ts_u32x4{0u, 0u, 0u, 0u};
-          if (i < piece.count && d < n) cf[a][k] = *reinterpret_cast<const ts_u32x4*>(u + (size_t)(piece.first + i) * u_width + c_at + d);
-        }
-      }
-    }
-    __syncthreads();
-    if (turn == 0) {
-#pragma unroll 1
-      for (int i = tid; i < SS_PIECE / 16 * SS_PIECE; i += 256) {
-        const int tile = i / SS_PIECE, j = i % SS_PIECE, r = 16 * tile - 1;
-        if (j <= r) before[tile][j] = steps.w[j] * __expf(steps.from(j, r));
-      }
-    }
-#pragma unroll
-    for (int plane = 1 - turn; plane >= 0; --plane)
-#pragma unroll
-      for (int k = 0; k < NK; ++k)
-#pragma unroll
-        for (int b = 0; b < PT; ++b) {
-          const ts_u32x4 sf = *reinterpret_cast<const ts_u32x4*>(&planes[(plane * PP + 16 * b + lo) * SROW + 32 * k + 8 * quad]);
-#pragma unroll
-          for (int a = 0; a < 2; ++a) acc[b][a] = ss_mfma(sf, cf[a][k], acc[b][a]);
-        }
+    if (i >= PP * (NP / 8)) continue;
+    *reinterpret_cast<ts_u32x4*>(&planes[c * SROW + d]) = middle;
+    *reinterpret_cast<ts_u32x4*>(&planes[(PP + c) * SROW + d]) = lower;
   }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+      if (16 * tiles[a] + lo >= piece.count || 32 * k + 8 * quad >= n) cf[a][k] = ts_u32x4{0u, 0u, 0u, 0u};
+  __syncthreads();
+#pragma unroll 1
+  for (int i = tid; i < SS_PIECE / 16 * SS_PIECE; i += 256) {
+    const int tile = i / SS_PIECE, j = i % SS_PIECE, r = 16 * tile - 1;
+    if (j <= r) before[tile][j] = steps.w[j] * __expf(steps.from(j, r));
+  }
+  auto multiply_state = [&](int plane) __attribute__((always_inline)) {
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+#pragma unroll
+      for (int b = 0; b < PT; ++b) {
+        const ts_u32x4 sf = *reinterpret_cast<const ts_u32x4*>(&planes[(plane * PP + 16 * b + lo) * SROW + 32 * k + 8 * quad]);
+#pragma unroll
+        for (int a = 0; a < 2; ++a) acc[b][a] = ss_mfma(sf, cf[a][k], acc[b][a]);
+      }
+  };
+  multiply_state(1);
+  multiply_state(0);
+  __syncthreads();
+#pragma unroll
+  for (int x = 0; x < ITEMS; ++x) {
+    const int i = tid + 256 * x, c = i / (NP / 8), d = (i % (NP / 8)) * 8;
+    if (i < PP * (NP / 8)) *reinterpret_cast<ts_u32x4*>(&planes[c * SROW + d]) = upper[x];
+  }
+  // B of half of the tokens at a time, and x of all: the first half's are on their way while the upper plane is multiplied.
+  ts_u32x4 bs[B_ITEMS], xs[X_ITEMS][2];
+  auto fetch_b = [&](int half) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < B_ITEMS; ++x) {
+      const int i = tid + 256 * x, j = half * HALF + i / (NP / 8), d = (i % (NP / 8)) * 8;
+      bs[x] = row_bytes(b_at, j, d < n ? d : 0);
+    }
+  };
+  auto put_b = [&](int half) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < B_ITEMS; ++x) {
+      const int i = tid + 256 * x, j = i / (NP / 8), d = (i % (NP / 8)) * 8;
+      *reinterpret_cast<ts_u32x4*>(&br[j * SROW + d]) = half * HALF + j < piece.count && d < n ? bs[x] : ts_u32x4{0u, 0u, 0u, 0u};
+    }
+  };
+  fetch_b(0);
+#pragma unroll
+  for (int x = 0; x < X_ITEMS; ++x)  // two tokens by eight columns a thread
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int i = tid + 256 * x, j = 2 * (i / (PP / 8)) + k, d = (i % (PP / 8)) * 8;
+      xs[x][k] = row_bytes(x_at, j, c0 + d < p ? d : 0);
+    }
+  __builtin_amdgcn_sched_barrier(0);
+  __syncthreads();
+  multiply_state(0);
   if (summing) {
     const float* held = piece_state + (head_state + p) * n;
 #pragma unroll
@@ -1156,29 +1209,22 @@ decaying_piece_out_kernel(float* __restrict__ y, float* __restrict__ norm, const
     for (int b = 0; b < PT; ++b) acc[b][a] *= by;
     sum_of[a] *= by;
   }
+  __syncthreads();  // the planes have been read: their place takes what follows
+  put_b(0);
+#pragma unroll
+  for (int x = 0; x < X_ITEMS; ++x) {
+    const int i = tid + 256 * x, q = i / (PP / 8), d = (i % (PP / 8)) * 8;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (c0 + d >= p || 2 * q + k >= piece.count) xs[x][k] = ts_u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) *reinterpret_cast<uint32_t*>(&xt[(d + e) * XROW + 2 * q]) = ss_pair(ss_half(xs[x][0], e), ss_half(xs[x][1], e));
+  }
   for (int half = 0; half * HALF < piece.count; ++half) {
-    __syncthreads();  // the planes, or B of the first half, have been read: their place takes what follows
-#pragma unroll 2
-    for (int i = tid; i < HALF * (NP / 8); i += 256) {
-      const int j = i / (NP / 8), d = (i % (NP / 8)) * 8;
-      ts_u32x4 raw = {0u, 0u, 0u, 0u};
-      if (half * HALF + j < piece.count && d < n)
-        raw = *reinterpret_cast<const ts_u32x4*>(u + (size_t)(piece.first + half * HALF + j) * u_width + b_at + d);
-      *reinterpret_cast<ts_u32x4*>(&br[j * SROW + d]) = raw;
-    }
-#pragma unroll 1
-    for (int i = tid; half == 0 && i < (SS_PIECE / 2) * (PP / 8); i += 256) {  // two tokens by eight columns a thread
-      const int q = i / (PP / 8), d = (i % (PP / 8)) * 8;
-      ts_u32x4 raw[2];
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        raw[k] = ts_u32x4{0u, 0u, 0u, 0u};
-        if (c0 + d < p && 2 * q + k < piece.count)
-          raw[k] = *reinterpret_cast<const ts_u32x4*>(u + (size_t)(piece.first + 2 * q + k) * u_width + x_at + d);
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        *reinterpret_cast<uint32_t*>(&xt[(d + e) * XROW + 2 * q]) = ss_pair(ss_half(raw[0], e), ss_half(raw[1], e));
+    if (half > 0) {
+      fetch_b(half);
+      __syncthreads();  // B of the first half has been read
+      put_b(half);
     }
     __syncthreads();
 #pragma unroll
@@ -1269,10 +1315,8 @@ decaying_piece_out_kernel(float* __restrict__ y, float* __restrict__ norm, const
       if (c0 + c >= p) continue;
       float v[4];
       if (RULE == SS_SELECTIVE) {
-        float x[4];
-        load_vec<bf16_t, 4>(u + (size_t)(piece.first + i) * u_width + x_at + c, x);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = fmaf(d_skip, x[e], acc[b][a][e]);
+        for (int e = 0; e < 4; ++e) v[e] = fmaf(d_skip, to_float(bf16_t{xt[(c + e) * XROW + i]}), acc[b][a][e]);
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = acc[b][a][e] * scale;
