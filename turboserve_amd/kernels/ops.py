@@ -2001,7 +2001,7 @@ class Ops:
         if not (2 <= parts <= 8 and k % 64 == 0 and k <= 6144 and matrix.dtype is torch.bfloat16 and matrix.shape[1] == k
                 and matrix.is_contiguous() and matrix.data_ptr() % 16 == 0):
             return False
-        plan = self._stream_plan(matrix.shape[0], k, None)
+        plan = self._stream_plan(matrix.shape[0], k, None, narrow=False)
         return plan is not None and plan[0] <= 16
 
     def _heads_product(self, heads: WaitingHeads, weight: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
@@ -2012,7 +2012,7 @@ class Ops:
         n, k = weight.shape
         if bias is not None:
             _need(bias.shape == (n,) and bias.dtype == torch.bfloat16 and bias.is_contiguous(), "bias must be bfloat16 [N]")
-        per_wave, splits, _ = self._stream_plan(n, k, None)
+        per_wave, splits, _ = self._stream_plan(n, k, None, narrow=False)
         partial = torch.empty((splits, 1, n), dtype=torch.float32, device=weight.device)
         _check(self.core.ts_gemm_stream_heads(_ptr(partial), _ptr(heads.sums), _ptr(heads.weights), parts, count, dim, _ptr(weight), _ptr(bias), n,
                                               per_wave, splits, self.stream()), "ts_gemm_stream_heads")
@@ -2767,7 +2767,7 @@ class Ops:
                                       splits, tile, x_rows, waves, depth, 1, 1.0, 0.0, 0.0, 0.0, self.stream()), "ts_gemm_wide")
         return partial
 
-    def _stream_plan(self, n: int, k: int, max_splits: int | None) -> tuple[int, int, int] | None:
+    def _stream_plan(self, n: int, k: int, max_splits: int | None, narrow: bool = True) -> tuple[int, int, int] | None:
         """(slices of 64 per wavefront, ranges of K, tile) of the streaming product: the fewest
         ranges that keep the memory busy (``_stream_cost``).  (us at one row: 3,584 x 3,584 as 1 / 2 / 4 ranges 8.1 / 6.2 / 7.2, 2,048 x
         8,192 as 1 / 2 / 4 14 / 10 / 7.7, 8,192 x 2,048 as 1 / 2 7.3 / 7.6.)  None where one range
@@ -2777,8 +2777,9 @@ class Ops:
         18,944 x 3,584 26.7 / 29.4 against 27.5 / 28.5).  Over a short K tiles of 16 weight rows as one range where tiles of 32 leave the last
         round up to half full (one / eight / 16 rows: 10,304 x 2,048 9.7 / 9.9 / 10.6 against 11.0 / 10.9 / 11.2 as two ranges, 12,288 x 2,048 10.5 / 10.7 /
         11.4 against 10.7 / 11.3 / 12.3, 18,944 x 2,048 14.2 / 14.8 / 16.0 against 15.4 / 15.8 / 16.6; gated, 10,304 x 2,560 11.1 / 12.0 / 14.2 against 12.5 /
-        13.2 / 14.8; as sums over 2,560 two ranges are the sooner, 10.9 / 11.4 / 12.2 against 11.0 / 12.0 / 14.3, over 1,536 it is the same)."""
-        key = (n, k, max_splits)
+        13.2 / 14.8; as sums over 2,560 two ranges are the sooner, 10.9 / 11.4 / 12.2 against 11.0 / 12.0 / 14.3, over 1,536 it is the same).
+        Not ``narrow``: for the kernels that make what they multiply (:meth:`_normed_product`, :meth:`_heads_product`), which have tiles of 32 alone."""
+        key = (n, k, max_splits, narrow)
         if key in self._stream_plans:
             return self._stream_plans[key]
         slices, tiles, units = -(-k // 64), -(-n // 32), self.compute_units
@@ -2794,7 +2795,7 @@ class Ops:
         plan = best[1:]
         if plan[1] == 1 and (max_splits == 1 or k > 4096) and tiles > 2 * units and 10 * units * -(-tiles // units) > 11 * tiles:
             plan = None
-        elif (1024 < k < 3072 if max_splits == 1 else 1536 < k <= 2048) and units < tiles < 3 * units and 0 < tiles % units <= units // 2:
+        elif narrow and (1024 < k < 3072 if max_splits == 1 else 1536 < k <= 2048) and units < tiles < 3 * units and 0 < tiles % units <= units // 2:
             plan = (-(-slices // 4), 1, 1)
         self._stream_plans[key] = plan
         return plan
@@ -2882,7 +2883,7 @@ class Ops:
                 or matrix.dtype is not torch.bfloat16 or not matrix.is_contiguous() or matrix.data_ptr() % 16
                 or n <= 32 * (-(-k // 1024) - 1) or (gated and n % 2)):
             return None
-        return self._stream_plan(n, k, 1 if gated else None)
+        return self._stream_plan(n, k, 1 if gated else None, narrow=False)
 
     def _normed_product(self, norm: WaitingNorm, weight: torch.Tensor, bias: torch.Tensor | None, *, gated: bool,
                         rule: tuple[float, ...] = (1.0, 0.0, 0.0)) -> torch.Tensor:
