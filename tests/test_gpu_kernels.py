@@ -1703,6 +1703,23 @@ def test_attention_prefill_mfma_of_ragged_blocks(ops, heads, kv_heads, dim, seqs
     torch.testing.assert_close(out.float().cpu(), case.expected, **tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("window", [100, 190, 222, 640])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(28, 4, 128), (8, 2, 64)])
+@pytest.mark.parametrize("seqs", [[(1000, 45)], [(900, 31), (701, 66), (20, 2)], [(448, 448), (433, 17)]])
+def test_attention_prefill_mfma_of_blocks_whose_window_leaves_many_keys(ops, heads, kv_heads, dim, seqs, window):
+    """A sliding window that leaves a block four to 22 windows of keys, about where they are walked in two halves: both ways, masks in the first
+    window of the earlier half and the last of the later one."""
+    case = PagedCase(torch.bfloat16, heads, kv_heads, dim, 16, seqs, window, seed=dim + window)
+    work = ops.prefill_blocks([q for _, q in seqs], [c for c, _ in seqs], 32, heads=heads, kv_heads=kv_heads, head_dim=dim, block_size=16, window=window)
+    assert work.ranges is None and 4 <= work.longest <= 22
+    out = torch.zeros(case.qsl[-1], heads * dim, dtype=torch.bfloat16, device=DEV)
+    ops.attention_prefill(
+        out, case.dev(case.q), heads * dim, case.dev(case.kp), case.dev(case.vp), case.dev(case.table),
+        case.ints(case.qsl), case.ints([c for c, _ in seqs]), work, heads, dim ** -0.5, window, max(c for c, _ in seqs), 32,
+    )
+    torch.testing.assert_close(out.float().cpu(), case.expected, **tol(torch.bfloat16))
+
+
 def shared_out_work(case, seqs, window, shares_wanted):
     """A work list in which every block of 32 rows with two or more windows of keys is shared out
     over up to ``shares_wanted`` workgroups, written out from the entry point's description."""

@@ -553,6 +553,59 @@ def test_prefill_work_list_shares_out_long_blocks():
     assert shared_out > 40
 
 
+@pytest.mark.parametrize("window", [0, 33, 333, 500])
+def test_the_prefill_attention_is_told_how_many_windows_its_longest_entry_walks(monkeypatch, window):
+    """Whether a block's windows are walked in two halves is chosen by the entries of the work list, shares and the layer's own window counted, not by the
+    step's longest context: a prompt of 1,000 tokens under a window of 333 keys has no block of more than twelve windows."""
+    import ctypes
+    import random
+    from types import SimpleNamespace
+
+    from turboserve_amd.kernels import ops as module
+
+    told = []
+
+    def shape(heads, kv_heads, page, per_block, per_unit):
+        ctypes.cast(per_block, ctypes.POINTER(ctypes.c_int))[0] = kv_heads
+        ctypes.cast(per_unit, ctypes.POINTER(ctypes.c_int))[0] = 2
+
+    lib = SimpleNamespace(ts_attention_prefill_rows_d32=lambda heads, kv_heads: 32, ts_attention_prefill_shape_d32=shape,
+                          ts_attention_prefill_d32=lambda *operands: told.append(operands) or 0)
+    monkeypatch.setattr(module, "load_module", lambda name: lib)
+    monkeypatch.setattr(module, "_gpu", lambda *tensors: None)
+    ops = object.__new__(module.Ops)
+    ops.device, ops.compute_units, ops.stream = torch.device("cpu"), 256, lambda: None
+    rng, shared = random.Random(window), 0
+
+    def launched(query_lens, context_lens, **given):
+        total, pages = sum(query_lens), torch.zeros(1, 2, 16, 32, dtype=torch.bfloat16)
+        ints = torch.zeros(len(query_lens) + 1, dtype=torch.int32)
+        work = ops.prefill_blocks(query_lens, context_lens, 32, heads=8, kv_heads=2, head_dim=32, block_size=16, window=window)
+        for blocks in (work, work.blocks):
+            ops.attention_prefill(torch.empty(total, 256, dtype=torch.bfloat16), torch.empty(total, 256, dtype=torch.bfloat16), 256, pages, pages.view(1, 2, 32, 16),
+                                  torch.zeros(len(query_lens), 4096, dtype=torch.int32), ints, ints, blocks, 8, 1.0, window or None, max(context_lens), 32)
+        return work, told[-2][19], told[-1][19]
+
+    assert launched([1000], [1000])[1] == {0: 32, 33: 2, 333: 12, 500: 17}[window]
+    ops.prefill_share_min_windows, ops.prefill_share_combine_cost = 4, 0
+    for _ in range(60):
+        query_lens = [rng.choice([1, 2, 31, 33, 64, 100, 300, 700]) for _ in range(rng.randint(1, 4))]
+        context_lens = [q + rng.choice([0, 5, 200, 3000, 20000]) for q in query_lens]
+        work, longest, bound = launched(query_lens, context_lens)
+        starts = [sum(query_lens[:i]) for i in range(len(query_lens))]
+
+        def whole(request, row):
+            offset = row - starts[request]
+            return module.prefill_block_windows(context_lens[request] - query_lens[request] + offset, min(32, query_lens[request] - offset), window)
+
+        ranges = [[0, 0, -1]] * work.blocks.shape[0] if work.ranges is None else work.ranges.tolist()
+        assert longest == max(r[1] or whole(*b) for b, r in zip(work.blocks.tolist(), ranges))
+        most = max(whole(*b) for b in work.blocks.tolist())  # a list without shares, of blocks alone: a bound
+        assert most <= bound <= most + (2 if window else 0)
+        shared += work.ranges is not None
+    assert (shared > 5) == (window != 33)
+
+
 def test_the_kept_token_array_follows_the_lists():
     """``Sequence.token_array`` is ``token_ids`` at every moment: through appended tokens, places
     taken for unread tokens and filled or dropped later, growth beyond what the array held, and a

@@ -1535,10 +1535,14 @@ constexpr int FED_MIN_HEADS = 5;  // fewer heads beside the feeder leave SIMDs w
 
 // PAIRED: eight wavefronts, two for every head: the second four take the later half of the block's windows, with LDS of their own, and leave
 // their sums in LDS for the first.  For grids that leave a workgroup a compute unit to itself: a block's rounds, each of which waits
-// for the one before, are half as many, and no launch puts the halves together.  From thirteen windows on (us, four / eight wavefronts, 28
-// heads of 128 on 4 KV heads: 299 tokens 13.2 / 13.7, 400 15.6 / 15.5, 512 17.8 / 17.2, 768 23.4 / 21.5, 1,000 28.2 / 25.3, 128 behind 512
-// 19.9 / 18.3, 256 behind 512 22.8 / 20.7; twice the wavefronts start later, and the halves' way through LDS takes 1 us).
-constexpr int PAIRED_MIN_KEYS = 13 * WINDOW_KEYS;
+// for the one before, are half as many, and no launch puts the halves together.  By the windows of the launch's longest entry, after the
+// layer's sliding window and the shares: from fourteen on (us, four / eight wavefronts, 28 heads of 128 on 4 KV heads: 299 tokens 13.0 / 13.5, 400
+// 15.2 / 15.2, 480 17.1 / 16.5, 1,000 28.5 / 24.5, 128 behind 512 19.9 / 18.3, 256 behind 512 22.8 / 20.7; twice the wavefronts start
+// later, and the halves' way through LDS takes 1 us), where a sliding window cuts contexts off from eight on, since most of their rounds test
+// for masks and take longer (1,000 tokens, a window of 64 keys, 3 of 32, 11.3 / 11.9, of 160, 6, 13.2 / 13.8, of 224, 8, 14.4 / 14.1, of 333, 12,
+// 17.2 / 16.3; 16 heads on 4, 300 behind 3,700, 160 13.4 / 13.2, 256 15.8 / 15.0).
+constexpr int PAIRED_MIN_WINDOWS = 14;
+constexpr int PAIRED_MIN_CUT_WINDOWS = 8;
 template <bool FED, bool PAIRED>
 __global__ void __launch_bounds__((FED ? FED_MAX_HEADS + 1 : PAIRED ? 2 * STAGE_WAVES : STAGE_WAVES) * TS_WAVE)
     __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -1992,7 +1996,7 @@ static int launch_prefill_wide(hipStream_t stream, uint16_t* out, const uint16_t
                                const uint16_t* k_pages, const uint16_t* v_pages, const int* block_table,
                                int table_width, const int* query_start_loc, const int* context_lens,
                                const int* blocks, int num_blocks, int heads, int kv_heads, int shift,
-                               ScoreRule scale_log2, int window, int max_context, const int* ranges,
+                               ScoreRule scale_log2, int window, int max_context, int longest, const int* ranges,
                                float* partial_acc, float* partial_ml, const int* combine, int num_combine) {
   constexpr size_t lds = (size_t)2 * (K_TILE + V_TILE) * sizeof(uint16_t);
   static_assert(lds <= 64 * 1024, "two workgroups' staged windows must fit in LDS");
@@ -2035,7 +2039,8 @@ static int launch_prefill_wide(hipStream_t stream, uint16_t* out, const uint16_t
                        partial_acc, partial_ml);
   } else {
     const int pair_blocks = (!ranges && total <= 2LL * compute_units) ? 1 : 0;
-    if (total <= compute_units && max_context > PAIRED_MIN_KEYS) {
+    const bool cut = window > 0 && max_context > window;
+    if (total <= compute_units && longest >= (cut ? PAIRED_MIN_CUT_WINDOWS : PAIRED_MIN_WINDOWS)) {
       constexpr size_t joined = (size_t)STAGE_WAVES * TS_WAVE * (D / 8 * 16 + 8), both = 2 * lds > joined ? 2 * lds : joined;
       static const bool raised = hipFuncSetAttribute((const void*)prefill_wide_kernel<false, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                      (int)both) == hipSuccess;
@@ -2136,7 +2141,8 @@ extern "C" int TS_SYM(ts_attention_decode_d)(
 // ts_attention_prefill_rows_d says for the geometry); blocks [num_blocks, 2] holds (request
 // index, first row) of each, rows being token rows of the step.  Writes the rows of
 // `out [T, heads * D]` the blocks cover.  max_context: the longest context among the requests, or 0
-// if the caller does not know it (it only helps to choose a launch plan).
+// if the caller does not know it (it only helps to choose a launch plan); longest: the most windows of 32 keys that an entry
+// of `blocks` walks, or a bound of them (likewise).
 // ranges (may be null; blocks of 32 rows only): [num_blocks, 3] = (first window, windows, slot) of
 // each entry of `blocks`.  An entry with slot -1 is a whole block (windows 0: all of them).  The
 // others are shares of a block's windows of 32 keys, counted from the block's first window (the
@@ -2170,7 +2176,7 @@ extern "C" void TS_SYM(ts_attention_prefill_shape_d)(int heads, int kv_heads, in
 extern "C" int TS_SYM(ts_attention_prefill_d)(
     void* out, const void* q, long q_stride, const void* k_pages, const void* v_pages, const int* block_table,
     int table_width, const int* query_start_loc, const int* context_lens, const int* blocks, int num_blocks,
-    int block_rows, int heads, int kv_heads, int block_size, float scale, float softcap, int window, int max_context,
+    int block_rows, int heads, int kv_heads, int block_size, float scale, float softcap, int window, int max_context, int longest,
     const int* ranges, void* partial_acc, void* partial_ml, const int* combine, int num_combine,
     hipStream_t stream) {
   if (num_blocks == 0) return TS_OK;
@@ -2188,7 +2194,7 @@ extern "C" int TS_SYM(ts_attention_prefill_d)(
   if (gsize >= 3)
     return launch_prefill_wide(stream, (uint16_t*)out, (const uint16_t*)q, q_stride, (const uint16_t*)k_pages,
                                (const uint16_t*)v_pages, block_table, table_width, query_start_loc, context_lens,
-                               blocks, num_blocks, heads, kv_heads, shift, score_rule(scale, softcap), window, max_context, ranges,
+                               blocks, num_blocks, heads, kv_heads, shift, score_rule(scale, softcap), window, max_context, longest, ranges,
                                (float*)partial_acc, (float*)partial_ml, combine, num_combine);
 #endif
   if (ranges) return TS_ERR_ARG;  // only blocks of 32 rows are shared out

@@ -174,7 +174,7 @@ def _attention_signatures(head_dim: int) -> dict[str, list]:
                                              c_void_p, c_void_p, c_void_p],
         f"ts_attention_prefill_d{head_dim}": [c_void_p, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int,
                                               c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float,
-                                              c_float, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
+                                              c_float, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
         f"ts_attention_prefill_rows_d{head_dim}": [c_int, c_int],
         f"ts_attention_prefill_shape_d{head_dim}": [c_int, c_int, c_int, c_void_p, c_void_p],
     }
@@ -303,10 +303,15 @@ def prefill_block_windows(first_position: int, rows: int, window: int) -> int:
 
 def prefill_share_list(query_lens, context_lens, rows: int, window: int, per_block: int, places: int,
                        min_windows: int, *, combine_cost: int = 20):
+    """:func:`prefill_work_list` without its last."""
+    return prefill_work_list(query_lens, context_lens, rows, window, per_block, places, min_windows, combine_cost)[:3]
+
+
+def prefill_work_list(query_lens, context_lens, rows: int, window: int, per_block: int, places: int, min_windows: int, combine_cost: int):
     """The work list of the prefill attention with the keys of long blocks shared out over several
-    workgroups, where that shortens the launch: ``(blocks, ranges, combine)`` as lists of
+    workgroups, where that shortens the launch: ``(blocks, ranges, combine, longest)``, lists of
     ``[request, first row]``, ``[first window, windows, slot]`` (slot -1, windows 0: a whole block) and
-    ``[first row, rows, first slot, shares]``; ``ranges`` and ``combine`` are empty where nothing
+    ``[first row, rows, first slot, shares]``, and the windows that the longest entry walks; ``ranges`` and ``combine`` are empty where nothing
     is shared out and the list is :func:`prefill_block_list`'s.
 
     An entry becomes ``per_block`` workgroups, ``places`` of which run at a time.  Sharing pays
@@ -329,7 +334,7 @@ def prefill_share_list(query_lens, context_lens, rows: int, window: int, per_blo
     longest = max((block[0] for block in whole), default=0)
     if (rows != PREFILL_WINDOW_KEYS or per_block < 1 or longest < 2 * min_windows
             or (len(whole) + 1) * per_block > places):
-        return plain, [], []
+        return plain, [], [], longest
 
     def shares_of(windows: int, size: int) -> int:
         return 1 if windows <= size else min(PREFILL_MAX_SHARES, -(-windows // size))
@@ -346,7 +351,7 @@ def prefill_share_list(query_lens, context_lens, rows: int, window: int, per_blo
             low = size + 1
     size = low
     if max(-(-block[0] // shares_of(block[0], size)) for block in whole) + combine_cost >= longest:
-        return plain, [], []
+        return plain, [], [], longest
     entries, combine, slot = [], [], 0
     for windows, index, row, here in whole:
         shares = shares_of(windows, size)
@@ -360,7 +365,13 @@ def prefill_share_list(query_lens, context_lens, rows: int, window: int, per_blo
             entries.append((min(each, windows - share * each), index, row, share * each, min(each, windows - share * each), slot))
             slot += 1
     entries.sort(key=lambda entry: -entry[0])
-    return [[e[1], e[2]] for e in entries], [[e[3], e[4], e[5]] for e in entries], combine
+    return [[e[1], e[2]] for e in entries], [[e[3], e[4], e[5]] for e in entries], combine, entries[0][0]
+
+
+def prefill_most_windows(max_context: int, rows: int, window: int) -> int:
+    """The most windows of 32 keys that a block of up to ``rows`` rows of requests of up to ``max_context`` keys can have."""
+    whole = -(-max_context // PREFILL_WINDOW_KEYS)
+    return min(whole, (window + rows - 2) // PREFILL_WINDOW_KEYS + 2) if window > 0 else whole
 
 
 @dataclass
@@ -371,6 +382,7 @@ class PrefillWork:
     ranges: torch.Tensor | None = None   # int32 [n, 3]: first window, windows, slot; None: whole blocks only
     combine: torch.Tensor | None = None  # int32 [c, 4]: first row, rows, first slot, shares
     slots: int = 0
+    longest: int | None = None           # windows of 32 keys that the longest entry walks, where known
 
 
 @dataclass(frozen=True)
@@ -2115,18 +2127,18 @@ class Ops:
         tail of the launch.  Given the geometry (and the layer's window), the keys of long
         blocks are shared out over several workgroups where whole blocks would leave compute
         units idle (:func:`prefill_share_list`): a short portion at the end of a long context."""
-        ranges, combine = [], []
+        ranges, combine, longest = [], [], None
         if heads and kv_heads and head_dim and block_size and rows == PREFILL_WINDOW_KEYS:
             per_block, per_unit = c_int(0), c_int(0)
             lib = load_module(build.attention_module(head_dim))
             getattr(lib, f"ts_attention_prefill_shape_d{head_dim}")(heads, kv_heads, block_size, ctypes.byref(per_block),
                                                                    ctypes.byref(per_unit))
-            blocks, ranges, combine = prefill_share_list(
+            blocks, ranges, combine, longest = prefill_work_list(
                 query_lens, context_lens, rows, int(window or 0), per_block.value, per_unit.value * self.compute_units,
-                self.prefill_share_min_windows, combine_cost=self.prefill_share_combine_cost)
+                self.prefill_share_min_windows, self.prefill_share_combine_cost)
         else:
             blocks = prefill_block_list(query_lens, context_lens, rows)
-        work = PrefillWork(torch.tensor(blocks, dtype=torch.int32).view(-1, 2).to(self.device))
+        work = PrefillWork(torch.tensor(blocks, dtype=torch.int32).view(-1, 2).to(self.device), longest=longest)
         if ranges:
             work.ranges = torch.tensor(ranges, dtype=torch.int32).view(-1, 3).to(self.device)
             work.combine = torch.tensor(combine, dtype=torch.int32).view(-1, 4).to(self.device)
@@ -2175,6 +2187,7 @@ class Ops:
         _need(max_context <= block_table.shape[1] * block_size, "block table does not cover the context")
         _need(block_rows == self.prefill_block_rows(head_dim, heads, kv_heads),
               f"blocks of {block_rows} rows are not what the kernel for this geometry takes")
+        longest = prefill_most_windows(int(max_context), block_rows, int(window or 0)) if work.longest is None else work.longest
         partial_acc = partial_ml = None
         num_combine = 0
         if work.ranges is not None:
@@ -2189,7 +2202,7 @@ class Ops:
         fn = getattr(lib, f"ts_attention_prefill_d{head_dim}")
         _check(fn(_ptr(out), _ptr(q), q_stride, _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
                   block_table.shape[1], _ptr(query_start_loc), _ptr(context_lens), _ptr(blocks), blocks.shape[0],
-                  block_rows, heads, kv_heads, block_size, float(scale), float(softcap), int(window or 0), int(max_context),
+                  block_rows, heads, kv_heads, block_size, float(scale), float(softcap), int(window or 0), int(max_context), longest,
                   _ptr(work.ranges), _ptr(partial_acc), _ptr(partial_ml), _ptr(work.combine), num_combine,
                   self.stream()),
                "ts_attention_prefill")
