@@ -1583,7 +1583,7 @@ prefill_wide_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, 
   const int pos0 = ctx - (row_end - query_start_loc[seq]) + (row0 - query_start_loc[seq]);  // position of row0
   const int cols = min(WIDE_ROWS, row_end - row0);
   const bool col_valid = col < cols;
-  const int p_col = col_valid ? pos0 + col : -1;  // an invalid column sees nothing and is never stored
+  const int p_col = col_valid ? pos0 + col : -1;  // an invalid column sees nothing where masks are applied
   const int lo_col = (window > 0 && p_col - window + 1 > 0) ? p_col - window + 1 : 0;
   const int p_last = pos0 + cols - 1;
   const int lo_first = (window > 0 && pos0 - window + 1 > 0) ? pos0 - window + 1 : 0;
@@ -1907,7 +1907,8 @@ prefill_wide_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ q, 
   }
   if (slot >= 0) {
     // A share of a block: the sums as they are, with the reference they were taken against.
-    // Columns past the block's rows saw nothing (m = -inf, zeros) and are written like the rest.
+    // Columns past the block's rows hold what a query of zeros sums up, or nothing (m = -inf), and are written like the rest;
+    // prefill_combine_kernel stops at the rows.
     if (wave_live) {
       const size_t entry = ((size_t)slot * heads + kvh * gsize + hg) * WIDE_ROWS + col;
       float* arow = partial_acc + entry * D + 4 * half;
