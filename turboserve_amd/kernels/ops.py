@@ -2788,10 +2788,13 @@ class Ops:
         asked for (27,648 x 5,120 at eight rows 48 against 46 us; 37,888 x 3,584, a last round two thirds full, 41.7 against
         43.9), where it is only the cheapest over a long K (at one / 16 rows 20,480 x 5,120 37.9 / 43.6 against 38.5 / 38.8, but
         18,944 x 3,584 26.7 / 29.4 against 27.5 / 28.5).  Over a short K tiles of 16 weight rows as one range where tiles of 32 leave the last
-        round up to half full (one / eight / 16 rows: 10,304 x 2,048 9.7 / 9.9 / 10.6 against 11.0 / 10.9 / 11.2 as two ranges, 12,288 x 2,048 10.5 / 10.7 /
-        11.4 against 10.7 / 11.3 / 12.3, 18,944 x 2,048 14.2 / 14.8 / 16.0 against 15.4 / 15.8 / 16.6; gated, 10,304 x 2,560 11.1 / 12.0 / 14.2 against 12.5 /
-        13.2 / 14.8; as sums over 2,560 two ranges are the sooner, 10.9 / 11.4 / 12.2 against 11.0 / 12.0 / 14.3, over 1,536 it is the same).
-        Not ``narrow``: for the kernels that make what they multiply (:meth:`_normed_product`, :meth:`_heads_product`), which have tiles of 32 alone."""
+        round up to half full: gated, 1,024 < K < 3,072 (10,304 x 2,560 at one / eight / 16 rows 11.1 / 12.0 / 14.2 against 12.5 / 13.2 / 14.8), and as sums
+        where K is 2,048, whose rows of 4 KB two ranges read in halves that lie in the same channels of the memory (16 rows a tile / two ranges of 32 /
+        one range of 32, 10,304 x 2,048 9.5 / 10.6 / 9.7, 9.3 / 10.5 / 10.2 and 10.2 / 10.8 / 11.0, 18,944 x 2,048 14.4 / 17.3 / 15.4, 14.3 / 17.3 / 15.1 and
+        15.6 / 17.6 / 15.9); beside it two ranges are as soon up to eight rows and sooner at 16 (10,304 x 1,792 8.6 / 8.4 / 8.7, 8.4 / 8.7 / 9.2 and 9.4 / 8.9 /
+        9.9, x 1,920 9.0 / 8.7, 8.9 / 9.0 and 10.0 / 9.4).
+        Not ``narrow``: for the kernels that make what they multiply (:meth:`_normed_product`, :meth:`_heads_product`), which have tiles of 32 alone:
+        one range there where K is 2,048 (a row normalised, one range / two, 8,704 x 2,048 9.9 / 10.4, 10,304 x 2,048 10.1 / 11.6; x 1,792 9.4 / 9.2)."""
         key = (n, k, max_splits, narrow)
         if key in self._stream_plans:
             return self._stream_plans[key]
@@ -2808,8 +2811,8 @@ class Ops:
         plan = best[1:]
         if plan[1] == 1 and (max_splits == 1 or k > 4096) and tiles > 2 * units and 10 * units * -(-tiles // units) > 11 * tiles:
             plan = None
-        elif narrow and (1024 < k < 3072 if max_splits == 1 else 1536 < k <= 2048) and units < tiles < 3 * units and 0 < tiles % units <= units // 2:
-            plan = (-(-slices // 4), 1, 1)
+        elif (1024 < k < 3072 if max_splits == 1 else k == 2048) and units < tiles < 3 * units and 0 < tiles % units <= units // 2:
+            plan = (-(-slices // 4), 1, 1 if narrow else 2)
         self._stream_plans[key] = plan
         return plan
 
