@@ -279,3 +279,27 @@ def test_spans_whose_parts_the_output_product_joins(pairs, span, parts):
     ops = object.__new__(Ops)
     ops.compute_units = 256
     assert ops._joined_parts(pairs, span) == parts
+
+
+@pytest.mark.parametrize("head_dim,keys,parts", [
+    (32, 128, 1), (32, 256, 1), (32, 257, 4), (32, 512, 4), (64, 128, 1), (64, 129, 3), (64, 256, 4), (96, 128, 1), (96, 129, 3), (128, 64, 1), (128, 65, 2),
+    (128, 512, 4), (192, 65, 2), (256, 64, 1), (256, 128, 2), (64, 640, 5),
+])
+def test_a_short_span_stays_whole_where_parts_cost_more_to_join_than_they_save(monkeypatch, head_dim, keys, parts):
+    """One request's attention in front of a product that joins parts: a workgroup a KV head over spans that it reads about as soon as that product has put
+    the parts together, by the head's size."""
+    from turboserve_amd.kernels import ops as module
+
+    launched = []
+    monkeypatch.setattr(module, "load_module", lambda name: SimpleNamespace(**{f"ts_attention_decode_d{head_dim}": lambda *of: launched.append(of) or 0}))
+    monkeypatch.setattr(module, "_gpu", lambda *tensors: None)
+    ops = object.__new__(Ops)
+    ops.compute_units, ops.stream, ops._stream_plans = 256, lambda: None, {}
+    heads, ints = 1024 // head_dim * 2, torch.zeros(2, dtype=torch.int32)
+    heads -= heads % 2
+    out = torch.zeros(1, heads * head_dim, dtype=torch.bfloat16)
+    pages, table = torch.zeros(2, 2, 16, head_dim, dtype=torch.bfloat16), torch.zeros(1, 64, dtype=torch.int32)
+    matrix = torch.zeros(512, heads * head_dim, dtype=torch.bfloat16)
+    waiting = ops.attention_decode(out, out, out.shape[1], pages, pages.view(2, 2, head_dim, 16), table, ints, ints[:1], 0, 1, heads, 1.0, None, keys, waits_for=matrix)
+    assert launched[0][19] == parts and (waiting is None) == (parts == 1)
+    assert parts == 1 or waiting.sums.shape == (heads, parts, head_dim)

@@ -1988,7 +1988,7 @@ class Ops:
         pairs = requests * kv_heads * -(-(heads // kv_heads) // 16)
         joined = waits_for is not None and requests == 1 and out.shape[0] == 1 and self._heads_wait(2, heads * head_dim, waits_for)
         splits = self._decode_parts(pairs, span, head_dim, shares)
-        if joined and splits == 1:
+        if joined and splits == 1 and span > self._joined_whole_keys(head_dim):
             splits = self._joined_parts(pairs, span)
         partial_acc = partial_ml = None
         if splits > 1:
@@ -2009,7 +2009,7 @@ class Ops:
         """Whether the product by ``matrix [N, K]`` puts together what ``parts`` workgroups left of one request's keys: up to eight (a
         range of K reads them all, once for every 32 weight rows), of up to 6,144 elements, where the streaming product runs.  A part is at
         least 64 keys of a bound that is a power of two in a recorded step, so with fewer than 32 KV heads these are bounds of 128 to 1,024 keys (65 to 1,024 of
-        the request's); from 1,025 on there are sixteen parts and more, and the launch that combines them."""
+        the request's; small heads from 129 or 257 on, :meth:`_joined_whole_keys`); from 1,025 on there are sixteen parts and more, and the launch that combines them."""
         if not (2 <= parts <= 8 and k % 64 == 0 and k <= 6144 and matrix.dtype is torch.bfloat16 and matrix.shape[1] == k
                 and matrix.is_contiguous() and matrix.data_ptr() % 16 == 0):
             return False
@@ -2029,6 +2029,14 @@ class Ops:
         _check(self.core.ts_gemm_stream_heads(_ptr(partial), _ptr(heads.sums), _ptr(heads.weights), parts, count, dim, _ptr(weight), _ptr(bias), n,
                                               per_wave, splits, self.stream()), "ts_gemm_stream_heads")
         return partial
+
+    @staticmethod
+    def _joined_whole_keys(head_dim: int) -> int:
+        """Spans of one request that stay whole where dividing them costs no launch (:meth:`_joined_parts`): what few workgroups have read about as soon as
+        the parts are put together.  Microseconds of attention and product, 16 heads on 4 KV heads, a hidden size of 2,048, whole / divided, keys of a
+        bound: heads of 32 100 of 128 5.7 / 6.5, 250 of 256 6.7 / 6.8, 260 of 300 7.2 / 6.9; of 64 (32 on 8) 100 of 128 8.1 / 8.3, 150 of 160 8.5 / 8.4;
+        of 96 100 of 128 7.7 / 8.0, 200 of 256 8.4 / 8.1; of 128 100 of 128 9.1 / 8.9; of 192 66 of 80 10.5 / 10.2; of 256 100 of 128 12.6 / 11.8."""
+        return 64 if head_dim >= 128 else max(128, 8192 // head_dim)
 
     def _joined_parts(self, pairs: int, span: int) -> int:
         """How many workgroups share one request's whole span where the product by the output matrix puts their parts together (:meth:`_heads_wait`),
