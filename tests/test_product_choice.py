@@ -297,6 +297,55 @@ def test_a_product_looks_at_its_operands_once(monkeypatch, m, kind):
     assert product()[0] == "block" and len(asked) == 2 and not planned
 
 
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (1, 8192, 2048, "stream"), (8, 2048, 8192, "stream"), (1, 20480, 5120, "tiled"), (40, 37888, 3584, "block"), (64, 8192, 2048, "block"),
+    (200, 16384, 2048, "block"), (160, 1024, 4096, "library"), (400, 8192, 1544, "wide"),
+])
+def test_the_unit_of_a_product_asks_for_the_products_choice_once(monkeypatch, m, n, k, kernel):
+    """max(y, 0)^2 in the product's launch where that is one range of the streaming or the block kernel, else behind the product that ``linear`` runs, whose
+    choice is not worked out a second time: a prompt of a small model is bound by the host."""
+    monkeypatch.setattr("turboserve_amd.kernels.ops._gpu", lambda *tensors: None)
+    ran, asked = [], []
+
+    class Squares(Planner):
+        def _block_product(self, x, weight, bias, *, plan, gated, sums, rule, squared=False):
+            ran.append(("block", squared))
+            return "block", plan[1] > 1
+
+        def gemm_stream(self, x, weight, bias=None, *, plan, gated=False, rule=None, squared=False):
+            ran.append(("stream", squared))
+            return "stream", plan[1] > 1
+
+        def gemm_wide(self, *operands, **more):
+            ran.append(("wide", False))
+            return "wide", more["plan"][1] > 1
+
+        def gemm_tiled(self, *operands, **more):
+            ran.append(("tiled", False))
+            return "tiled", True
+
+        def _library_product(self, *operands):
+            ran.append(("library", False))
+            return "library", False
+
+        def activate(self, product, kind, dtype):
+            assert kind == "relu_squared" and dtype == torch.bfloat16
+            ran.append("unit")
+            return product
+
+    ops = Squares()
+    ops.time_wide_choices = False
+    for name in ("block_supported", "_own_choice", "_stream_runs", "_block_few_runs", "_wide_runs"):
+        monkeypatch.setattr(ops, name, lambda *of, name=name, real=getattr(ops, name): asked.append(name) or real(*of), raising=False)
+    x, w = operands(m, n, k)
+    _, ranges = ops.linear_relu_squared(x, w)
+    alone = kernel in ("stream", "block") and not ranges
+    assert ran == ([(kernel, True)] if alone else [(kernel, False), "unit"])
+    assert kernel == "tiled" or max(map(asked.count, asked)) == 1
+    ran.clear()
+    assert ops.linear(x, w)[0] == kernel  # the same product without the unit
+
+
 def test_one_range_with_a_nearly_empty_last_round_is_left_to_the_tiled_product():
     ops = Planner()
     assert ops._stream_plan(20480, 5120, None) is None and ops._stream_plan(27648, 5120, 1) is None and ops._stream_plan(17408, 2048, 1) is None

@@ -3271,24 +3271,35 @@ class Ops:
         """``max(x @ weight^T, 0)^2`` in the dtype of ``x``: :meth:`linear` and :meth:`activate`, in one launch where the product is one range of
         K of the streaming or the block kernel, which then square its 32-bit sums and round once (us, 8,192 x 2,048 with 2,000 / 300 / 8 rows, product
         and activation / one launch: 67.4 / 54.6, 22.6 / 19.3, 9.4 / 7.3)."""
+        product = None  # as :meth:`linear` makes it, by a choice that is asked for once
         if not isinstance(x, WaitingNorm) and x.dtype == torch.bfloat16 and x.dim() == 2:
-            rule, (n, k) = (1.0, 0.0, 0.0), weight.shape
-            if x.shape[0] <= self.skinny_max_rows:
-                if self.skinny_supported(x, weight):
-                    _gpu(x, weight)
-                    block = self._block_few_runs(x, weight, None, None)
-                    if block is not None and block[1] == 1:
-                        return self._block_product(x, weight, None, plan=block, gated=False, sums=False, rule=rule, squared=True)
-                    stream = self._stream_runs(x, weight, None) if block is None else None
-                    if stream is not None and stream[1] == 1:
-                        return self.gemm_stream(x, weight, plan=stream, squared=True)
-            elif self.skinny_supported_any_rows(x, weight):
+            (m, k), n, rule = x.shape, weight.shape[0], (1.0, 0.0, 0.0)
+            if m <= self.skinny_max_rows and self.skinny_supported(x, weight):
                 _gpu(x, weight)
-                m = x.shape[0]
-                block, plan, _, untimed = self._own_choice(m, n, k, "one", self.block_supported(x, weight))
-                if block and self._wide_runs(m, n, k, "one", untimed, self._own_product(x, weight, None, "one")[0],
-                                             lambda: self._library_product(x, weight, None, None)):
+                streams = m <= self.stream_max_rows
+                plan = self._stream_runs(x, weight, None) if streams else self._block_few_runs(x, weight, None, None)
+                alone = plan is not None and plan[1] == 1
+                if plan is not None:
+                    product = self.gemm_stream(x, weight, plan=plan, squared=alone) if streams else \
+                        self._block_product(x, weight, None, plan=plan, gated=False, sums=not alone, rule=rule, squared=alone)
+                if alone:
+                    return product
+            elif m > self.skinny_max_rows and self.skinny_supported_any_rows(x, weight):
+                _gpu(x, weight)
+                block, plan, sums, untimed = self._own_choice(m, n, k, "one", self.block_supported(x, weight))
+
+                def own() -> torch.Tensor:
+                    return (self._block_product if block else self.gemm_wide)(x, weight, None, plan=plan, gated=False, sums=sums, rule=rule)
+
+                def library() -> torch.Tensor:
+                    return self._library_product(x, weight, None, None)
+
+                runs = self._wide_runs(m, n, k, "one", untimed, own, library)
+                if block and runs:
                     return self._block_product(x, weight, None, plan=plan, gated=False, sums=False, rule=rule, squared=True)
+                product = own() if runs else library()
+        if product is not None:
+            return self.activate(product, "relu_squared", x.dtype)
         return self.activate(self.linear(x, weight), "relu_squared", x.dtype)
 
     def linear_float32_out(self, x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
