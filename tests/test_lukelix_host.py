@@ -270,3 +270,63 @@ def test_the_plain_model_reads_another_layers_keys():
     last = dict(tensors, bigram=tensors["bigram"].clone())
     last["bigram"][7] += 1.0
     assert float((plain.forward(config, last, tokens)[0] - base[0]).abs().max()) > 1e-3
+
+
+class Launches:
+    """The library's entry points: notes what was asked for."""
+
+    def __init__(self):
+        self.names = []
+
+    def __getattr__(self, name):
+        return lambda *operands: self.names.append(name) or 0
+
+
+def bare_ops(monkeypatch):
+    from turboserve_amd.kernels import ops as module
+
+    monkeypatch.setattr(module, "_gpu", lambda *tensors: None)
+    ops = object.__new__(module.Ops)
+    ops.core, ops.stream, ops.compute_units = Launches(), lambda: None, 256
+    return ops
+
+
+def placed(shape, dtype, off):
+    """A contiguous tensor that begins `off` elements behind a multiple of 16 bytes."""
+    count = torch.Size(shape).numel()
+    return torch.zeros(count + off, dtype=dtype)[off:].view(shape)
+
+
+@pytest.mark.parametrize("shifted,off", [(None, 0), ("proj", 1), ("held", 1), ("state", 2), ("gain", 4)])
+def test_a_token_in_two_launches_is_for_operands_on_16_bytes(monkeypatch, shifted, off):
+    """Whatever else the three launches take they still get: nothing is refused that they took."""
+    ops = bare_ops(monkeypatch)
+    heads, groups, n, p, tokens = 4, 2, 32, 16, 3
+    inner, channels = heads * p, heads * p + 2 * groups * n
+    width = inner + channels + heads
+    at = {name: off if name == shifted else 0 for name in ("proj", "held", "state", "gain")}
+    ints, bf16 = torch.zeros(tokens + 1, dtype=torch.int32), torch.bfloat16
+    proj, held = placed((2, tokens, width), torch.float32, at["proj"]), placed((4, 3, channels), torch.float32, at["held"])
+    state, gain = placed((4, heads, p, n), torch.float32, at["state"]), placed((inner,), bf16, at["gain"])
+    taps, numbers = torch.zeros(channels, 4, dtype=bf16), torch.zeros(heads)
+    out = ops.selective_token(proj, inner, taps, None, held, inner + channels, numbers, numbers, numbers, state, ints, heads=heads, groups=groups, state_dim=n,
+                              value_dim=p, z_at=0, gain=gain, eps=1e-6, parts=2, dtype=bf16)
+    assert (out is None) == (shifted is not None) and ops.core.names == ([] if shifted else ["ts_selective_token"])
+    u = ops.short_conv(proj, inner, taps, held, ints, ints, ints, tokens=tokens, num_seqs=tokens, dtype=bf16, silu=True)
+    y = ops.selective_state(u, proj, inner + channels, numbers, numbers, numbers, state, ints, ints, num_seqs=tokens, heads=heads, groups=groups, state_dim=n,
+                            value_dim=p, dtype=bf16)
+    assert ops.gated_group_norm(y, proj, 0, gain, 1e-6, 2, bf16).shape == (tokens, inner)
+
+
+@pytest.mark.parametrize("shifted", [None, "state", "sums"])
+def test_the_states_in_one_launch_are_for_slots_on_16_bytes(monkeypatch, shifted):
+    ops = bare_ops(monkeypatch)
+    heads, n, p, tokens = 64, 128, 48, 2048
+    width = heads * p + 2 * n + 2 * heads
+    u, ints, numbers = torch.zeros(tokens, width, dtype=torch.bfloat16), torch.zeros(2, dtype=torch.int32), torch.ones(heads)
+    state, sums = placed((2, heads, p, n), torch.float32, shifted == "state"), placed((2, heads, n), torch.float32, shifted == "sums")
+    plan = (torch.zeros(16, 4, dtype=torch.int32), torch.zeros(1, 4, dtype=torch.int32), 16, 1, 16)
+    ops.decaying_state("gated", u, (0, heads * p, heads * p + n), state, ints, ints, num_seqs=1, heads=heads, groups=1, state_dim=n, value_dim=p,
+                       dtype=torch.bfloat16, proj=u, first_gate=heads * p + 2 * n, numbers=(numbers, numbers), cap=15.0, sums=sums, tops=torch.zeros(2, heads), plan=plan)
+    cut = ["ts_decaying_pass", "ts_decaying_pieces"] if shifted is None else ["ts_decaying_pieces", "ts_decaying_carry", "ts_decaying_pieces"]
+    assert ops.core.names == [*cut, "ts_decaying_walk"]

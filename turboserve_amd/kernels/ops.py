@@ -1331,7 +1331,8 @@ class Ops:
                     _ptr(y), _ptr(norm), _ptr(piece_state), _ptr(decays), _ptr(piece_top), _ptr(rounded), *rows, *gates, _ptr(pieces),
                     n_pieces, heads, groups, state_dim, value_dim, code, mode, self.stream()), "ts_decaying_pieces")
 
-            if self._decaying_passes(n_pieces, first, longest[0] if longest else n_pieces - first + 1, heads, state_dim, held):
+            on_lines = (state.data_ptr() | (0 if sums is None else sums.data_ptr())) % 16 == 0
+            if on_lines and self._decaying_passes(n_pieces, first, longest[0] if longest else n_pieces - first + 1, heads, state_dim, held):
                 _check(self.core.ts_decaying_pass(
                     _ptr(state), _ptr(sums), _ptr(tops), _ptr(state_slots), _ptr(carries), first, _ptr(pieces), _ptr(piece_state), _ptr(piece_top),
                     _ptr(rounded), *rows, *gates[:9], heads, groups, state_dim, value_dim, code, self.stream()), "ts_decaying_pass")
@@ -1371,12 +1372,13 @@ class Ops:
         """A step of single tokens of a selective state space, from its projection to what the output matrix multiplies: :meth:`short_conv` (with
         ``silu``), :meth:`selective_state` and :meth:`gated_group_norm` in two launches, the same bits, or None where they are three: for other
         than four taps, state rows of more than 128, more than eight partial sums or a plain bfloat16 projection, sizes that four elements do not
-        divide, and from 256 parts of rows on, where the norm is another kernel (us a layer, 64 heads of 128 x 64, eight tokens, three launches 3.8 +
+        divide, operands that do not begin on 16 bytes, more columns of B and C than a grid has workgroups for, and from 256 parts of rows on, where the norm is another kernel (us a layer, 64 heads of 128 x 64, eight tokens, three launches 3.8 +
         9.0 + 3.9, two 9.0 + 4.2; a step of nine such layers 486 / 463)."""
         tokens, width = proj.shape[-2], proj.shape[-1]
         inner, channels = heads * value_dim, heads * value_dim + 2 * groups * state_dim
         if (proj.dtype != torch.float32 or taps.shape[1] != 4 or not 4 <= state_dim <= 128 or state_dim % 4 or value_dim % 4 or inner % parts
-                or inner // parts > 1024 or (inner // parts) % 4 or width % 4 or z_at % 4 or tokens * parts >= 256 or proj.data_ptr() % 16
+                or inner // parts > 1024 or (inner // parts) % 4 or width % 4 or z_at % 4 or tokens * parts >= 256 or groups * state_dim > 1 << 20
+                or (proj.data_ptr() | held.data_ptr() | state.data_ptr() | gain.data_ptr()) % 16
                 or (proj.dim() == 3 and (proj.shape[0] > 8 or proj.stride(0) % 4))):
             return None
         _gpu(proj, taps, bias, held, dt_bias, a_log, skip, state, state_slots, gain)
@@ -1390,7 +1392,7 @@ class Ops:
               "the state must be float32 [slots, H, P, N]")
         for t in (dt_bias, a_log, skip):
             _need(t.shape == (heads,) and t.dtype == torch.float32 and t.is_contiguous(), "a rule's numbers must be float32 [H]")
-        _need(heads % groups == 0 and gain.shape == (inner,) and gain.dtype == dtype and gain.is_contiguous() and gain.data_ptr() % 16 == 0
+        _need(heads % groups == 0 and gain.shape == (inner,) and gain.dtype == dtype and gain.is_contiguous()
               and 0 <= z_at and z_at + inner <= width and 0 <= dt_at and dt_at + heads <= width and state_slots.numel() >= tokens,
               "the gates' columns inside the projection, a gain [H P] of the run dtype, a slot a token")
         y = torch.empty((tokens, inner), dtype=torch.float32, device=proj.device)
