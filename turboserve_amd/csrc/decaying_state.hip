@@ -797,13 +797,11 @@ __device__ __forceinline__ int ss_head(int turn, int heads) { return heads % 8 =
 // side by side and a launch that puts them together take 32; one piece 6.6 against 12.8 (alone, in a graph).
 // piece_state [pieces][H][P (gated: + 1, n)][N]; piece_top [pieces][H] (gated): m before each piece.  The slot's own m stays until the
 // finish, since every workgroup here reads it.
-// `to` and `lds` are the same memory: B goes there through the one name, all else uses the other, and __restrict__ keeps the compiler from
-// waiting for every load in flight before every read.  So it must not see that two reads have one address: the slots of what is
-// read behind a barrier have come through an asm behind it.  An edit has to keep that.
+// The wavefronts that ask for loads to LDS read nothing of what those bring, so no wait of the compiler's own stands in their way.
 #define SS_TABLE 16
 template <typename P, int RULE, int ROWS>
 __device__ __forceinline__ void
-decaying_pass(ss_lds_u16* __restrict__ to, ss_lds_u16* __restrict__ lds, SsSteps<RULE>* steps, float (*ends)[SS_PIECE], float* decay_of, float* most_of,
+decaying_pass(ss_lds_u16* lds, SsSteps<RULE>* steps, float (*ends)[SS_PIECE], float* decay_of, float* most_of,
               float* __restrict__ state, float* __restrict__ sums, const float* __restrict__ tops, const int* __restrict__ state_slots,
               const SsCarry* __restrict__ carries, const SsPiece* __restrict__ pieces, float* __restrict__ piece_state,
               float* __restrict__ piece_top, const bf16_t* __restrict__ u, SsRows rows, const P* __restrict__ proj, SsGates gates, int heads,
@@ -847,7 +845,7 @@ decaying_pass(ss_lds_u16* __restrict__ to, ss_lds_u16* __restrict__ lds, SsSteps
                                                                             ((piece.count - 1) * u_width + min(n - n0, ROWS)) * 2, 0x00027000);
 #pragma unroll
     for (int y = 0; y < B_LOADS; ++y)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, to + 2 * X_PIECE + slot * B_PIECE + (HALF * y + TS_WAVE * (wave % 4)) * 8, 16, b_off[y], 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer, lds + 2 * X_PIECE + slot * B_PIECE + (HALF * y + TS_WAVE * (wave % 4)) * 8, 16, b_off[y], 0, 0, 0);
   };
   struct Part {
     ts_u32x4 x[X_ITEMS];
@@ -915,8 +913,7 @@ decaying_pass(ss_lds_u16* __restrict__ to, ss_lds_u16* __restrict__ lds, SsSteps
   };
   // Of piece i, whose x and B lie in LDS.
   auto multiply = [&](int i, int slot_b) __attribute__((always_inline)) {
-    int x_now = i % 2 * X_PIECE, b_now = 2 * X_PIECE + slot_b * B_PIECE;
-    asm volatile("" : "+s"(x_now), "+s"(b_now));
+    const int x_now = i % 2 * X_PIECE, b_now = 2 * X_PIECE + slot_b * B_PIECE;
     constexpr int STEPS = SS_PIECE / 32;
     ts_u32x4 bf[STEPS][2], xf[STEPS][3];
 #pragma unroll
@@ -1035,7 +1032,7 @@ decaying_pass_kernel(float* __restrict__ state, float* __restrict__ sums, const 
   __shared__ SsSteps<RULE> steps[8];
   __shared__ __attribute__((aligned(16))) float ends[SS_TABLE][SS_PIECE];  // the tokens' weights at their piece's end
   __shared__ float decay_of[SS_TABLE], most_of[SS_TABLE];
-  decaying_pass<P, RULE, ROWS>((ss_lds_u16*)ss_lds, (ss_lds_u16*)ss_lds, steps, ends, decay_of, most_of, state, sums, tops, state_slots, carries,
+  decaying_pass<P, RULE, ROWS>((ss_lds_u16*)ss_lds, steps, ends, decay_of, most_of, state, sums, tops, state_slots, carries,
                                pieces, piece_state, piece_top, u, rows, proj, gates, heads, groups, n, p);
 }
 
