@@ -214,6 +214,26 @@ def test_the_convolution_of_rows_moves_the_state_on(ops, taps, lead):
     assert torch.equal(*outs) and torch.equal(*states)
 
 
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("lengths", [[40, 9] + [1] * 13, [33], [2] * 20, [3, 8, 16, 7] + [1] * 63])
+def test_the_convolution_moves_the_state_on_two_ways(ops, monkeypatch, taps, lengths):
+    """In the launch of the rows or by one behind it: the bits of the kernel that takes a row a workgroup."""
+    g = torch.Generator().manual_seed(10 * taps + len(lengths))
+    channels, width, first, tokens = 36, 44, 4, sum(lengths)
+    starts, slots = [sum(lengths[:i]) for i in range(len(lengths) + 1)], ints([2 * (len(lengths) - 1 - i) for i in range(len(lengths))])
+    seqs = ints([j for j, n in enumerate(lengths) for _ in range(n)])
+    proj = torch.randn(tokens, width, generator=g).bfloat16().to(DEV)
+    weight, bias = torch.randn(channels, taps, generator=g).bfloat16().to(DEV), torch.randn(channels, generator=g).bfloat16().to(DEV)
+    results = []
+    for given, moves in ((proj, True), (proj, False), (proj.float().unsqueeze(0), False)):
+        monkeypatch.setattr(type(ops), "_conv_moves", staticmethod(lambda *sizes: moves))
+        state = torch.randn(2 * len(lengths) + 1, max(taps - 1, 1), channels, generator=torch.Generator().manual_seed(taps)).to(DEV)
+        results.append((ops.short_conv(given, first, weight, state, slots, seqs, ints(starts), tokens=tokens, num_seqs=len(lengths), dtype=torch.bfloat16,
+                                       bias=bias, silu=False), state))
+    for out, state in results[:2]:
+        assert torch.equal(out, results[2][0]) and torch.equal(state, results[2][1])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads,kv_heads,dim,vdim,turned,tokens", [(4, 2, 16, 24, 8, 40), (3, 3, 12, 12, 12, 5), (2, 1, 128, 128, 128, 70),
                                                                    (1, 1, 64, 32, 6, 33), (6, 0, 32, 32, 16, 90), (3, 0, 20, 20, 4, 2), (2, 2, 72, 40, 40, 37)])

@@ -330,3 +330,48 @@ def test_the_states_in_one_launch_are_for_slots_on_16_bytes(monkeypatch, shifted
                        dtype=torch.bfloat16, proj=u, first_gate=heads * p + 2 * n, numbers=(numbers, numbers), cap=15.0, sums=sums, tops=torch.zeros(2, heads), plan=plan)
     cut = ["ts_decaying_pass", "ts_decaying_pieces"] if shifted is None else ["ts_decaying_pieces", "ts_decaying_carry", "ts_decaying_pieces"]
     assert ops.core.names == [*cut, "ts_decaying_walk"]
+
+
+@pytest.mark.parametrize("taps,lengths,moves", [
+    (1, [40], True), (2, [2000] + [1] * 63, True), (2, [2] * 20, True), (3, [2000], True), (4, [2000], True), (4, [500] * 4, True), (4, [9] * 20, True), (4, [2] * 20, False),
+    (4, [2000, 1], False), (4, [300] + [1] * 8, False), (5, [2000], True), (8, [40], True), (8, [500, 500], False), (8, [2000, 1], False),
+])
+def test_a_tile_of_many_requests_leaves_their_inputs_to_a_launch_of_its_own(monkeypatch, taps, lengths, moves):
+    """The rows' launch moves one request on after another; the launch behind it all of them side by side."""
+    ops = bare_ops(monkeypatch)
+    asked = []
+    ops.core = type("Core", (), {"ts_short_conv": staticmethod(lambda *of: asked.append(of) or 0)})()
+    tokens, ints = sum(lengths), torch.zeros(sum(lengths) + 1, dtype=torch.int32)
+    taps_of = torch.zeros(8, taps, dtype=torch.bfloat16)
+    ops.short_conv(torch.zeros(tokens, 8, dtype=torch.bfloat16), 0, taps_of, torch.zeros(len(lengths), max(taps - 1, 1), 8), ints, ints, ints, tokens=tokens,
+                   num_seqs=len(lengths), dtype=torch.bfloat16, singles=lengths.count(1))
+    assert asked[0][-3] == int(moves)
+
+
+@pytest.mark.parametrize("part", ["mamba2", "delta", "attention"])
+def test_the_convolution_is_told_how_many_requests_bring_one_token(part):
+    from types import SimpleNamespace
+
+    from turboserve_amd.parts.attention import GroupedQueryAttention
+    from turboserve_amd.parts.delta import GatedDeltaRule
+    from turboserve_amd.parts.mamba2 import Mamba2
+
+    told = []
+
+    class Told(Exception):
+        pass
+
+    def short_conv(*operands, **more):
+        told.append(more["singles"])
+        raise Told
+
+    class Any(SimpleNamespace):
+        def __getattr__(self, name):
+            return 1
+
+    ops = SimpleNamespace(linear=lambda x, *rest, **more: x, short_conv=short_conv)
+    layer = Any(runtime=SimpleNamespace(ops=ops, dtype=torch.bfloat16))
+    ctx = Any(num_tokens=9, num_seqs=5, num_decode_seqs=4, carried={})
+    with pytest.raises(Told):
+        {"mamba2": Mamba2, "delta": GatedDeltaRule, "attention": GroupedQueryAttention}[part].heads_out(layer, torch.zeros(9, 8), ctx, (Any(), Any()))
+    assert told == [4]

@@ -9,9 +9,9 @@
 // where given, is added; with `activation` 1 the result then goes through silu.  The result is [T, channels] of type T, or 32-bit.
 //
 // In a step whose requests all bring one token, the thread that computes a channel of a request also moves the channel's state on.  Prompt
-// portions in bfloat16 take four channels by eight rows a thread (short_conv_rows_kernel), the same arithmetic, and move the
-// state on in the same launch, too.  Behind the general kernel a second one (short_conv_carry_kernel) moves each request's last K - 1
-// inputs into its slot.
+// portions in bfloat16 take four channels by eight rows a thread (short_conv_rows_kernel), the same arithmetic, and, asked to, move the
+// state on in the same launch, too.  Behind that kernel otherwise, and behind the general one, a second one (short_conv_carry_kernel) moves each
+// request's last K - 1 inputs into its slot.
 #include "vec.hpp"
 
 template <typename P>
@@ -105,11 +105,12 @@ short_conv_single_kernel(const P* proj, const T* taps, const int* state_slots, f
 // accesses; every input row is read once for all the taps that want it (and the taps of a thread's channels once).  A
 // row's request is the same for all threads of a block, so the cases below are uniform branches.  Per element the
 // sums of the kernel above.
-// The thread whose tile holds a request's first row computes all rows that look at the request's state, those behind the
-// tile among them (the next tile leaves them out), and so can move the state on itself: a launch for that alone was 5 us of the 19 that
-// 6,144 channels of 2,000 rows took, and the next kernel waited for it.
+// MOVES: the thread whose tile holds a request's first row computes all rows that look at the request's state, those behind the
+// tile among them (the next tile leaves them out), and so can move the state on itself, without a launch for that alone that the next kernel
+// waits for (6,144 channels of 2,000 rows, four taps, 15.2 -> 13.1 us, 17.6 without the test for tiles inside a request).  It does so for
+// one request after another, three trips to memory each, so a tile of many short requests holds the launch up: Ops.short_conv chooses.
 #define SC_TILE 8
-template <typename O, int K>
+template <typename O, int K, bool MOVES>
 __global__ void __launch_bounds__(256)
 short_conv_rows_kernel(O* __restrict__ out, const bf16_t* __restrict__ proj, int width, int first_col, int channels,
                        const bf16_t* __restrict__ taps, const bf16_t* __restrict__ bias, float* __restrict__ state,
@@ -177,10 +178,10 @@ short_conv_rows_kernel(O* __restrict__ out, const bf16_t* __restrict__ proj, int
     const int seq = token_seq[t];
     const int index = t - query_start_loc[seq];  // the token's place in its request's portion
     if (index == 0) begins |= 1 << j;
-    if (index < K - 1 && index > j) continue;  // the tile before computes it
+    if (MOVES && index < K - 1 && index > j) continue;  // the tile before computes it
     row(t, seq, index, [&](int f) __attribute__((always_inline)) { return raw[j + f]; });
   }
-  if (K == 1 || begins == 0) return;
+  if (!MOVES || begins == 0) return;
   const int begin = query_start_loc[last_seq];
   if (begin >= t0) {
     const int end = min(begin + K - 1, query_start_loc[last_seq + 1]);
@@ -234,11 +235,12 @@ static int launch_short_conv_carry(float* state, const void* proj, int splits, l
   return ts_launch_status();
 }
 
-// dtype: the run's type (taps, and the projection unless it is partial sums); out_f32: a 32-bit result.
+// dtype: the run's type (taps, and the projection unless it is partial sums); out_f32: a 32-bit result; moves: the kernel of
+// prompt portions moves the state on itself.
 extern "C" int ts_short_conv(void* out, int out_f32, const void* proj, int in_f32, int splits, long split_stride, int width,
                              int first_col, int channels, const void* taps, const void* bias, int k, float* state,
                              const int* state_slots, const int* token_seq, const int* query_start_loc, int tokens,
-                             int num_seqs, int activation, int dtype, hipStream_t stream) {
+                             int num_seqs, int activation, int moves, int dtype, hipStream_t stream) {
   if (tokens == 0) return TS_OK;
   if (!out || !proj || !taps || (!state && k > 1) || !state_slots || !token_seq || !query_start_loc) return TS_ERR_ARG;
   if (k < 1 || k > SC_MAX_TAPS || channels < 1 || first_col < 0 || first_col + channels > width || splits < 1) return TS_ERR_SHAPE;
@@ -249,20 +251,24 @@ extern "C" int ts_short_conv(void* out, int out_f32, const void* proj, int in_f3
   if (dtype == TS_BF16 && !in_f32 && !single && tokens >= 32 && channels % 4 == 0 && width % 4 == 0 && first_col % 4 == 0 &&
       ((uintptr_t)proj | (uintptr_t)out | (uintptr_t)state | (uintptr_t)taps) % 16 == 0) {
     const dim3 wide((tokens + SC_TILE - 1) / SC_TILE, (channels / 4 + 255) / 256);
-#define SC_ROWS(K)                                                                                                       \
-  case K:                                                                                                                \
-    if (out_f32)                                                                                                         \
-      hipLaunchKernelGGL((short_conv_rows_kernel<float, K>), wide, block, 0, stream, (float*)out, (const bf16_t*)proj, width,       \
-                         first_col, channels, (const bf16_t*)taps, (const bf16_t*)bias, state, state_slots, token_seq, query_start_loc, activation, tokens);  \
-    else                                                                                                                 \
-      hipLaunchKernelGGL((short_conv_rows_kernel<bf16_t, K>), wide, block, 0, stream, (bf16_t*)out, (const bf16_t*)proj, width,     \
-                         first_col, channels, (const bf16_t*)taps, (const bf16_t*)bias, state, state_slots, token_seq, query_start_loc, activation, tokens);  \
+#define SC_ROWS_GO(O, K, MOVES)                                                                                                                  \
+  hipLaunchKernelGGL((short_conv_rows_kernel<O, K, MOVES>), wide, block, 0, stream, (O*)out, (const bf16_t*)proj, width, first_col, channels,   \
+                     (const bf16_t*)taps, (const bf16_t*)bias, state, state_slots, token_seq, query_start_loc, activation, tokens)
+#define SC_ROWS(K)                                       \
+  case K:                                                \
+    if (out_f32 && moves) SC_ROWS_GO(float, K, (K > 1)); \
+    else if (out_f32) SC_ROWS_GO(float, K, false);       \
+    else if (moves) SC_ROWS_GO(bf16_t, K, (K > 1));      \
+    else SC_ROWS_GO(bf16_t, K, false);                   \
     break;
     switch (k) {
       SC_ROWS(1) SC_ROWS(2) SC_ROWS(3) SC_ROWS(4) SC_ROWS(5) SC_ROWS(6) SC_ROWS(7) SC_ROWS(8)
     }
 #undef SC_ROWS
-    return ts_launch_status();
+#undef SC_ROWS_GO
+    const int status = ts_launch_status();
+    if ((moves && k > 1) || status != TS_OK) return status;
+    return launch_short_conv_carry<bf16_t>(state, proj, 1, 0, width, first_col, channels, k, state_slots, query_start_loc, num_seqs, stream);
   }
   if (single && k == 4 && splits <= 8 && (dtype == TS_F32 || (dtype == TS_BF16 && in_f32))) {
 #define SC_SINGLE(T, O, BATCH)                                                                                                      \

@@ -98,7 +98,7 @@ _SIGNATURES: dict[str, dict[str, list]] = {
                              c_int, c_int, c_void_p, c_int, c_long, c_void_p],
         "ts_scale_cap": [c_void_p, c_long, c_float, c_float, c_void_p],
         "ts_short_conv": [c_void_p, c_int, c_void_p, c_int, c_int, c_long, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p,
-                          c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
+                          c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
         "ts_decaying_walk": [*[c_void_p] * 6, c_int, c_int, c_long, *[c_int] * 4, c_void_p, c_int, c_int, c_long, c_int, c_int, c_void_p,
                              c_void_p, c_float, c_void_p, c_float, c_void_p, c_void_p, *[c_int] * 8, c_void_p],
         "ts_decaying_pass": [*[c_void_p] * 5, c_int, *[c_void_p] * 4, *[c_int] * 4, c_void_p, c_int, c_int, c_long, c_int, c_int, c_void_p,
@@ -1085,13 +1085,14 @@ class Ops:
 
     def short_conv(self, proj: torch.Tensor, first_col: int, taps: torch.Tensor, state: torch.Tensor, state_slots: torch.Tensor,
                    token_seq: torch.Tensor, query_start_loc: torch.Tensor, *, tokens: int, num_seqs: int, dtype: torch.dtype,
-                   silu: bool = False, out_float32: bool = False, bias: torch.Tensor | None = None) -> torch.Tensor:
+                   silu: bool = False, out_float32: bool = False, bias: torch.Tensor | None = None, singles: int = 0) -> torch.Tensor:
         """A short causal convolution over time on the ``C`` columns of ``proj`` from ``first_col`` on (``taps [C,
         K]``: ``y_t = sum_j taps[:, j] u_(t - K + 1 + j)``), continuing every request from the ``K - 1`` inputs its
         state slot holds (``state [slots, max(K - 1, 1), C]`` 32-bit, oldest first) and leaving its last ``K - 1``
         inputs there.
         ``proj`` is ``[T, W]`` of the run dtype or 32-bit partial sums.  Returns ``[T, C]`` of the run dtype (32-bit
-        with ``out_float32``), plus ``bias [C]`` where given, through ``silu`` if asked."""
+        with ``out_float32``), plus ``bias [C]`` where given, through ``silu`` if asked.  ``singles``: how many of the requests are known to bring one
+        token (they choose the launches, not the result)."""
         _gpu(proj, taps, bias, state, state_slots, token_seq, query_start_loc)
         _i32(state_slots, "state_slots")
         _i32(token_seq, "token_seq")
@@ -1113,8 +1114,20 @@ class Ops:
         code = dtype_code(dtype)
         _check(self.core.ts_short_conv(_ptr(out), 1 if wide else 0, _ptr(proj), is_f32, splits, stride, width, first_col, channels,
                                        _ptr(taps), _ptr(bias), k, _ptr(state), _ptr(state_slots), _ptr(token_seq), _ptr(query_start_loc),
-                                       tokens, num_seqs, 1 if silu else 0, code, self.stream()), "ts_short_conv")
+                                       tokens, num_seqs, 1 if silu else 0, 1 if self._conv_moves(k, tokens, num_seqs, singles) else 0, code,
+                                       self.stream()), "ts_short_conv")
         return out
+
+    @staticmethod
+    def _conv_moves(taps: int, tokens: int, num_seqs: int, singles: int) -> bool:
+        """Whether the launch that convolves prompt portions moves the requests' inputs on itself, one request of a tile of eight rows after another, or a
+        launch behind it does, all of them side by side.  (us, 6,144 / 512 channels, itself / behind: two taps, 40 rows 4.8 / 6.9 and 4.4 / 5.9, 64
+        requests in 103 rows 7.2 / 8.8 and 6.5 / 7.6; four, 2,000 rows 13.1 / 15.2 and 6.2 / 7.2, 200 requests of nine 18.7 / 25.2 and 7.2 / 7.9, 40 of
+        five 9.2 / 10.0 and 8.0 / 7.6, 2,000 rows and 63 single tokens 25.1 / 21.5 and 11.2 / 9.6, and eight 20.2 / 18.1 and 10.6 / 9.2; eight, 2,000 rows
+        19.2 / 20.2 and 9.4 / 9.8, two requests of 500 18.9 / 16.6 and 11.5 / 9.9, 16 of 33 20.6 / 15.8 and 13.0 / 10.1.)"""
+        if taps <= 2:
+            return True
+        return singles == 0 and tokens >= 8 * num_seqs if taps <= 4 else num_seqs == 1
 
     def delta_rule(self, u: torch.Tensor, proj: torch.Tensor, *, beta_at: int, decay_at: int, gate_at: int, a2: torch.Tensor,
                    dt_bias: torch.Tensor, a_log: torch.Tensor, g2: torch.Tensor, gain: torch.Tensor, eps: float,

@@ -319,7 +319,7 @@ class GroupedQueryAttention(Mixer):
             cache, held = cache
             # q, k and v of the step through the convolution; the gate's columns stay in `proj`.
             qkv = ops.short_conv(proj, 0, self.conv_weight, held.state, ctx.state_slots, ctx.token_seq, ctx.query_start_loc,
-                                 tokens=ctx.num_tokens, num_seqs=ctx.num_seqs, dtype=self.runtime.dtype)
+                                 tokens=ctx.num_tokens, num_seqs=ctx.num_seqs, dtype=self.runtime.dtype, singles=ctx.num_decode_seqs)
         elif self.gate_name is not None:
             shape["tail"] = self.num_heads
         if self.values_are_keys:

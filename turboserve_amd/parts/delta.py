@@ -139,7 +139,7 @@ class GatedDeltaRule(Mixer):
         memory, held = cache
         proj = ops.linear(x, self.fused)
         u = ops.short_conv(proj, 0, self.conv_weight, held.state, ctx.state_slots, ctx.token_seq, ctx.query_start_loc,
-                           tokens=ctx.num_tokens, num_seqs=ctx.num_seqs, dtype=dtype, silu=True, out_float32=True)
+                           tokens=ctx.num_tokens, num_seqs=ctx.num_seqs, dtype=dtype, silu=True, out_float32=True, singles=ctx.num_decode_seqs)
         return ops.delta_rule(u, proj, beta_at=self.beta_at, decay_at=self.decay_at, gate_at=self.gate_at, a2=self.a2,
                               dt_bias=self.dt, a_log=self.a_log, g2=self.g2, gain=self.gain, eps=self.norm_eps,
                               state=memory.state, state_slots=ctx.state_slots, query_start_loc=ctx.query_start_loc,

@@ -116,7 +116,8 @@ class Mamba2(Mixer):
             if out is not None:
                 return out
         u = ops.short_conv(proj, self.inner, self.conv_weight, held.state, ctx.state_slots, ctx.token_seq, ctx.query_start_loc,
-                           tokens=ctx.num_tokens, num_seqs=ctx.num_seqs, dtype=dtype, silu=True, bias=self.conv_bias)
+                           tokens=ctx.num_tokens, num_seqs=ctx.num_seqs, dtype=dtype, silu=True, bias=self.conv_bias,
+                           singles=ctx.num_decode_seqs)
         plan = ops.decaying_plan(ctx, dtype, self.state_dim, self.value_dim)
         y = ops.selective_state(u, proj, self.inner + self.channels, self.dt_bias, self.a_log, self.skip, memory.state, ctx.state_slots,
                                 ctx.query_start_loc, num_seqs=ctx.num_seqs, heads=self.num_heads, groups=self.groups,
