@@ -346,6 +346,13 @@ def test_the_unit_of_a_product_asks_for_the_products_choice_once(monkeypatch, m,
     assert ops.linear(x, w)[0] == kernel  # the same product without the unit
 
 
+@pytest.mark.parametrize("n,k,ranges", [(8320, 3136, 3), (8320, 3584, 3), (8704, 3584, 3), (8320, 4608, 4), (9728, 3584, 3), (12288, 3584, 2), (18944, 3584, 2), (2048, 8192, 3)])
+def test_finer_grids_over_a_long_k_leave_a_wavefront_five_slices(n, k, ranges):
+    """Five ranges of 8,320 x 3,584, three slices a wavefront, were slower than three."""
+    per_wave, splits, tile = Planner()._stream_plan(n, k, None)
+    assert (splits, tile) == (ranges, 2) and per_wave == -(-k // 64 // (4 * ranges)) and per_wave >= 5
+
+
 def test_one_range_with_a_nearly_empty_last_round_is_left_to_the_tiled_product():
     ops = Planner()
     assert ops._stream_plan(20480, 5120, None) is None and ops._stream_plan(27648, 5120, 1) is None and ops._stream_plan(17408, 2048, 1) is None

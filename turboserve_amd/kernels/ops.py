@@ -2826,7 +2826,7 @@ class Ops:
         for want in range(1, min(max_splits or 8, 8) + 1):
             per_wave = -(-slices // (4 * want))
             splits = -(-slices // (4 * per_wave))
-            if splits != want:
+            if splits != want or (splits > 1 and per_wave < 5 and tiles > units and k > 3072 and k % 4096):
                 continue
             cost = self._stream_cost(n, k, splits)
             if best is None or cost < best[0]:
@@ -2846,7 +2846,9 @@ class Ops:
         where some units have two workgroups or more (at 36 grids that give some units two and some one look as soon as finer ones; one / eight
         rows, 12,288 x 3,584 as one / two ranges 16.5 / 15.6 and 17.8 / 16.1, 18,944 x 3,584 24.9 / 22.3 and 25.1 / 22.7, 12,288 x 5,120
         23.9 / 21.4 and 25.1 / 21.8, x 6,144 27.6 / 26.1 and 29.9 / 26.8; not of multiples of 4,096, whose ranges lie in the same
-        channels of the memory, x 4,096 17.8 / 20.2 and 18.8 / 20.5; 13,312 x 2,560 13.0 / 14.0 and 14.8 / 14.1)."""
+        channels of the memory, x 4,096 17.8 / 20.2 and 18.8 / 20.5; 13,312 x 2,560 13.0 / 14.0 and 14.8 / 14.1).  The finer grids leave a wavefront no fewer than
+        five slices (8,320 x 3,584 as three / four / five ranges, five, four and three slices, 11.9 / 12.3 / 13.2 and 12.1 / 12.2 / 13.1, x 3,136 11.0 / 11.1 /
+        11.8)."""
         rounds = -(-(-(-n // 32) * splits) // self.compute_units)
         rate = 31e3 if rounds > 1 and k > 3072 and k % 4096 else 36e3
         return max(2.0 * n * k / 6.6e6, rounds * 64.0 * k / splits / rate) + 0.12 * splits
