@@ -332,6 +332,17 @@ def test_the_states_in_one_launch_are_for_slots_on_16_bytes(monkeypatch, shifted
     assert ops.core.names == [*cut, "ts_decaying_walk"]
 
 
+@pytest.mark.parametrize("heads,n,columns,requests,tokens,passes", [
+    (64, 128, 64, 1, 128, True), (64, 128, 64, 1, 2000, True), (8, 128, 256, 6, 300, True), (8, 256, 512, 1, 2048, True), (8, 256, 513, 1, 2048, False),
+    (16, 64, 64, 1, 2048, False), (32, 128, 128, 20, 100, False), (4, 16, 64, 1, 300, True), (4, 16, 64, 1, 1000, False), (64, 16, 64, 8, 500, True),
+    (64, 64, 65, 4, 300, False), (24, 16, 64, 16, 100, True),
+])
+def test_which_way_the_states_before_the_pieces_are_made(monkeypatch, heads, n, columns, requests, tokens, passes):
+    """The sooner of two launches side by side and one that takes a request's pieces one behind the other, as measured."""
+    longest = -(-tokens // 128)
+    assert bare_ops(monkeypatch)._decaying_passes(longest * requests, requests, longest, heads, n, columns) == passes
+
+
 @pytest.mark.parametrize("taps,lengths,moves", [
     (1, [40], True), (2, [2000] + [1] * 63, True), (2, [2] * 20, True), (3, [2000], True), (4, [2000], True), (4, [500] * 4, True), (4, [9] * 20, True), (4, [2] * 20, False),
     (4, [2000, 1], False), (4, [300] + [1] * 8, False), (5, [2000], True), (8, [40], True), (8, [500, 500], False), (8, [2000, 1], False),
