@@ -335,7 +335,7 @@ def test_the_states_in_one_launch_are_for_slots_on_16_bytes(monkeypatch, shifted
 @pytest.mark.parametrize("heads,n,columns,requests,tokens,passes", [
     (64, 128, 64, 1, 128, True), (64, 128, 64, 1, 2000, True), (8, 128, 256, 6, 300, True), (8, 256, 512, 1, 2048, True), (8, 256, 513, 1, 2048, False),
     (16, 64, 64, 1, 2048, False), (32, 128, 128, 20, 100, False), (4, 16, 64, 1, 300, True), (4, 16, 64, 1, 1000, False), (64, 16, 64, 8, 500, True),
-    (64, 64, 65, 4, 300, False), (24, 16, 64, 16, 100, True),
+    (64, 64, 65, 4, 300, False), (24, 16, 64, 16, 100, True), (16, 64, 64, 20, 40, False), (64, 128, 129, 1, 33, False), (16, 64, 64, 8, 40, True),
 ])
 def test_which_way_the_states_before_the_pieces_are_made(monkeypatch, heads, n, columns, requests, tokens, passes):
     """The sooner of two launches side by side and one that takes a request's pieces one behind the other, as measured."""

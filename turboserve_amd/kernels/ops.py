@@ -1266,18 +1266,19 @@ class Ops:
     def _decaying_passes(self, pieces: int, requests: int, longest: int, heads: int, state_dim: int, columns: int) -> bool:
         """Whether the states before a step's pieces are made a request's pieces one behind the other (``ts_decaying_pass``), not side by
         side and put together by a launch of its own.  By a small model, in microseconds: a workgroup has a compute unit to itself and takes 3.5
-        and 1.05 a piece of its request (``longest`` at most; 1.15 where it weighs the x of 64 columns), side by side it is 11 to 13 and 2.4 for every
-        million elements of a piece's state
+        and 1.05 a piece of its request (``longest`` at most; 1.15 where it weighs the x of 64 columns), rounds of workgroups 3.5 more, side by side it is 11
+        to 13 and 2.8 for every million elements of a piece's state
         (side by side / one behind the other, heads x rows x columns: 64 x 128 x 64, one prompt of 128 / 512 / 2,000 tokens 12.8 / 6.6,
         18.1 / 9.8, 32.2 / 22.5; 8 x 128 x 256, of 2,048 24.2 / 19.1, six of 300 24.9 / 19.3; 8 x 256 x 512 53.4 / 41.7, with the sum of
         keys, a third round for few, 57.5 / 66.2; 16 x 64 x 64, 32 workgroups, 14.2 / 17.2; 32 x 128 x 128, 20 of 100 tokens, 20 rounds,
-        47.3 / 84.6; with the outputs, 4 x 16 x 64, one prompt of 300 / 1,000 tokens 19.4 / 16.6, 20.1 / 22.7, 64 x 64 x 64 with the sum of keys, four of 300
-        40.4 / 42.3).  Over 370 sizes (three rules, 4 to 64 heads, rows of 16 to 256, one to 16 requests of 100 to 8,000 tokens) what it picks takes 0.2%
-        more than the sooner way on average, at most 7%."""
+        47.3 / 84.6; with the outputs, 4 x 16 x 64, one prompt of 300 / 1,000 tokens 19.4 / 16.6, 20.1 / 22.7, 16 x 64 x 64, 20 of 40 19.8 / 23.5, 64 x 64 x 64
+        with the sum of keys, four of 300 40.4 / 42.3, 64 x 128 x 128 with it, one of 33 23.4 / 26.7).  Over 730 sizes (three rules, 4 to 64 heads, rows
+        of 16 to 256, one to 20 requests of 33 to 8,000 tokens) what it picks takes 0.2% more than the sooner way on average, at most 11%."""
         rows = 32 if state_dim <= 32 else 64 if state_dim <= 64 else 128
         workgroups = heads * requests * -(-state_dim // rows) * -(-columns // (2048 // rows))
-        behind = -(-workgroups // self.compute_units) * (3.5 + (1.15 if rows == 32 else 1.05) * longest)
-        return behind < 11.0 + min(state_dim, 128) / 64 + 2.4e-6 * pieces * heads * max(state_dim, 32) * columns
+        rounds = -(-workgroups // self.compute_units)
+        behind = rounds * (3.5 + (1.15 if rows == 32 else 1.05) * longest) + (3.5 if rounds > 1 else 0.0)
+        return behind < 11.0 + min(state_dim, 128) / 64 + 2.8e-6 * pieces * heads * max(state_dim, 32) * columns
 
     def decaying_state(self, rule: str, u: torch.Tensor, columns: tuple[int, int, int], state: torch.Tensor, state_slots: torch.Tensor,
                        query_start_loc: torch.Tensor, *, num_seqs: int, heads: int, groups: int, state_dim: int, value_dim: int,
