@@ -1380,7 +1380,8 @@ gated_group_norm_kernel(T* __restrict__ out, const float* __restrict__ y, const 
 }
 
 // The same bits for a prompt's many parts of up to 256 CHUNKS elements: a wavefront a part, four a workgroup, which meet nowhere; a part's quads
-// and their sums lie as a workgroup's wavefronts have them above.  64 MB for 2,000 rows of eight parts of 512: 13.5 -> 12.8 us.
+// and their sums lie as a workgroup's wavefronts have them above.  Parts of 512, eight a row, a workgroup / a wavefront a part with the same
+// arithmetic: 1,000 rows 7.3 / 7.1 us, 2,000 (64 MB) 12.6 / 12.0, 4,096 29.0 / 23.2; four of 256, 2,000 rows 4.8 / 4.4.
 template <typename T, int CHUNKS>
 __global__ void __launch_bounds__(256)
 gated_group_norm_rows_kernel(T* __restrict__ out, const float* __restrict__ y, const T* __restrict__ proj, int width, int z_at,
@@ -1817,8 +1818,8 @@ static int launch_gated_group_norm(void* out, const float* y, const void* proj, 
       return ts_launch_status();
     }
     // A wavefront a part where the projection is one of 16 bits and there are parts enough that four a workgroup fill the units (us, a workgroup /
-    // a wavefront a part of 512, eight a row: 32 rows 2.6 / 2.8, 128 2.9 / 3.0, 192 3.3 / 3.2, 512 4.5 / 4.2, 1,024 7.1 / 6.5; of two partial
-    // sums, which a workgroup asks for sooner, 32 rows 2.8 / 3.4, 256 4.0 / 4.2).
+    // a wavefront a part of 512, eight a row: 32 rows 2.6 / 2.8, 128 2.9 / 3.0, as soon from 192 to 512, 3.1 and 4.9, and the sooner beyond, figures
+    // at the kernel; of two partial sums, which a workgroup asks for sooner, 32 rows 2.8 / 3.4, 256 4.0 / 4.2).
     const long items = (long)tokens * parts;
     if constexpr (sizeof(P) == 2) {
 #define GN_ROWS(CHUNKS)                                                                                                                     \
